@@ -1280,6 +1280,11 @@ static void launch_riding_norm(const GemmArgs& a, hipStream_t st) {
   else launch_rmsnorm_rows(a.C, a.norm_w, a.norm_out, a.M, a.N, a.ldc, a.N, a.norm_eps, st);
 }
 
+static bool plan_from_env() {   // a tile or split factor forced for an A/B (plan_gemm)
+  static const bool on = getenv("AHA_GEMM_TILE") != nullptr || getenv("AHA_GEMM_SPLITK") != nullptr;
+  return on;
+}
+
 void launch_gemm(const GemmArgs& a_in, hipStream_t st) {
   if (a_in.M <= 0 || a_in.N <= 0) return;
   GemmArgs a = a_in;
@@ -1293,6 +1298,18 @@ void launch_gemm(const GemmArgs& a_in, hipStream_t st) {
   static const int e_prow = [] { const char* e = getenv("AHA_GEMM_PARTIAL_ROWS"); return e ? atoi(e) : 1; }();
   a.partial_rows = e_prow;
   const GemmPlan plan = plan_gemm(a);
+  // Few rows: the kernel that streams W once and joins its K shares in LDS, where it is expected below the tiled plan -- which for its part cannot
+  // be faster than W's bytes at the 4.2 TB/s its staging reaches with few rows (18.1 us for 71 MB on average at 8 rows, 46 us for 201 MB at 32)
+  // and ~5 us of a reduce pass.  (4096 x 12288: 25.9 us against 24 + 5 at 32 rows, 35.5 against 24 + 5 at 64: there the tiles stay.)
+  if (g_force_tile == 0 && !plan_from_env() && gemm_skinny_ok(a)) {
+    int r8;
+    const double tiled = std::max(plan.cost, (double)a.N * a.K * 2.0 / 4.2e6 + (plan.splitk > 1 ? 5.0 : 2.0));
+    if (gemm_skinny_plan(a, &r8) < tiled) {
+      launch_gemm_skinny(a, st);
+      if (a.norm_w) launch_riding_norm(a, st);
+      return;
+    }
+  }
   // Ragged N (ViT fc1: N = 4304 = 16 x 256 + 208): the 17th column of 256^2 tiles makes 272 units = two rounds on 256 CUs for
   // 1.06 rounds of work.  Where the model says it pays, the columns up to the last multiple of 256 run as one GEMM and the
   // remaining columns as a second one (sub-views of W / C / bias / residual: same rounding, same results).

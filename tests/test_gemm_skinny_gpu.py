@@ -1,0 +1,46 @@
+"""-m gpu: the few-row GEMM (csrc/kernels_gemm_skinny.hip), which launch_gemm takes by itself for these shapes, against the oracle chain."""
+import pytest
+import torch
+
+from oracle import qwen3 as oq
+from tests.test_ops_gpu import NM, assert_close_ulps, rnd
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [
+    (8, 64),         # one eight-row group, one k chunk for four waves
+    (1000, 192),     # N ends inside a block of 16, 24, 32 and 48 rows; fewer chunks than waves
+    (6144, 320),     # 24 rows per block: half a fragment unused
+    (12320, 448),    # 48 rows per block, the last block short
+    (40, 4160),      # more chunks than ring stages, an uneven share per wave
+])
+def test_few_rows_every_row_count_and_block_width(gpu, M, N, K):
+    """One f32 sum per element, rounded once per op as in the tiled kernels: a sum next to a rounding boundary moves one op's result by one ulp, so
+    1 ulp for the plain product, 2 behind bias and residual, 3 behind the GELU (whose hardware exp2 adds one; no share of equal bits is asked for:
+    far in its tail the results are below 2^-8 of the rms and carry no comparable bits).  The rows behind M of the output stay untouched."""
+    from aha_amd import ops, _lib
+    from aha_amd._lib import check, lib
+    A, W, b, r = rnd((M, K), 51), rnd((N, K), 52, 0.05), rnd((N,), 53, 0.5), rnd((M, N), 54)
+    Ad, Wd, bd, rd = (t.to(gpu) for t in (A, W, b, r))
+    out = torch.full((M + 3, N), 7.0, dtype=torch.bfloat16, device=gpu)
+    check(lib().aha_hip_gemm(Ad.data_ptr(), Wd.data_ptr(), out.data_ptr(), M, N, K, K, K, N, None, None, _lib.ACT_NONE, torch.cuda.current_stream().cuda_stream))
+    assert_close_ulps(out[:M], NM.linear(A.float(), W.float()), 1, None, "plain")
+    assert (out[M:] == 7.0).all()
+    assert torch.equal(ops.gemm(Ad, Wd), out[:M])
+    full = ops.gemm(Ad, Wd, bd, rd, _lib.ACT_NONE)
+    assert_close_ulps(full, NM.r(r.float() + NM.linear(A.float(), W.float(), b.float())), 2, None, "bias + residual")
+    gelu = NM.r(torch.nn.functional.gelu(NM.linear(A.float(), W.float(), b.float()), approximate="tanh"))
+    assert_close_ulps(ops.gemm(Ad, Wd, bd, None, _lib.ACT_GELU_TANH), gelu, 3, None, "bias + gelu")
+
+
+@pytest.mark.parametrize("M", [1, 8, 13, 31, 64])
+@pytest.mark.parametrize("I,K", [(16, 64), (1008, 256), (3072, 1024), (12288, 128)])
+def test_few_rows_gate_up_pairs(gpu, M, I, K):
+    """Gate and up rows in groups of eight per block, the product in the epilogue (interleaved layout of the model loader)."""
+    from aha_amd import ops, _lib
+    A, Wg, Wu = rnd((M, K), 61), rnd((I, K), 62, 0.05), rnd((I, K), 63, 0.05)
+    ref = NM.r(NM.r(oq.silu(NM.linear(A.float(), Wg.float()))) * NM.linear(A.float(), Wu.float()))
+    got = ops.gemm(A.to(gpu), ops.interleave_gate_up(Wg, Wu).to(gpu), None, None, _lib.ACT_SILU_MUL_PAIRS)
+    assert_close_ulps(got, ref, 3, None, "gate * up")
