@@ -50,6 +50,9 @@ void launch_argmax_partials(const float* blk_max, const uint32_t* blk_idx, int n
 void launch_argmax_pair(const float* blk_max, const uint32_t* blk_idx, int n, int row0, float* pairs, int rank, int T, hipStream_t st);
 void launch_argmax_pick(const float* pairs, int T, uint32_t* out, hipStream_t st);
 void launch_argmax_f32(const float* x, int64_t n, float* ws_max, uint32_t* ws_idx, uint32_t* out, hipStream_t st);
+// arg-max of each of `rows` rows (pitch ld) -> out[row]; ws_*: rows * argmax_f32_blocks(n) entries; rows <= 65535
+int argmax_f32_blocks(int64_t n);
+void launch_argmax_f32_rows(const float* x, int64_t n, int64_t ld, int rows, float* ws_max, uint32_t* ws_idx, uint32_t* out, hipStream_t st);
 
 // D11 candidates (kernels_sample.hip): repeat penalty into a working copy of the logits; k largest + full-vocabulary softmax
 // normaliser.  cand_* hold (sample_stage1_waves(V) + 16) * 64 entries (stage-1 candidates, then the 16 x k intermediates),

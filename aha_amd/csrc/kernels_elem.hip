@@ -402,9 +402,11 @@ __device__ __forceinline__ void wave_argmax(float& bv, uint32_t& bi) {
   }
 }
 __global__ __launch_bounds__(256) void argmax_partials_kernel(const float* __restrict__ pv, const uint32_t* __restrict__ pi,
-                                                              int n, uint32_t* __restrict__ out) {
+                                                              int n, uint32_t* __restrict__ out) {   // one block per row of n partials
   __shared__ float sv[4];
   __shared__ uint32_t si[4];
+  pv += (int64_t)blockIdx.x * n;
+  pi += (int64_t)blockIdx.x * n;
   float bv = -INFINITY;
   uint32_t bi = 0xffffffffu;
   for (int i = threadIdx.x; i < n; i += 256) argmax_combine(bv, bi, pv[i], pi[i]);
@@ -413,7 +415,7 @@ __global__ __launch_bounds__(256) void argmax_partials_kernel(const float* __res
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int w = 1; w < 4; ++w) argmax_combine(bv, bi, sv[w], si[w]);
-    *out = bi;
+    out[blockIdx.x] = bi;
   }
 }
 // vocab-parallel lm_head: pairs[2r] = this rank's max logit, pairs[2r+1] = its GLOBAL index (exact in f32: < 2^24), every
@@ -452,10 +454,11 @@ void launch_argmax_pick(const float* pairs, int T, uint32_t* out, hipStream_t st
 void launch_argmax_partials(const float* blk_max, const uint32_t* blk_idx, int n, uint32_t* out, hipStream_t st) {
   hipLaunchKernelGGL(argmax_partials_kernel, dim3(1), dim3(256), 0, st, blk_max, blk_idx, n, out);
 }
-__global__ __launch_bounds__(256) void argmax_f32_stage1(const float* __restrict__ x, int64_t n, float* __restrict__ pv,
-                                                         uint32_t* __restrict__ pi) {
+__global__ __launch_bounds__(256) void argmax_f32_stage1(const float* __restrict__ x, int64_t n, int64_t ld, float* __restrict__ pv,
+                                                         uint32_t* __restrict__ pi) {   // blockIdx.y: row
   __shared__ float sv[4];
   __shared__ uint32_t si[4];
+  x += blockIdx.y * ld;
   float bv = -INFINITY;
   uint32_t bi = 0xffffffffu;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
@@ -468,14 +471,20 @@ __global__ __launch_bounds__(256) void argmax_f32_stage1(const float* __restrict
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int w = 1; w < 4; ++w) argmax_combine(bv, bi, sv[w], si[w]);
-    pv[blockIdx.x] = bv;
-    pi[blockIdx.x] = bi;
+    pv[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = bv;
+    pi[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = bi;
   }
 }
+int argmax_f32_blocks(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>((n + 4095) / 4096, 256)); }
+// Two launches for any number of rows: a batched step's 32 rows took 64 launches, 31 x (5.0 + 2.8) us and as many gaps of a 6 ms step.
+void launch_argmax_f32_rows(const float* x, int64_t n, int64_t ld, int rows, float* ws_max, uint32_t* ws_idx, uint32_t* out, hipStream_t st) {
+  if (rows <= 0) return;
+  const int blocks = argmax_f32_blocks(n);
+  hipLaunchKernelGGL(argmax_f32_stage1, dim3(blocks, rows), dim3(256), 0, st, x, n, ld, ws_max, ws_idx);
+  hipLaunchKernelGGL(argmax_partials_kernel, dim3(rows), dim3(256), 0, st, ws_max, ws_idx, blocks, out);
+}
 void launch_argmax_f32(const float* x, int64_t n, float* ws_max, uint32_t* ws_idx, uint32_t* out, hipStream_t st) {
-  const int blocks = (int)((n + 4095) / 4096 < 256 ? (n + 4095) / 4096 : 256);
-  hipLaunchKernelGGL(argmax_f32_stage1, dim3(blocks > 0 ? blocks : 1), dim3(256), 0, st, x, n, ws_max, ws_idx);
-  launch_argmax_partials(ws_max, ws_idx, blocks > 0 ? blocks : 1, out, st);
+  launch_argmax_f32_rows(x, n, 0, 1, ws_max, ws_idx, out, st);
 }
 
 }  // namespace aha

@@ -97,7 +97,10 @@ int ensure_want(aha_model* m, size_t n) {
   if (rc) return rc;
   l.cap_want = 0;
   const size_t cap = (size_t)round_up((int64_t)n, 16);
-  if ((rc = grow(m, l.want_bufs, cap * l.ld * (l.f32 ? 4 : 2), &l.fin)) || (rc = grow(m, l.want_bufs, cap * l.Vp * 4, (void**)&l.logits))) return rc;
+  if ((rc = grow(m, l.want_bufs, cap * l.ld * (l.f32 ? 4 : 2), &l.fin)) || (rc = grow(m, l.want_bufs, cap * l.Vp * 4, (void**)&l.logits)) ||
+      (rc = grow(m, l.want_bufs, cap * argmax_f32_blocks(m->desc.vocab_size) * 4, (void**)&l.am_max)) ||
+      (rc = grow(m, l.want_bufs, cap * argmax_f32_blocks(m->desc.vocab_size) * 4, (void**)&l.am_idx)))
+    return rc;
   l.cap_want = cap;
   return AHA_OK;
 }
@@ -748,7 +751,7 @@ int layered_forward_batch(aha_model* m, const aha_batch_entry* en, size_t n_en, 
       argmax_single(m);
       m->have_logits = true;
     } else if (argmax_out) {
-      for (size_t i = 0; i < n; ++i) launch_argmax_f32(lg + i * l.Vp, V, m->d_blk_max, m->d_blk_idx, dam + w0 + i, m->stream);
+      launch_argmax_f32_rows(lg, V, l.Vp, (int)n, l.am_max, l.am_idx, dam + w0, m->stream);
     }
     if (logits_out)
       AHA_HIP_CHECK(hipMemcpy2DAsync(logits_out + w0 * V, V * 4, lg, (size_t)l.Vp * 4, V * 4, n, hipMemcpyDeviceToHost, m->stream));

@@ -94,6 +94,8 @@ struct LayeredModel {
   // step buffers, grown on demand
   size_t cap_rows = 0, cap_ents = 0, cap_want = 0;
   float *xa = nullptr, *xb = nullptr, *vfirst = nullptr, *logits = nullptr;
+  float* am_max = nullptr;      // arg-max partials of the wanted rows
+  uint32_t* am_idx = nullptr;
   void *h = nullptr, *qkv = nullptr, *q = nullptr, *o = nullptr, *z = nullptr, *y = nullptr, *fin = nullptr, *ws = nullptr;
   size_t ws_bytes = 0;
   std::vector<float*> ropetab;
