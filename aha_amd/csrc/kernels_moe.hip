@@ -4,7 +4,7 @@
 //   moe_slots_kernel    slots: an expert's (token, choice) pairs one after the other; tiles of `bm` slots of one expert
 //   moe_gemm_kernel     bf16, 128 x 128 tiles (many tokens per expert), rows gathered by slot
 //   moe_gemm256_kernel  bf16, 256 x 256 tiles (kernels_moe256.hip)
-//   moe_gemm_rows_kernel  bf16, 16 x 64 tiles, operands straight to registers (few tokens per expert)
+//   moe_gemm_few_kernel  bf16, up to 32 slots x 16 or 48 weight rows, whole K (few tokens per expert)
 //   moe_gemm_f32_kernel   the 32-bit mode
 #include <math.h>
 
@@ -15,6 +15,7 @@
 #include "attn_common.h"
 #include "kernels_prenorm.h"
 #include "rows_common.h"
+#include "skinny_body.h"
 
 namespace aha {
 
@@ -207,52 +208,64 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
   }
 }
 
-// ---- 16 slots x 64 columns: the k range dealt to the four waves, their sums joined in LDS ---------------------------------------------------------
-template <bool GATHER, bool PAIRS>
-__global__ __launch_bounds__(256) void moe_gemm_rows_kernel(MoeGemmArgs a, MoeRouting r, int ntn) {
-  __shared__ float red[3][4][64][4];
-  const int mt = blockIdx.x / ntn;
-  if (mt >= *r.n_tiles) return;
-  const int n0 = ((int)blockIdx.x - mt * ntn) * 64;
-  const int ex = r.tiles[mt * 3], s0 = r.tiles[mt * 3 + 1], ns = r.tiles[mt * 3 + 2];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, G = lane >> 4, c = lane & 15;
-  const int slot = s0 + min(c, ns - 1);
-  const bf16_t* A = (const bf16_t*)a.A + (int64_t)(GATHER ? r.slot_row[slot] : slot) * a.lda + G * 8;
-  const bf16_t* W = (const bf16_t*)a.W + ((int64_t)ex * a.n + n0 + c) * a.k + G * 8;   // (n is a multiple of 64)
-  f32x4_t acc[4];
+// ---- few slots per expert: up to 32 of them against R8 * 8 weight rows, whole K (skinny_body.h) ---------------------------------------------------
+// Bound by the chosen experts' weights.  Tiles of 32 slots, so that an expert with 17 to 32 of them still reads its weights once; the ring has the
+// activation rows a tile needs (8, 16 or 32).  MI355X, 32 tokens x 2 of 32 experts at the 8B sizes: gate + up (1.4 GB) 348 -> 212 us, down
+// (0.7 GB) 160 -> 107 us (6.6 TB/s) against 16 x 64 tiles that loaded fragments to registers (16 rows x 64 bytes per request).
+constexpr int MOE_FEW = 32;
+
+template <int R8, int M8, bool GATHER, bool PAIRS>
+__device__ __forceinline__ void moe_few_body(const MoeGemmArgs& a, const MoeRouting& r, int n_blk, int ex, int s0, int ns, char* smem) {
+  constexpr int MT = (M8 + 1) / 2;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), G = lane >> 4, c = lane & 15;
+  const bf16_t* W = (const bf16_t*)a.W + (int64_t)ex * a.n * a.k;
+  const bf16_t* src[R8 + M8];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const int nk = a.k / 32;
-#pragma unroll 2
-  for (int k = wave; k < nk; k += 4) {
-    const bf16x8_t af = as_frag(ld16(A + k * 32));
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = mfma16(as_frag(ld_nt16(W + (int64_t)i * 16 * a.k + k * 32)), af, acc[i]);
-  }
-  if (wave > 0) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<f32x4_t*>(red[wave - 1][i][lane]) = acc[i];
-  }
-  __syncthreads();
-  if (wave > 0 || c >= ns) return;
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int w = 0; w < 3; ++w) acc[i] += *reinterpret_cast<const f32x4_t*>(red[w][i][lane]);
-  bf16_t* o = (bf16_t*)a.C + (int64_t)slot * a.ldc;
-  if constexpr (PAIRS) {
-    const float w = r.slot_w[slot];
-#pragma unroll
-    for (int i = 0; i < 4; i += 2) {
-      float f[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) f[q] = silu_fast(w * acc[i][q]) * (w * acc[i + 1][q]);
-      *reinterpret_cast<uint2*>(o + n0 / 2 + i * 8 + G * 4) = make_uint2(pack_bf(f[0], f[1]), pack_bf(f[2], f[3]));
+  for (int q = 0; q < R8 + M8; ++q) {
+    const int local = (q < R8 ? q : q - R8) * 8 + (lane >> 3), piece = skinny_piece(local, lane);
+    if (q >= R8) {
+      const int slot = s0 + min(local, ns - 1);
+      src[q] = (const bf16_t*)a.A + (int64_t)(GATHER ? r.slot_row[slot] : slot) * a.lda + piece;
+    } else if (PAIRS) {   // eight gate rows, then the eight up rows of the same columns
+      const int col = (n_blk * (R8 / 2) + q / 2) * 8 + (lane >> 3);
+      src[q] = W + (int64_t)min((col >> 4) * 32 + (q & 1) * 16 + (col & 15), a.n - 1) * a.k + piece;
+    } else {
+      src[q] = W + (int64_t)min(n_blk * (R8 * 8) + local, a.n - 1) * a.k + piece;
     }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<uint2*>(o + n0 + i * 16 + G * 4) = make_uint2(pack_bf(acc[i][0], acc[i][1]), pack_bf(acc[i][2], acc[i][3]));
   }
+  skinny_sums<R8, M8>(src, a.k / 64, smem, wave, lane);
+  for (int i = wave; i < (R8 / 2) * MT; i += SKINNY_WAVES) {
+    const int f = i / MT, row = (i - f * MT) * 16 + c;
+    if (row >= ns) continue;
+    bf16_t* o = (bf16_t*)a.C + (int64_t)(s0 + row) * a.ldc;
+    if constexpr (PAIRS) {
+      const int col = (n_blk * (R8 / 2) + f) * 8 + G * 4;
+      if (G >= 2 || col >= a.n / 2) continue;
+      const float w = r.slot_w[s0 + row];
+      const f32x4_t g = skinny_total<R8, M8>(smem, i, lane), u = skinny_total<R8, M8>(smem, i, lane + 32);
+      float v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] = silu_fast(w * g[q]) * (w * u[q]);
+      *reinterpret_cast<uint2*>(o + col) = make_uint2(pack_bf(v[0], v[1]), pack_bf(v[2], v[3]));
+    } else {
+      const int n = n_blk * (R8 * 8) + f * 16 + G * 4;
+      if (n >= a.n) continue;
+      const f32x4_t v = skinny_total<R8, M8>(smem, i, lane);
+      *reinterpret_cast<uint2*>(o + n) = make_uint2(pack_bf(v[0], v[1]), pack_bf(v[2], v[3]));
+    }
+  }
+}
+
+template <int R8, bool GATHER, bool PAIRS>
+__global__ __launch_bounds__(SKINNY_WAVES * 64) void moe_gemm_few_kernel(MoeGemmArgs a, MoeRouting r, int ntn) {
+  static_assert(R8 % 2 == 0, "whole fragments");
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int mt = blockIdx.x / ntn, n_blk = (int)blockIdx.x - mt * ntn;
+  if (mt >= *r.n_tiles) return;
+  const int ex = r.tiles[mt * 3], s0 = r.tiles[mt * 3 + 1], ns = r.tiles[mt * 3 + 2];
+  if (ns <= 8) moe_few_body<R8, 1, GATHER, PAIRS>(a, r, n_blk, ex, s0, ns, smem);
+  else if (ns <= 16) moe_few_body<R8, 2, GATHER, PAIRS>(a, r, n_blk, ex, s0, ns, smem);
+  else moe_few_body<R8, 4, GATHER, PAIRS>(a, r, n_blk, ex, s0, ns, smem);
 }
 
 // ---- 32-bit mode: 64 x 64 tiles on v_mfma_f32_16x16x4_f32 (kernels_layered.hip gemm_f32_kernel with gathered rows) -----------------------------------
@@ -302,7 +315,7 @@ __global__ __launch_bounds__(256) void moe_gemm_f32_kernel(MoeGemmArgs a, MoeRou
 
 int moe_max_tiles(int rows, int top, int experts, int bm) { return (rows * top + bm - 1) / bm + std::min(experts, rows * top); }
 
-int moe_tile_rows(int slots, int experts, bool f32) { return f32 ? 64 : slots <= 24 * experts ? 16 : slots >= 96 * experts ? 2 * TM : TM; }
+int moe_tile_rows(int slots, int experts, bool f32) { return f32 ? 64 : slots <= 24 * experts ? MOE_FEW : slots >= 96 * experts ? 2 * TM : TM; }
 
 void launch_moe_route(const float* z, int64_t ldz, int rows, int experts, int top, int bm, const MoeRouting& r, hipStream_t st) {
   if (rows <= 0) return;
@@ -330,9 +343,16 @@ void launch_moe_gemm(const MoeGemmArgs& a, const MoeRouting& r, int bm, bool f32
   }
   auto go = [&](auto ga, auto pa) {
     constexpr bool GA = decltype(ga)::value, PA = decltype(pa)::value;
-    if (bm == 16) {
-      const int ntn = a.n / 64;
-      hipLaunchKernelGGL((moe_gemm_rows_kernel<GA, PA>), dim3((unsigned)(mt * ntn)), dim3(256), 0, st, a, r, ntn);
+    if (bm == MOE_FEW) {
+      // 48 weight rows per block; 16 where the tiles (at most one per expert while slots are few) would leave CUs without a block
+      auto few = [&](auto r8) {
+        constexpr int R8 = decltype(r8)::value, lds = std::max({skinny_lds(R8, 1), skinny_lds(R8, 2), skinny_lds(R8, 4)});
+        const int ntn = (a.n + R8 * 8 - 1) / (R8 * 8);
+        if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(moe_gemm_few_kernel<R8, GA, PA>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        hipLaunchKernelGGL((moe_gemm_few_kernel<R8, GA, PA>), dim3((unsigned)(mt * ntn)), dim3(SKINNY_WAVES * 64), lds, st, a, r, ntn);
+      };
+      if (std::min(a.experts, a.slots) * ((a.n + 47) / 48) >= 512) few(std::integral_constant<int, 6>{});
+      else few(std::integral_constant<int, 2>{});
     } else {
       const int ntn = (a.n + TN - 1) / TN, parts = bm / TM;
       const unsigned nb = (unsigned)((mt * parts * ntn + 7) / 8 * 8);

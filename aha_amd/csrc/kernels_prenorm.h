@@ -253,7 +253,7 @@ struct MoeGemmArgs {
   int gather;                        // A rows through slot_row
   int pairs;                         // bf16: silu(w g) * (w u) of the 16-column gate / up blocks, C has n / 2 columns; f32: always plain
 };
-int moe_tile_rows(int slots, int experts, bool f32);   // the bm to route with: 16 (few slots per expert), 64, 128 or 256 (many)
+int moe_tile_rows(int slots, int experts, bool f32);   // the bm to route with: 32 (few slots per expert), 64, 128 or 256 (many)
 void launch_moe_gemm(const MoeGemmArgs& a, const MoeRouting& r, int bm, bool f32, hipStream_t st);
 void launch_moe_gemm256(const MoeGemmArgs& a, const MoeRouting& r, int max_tiles, hipStream_t st);   // bf16, tiles of 256 slots (kernels_moe256.hip)
 

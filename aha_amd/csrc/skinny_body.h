@@ -1,0 +1,95 @@
+// Shared device code of the few-row products (kernels_gemm_skinny.hip: dense; kernels_moe.hip: experts with few slots).  A block of four waves owns
+// R8 * 8 weight rows, M8 * 8 activation rows and the whole K range; why and what it measured: kernels_gemm_skinny.hip.
+#pragma once
+#include "common.h"
+
+namespace aha {
+
+namespace {
+
+constexpr int SKINNY_WAVES = 4;
+// three stages hide a request's latency; wide ones have enough in flight with two (and three of them leave one block per CU)
+constexpr int skinny_stages(int r8, int m8) { return r8 + m8 <= 6 ? 3 : 2; }
+constexpr int skinny_lds(int r8, int m8) {
+  const int ring = SKINNY_WAVES * skinny_stages(r8, m8) * (r8 + m8) * 1024 + ((r8 | m8) & 1) * 1024;   // odd: half a fragment is read behind the last stage
+  const int sums = SKINNY_WAVES * ((r8 + 1) / 2) * ((m8 + 1) / 2) * 1024;
+  return ring > sums ? ring : sums;
+}
+
+// 16-byte piece `slot` of row `row` inside a stage's [rows][64] bf16 image
+__device__ __forceinline__ int skinny_swz(int row, int slot) { return row * 128 + ((slot ^ ((row >> 1) & 7)) << 4); }
+// which piece of its row lane `lane` of a request fetches (a request: eight rows, eight lanes each)
+__device__ __forceinline__ int skinny_piece(int local_row, int lane) { return ((lane & 7) ^ ((local_row >> 1) & 7)) * 8; }
+
+// src[r]: where this lane's piece of row group r (R8 weight groups, then M8 activation groups) starts at k = 0.  On return the waves' sums of the
+// 16 x 16 fragments (weight fragment r, activation fragment m) lie in LDS and every wave may read them (skinny_total).
+template <int R8, int M8>
+__device__ __forceinline__ void skinny_sums(const bf16_t* (&src)[R8 + M8], int nc, char* smem, int wave, int lane) {
+  typedef __attribute__((address_space(3))) void* lds_t;
+  typedef const __attribute__((address_space(1))) void* glb_t;
+  constexpr int NF = (R8 + 1) / 2, MT = (M8 + 1) / 2, PER = R8 + M8, S = skinny_stages(R8, M8);
+  constexpr int LEFT = (S - 1) * PER;   // requests of the later stages
+  static_assert(LEFT < 64, "vmcnt has six bits");
+  const int G = lane >> 4, c = lane & 15;
+  char* ring = smem + wave * (S * PER * 1024);
+  f32x4_t acc[NF][MT];
+#pragma unroll
+  for (int r = 0; r < NF; ++r)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[r][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  auto load = [&](int u, int ch) {   // (past the end: the last chunk again, never used)
+    const int k = min(ch, nc - 1) * 64;
+#pragma unroll
+    for (int r = 0; r < R8; ++r) __builtin_amdgcn_global_load_lds((glb_t)(src[r] + k), (lds_t)(ring + (u * PER + r) * 1024), 16, 0, 2);   // weights: non-temporal
+#pragma unroll
+    for (int r = R8; r < PER; ++r) __builtin_amdgcn_global_load_lds((glb_t)(src[r] + k), (lds_t)(ring + (u * PER + r) * 1024), 16, 0, 0);
+  };
+#pragma unroll
+  for (int u = 0; u < S; ++u) load(u, wave + u * SKINNY_WAVES);
+  int u = 0;
+  for (int ch = wave; ch < nc; ch += SKINNY_WAVES) {
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (LEFT & 15) | ((LEFT >> 4) << 14));
+    __builtin_amdgcn_sched_barrier(0);
+    const char *sw = ring + u * PER * 1024, *sa = sw + R8 * 1024;
+    bf16x8_t wf[2][NF], af[2][MT];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int r = 0; r < NF; ++r) wf[h][r] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(sw + skinny_swz(r * 16 + c, h * 4 + G)));
+#pragma unroll
+      for (int m = 0; m < MT; ++m) af[h][m] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(sa + skinny_swz(m * 16 + c, h * 4 + G)));
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int r = 0; r < NF; ++r)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[r][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[h][r], af[h][m], acc[r][m], 0, 0, 0);
+    __builtin_amdgcn_s_waitcnt(0xC07F);   // the stage's fragments are in registers: it may be filled again
+    __builtin_amdgcn_sched_barrier(0);
+    load(u, ch + S * SKINNY_WAVES);
+    u = u + 1 == S ? 0 : u + 1;
+  }
+  __builtin_amdgcn_s_waitcnt(0x0F70);   // no DMA may land in what becomes the sums' space
+  __syncthreads();
+  auto red = reinterpret_cast<f32x4_t(*)[NF * MT][64]>(smem);
+#pragma unroll
+  for (int r = 0; r < NF; ++r)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) red[wave][r * MT + m][lane] = acc[r][m];
+  __syncthreads();
+}
+
+// the four waves' sums of fragment pair i = r * MT + m for lane l: weight rows r * 16 + (l >> 4) * 4 .. + 4, activation row m * 16 + (l & 15)
+template <int R8, int M8>
+__device__ __forceinline__ f32x4_t skinny_total(const char* smem, int i, int l) {
+  auto red = reinterpret_cast<const f32x4_t(*)[((R8 + 1) / 2) * ((M8 + 1) / 2)][64]>(smem);
+  f32x4_t s = red[0][i][l];
+#pragma unroll
+  for (int w = 1; w < SKINNY_WAVES; ++w) s += red[w][i][l];
+  return s;
+}
+
+}  // namespace
+
+}  // namespace aha
