@@ -6,6 +6,8 @@
 // q head h reads kv head h / (heads / kv heads).  Scores, maxima, exponentials and sums are f32; P feeds the MFMA as bf16.
 #include <algorithm>
 
+#include <type_traits>
+
 #include "attn_prefill_body.h"
 
 namespace aha {
@@ -327,66 +329,92 @@ __global__ __launch_bounds__(CD_NT) void attn_chunk_decode_kernel(ChunkDecodeArg
   }
 }
 
-// ---- any dims, token-major pages: one wave per (row, head) ---------------------------------------------------------------------------
-// 64 keys at a time, lane = key for the scores, lanes = value dims for P.V (the probabilities travel through LDS)
-template <typename T>
-__device__ __forceinline__ float ld_act(const T* p);
-template <>
-__device__ __forceinline__ float ld_act<float>(const float* p) { return *p; }
-template <>
-__device__ __forceinline__ float ld_act<bf16_t>(const bf16_t* p) { return bf2f(*p); }
-__device__ __forceinline__ void st_act(float* p, float v) { *p = v; }
-__device__ __forceinline__ void st_act(bf16_t* p, float v) { *p = f2bf(v); }
-
-constexpr int ROWS_MAX_DV = 1024;   // 16 value dims per lane
-template <typename T>
-__global__ __launch_bounds__(64) void attn_chunk_rows_kernel(ChunkAttnArgs a, SeqBatch b) {
-  extern __shared__ __attribute__((aligned(16))) float sh[];   // q (dim), then 64 probabilities
-  const int r = blockIdx.x, head = blockIdx.y, lane = threadIdx.x;
+// ---- any dims, token-major pages: a block per (row, head) ------------------------------------------------------------------------------
+// 64 keys at a time, lane = key for the scores, lanes = value dims for P.V.  What bounds it is the chain load -> score -> softmax -> load -> sum of
+// one page: the four waves take the row's pages in turn and join (max, sum, O) in LDS, a lane's key row comes in 16-byte pieces and the values of
+// eight keys are requested at once.  (One wave per row with scalar loads: 125 us per launch at 2 x 150 positions of 16 heads x 128 in 32 bits;
+// 32 us here.)
+constexpr int ROWS_MAX_DV = 1024, ROWS_NW = 4;
+template <typename T, int NV>   // vdim <= NV * 64
+__global__ __launch_bounds__(ROWS_NW * 64) void attn_chunk_rows_kernel(ChunkAttnArgs a, SeqBatch b) {
+  extern __shared__ __attribute__((aligned(16))) float sh[];   // q (dim, padded to 4), then per wave O (NV * 64), max and sum
+  typedef const __attribute__((address_space(1))) T* gptr_t;
+  typedef T __attribute__((ext_vector_type(4))) t4;
+  typedef const __attribute__((address_space(1))) t4* g4_t;
+  auto widen = [](T v) {
+    if constexpr (std::is_same<T, float>::value) return v;
+    else return bf2f(v);
+  };
+  const int r = blockIdx.x, head = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const SeqEntry e = seq_entry_at(b, b.has_one ? 0 : b.row_entry[r]);
   const int pos = e.pos0 + r - e.row0, lo = a.chunk > 0 ? pos / a.chunk * a.chunk : 0;
-  const int kvhd = head / (a.heads / a.kv.kvh);
-  float* ps = sh + a.dim;
+  const int kvhd = head / (a.heads / a.kv.kvh), dim4 = (a.dim + 3) & ~3;
+  float *os = sh + dim4, *ml = os + ROWS_NW * NV * 64;
   const T* q = (const T*)a.q + ((int64_t)r * a.heads + head) * a.kv.dq;
-  for (int d = lane; d < a.dim; d += 64) sh[d] = ld_act<T>(q + d);
+  for (int d = tid; d < dim4; d += ROWS_NW * 64) sh[d] = d < a.dim ? widen(q[d]) : 0.f;
   __syncthreads();
-  float m = a.sink ? 0.f : -INFINITY, l = a.sink ? 1.f : 0.f, o[ROWS_MAX_DV / 64];
+  const bool vec = ((a.dim | a.kv.dq) & 3) == 0;   // whole aligned groups of four
+  float m = a.sink && wave == 0 ? 0.f : -INFINITY, l = a.sink && wave == 0 ? 1.f : 0.f, o[NV];
 #pragma unroll
-  for (int i = 0; i < ROWS_MAX_DV / 64; ++i) o[i] = 0.f;
-  for (int pg = lo / KV_PAGE_TOKENS; pg <= pos / KV_PAGE_TOKENS; ++pg) {
-    const T* kp = reinterpret_cast<const T*>(a.kv.tab[(int64_t)e.slot * a.kv.ld + pg] + a.kv.layer_off);
-    const T* vp = kp + (int64_t)a.kv.kvh * KV_PAGE_TOKENS * a.kv.dq + (int64_t)kvhd * KV_PAGE_TOKENS * a.kv.dv;
-    const T* kr = kp + ((int64_t)kvhd * KV_PAGE_TOKENS + lane) * a.kv.dq;
+  for (int i = 0; i < NV; ++i) o[i] = 0.f;
+  for (int pg = lo / KV_PAGE_TOKENS + wave; pg <= pos / KV_PAGE_TOKENS; pg += ROWS_NW) {
+    const gptr_t kp = reinterpret_cast<gptr_t>(a.kv.tab[(int64_t)e.slot * a.kv.ld + pg] + a.kv.layer_off);
+    const gptr_t vp = kp + (int64_t)a.kv.kvh * KV_PAGE_TOKENS * a.kv.dq + (int64_t)kvhd * KV_PAGE_TOKENS * a.kv.dv;
+    const gptr_t kr = kp + ((int64_t)kvhd * KV_PAGE_TOKENS + lane) * a.kv.dq;
     const int t = pg * KV_PAGE_TOKENS + lane;
-    float s = -INFINITY;
-    if (t >= lo && t <= pos) {
-      float dot = 0.f;
-      for (int d = 0; d < a.dim; ++d) dot = fmaf(sh[d], ld_act<T>(kr + d), dot);
-      s = dot * a.scale;
+    float dot;
+    if (vec) {
+      f32x4_t d4 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+      for (int d = 0; d < a.dim; d += 4) {
+        const t4 k4 = *reinterpret_cast<g4_t>(kr + d);
+        const f32x4_t q4 = *reinterpret_cast<const f32x4_t*>(sh + d);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d4[i] = fmaf(q4[i], widen(k4[i]), d4[i]);
+      }
+      dot = (d4[0] + d4[1]) + (d4[2] + d4[3]);
+    } else {
+      dot = 0.f;
+      for (int d = 0; d < a.dim; ++d) dot = fmaf(sh[d], widen(kr[d]), dot);
     }
+    const float s = t >= lo && t <= pos ? dot * a.scale : -INFINITY;
     const float m_new = fmaxf(m, wave_max(s));   // (a visited page holds at least one visible key)
-    const float al = expf(m - m_new), p = expf(s - m_new);
+    const float al = m == -INFINITY ? 0.f : expf(m - m_new), p = s == -INFINITY ? 0.f : expf(s - m_new);
     l = l * al + wave_sum(p);
     m = m_new;
-    ps[lane] = p;
-    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NV; ++i) o[i] *= al;
     const int k0 = max(0, lo - pg * KV_PAGE_TOKENS), k1 = min(KV_PAGE_TOKENS - 1, pos - pg * KV_PAGE_TOKENS);
+#pragma unroll 8
+    for (int k = k0; k <= k1; ++k) {
+      const float pk = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(p), k));
 #pragma unroll
-    for (int i = 0; i < ROWS_MAX_DV / 64; ++i) {
-      if (i * 64 >= a.vdim) break;
-      const int d = min(lane + i * 64, a.vdim - 1);   // (surplus lanes repeat the last dim; only the store below is masked)
-      float acc = o[i] * al;
-      for (int k = k0; k <= k1; ++k) acc = fmaf(ps[k], ld_act<T>(vp + (int64_t)k * a.kv.dv + d), acc);
-      o[i] = acc;
+      for (int i = 0; i < NV; ++i) o[i] = fmaf(pk, widen(vp[(int64_t)k * a.kv.dv + min(lane + i * 64, a.vdim - 1)]), o[i]);   // (surplus lanes repeat the last dim)
     }
-    __syncthreads();
   }
-  const float inv = 1.0f / l;
-  T* op = (T*)a.o + (int64_t)r * a.ldo + (int64_t)head * a.dvo;
 #pragma unroll
-  for (int i = 0; i < ROWS_MAX_DV / 64; ++i) {
-    const int d = lane + i * 64;
-    if (d < a.vdim) st_act(op + d, o[i] * inv);
+  for (int i = 0; i < NV; ++i) os[(wave * NV + i) * 64 + lane] = o[i];
+  if (lane == 0) {
+    ml[wave] = m;
+    ml[ROWS_NW + wave] = l;
+  }
+  __syncthreads();
+  float mx = ml[0], f[ROWS_NW], z = 0.f;
+#pragma unroll
+  for (int w = 1; w < ROWS_NW; ++w) mx = fmaxf(mx, ml[w]);
+#pragma unroll
+  for (int w = 0; w < ROWS_NW; ++w) {
+    f[w] = ml[w] == -INFINITY ? 0.f : expf(ml[w] - mx);
+    z = fmaf(ml[ROWS_NW + w], f[w], z);
+  }
+  const float inv = 1.0f / z;
+  T* op = (T*)a.o + (int64_t)r * a.ldo + (int64_t)head * a.dvo;
+  for (int d = tid; d < a.vdim; d += ROWS_NW * 64) {
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < ROWS_NW; ++w) v = fmaf(os[w * NV * 64 + d], f[w], v);
+    if constexpr (std::is_same<T, float>::value) op[d] = v * inv;
+    else op[d] = f2bf(v * inv);
   }
 }
 
@@ -462,10 +490,22 @@ void launch_chunk_attn_decode(const ChunkDecodeArgs& a, const SeqBatch& b, hipSt
 
 void launch_chunk_attn_rows(const ChunkAttnArgs& a, const SeqBatch& b, bool f32, hipStream_t st) {
   if (b.rows <= 0) return;
-  const dim3 grid((unsigned)b.rows, (unsigned)a.heads), block(64);
-  const size_t lds = (size_t)(a.dim + 64) * 4;
-  if (f32) hipLaunchKernelGGL(attn_chunk_rows_kernel<float>, grid, block, lds, st, a, b);
-  else hipLaunchKernelGGL(attn_chunk_rows_kernel<bf16_t>, grid, block, lds, st, a, b);
+  auto go = [&](auto t, auto nv) {
+    using T = decltype(t);
+    constexpr int NV = decltype(nv)::value;
+    const size_t lds = (size_t)(((a.dim + 3) & ~3) + ROWS_NW * NV * 64 + 2 * ROWS_NW) * 4;
+    if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(attn_chunk_rows_kernel<T, NV>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipLaunchKernelGGL((attn_chunk_rows_kernel<T, NV>), dim3((unsigned)b.rows, (unsigned)a.heads), dim3(ROWS_NW * 64), lds, st, a, b);
+  };
+  auto dims = [&](auto t) {
+    using std::integral_constant;
+    if (a.vdim <= 64) go(t, integral_constant<int, 1>{});
+    else if (a.vdim <= 128) go(t, integral_constant<int, 2>{});
+    else if (a.vdim <= 256) go(t, integral_constant<int, 4>{});
+    else go(t, integral_constant<int, ROWS_MAX_DV / 64>{});
+  };
+  if (f32) dims(float{});
+  else dims(bf16_t{});
 }
 
 }  // namespace aha

@@ -61,3 +61,27 @@ def test_argmax_of_many_rows(gpu, n):
     assert (am == lg.argmax(1)).all()
     m.seq_close(s)
     m.close()
+
+
+@pytest.mark.parametrize("rows", [1, 8, 9, 17, 33, 64, 65, 96, 131])
+@pytest.mark.parametrize("dim,vdim,chunk", [(32, 64, 0), (21, 40, 50), (64, 136, 1000), (20, 300, 7)])
+def test_32_bit_mode_by_row_count(gpu, rows, dim, vdim, chunk):
+    """The 32-bit mode's products (few rows by 8 / 16 / 32 / 64, tiles of 32 rows with a short last one) and its attention (pages dealt to four
+    waves, head dims with and without whole groups of four, every width class of the values, chunks that leave waves without a page): a prompt of
+    `rows` tokens and one more token behind it, within the layer-list decoders' bound for 32 bits (2e-5 of the logits' spread)."""
+    from aha_amd.configs_layered import DosovikConfig, LayerConfig
+    from oracle import dosovik as D
+    lay = LayerConfig(heads=4, kv_heads=2, dim=dim, vdim=vdim, chunk=chunk, rope_dims=16, rope_base=1e4, scale=dim ** -0.5, ff=200)
+    cfg = DosovikConfig(hidden_size=200, vocab_size=1000, layers=[lay, lay], embed_scale=14.0, post_norm_alpha=1.3, compute_dtype="float32")
+    w = weights_layered.dosovik_weights(cfg, seed=5)
+    m = HipInferenceModel(cfg, {k: v.to(gpu) for k, v in w.items()})
+    ids = torch.randint(0, 1000, (rows + 1,), generator=torch.Generator().manual_seed(rows)).tolist()
+    js = cfg.to_json()
+    for l in js["layers"]:
+        l["mixer"]["mask"]["size"] = l["mixer"]["mask"]["size"] or 1 << 20
+    ref = D.forward(js, {k: v.double() for k, v in w.items()}, ids).numpy()
+    s = m.seq_open()
+    got = np.concatenate([m.forward_batch([(s, ids[:rows], list(range(rows)))])[0], m.forward_batch([(s, ids[rows:], [0])])[0]])
+    assert np.abs(got - ref).max() < 2e-5 * ref.std() * 4 and np.sqrt(((got - ref) ** 2).mean()) < 2e-5 * ref.std()
+    m.seq_close(s)
+    m.close()
