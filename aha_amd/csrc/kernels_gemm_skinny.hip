@@ -24,17 +24,17 @@ template <int R8, int M8, bool PAIRS>
 __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(GemmArgs a) {
   constexpr int NF = (R8 + 1) / 2, MT = (M8 + 1) / 2, PER = R8 + M8;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), G = lane >> 4, c = lane & 15;
-  const bf16_t* src[PER];
+  const char* src[PER];
 #pragma unroll
   for (int r = 0; r < PER; ++r) {
     const int local = (r < R8 ? r : r - R8) * 8 + (lane >> 3), piece = skinny_piece(local, lane);
     if (r >= R8) {
-      src[r] = (const bf16_t*)a.A + (int64_t)min(local, a.M - 1) * a.lda + piece;
+      src[r] = (const char*)a.A + (int64_t)min(local, a.M - 1) * a.lda * 2 + piece;
     } else if (PAIRS) {   // eight gate rows, then the eight up rows of the same columns (16-row blocks alternate in W)
       const int col = ((int)blockIdx.x * (R8 / 2) + r / 2) * 8 + (lane >> 3);
-      src[r] = (const bf16_t*)a.W + (int64_t)min((col >> 4) * 32 + (r & 1) * 16 + (col & 15), a.N - 1) * a.ldw + piece;
+      src[r] = (const char*)a.W + (int64_t)min((col >> 4) * 32 + (r & 1) * 16 + (col & 15), a.N - 1) * a.ldw * 2 + piece;
     } else {
-      src[r] = (const bf16_t*)a.W + (int64_t)min((int)blockIdx.x * (R8 * 8) + local, a.N - 1) * a.ldw + piece;
+      src[r] = (const char*)a.W + (int64_t)min((int)blockIdx.x * (R8 * 8) + local, a.N - 1) * a.ldw * 2 + piece;
     }
   }
   skinny_sums<R8, M8>(src, a.K / 64, gemm_smem, wave, lane);

@@ -5,7 +5,6 @@
 //   rope_pairs_kernel      (cos, sin) of a step's angles, once for all layers of the same rotation
 //   qkv_post_kernel        q / k norm over the whole projection, rotation, value mixing, KV append
 //   polynorm_rows_kernel   a N(z) + b N(z^2) + c N(z^3) + e
-//   gemm_f32_kernel        the 32-bit mode's matrix product (f32 MFMA)
 #include <math.h>
 
 #include <algorithm>
@@ -593,52 +592,6 @@ __global__ __launch_bounds__(NTH) void polynorm_rows_kernel(PolyNormArgs a) {
   }
 }
 
-// 64 x 64 tile, four waves of 16 x 64 on v_mfma_f32_16x16x4_f32 (lane l: row / column l & 15, k = l >> 4)
-constexpr int FBK = 32, FPITCH = FBK + 1;
-// (blockIdx.z: one of a batch of products, its operands sa / sw / sc elements behind the first's)
-__global__ __launch_bounds__(NT) void gemm_f32_kernel(const float* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int64_t ldw,
-                                                      float* __restrict__ C, int64_t ldc, int M, int N, int K, int64_t sa, int64_t sw, int64_t sc) {
-  A += blockIdx.z * sa;
-  W += blockIdx.z * sw;
-  C += blockIdx.z * sc;
-  __shared__ float as[64 * FPITCH], ws[64 * FPITCH];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, G = lane >> 4;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  f32x4_t acc[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < K; k0 += FBK) {
-#pragma unroll
-    for (int i = 0; i < 64 * FBK / 4 / NT; ++i) {
-      const int p = tid + i * NT, row = p >> 3, kk = (p & 7) * 4;
-      float4 v = make_float4(0.f, 0.f, 0.f, 0.f), w = v;
-      if (m0 + row < M) v = *reinterpret_cast<const float4*>(A + (int64_t)(m0 + row) * lda + k0 + kk);
-      if (n0 + row < N) w = wbf4(W, (int64_t)(n0 + row) * ldw + k0 + kk);
-      float *da = as + row * FPITCH + kk, *dw = ws + row * FPITCH + kk;
-      da[0] = v.x; da[1] = v.y; da[2] = v.z; da[3] = v.w;
-      dw[0] = w.x; dw[1] = w.y; dw[2] = w.z; dw[3] = w.w;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < FBK; k += 4) {
-      const float av = as[(wave * 16 + c) * FPITCH + k + G];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, ws[(j * 16 + c) * FPITCH + k + G], acc[j], 0, 0, 0);
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int n = n0 + j * 16 + c;
-    if (n >= N) continue;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = m0 + wave * 16 + G * 4 + r;
-      if (m < M) C[(int64_t)m * ldc + n] = acc[j][r];
-    }
-  }
-}
-
 template <typename T, bool EMBED>
 void postnorm_conv_t(const PostNormArgs& a, const SeqBatch& b, hipStream_t st) {
   // rows per block: a tile repeats the norm of its taps - 1 preceding rows, a short grid leaves CUs idle
@@ -728,13 +681,6 @@ void launch_polynorm_rows(const PolyNormArgs& a, bool f32, hipStream_t st) {
   else if (a.ld <= 12288) go(polynorm_rows_kernel<bf16_t, 512, 6>, 512);
   else if (a.ld <= 16384) go(polynorm_rows_kernel<bf16_t, 512, 8>, 512);
   else go(polynorm_rows_kernel<bf16_t, 512, 0>, 512);
-}
-
-void launch_gemm_f32(const float* A, int64_t lda, const void* W, int64_t ldw, float* C, int64_t ldc, int M, int N, int K, hipStream_t st, int batch,
-                     int64_t sa, int64_t sw, int64_t sc) {
-  if (M <= 0 || N <= 0 || batch <= 0) return;
-  hipLaunchKernelGGL(gemm_f32_kernel, dim3((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64), (unsigned)batch), dim3(NT), 0, st, A, lda, (const bf16_t*)W,
-                     ldw, C, ldc, M, N, K, sa, sw, sc);
 }
 
 }  // namespace aha

@@ -218,19 +218,19 @@ template <int R8, int M8, bool GATHER, bool PAIRS>
 __device__ __forceinline__ void moe_few_body(const MoeGemmArgs& a, const MoeRouting& r, int n_blk, int ex, int s0, int ns, char* smem) {
   constexpr int MT = (M8 + 1) / 2;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), G = lane >> 4, c = lane & 15;
-  const bf16_t* W = (const bf16_t*)a.W + (int64_t)ex * a.n * a.k;
-  const bf16_t* src[R8 + M8];
+  const char* W = (const char*)((const bf16_t*)a.W + (int64_t)ex * a.n * a.k);
+  const char* src[R8 + M8];
 #pragma unroll
   for (int q = 0; q < R8 + M8; ++q) {
     const int local = (q < R8 ? q : q - R8) * 8 + (lane >> 3), piece = skinny_piece(local, lane);
     if (q >= R8) {
       const int slot = s0 + min(local, ns - 1);
-      src[q] = (const bf16_t*)a.A + (int64_t)(GATHER ? r.slot_row[slot] : slot) * a.lda + piece;
+      src[q] = (const char*)a.A + (int64_t)(GATHER ? r.slot_row[slot] : slot) * a.lda * 2 + piece;
     } else if (PAIRS) {   // eight gate rows, then the eight up rows of the same columns
       const int col = (n_blk * (R8 / 2) + q / 2) * 8 + (lane >> 3);
-      src[q] = W + (int64_t)min((col >> 4) * 32 + (q & 1) * 16 + (col & 15), a.n - 1) * a.k + piece;
+      src[q] = W + (int64_t)min((col >> 4) * 32 + (q & 1) * 16 + (col & 15), a.n - 1) * a.k * 2 + piece;
     } else {
-      src[q] = W + (int64_t)min(n_blk * (R8 * 8) + local, a.n - 1) * a.k + piece;
+      src[q] = W + (int64_t)min(n_blk * (R8 * 8) + local, a.n - 1) * a.k * 2 + piece;
     }
   }
   skinny_sums<R8, M8>(src, a.k / 64, smem, wave, lane);

@@ -9,25 +9,30 @@ namespace {
 
 constexpr int SKINNY_WAVES = 4;
 // three stages hide a request's latency; wide ones have enough in flight with two (and three of them leave one block per CU)
-constexpr int skinny_stages(int r8, int m8) { return r8 + m8 <= 6 ? 3 : 2; }
-constexpr int skinny_lds(int r8, int m8) {
-  const int ring = SKINNY_WAVES * skinny_stages(r8, m8) * (r8 + m8) * 1024 + ((r8 | m8) & 1) * 1024;   // odd: half a fragment is read behind the last stage
+constexpr int skinny_stages(int requests) { return requests <= 6 ? 3 : 2; }
+constexpr int skinny_requests(int r8, int m8, bool f32) { return r8 + (f32 ? 2 : 1) * m8; }
+constexpr int skinny_lds(int r8, int m8, bool f32 = false) {
+  const int per = skinny_requests(r8, m8, f32);
+  const int ring = SKINNY_WAVES * skinny_stages(per) * per * 1024 + ((r8 | m8) & 1) * 1024;   // odd: half a fragment is read behind the last stage
   const int sums = SKINNY_WAVES * ((r8 + 1) / 2) * ((m8 + 1) / 2) * 1024;
   return ring > sums ? ring : sums;
 }
 
 // 16-byte piece `slot` of row `row` inside a stage's [rows][64] bf16 image
 __device__ __forceinline__ int skinny_swz(int row, int slot) { return row * 128 + ((slot ^ ((row >> 1) & 7)) << 4); }
-// which piece of its row lane `lane` of a request fetches (a request: eight rows, eight lanes each)
-__device__ __forceinline__ int skinny_piece(int local_row, int lane) { return ((lane & 7) ^ ((local_row >> 1) & 7)) * 8; }
+// the byte offset inside its 128-byte line that lane `lane` of a request fetches (a request: eight rows, eight lanes each)
+__device__ __forceinline__ int skinny_piece(int local_row, int lane) { return ((lane & 7) ^ ((local_row >> 1) & 7)) * 16; }
 
-// src[r]: where this lane's piece of row group r (R8 weight groups, then M8 activation groups) starts at k = 0.  On return the waves' sums of the
-// 16 x 16 fragments (weight fragment r, activation fragment m) lie in LDS and every wave may read them (skinny_total).
-template <int R8, int M8>
-__device__ __forceinline__ void skinny_sums(const bf16_t* (&src)[R8 + M8], int nc, char* smem, int wave, int lane) {
+// src[r]: where this lane's piece of request r starts at k = 0 -- R8 weight groups (bf16), then M8 activation groups (bf16); F32: activations are f32,
+// a row's 64 k are two requests, the first halves of all groups before the second halves.  The 32-bit form multiplies on
+// v_mfma_f32_16x16x4_f32 (weights widened exactly): in step (h, j) lane group G feeds k = (h * 4 + G) * 8 + j of both operands.
+// On return the waves' sums of the 16 x 16 fragments (weight fragment r, activation fragment m) lie in LDS and every wave may read them
+// (skinny_total).
+template <int R8, int M8, bool F32 = false>
+__device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R8, M8, F32)], int nc, char* smem, int wave, int lane) {
   typedef __attribute__((address_space(3))) void* lds_t;
   typedef const __attribute__((address_space(1))) void* glb_t;
-  constexpr int NF = (R8 + 1) / 2, MT = (M8 + 1) / 2, PER = R8 + M8, S = skinny_stages(R8, M8);
+  constexpr int NF = (R8 + 1) / 2, MT = (M8 + 1) / 2, PER = skinny_requests(R8, M8, F32), S = skinny_stages(PER);
   constexpr int LEFT = (S - 1) * PER;   // requests of the later stages
   static_assert(LEFT < 64, "vmcnt has six bits");
   const int G = lane >> 4, c = lane & 15;
@@ -38,11 +43,11 @@ __device__ __forceinline__ void skinny_sums(const bf16_t* (&src)[R8 + M8], int n
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[r][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   auto load = [&](int u, int ch) {   // (past the end: the last chunk again, never used)
-    const int k = min(ch, nc - 1) * 64;
+    const int k = min(ch, nc - 1) * 128, ka = F32 ? 2 * k : k;
 #pragma unroll
     for (int r = 0; r < R8; ++r) __builtin_amdgcn_global_load_lds((glb_t)(src[r] + k), (lds_t)(ring + (u * PER + r) * 1024), 16, 0, 2);   // weights: non-temporal
 #pragma unroll
-    for (int r = R8; r < PER; ++r) __builtin_amdgcn_global_load_lds((glb_t)(src[r] + k), (lds_t)(ring + (u * PER + r) * 1024), 16, 0, 0);
+    for (int r = R8; r < PER; ++r) __builtin_amdgcn_global_load_lds((glb_t)(src[r] + ka), (lds_t)(ring + (u * PER + r) * 1024), 16, 0, 0);
   };
 #pragma unroll
   for (int u = 0; u < S; ++u) load(u, wave + u * SKINNY_WAVES);
@@ -51,20 +56,42 @@ __device__ __forceinline__ void skinny_sums(const bf16_t* (&src)[R8 + M8], int n
     __builtin_amdgcn_s_waitcnt(0x0F70 | (LEFT & 15) | ((LEFT >> 4) << 14));
     __builtin_amdgcn_sched_barrier(0);
     const char *sw = ring + u * PER * 1024, *sa = sw + R8 * 1024;
-    bf16x8_t wf[2][NF], af[2][MT];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-#pragma unroll
-      for (int r = 0; r < NF; ++r) wf[h][r] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(sw + skinny_swz(r * 16 + c, h * 4 + G)));
-#pragma unroll
-      for (int m = 0; m < MT; ++m) af[h][m] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(sa + skinny_swz(m * 16 + c, h * 4 + G)));
-    }
+    u32x4_t wf[2][NF];
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int r = 0; r < NF; ++r)
+      for (int r = 0; r < NF; ++r) wf[h][r] = *reinterpret_cast<const u32x4_t*>(sw + skinny_swz(r * 16 + c, h * 4 + G));
+    if constexpr (F32) {
+      f32x4_t af[2][MT][2];
 #pragma unroll
-        for (int m = 0; m < MT; ++m) acc[r][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[h][r], af[h][m], acc[r][m], 0, 0, 0);
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int q = 0; q < 2; ++q) af[h][m][q] = *reinterpret_cast<const f32x4_t*>(sa + h * (M8 * 1024) + skinny_swz(m * 16 + c, 2 * G + q));
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+#pragma unroll
+          for (int r = 0; r < NF; ++r) {
+            const float w = j & 1 ? hi_bf(wf[h][r][j >> 1]) : lo_bf(wf[h][r][j >> 1]);
+#pragma unroll
+            for (int m = 0; m < MT; ++m) acc[r][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, af[h][m][j >> 2][j & 3], acc[r][m], 0, 0, 0);
+          }
+    } else {
+      bf16x8_t af[2][MT];
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) af[h][m] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(sa + skinny_swz(m * 16 + c, h * 4 + G)));
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int r = 0; r < NF; ++r)
+#pragma unroll
+          for (int m = 0; m < MT; ++m) acc[r][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[h][r]), af[h][m], acc[r][m], 0, 0, 0);
+    }
     __builtin_amdgcn_s_waitcnt(0xC07F);   // the stage's fragments are in registers: it may be filled again
     __builtin_amdgcn_sched_barrier(0);
     load(u, ch + S * SKINNY_WAVES);
