@@ -201,6 +201,7 @@ struct GemmArgs {
   void* sk_counters = nullptr;   // optional SK_MAX_COUNTERS zeroed u32 words that belong to `workspace` (one per tile cut along K by the
                                  // persistent kernel, kernels_gemm_sk.hip; every launch leaves them zero again)
   int tile_group = 8;            // band width of the grouped tile order inside an XCD's run (kernels_gemm.hip tile_of_block); 0 = plain
+  int few_rows = 1;              // 0: not the few-row kernel (kernels_gemm_skinny.hip) whatever M is
   int partial_rows = 1;          // ACT_PARTIAL_F32 on the four-wave kernel: f32 sums stored in row order through LDS (0: fragment order; A/B)
   // Row groups (launch_gemm_grouped; tensor-parallel prefill: the staging layout of the chunked all-gather, csrc/model.hip
   // norm_gather_gemm): `groups` row segments of M rows each share W.  Segment g reads A rows [g * a_gstride, + M) and writes C rows

@@ -101,8 +101,14 @@ double gemm_skinny_plan(const GemmArgs& a, int* r8_out) {
   return best;
 }
 
+// K < 768 stays with the tiled kernels: they run unsplit there, so a row's bits do not depend on how many rows share the call (row slices of a
+// sequence-parallel prompt), for 1.5 to 4 us more per launch (K = 256: 5.1 against 2.7 us, 512: 6.8 against 3.0, 768: 8.5 against 3.3; 8 rows, 2048
+// columns).  So do 33 to 64 rows of a matrix below 2 MB (512 x 1024: 10.2 against 5.2 us).  Only small models have either -- the full-size ones have
+// K >= 768 throughout their text stacks, and their one small matrix, the router, is met by 33 to 64 rows only in that band -- and they keep the
+// results they had.
 bool gemm_skinny_ok(const GemmArgs& a) {
-  return a.M >= 1 && a.M <= 64 && a.K >= 64 && a.K % 64 == 0 && a.N % 8 == 0 && a.groups == 1 && (a.act != ACT_SILU_MUL_PAIRS || a.N % 32 == 0);
+  return a.few_rows && a.M >= 1 && a.M <= 64 && a.K >= 768 && a.K % 64 == 0 && a.N % 8 == 0 && a.groups == 1 && (a.act != ACT_SILU_MUL_PAIRS || a.N % 32 == 0) &&
+         (a.M <= 32 || (int64_t)a.N * a.K >= 1 << 20);
 }
 
 void launch_gemm_skinny(const GemmArgs& a, hipStream_t st) {

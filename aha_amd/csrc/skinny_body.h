@@ -37,11 +37,13 @@ __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R
   static_assert(LEFT < 64, "vmcnt has six bits");
   const int G = lane >> 4, c = lane & 15;
   char* ring = smem + wave * (S * PER * 1024);
-  f32x4_t acc[NF][MT];
+  f32x4_t acc[2][NF][MT];   // the two halves of a chunk in chains of their own: half the dependent steps, half the roundings in a row
 #pragma unroll
-  for (int r = 0; r < NF; ++r)
+  for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int m = 0; m < MT; ++m) acc[r][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int r = 0; r < NF; ++r)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) acc[h][r][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   auto load = [&](int u, int ch) {   // (past the end: the last chunk again, never used)
     const int k = min(ch, nc - 1) * 128, ka = F32 ? 2 * k : k;
 #pragma unroll
@@ -77,7 +79,7 @@ __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R
           for (int r = 0; r < NF; ++r) {
             const float w = j & 1 ? hi_bf(wf[h][r][j >> 1]) : lo_bf(wf[h][r][j >> 1]);
 #pragma unroll
-            for (int m = 0; m < MT; ++m) acc[r][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, af[h][m][j >> 2][j & 3], acc[r][m], 0, 0, 0);
+            for (int m = 0; m < MT; ++m) acc[h][r][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, af[h][m][j >> 2][j & 3], acc[h][r][m], 0, 0, 0);
           }
     } else {
       bf16x8_t af[2][MT];
@@ -90,7 +92,7 @@ __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R
 #pragma unroll
         for (int r = 0; r < NF; ++r)
 #pragma unroll
-          for (int m = 0; m < MT; ++m) acc[r][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[h][r]), af[h][m], acc[r][m], 0, 0, 0);
+          for (int m = 0; m < MT; ++m) acc[h][r][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[h][r]), af[h][m], acc[h][r][m], 0, 0, 0);
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);   // the stage's fragments are in registers: it may be filled again
     __builtin_amdgcn_sched_barrier(0);
@@ -103,7 +105,7 @@ __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R
 #pragma unroll
   for (int r = 0; r < NF; ++r)
 #pragma unroll
-    for (int m = 0; m < MT; ++m) red[wave][r * MT + m][lane] = acc[r][m];
+    for (int m = 0; m < MT; ++m) red[wave][r * MT + m][lane] = acc[0][r][m] + acc[1][r][m];
   __syncthreads();
 }
 
@@ -111,10 +113,8 @@ __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R
 template <int R8, int M8>
 __device__ __forceinline__ f32x4_t skinny_total(const char* smem, int i, int l) {
   auto red = reinterpret_cast<const f32x4_t(*)[((R8 + 1) / 2) * ((M8 + 1) / 2)][64]>(smem);
-  f32x4_t s = red[0][i][l];
-#pragma unroll
-  for (int w = 1; w < SKINNY_WAVES; ++w) s += red[w][i][l];
-  return s;
+  static_assert(SKINNY_WAVES == 4, "joined in pairs");
+  return (red[0][i][l] + red[1][i][l]) + (red[2][i][l] + red[3][i][l]);
 }
 
 }  // namespace

@@ -10,11 +10,11 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32, 33, 64])
 @pytest.mark.parametrize("N,K", [
-    (8, 64),         # one eight-row group, one k chunk for four waves
-    (1000, 192),     # N ends inside a block of 16, 24, 32 and 48 rows; fewer chunks than waves
-    (6144, 320),     # 24 rows per block: half a fragment unused
-    (12320, 448),    # 48 rows per block, the last block short
-    (40, 4160),      # more chunks than ring stages, an uneven share per wave
+    (8, 768),        # one eight-row group, as many k chunks per wave as ring stages
+    (1264, 832),     # N ends inside a block of 16, 24, 32 and 48 rows; an uneven share of chunks per wave
+    (6144, 768),     # 24 rows per block: half a fragment unused
+    (12320, 832),    # 48 rows per block, the last block short
+    (40, 4160),      # many chunks
 ])
 def test_few_rows_every_row_count_and_block_width(gpu, M, N, K):
     """One f32 sum per element, rounded once per op as in the tiled kernels: a sum next to a rounding boundary moves one op's result by one ulp, so
@@ -36,7 +36,7 @@ def test_few_rows_every_row_count_and_block_width(gpu, M, N, K):
 
 
 @pytest.mark.parametrize("M", [1, 8, 13, 31, 64])
-@pytest.mark.parametrize("I,K", [(16, 64), (1008, 256), (3072, 1024), (12288, 128)])
+@pytest.mark.parametrize("I,K", [(16, 768), (1008, 832), (3072, 1024), (12288, 768)])
 def test_few_rows_gate_up_pairs(gpu, M, I, K):
     """Gate and up rows in groups of eight per block, the product in the epilogue (interleaved layout of the model loader)."""
     from aha_amd import ops, _lib
