@@ -24,20 +24,25 @@ constexpr int ATTN_DECODE_FUSED_LDS = 16 * 128 * 2 + 128 * 2 + 128 * 2 + ATTN_DE
 //   * in the page loop K and V of a page are separate register buffers re-requested as soon as their MFMAs have
 //     consumed them (K(next) right after QK^T, V(next) right after P.V), so a wave always has 16-32 KB in flight.
 // smem: ATTN_DECODE_FUSED_LDS bytes, 16-byte aligned.  Returns true in the one block per kv head that wrote the output.
+//
+// DEFER: the blocks leave their partials to the o_proj matvec, whose prologue merges up to eight of them (kernels_gemv_fused.hip MergePro): the kernel
+// boundary orders the plain stores, and the publish -> acknowledge -> arrive -> re-read chain of the last-block merge (1.9 + 0.7 + 2.3 of 9.7 us at
+// 1536 positions) is gone.
+template <int NW, bool DEFER>
 __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs& a, char* smem, const int kvhd, const int split,
                                                        const int nsplit) {
-  constexpr int NW = ATTN_DECODE_NW, NT = NW * 64;
+  constexpr int NT = NW * 64;
   bf16_t* qs = reinterpret_cast<bf16_t*>(smem);                 // [16][128]
   bf16_t* ksn = qs + 16 * 128;                                  // [128]
   bf16_t* vsn = ksn + 128;                                      // [128]
-  float* mo = reinterpret_cast<float*>(vsn + 128);              // per wave O^T [NW][d 128][q 16]
-  float* mm = mo + NW * 128 * 16;                               // [NW][16]
+  const int g = a.nh / a.kvh, P = DEFER ? g : 16;               // P: q slots kept per dim
+  float* mo = reinterpret_cast<float*>(vsn + 128);              // per wave O^T [NW][d 128][q P]
+  float* mm = mo + NW * 128 * P;                                // [NW][16]
   float* mlz = mm + NW * 16;                                    // [NW][16]
   const int tid = (int)threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, G = lane >> 4, c = lane & 15;
-  const int g = a.nh / a.kvh;
-  const int nunits = nsplit * NW, unit = split * NW + wave;
+  const int nunits = nsplit * NW, unit = DEFER ? wave * nsplit + split : split * NW + wave;   // (DEFER: neighbouring pages to different blocks)
   const int L = a.kv_len_v, slot_new = a.kv_start_v;
   const int L_old = L - 1;  // tokens already in the pages; the new one is handled from LDS
   const int npages = (L_old + KV_PAGE_TOKENS - 1) / KV_PAGE_TOKENS;
@@ -218,13 +223,15 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
   }
   l = group_sum(l);
 
-  // ---- merge the 4 waves through LDS, leave one partial per (split, head) ---------------------------------------------
+  // ---- merge the waves through LDS, leave one partial per (split, head) ---------------------------------------------
   {
-    float* wo = mo + wave * (128 * 16);
+    float* wo = mo + wave * (128 * P);
+    if (!DEFER || c < g) {
 #pragma unroll
-    for (int ds = 0; ds < 8; ++ds)
+      for (int ds = 0; ds < 8; ++ds)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) wo[(ds * 16 + G * 4 + r) * 16 + c] = o[ds][r];
+        for (int r = 0; r < 4; ++r) wo[(ds * 16 + G * 4 + r) * P + c] = o[ds][r];
+    }
     if (G == 0) {
       mm[wave * 16 + c] = m;
       mlz[wave * 16 + c] = l;
@@ -246,7 +253,7 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
       const float mw = mm[w * 16 + q];
       const float wt = (mw == -INFINITY) ? 0.f : __expf(mw - M);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc[e] = fmaf(wt, mo[w * (128 * 16) + (d0 + e) * 16 + q], acc[e]);
+      for (int e = 0; e < 4; ++e) acc[e] = fmaf(wt, mo[w * (128 * P) + (d0 + e) * P + q], acc[e]);
       ls = fmaf(wt, mlz[w * 16 + q], ls);
     }
     const int head = kvhd * g + q;
@@ -256,6 +263,9 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
       w2.x = pack_bf(acc[0] * inv, acc[1] * inv);
       w2.y = pack_bf(acc[2] * inv, acc[3] * inv);
       *reinterpret_cast<uint2*>((bf16_t*)a.o + head * 128 + d0) = w2;
+    } else if constexpr (DEFER) {
+      *reinterpret_cast<float4*>(a.part_o + ((int64_t)split * a.nh + head) * 128 + d0) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+      if (d0 == 0) *reinterpret_cast<float2*>(a.part_ml + ((int64_t)split * a.nh + head) * 2) = make_float2(M, ls);
     } else {
       const u32x4_t v = {__float_as_uint(acc[0]), __float_as_uint(acc[1]), __float_as_uint(acc[2]), __float_as_uint(acc[3])};
       __builtin_amdgcn_raw_buffer_store_b128(v, rsrc_w, (uint32_t)(((size_t)split * a.nh + head) * 128 + d0) * 4, 0, 16 /* sc1 */);
@@ -266,9 +276,9 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
       }
     }
   }
-  if (single) {
+  if (single || DEFER) {
     stamp(5);
-    return true;
+    return single;
   }
   stamp(3);
 

@@ -41,6 +41,14 @@ struct GemvArgs {
   float softcap = 0.f;      // GEMV_LOGITS: > 0: logits are softcap * tanh(logits / softcap)
 };
 void launch_gemv(const GemvArgs& a, GemvEpi epi, hipStream_t st);
+// y = residual + W . bf16(merge of nsplit attention partials (up to 8; 4 where K > 2048)): part_o (nsplit, heads, 128), part_ml (nsplit, heads, 2 = max, sum);
+// K = heads * 128 <= 4096, epilogue GEMV_RESIDUAL (kernels_gemv_fused.hip)
+struct GemvMerge {
+  const float* part_o;
+  const float* part_ml;
+  int nsplit, heads;
+};
+void launch_gemv_merge(const GemvArgs& a, const GemvMerge& p, hipStream_t st);
 struct GemvPlan { int R, U, grid; };   // rows per wave, 512-column chunks per load group, persistent blocks
 GemvPlan plan_gemv(int N, int K, GemvEpi epi);
 int gemv_num_tiles(int N, int K);  // number of (max,idx) partials GEMV_LOGITS writes
@@ -130,6 +138,9 @@ struct AttnDecodeFusedArgs {
   float eps, scale;
 };
 void launch_attn_decode_fused(const AttnDecodeFusedArgs& a, hipStream_t st);
+// The same with the partials left for launch_gemv_merge (nsplit > 1; a single split writes `o`): nsplit from attn_decode_defer_splits, 0 = not here
+int attn_decode_defer_splits(int npages, int nq);
+void launch_attn_decode_defer(const AttnDecodeFusedArgs& a, hipStream_t st);
 
 struct AttnPrefillArgs {
   const void* q;           // (S, nh*d) bf16

@@ -16,6 +16,8 @@
 //                         B = P^T (col = q c,    k = the two S^T fragments of token sub-tiles 2kk, 2kk+1, in registers)
 //                         C[reg] = O[q c][dim G*4+reg]
 // so no operand ever needs a transpose or a cross-lane shuffle; page layout and the V slot permutation: common.h.
+#include <algorithm>
+
 #include <stdio.h>
 #include <stdlib.h>
 
@@ -150,13 +152,32 @@ __global__ __launch_bounds__(128) void attn_decode_combine_kernel(AttnDecodeArgs
 
 __global__ __launch_bounds__(256, 2) void attn_decode_fused_kernel(AttnDecodeFusedArgs a) {
   __shared__ __attribute__((aligned(16))) char smem[ATTN_DECODE_FUSED_LDS];
-  attn_decode_fused_body(a, smem, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.y);
+  attn_decode_fused_body<ATTN_DECODE_NW, false>(a, smem, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.y);
+}
+__global__ __launch_bounds__(256, 2) void attn_decode_defer_kernel(AttnDecodeFusedArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem_defer[];
+  attn_decode_fused_body<ATTN_DECODE_NW, true>(a, smem_defer, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.y);
 }
 
 }  // namespace
 
 void launch_attn_decode_fused(const AttnDecodeFusedArgs& a, hipStream_t st) {
   hipLaunchKernelGGL(attn_decode_fused_kernel, dim3(a.kvh, a.nsplit), dim3(256), 0, st, a);
+}
+
+// How many partials (0: the merge belongs inside the launch).  A CU streams ~56 bytes per ns here, half a microsecond per page of a kv head, so two
+// pages per block while the partials last; every partial costs the o_proj matvec another 4 bytes per column and block from L2 (0.6B widths: +0.2 us
+// for 4, +0.6 us for 8; 8B widths: +2.1 us for 4, so nothing is split there before a block has more than four pages).
+// At six pages per block the launch that merges by itself is as fast.
+int attn_decode_defer_splits(int npages, int nq) {
+  if (nq > 4096) return 0;   // (the prologue holds the partials of 4096 columns in registers)
+  const int most = nq <= 2048 ? 8 : 4;
+  if (npages > 6 * most) return 0;
+  return nq > 2048 && npages <= 4 ? 1 : std::min((npages + 1) / 2, most);
+}
+void launch_attn_decode_defer(const AttnDecodeFusedArgs& a, hipStream_t st) {
+  const int lds = 16 * 128 * 2 + 2 * 128 * 2 + ATTN_DECODE_NW * 128 * (a.nh / a.kvh) * 4 + 2 * ATTN_DECODE_NW * 16 * 4;
+  hipLaunchKernelGGL(attn_decode_defer_kernel, dim3(a.kvh, a.nsplit), dim3(256), lds, st, a);
 }
 
 static int g_attn_smx_override = -1;

@@ -3,6 +3,7 @@
 //       every block rebuilds h (the matvec's input) in LDS; what the convolution takes from earlier tokens arrives as ONE vector, the
 //       weighted sum prepared when those tokens ran (ConvIn::hist).  Block j < XP also writes column group j of x and, behind its weight
 //       stream, of the sequence's new history and the next token's weighted sum.
+//   attention merge:               h = the split-KV attention partials of a decode step joined (attn_decode_body.h, DEFER)
 //   PolyNorm:                      h = a N(z) + b N(z^2) + c N(z^3) + e: the three row sums in the prologue
 #include "gemv_prologues.h"
 
@@ -114,6 +115,58 @@ struct PolyNormPro {
   __device__ __forceinline__ void finish(int, int) {}
 };
 
+// Every block joins all heads: nsplit x 16 KB (32 heads) from L2, requested ahead of the first weight tile -- under a microsecond of it shows.  A wave's
+// group j of 256 columns is two heads; weights and normalisation per head are recomputed by its 32 threads.
+template <int XP, int MS>
+struct MergePro {
+  GemvMerge p;
+  int K;
+  float4 v[XP][MS];
+  float2 ml[XP][MS];
+  __device__ __forceinline__ void request(int tid) {
+#pragma unroll
+    for (int j = 0; j < XP; ++j) {
+      const int k = min((tid + j * GEMV_THREADS) * 4, K - 4), head = k >> 7;
+#pragma unroll
+      for (int s = 0; s < MS; ++s) {
+        const int64_t at = (int64_t)min(s, p.nsplit - 1) * p.heads;
+        ml[j][s] = *reinterpret_cast<const float2*>(p.part_ml + (at + head) * 2);
+        v[j][s] = *reinterpret_cast<const float4*>(p.part_o + at * 128 + k);
+      }
+    }
+  }
+  __device__ __forceinline__ void stage(float* xs, float*, int tid, int, int nchunks) {
+#pragma unroll
+    for (int j = 0; j < XP; ++j) {
+      const int k = (tid + j * GEMV_THREADS) * 4;
+      if (k >= (nchunks << 9)) continue;
+      float M = ml[j][0].x;
+#pragma unroll
+      for (int s = 1; s < MS; ++s) M = fmaxf(M, ml[j][s].x);   // (surplus slots repeat the last split)
+      float4 h = make_float4(0.f, 0.f, 0.f, 0.f);
+      float z = 0.f;
+#pragma unroll
+      for (int s = 0; s < MS; ++s) {
+        const float w = s < p.nsplit && ml[j][s].x != -INFINITY ? __expf(ml[j][s].x - M) : 0.f;
+        z = fmaf(w, ml[j][s].y, z);
+        h.x = fmaf(w, v[j][s].x, h.x); h.y = fmaf(w, v[j][s].y, h.y); h.z = fmaf(w, v[j][s].z, h.z); h.w = fmaf(w, v[j][s].w, h.w);
+      }
+      const float inv = 1.0f / z;
+      // the attention output tensor is bf16
+      *xs4(xs, k) = k < K ? make_float4(rbf(h.x * inv), rbf(h.y * inv), rbf(h.z * inv), rbf(h.w * inv)) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  }
+  __device__ __forceinline__ void finish(int, int) {}
+};
+
+template <int R, int U, bool FAST, int XP, int MS>
+__global__ __launch_bounds__(GEMV_THREADS) void gemv_merge_kernel(GemvArgs a, GemvMerge p) {
+  extern __shared__ __attribute__((aligned(16))) float xs[];
+  MergePro<XP, MS> pro;
+  pro.p = p;
+  pro.K = a.K;
+  gemv_body<R, U, GEMV_RESIDUAL, false, FAST>(a, xs, (int)blockIdx.x, (int)gridDim.x, [] {}, pro);
+}
 template <int R, int U, int EPI, bool FAST, int XP>
 __global__ __launch_bounds__(GEMV_THREADS) void gemv_postnorm_kernel(GemvArgs a, GemvPostNorm p) {
   extern __shared__ __attribute__((aligned(16))) float xs[];
@@ -155,6 +208,31 @@ void launch_gemv_postnorm(const GemvArgs& a, const GemvPostNorm& p, GemvEpi epi,
     else if (a.K <= 4096) run(std::integral_constant<int, 4>{});
     else run(std::integral_constant<int, 8>{});
   });
+}
+
+void launch_gemv_merge(const GemvArgs& a, const GemvMerge& p, hipStream_t st) {
+  const GemvPlan pl = plan_gemv(a.N, a.K, GEMV_RESIDUAL);
+  auto go = [&](auto r, auto u) {
+    constexpr int R = decltype(r)::value, U = decltype(u)::value;
+    const dim3 grid(pl.grid), block(GEMV_THREADS);
+    auto run = [&](auto fast, auto xp, auto ms) {
+      hipLaunchKernelGGL((gemv_merge_kernel<R, U, decltype(fast)::value, decltype(xp)::value, decltype(ms)::value>), grid, block, fused_lds(a), st, a, p);
+    };
+    using std::integral_constant;
+    auto by_k = [&](auto fast) {
+      if (a.K > 2048) run(fast, integral_constant<int, 4>{}, integral_constant<int, 4>{});
+      else if (p.nsplit > 4) run(fast, integral_constant<int, 2>{}, integral_constant<int, 8>{});
+      else run(fast, integral_constant<int, 2>{}, integral_constant<int, 4>{});
+    };
+    if (a.K % (512 * U) != 0) by_k(std::false_type{});
+    else by_k(std::true_type{});
+  };
+  using std::integral_constant;   // (the load groups of kernels_gemv.hip; an output this long with K <= 4096 has 16 loads in flight per wave)
+  if (pl.R == 4) go(integral_constant<int, 4>{}, integral_constant<int, 4>{});
+  else if (pl.R == 2) pl.U >= 8 ? go(integral_constant<int, 2>{}, integral_constant<int, 8>{}) : go(integral_constant<int, 2>{}, integral_constant<int, 2>{});
+  else if (pl.U >= 8) go(integral_constant<int, 1>{}, integral_constant<int, 8>{});
+  else if (pl.U >= 4) go(integral_constant<int, 1>{}, integral_constant<int, 4>{});
+  else go(integral_constant<int, 1>{}, integral_constant<int, 1>{});
 }
 
 void launch_gemv_polynorm(const GemvArgs& a, const PolyNormArgs& p, GemvEpi epi, hipStream_t st) {

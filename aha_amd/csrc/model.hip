@@ -1388,6 +1388,10 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after) {
   const int div = e_div ? std::max(1, atoi(e_div)) : 4;
   int nsplit = (npages + div - 1) / div;
   nsplit = std::max(1, std::min(std::min(nsplit, m->max_nsplit), 1024 / (nh / kvh)));  // g * nsplit <= 1024: LDS tables of the split merge
+  // short and middle contexts: the merge of the splits in the o_proj matvec (one GPU)
+  int defer = e_div ? 0 : attn_decode_defer_splits(npages, nq);
+  if (defer > 1 && m->tp_size > 1) defer = 0;
+  if (defer) nsplit = defer;
   for (int li = 0; li < c.num_hidden_layers; ++li) {
     const LayerWeights& L = m->layers[li];
     {  // h = RMSNorm(x); qkv = h Wqkv^T                      (qwen3/model.rs:79, modules.rs:538-552)
@@ -1405,7 +1409,7 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after) {
       a.kv = model_kv_layer(m, li); a.kv_start_v = (int)kv_len_after - 1; a.kv_len_v = (int)kv_len_after;
       a.part_o = m->d_part_o; a.part_ml = m->d_part_ml; a.nh = nh; a.kvh = kvh; a.nsplit = nsplit; a.eps = c.rms_norm_eps;
       a.scale = m->attn_scale; a.o = m->d_attn; a.head_ctr = m->d_bar + DECODE_HEAD_CTR_WORD;
-      if (nsplit > 1) m->head_ctr_base += (unsigned)nsplit;  // a single split never touches the counter
+      if (nsplit > 1 && !defer) m->head_ctr_base += (unsigned)nsplit;  // (neither a single split nor a deferred merge touches the counter)
       a.ctr_target = m->head_ctr_base;
       static const char* e_at = getenv("AHA_ATTN_TRACE");
       if (e_at && atoi(e_at)) {
@@ -1422,10 +1426,12 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after) {
       const double gemv_bytes = (double)g.N * g.K * 2 + g.K * 2.0 + g.N * 4.0;
       {
         ProfScope ps(m, "attn_decode", attn_bytes, 4.0 * kv_len_after * nq);
-        launch_attn_decode_fused(a, st);
+        if (defer) launch_attn_decode_defer(a, st);
+        else launch_attn_decode_fused(a, st);
       }
       ProfScope ps(m, "gemv", gemv_bytes, 2.0 * g.N * g.K);
-      gemv_row_parallel(m, g);
+      if (defer > 1) launch_gemv_merge(g, GemvMerge{m->d_part_o, m->d_part_ml, nsplit, nh}, st);
+      else gemv_row_parallel(m, g);
     } else {  // three-launch variant (A/B knob AHA_DECODE_FUSED=0)
       {  // q/k norm + rope + append                            (modules.rs:544-566)
         RopeArgs r{};

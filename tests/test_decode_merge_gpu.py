@@ -1,0 +1,42 @@
+"""-m gpu: decode attention whose split-KV partials are merged by the o_proj matvec (attn_decode_defer_kernel + gemv_merge_kernel), against the form
+that launches norm, attention and combine by themselves."""
+import numpy as np
+import pytest
+
+from aha_amd.configs import tiny_qwen3
+from aha_amd.weights import qwen3_text_weights
+from tests.test_model_gpu import LOGIT_RMS_STD, LOGIT_TOL_STD, ids_for
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("heads,kv_heads,lens", [
+    (4, 2, [126, 127, 128, 255, 1022, 3070]),       # 1 -> 2 splits, whole pages, 8 splits and the last length merged this way
+    (6, 2, [190, 700]),                             # 768 columns: no whole chunk groups for the matvec
+    (1, 1, [320]),                                  # one head, 128 columns
+    (16, 1, [449]),                                 # sixteen query heads in one block, 2048 columns
+    (32, 8, [128, 1534, 1535, 1536]),               # 4096 columns: 4 splits, the first length beyond them
+])
+def test_partials_merged_by_the_projection(gpu, monkeypatch, heads, kv_heads, lens):
+    """Two layers, three steps from each length on; the bound is that of the two decode forms' own test (test_model_gpu.py): the same arithmetic per
+    token, another merge order."""
+    from aha_amd.model import HipInferenceModel
+    cfg = tiny_qwen3(layers=2, hidden=512, heads=heads, kv_heads=kv_heads, inter=512, vocab=1024)
+    w = qwen3_text_weights(cfg, seed=4)
+    monkeypatch.setenv("AHA_DECODE_FUSED", "1")
+    merged = HipInferenceModel(cfg, w)
+    monkeypatch.setenv("AHA_DECODE_FUSED", "0")
+    plain = HipInferenceModel(cfg, w)
+    for S in lens:
+        ids = ids_for(cfg, S, 7 + S)
+        merged.clear_cache(); plain.clear_cache()
+        _, tok = plain.forward_initial(ids, 0)
+        merged.forward_initial(ids, 0)
+        for step in range(3):
+            a, am = plain.forward_step(tok, S + step)
+            b, _ = merged.forward_step(tok, S + step)
+            std = float(a.std())
+            assert np.isfinite(b).all()
+            assert float(np.abs(a - b).max()) <= LOGIT_TOL_STD * std and float(np.sqrt(((a - b) ** 2).mean())) <= LOGIT_RMS_STD * std, (S, step)
+            tok = am
+    merged.close(); plain.close()
