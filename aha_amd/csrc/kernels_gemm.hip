@@ -1094,11 +1094,13 @@ GemmPlan plan_gemm(const GemmArgs& a) {
   const bool can_split = a.act != ACT_SILU_MUL_PAIRS && a.act != ACT_PARTIAL_F32 && a.workspace != nullptr && (a.N & 3) == 0;
   GemmPlan best{128, 1};
   double best_cost = cost128;
-  // 256 x 128 tiles on the eight-wave ring kernel (plan tile 2128): where the 128^2 tiling overflows one block per CU and this one does not
+  // 256 x 128 tiles on the eight-wave ring kernel (plan tile 2128): where the 128^2 tiling overflows one block per CU and this one does not.
+  // 129 to 255 rows fill two rows of 128^2 tiles and one of these: at any K, since the launch it replaces runs single-stage blocks two to a CU
+  // (205 x 24576 x 4096: 92 -> 68 us).
   static const bool tall_on = [] { const char* e = getenv("AHA_GEMM_TALL"); return e ? atoi(e) != 0 : true; }();
   static const double lat_tall = [] { const char* e = getenv("AHA_GEMM_LAT_TALL"); return e ? atof(e) : 0.85; }();
   const double t2128 = (double)((a.M + 255) / 256) * ((a.N + 127) / 128);
-  if (tall_on && a.M >= 256 && nk >= 8 && nk <= 24 && t128 > (double)gemm_streamk_cus() && t2128 <= (double)gemm_streamk_cus() && !e_tile && !e_sk &&
+  if (tall_on && nk >= 8 && (a.M >= 256 ? nk <= 24 : a.M > 128) && t128 > (double)gemm_streamk_cus() && t2128 <= (double)gemm_streamk_cus() && !e_tile && !e_sk &&
       a.act != ACT_PARTIAL_F32) {
     const double c = nk * lat_tall + 5.0;   // (a riding norm is a launch of its own here as behind the 128^2 tiling this competes with)
     if (c < best_cost) {
@@ -1223,7 +1225,7 @@ GemmPlan plan_gemm(const GemmArgs& a) {
   static const char* e_dbg = getenv("AHA_GEMM_PLAN_DEBUG");
   if (e_dbg && atoi(e_dbg)) fprintf(stderr, "[gemm plan] M=%d N=%d K=%d act=%d -> tile %d splitk %d%s (cost %.1f us, 128^2 %.1f us)\n", a.M, a.N, a.K, a.act, best.tile, best.splitk, best.streamk ? " persistent" : "", best_cost, cost128);
   best.cost = best_cost;
-  if (a.M < 256 && best.tile != 128) best = GemmPlan{128, 1, cost128};
+  if (a.M < 256 && best.tile != 128 && best.tile != 2128) best = GemmPlan{128, 1, cost128};
   if (e_tile && atoi(e_tile) == 128) best = GemmPlan{128, 1, cost128};
   return best;
 }
