@@ -491,22 +491,66 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(SsmStepArgs a, SeqBatch b
   const float A = a.p.a[h], D = a.p.d[h];
   const float* hin = a.h.hist + (int64_t)e.slot * a.h.slot_stride + (int64_t)e.hist_in * (taps - 1) * cp;
   float* hout = a.h.hist + (int64_t)e.slot * a.h.slot_stride + (int64_t)e.hist_out * (taps - 1) * cp;
-  for (int i = tid; i < 2 * np + VT * 16; i += 256) {
-    const bool is_x = i >= 2 * np;
-    const int ch = is_x ? h * a.d.vdp + vs * 16 + i - 2 * np : inner + (i < np ? grp * np + i : a.d.groups * np + grp * np + i - np);
-    const float cur = Act<TI>::ld(row + a.in.c_off + ch);
-    float acc = fmaf(a.p.conv_w[(int64_t)(taps - 1) * cp + ch], cur, a.p.conv_b[ch]);
-    const bool owner = is_x || (h == grp * hpg && vs == 0);
-    float prev = cur;
-    for (int q = 0; q < taps - 1; ++q) {   // the input q + 1 tokens back
-      const float x = e.pos0 - 1 - q >= 0 ? hin[(int64_t)q * cp + ch] : 0.f;
-      acc = fmaf(a.p.conv_w[(int64_t)(taps - 2 - q) * cp + ch], x, acc);
-      if (owner) hout[(int64_t)q * cp + ch] = prev;
-      prev = x;
-    }
+  // The block's channels: x, B and C, NIT per thread.  Inputs, weights and history of up to HT + 1 taps are requested together and the new history is
+  // stored behind them: a store between two loads orders them, and tap by tap, channel by channel the chain was most of the launch (0.6B widths,
+  // one sequence: 7.5 -> 5.1 us; 8B widths, 32 sequences: 69 -> 60 us).
+  constexpr int NIT = (2 * NI * 64 + VT * 16 + 255) / 256, HT = 4;
+  const int total = 2 * np + VT * 16;
+  auto channel = [&](int i) { return i >= 2 * np ? h * a.d.vdp + vs * 16 + i - 2 * np : inner + (i < np ? grp * np + i : a.d.groups * np + grp * np + i - np); };
+  auto put = [&](int i, float acc) {
     acc = silu_f32(acc);
-    if (is_x) xs[i - 2 * np] = acc;
+    if (i >= 2 * np) xs[i - 2 * np] = acc;
     else bc[i < np ? i : NI * 64 + i - np] = acc;
+  };
+  if (taps >= 2 && taps <= HT + 1) {
+    float cur[NIT], wl[NIT], bias[NIT], x[NIT][HT], w[NIT][HT];
+#pragma unroll
+    for (int k = 0; k < NIT; ++k) {
+      const int ch = channel(min(tid + k * 256, total - 1));
+      cur[k] = Act<TI>::ld(row + a.in.c_off + ch);
+      wl[k] = a.p.conv_w[(int64_t)(taps - 1) * cp + ch];
+      bias[k] = a.p.conv_b[ch];
+#pragma unroll
+      for (int q = 0; q < HT; ++q) {   // (taps that are not there: the oldest one again)
+        const int qq = min(q, taps - 2);
+        x[k][q] = hin[(int64_t)qq * cp + ch];
+        w[k][q] = a.p.conv_w[(int64_t)(taps - 2 - qq) * cp + ch];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < NIT; ++k) {
+      const int i = tid + k * 256;
+      if (i >= total) continue;
+      float acc = fmaf(wl[k], cur[k], bias[k]);
+#pragma unroll
+      for (int q = 0; q < HT; ++q) {
+        if (q >= taps - 1) continue;
+        if (e.pos0 - 1 - q < 0) x[k][q] = 0.f;
+        acc = fmaf(w[k][q], x[k][q], acc);
+      }
+      put(i, acc);
+      if (i >= 2 * np || (h == grp * hpg && vs == 0)) {
+        const int ch = channel(i);
+#pragma unroll
+        for (int q = 0; q < HT; ++q)
+          if (q < taps - 1) hout[(int64_t)q * cp + ch] = q == 0 ? cur[k] : x[k][q > 0 ? q - 1 : 0];
+      }
+    }
+  } else {
+    for (int i = tid; i < total; i += 256) {
+      const int ch = channel(i);
+      const float cur = Act<TI>::ld(row + a.in.c_off + ch);
+      float acc = fmaf(a.p.conv_w[(int64_t)(taps - 1) * cp + ch], cur, a.p.conv_b[ch]);
+      const bool owner = i >= 2 * np || (h == grp * hpg && vs == 0);
+      float prev = cur;
+      for (int q = 0; q < taps - 1; ++q) {   // the input q + 1 tokens back
+        const float x = e.pos0 - 1 - q >= 0 ? hin[(int64_t)q * cp + ch] : 0.f;
+        acc = fmaf(a.p.conv_w[(int64_t)(taps - 2 - q) * cp + ch], x, acc);
+        if (owner) hout[(int64_t)q * cp + ch] = prev;
+        prev = x;
+      }
+      put(i, acc);
+    }
   }
   const float dt = softplus_f32(dtz), da = expf(A * dt);
   __syncthreads();
