@@ -68,6 +68,7 @@ void launch_argmax_f32_rows(const float* x, int64_t n, int64_t ld, int rows, flo
 int sample_stage1_waves(int V);
 bool sample_shape_ok(int V, int k);
 void launch_repeat_penalty(const float* logits, float* work, const uint32_t* ctx, int n, float penalty, int V, hipStream_t st);
+size_t sample_index_words(int V);   // u32 words of launch_topk_candidates' cand_idx
 void launch_topk_candidates(const float* x, int V, int k, float inv_temp, float* cand_val, unsigned* cand_idx, float* part_m,
                             float* part_s, float* out_val, unsigned* out_idx, float* out_ms, hipStream_t st);
 

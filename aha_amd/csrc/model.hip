@@ -465,7 +465,7 @@ int model_sample_candidates(aha_model* m, const uint32_t* ctx, size_t n_ctx, flo
   constexpr size_t OUT_WORDS = 64 + 2 + 64;
   if (!m->d_samp_f) {
     const size_t nc = ((size_t)nw + 16) * 64;  // stage-1 candidates + the 16 x 64 intermediates behind them
-    const size_t nf = nc + 2 * (size_t)nw + OUT_WORDS, nu = nc;
+    const size_t nf = nc + 2 * (size_t)nw + OUT_WORDS, nu = sample_index_words(V);
     void *pw = nullptr, *pf = nullptr, *pu = nullptr;
     if (int rc = dev_alloc(m, (size_t)V * 4, &pw, false)) return rc;
     if (int rc = dev_alloc(m, nf * 4, &pf, false)) return rc;

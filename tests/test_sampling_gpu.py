@@ -153,3 +153,25 @@ def test_stream_loop_device_chunks_equal_host_loop(gpu):
         assert b[:len(a)] == a and len(b) in (len(a), len(a) + 1)   # the stream loop runs sample_len iterations, the generic one sample_len - 1 steps after the prefill
     finally:
         m.close()
+
+
+@pytest.mark.parametrize("vocab", [64, 512, 513, 33000])
+def test_where_the_candidates_lie(gpu, vocab):
+    """An infinite penalty over all tokens but a few (non-negative logits become 0, the others -inf) puts the candidates where it is told: all in one
+    wave's 512 entries, one in each of several waves, nowhere (zeros and -inf only), with vocabularies of fewer waves than k and of a partial last wave."""
+    cfg, m = make(vocab)
+    try:
+        logits, _ = m.forward_initial([3, 4], 0)
+        every = np.arange(vocab)
+        last = every[(vocab - 1) // 512 * 512:]
+        for keep in (every[:0], last, every[::509], every[-1:], every):
+            ctx = [int(i) for i in np.setdiff1d(every, keep)]
+            for k in (1, 20, 64):
+                vals, idx, mx, se = m.sample_candidates(ctx, float("inf"), 1.0, k)
+                ref = osamp.apply_repeat_penalty(logits, float("inf"), ctx) if ctx else logits
+                rv, ri, rmx, rse = osamp.topk_candidates(ref, k, 1.0)
+                np.testing.assert_array_equal(idx, ri)
+                np.testing.assert_array_equal(vals.view(np.uint32), rv.view(np.uint32))
+                assert np.float32(mx) == np.float32(rmx) and abs(se - rse) <= 2e-5 * rse
+    finally:
+        m.close()
