@@ -718,6 +718,15 @@ int aha_hip_embed(aha_model* m, const uint32_t* input_ids, size_t n_ids, float* 
   return model_embed(m, input_ids, n_ids, out);
   API_GUARD_END
 }
+int aha_hip_embed_multi(aha_model* m, const uint32_t* input_ids, const uint64_t* n_ids, size_t n_docs, float* out) {
+  API_GUARD_BEGIN
+  if (!m) {
+    set_error("null model");
+    return AHA_ERR_INVALID;
+  }
+  return model_embed_multi(m, input_ids, n_ids, n_docs, out);
+  API_GUARD_END
+}
 int aha_hip_config_parse(const char* model_dir, aha_model_desc* out) {
   API_GUARD_BEGIN
   if (!model_dir || !out) {

@@ -181,6 +181,9 @@ struct AttnPrefillArgs {
   int chunk = 0, sink = 0;
 };
 void launch_attn_prefill(const AttnPrefillArgs& a, hipStream_t st);
+// Sequences of their own (a.seqs: n entries, none longer than max_len; head_dim 128, causal); only where the f32 score chain runs (takes_seqs)
+bool attn_prefill_takes_seqs(float scale);
+void launch_attn_prefill_seqs(const AttnPrefillArgs& a, int n, int max_len, hipStream_t st);
 bool attn_prefill_takes_qfuse(const AttnPrefillArgs& a);   // would launch_attn_prefill run a kernel that norms + rotates Q itself for these arguments?
 // the one-wave-per-SIMD, 64-q-rows-per-wave form (kernels_attn64.hip); false = not a shape of that kernel, nothing launched
 bool launch_attn_prefill64(const AttnPrefillArgs& a, hipStream_t st, int pipe);

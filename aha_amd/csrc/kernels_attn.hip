@@ -217,6 +217,11 @@ static int attn_prefill_form(const AttnPrefillArgs& a, int smx) {
   if (form == 65 || (form < 0 && auto64)) return 65;
   return 0;
 }
+bool attn_prefill_takes_seqs(float scale) {
+  AttnPrefillArgs a{};
+  a.scale = scale;
+  return attn_prefill_smx(a) == 3 && g_attn_form_override < 0;
+}
 bool attn_prefill_takes_qfuse(const AttnPrefillArgs& a) {
   static const bool on = [] { const char* e = getenv("AHA_ATTN_QFUSE"); return e ? atoi(e) != 0 : true; }();
   return on && a.d == 128 && attn_prefill_form(a, attn_prefill_smx(a)) == 0;

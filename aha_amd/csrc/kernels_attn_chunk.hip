@@ -434,6 +434,25 @@ void dispatch_dims(int dq, int dv, F&& f) {
   else inner(std::integral_constant<int, 256>{});
 }
 
+template <int DQK, int DV>
+void launch_seqs(AttnPrefillArgs a, int n, int max_len, hipStream_t st) {
+  const int nwv = (int64_t)((max_len + 127) / 128) * a.nh * n >= 512 ? 8 : 4;
+  const int nqb = (max_len + 16 * nwv - 1) / (16 * nwv);
+  const bool xcd_order = a.kvh % 8 == 0;
+  a.nqb = xcd_order ? nqb : 0;
+  const dim3 grid = xcd_order ? dim3((unsigned)(nqb * a.nh), (unsigned)n) : dim3((unsigned)nqb, (unsigned)n, (unsigned)a.nh), block(nwv * 64);
+  const size_t stage = (size_t)2 * KV_PAGE_TOKENS * 2 * (DQK + DV), epi = a.epi_rows ? (size_t)nwv * 16 * (DV * 2 + 16) : 0;
+  const size_t lds = std::max(stage, epi);
+  auto go = [&](auto nw) {
+    constexpr int NW = decltype(nw)::value;
+    auto k = attn_prefill_kernel<DQK, DV, 1, NW, false, 0, 3, 1>;
+    if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipLaunchKernelGGL(k, grid, block, lds, st, a, nullptr);
+  };
+  if (nwv == 8) go(std::integral_constant<int, 8>{});
+  else go(std::integral_constant<int, 4>{});
+}
+
 }  // namespace
 
 bool chunk_attn_dims_ok(int dim, int vdim, int* dq, int* dv) {
@@ -452,25 +471,16 @@ void launch_chunk_attn_prefill(const ChunkAttnArgs& c, const SeqBatch& b, hipStr
   a.causal = 1;
   a.scale = c.scale;
   a.seqs = b.entries; a.seq_tab_ld = c.kv.ld; a.chunk = c.chunk; a.sink = c.sink;
-  const int nwv = (int64_t)((b.max_len + 127) / 128) * c.heads * b.n >= 512 ? 8 : 4;
-  const int nqb = (b.max_len + 16 * nwv - 1) / (16 * nwv);
-  const bool xcd_order = a.kvh % 8 == 0;
-  a.nqb = xcd_order ? nqb : 0;
-  const dim3 grid = xcd_order ? dim3((unsigned)(nqb * a.nh), (unsigned)b.n) : dim3((unsigned)nqb, (unsigned)b.n, (unsigned)a.nh), block(nwv * 64);
   a.epi_rows = a.d % 8 == 0 && a.d <= 128 && ((uintptr_t)a.o & 15) == 0;
-  dispatch_dims(c.kv.dq, c.kv.dv, [&](auto q, auto v) {
-    constexpr int DQK = decltype(q)::value, DV = decltype(v)::value;
-    const size_t stage = (size_t)2 * KV_PAGE_TOKENS * 2 * (DQK + DV), epi = a.epi_rows ? (size_t)nwv * 16 * (DV * 2 + 16) : 0;
-    const size_t lds = std::max(stage, epi);
-    auto go = [&](auto nw) {
-      constexpr int NW = decltype(nw)::value;
-      auto k = attn_prefill_kernel<DQK, DV, 1, NW, false, 0, 3, 1>;
-      if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      hipLaunchKernelGGL(k, grid, block, lds, st, a, nullptr);
-    };
-    if (nwv == 8) go(std::integral_constant<int, 8>{});
-    else go(std::integral_constant<int, 4>{});
-  });
+  dispatch_dims(c.kv.dq, c.kv.dv, [&](auto q, auto v) { launch_seqs<decltype(q)::value, decltype(v)::value>(a, b.n, b.max_len, st); });
+}
+
+// the Qwen3 stack's head dims, q heads raw or rotated (AttnPrefillArgs::q_norm_w)
+void launch_attn_prefill_seqs(const AttnPrefillArgs& a_in, int n, int max_len, hipStream_t st) {
+  if (n <= 0) return;
+  AttnPrefillArgs a = a_in;
+  a.epi_rows = ((uintptr_t)a.o & 15) == 0;
+  launch_seqs<128, 128>(a, n, max_len, st);
 }
 
 void launch_chunk_attn_decode(const ChunkDecodeArgs& a, const SeqBatch& b, hipStream_t st) {

@@ -168,6 +168,7 @@ struct aha_model {
   size_t samp_ctx_cap = 0;
   // prefill scratch (grown on demand)
   size_t pf_cap = 0;
+  void* d_docs = nullptr;        // joint prefill of documents (model_embed_multi): their SeqEntry records, then their last rows' numbers
   uint32_t* p_ids = nullptr;
   int32_t* p_pos = nullptr;
   void *p_x = nullptr, *p_h = nullptr, *p_qkv = nullptr, *p_q = nullptr, *p_attn = nullptr, *p_act = nullptr;
@@ -201,6 +202,7 @@ inline bool arch_computes_f32(int32_t arch) { return arch_is_layered(arch); }
 int model_create(aha_ctx* ctx, const aha_model_desc* desc, const aha_tensor_view* w, size_t nw, aha_model** out);
 void model_destroy(aha_model* m);
 int model_embed(aha_model* m, const uint32_t* ids, size_t n, float* out);
+int model_embed_multi(aha_model* m, const uint32_t* ids, const uint64_t* lens, size_t n_docs, float* out);
 int model_forward_initial(aha_model* m, const uint32_t* ids, size_t n, size_t offset, const aha_mm_input* mm,
                           float* logits_out, uint32_t* argmax_out);
 int model_forward_step(aha_model* m, uint32_t token, size_t offset, float* logits_out, uint32_t* argmax_out);

@@ -427,7 +427,12 @@ class HipInferenceModel:
     def embed_multi(self, inputs: Sequence[Sequence[int]]) -> np.ndarray:
         if len(inputs) == 0:
             raise ValueError("embedding input cannot be empty")  # qwen3_embedding/mod.rs:39-41
-        return np.stack([self.embed_one(x) for x in inputs], 0)
+        docs = [np.asarray(x, dtype=np.uint32).reshape(-1) for x in inputs]
+        ids, lens = np.concatenate(docs), np.array([d.size for d in docs], dtype=np.uint64)
+        out = np.empty((len(docs), self.text_cfg.hidden_size), dtype=np.float32)
+        check(lib().aha_hip_embed_multi(self.handle, ids.ctypes.data_as(C.POINTER(C.c_uint32)), lens.ctypes.data_as(C.POINTER(C.c_uint64)), len(docs),
+                                        out.ctypes.data_as(C.POINTER(C.c_float))))
+        return out
 
     def rerank(self, query_ids: Sequence[int], documents_ids: Sequence[Sequence[int]]) -> np.ndarray:
         """Qwen3Reranker::rerank (qwen3_reranker/mod.rs:23-31): cosine_similarity_no_l2(query, docs) on normalised vectors."""

@@ -199,6 +199,8 @@ int aha_hip_get_rope_index_mm(const aha_model_desc* desc, const uint32_t* input_
  * Qwen3Reranker::rerank (qwen3_reranker/mod.rs:23-31) is the dot product of two such vectors
  * (cosine_similarity_no_l2, modules.rs:1381-1389) -- host arithmetic on the caller's side. */
 int aha_hip_embed(aha_model* m, const uint32_t* input_ids, size_t n_ids, float* out);
+/* n_docs documents, their ids one after another (n_ids[d] of document d) -> out[n_docs][hidden_size]: documents that fit together share one prefill. */
+int aha_hip_embed_multi(aha_model* m, const uint32_t* input_ids, const uint64_t* n_ids, size_t n_docs, float* out);
 
 /* ---- checkpoint directory -> model (XxxGenerateModel::init minus tokenizer / chat template) --------------------------
  * aha_hip_config_parse: <dir>/config.json -> aha_model_desc, the same field mapping serde does into Qwen3Config

@@ -74,3 +74,27 @@ def test_embed_errors(pair):
         m.embed_multi([])
     with pytest.raises(AhaHipError, match="out of range"):
         m.embed_one([cfg.vocab_size])
+
+
+@pytest.mark.parametrize("heads, kv_heads", [(4, 2), (16, 8)])
+def test_documents_together(gpu, heads, kv_heads):
+    """embed_multi's joint prefill, document lengths around a cache page (64) and around the rows that one prefill takes (4096), with one-token documents
+    between: each vector within the bound of test_embed_matches_oracle of what the document gives alone, both being within half of it of the exact one."""
+    from aha_amd._lib import AhaHipError
+    from aha_amd.model import HipInferenceModel
+    cfg = tiny_qwen3(layers=2, hidden=256, heads=heads, kv_heads=kv_heads, inter=512, vocab=2048)
+    m = HipInferenceModel(cfg, qwen3_text_weights(cfg, seed=1))
+    try:
+        for lens in ([2, 3], [63, 1, 64, 65, 300, 2, 129], [2000, 2100, 7], [4097, 5, 4095, 1, 1], [90] * 70):
+            docs = seqs_for(cfg, lens, len(lens))
+            got = m.embed_multi(docs)
+            ref = np.stack([m.embed_one(x) for x in docs])
+            assert got.shape == ref.shape and m.cache_len() == 0
+            rms = np.sqrt((ref ** 2).mean(1))
+            assert float((np.abs(got - ref).max(1) / rms).max()) <= 0.04
+            assert float((got * ref).sum(1).min()) >= 0.9995
+        for bad in ([[1, 2], [3, 4], []], [[1, 2], [3, cfg.vocab_size], [5, 6]]):
+            with pytest.raises(AhaHipError, match="empty|out of range"):
+                m.embed_multi(bad)
+    finally:
+        m.close()
