@@ -455,16 +455,17 @@ __global__ __launch_bounds__(256) void latent_merge_kernel(LatentMergeArgs a) {
   // The splits' sums, 32 of them requested at once and ahead of the weights that join them (one after the other behind the weights' barrier, the 64 of
   // a 4096-position window made the launch 8.8 us; 6.6 now).  Past the end the last one again, never used.
   constexpr int NB = RQ <= 2 ? 32 : 16;
-  const float* part[RQ];
+  const char* part = reinterpret_cast<const char*>(a.part_o + at * rp);
+  uint32_t col[RQ];   // (byte offsets: LATENT_MAX_SPLIT x heads x rp floats, latent_decode_ok)
   float v[RQ][NB];
   auto request = [&](int s0) {
 #pragma unroll
-    for (int q = 0; q < RQ; ++q)
+    for (int j = 0; j < NB; ++j)
 #pragma unroll
-      for (int j = 0; j < NB; ++j) v[q][j] = part[q][(int64_t)min(s0 + j, a.nsplit - 1) * heads * rp];
+      for (int q = 0; q < RQ; ++q) v[q][j] = *reinterpret_cast<const float*>(part + (col[q] + (uint32_t)(min(s0 + j, a.nsplit - 1) * heads * rp) * 4u));
   };
 #pragma unroll
-  for (int q = 0; q < RQ; ++q) part[q] = a.part_o + at * rp + min(q * 256 + tid, rp - 1);
+  for (int q = 0; q < RQ; ++q) col[q] = (uint32_t)min(q * 256 + tid, rp - 1) * 4u;
   request(0);
   if (tid < 64) {
     float2 ml = make_float2(-INFINITY, 0.f);
@@ -614,7 +615,7 @@ void launch_latent_prefill(const LatentPrefillArgs& a, const SeqBatch& b, hipStr
 }
 
 int latent_decode_blocks_per_cu(const LatentDims& d) { return std::max(1, std::min(2, 160 * 1024 / latent_decode_lds(d))); }
-bool latent_decode_ok(const LatentDims& d) { return d.rp <= 1024 && latent_decode_lds(d) <= 160 * 1024 && d.scale > 0.f; }
+bool latent_decode_ok(const LatentDims& d) { return d.rp <= 1024 && (int64_t)d.heads * d.rp < 1 << 24 && latent_decode_lds(d) <= 160 * 1024 && d.scale > 0.f; }
 
 void launch_latent_decode(const LatentDecodeArgs& a, const SeqBatch& b, hipStream_t st) {
   if (b.n <= 0) return;
