@@ -11,8 +11,8 @@ constexpr int ATTN_DECODE_FUSED_LDS = 16 * 128 * 2 + 128 * 2 + 128 * 2 + ATTN_DE
 // ---- decode, fused: q/k RMSNorm + (M-)RoPE + KV append + split-KV attention + in-block merge --------------------
 // One launch replaces qknorm_rope_kernel + attn_decode_kernel + the combine: every block redoes the (tiny) norm/rope of
 // its kv head's g query heads and of the new key in LDS (QKNormAttention::forward, modules.rs:538-557), block (kvhd, 0)
-// appends the new K/V to the cache page (modules.rs:558-566), all blocks attend over the OLD tokens from the pages, unit
-// 0 adds the new token from LDS, the 4 waves of a block are merged through LDS, one un-normalised partial per
+// appends the new K/V to the cache page (modules.rs:558-566), all blocks attend over the OLD tokens from the pages, the
+// last unit begins with the new token from LDS, the 4 waves of a block are merged through LDS, one un-normalised partial per
 // (split, head) is published, and the LAST split block of the kv head to arrive merges the splits and writes the bf16
 // attention output.
 //
@@ -35,8 +35,8 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
   bf16_t* qs = reinterpret_cast<bf16_t*>(smem);                 // [16][128]
   bf16_t* ksn = qs + 16 * 128;                                  // [128]
   bf16_t* vsn = ksn + 128;                                      // [128]
-  const int g = a.nh / a.kvh, P = DEFER ? g : 16;               // P: q slots kept per dim
-  float* mo = reinterpret_cast<float*>(vsn + 128);              // per wave O^T [NW][d 128][q P]
+  const int g = a.nh / a.kvh, P = DEFER ? g : 16;               // P: q slots
+  float* mo = reinterpret_cast<float*>(vsn + 128);              // per wave O [NW][q P][d 128]
   float* mm = mo + NW * 128 * P;                                // [NW][16]
   float* mlz = mm + NW * 16;                                    // [NW][16]
   const int tid = (int)threadIdx.x;
@@ -162,6 +162,27 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
 #pragma unroll
   for (int i = 0; i < 8; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
+  // The new token, from LDS: the running state of the last unit (never the one with the most pages) begins with it, under the unit's page fetch.
+  // (Behind unit 0's pages, and with the waves' sums merged by dwords, the part after the pages was 1.49 us of the slowest block; 0.57 now.)
+  if (unit == nunits - 1) {
+    float d4[4] = {0.f, 0.f, 0.f, 0.f};
+    const u32x4_t* qr = reinterpret_cast<const u32x4_t*>(qs + min(c, g - 1) * 128 + G * 32);
+    const u32x4_t* kr = reinterpret_cast<const u32x4_t*>(ksn + G * 32);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const u32x4_t qv = qr[j], kv = kr[j];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) d4[e] = fmaf(hi_bf(qv[e]), hi_bf(kv[e]), fmaf(lo_bf(qv[e]), lo_bf(kv[e]), d4[e]));
+    }
+    m = rbf(rbf(group_sum((d4[0] + d4[1]) + (d4[2] + d4[3]))) * a.scale);
+    l = G == 0 ? 1.f : 0.f;
+#pragma unroll
+    for (int ds = 0; ds < 8; ++ds) {
+      const uint2 v = *reinterpret_cast<const uint2*>(vsn + ds * 16 + G * 4);
+      o[ds] = f32x4_t{lo_bf(v.x), hi_bf(v.x), lo_bf(v.y), hi_bf(v.y)};
+    }
+  }
+
   // One page of this unit.  MORE (compile time): the unit has another page after this one -- its K is requested right
   // after QK^T and its V right after P.V, unconditionally, so the register buffers are plain loop-carried values (a
   // run-time `if (more) load` makes them phis that the compiler resolves with copies and a vmcnt(0) at the loop end).
@@ -203,34 +224,14 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
     do_page(std::false_type{});
   }
   stamp(2);
-  if (unit == 0) {  // the new token: score from LDS, one more online-softmax step
-    float dot = 0.f;
-    const bf16_t* qr = qs + min(c, g - 1) * 128 + G * 32;
-    const bf16_t* kr = ksn + G * 32;
-#pragma unroll
-    for (int j = 0; j < 32; ++j) dot = fmaf(bf2f(qr[j]), bf2f(kr[j]), dot);
-    dot = group_sum(dot);
-    const float s = rbf(rbf(dot) * a.scale);
-    const float m_new = fmaxf(m, s);
-    const float alpha = __expf(m - m_new);
-    const float p = rbf(__expf(s - m_new));  // P feeds the MFMA as bf16 on the page path: same rounding here
-    l = l * alpha + (G == 0 ? __expf(s - m_new) : 0.f);
-    m = m_new;
-#pragma unroll
-    for (int ds = 0; ds < 8; ++ds)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[ds][r] = fmaf(p, bf2f(vsn[ds * 16 + G * 4 + r]), o[ds][r] * alpha);
-  }
   l = group_sum(l);
 
   // ---- merge the waves through LDS, leave one partial per (split, head) ---------------------------------------------
   {
     float* wo = mo + wave * (128 * P);
-    if (!DEFER || c < g) {
+    if (c < g) {
 #pragma unroll
-      for (int ds = 0; ds < 8; ++ds)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) wo[(ds * 16 + G * 4 + r) * P + c] = o[ds][r];
+      for (int ds = 0; ds < 8; ++ds) *reinterpret_cast<f32x4_t*>(wo + c * 128 + ds * 16 + G * 4) = o[ds];
     }
     if (G == 0) {
       mm[wave * 16 + c] = m;
@@ -252,8 +253,9 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
     for (int w = 0; w < NW; ++w) {
       const float mw = mm[w * 16 + q];
       const float wt = (mw == -INFINITY) ? 0.f : __expf(mw - M);
+      const f32x4_t ow = *reinterpret_cast<const f32x4_t*>(mo + w * (128 * P) + q * 128 + d0);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc[e] = fmaf(wt, mo[w * (128 * P) + (d0 + e) * P + q], acc[e]);
+      for (int e = 0; e < 4; ++e) acc[e] = fmaf(wt, ow[e], acc[e]);
       ls = fmaf(wt, mlz[w * 16 + q], ls);
     }
     const int head = kvhd * g + q;
@@ -277,7 +279,7 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
     }
   }
   if (single || DEFER) {
-    stamp(5);
+    for (int k = 3; k <= 5; ++k) stamp(k);
     return single;
   }
   stamp(3);
