@@ -390,17 +390,6 @@ void launch_kv_pack_pages(const void* k, const void* v, KvLayer kv, int L, hipSt
 }
 
 // ---- D11: greedy argmax (first maximal index, as candle's argmax / Sampling::ArgMax) ---------------------------
-__device__ __forceinline__ void argmax_combine(float& bv, uint32_t& bi, float v, uint32_t i) {
-  if (v > bv || (v == bv && i < bi)) { bv = v; bi = i; }
-}
-__device__ __forceinline__ void wave_argmax(float& bv, uint32_t& bi) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(bv, o, 64);
-    const uint32_t oi = __shfl_xor(bi, o, 64);
-    argmax_combine(bv, bi, ov, oi);
-  }
-}
 __global__ __launch_bounds__(256) void argmax_partials_kernel(const float* __restrict__ pv, const uint32_t* __restrict__ pi,
                                                               int n, uint32_t* __restrict__ out) {   // one block per row of n partials
   __shared__ float sv[4];

@@ -868,7 +868,7 @@ static int push_state(aha_model* m, uint32_t token, const int64_t pos[3], size_t
 
 // final RMSNorm (qwen3/model.rs:186) fused into the lm_head matvec of the LAST position only (model.rs:187,142),
 // f32 logits + argmax partials -> d_state->next_token
-static void enqueue_lm_head(aha_model* m, const void* x_last) {
+static void enqueue_lm_head(aha_model* m, const void* x_last, bool arg_max = true) {
   const aha_model_desc& c = m->desc;
   GemvArgs g{};
   g.W = m->lm_head;
@@ -885,6 +885,7 @@ static void enqueue_lm_head(aha_model* m, const void* x_last) {
     ProfScope ps(m, "gemv", (double)m->lm_rows * c.hidden_size * 2 + c.hidden_size * 2 + m->lm_rows * 4.0, 2.0 * m->lm_rows * c.hidden_size);
     launch_gemv(g, GEMV_LOGITS, m->stream);
   }
+  if (!arg_max) return;
   ProfScope ps(m, "argmax", 0, 0);
   const int ntiles = gemv_num_tiles(m->lm_rows, c.hidden_size);
   if (m->lm_rows == c.vocab_size) {
@@ -1309,8 +1310,7 @@ __global__ void embed_state_kernel(const bf16_t* __restrict__ table, const StepS
     rope[64 + i] = rbf(sinf(ang));
   }
 }
-__global__ void advance_state_kernel(StepState* st, uint32_t* token_log, uint32_t* host_ring, uint32_t* host_done) {
-  const uint32_t t = st->next_token;
+__device__ __forceinline__ void advance_state(StepState* st, uint32_t t, uint32_t* token_log, uint32_t* host_ring, uint32_t* host_done) {
   const int32_t step = st->step;
   token_log[step & 0xffff] = t;
   st->step = step + 1;
@@ -1323,6 +1323,39 @@ __global__ void advance_state_kernel(StepState* st, uint32_t* token_log, uint32_
   // publish to the host: token first, then the count (release at system scope: the host reads the count, then the slot)
   __hip_atomic_store(host_ring + ((uint32_t)step % RING_CAP), t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   __hip_atomic_store(host_done, (uint32_t)step + 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__global__ void advance_state_kernel(StepState* st, uint32_t* token_log, uint32_t* host_ring, uint32_t* host_done) {
+  advance_state(st, st->next_token, token_log, host_ring, host_done);
+}
+// Between two steps of the greedy loop in one launch: the arg-max of the lm_head's partials (argmax_partials_kernel), advance_state_kernel, and the next
+// step's embed_state_kernel.  One block: three dependent round trips to memory (partials, embedding row, the publication) -- 5.1 us where the three launches
+// took 4.6 + 4.5 + 4.6 and their gaps.
+__global__ __launch_bounds__(1024) void next_step_kernel(const float* __restrict__ pv, const uint32_t* __restrict__ pi, int n, StepState* st, const bf16_t* __restrict__ table,
+                                                         int vocab, int H, bf16_t* __restrict__ out, const float* __restrict__ inv_freq, const int32_t* __restrict__ axis_map,
+                                                         float* __restrict__ rope, uint32_t* token_log, uint32_t* host_ring, uint32_t* host_done) {
+  __shared__ float sv[16];
+  __shared__ uint32_t si[16];
+  const int tid = threadIdx.x;
+  float bv = -INFINITY;
+  uint32_t bi = 0xffffffffu;
+  if (tid < 64) {   // (the positions are used up in front of the barrier: the state changes behind it)
+    const float ang = (float)(st->pos[axis_map[tid]] + 1) * inv_freq[tid];
+    rope[tid] = rbf(cosf(ang));
+    rope[64 + tid] = rbf(sinf(ang));
+  }
+  for (int i = tid; i < n; i += 1024) argmax_combine(bv, bi, pv[i], pi[i]);
+  wave_argmax(bv, bi);
+  if ((tid & 63) == 0) { sv[tid >> 6] = bv; si[tid >> 6] = bi; }
+  __syncthreads();
+  bv = sv[0], bi = si[0];
+#pragma unroll
+  for (int w = 1; w < 16; ++w) argmax_combine(bv, bi, sv[w], si[w]);
+  const u32x4_t* src = reinterpret_cast<const u32x4_t*>(table + (size_t)min(bi, (uint32_t)vocab - 1u) * H);   // (no arg-max at all: NaN logits)
+  for (int i = tid; i < H / 8; i += 1024) reinterpret_cast<u32x4_t*>(out)[i] = src[i];
+  if (tid == 1023) {
+    st->next_token = bi;
+    advance_state(st, bi, token_log, host_ring, host_done);
+  }
 }
 
 // AHA_GEMV_TRACE=1: in-kernel timeline of the decode matvecs (launch-per-op path), dumped by fetch_outputs
@@ -1367,7 +1400,8 @@ static void gemv_trace_dump(aha_model* m) {
   }
 }
 
-static void enqueue_decode_step(aha_model* m, size_t kv_len_after) {
+// row_ready: the step's embedding row and rope table are there already (next_step_kernel); arg_max: next_token is left in the state
+static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_ready = false, bool arg_max = true) {
   if (m->layered) {
     const int rc = layered_enqueue_step(m, kv_len_after);
     if (rc && !m->async_rc) m->async_rc = rc;
@@ -1377,7 +1411,7 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after) {
   const int H = c.hidden_size, I = c.intermediate_size, d = c.head_dim, nh = c.num_attention_heads, kvh = c.num_key_value_heads;
   const int nq = nh * d, nkv = kvh * d;
   hipStream_t st = m->stream;
-  {
+  if (!row_ready) {
     ProfScope ps(m, "elem", H * 4.0, 0);
     hipLaunchKernelGGL(embed_state_kernel, dim3(1), dim3(256), 0, st, (const bf16_t*)m->embed, m->d_state, (bf16_t*)m->d_x, H,
                        m->d_inv_freq, m->d_axis_map, m->d_rope);
@@ -1471,7 +1505,7 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after) {
       gemv_row_parallel(m, g);
     }
   }
-  enqueue_lm_head(m, m->d_x);
+  enqueue_lm_head(m, m->d_x, arg_max);
 }
 
 int model_forward_step(aha_model* m, uint32_t token, size_t offset, float* logits_out, uint32_t* argmax_out) {
@@ -1586,13 +1620,21 @@ int model_decode_greedy(aha_model* m, uint32_t first_token, size_t offset, size_
   // queues `ahead` more steps and then waits for ever in their all-reduces).  Under TP the schedule is therefore a function of the
   // token sequence alone: whole groups of `ahead` steps, the next group only after every token of the last one has been read.
   const bool lockstep = m->tp_size > 1;
+  const bool joined = !m->layered && m->lm_rows == c.vocab_size;
   while (seen < max_new && !stop) {
     size_t want = 0;
     if (!lockstep) want = enq < max_new && enq - seen < ahead ? std::min(max_new - enq, ahead - (enq - seen)) : 0;
     else if (seen == enq) want = std::min(max_new - enq, ahead);
     for (size_t i = 0; i < want; ++i) {
-      enqueue_decode_step(m, base_len + enq + 1);
-      hipLaunchKernelGGL(advance_state_kernel, dim3(1), dim3(1), 0, m->stream, m->d_state, m->d_token_log, m->h_ring_dev, m->h_done_dev);
+      enqueue_decode_step(m, base_len + enq + 1, joined && enq > 0, !joined);
+      if (joined) {
+        ProfScope ps(m, "argmax", 0, 0);
+        hipLaunchKernelGGL(next_step_kernel, dim3(1), dim3(1024), 0, m->stream, m->d_blk_max, m->d_blk_idx, gemv_num_tiles(c.vocab_size, c.hidden_size), m->d_state,
+                           (const bf16_t*)m->embed, c.vocab_size, c.hidden_size, (bf16_t*)m->d_x, m->d_inv_freq, m->d_axis_map, m->d_rope, m->d_token_log, m->h_ring_dev,
+                           m->h_done_dev);
+      } else {
+        hipLaunchKernelGGL(advance_state_kernel, dim3(1), dim3(1), 0, m->stream, m->d_state, m->d_token_log, m->h_ring_dev, m->h_done_dev);
+      }
       ++enq;
     }
     AHA_HIP_CHECK(hipGetLastError());

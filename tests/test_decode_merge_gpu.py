@@ -40,3 +40,30 @@ def test_partials_merged_by_the_projection(gpu, monkeypatch, heads, kv_heads, le
             assert float(np.abs(a - b).max()) <= LOGIT_TOL_STD * std and float(np.sqrt(((a - b) ** 2).mean())) <= LOGIT_RMS_STD * std, (S, step)
             tok = am
     merged.close(); plain.close()
+
+
+@pytest.mark.parametrize("hidden, vocab", [(256, 64), (256, 5000), (1024, 70001)])
+def test_between_two_steps(gpu, hidden, vocab):
+    """The launch between two steps of the greedy loop (arg-max, state, embedding row, rope table) against the same tokens fed one by one: the kernels
+    in between are the same, so tokens and the last logits agree exactly; fewer and more partials than threads, two calls in a row."""
+    from aha_amd.configs import tiny_qwen3
+    from aha_amd.model import HipInferenceModel
+    from aha_amd.weights import qwen3_text_weights
+    cfg = tiny_qwen3(layers=2, hidden=hidden, heads=4, kv_heads=2, inter=512, vocab=vocab)
+    m = HipInferenceModel(cfg, qwen3_text_weights(cfg, seed=2))
+    try:
+        prompt = [int(t) for t in np.random.default_rng(vocab).integers(0, vocab, 61)]
+        _, first = m.forward_initial(prompt, 0)
+        got = m.decode_greedy(first, 61, 5)
+        got += m.decode_greedy(got[-1], 66, 4)
+        last = m.last_logits()
+        m.clear_cache()
+        _, tok = m.forward_initial(prompt, 0)
+        ref = []
+        for i in range(9):
+            logits, tok = m.forward_step(tok, 61 + i)
+            ref.append(int(tok))
+        assert got == ref
+        np.testing.assert_array_equal(last, logits)
+    finally:
+        m.close()
