@@ -17,9 +17,12 @@ namespace {
 // ---- decode ----------------------------------------------------------------------------------------------------------------------
 // Block (split, kv head, sequence), four waves; wave w of split s is unit s * 4 + w and takes the chunk's pages unit, unit + units, ...
 // Every block redoes the small per-token work (sums of squares over the whole q / k projections, norm + rotation of its g query heads and of
-// the new key, the new value); split 0 appends the new key and value to the page, unit 0 scores the new token from LDS and owns the sink.
+// the new key, the new value); split 0 appends the new key and value to the page, unit 0 owns the sink, the last
+// unit begins with the new token from LDS.
 // Partials: one un-normalised (max, sum, O) per split and head, written through to memory; the split block that arrives last at the kv head's
 // counter merges them, writes the output and resets the counter.
+// What bounds it is the work in front of and behind the pages: 14.6 us at 8 sequences of ~260 positions (32 / 8 heads x 128) with the sums read by
+// elements, the last page requested twice, the new token scored behind unit 0's pages and the waves merged by dwords; 11.4 us as it is.
 // TI: type of the qkv row (float behind the decode matvec, bf16 behind a GEMM).
 constexpr int CD_NW = 4, CD_NT = CD_NW * 64;
 template <int DQK, int DV>
@@ -39,7 +42,7 @@ __global__ __launch_bounds__(CD_NT) void attn_chunk_decode_kernel(ChunkDecodeArg
   bf16_t* qs = reinterpret_cast<bf16_t*>(smem);    // [16][DQK]
   bf16_t* ksn = qs + 16 * DQK;                     // [DQK]
   bf16_t* vsn = ksn + DQK;                         // [DV]
-  float* mo = reinterpret_cast<float*>(vsn + DV);  // per wave O^T [CD_NW][DV][16]
+  float* mo = reinterpret_cast<float*>(vsn + DV);  // per wave O [CD_NW][16][DV]
   float* mm = mo + CD_NW * DV * 16;                // [CD_NW][16]
   float* mlz = mm + CD_NW * 16;                    // [CD_NW][16]
   __shared__ float red[2][CD_NW];
@@ -87,8 +90,40 @@ __global__ __launch_bounds__(CD_NT) void attn_chunk_decode_kernel(ChunkDecodeArg
     if (unit < npages) b0 = page_base(unit);
     float sq = 0.f, sk = 0.f;
     constexpr int BQ = 8;   // columns of the row requested together
+    // the row in 16-byte pieces where it lies so (every head dim that is a multiple of 8 does)
+    const bool wide = p.ld % 8 == 0 && p.k_off % 8 == 0 && nq % 8 == 0 && nk % 8 == 0 && (((uintptr_t)p.qkv | (uintptr_t)p.bias) & 15) == 0;
     auto sumsq = [&](int off, int n) {
       float s = 0.f;
+      if (wide) {
+        for (int i0 = tid * 8; i0 < n; i0 += CD_NT * 16) {
+          float v[2][8];
+          f32x4_t bi[2][2];
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const int i = off + min(i0 + j * CD_NT * 8, n - 8);
+            if constexpr (std::is_same<TI, float>::value) {
+              *reinterpret_cast<f32x4_t*>(v[j]) = *reinterpret_cast<const f32x4_t*>((const float*)row + i);
+              *reinterpret_cast<f32x4_t*>(v[j] + 4) = *reinterpret_cast<const f32x4_t*>((const float*)row + i + 4);
+            } else {
+              const u32x4_t w = ld16((const bf16_t*)row + i);
+#pragma unroll
+              for (int k = 0; k < 4; ++k) { v[j][2 * k] = lo_bf(w[k]); v[j][2 * k + 1] = hi_bf(w[k]); }
+            }
+#pragma unroll
+            for (int k = 0; k < 2; ++k) bi[j][k] = p.bias ? *reinterpret_cast<const f32x4_t*>(p.bias + i + 4 * k) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+          }
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            if (i0 + j * CD_NT * 8 < n) {
+#pragma unroll
+              for (int k = 0; k < 8; ++k) {
+                const float x = v[j][k] + bi[j][k >> 2][k & 3];
+                s = fmaf(x, x, s);
+              }
+            }
+        }
+        return s;
+      }
       for (int i0 = tid; i0 < n; i0 += CD_NT * BQ) {
         float v[BQ];
 #pragma unroll
@@ -194,9 +229,29 @@ __global__ __launch_bounds__(CD_NT) void attn_chunk_decode_kernel(ChunkDecodeArg
   f32x4_t o[DS];
 #pragma unroll
   for (int i = 0; i < DS; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  for (int page = unit; page < npages; page += nunits) {
-    const bool more = page + nunits < npages;
-    const uint64_t nb = more ? page_base(page + nunits) : page_base(page);   // (the last request is repeated, nobody reads it)
+  if (unit == nunits - 1) {   // the new token, from LDS: this unit's running state begins with it, under its page fetch
+    float d4[4] = {0.f, 0.f, 0.f, 0.f};
+    const u32x4_t* qr = reinterpret_cast<const u32x4_t*>(qs + min(c, g - 1) * DQK + G * (DQK / 4));
+    const u32x4_t* kr = reinterpret_cast<const u32x4_t*>(ksn + G * (DQK / 4));
+#pragma unroll
+    for (int j = 0; j < DQK / 32; ++j) {
+      const u32x4_t qv = qr[j], kv = kr[j];
+#pragma unroll
+      for (int x = 0; x < 4; ++x) d4[x] = fmaf(hi_bf(qv[x]), hi_bf(kv[x]), fmaf(lo_bf(qv[x]), lo_bf(kv[x]), d4[x]));
+    }
+    m = group_sum((d4[0] + d4[1]) + (d4[2] + d4[3])) * a.scale;
+    l = G == 0 ? 1.f : 0.f;
+#pragma unroll
+    for (int ds = 0; ds < DS; ++ds) {
+      const uint2 v = *reinterpret_cast<const uint2*>(vsn + ds * 16 + G * 4);
+      o[ds] = f32x4_t{lo_bf(v.x), hi_bf(v.x), lo_bf(v.y), hi_bf(v.y)};
+    }
+  }
+  int page = unit;
+  auto do_page = [&](auto more_tag) {   // MORE: the unit has another page after this one, requested as soon as the registers are free
+    constexpr bool MORE = decltype(more_tag)::value;
+    uint64_t nb = 0;
+    if (MORE) nb = page_base(page + nunits);
     f32x4_t st[4];
 #pragma unroll
     for (int sub = 0; sub < 4; ++sub) {
@@ -205,7 +260,7 @@ __global__ __launch_bounds__(CD_NT) void attn_chunk_decode_kernel(ChunkDecodeArg
       for (int k4 = 0; k4 < KS; ++k4) st[sub] = mfma16(as_frag(kf[sub][k4]), qf[k4], st[sub]);
     }
     __builtin_amdgcn_sched_barrier(0);
-    load_k(nb);
+    if (MORE) load_k(nb);
     __builtin_amdgcn_sched_barrier(0);
     float alpha;
     bf16x8_t pf[2];
@@ -218,35 +273,23 @@ __global__ __launch_bounds__(CD_NT) void attn_chunk_decode_kernel(ChunkDecodeArg
       for (int kk = 0; kk < 2; ++kk) o[ds] = mfma16(as_frag(vf[ds][kk]), pf[kk], o[ds]);
     }
     __builtin_amdgcn_sched_barrier(0);
-    load_v(nb);
+    if (MORE) load_v(nb);
     __builtin_amdgcn_sched_barrier(0);
-  }
-  if (unit == 0) {   // the new token from LDS
-    float dot = 0.f;
-    const bf16_t* qr = qs + min(c, g - 1) * DQK + G * (DQK / 4);
-    const bf16_t* kr = ksn + G * (DQK / 4);
-#pragma unroll 8
-    for (int j = 0; j < DQK / 4; ++j) dot = fmaf(bf2f(qr[j]), bf2f(kr[j]), dot);
-    const float s = group_sum(dot) * a.scale;
-    const float m_new = fmaxf(m, s);
-    const float alpha = __expf(m - m_new), pr = __expf(s - m_new);
-    const float pb = rbf(pr);   // P feeds the MFMA as bf16 on the page path: same rounding here
-    l = l * alpha + (G == 0 ? pr : 0.f);
-    m = m_new;
-#pragma unroll
-    for (int ds = 0; ds < DS; ++ds)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[ds][r] = fmaf(pb, bf2f(vsn[ds * 16 + G * 4 + r]), o[ds][r] * alpha);
+    page += nunits;
+  };
+  if (page < npages) {
+    while (page + nunits < npages) do_page(std::true_type{});
+    do_page(std::false_type{});
   }
   l = group_sum(l);
 
   // ---- merge the four waves through LDS ---------------------------------------------------------------------------------------------
   {
     float* wo = mo + wave * (DV * 16);
+    if (c < g) {
 #pragma unroll
-    for (int ds = 0; ds < DS; ++ds)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) wo[(ds * 16 + G * 4 + r) * 16 + c] = o[ds][r];
+      for (int ds = 0; ds < DS; ++ds) *reinterpret_cast<f32x4_t*>(wo + c * DV + ds * 16 + G * 4) = o[ds];
+    }
     if (G == 0) {
       mm[wave * 16 + c] = m;
       mlz[wave * 16 + c] = l;
@@ -268,8 +311,9 @@ __global__ __launch_bounds__(CD_NT) void attn_chunk_decode_kernel(ChunkDecodeArg
     for (int w = 0; w < CD_NW; ++w) {
       const float mw = mm[w * 16 + q];
       const float wt = (mw == -INFINITY) ? 0.f : __expf(mw - M);
+      const f32x4_t ow = *reinterpret_cast<const f32x4_t*>(mo + w * (DV * 16) + q * DV + d0);
 #pragma unroll
-      for (int x = 0; x < 4; ++x) acc[x] = fmaf(wt, mo[w * (DV * 16) + (d0 + x) * 16 + q], acc[x]);
+      for (int x = 0; x < 4; ++x) acc[x] = fmaf(wt, ow[x], acc[x]);
       ls = fmaf(wt, mlz[w * 16 + q], ls);
     }
     if (single) {
