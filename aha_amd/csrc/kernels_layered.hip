@@ -178,6 +178,64 @@ __global__ __launch_bounds__(NTH) void postnorm_conv_kernel(PostNormArgs a, SeqB
   }
 }
 
+// The same where every sequence brings one row, ld <= 4 * NTH: a block per row, a thread its four columns.  Eight rows are eight blocks, so the launch is
+// its chain of round trips -- entry, history, and in the general kernel one more per tap, per weight row and behind the norm (6.0 us at 8 rows of 4096
+// columns, 3 taps); here everything that the entry does not decide is requested in front of it, the history right behind: 4.1 us.
+template <typename T, int NTH, int TAPS, bool EMBED>
+__global__ __launch_bounds__(NTH) void postnorm_conv_step_kernel(PostNormArgs a, SeqBatch b) {
+  constexpr int NH = TAPS - 1;
+  __shared__ float red[NTH / 64];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ld = (int)a.ld, r = (int)blockIdx.x;
+  const bool in = wave * 256 < ld;
+  const int c = min(tid * 4, ld - 4);
+  const int ei = entry_of_row(b, r);
+  float4 v, y = make_float4(0.f, 0.f, 0.f, 0.f), nw = y, w[TAPS], hist[NH];
+  if (EMBED) {
+    v = wbf4((const bf16_t*)a.embed + (int64_t)a.ids[r] * ld, c);
+  } else {
+    v = *reinterpret_cast<const float4*>(a.x_in + (int64_t)r * ld + c);
+    if (a.y) y = Act<T>::ld4((const T*)a.y + (int64_t)r * a.ldy + c);
+    nw = wbf4(a.norm_w, c);
+  }
+#pragma unroll
+  for (int j = 0; j < TAPS; ++j) w[j] = wbf4(a.conv.w, (int64_t)j * ld + c);
+  const SeqEntry e = seq_entry_at(b, ei);
+  float* base = a.conv.hist + (int64_t)e.slot * a.conv.slot_stride + c;
+  const float* hi = base + (int64_t)e.hist_in * TAPS * ld;
+#pragma unroll
+  for (int k = 0; k < NH; ++k) {   // hist[k]: the input k + 1 tokens ago
+    hist[k] = *reinterpret_cast<const float4*>(hi + (int64_t)k * ld);
+    if (e.pos0 < k + 1) hist[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  if (EMBED) {
+    v = make_float4(v.x * a.embed_scale, v.y * a.embed_scale, v.z * a.embed_scale, v.w * a.embed_scale);
+    if (!in) v = make_float4(0.f, 0.f, 0.f, 0.f);
+  } else {
+    v = a.y ? make_float4(fmaf(a.alpha, v.x, y.x), fmaf(a.alpha, v.y, y.y), fmaf(a.alpha, v.z, y.z), fmaf(a.alpha, v.w, y.w))
+            : make_float4(a.alpha * v.x, a.alpha * v.y, a.alpha * v.z, a.alpha * v.w);
+    if (!in) v = make_float4(0.f, 0.f, 0.f, 0.f);
+    const float ss = block_sum_n<NTH>((v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w), red);
+    const float rinv = 1.0f / sqrtf(ss / (float)a.width + a.eps);
+    v = make_float4(v.x * rinv * (1.f + nw.x), v.y * rinv * (1.f + nw.y), v.z * rinv * (1.f + nw.z), v.w * rinv * (1.f + nw.w));
+  }
+  if (!in) return;
+  auto tap = [](float4& s, float4 t, float4 x) { s.x = fmaf(t.x, x.x, s.x); s.y = fmaf(t.y, x.y, s.y); s.z = fmaf(t.z, x.z, s.z); s.w = fmaf(t.w, x.w, s.w); };
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f), next = acc;   // next: the weighted sum of what the next token finds behind it
+#pragma unroll
+  for (int j = 0; j < NH; ++j) tap(acc, w[j], hist[NH - 1 - j]);
+  tap(acc, w[NH], v);
+#pragma unroll
+  for (int k = NH - 1; k >= 1; --k) tap(next, w[NH - 1 - k], hist[k - 1]);
+  tap(next, w[NH - 1], v);
+  *reinterpret_cast<float4*>(a.x_out + (int64_t)r * ld + c) = v;
+  Act<T>::st4((T*)a.h_out + (int64_t)r * ld + c, make_float4(v.x + acc.x, v.y + acc.y, v.z + acc.z, v.w + acc.w));
+  float* ho = base + (int64_t)e.hist_out * TAPS * ld;
+  *reinterpret_cast<float4*>(ho) = v;
+#pragma unroll
+  for (int k = 1; k < NH; ++k) *reinterpret_cast<float4*>(ho + (int64_t)k * ld) = hist[k - 1];
+  *reinterpret_cast<float4*>(ho + (int64_t)NH * ld) = next;
+}
+
 // The same for up to four taps, prompt-sized steps: the tile's rows and the TAPS - 1 in front of them in registers at once -- one round of loads,
 // one barrier for all the sums -- instead of row by row.  NV = 1: 4 * NTH columns.
 template <typename T, int NTH, int TAPS, int TILE>
@@ -596,6 +654,21 @@ template <typename T, bool EMBED>
 void postnorm_conv_t(const PostNormArgs& a, const SeqBatch& b, hipStream_t st) {
   // rows per block: a tile repeats the norm of its taps - 1 preceding rows, a short grid leaves CUs idle
   using std::integral_constant;
+  if (b.max_len == 1 && a.h_out && a.conv.taps >= 2 && a.conv.taps <= 4 && a.ld <= 4096) {
+    auto step = [&](auto nth, auto taps) {
+      constexpr int NTH = decltype(nth)::value, TAPS = decltype(taps)::value;
+      hipLaunchKernelGGL((postnorm_conv_step_kernel<T, NTH, TAPS, EMBED>), dim3((unsigned)b.rows), dim3(NTH), 0, st, a, b);
+    };
+    auto by_taps = [&](auto nth) {
+      if (a.conv.taps == 2) step(nth, integral_constant<int, 2>{});
+      else if (a.conv.taps == 3) step(nth, integral_constant<int, 3>{});
+      else step(nth, integral_constant<int, 4>{});
+    };
+    if (a.ld <= 1024) by_taps(integral_constant<int, 256>{});
+    else if (a.ld <= 2048) by_taps(integral_constant<int, 512>{});
+    else by_taps(integral_constant<int, 1024>{});
+    return;
+  }
   if constexpr (!EMBED) {
     if (b.max_len > 1 && a.y && a.h_out && a.conv.taps >= 2 && a.conv.taps <= 4 && a.ld <= 4096) {
       auto tiled = [&](auto nth, auto taps, auto tl) {
