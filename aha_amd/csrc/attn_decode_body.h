@@ -6,13 +6,13 @@
 namespace aha {
 
 constexpr int ATTN_DECODE_NW = 4;  // waves (= KV units) per workgroup
-constexpr int ATTN_DECODE_FUSED_LDS = 16 * 128 * 2 + 128 * 2 + 128 * 2 + ATTN_DECODE_NW * 128 * 16 * 4 + 2 * ATTN_DECODE_NW * 16 * 4;  // bytes
+constexpr int ATTN_DECODE_FUSED_LDS = 16 * 128 * 2 + 128 * 2 + 128 * 2 + ATTN_DECODE_NW * 128 * 16 * 4 + (2 * ATTN_DECODE_NW + 1) * 16 * 4;  // bytes
 
 // ---- decode, fused: q/k RMSNorm + (M-)RoPE + KV append + split-KV attention + in-block merge --------------------
 // One launch replaces qknorm_rope_kernel + attn_decode_kernel + the combine: every block redoes the (tiny) norm/rope of
 // its kv head's g query heads and of the new key in LDS (QKNormAttention::forward, modules.rs:538-557), block (kvhd, 0)
 // appends the new K/V to the cache page (modules.rs:558-566), all blocks attend over the OLD tokens from the pages, the
-// last unit begins with the new token from LDS, the 4 waves of a block are merged through LDS, one un-normalised partial per
+// 4 waves of a block are merged through LDS (the new token's share, from LDS, with those of the last split), one un-normalised partial per
 // (split, head) is published, and the LAST split block of the kv head to arrive merges the splits and writes the bf16
 // attention output.
 //
@@ -39,6 +39,7 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
   float* mo = reinterpret_cast<float*>(vsn + 128);              // per wave O [NW][q P][d 128]
   float* mm = mo + NW * 128 * P;                                // [NW][16]
   float* mlz = mm + NW * 16;                                    // [NW][16]
+  float* snew = mlz + NW * 16;                                  // [16]: the new token's scores (blocks of the last split)
   const int tid = (int)threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, G = lane >> 4, c = lane & 15;
@@ -162,8 +163,9 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
 #pragma unroll
   for (int i = 0; i < 8; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  // The new token, from LDS: the running state of the last unit (never the one with the most pages) begins with it, under the unit's page fetch.
-  // (Behind unit 0's pages, and with the waves' sums merged by dwords, the part after the pages was 1.49 us of the slowest block; 0.57 now.)
+  // The new token's scores, by the last unit (never the one with the most pages): the merge of the waves takes the token in as a share of its own, so
+  // the pages' shares do not depend on where it is.  (Behind unit 0's pages, and with the waves' sums merged by dwords, what followed the pages was
+  // 1.49 us of the slowest block; 0.6 now.  At the head of unit 0 it cost 0.4 us in front of the first page.)
   if (unit == nunits - 1) {
     float d4[4] = {0.f, 0.f, 0.f, 0.f};
     const u32x4_t* qr = reinterpret_cast<const u32x4_t*>(qs + min(c, g - 1) * 128 + G * 32);
@@ -174,13 +176,8 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
 #pragma unroll
       for (int e = 0; e < 4; ++e) d4[e] = fmaf(hi_bf(qv[e]), hi_bf(kv[e]), fmaf(lo_bf(qv[e]), lo_bf(kv[e]), d4[e]));
     }
-    m = rbf(rbf(group_sum((d4[0] + d4[1]) + (d4[2] + d4[3]))) * a.scale);
-    l = G == 0 ? 1.f : 0.f;
-#pragma unroll
-    for (int ds = 0; ds < 8; ++ds) {
-      const uint2 v = *reinterpret_cast<const uint2*>(vsn + ds * 16 + G * 4);
-      o[ds] = f32x4_t{lo_bf(v.x), hi_bf(v.x), lo_bf(v.y), hi_bf(v.y)};
-    }
+    const float s = rbf(rbf(group_sum((d4[0] + d4[1]) + (d4[2] + d4[3]))) * a.scale);
+    if (G == 0) snew[c] = s;
   }
 
   // One page of this unit.  MORE (compile time): the unit has another page after this one -- its K is requested right
@@ -245,10 +242,16 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
   const auto rsrc_w = __builtin_amdgcn_make_buffer_rsrc(a.part_o, 0, (int)((size_t)nsplit * a.nh * 128 * 4), 0x00020000);
   for (int item = tid; item < g * 32; item += NT) {
     const int q = item >> 5, d0 = (item & 31) * 4;
-    float M = -INFINITY;
+    const bool own = split == nsplit - 1;   // the new token is this block's
+    float M = own ? snew[q] : -INFINITY;
 #pragma unroll
     for (int w = 0; w < NW; ++w) M = fmaxf(M, mm[w * 16 + q]);
     float acc[4] = {0.f, 0.f, 0.f, 0.f}, ls = 0.f;
+    if (own) {
+      const uint2 v = *reinterpret_cast<const uint2*>(vsn + d0);
+      ls = __expf(snew[q] - M);
+      acc[0] = ls * lo_bf(v.x), acc[1] = ls * hi_bf(v.x), acc[2] = ls * lo_bf(v.y), acc[3] = ls * hi_bf(v.y);
+    }
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
       const float mw = mm[w * 16 + q];

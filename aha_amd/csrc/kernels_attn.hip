@@ -176,7 +176,7 @@ int attn_decode_defer_splits(int npages, int nq) {
   return nq > 2048 && npages <= 4 ? 1 : std::min((npages + 1) / 2, most);
 }
 void launch_attn_decode_defer(const AttnDecodeFusedArgs& a, hipStream_t st) {
-  const int lds = 16 * 128 * 2 + 2 * 128 * 2 + ATTN_DECODE_NW * 128 * (a.nh / a.kvh) * 4 + 2 * ATTN_DECODE_NW * 16 * 4;
+  const int lds = 16 * 128 * 2 + 2 * 128 * 2 + ATTN_DECODE_NW * 128 * (a.nh / a.kvh) * 4 + (2 * ATTN_DECODE_NW + 1) * 16 * 4;
   hipLaunchKernelGGL(attn_decode_defer_kernel, dim3(a.kvh, a.nsplit), dim3(256), lds, st, a);
 }
 
