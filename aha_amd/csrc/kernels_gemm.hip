@@ -1306,7 +1306,7 @@ void launch_gemm(const GemmArgs& a_in, hipStream_t st) {
   if (g_force_tile == 0 && !plan_from_env() && gemm_skinny_ok(a)) {
     int r8;
     const double tiled = std::max(plan.cost, (double)a.N * a.K * 2.0 / 4.2e6 + (plan.splitk > 1 ? 5.0 : 2.0));
-    if (gemm_skinny_plan(a, &r8) < tiled) {
+    if (gemm_skinny_plan(a, &r8) + (a.norm_w && plan.splitk > 1 ? 3.0 : 0.0) < tiled) {   // (a norm that the reduce pass would have taken along: its own launch)
       launch_gemm_skinny(a, st);
       if (a.norm_w) launch_riding_norm(a, st);
       return;

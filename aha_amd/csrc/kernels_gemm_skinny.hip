@@ -1,4 +1,4 @@
-// Projection GEMM for few rows (M <= 64: batched decode steps, short prompts): C[M,N] = A[M,K] . W[N,K]^T with the epilogues of kernels_gemm.hip.
+// Projection GEMM for few rows (M <= 64: batched decode steps, short prompts; to 256 where row tiles of 64 fit into one round): C[M,N] = A[M,K] . W[N,K]^T with the epilogues of kernels_gemm.hip.
 //
 // What bounds it is the weight matrix, read once from HBM; the 128-row tiles of kernels_gemm.hip stage 16 times the rows a batch of eight has and
 // need K slices and a reduce pass to fill the chip.  Here a block owns R8 * 8 weight rows and the whole K range, its four waves take the 64-wide
@@ -13,6 +13,10 @@
 // Measured on MI355X, back to back from HBM, 8 rows (in brackets: the split-K ring kernel + its reduce pass it replaces, inside a batched step):
 //   6144 x 4096 10.4 us (4.8 TB/s), 4096 x 4096 8.1, 12288 x 4096 18.0 (5.6), 4096 x 12288 17.9 (5.6), 24576 x 4096 33.1 (6.1)
 //   [18.1 + 4.6 us on average over the first four]; 32 rows: 12.1, 10.1, 19.7, 25.9, 37.2; 64 rows: 15.5, 13.4, 23.3, 35.5, 45.9
+//   64-row tiles, 96 / 128 rows (tiled kernels with their reduce pass): 4096 x 1024 6.7 / 6.9 us (10.7 / 10.7), 6144 x 1024 8.5 / 8.6 (12.1 / 12.9),
+//   1024 x 2048 7.0 / 7.7 (11.3 / 12.1), 1024 x 3072 9.0 / 10.2 (12.3 / 13.2); a 0.6B prompt of 96 / 128 / 180 / 250 tokens 1.66 / 1.67 / 1.95 / 2.03 ms
+//   (1.97 / 2.06 / 2.07 / 2.14), of 300 2.14 (2.09): 256 rows at most.  The 8B shapes stay on the tiles:
+//   their weight rows need more than one round or a longer K than a block streams in the tiles' time (6144 x 4096, 96 rows: 21.3 against 21.0).
 #include "gemm256_body.h"
 #include "skinny_body.h"
 
@@ -29,7 +33,7 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(GemmArgs
   for (int r = 0; r < PER; ++r) {
     const int local = (r < R8 ? r : r - R8) * 8 + (lane >> 3), piece = skinny_piece(local, lane);
     if (r >= R8) {
-      src[r] = (const char*)a.A + (int64_t)min(local, a.M - 1) * a.lda * 2 + piece;
+      src[r] = (const char*)a.A + (int64_t)min((int)blockIdx.y * 64 + local, a.M - 1) * a.lda * 2 + piece;
     } else if (PAIRS) {   // eight gate rows, then the eight up rows of the same columns (16-row blocks alternate in W)
       const int col = ((int)blockIdx.x * (R8 / 2) + r / 2) * 8 + (lane >> 3);
       src[r] = (const char*)a.W + (int64_t)min((col >> 4) * 32 + (r & 1) * 16 + (col & 15), a.N - 1) * a.ldw * 2 + piece;
@@ -39,7 +43,7 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(GemmArgs
   }
   skinny_sums<R8, M8>(src, a.K / 64, gemm_smem, wave, lane);
   for (int i = wave; i < NF * MT; i += SKINNY_WAVES) {
-    const int r = i / MT, m = (i - r * MT) * 16 + c;
+    const int r = i / MT, m = (int)blockIdx.y * 64 + (i - r * MT) * 16 + c;
     if (m >= a.M) continue;
     if constexpr (PAIRS) {   // rows 0-7 of a fragment: gate, 8-15: up
       if (G >= 2) continue;
@@ -72,7 +76,7 @@ void launch_one(const GemmArgs& a, hipStream_t st) {
   constexpr int lds = skinny_lds(R8, M8);
   if (lds > 64 * 1024)
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_skinny_kernel<R8, M8, PAIRS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  hipLaunchKernelGGL((gemm_skinny_kernel<R8, M8, PAIRS>), dim3((unsigned)((a.N + R8 * 8 - 1) / (R8 * 8))), dim3(SKINNY_WAVES * 64), lds, st, a);
+  hipLaunchKernelGGL((gemm_skinny_kernel<R8, M8, PAIRS>), dim3((unsigned)((a.N + R8 * 8 - 1) / (R8 * 8)), (unsigned)((a.M + 63) / 64)), dim3(SKINNY_WAVES * 64), lds, st, a);
 }
 
 template <int R8, bool PAIRS>
@@ -92,7 +96,9 @@ double gemm_skinny_plan(const GemmArgs& a, int* r8_out) {
   double best = 1e30;
   for (int r8 : {2, 3, 4, 6}) {
     if (a.act == ACT_SILU_MUL_PAIRS && r8 == 3) continue;   // (gate and up rows in eights)
-    const double rounds = ceil(((a.N + r8 * 8 - 1) / (r8 * 8)) / 256.0), c = 3.0 + rounds * (r8 + 0.4 * m8) * a.K * 16.0 / 30e3;
+    const double rounds = ceil(((a.N + r8 * 8 - 1) / (r8 * 8)) * ((a.M + 63) / 64) / 256.0);
+    if (a.M > 64 && rounds > 1) continue;   // (4096 x 1024, 180 rows, 384 blocks: 12.0 us against 10.9 of the tiles)
+    const double c = 3.0 + rounds * (r8 + 0.4 * m8) * a.K * 16.0 / 30e3;
     if (c < best) {
       best = c;
       *r8_out = r8;
@@ -103,12 +109,12 @@ double gemm_skinny_plan(const GemmArgs& a, int* r8_out) {
 
 // K < 768 stays with the tiled kernels: they run unsplit there, so a row's bits do not depend on how many rows share the call (row slices of a
 // sequence-parallel prompt), for 1.5 to 4 us more per launch (K = 256: 5.1 against 2.7 us, 512: 6.8 against 3.0, 768: 8.5 against 3.3; 8 rows, 2048
-// columns).  So do 33 to 64 rows of a matrix below 2 MB (512 x 1024: 10.2 against 5.2 us).  Only small models have either -- the full-size ones have
+// columns).  So do 33 to 64 rows of a matrix below 2 MB (512 x 1024: 10.2 against 5.2 us) and more rows of one below 4 MB.  Only small models have either -- the full-size ones have
 // K >= 768 throughout their text stacks, and their one small matrix, the router, is met by 33 to 64 rows only in that band -- and they keep the
 // results they had.
 bool gemm_skinny_ok(const GemmArgs& a) {
-  return a.few_rows && a.M >= 1 && a.M <= 64 && a.K >= 768 && a.K % 64 == 0 && a.N % 8 == 0 && a.groups == 1 && (a.act != ACT_SILU_MUL_PAIRS || a.N % 32 == 0) &&
-         (a.M <= 32 || (int64_t)a.N * a.K >= 1 << 20);
+  return a.few_rows && a.M >= 1 && a.M <= 256 && a.K >= 768 && a.K % 64 == 0 && a.N % 8 == 0 && a.groups == 1 && (a.act != ACT_SILU_MUL_PAIRS || a.N % 32 == 0) &&
+         (a.M <= 32 || (int64_t)a.N * a.K >= (a.M <= 64 ? 1 << 20 : 1 << 21));
 }
 
 void launch_gemm_skinny(const GemmArgs& a, hipStream_t st) {

@@ -44,3 +44,19 @@ def test_few_rows_gate_up_pairs(gpu, M, I, K):
     ref = NM.r(NM.r(oq.silu(NM.linear(A.float(), Wg.float()))) * NM.linear(A.float(), Wu.float()))
     got = ops.gemm(A.to(gpu), ops.interleave_gate_up(Wg, Wu).to(gpu), None, None, _lib.ACT_SILU_MUL_PAIRS)
     assert_close_ulps(got, ref, 3, None, "gate * up")
+
+
+@pytest.mark.parametrize("M", [65, 128, 129, 256])
+@pytest.mark.parametrize("N,K,pairs", [(1024, 2048, False), (2056, 1088, False), (2720, 832, True)])
+def test_row_tiles(gpu, M, N, K, pairs):
+    """More than 64 rows in tiles of 64: the first and last of a tile, the last row count that comes here; bounds as above."""
+    from aha_amd import ops, _lib
+    A, W = rnd((M, K), 71), rnd((N, K), 72, 0.05)
+    if pairs:
+        ref = NM.r(NM.r(oq.silu(NM.linear(A.float(), W[:N // 2].float()))) * NM.linear(A.float(), W[N // 2:].float()))
+        assert_close_ulps(ops.gemm(A.to(gpu), ops.interleave_gate_up(W[:N // 2], W[N // 2:]).to(gpu), None, None, _lib.ACT_SILU_MUL_PAIRS), ref, 3, None, "gate * up")
+        return
+    b, r = rnd((N,), 73, 0.5), rnd((M, N), 74)
+    assert_close_ulps(ops.gemm(A.to(gpu), W.to(gpu)), NM.linear(A.float(), W.float()), 1, None, "plain")
+    full = ops.gemm(A.to(gpu), W.to(gpu), b.to(gpu), r.to(gpu), _lib.ACT_NONE)
+    assert_close_ulps(full, NM.r(r.float() + NM.linear(A.float(), W.float(), b.float())), 2, None, "bias + residual")
