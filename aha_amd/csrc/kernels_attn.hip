@@ -168,7 +168,9 @@ void launch_attn_decode_fused(const AttnDecodeFusedArgs& a, hipStream_t st) {
 // How many partials (0: the merge belongs inside the launch).  A CU streams ~56 bytes per ns here, half a microsecond per page of a kv head, so two
 // pages per block while the partials last; every partial costs the o_proj matvec another 4 bytes per column and block from L2 (0.6B widths: +0.2 us
 // for 4, +0.6 us for 8; 8B widths: +2.1 us for 4, so nothing is split there before a block has more than four pages).
-// At six pages per block the launch that merges by itself is as fast.
+// At six pages per block the launch that merges by itself is as fast.  Attention + o_proj before (merge by the last block) and with the deferred merge:
+// 14.5 -> 10.5 us at 450 positions and 14.9 -> 13.7 at 2200 of 0.6B, 18.6 -> 18.0 at 900 of 8B; with the new token and the waves' sums as they are now
+// (attn_decode_body.h) another 0.9 less.
 int attn_decode_defer_splits(int npages, int nq) {
   if (nq > 4096) return 0;   // (the prologue holds the partials of 4096 columns in registers)
   const int most = nq <= 2048 ? 8 : 4;
