@@ -1,5 +1,6 @@
 // Row-wise / index kernels of the Qwen3 decoder stack: embedding gather (D0), RMSNorm rows (D3),
 // q/k-norm + rotary + KV append (D4/D5/D6, M1), argmax (D11).  All HBM-bound: 16-byte accesses, one wave per row.
+#include "argmax.h"
 #include "common.h"
 #include "kernels.h"
 

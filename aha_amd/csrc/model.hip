@@ -13,6 +13,7 @@
 #include <algorithm>
 #include <chrono>
 
+#include "argmax.h"
 #include "common.h"
 #include "audio.h"
 #include "layered.h"
