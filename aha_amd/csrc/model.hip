@@ -1720,7 +1720,7 @@ int model_embed_multi(aha_model* m, const uint32_t* ids, const uint64_t* lens, s
     set_error("embed: out or lens is null, or there are no documents");
     return AHA_ERR_INVALID;
   }
-  if (m->desc.arch != AHA_ARCH_QWEN3) return model_embed(m, ids, 0, out);   // (the refusal)
+  if (!ids || m->desc.arch != AHA_ARCH_QWEN3) return model_embed(m, ids, 0, out);   // (the refusal)
   const int H = m->desc.hidden_size;
   const bool joint = m->tp_size <= 1 && m->cp_size <= 1 && m->desc.head_dim == 128 && attn_prefill_takes_seqs(m->attn_scale);
   auto padded = [](size_t n) { return (n + KV_PAGE_TOKENS - 1) / KV_PAGE_TOKENS * KV_PAGE_TOKENS; };

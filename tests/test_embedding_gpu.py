@@ -76,6 +76,20 @@ def test_embed_errors(pair):
         m.embed_one([cfg.vocab_size])
 
 
+def test_documents_without_ids_are_refused(pair):
+    """aha_hip_embed_multi with a null id array, whatever the lengths say, as aha_hip_embed refuses it; nothing is written."""
+    import ctypes as C
+    from aha_amd._lib import lib
+    cfg, m, _ = pair
+    out = np.full((3, cfg.hidden_size), 7, dtype=np.float32)
+    fp, up = C.POINTER(C.c_float), C.POINTER(C.c_uint64)
+    for lens in ([5, 9, 2], [1, 4, 4], [0, 0, 0]):
+        n = np.array(lens, dtype=np.uint64)
+        one = lib().aha_hip_embed(m.handle, None, lens[0], out.ctypes.data_as(fp))
+        assert lib().aha_hip_embed_multi(m.handle, None, n.ctypes.data_as(up), 3, out.ctypes.data_as(fp)) == one == -1
+    assert (out == 7).all() and m.cache_len() == 0
+
+
 @pytest.mark.parametrize("heads, kv_heads", [(4, 2), (16, 8)])
 def test_documents_together(gpu, heads, kv_heads):
     """embed_multi's joint prefill, document lengths around a cache page (64) and around the rows that one prefill takes (4096), with one-token documents
