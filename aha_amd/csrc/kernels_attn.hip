@@ -190,6 +190,10 @@ void set_attn_form_override(int form) { g_attn_form_override = form; }
 // The kernel form launch_attn_prefill picks for these arguments: 0 = this file's 16-rows-per-wave kernel, 64 / 65 = kernels_attn64.hip
 static int attn_prefill_form(const AttnPrefillArgs& a, int smx);
 static int attn_prefill_smx(const AttnPrefillArgs& a);
+static int attn_form_asked() {   // set_attn_form_override, else AHA_ATTN_FORM; -1 = automatic
+  static const int form_env = [] { const char* e = getenv("AHA_ATTN_FORM"); return e ? atoi(e) : -1; }();
+  return g_attn_form_override >= 0 ? g_attn_form_override : form_env;
+}
 static int attn_prefill_smx(const AttnPrefillArgs& a) {
   static const int smx_env = [] { const char* e = getenv("AHA_ATTN_SMX"); return e ? atoi(e) : 3; }();
   union { float f; uint32_t u; } sb;
@@ -204,8 +208,7 @@ static int attn_prefill_form(const AttnPrefillArgs& a, int smx) {
   // The kernel form.  AHA_ATTN_FORM / set_attn_form_override: 16 = this file's 16-rows-per-wave kernel, 64 = the one-wave-per-SIMD kernel
   // with 64 rows per wave (kernels_attn64.hip) with a tile's parts in program order, 65 = the same software-pipelined inside the wave;
   // unset = automatic: form 65 (f32 chain only) once its 256-row blocks fill the chip.
-  static const int form_env = [] { const char* e = getenv("AHA_ATTN_FORM"); return e ? atoi(e) : -1; }();
-  const int form = g_attn_form_override >= 0 ? g_attn_form_override : form_env;
+  const int form = attn_form_asked();
   if (smx != 3 || form == 16) return 0;
   const int64_t blocks64 = (a.rows_hint > 0 ? (int64_t)(a.rows_hint + 255) / 256 : (int64_t)((a.S + 255) / 256 + (a.S2 + 255) / 256)) * a.nh;
   // One 4-wave workgroup per CU: a full launch is rounds of 256 workgroups.  Same-box A/B against the 16-row kernel (scripts/attn64_ab.py,
@@ -222,7 +225,7 @@ static int attn_prefill_form(const AttnPrefillArgs& a, int smx) {
 bool attn_prefill_takes_seqs(float scale) {
   AttnPrefillArgs a{};
   a.scale = scale;
-  return attn_prefill_smx(a) == 3 && g_attn_form_override < 0;
+  return attn_prefill_smx(a) == 3 && attn_form_asked() < 0;
 }
 bool attn_prefill_takes_qfuse(const AttnPrefillArgs& a) {
   static const bool on = [] { const char* e = getenv("AHA_ATTN_QFUSE"); return e ? atoi(e) != 0 : true; }();

@@ -112,3 +112,32 @@ def test_documents_together(gpu, heads, kv_heads):
                 m.embed_multi(bad)
     finally:
         m.close()
+
+
+@pytest.mark.parametrize("how", ["environment", "hook"])
+def test_documents_one_by_one_in_a_form_that_was_asked_for(gpu, how):
+    """AHA_ATTN_FORM (read once per process: a child) and aha_hip_debug_attn_form name the attention kernel of every prefill: no joint one, the vectors of
+    embed_one bit for bit."""
+    import os
+    import subprocess
+    import sys
+    code = """
+import numpy as np
+from aha_amd._lib import lib
+from aha_amd.model import HipInferenceModel
+from tests.test_embedding_gpu import qwen3_text_weights, seqs_for, tiny_qwen3
+cfg = tiny_qwen3(layers=2, hidden=256, heads=4, kv_heads=2, inter=512, vocab=2048)
+m = HipInferenceModel(cfg, qwen3_text_weights(cfg, seed=1))
+docs = seqs_for(cfg, [300, 129, 200], 5)
+if %r == "hook":
+    lib().aha_hip_debug_attn_form(64)
+np.testing.assert_array_equal(m.embed_multi(docs), np.stack([m.embed_one(x) for x in docs]))
+m.close()
+""" % how
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    env = dict(os.environ, PYTHONPATH=root)
+    env.pop("AHA_ATTN_FORM", None)
+    if how == "environment":
+        env["AHA_ATTN_FORM"] = "64"
+    r = subprocess.run([sys.executable, "-c", code], cwd=root, env=env, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
