@@ -276,6 +276,14 @@ int aha_hip_get_profile(aha_model* m, const char* kernel_class, double* total_ms
   if (flops) *flops = a.flops;
   return AHA_OK;
 }
+int aha_hip_debug_memory_limit(aha_model* m, size_t bytes) {
+  if (!m) {
+    set_error("null model");
+    return AHA_ERR_INVALID;
+  }
+  m->mem_left = bytes;
+  return AHA_OK;
+}
 int aha_hip_debug_scramble_pages(aha_model* m, int enable) {
   if (!m) return AHA_ERR_INVALID;
   m->scramble_pages = enable != 0;

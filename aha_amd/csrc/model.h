@@ -177,6 +177,8 @@ struct aha_model {
   size_t gemm_ws_bytes = 0;
   void* d_sk_ctrs = nullptr;    // SK_MAX_COUNTERS zeroed u32: per-tile arrival counters of the persistent GEMM kernel (kernels_gemm_sk.hip)
   std::vector<void*> pf_owned;
+  size_t pf_bytes = 0;           // what pf_owned holds
+  size_t mem_left = SIZE_MAX;    // aha_hip_debug_memory_limit
   // vision tower (Qwen3-VL)
   aha::VisionModel* vision = nullptr;
   // audio tower (Qwen3-ASR)

@@ -70,6 +70,14 @@ int prof_collect(aha_model* m) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
+// hipMalloc of what grows with requests (cache slabs, prefill scratch), within aha_hip_debug_memory_limit
+static hipError_t limited_malloc(aha_model* m, void** p, size_t bytes) {
+  if (bytes > m->mem_left) return hipErrorOutOfMemory;
+  const hipError_t e = hipMalloc(p, bytes);
+  if (e == hipSuccess) m->mem_left -= bytes;
+  return e;
+}
+
 int dev_alloc(aha_model* m, size_t bytes, void** out, bool zero) {
   void* p = nullptr;
   hipError_t e = hipMalloc(&p, bytes ? bytes : 16);
@@ -294,7 +302,7 @@ static int upload_gate_up(aha_model* m, const aha_tensor_view* g, const aha_tens
 int alloc_slab(aha_model* m) {
   void* p = nullptr;
   const size_t bytes = m->slab_bytes;
-  hipError_t e = hipMalloc(&p, bytes);
+  hipError_t e = limited_malloc(m, &p, bytes);
   if (e != hipSuccess) {
     set_error("KV slab hipMalloc of " + std::to_string(bytes) + " bytes failed: " + hipGetErrorString(e));
     return e == hipErrorOutOfMemory ? AHA_ERR_OOM : AHA_ERR_HIP;
@@ -811,24 +819,30 @@ void model_destroy(aha_model* m) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-static int ensure_prefill_scratch(aha_model* m, size_t S) {
-  if (S <= m->pf_cap) return AHA_OK;
+static int free_prefill_scratch(aha_model* m) {
   AHA_HIP_CHECK(hipStreamSynchronize(m->stream));
   for (void* p : m->pf_owned) hipFree(p);
   m->pf_owned.clear();
-  m->pf_cap = 0;
+  m->mem_left += m->pf_bytes;
+  m->pf_bytes = m->pf_cap = 0;
+  return AHA_OK;
+}
+static int ensure_prefill_scratch(aha_model* m, size_t S) {
+  if (S <= m->pf_cap) return AHA_OK;
+  if (int e = free_prefill_scratch(m)) return e;
   const aha_model_desc& c = m->desc;
   const size_t cap = (S + 255) / 256 * 256;
   const size_t H = c.hidden_size, I = c.intermediate_size, nq = (size_t)c.num_attention_heads * c.head_dim,
                nkv = (size_t)c.num_key_value_heads * c.head_dim;
   auto al = [&](size_t bytes, void** out) -> int {
     void* p = nullptr;
-    hipError_t e = hipMalloc(&p, bytes);
+    hipError_t e = limited_malloc(m, &p, bytes);
     if (e != hipSuccess) {
       set_error(std::string("prefill scratch hipMalloc failed: ") + hipGetErrorString(e));
       return e == hipErrorOutOfMemory ? AHA_ERR_OOM : AHA_ERR_HIP;
     }
     m->pf_owned.push_back(p);
+    m->pf_bytes += bytes;
     *out = p;
     return AHA_OK;
   };
@@ -1713,7 +1727,8 @@ int model_embed(aha_model* m, const uint32_t* ids, size_t n, float* out) {
 // eight documents of 75 to 600 tokens were 15.9 ms one by one, 3.9 ms together.  Each begins on a cache page of its own (its rows are padded to
 // whole pages by repeating its last token, behind everything its last position sees), so row = cache slot as in any prefill and only the attention
 // knows about documents.  4096 rows fill the chip with the narrowest GEMM (N = 1024: 256 tiles); a document alone, of one token (a decode step) or
-// longer than that runs as before, and so does everything where the joint prefill finds no memory.
+// longer than that runs as before, and so does everything where the joint prefill finds no memory: its scratch, larger than a single document's, is
+// given back first.
 constexpr size_t EMBED_ROWS = 4096;
 int model_embed_multi(aha_model* m, const uint32_t* ids, const uint64_t* lens, size_t n_docs, float* out) {
   if (!out || !lens || n_docs == 0) {
@@ -1722,7 +1737,7 @@ int model_embed_multi(aha_model* m, const uint32_t* ids, const uint64_t* lens, s
   }
   if (!ids || m->desc.arch != AHA_ARCH_QWEN3) return model_embed(m, ids, 0, out);   // (the refusal)
   const int H = m->desc.hidden_size;
-  const bool joint = m->tp_size <= 1 && m->cp_size <= 1 && m->desc.head_dim == 128 && attn_prefill_takes_seqs(m->attn_scale);
+  bool joint = m->tp_size <= 1 && m->cp_size <= 1 && m->desc.head_dim == 128 && attn_prefill_takes_seqs(m->attn_scale);
   auto padded = [](size_t n) { return (n + KV_PAGE_TOKENS - 1) / KV_PAGE_TOKENS * KV_PAGE_TOKENS; };
   for (size_t d = 0, pos = 0; d < n_docs;) {
     std::vector<SeqEntry> docs;
@@ -1753,6 +1768,8 @@ int model_embed_multi(aha_model* m, const uint32_t* ids, const uint64_t* lens, s
       }
       if (rc != AHA_ERR_OOM) return rc;
       (void)hipGetLastError();
+      joint = false;   // (the rest one by one too)
+      if ((rc = free_prefill_scratch(m))) return rc;
     }
     if (int rc = model_embed(m, ids + pos, lens[d], out + d * H)) return rc;
     pos += lens[d++];

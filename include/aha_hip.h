@@ -399,6 +399,9 @@ int aha_hip_get_profile(aha_model* m, const char* kernel_class, double* total_ms
                         double* flops);
 /* Debug knob for the paged-KV property tests: 1 => hand out physical pages in a scrambled order. */
 int aha_hip_debug_scramble_pages(aha_model* m, int enable);
+/* Test hook: how many more bytes this model's cache slabs and prefill scratch may take before they fail with AHA_ERR_OOM (scratch that is freed
+ * counts back); a new model has no limit. */
+int aha_hip_debug_memory_limit(aha_model* m, size_t bytes);
 /* Copies the last hidden state before lm_head (hidden_size floats) / the image embeddings of the last
  * forward_initial (rows x out_hidden floats) to the host, for parity tests of intermediate tensors. */
 int aha_hip_debug_last_hidden(aha_model* m, float* out, size_t n);

@@ -141,3 +141,29 @@ m.close()
         env["AHA_ATTN_FORM"] = "64"
     r = subprocess.run([sys.executable, "-c", code], cwd=root, env=env, capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, r.stderr[-2000:]
+
+
+def test_documents_in_little_memory(gpu):
+    """Whatever memory is left: documents that fit one by one are embedded together or one by one, never refused (the joint prefill's scratch, larger
+    than a single document's, may leave no room for the cache slab that both need)."""
+    from aha_amd._lib import AhaHipError, check, lib
+    from aha_amd.model import HipInferenceModel
+    cfg = tiny_qwen3(layers=2, hidden=256, heads=4, kv_heads=2, inter=512, vocab=2048)
+    w = qwen3_text_weights(cfg, seed=1)
+    docs = seqs_for(cfg, [900] * 4 + [30], 5)
+    outcomes = set()
+    for limit in range(8 << 20, 120 << 20, 4 << 20):
+        alone, together = [], []
+        for out, call in ((alone, lambda m: np.stack([m.embed_one(x) for x in docs])), (together, lambda m: m.embed_multi(docs))):
+            m = HipInferenceModel(cfg, w)
+            check(lib().aha_hip_debug_memory_limit(m.handle, limit))
+            try:
+                out.append(call(m))
+            except AhaHipError as e:
+                assert "hipMalloc" in str(e)
+            m.close()
+        assert len(alone) <= len(together), limit
+        outcomes.add((len(alone), len(together)))
+        if alone:
+            assert float((alone[0] * together[0]).sum(1).min()) >= 0.9995
+    assert outcomes == {(0, 0), (1, 1)}   # the limits range from too little for a document to room for all
