@@ -102,7 +102,7 @@ __global__ __launch_bounds__(64 * S1_WAVES_PER_BLOCK) void topk_stage1_kernel(co
 #pragma unroll
   for (int j = 0; j < S1_C; ++j)
     if (id[j] != NO_IDX) s += __expf((v[j] - wm) * inv_temp);
-  s = wave_sum(s);
+  s = wm == -INFINITY ? 0.f : wave_sum(s);   // (a wave of -inf only: nothing, not the NaN of (-inf) - (-inf))
   if (lane == 0) {
     part_m[w] = wm;
     part_s[w] = s;
@@ -141,7 +141,7 @@ __global__ __launch_bounds__(64 * S1_WAVES_PER_BLOCK) void topk_heads_kernel(con
 #pragma unroll
   for (int j = 0; j < S1_C; ++j)
     if (base + j * 64 + lane < V) s += __expf((v[j] - wm) * inv_temp);
-  s = wave_sum(s);
+  s = wm == -INFINITY ? 0.f : wave_sum(s);   // (a wave of -inf only: nothing, not the NaN of (-inf) - (-inf))
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     const uint64_t other = __shfl_xor(best, o, 64);

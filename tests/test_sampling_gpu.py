@@ -175,3 +175,31 @@ def test_where_the_candidates_lie(gpu, vocab):
                 assert np.float32(mx) == np.float32(rmx) and abs(se - rse) <= 2e-5 * rse
     finally:
         m.close()
+
+
+@pytest.mark.parametrize("vocab,ks", [(513, (1, 20, 64)), (262144, (1, 20, 40)), (262145, (1, 20, 39))])
+def test_a_wave_of_minus_infinity(gpu, vocab, ks):
+    """A last wave of one entry that is -inf (vocabularies of 513 and 262145) adds nothing to the normaliser.  262144 entries are the most that the
+    launches of topk_heads_kernel take, 262145 the fewest for the rounds over all candidates (whose second stage holds 20480: k <= 39 there)."""
+    cfg, m = make(vocab)
+    try:
+        last = np.arange((vocab - 1) // 512 * 512, vocab)
+        for seed in range(40):   # a prompt whose last logit is negative: an infinite penalty makes it -inf
+            m.clear_cache()
+            logits, _ = m.forward_initial([int(t) for t in np.random.default_rng(seed).integers(0, vocab, 3)], 0)
+            if logits[-1] < 0:
+                break
+        neg = [int(i) for i in last[logits[last] < 0]]
+        assert neg
+        for ctx in ([neg[-1]], neg, [3, neg[-1], 5]):
+            for k in ks:
+                vals, idx, mx, se = m.sample_candidates(ctx, float("inf"), 0.9, k)
+                rv, ri, rmx, rse = osamp.topk_candidates(osamp.apply_repeat_penalty(logits, float("inf"), ctx), k, 0.9)
+                np.testing.assert_array_equal(idx, ri)
+                np.testing.assert_array_equal(vals.view(np.uint32), rv.view(np.uint32))
+                assert np.float32(mx) == np.float32(rmx) and abs(se - rse) <= 2e-5 * rse
+        if vocab > 262144:
+            with pytest.raises(_lib.AhaHipError):
+                m.sample_candidates([], 1.0, 1.0, ks[-1] + 1)
+    finally:
+        m.close()
