@@ -119,8 +119,10 @@ __global__ __launch_bounds__(64 * S1_WAVES_PER_BLOCK) void topk_stage1_kernel(co
 // heads: every wave's largest entry and softmax partial; rounds: the k-th largest head bounds the k-th largest logit from below, so a wave emits only
 // while its next entry is not below it (most emit none); final: one block ranks the k to k * k entries that are left by counting.
 // Rounds over all waves' candidates, whoever could still win, were 67 us at 151 936 logits and k = 20 (14 + 27 + 25 us of dependent wave reductions);
-// 5 + 12 + 6 us here.
-constexpr int HEADS = 512, FINAL_CAP = 64 * 64;
+// 5 + 12 + 6 us here.  Each round is 2.8 us of the call there and 0.2 us here, each wave's head 0.04 us here (every block compares all of them): up to a
+// k per 70 waves the rounds are as fast or faster (call of the host in us, rounds / bound: 151 936 logits, k = 1 / 2 / 4: 35.4 / 42.7, 38.2 / 43.3,
+// 43.7 / 43.9; 262 144, k = 1 / 7: 38.6 / 52.7, 55.8 / 53.6; 65 536, k = 1 / 2: 35.1 / 36.3, 37.9 / 36.5; 32 768, k = 1: 34.3 / 34.3).
+constexpr int HEADS = 512, HEADS_PER_ROUND = 70, FINAL_CAP = 64 * 64;
 __global__ __launch_bounds__(64 * S1_WAVES_PER_BLOCK) void topk_heads_kernel(const float* x, int V, float inv_temp, uint64_t* heads, float* part_m, float* part_s) {
   const int lane = threadIdx.x & 63, w = blockIdx.x * S1_WAVES_PER_BLOCK + (threadIdx.x >> 6), base = w * S1_WAVE_ELEMS;
   if (base >= V) return;
@@ -249,7 +251,7 @@ __global__ __launch_bounds__(1024) void topk_final_kernel(const float* x, const 
   }
 }
 
-// ---- larger vocabularies: rounds over all candidates ------------------------------------------------------------------------------------------------
+// ---- larger vocabularies, few candidates of many waves: rounds over all candidates ------------------------------------------------------------------------------------------------
 constexpr int S2_WAVES = 16;
 constexpr int S2_C = 20;  // 16 waves x 64 lanes x 20 >= 297 stage-1 waves x 64 candidates
 
@@ -316,7 +318,7 @@ __global__ __launch_bounds__(64) void topk_stage2b_kernel(const float* mid_val, 
 }  // namespace
 
 int sample_stage1_waves(int V) { return (V + S1_WAVE_ELEMS - 1) / S1_WAVE_ELEMS; }
-// u32 words of launch_topk_candidates' index array
+// u32 words of launch_topk_candidates' index array, whichever launches it takes
 size_t sample_index_words(int V) {
   const size_t nw = sample_stage1_waves(V);
   return nw <= (size_t)HEADS ? 2 * (nw * 64 + HEADS) + HEADS : (nw + 16) * 64;
@@ -333,7 +335,7 @@ void launch_topk_candidates(const float* x, int V, int k, float inv_temp, float*
                             float* part_s, float* out_val, unsigned* out_idx, float* out_ms, hipStream_t st) {
   const int nw = sample_stage1_waves(V);
   const dim3 blocks((nw + S1_WAVES_PER_BLOCK - 1) / S1_WAVES_PER_BLOCK), threads(64 * S1_WAVES_PER_BLOCK);
-  if (nw <= HEADS) {
+  if (nw <= HEADS && k * HEADS_PER_ROUND > nw) {
     uint64_t* cand = reinterpret_cast<uint64_t*>(cand_idx);   // (sample_index_words: keys of all waves' k best, then heads and counts)
     uint64_t* heads = cand + (size_t)nw * 64;
     int* count = reinterpret_cast<int*>(heads + HEADS);

@@ -177,10 +177,11 @@ def test_where_the_candidates_lie(gpu, vocab):
         m.close()
 
 
-@pytest.mark.parametrize("vocab,ks", [(513, (1, 20, 64)), (262144, (1, 20, 40)), (262145, (1, 20, 39))])
+@pytest.mark.parametrize("vocab,ks", [(513, (1, 20, 64)), (71681, (1, 2, 3)), (262144, (1, 20, 40)), (262145, (1, 20, 39))])
 def test_a_wave_of_minus_infinity(gpu, vocab, ks):
     """A last wave of one entry that is -inf (vocabularies of 513 and 262145) adds nothing to the normaliser.  262144 entries are the most that the
-    launches of topk_heads_kernel take, 262145 the fewest for the rounds over all candidates (whose second stage holds 20480: k <= 39 there)."""
+    launches of topk_heads_kernel take, 262145 the fewest for the rounds over all candidates (whose second stage holds 20480: k <= 39 there); 71681
+    are 141 waves, k = 2 the last that takes the rounds."""
     cfg, m = make(vocab)
     try:
         last = np.arange((vocab - 1) // 512 * 512, vocab)
