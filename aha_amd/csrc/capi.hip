@@ -341,6 +341,14 @@ int aha_hip_debug_plan_gemm(int32_t M, int32_t N, int32_t K, int32_t act, int32_
   out3[0] = o[0]; out3[1] = o[1]; out3[2] = o[2];
   return AHA_OK;
 }
+int aha_hip_debug_few_rows_gemm(int32_t M, int32_t N, int32_t K, int32_t act, int32_t has_bias, int32_t has_residual, size_t workspace_bytes) {
+  if (M <= 0 || N <= 0 || K <= 0) {
+    set_error("debug_few_rows_gemm: bad argument");
+    return AHA_ERR_INVALID;
+  }
+  int o[3];
+  return debug_plan_gemm(M, N, K, act, has_bias != 0, (has_residual & 1) != 0, workspace_bytes, o, (has_residual & 2) != 0);
+}
 int aha_hip_debug_streamk_plan(int32_t M, int32_t N, int32_t K, int32_t tile_n, int32_t workers, size_t workspace_bytes, int32_t* out,
                                int32_t cap, int32_t* off_out, int32_t* info7) {
   if (!out || cap < 0 || M <= 0 || N <= 0 || K <= 0) {

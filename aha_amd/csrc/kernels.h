@@ -227,6 +227,7 @@ void launch_gemm(const GemmArgs& a, hipStream_t st);
 // few rows (kernels_gemm_skinny.hip): launch_gemm's choice where its estimate is below the tiled plans'
 bool gemm_skinny_ok(const GemmArgs& a);
 double gemm_skinny_plan(const GemmArgs& a, int* r8_out);
+int gemm_skinny_rounds(const GemmArgs& a, int r8);   // blocks of r8 * 8 weight rows over the CUs
 void launch_gemm_skinny(const GemmArgs& a, hipStream_t st);
 // One launch over all row segments on the four-wave 256 x 256 / 256 x 192 kernels (plain and gate+up epilogues, whole K tiles, M >= 256);
 // any other shape: one launch_gemm per segment.  Every output element is the same K-ordered sum as in an ungrouped GEMM over its row.
@@ -246,7 +247,8 @@ void set_gemm_reserved_cus(int n);     // CUs the persistent GEMM leaves free (R
 bool acquire_gemm_cu_reservation(int cus);   // the automatic, reference-counted reservation of a communication stream (kernels_gemm_sk.hip)
 void release_gemm_cu_reservation();
 int debug_streamk_plan(int M, int N, int K, int tile_n, int workers, int group, size_t ws_bytes, int* out, int cap, int* off_out, int* info);
-void debug_plan_gemm(int M, int N, int K, int act, bool has_bias, bool has_res, size_t ws_bytes, int* out, bool has_norm = false);   // host only: {tile, splitk, n_split} of the tiled kernels
+// host only: {tile, splitk, n_split} of the tiled kernels; returns the few-row kernel's weight rows per block where that one is taken, else 0
+int debug_plan_gemm(int M, int N, int K, int act, bool has_bias, bool has_res, size_t ws_bytes, int* out, bool has_norm = false);
 void set_gemm_plan_override(int tile, int splitk);  // tests: force the 128 / 256 tile kernel and a split-K factor; 0 = automatic
 void get_gemm_workspace(void** ws, size_t* bytes, void** sk_counters);
 struct GemmWorkspaceScope {   // nests: the vision tower's own workspace inside the prefill's

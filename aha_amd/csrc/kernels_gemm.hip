@@ -1232,9 +1232,30 @@ GemmPlan plan_gemm(const GemmArgs& a) {
 
 }  // namespace
 
+static bool plan_from_env() {   // a tile or split factor forced for an A/B (plan_gemm)
+  static const bool on = getenv("AHA_GEMM_TILE") != nullptr || getenv("AHA_GEMM_SPLITK") != nullptr;
+  return on;
+}
+// Few rows: the kernel that streams W once and joins its K shares in LDS, where it is expected below the tiled plan -- which for its part cannot be
+// faster than W's bytes at what its staging reaches with few rows: 4.2 TB/s (18.1 us for 71 MB on average at 8 rows, 46 us for 201 MB at 32) and ~5 us
+// of a reduce pass.  (4096 x 12288: 25.9 us against 24 + 5 at 32 rows, 35.5 against 24 + 5 at 64: there the tiles stay.)  Behind a long W, where the
+// few-row kernel needs more than one round, 4.84 TB/s, 4 us of the pairs' epilogue, and 2 % for the estimates' spread (32768 x 4096: 60.9 us at 8 rows and
+// 61.9 at 64, 151936 x 1024: 65.8 and 73.1, 24576 x 4096 pairs: 44.8 and 47.1); the choice is at most 3.5 % behind the better one at the shapes of
+// gemm_skinny_plan.
+static bool takes_few_rows(const GemmArgs& a, const GemmPlan& plan, int* r8) {
+  if (g_force_tile != 0 || plan_from_env() || !gemm_skinny_ok(a)) return false;
+  const double bytes = (double)a.N * a.K * 2.0;
+  const bool slices = plan.splitk > 1;
+  const double few = gemm_skinny_plan(a, r8) + (a.norm_w && slices ? 3.0 : 0.0);   // (a norm that the reduce pass would have taken along: its own launch)
+  if (few < 1e30 && gemm_skinny_rounds(a, *r8) > 1)
+    return few * 1.02 < std::max(plan.cost, bytes / 4.84e6 + (slices ? 8.0 : 2.0) + (a.act == ACT_SILU_MUL_PAIRS ? 4.0 : 0.0));
+  return few < std::max(plan.cost, bytes / 4.2e6 + (slices ? 5.0 : 2.0));
+}
+
 // The launch(es) launch_gemm would issue for a shape, without issuing them (host only): out[0..2] = {tile, splitk, 1 if the columns are
-// split into a multiple of 256 + a tail launch}.  `ws_bytes` > 0 stands for a caller workspace of that size.
-void debug_plan_gemm(int M, int N, int K, int act, bool has_bias, bool has_res, size_t ws_bytes, int* out, bool has_norm) {
+// split into a multiple of 256 + a tail launch}.  `ws_bytes` > 0 stands for a caller workspace of that size.  These are the tiled kernels' plans:
+// returns the few-row kernel's weight rows per block where launch_gemm takes that one instead, else 0.
+int debug_plan_gemm(int M, int N, int K, int act, bool has_bias, bool has_res, size_t ws_bytes, int* out, bool has_norm) {
   GemmArgs a{};
   a.M = M; a.N = N; a.K = K; a.lda = K; a.ldw = K; a.ldc = act == ACT_SILU_MUL_PAIRS ? N / 2 : N; a.act = act;
   static int dummy;
@@ -1253,6 +1274,8 @@ void debug_plan_gemm(int M, int N, int K, int act, bool has_bias, bool has_res, 
     const GemmPlan pm = plan_gemm(am), pt = plan_gemm(at);
     if (pm.cost + pt.cost + 3.0 < plan.cost) { out[0] = pm.tile; out[1] = pm.splitk; out[2] = 1; }
   }
+  int r8;
+  return takes_few_rows(a, plan, &r8) ? r8 * 8 : 0;
 }
 
 void set_gemm_plan_override(int tile, int splitk) {
@@ -1282,11 +1305,6 @@ static void launch_riding_norm(const GemmArgs& a, hipStream_t st) {
   else launch_rmsnorm_rows(a.C, a.norm_w, a.norm_out, a.M, a.N, a.ldc, a.N, a.norm_eps, st);
 }
 
-static bool plan_from_env() {   // a tile or split factor forced for an A/B (plan_gemm)
-  static const bool on = getenv("AHA_GEMM_TILE") != nullptr || getenv("AHA_GEMM_SPLITK") != nullptr;
-  return on;
-}
-
 void launch_gemm(const GemmArgs& a_in, hipStream_t st) {
   if (a_in.M <= 0 || a_in.N <= 0) return;
   GemmArgs a = a_in;
@@ -1300,17 +1318,11 @@ void launch_gemm(const GemmArgs& a_in, hipStream_t st) {
   static const int e_prow = [] { const char* e = getenv("AHA_GEMM_PARTIAL_ROWS"); return e ? atoi(e) : 1; }();
   a.partial_rows = e_prow;
   const GemmPlan plan = plan_gemm(a);
-  // Few rows: the kernel that streams W once and joins its K shares in LDS, where it is expected below the tiled plan -- which for its part cannot
-  // be faster than W's bytes at the 4.2 TB/s its staging reaches with few rows (18.1 us for 71 MB on average at 8 rows, 46 us for 201 MB at 32)
-  // and ~5 us of a reduce pass.  (4096 x 12288: 25.9 us against 24 + 5 at 32 rows, 35.5 against 24 + 5 at 64: there the tiles stay.)
-  if (g_force_tile == 0 && !plan_from_env() && gemm_skinny_ok(a)) {
-    int r8;
-    const double tiled = std::max(plan.cost, (double)a.N * a.K * 2.0 / 4.2e6 + (plan.splitk > 1 ? 5.0 : 2.0));
-    if (gemm_skinny_plan(a, &r8) + (a.norm_w && plan.splitk > 1 ? 3.0 : 0.0) < tiled) {   // (a norm that the reduce pass would have taken along: its own launch)
-      launch_gemm_skinny(a, st);
-      if (a.norm_w) launch_riding_norm(a, st);
-      return;
-    }
+  int r8;
+  if (takes_few_rows(a, plan, &r8)) {
+    launch_gemm_skinny(a, st);
+    if (a.norm_w) launch_riding_norm(a, st);
+    return;
   }
   // Ragged N (ViT fc1: N = 4304 = 16 x 256 + 208): the 17th column of 256^2 tiles makes 272 units = two rounds on 256 CUs for
   // 1.06 rounds of work.  Where the model says it pays, the columns up to the last multiple of 256 run as one GEMM and the

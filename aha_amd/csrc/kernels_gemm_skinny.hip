@@ -17,6 +17,8 @@
 //   1024 x 2048 7.0 / 7.7 (11.3 / 12.1), 1024 x 3072 9.0 / 10.2 (12.3 / 13.2); a 0.6B prompt of 96 / 128 / 180 / 250 tokens 1.66 / 1.67 / 1.95 / 2.03 ms
 //   (1.97 / 2.06 / 2.07 / 2.14), of 300 2.14 (2.09): 256 rows at most.  The 8B shapes stay on the tiles:
 //   their weight rows need more than one round or a longer K than a block streams in the tiles' time (6144 x 4096, 96 rows: 21.3 against 21.0).
+#include <algorithm>
+
 #include "gemm256_body.h"
 #include "skinny_body.h"
 
@@ -89,16 +91,31 @@ void launch_rows(const GemmArgs& a, hipStream_t st) {
 
 }  // namespace
 
-// Weight rows per block / 8, and the estimated microseconds.  A block streams its weight rows and, from L2, A's rows (0.4 of the price per byte);
-// a CU does ~30 bytes per ns of that mix, and launch, first request and the joined sums cost ~3 us (fitted to 8 .. 64 rows of the shapes above).
+int gemm_skinny_rounds(const GemmArgs& a, int r8) { return ((a.N + r8 * 8 - 1) / (r8 * 8) * ((a.M + 63) / 64) + 255) / 256; }
+
+// Weight rows per block / 8, and the estimated microseconds.  One round (a block per CU): a block streams its weight rows and, from L2, A's rows (0.4 of
+// the price per byte); a CU does ~30 bytes per ns of that mix, and launch, first request and the joined sums cost ~3 us (fitted to 8 .. 64 rows of the
+// shapes above).
+// More rounds, up to 64 rows (4096 x 1024, 180 rows, 384 blocks: 12.0 us against 10.9 of the tiles): a CU requests at most 60 bytes of weights per ns and
+// the chip delivers at most 8.2 TB/s (32 rows per block that lie whole 256 KB apart: 1.34 times as long, their requests meet in the same channels),
+// rounded where the two meet; A's rows at 96 bytes per ns and CU, the last row's repetitions for nothing; a block's first requests and the joined sums
+// show where no neighbour on the CU covers them.  Fitted to 23 shapes (512 x 4096 to 151936 x 4096) at 1 to 64 rows with every R8, 6 % off on average.
+// The price of one round times their number said 41 us with 32 rows per block for 32768 x 4096 and 8 rows (60.6; 44.5 with 48) and 76 us for
+// 151936 x 1024 and 64 rows (102; the tiles 73).
 double gemm_skinny_plan(const GemmArgs& a, int* r8_out) {
   const int m8 = a.M <= 8 ? 1 : a.M <= 16 ? 2 : a.M <= 32 ? 4 : 8;
+  const double chunk = a.K * 16.0;   // bytes of eight rows
   double best = 1e30;
   for (int r8 : {2, 3, 4, 6}) {
     if (a.act == ACT_SILU_MUL_PAIRS && r8 == 3) continue;   // (gate and up rows in eights)
-    const double rounds = ceil(((a.N + r8 * 8 - 1) / (r8 * 8)) * ((a.M + 63) / 64) / 256.0);
-    if (a.M > 64 && rounds > 1) continue;   // (4096 x 1024, 180 rows, 384 blocks: 12.0 us against 10.9 of the tiles)
-    const double c = 3.0 + rounds * (r8 + 0.4 * m8) * a.K * 16.0 / 30e3;
+    const int rounds = gemm_skinny_rounds(a, r8);
+    double c = 3.0 + (r8 + 0.4 * m8) * chunk / 30e3;
+    if (rounds > 1) {
+      if (a.M > 64) continue;
+      const int resident = std::min(4, 160 * 1024 / skinny_lds(r8, m8)), rows8 = (a.M + 7) / 8;
+      const double cu = rounds * r8 * chunk / 60e3, chip = a.N / 8 * chunk / 8.2e6 * (r8 == 4 && a.ldw * 64 % (256 << 10) == 0 ? 1.34 : 1.0);
+      c = 3.5 + sqrt(cu * cu + chip * chip) + rounds * rows8 * chunk / 96e3 + ((rounds + resident - 1) / resident - 1) * 0.25 * rows8 + 0.075 * rounds * m8;
+    }
     if (c < best) {
       best = c;
       *r8_out = r8;

@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+from aha_amd import _lib
 from oracle import qwen3 as oq
 from tests.test_ops_gpu import NM, assert_close_ulps, rnd
 
@@ -60,3 +61,29 @@ def test_row_tiles(gpu, M, N, K, pairs):
     assert_close_ulps(ops.gemm(A.to(gpu), W.to(gpu)), NM.linear(A.float(), W.float()), 1, None, "plain")
     full = ops.gemm(A.to(gpu), W.to(gpu), b.to(gpu), r.to(gpu), _lib.ACT_NONE)
     assert_close_ulps(full, NM.r(r.float() + NM.linear(A.float(), W.float(), b.float())), 2, None, "bias + residual")
+
+
+def rows_per_block(M, N, K, act=0):
+    return _lib.lib().aha_hip_debug_few_rows_gemm(M, N, K, act, 0, 0, 1 << 30)   # 0: the tiled kernels
+
+
+@pytest.mark.parametrize("N,K,width,M", [(N, K, w, M) for N, K, w, most in [(1272, 832, 16, 64), (5000, 832, 24, 64), (12312, 768, 32, 33), (12280, 832, 48, 64)]
+                                         for M in (1, 8, 9, 16, 17, 32, 33, 64) if M <= most])
+def test_block_width_with_pitches(gpu, N, K, width, M):
+    """Every width of a block (asked for, so that a change of the cost model does not empty this test), N ending inside the last one, with rows of A, W,
+    bias + residual and C that lie further apart than they are long; what lies between C's rows and behind them stays untouched.  1 ulp for the plain
+    product, 2 behind bias and residual, as above."""
+    from aha_amd._lib import check, lib
+    assert rows_per_block(M, N, K) == width and N % width != 0
+    lda, ldw, ldc = K + 8, K + 24, N + 12
+    A, W, b, r = rnd((M, lda), 81), rnd((N, ldw), 82, 0.05), rnd((N,), 83, 0.5), rnd((M, ldc), 84)
+    Ad, Wd, bd, rd = (t.to(gpu) for t in (A, W, b, r))
+    ref = NM.linear(A[:, :K].float(), W[:, :K].float())
+    st = torch.cuda.current_stream().cuda_stream
+    for bias, res, want, ulps in ((None, None, ref, 1),
+                                  (bd, rd, NM.r(r[:, :N].float() + NM.linear(A[:, :K].float(), W[:, :K].float(), b.float())), 2)):
+        out = torch.full((M + 2, ldc), 7.0, dtype=torch.bfloat16, device=gpu)
+        check(lib().aha_hip_gemm(Ad.data_ptr(), Wd.data_ptr(), out.data_ptr(), M, N, K, lda, ldw, ldc, bias.data_ptr() if bias is not None else None,
+                                 res.data_ptr() if res is not None else None, _lib.ACT_NONE, st))
+        assert_close_ulps(out[:M, :N], want, ulps, None, "pitched")
+        assert (out[:M, N:] == 7.0).all() and (out[M:] == 7.0).all()

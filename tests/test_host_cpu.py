@@ -285,6 +285,33 @@ def test_gemm_plans_of_the_baseline_shapes(hip_lib):
         assert hip_lib.aha_hip_debug_plan_gemm(0, 1, 1, 0, 0, 0, 0, (ctypes.c_int32 * 3)()) == 0
 
 
+def test_few_row_gemm_where_it_is_the_faster_one(hip_lib):
+    """csrc/kernels_gemm_skinny.hip gemm_skinny_plan against the tiled plans: weight rows per block of the few-row kernel, 0 where the tiles run.  Times on
+    MI355X from HBM in us, few-row kernel with 16 / 24 / 32 / 48 weight rows | tiles."""
+    from aha_amd import _lib
+    P = _lib.ACT_SILU_MUL_PAIRS
+
+    def rows(M, N, K, act=_lib.ACT_NONE, res=0):
+        return hip_lib.aha_hip_debug_few_rows_gemm(M, N, K, act, 0, res, 1 << 30)
+    # long outputs (vocabularies): few rows stream the weights in blocks of 48, more of them leave no second block on the CU and the tiles win
+    assert rows(8, 32768, 4096) == 48 and rows(32, 32768, 4096) == 48       # 44.5 / 45.7 / 60.7 / 44.5 | 60.9, 64.9 / 59.0 / 64.9 / 50.8 | 61.0
+    assert rows(64, 32768, 4096) == 0                                       # 88.9 / 81.7 / 80.2 / 67.0 | 61.9
+    assert rows(8, 151936, 1024) == 48 and rows(33, 151936, 1024) == rows(64, 151936, 1024) == 0     # 92.1, 101 at best | 68.1, 73.1
+    assert rows(16, 151936, 4096) == 48 and rows(64, 151936, 4096) == 0     # 202 | 253, 294 | 258
+    assert rows(64, 64000, 2048) == 0 and rows(48, 16384, 4096) == 0        # 76.7 | 65.6, 38.6 | 36.5
+    assert rows(24, 32768, 1024) == rows(48, 16384, 1024) == 0              # 15.8, 12.7 at best | 14.3, 11.7
+    # the 8B and 0.6B projections keep it
+    assert [rows(M, 24576, 4096, P) for M in (8, 33, 48)] == [48] * 3       # 33.9, 39.9, 42.6 | 44.8, 45.5, 46.3
+    assert [rows(M, 12288, 4096) for M in (9, 64)] == [48] * 2              # 19.2, 23.9 | 27.3, 29.9
+    assert rows(8, 6144, 4096) == 24 and rows(8, 4096, 4096, res=1) == rows(8, 4096, 12288, res=1) == 16
+    assert all(rows(M, 1024, 3072, res=1) == 16 for M in (1, 32, 64)) and rows(64, 4096, 1024) > 0
+    # never: short K, small matrices from 33 rows on, more than one round of row tiles; a norm behind K slices makes it dearer
+    assert rows(8, 4096, 704) == rows(33, 512, 1024) == rows(205, 24576, 4096, P) == rows(96, 6144, 4096) == 0
+    assert rows(48, 4096, 4096, res=1) == 16 and rows(48, 4096, 4096, res=3) == 0
+    with pytest.raises(Exception):
+        assert rows(0, 1, 1) >= 0
+
+
 @pytest.mark.parametrize("S", [512, 1542, 2048, 8192, 40980, 131072])
 @pytest.mark.parametrize("world", [2, 3, 4, 8])
 def test_context_parallel_plan_partitions_the_prompt(hip_lib, S, world):
