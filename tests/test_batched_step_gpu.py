@@ -19,14 +19,14 @@ def moe_model(gpu, experts, top, ff, shared, hidden=256, vocab=5000):
     return cfg, w, HipInferenceModel(cfg, {k: v.to(gpu) for k, v in w.items()})
 
 
-@pytest.mark.parametrize("rows", [2, 7, 8, 9, 16, 17, 31, 33, 70])
-@pytest.mark.parametrize("experts,top,ff,shared", [(1, 1, 96, 0), (3, 2, 200, 64), (64, 3, 72, 0)])
-def test_experts_with_few_slots(gpu, rows, experts, top, ff, shared):
+@pytest.mark.parametrize("experts,top,ff,shared,hidden,rows", [(*c, 256, r) for c in [(1, 1, 96, 0), (3, 2, 200, 64), (64, 3, 72, 0)]
+                                                               for r in (2, 7, 8, 9, 16, 17, 31, 33, 70)] + [(48, 3, 200, 0, 512, r) for r in (33, 200, 380)])
+def test_experts_with_few_slots(gpu, experts, top, ff, shared, hidden, rows):
     """1 to 70 slots per expert (8, 16 and 32 activation rows per tile, one tile and several, an expert without slots), widths that end inside a
-    block of 16 and 48 weight rows: `rows` sequences of one token each, every one against the restatement in 64 bits; the bound is the layer-list
+    block of 16 weight rows, and of 48 (48 experts x 11 blocks: both products, about 2, 12 and 24 slots per expert): `rows` sequences of one token each, every one against the restatement in 64 bits; the bound is the layer-list
     decoders' (3 % of the logits' spread in bf16).  Left out are rows whose best unchosen expert is closer to the chosen ones than bf16 rounding of
     the stream can move a router logit (0.02 of the logits' spread)."""
-    cfg, w, m = moe_model(gpu, experts, top, ff, shared)
+    cfg, w, m = moe_model(gpu, experts, top, ff, shared, hidden)
     w64, c = {k: v.double() for k, v in w.items()}, cfg.to_json()
     ids = torch.randint(0, cfg.vocab_size, (rows,), generator=torch.Generator().manual_seed(rows)).tolist()
     seqs = [m.seq_open() for _ in ids]
@@ -82,6 +82,24 @@ def test_32_bit_mode_by_row_count(gpu, rows, dim, vdim, chunk):
     ref = D.forward(js, {k: v.double() for k, v in w.items()}, ids).numpy()
     s = m.seq_open()
     got = np.concatenate([m.forward_batch([(s, ids[:rows], list(range(rows)))])[0], m.forward_batch([(s, ids[rows:], [0])])[0]])
+    assert np.abs(got - ref).max() < 2e-5 * ref.std() * 4 and np.sqrt(((got - ref) ** 2).mean()) < 2e-5 * ref.std()
+    m.seq_close(s)
+    m.close()
+
+
+@pytest.mark.parametrize("rows", [1, 9, 17])
+def test_32_bit_head_in_wide_blocks(gpu, rows):
+    """A vocabulary whose head makes 515 blocks of 48 weight rows, the last one short, for 8, 16 and 32 activation rows; the bound of the test above."""
+    from aha_amd.configs_layered import DosovikConfig, LayerConfig
+    from oracle import dosovik as D
+    lay = LayerConfig(heads=4, kv_heads=2, dim=32, vdim=32, chunk=1 << 20, rope_dims=16, rope_base=1e4, scale=32 ** -0.5, ff=200)
+    cfg = DosovikConfig(hidden_size=200, vocab_size=24700, layers=[lay], embed_scale=14.0, post_norm_alpha=1.3, compute_dtype="float32")
+    w = weights_layered.dosovik_weights(cfg, seed=6)
+    m = HipInferenceModel(cfg, {k: v.to(gpu) for k, v in w.items()})
+    ids = torch.randint(0, 24700, (rows,), generator=torch.Generator().manual_seed(rows)).tolist()
+    ref = D.forward(cfg.to_json(), {k: v.double() for k, v in w.items()}, ids).numpy()
+    s = m.seq_open()
+    got, _ = m.forward_batch([(s, ids, list(range(rows)))])
     assert np.abs(got - ref).max() < 2e-5 * ref.std() * 4 and np.sqrt(((got - ref) ** 2).mean()) < 2e-5 * ref.std()
     m.seq_close(s)
     m.close()

@@ -1,4 +1,5 @@
-"""-m gpu: the few-row GEMM (csrc/kernels_gemm_skinny.hip), which launch_gemm takes by itself for these shapes, against the oracle chain."""
+"""-m gpu: the few-row GEMM (csrc/kernels_gemm_skinny.hip), which launch_gemm takes by itself for these shapes (where it does not, the tiled kernels
+are held to the same bounds: the cases say so), against the oracle chain."""
 import pytest
 import torch
 
@@ -11,11 +12,11 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32, 33, 64])
 @pytest.mark.parametrize("N,K", [
-    (8, 768),        # one eight-row group, as many k chunks per wave as ring stages
+    (8, 768),        # one eight-row group, as many k chunks per wave as ring stages; 33 and 64 rows: the tiles (below 2 MB)
     (1264, 832),     # N ends inside a block of 16, 24, 32 and 48 rows; an uneven share of chunks per wave
     (6144, 768),     # 24 rows per block: half a fragment unused
-    (12320, 832),    # 48 rows per block, the last block short
-    (40, 4160),      # many chunks
+    (12320, 832),    # 32 rows per block in two rounds; 64 rows: the tiles
+    (40, 4160),      # many chunks; 33 and 64 rows: the tiles
 ])
 def test_few_rows_every_row_count_and_block_width(gpu, M, N, K):
     """One f32 sum per element, rounded once per op as in the tiled kernels: a sum next to a rounding boundary moves one op's result by one ulp, so
@@ -39,7 +40,8 @@ def test_few_rows_every_row_count_and_block_width(gpu, M, N, K):
 @pytest.mark.parametrize("M", [1, 8, 13, 31, 64])
 @pytest.mark.parametrize("I,K", [(16, 768), (1008, 832), (3072, 1024), (12288, 768)])
 def test_few_rows_gate_up_pairs(gpu, M, I, K):
-    """Gate and up rows in groups of eight per block, the product in the epilogue (interleaved layout of the model loader)."""
+    """Gate and up rows in groups of eight per block, the product in the epilogue (interleaved layout of the model loader).  64 rows of the first and the
+    last shape: the tiles."""
     from aha_amd import ops, _lib
     A, Wg, Wu = rnd((M, K), 61), rnd((I, K), 62, 0.05), rnd((I, K), 63, 0.05)
     ref = NM.r(NM.r(oq.silu(NM.linear(A.float(), Wg.float()))) * NM.linear(A.float(), Wu.float()))
@@ -87,3 +89,35 @@ def test_block_width_with_pitches(gpu, N, K, width, M):
                                  res.data_ptr() if res is not None else None, _lib.ACT_NONE, st))
         assert_close_ulps(out[:M, :N], want, ulps, None, "pitched")
         assert (out[:M, N:] == 7.0).all() and (out[M:] == 7.0).all()
+
+
+@pytest.mark.parametrize("M", [129, 192, 193, 255])
+@pytest.mark.parametrize("act", ["plain", "bias + residual", "gate * up"])
+def test_one_row_of_tall_tiles(gpu, M, act):
+    """129 to 255 rows of a long W on the automatic plan: 256 x 128 tiles, the only row of them partly filled, the last column of them too; rows of A and
+    W further apart than they are long.  Bounds as above."""
+    import ctypes
+    from aha_amd._lib import check, lib
+    pairs = act == "gate * up"
+    N, K, code = (16544 if pairs else 16520), 640, _lib.ACT_SILU_MUL_PAIRS if pairs else _lib.ACT_NONE
+    plan = (ctypes.c_int32 * 3)()
+    check(lib().aha_hip_debug_plan_gemm(M, N, K, code, act == "bias + residual", act == "bias + residual", 1 << 30, plan))
+    assert tuple(plan) == (2128, 1, 0) and rows_per_block(M, N, K, code) == 0
+    from aha_amd import ops
+    A, W = rnd((M, K + 8), 91), rnd((N, K), 92, 0.05)
+    Ad = A.to(gpu)
+    ref = NM.linear(A[:, :K].float(), W.float())
+    st = torch.cuda.current_stream().cuda_stream
+    Wd = (ops.interleave_gate_up(W[:N // 2], W[N // 2:]) if pairs else W).to(gpu)
+    No = N // 2 if pairs else N
+    b, r = rnd((N,), 93, 0.5), rnd((M, No), 94)
+    bd, rd = b.to(gpu), r.to(gpu)
+    out = torch.full((M + 2, No), 7.0, dtype=torch.bfloat16, device=gpu)
+    res = act == "bias + residual"
+    check(lib().aha_hip_gemm(Ad.data_ptr(), Wd.data_ptr(), out.data_ptr(), M, N, K, K + 8, K, No, bd.data_ptr() if res else None, rd.data_ptr() if res else None, code, st))
+    if pairs:
+        ref = NM.r(NM.r(oq.silu(ref[:, :N // 2])) * ref[:, N // 2:])
+    elif res:
+        ref = NM.r(r.float() + NM.linear(A[:, :K].float(), W.float(), b.float()))
+    assert_close_ulps(out[:M], ref, {"plain": 1, "bias + residual": 2, "gate * up": 3}[act], None, act)
+    assert (out[M:] == 7.0).all()
