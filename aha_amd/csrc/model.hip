@@ -1438,7 +1438,7 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_read
   int nsplit = (npages + div - 1) / div;
   nsplit = std::max(1, std::min(std::min(nsplit, m->max_nsplit), 1024 / (nh / kvh)));  // g * nsplit <= 1024: LDS tables of the split merge
   // short and middle contexts: the merge of the splits in the o_proj matvec (one GPU)
-  int defer = e_div ? 0 : attn_decode_defer_splits(npages, nq);
+  int defer = e_div || !m->decode_fused ? 0 : attn_decode_defer_splits(npages, nq);
   if (defer > 1 && m->tp_size > 1) defer = 0;
   if (defer) nsplit = defer;
   for (int li = 0; li < c.num_hidden_layers; ++li) {

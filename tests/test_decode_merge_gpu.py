@@ -67,3 +67,37 @@ def test_between_two_steps(gpu, hidden, vocab):
         np.testing.assert_array_equal(last, logits)
     finally:
         m.close()
+
+
+def test_three_launch_form_keeps_its_splits(gpu):
+    """AHA_DECODE_FUSED=0 has a combine launch of its own and splits the cache as AHA_ATTN_PAGES_PER_BLOCK says (four pages when unset; read once per
+    process: children), whatever the merging form would choose: the same logits, bit for bit, with the variable at its default and unset."""
+    import os
+    import subprocess
+    import sys
+    code = """
+import hashlib
+from aha_amd.configs import tiny_qwen3
+from aha_amd.model import HipInferenceModel
+from aha_amd.weights import qwen3_text_weights
+from tests.test_model_gpu import ids_for
+cfg = tiny_qwen3(layers=2, hidden=512, heads=4, kv_heads=2, inter=512, vocab=1024)
+m = HipInferenceModel(cfg, qwen3_text_weights(cfg, seed=4))
+h = hashlib.sha256()
+for S in (190, 2200, 3000):
+    m.clear_cache()
+    _, tok = m.forward_initial(ids_for(cfg, S, S), 0)
+    for i in range(2):
+        logits, tok = m.forward_step(tok, S + i)
+        h.update(logits.tobytes())
+m.close()
+print("LOGITS", h.hexdigest())
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    seen = []
+    for extra in ({}, {"AHA_ATTN_PAGES_PER_BLOCK": "4"}):
+        env = dict({k: v for k, v in os.environ.items() if k != "AHA_ATTN_PAGES_PER_BLOCK"}, PYTHONPATH=root, AHA_DECODE_FUSED="0", **extra)
+        r = subprocess.run([sys.executable, "-c", code], cwd=root, env=env, capture_output=True, text=True, timeout=100)
+        assert r.returncode == 0, r.stderr[-2000:]
+        seen.append([ln for ln in r.stdout.splitlines() if ln.startswith("LOGITS")][0])
+    assert seen[0] == seen[1]
