@@ -425,6 +425,9 @@ class HipInferenceModel:
         return out
 
     def embed_multi(self, inputs: Sequence[Sequence[int]]) -> np.ndarray:
+        """One vector per document (the rows of the result), those that fit together by one prefill: a vector agrees with embed_one's to the rounding of
+        bf16 sums and not bit for bit, and which documents share the call decides about its last bits; equal documents that share a prefill get equal
+        vectors."""
         if len(inputs) == 0:
             raise ValueError("embedding input cannot be empty")  # qwen3_embedding/mod.rs:39-41
         docs = [np.asarray(x, dtype=np.uint32).reshape(-1) for x in inputs]
@@ -436,8 +439,10 @@ class HipInferenceModel:
 
     def rerank(self, query_ids: Sequence[int], documents_ids: Sequence[Sequence[int]]) -> np.ndarray:
         """Qwen3Reranker::rerank (qwen3_reranker/mod.rs:23-31): cosine_similarity_no_l2(query, docs) on normalised vectors."""
-        q = self.embed_one(query_ids)[None, :]
-        return (q @ self.embed_multi(documents_ids).T)[0]
+        if len(documents_ids) == 0:
+            raise ValueError("embedding input cannot be empty")
+        v = self.embed_multi([query_ids, *documents_ids])   # (the query among the documents: a document that repeats it scores 1)
+        return (v[:1] @ v[1:].T)[0]
 
     def cache_len(self) -> int:
         return int(lib().aha_hip_cache_len(self.handle))

@@ -199,7 +199,10 @@ int aha_hip_get_rope_index_mm(const aha_model_desc* desc, const uint32_t* input_
  * Qwen3Reranker::rerank (qwen3_reranker/mod.rs:23-31) is the dot product of two such vectors
  * (cosine_similarity_no_l2, modules.rs:1381-1389) -- host arithmetic on the caller's side. */
 int aha_hip_embed(aha_model* m, const uint32_t* input_ids, size_t n_ids, float* out);
-/* n_docs documents, their ids one after another (n_ids[d] of document d) -> out[n_docs][hidden_size]: documents that fit together share one prefill. */
+/* n_docs documents, their ids one after another (n_ids[d] of document d) -> out[n_docs][hidden_size]: documents that fit together share one prefill.
+ * A vector agrees with aha_hip_embed's to the rounding of bf16 sums, not bit for bit: the kernels, and with them the order of the sums, follow the rows
+ * of the whole prefill, so a document's last bits depend on its companions (its distance from the exact vector does not).  Equal documents of one
+ * prefill get equal vectors.  Documents of one token, of more than 4096, and one that is left alone run as aha_hip_embed does. */
 int aha_hip_embed_multi(aha_model* m, const uint32_t* input_ids, const uint64_t* n_ids, size_t n_docs, float* out);
 
 /* ---- checkpoint directory -> model (XxxGenerateModel::init minus tokenizer / chat template) --------------------------

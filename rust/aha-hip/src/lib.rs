@@ -238,6 +238,7 @@ pub mod sys {
         ) -> i32;
         pub fn aha_hip_cp_init_rccl(m: *mut AhaModel, unique_id128: *const c_void) -> i32;
         pub fn aha_hip_embed(m: *mut AhaModel, ids: *const u32, n_ids: usize, out: *mut f32) -> i32;
+        pub fn aha_hip_embed_multi(m: *mut AhaModel, ids: *const u32, n_ids: *const u64, n_docs: usize, out: *mut f32) -> i32;
         pub fn aha_hip_cache_len(m: *const AhaModel) -> usize;
         pub fn aha_hip_audio_resample(
             ctx: *mut AhaCtx,

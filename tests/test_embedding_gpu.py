@@ -167,3 +167,20 @@ def test_documents_in_little_memory(gpu):
         if alone:
             assert float((alone[0] * together[0]).sum(1).min()) >= 0.9995
     assert outcomes == {(0, 0), (1, 1)}   # the limits range from too little for a document to room for all
+
+
+def test_a_document_that_repeats_the_query_scores_one(gpu):
+    """Among other documents too, at widths where the kernels follow the number of rows (K >= 768: few rows alone, tiles together); equal documents of
+    one call get equal vectors."""
+    from aha_amd.model import HipInferenceModel
+    cfg = tiny_qwen3(layers=4, hidden=1024, heads=8, kv_heads=2, inter=3072, vocab=2048)
+    m = HipInferenceModel(cfg, qwen3_text_weights(cfg, seed=2))
+    q, a, b = seqs_for(cfg, [19, 230, 77], 9)
+    s = m.rerank(q, [a, q, b, q])
+    assert abs(float(s[1]) - 1) < 1e-5 and s[1] == s[3] and s[0] < 0.999 and s[2] < 0.999
+    v = m.embed_multi([b, q, a, b, q])
+    np.testing.assert_array_equal(v[0], v[3])
+    np.testing.assert_array_equal(v[1], v[4])
+    with pytest.raises(ValueError, match="cannot be empty"):
+        m.rerank(q, [])
+    m.close()
