@@ -268,7 +268,7 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void moe_gemm_few_kernel(MoeGemm
   else moe_few_body<R8, 4, GATHER, PAIRS>(a, r, n_blk, ex, s0, ns, smem);
 }
 
-// ---- 32-bit mode: 64 x 64 tiles on v_mfma_f32_16x16x4_f32 (kernels_layered.hip gemm_f32_kernel with gathered rows) -----------------------------------
+// ---- 32-bit mode: 64 x 64 tiles on v_mfma_f32_16x16x4_f32 (kernels_gemm_f32.hip gemm_f32_any_kernel with gathered rows) --------------------------------
 constexpr int FBK = 32, FPITCH = FBK + 1;
 template <bool GATHER>
 __global__ __launch_bounds__(256) void moe_gemm_f32_kernel(MoeGemmArgs a, MoeRouting r) {

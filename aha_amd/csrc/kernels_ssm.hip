@@ -493,7 +493,7 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(SsmStepArgs a, SeqBatch b
   float* hout = a.h.hist + (int64_t)e.slot * a.h.slot_stride + (int64_t)e.hist_out * (taps - 1) * cp;
   // The block's channels: x, B and C, NIT per thread.  Inputs, weights and history of up to HT + 1 taps are requested together and the new history is
   // stored behind them: a store between two loads orders them, and tap by tap, channel by channel the chain was most of the launch (0.6B widths,
-  // one sequence: 7.5 -> 5.1 us; 8B widths, 32 sequences: 69 -> 60 us).
+  // one sequence: 7.5 -> 5.3 us; 8B widths, 32 sequences, bound by the 268 MB of their states: 60.7 -> 59.7 us).
   constexpr int NIT = (2 * NI * 64 + VT * 16 + 255) / 256, HT = 4;
   const int total = 2 * np + VT * 16;
   auto channel = [&](int i) { return i >= 2 * np ? h * a.d.vdp + vs * 16 + i - 2 * np : inner + (i < np ? grp * np + i : a.d.groups * np + grp * np + i - np); };

@@ -1724,7 +1724,7 @@ int model_embed(aha_model* m, const uint32_t* ids, size_t n, float* out) {
 
 // Several documents: as many consecutive ones as fit into EMBED_ROWS rows go through the decoder stack as ONE prefill.  A document of a few hundred
 // rows leaves most of the chip idle in every GEMM of a small model (0.6B, 300 rows: N = 1024 gives 24 tiles of 128^2) and each costs its launches:
-// eight documents of 75 to 600 tokens were 15.9 ms one by one, 3.9 ms together.  Each begins on a cache page of its own (its rows are padded to
+// eight documents of 75 to 600 tokens were 16.1 ms one by one, 4.1 ms together.  Each begins on a cache page of its own (its rows are padded to
 // whole pages by repeating its last token, behind everything its last position sees), so row = cache slot as in any prefill and only the attention
 // knows about documents.  4096 rows fill the chip with the narrowest GEMM (N = 1024: 256 tiles); a document alone, of one token (a decode step) or
 // longer than that runs as before, and so does everything where the joint prefill finds no memory: its scratch, larger than a single document's, is
