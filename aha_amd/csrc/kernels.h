@@ -216,7 +216,7 @@ struct GemmArgs {
   void* sk_counters = nullptr;   // optional SK_MAX_COUNTERS zeroed u32 words that belong to `workspace` (one per tile cut along K by the
                                  // persistent kernel, kernels_gemm_sk.hip; every launch leaves them zero again)
   int tile_group = 8;            // band width of the grouped tile order inside an XCD's run (kernels_gemm.hip tile_of_block); 0 = plain
-  int few_rows = 1;              // 0: not the few-row kernel (kernels_gemm_skinny.hip) whatever M is
+  int few_rows = 1;              // the few-row kernel (kernels_gemm_skinny.hip): 0 never, 1 where it is expected to be faster, 2 wherever it can
   int partial_rows = 1;          // ACT_PARTIAL_F32 on the four-wave kernel: f32 sums stored in row order through LDS (0: fragment order; A/B)
   // Row groups (launch_gemm_grouped; tensor-parallel prefill: the staging layout of the chunked all-gather, csrc/model.hip
   // norm_gather_gemm): `groups` row segments of M rows each share W.  Segment g reads A rows [g * a_gstride, + M) and writes C rows
@@ -226,6 +226,7 @@ struct GemmArgs {
 void launch_gemm(const GemmArgs& a, hipStream_t st);
 // few rows (kernels_gemm_skinny.hip): launch_gemm's choice where its estimate is below the tiled plans'
 bool gemm_skinny_ok(const GemmArgs& a);
+bool gemm_takes_few_rows(const GemmArgs& a);   // (launch_gemm's choice; host only)
 double gemm_skinny_plan(const GemmArgs& a, int* r8_out);
 int gemm_skinny_rounds(const GemmArgs& a, int r8);   // blocks of r8 * 8 weight rows over the CUs
 void launch_gemm_skinny(const GemmArgs& a, hipStream_t st);

@@ -1246,7 +1246,9 @@ static bool takes_few_rows(const GemmArgs& a, const GemmPlan& plan, int* r8) {
   if (g_force_tile != 0 || plan_from_env() || !gemm_skinny_ok(a)) return false;
   const double bytes = (double)a.N * a.K * 2.0;
   const bool slices = plan.splitk > 1;
-  const double few = gemm_skinny_plan(a, r8) + (a.norm_w && slices ? 3.0 : 0.0);   // (a norm that the reduce pass would have taken along: its own launch)
+  const double plan_us = gemm_skinny_plan(a, r8);
+  if (a.few_rows == 2) return plan_us < 1e30;
+  const double few = plan_us + (a.norm_w && slices ? 3.0 : 0.0);   // (a norm that the reduce pass would have taken along: its own launch)
   if (few < 1e30 && gemm_skinny_rounds(a, *r8) > 1)
     return few * 1.02 < std::max(plan.cost, bytes / 4.84e6 + (slices ? 8.0 : 2.0) + (a.act == ACT_SILU_MUL_PAIRS ? 4.0 : 0.0));
   return few < std::max(plan.cost, bytes / 4.2e6 + (slices ? 5.0 : 2.0));
@@ -1305,14 +1307,23 @@ static void launch_riding_norm(const GemmArgs& a, hipStream_t st) {
   else launch_rmsnorm_rows(a.C, a.norm_w, a.norm_out, a.M, a.N, a.ldc, a.N, a.norm_eps, st);
 }
 
+static void use_thread_workspace(GemmArgs& a) {
+  if (a.workspace != nullptr) return;
+  a.workspace = tl_ws;
+  a.workspace_bytes = tl_ws_bytes;
+  a.sk_counters = tl_sk_counters;
+}
+bool gemm_takes_few_rows(const GemmArgs& a_in) {
+  GemmArgs a = a_in;
+  use_thread_workspace(a);
+  int r8;
+  return gemm_skinny_ok(a) && takes_few_rows(a, plan_gemm(a), &r8);
+}
+
 void launch_gemm(const GemmArgs& a_in, hipStream_t st) {
   if (a_in.M <= 0 || a_in.N <= 0) return;
   GemmArgs a = a_in;
-  if (a.workspace == nullptr) {
-    a.workspace = tl_ws;
-    a.workspace_bytes = tl_ws_bytes;
-    a.sk_counters = tl_sk_counters;
-  }
+  use_thread_workspace(a);
   static const int e_grp = [] { const char* e = getenv("AHA_GEMM_GROUP"); return e ? atoi(e) : 8; }();
   a.tile_group = e_grp;
   static const int e_prow = [] { const char* e = getenv("AHA_GEMM_PARTIAL_ROWS"); return e ? atoi(e) : 1; }();

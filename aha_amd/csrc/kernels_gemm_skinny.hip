@@ -131,7 +131,7 @@ double gemm_skinny_plan(const GemmArgs& a, int* r8_out) {
 // results they had.
 bool gemm_skinny_ok(const GemmArgs& a) {
   return a.few_rows && a.M >= 1 && a.M <= 256 && a.K >= 768 && a.K % 64 == 0 && a.N % 8 == 0 && a.groups == 1 && (a.act != ACT_SILU_MUL_PAIRS || a.N % 32 == 0) &&
-         (a.M <= 32 || (int64_t)a.N * a.K >= (a.M <= 64 ? 1 << 20 : 1 << 21));
+         (a.few_rows == 2 || a.M <= 32 || (int64_t)a.N * a.K >= (a.M <= 64 ? 1 << 20 : 1 << 21));
 }
 
 void launch_gemm_skinny(const GemmArgs& a, hipStream_t st) {

@@ -1079,8 +1079,13 @@ static int gemm_row_parallel(aha_model* m, GemmArgs g, int rows_per_rank = 0) {
       if (on_comm_stream && hipEventRecord(m->ev_comm, m->comm_stream) == hipSuccess) (void)hipStreamWaitEvent(m->stream, m->ev_comm, 0);
       return code;
     };
+    GemmArgs whole = g;   // (the unchunked launch below)
+    whole.residual = nullptr;
+    whole.act = ACT_PARTIAL_F32;
+    const int few_rows = gemm_takes_few_rows(whole) ? 2 : 0;   // every block on the kernel of the whole projection: the same sums, however it is cut
     for (int j = 0; j < nch; ++j) {
       GemmArgs gj = g;
+      gj.few_rows = few_rows;
       gj.W = (const bf16_t*)g.W + (int64_t)j * Nc * g.ldw;
       gj.C = m->p_partial + (size_t)j * rows_pad * Nc;
       gj.N = Nc;

@@ -430,6 +430,43 @@ def test_tp2_column_chunked_reduce_scatter_equals_the_unchunked_paths(gpu, S, mo
         np.testing.assert_array_equal(outs[mode][1], outs["allreduce"][1])
 
 
+@pytest.mark.parametrize("S", [5, 40, 96, 250])
+def test_tp2_prefill_of_few_rows_at_wide_layers(gpu, S, monkeypatch):
+    """The three paths of the two tests above where the row-parallel projections of a rank (2048 x 1024) run on the few-row kernel, which the widths there
+    (K < 768) never reach: 1 to 32 rows, up to 64, and row tiles.  A column block (512 x 1024) would take the tiled kernels by itself from 33 rows on; it
+    keeps the whole projection's kernel, so the logits stay equal bit for bit."""
+    from aha_amd import _lib
+    from aha_amd.model import HipInferenceModel
+    few = _lib.lib().aha_hip_debug_few_rows_gemm
+    partial = 5   # common.h ACT_PARTIAL_F32
+    assert few(S, 2048, 1024, partial, 0, 0, 1 << 30) > 0 and (few(S, 512, 1024, partial, 0, 0, 1 << 30) > 0) == (S <= 32)
+    cfg = tiny_qwen3(layers=2, hidden=2048, heads=16, kv_heads=4, inter=2048, vocab=1024)
+    w = qwen3_text_weights(cfg, seed=0)
+    ids = [int(x) for x in np.random.default_rng(S).integers(0, cfg.vocab_size, size=S)]
+    outs = {}
+    for mode in ("allreduce", "sp", "sp_chunked"):
+        monkeypatch.setenv("AHA_TP_OVERLAP_MIN_ROWS", "1" if mode == "sp_chunked" else "1000000")
+        red = TwoRankSum()
+        sp = mode != "allreduce"
+        ranks = [HipInferenceModel(cfg, w, tp_rank=r, tp_size=2, allreduce=lambda p, n, r=r: red.allreduce(r, p, n),
+                                   reduce_scatter=(lambda p, n, r=r: red.reduce_scatter(r, p, n)) if sp else None,
+                                   all_gather=(lambda p, n, r=r: red.all_gather(r, p, n)) if sp else None) for r in range(2)]
+        got = run_ranks([lambda m=m: m.forward_initial(ids, 0)[0].copy() for m in ranks])
+        np.testing.assert_array_equal(got[0], got[1])
+        if sp:
+            assert red.rs_calls == 2 * cfg.num_hidden_layers * (4 if mode == "sp_chunked" else 1)
+        outs[mode] = got[0]
+        for m in ranks:
+            m.close()
+    np.testing.assert_array_equal(outs["sp"], outs["allreduce"])
+    np.testing.assert_array_equal(outs["sp_chunked"], outs["allreduce"])
+    single = HipInferenceModel(cfg, w)
+    # 22 roundings to bf16 between a token and its logits (ten per layer, the last norm, the logits), half an ulp = 2^-9 at most and 2^-9 / sqrt(3) in the
+    # mean of squares each; where they all fall differently on the two sides: sqrt(2 * 22) * 2^-9 / sqrt(3) = 0.0075
+    close(outs["sp"], single.forward_initial(ids, 0)[0], f"tp2 prefill of {S} rows", rms=0.0075)
+    single.close()
+
+
 @pytest.mark.parametrize("S,tile", [(1200, 256), (1201, 256), (1100, 192), (700, 128)])
 def test_tp2_chunked_all_gather_equals_the_single_all_gather(gpu, S, tile, monkeypatch):
     """Round 4 (model.hip norm_gather_gemm): the all-gather of the normalised rows in front of the column-parallel projections runs in row
