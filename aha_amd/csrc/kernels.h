@@ -231,7 +231,8 @@ double gemm_skinny_plan(const GemmArgs& a, int* r8_out);
 int gemm_skinny_rounds(const GemmArgs& a, int r8);   // blocks of r8 * 8 weight rows over the CUs
 void launch_gemm_skinny(const GemmArgs& a, hipStream_t st);
 // One launch over all row segments on the four-wave 256 x 256 / 256 x 192 kernels (plain and gate+up epilogues, whole K tiles, M >= 256);
-// any other shape: one launch_gemm per segment.  Every output element is the same K-ordered sum as in an ungrouped GEMM over its row.
+// any other shape: one launch_gemm per segment.  On the same kernel every output element is the same K-ordered sum as in an ungrouped GEMM over its
+// row; a short segment's own plan may be another (K slices, the few-row kernel).
 void launch_gemm_grouped(const GemmArgs& a, hipStream_t st);
 // split-K scratch used by launch_gemm calls of this THREAD whose GemmArgs carry none (the model sets it per forward)
 void set_gemm_workspace(void* ws, size_t bytes, void* sk_counters = nullptr);

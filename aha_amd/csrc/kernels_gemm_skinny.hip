@@ -129,6 +129,8 @@ double gemm_skinny_plan(const GemmArgs& a, int* r8_out) {
 // columns).  So do 33 to 64 rows of a matrix below 2 MB (512 x 1024: 10.2 against 5.2 us) and more rows of one below 4 MB.  Only small models have either -- the full-size ones have
 // K >= 768 throughout their text stacks, and their one small matrix, the router, is met by 33 to 64 rows only in that band -- and they keep the
 // results they had.
+// few_rows = 2: a column block of a projection that takes this kernel as a whole, whatever the block's own size (an element's sum has the same order for
+// every R8 and M8).
 bool gemm_skinny_ok(const GemmArgs& a) {
   return a.few_rows && a.M >= 1 && a.M <= 256 && a.K >= 768 && a.K % 64 == 0 && a.N % 8 == 0 && a.groups == 1 && (a.act != ACT_SILU_MUL_PAIRS || a.N % 32 == 0) &&
          (a.few_rows == 2 || a.M <= 32 || (int64_t)a.N * a.K >= (a.M <= 64 ? 1 << 20 : 1 << 21));

@@ -251,7 +251,7 @@ __global__ __launch_bounds__(1024) void topk_final_kernel(const float* x, const 
   }
 }
 
-// ---- larger vocabularies, few candidates of many waves: rounds over all candidates ------------------------------------------------------------------------------------------------
+// ---- larger vocabularies, few candidates of many waves: rounds over all candidates ----------------------------------------------------------------
 constexpr int S2_WAVES = 16;
 constexpr int S2_C = 20;  // 16 waves x 64 lanes x 20 >= 297 stage-1 waves x 64 candidates
 

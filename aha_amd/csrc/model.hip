@@ -1158,8 +1158,9 @@ static int prefill_norm(aha_model* m, const void* w, int S, int rows_per_rank) {
 // Every rank's row slice [r * spr, + spr) is cut at the same offsets into chunks of w rows (a multiple of 256: whole row tiles); chunk c
 // of all ranks is gathered into its own block of the staging buffer, laid out [rank][rows of the chunk] as ncclAllGather delivers it, on
 // the communication stream, while the matrix cores run chunk c - 1: ONE grouped GEMM launch per chunk (launch_gemm_grouped: T row
-// segments of the staging block -> the token-order rows r * spr + off .. of the output).  Rows are independent in a GEMM, so every
-// output element is the same K-ordered sum as in the unchunked form (tests/test_tp_gpu.py: bit-identical logits and KV).
+// segments of the staging block -> the token-order rows r * spr + off .. of the output).  Rows are independent in a GEMM, so on the same
+// kernel every output element is the same K-ordered sum as in the unchunked form (tests/test_tp_gpu.py: bit-identical logits and KV with the tile pinned;
+// the automatic plan of a short last chunk may be another than the whole prompt's).
 // cfg 5 on 8 GPUs: the gather moves 7/8 x 336 MB per rank in front of 0.25 ms (qkv) / 0.95 ms (gate+up) of GEMM per rank.
 static int tp_ag_chunk_rows(const aha_model* m, int S, int spr) {
   const char* e = getenv("AHA_TP_AG_CHUNKS");
