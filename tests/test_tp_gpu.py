@@ -438,7 +438,7 @@ def test_tp2_prefill_of_few_rows_at_wide_layers(gpu, S, monkeypatch):
     from aha_amd import _lib
     from aha_amd.model import HipInferenceModel
     few = _lib.lib().aha_hip_debug_few_rows_gemm
-    partial = 5   # common.h ACT_PARTIAL_F32
+    partial = 5   # csrc/kernels.h ACT_PARTIAL_F32
     assert few(S, 2048, 1024, partial, 0, 0, 1 << 30) > 0 and (few(S, 512, 1024, partial, 0, 0, 1 << 30) > 0) == (S <= 32)
     cfg = tiny_qwen3(layers=2, hidden=2048, heads=16, kv_heads=4, inter=2048, vocab=1024)
     w = qwen3_text_weights(cfg, seed=0)
