@@ -17,6 +17,8 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-u
 # no packed f32 arithmetic: some operand forms of v_pk_{add,mul,fma}_f32 were measured to read the wrong element (profiles/r03_simd_coresidency.md),
 # and hipcc forms them from ordinary float code.  (The host pass does not know the feature and warns; harmless.)
 FLAGS += ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+# the first 14 dwords of scalar kernel parameters are put into scalar registers by the launch (a kernel that takes a struct first is not touched)
+FLAGS += ["-Xarch_device", "-mllvm=-amdgpu-kernarg-preload-count=16"]
 # Debug builds (measurement scripts only; never the shipped library): AHA_BUILD_DEFINES="-DAHA_DEBUG_KERNELS" compiles the ablation / trace
 # instantiations and their environment dispatch in (README "Debug kernels"); the flags are part of the build digest.
 FLAGS += [f for f in os.environ.get("AHA_BUILD_DEFINES", "").split() if f.startswith("-D")]

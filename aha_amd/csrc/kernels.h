@@ -137,6 +137,7 @@ struct AttnDecodeFusedArgs {
   unsigned long long* trace;  // optional timeline (AHA_ATTN_TRACE)
   int nh, kvh, nsplit;
   float eps, scale;
+  int traced = 1;           // deferred merge only: `trace` is there (known without a load)
 };
 void launch_attn_decode_fused(const AttnDecodeFusedArgs& a, hipStream_t st);
 // The same with the partials left for launch_gemv_merge (nsplit > 1; a single split writes `o`): nsplit from attn_decode_defer_splits, 0 = not here

@@ -19,9 +19,9 @@ namespace aha {
 namespace {
 
 template <int R, int U, int EPI, bool FAST>
-__global__ __launch_bounds__(GEMV_THREADS) void gemv_kernel(GemvArgs a) {
+__global__ __launch_bounds__(GEMV_THREADS) void gemv_kernel(GEMV_HOT_PARAMS, GemvArgs rest) {
   extern __shared__ __attribute__((aligned(16))) float xs[];  // K f32 + 8 floats reduction scratch
-  gemv_body<R, U, EPI, false, FAST>(a, xs, (int)blockIdx.x, (int)gridDim.x, [] {});
+  gemv_body<R, U, EPI, false, FAST>(gemv_args<EPI>(rest, GEMV_HOT), xs, (int)blockIdx.x, nblk, [] {});
 }
 
 }  // namespace
@@ -88,8 +88,8 @@ static void launch_gemv_epi(const GemvArgs& a, const GemvPlan& p, hipStream_t st
   const bool fast = fast_ok && a.K % (512 * p.U) == 0 && !a.cached && a.N >= 1;
 #define GV(RR, UU)                                                                            \
   do {                                                                                        \
-    if (fast) hipLaunchKernelGGL((gemv_kernel<RR, UU, EPI, true>), grid, block, lds, st, a);  \
-    else hipLaunchKernelGGL((gemv_kernel<RR, UU, EPI, false>), grid, block, lds, st, a);      \
+    if (fast) hipLaunchKernelGGL((gemv_kernel<RR, UU, EPI, true>), grid, block, lds, st, GEMV_HOT_ARGS(a, EPI, p.grid), a);  \
+    else hipLaunchKernelGGL((gemv_kernel<RR, UU, EPI, false>), grid, block, lds, st, GEMV_HOT_ARGS(a, EPI, p.grid), a);      \
   } while (0)
   if (p.R == 4) {
     if (p.U >= 4) GV(4, 4); else if (p.U == 2) GV(4, 2); else GV(4, 1);

@@ -160,12 +160,13 @@ struct MergePro {
 };
 
 template <int R, int U, bool FAST, int XP, int MS>
-__global__ __launch_bounds__(GEMV_THREADS) void gemv_merge_kernel(GemvArgs a, GemvMerge p) {
+__global__ __launch_bounds__(GEMV_THREADS) void gemv_merge_kernel(const float* part_o, const float* part_ml, const void* W, const void* residual, unsigned long long* trace, int N, int K, int nsplit, int nblk,
+                                                                    GemvArgs rest) {
   extern __shared__ __attribute__((aligned(16))) float xs[];
   MergePro<XP, MS> pro;
-  pro.p = p;
-  pro.K = a.K;
-  gemv_body<R, U, GEMV_RESIDUAL, false, FAST>(a, xs, (int)blockIdx.x, (int)gridDim.x, [] {}, pro);
+  pro.p = GemvMerge{part_o, part_ml, nsplit, K >> 7};
+  pro.K = K;
+  gemv_body<R, U, GEMV_RESIDUAL, false, FAST>(gemv_args<GEMV_RESIDUAL>(rest, nullptr, W, nullptr, residual, trace, N, K, 0.f), xs, (int)blockIdx.x, nblk, [] {}, pro);
 }
 template <int R, int U, int EPI, bool FAST, int XP>
 __global__ __launch_bounds__(GEMV_THREADS) void gemv_postnorm_kernel(GemvArgs a, GemvPostNorm p) {
@@ -216,7 +217,8 @@ void launch_gemv_merge(const GemvArgs& a, const GemvMerge& p, hipStream_t st) {
     constexpr int R = decltype(r)::value, U = decltype(u)::value;
     const dim3 grid(pl.grid), block(GEMV_THREADS);
     auto run = [&](auto fast, auto xp, auto ms) {
-      hipLaunchKernelGGL((gemv_merge_kernel<R, U, decltype(fast)::value, decltype(xp)::value, decltype(ms)::value>), grid, block, fused_lds(a), st, a, p);
+      hipLaunchKernelGGL((gemv_merge_kernel<R, U, decltype(fast)::value, decltype(xp)::value, decltype(ms)::value>), grid, block, fused_lds(a), st, p.part_o, p.part_ml, a.W, a.residual, a.trace, a.N, a.K, p.nsplit, pl.grid,
+                         a);
     };
     using std::integral_constant;
     auto by_k = [&](auto fast) {
