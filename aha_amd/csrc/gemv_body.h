@@ -35,16 +35,19 @@ struct gemv_mapped<Pro, std::enable_if_t<Pro::MAPPED>> : std::true_type {};
 // What a matvec needs before its first loads can go out travels as leading scalar parameters: up to 14 dwords of them are in scalar registers when a
 // wave starts (-amdgpu-kernarg-preload-count, build.py), where a member of the argument struct, or gridDim, is a load from the argument buffer that
 // every CU waits for first.  With it in the matvecs and the decode attention a 0.6B step's 141 dependent launches take 0.3 us less each: 222 -> 209 ms
-// for 2048 + 256 tokens, 213 -> 209 ms for an 8B answer of 64 tokens, the same bits.  aux: the up matrix of GEMV_SILU_MUL, else the residual.
+// for 2048 + 256 tokens, 213 -> 209 ms for an 8B answer of 64 tokens, the same bits.  aux: the up matrix of GEMV_SILU_MUL, else the residual
+// (GEMV_AXPY_F32: the 32-bit one).
 #define GEMV_HOT_PARAMS const void *x, const void *W, const void *norm_w, const void *aux, unsigned long long *trace, int N, int K, float eps, int nblk
 #define GEMV_HOT x, W, norm_w, aux, trace, N, K, eps
-#define GEMV_HOT_ARGS(a, epi, grid) (a).x, (a).W, (a).norm_w, (epi) == GEMV_SILU_MUL ? (a).W2 : (a).residual, (a).trace, (a).N, (a).K, (a).eps, (int)(grid)
+#define GEMV_HOT_ARGS(a, epi, grid) (a).x, (a).W, (a).norm_w, (epi) == GEMV_SILU_MUL ? (a).W2 : (epi) == GEMV_AXPY_F32 ? (const void*)(a).res_f32 : (a).residual, (a).trace, (a).N, (a).K, (a).eps, (int)(grid)
 template <int EPI>
 __device__ __forceinline__ GemvArgs gemv_args(GemvArgs a, const void* x, const void* W, const void* norm_w, const void* aux, unsigned long long* trace, int N, int K, float eps) {
   a.x = x;
   a.W = W;
   a.norm_w = norm_w;
-  (EPI == GEMV_SILU_MUL ? a.W2 : a.residual) = aux;
+  if (EPI == GEMV_SILU_MUL) a.W2 = aux;
+  else if (EPI == GEMV_AXPY_F32) a.res_f32 = (const float*)aux;
+  else a.residual = aux;
   a.trace = trace;
   a.N = N;
   a.K = K;

@@ -12,7 +12,7 @@
 // Rounding points follow the reference's op boundaries: Linear output -> bf16, then each further op -> bf16.
 #include <stdlib.h>
 
-#include "gemv_body.h"
+#include "gemv_row_body.h"
 
 namespace aha {
 
@@ -22,6 +22,12 @@ template <int R, int U, int EPI, bool FAST>
 __global__ __launch_bounds__(GEMV_THREADS) void gemv_kernel(GEMV_HOT_PARAMS, GemvArgs rest) {
   extern __shared__ __attribute__((aligned(16))) float xs[];  // K f32 + 8 floats reduction scratch
   gemv_body<R, U, EPI, false, FAST>(gemv_args<EPI>(rest, GEMV_HOT), xs, (int)blockIdx.x, nblk, [] {});
+}
+
+template <int R, int U, int EPI, bool NORM>
+__global__ __launch_bounds__(GEMV_THREADS) void gemv_row_kernel(GEMV_HOT_PARAMS, GemvArgs rest) {
+  RowNormPro<U, NORM> pro{(const bf16_t*)x, (const bf16_t*)norm_w, eps};
+  gemv_row_body<R, U, EPI>(rest, W, aux, trace, N, (int)blockIdx.x, nblk, pro);
 }
 
 }  // namespace
@@ -79,8 +85,43 @@ GemvPlan plan_gemv(int N, int K, GemvEpi epi) {
 
 int gemv_num_tiles(int N, int K) { return plan_gemv(N, K, GEMV_LOGITS).grid; }
 
+// gemv_row_kernel where a wave's load group is a whole row of up to 3072 columns (0.6B: 2048 + 256 tokens
+// 209 -> 182 ms, 19 + 12 sampled ones 10.4 -> 9.1; at 4096 columns and 8B outputs the vector's registers cost a block per CU and the launch streams for longer than it ramps: 208.7 -> 210.3 ms per
+// 64-token answer with it).  false = not such a shape, nothing launched.
+template <int EPI>
+static bool launch_gemv_row(const GemvArgs& a, const GemvPlan& p, hipStream_t st) {
+  if (a.K % 512 != 0 || a.cached || a.h_out != nullptr || p.R > 2 || a.N < 1) return false;
+  auto go = [&](auto r, auto u) {
+    constexpr int R = decltype(r)::value, U = decltype(u)::value;
+    constexpr bool CAN_NORM = EPI == GEMV_STORE || EPI == GEMV_SILU_MUL || EPI == GEMV_PARTIAL_F32;
+    const dim3 grid(p.grid), block(GEMV_THREADS);
+    if (a.norm_w == nullptr) {
+      hipLaunchKernelGGL((gemv_row_kernel<R, U, EPI, false>), grid, block, 0, st, GEMV_HOT_ARGS(a, EPI, p.grid), a);
+      return true;
+    }
+    if constexpr (CAN_NORM) hipLaunchKernelGGL((gemv_row_kernel<R, U, EPI, true>), grid, block, 0, st, GEMV_HOT_ARGS(a, EPI, p.grid), a);
+    return CAN_NORM;
+  };
+  using std::integral_constant;
+  const int u = a.K / 512;
+  if (p.R == 2) {
+    if (u == 2) return go(integral_constant<int, 2>{}, integral_constant<int, 2>{});
+    if constexpr (EPI != GEMV_SILU_MUL)
+      if (u == 4) return go(integral_constant<int, 2>{}, integral_constant<int, 4>{});
+    return false;
+  }
+  if (u == 2) return go(integral_constant<int, 1>{}, integral_constant<int, 2>{});
+  if (u == 3) return go(integral_constant<int, 1>{}, integral_constant<int, 3>{});
+  if (u == 4) return go(integral_constant<int, 1>{}, integral_constant<int, 4>{});
+  if constexpr (EPI != GEMV_SILU_MUL)   // (two matrices: two buffers of that many loads leave two blocks per CU)
+    if (u == 6) return go(integral_constant<int, 1>{}, integral_constant<int, 6>{});
+  return false;
+}
+
 template <int EPI>
 static void launch_gemv_epi(const GemvArgs& a, const GemvPlan& p, hipStream_t st) {
+  if constexpr (EPI != GEMV_LOGITS)
+    if (launch_gemv_row<EPI>(a, p, st)) return;
   const size_t lds = (size_t)((a.K + 511) / 512) * 512 * 4 + 64;
   dim3 grid(p.grid), block(GEMV_THREADS);
   // FAST form (gemv_body.h): every chunk group full and in range, weights non-temporal

@@ -71,6 +71,22 @@ def test_gemv(gpu, N, K, fuse_norm, residual):
     assert_close_ulps(got, ref, 1, 0.98, "gemv")
 
 
+@pytest.mark.parametrize("K", [1024, 1536, 2048, 3072])
+@pytest.mark.parametrize("N", [1, 7, 1030, 3073, 4101, 8195])
+def test_gemv_one_load_group_per_row(gpu, N, K):
+    """gemv_row_body.h: odd ends of the last tile, one to three tiles per block, one and two rows per wave; with and without norm / residual, and gate + up."""
+    from aha_amd import ops
+    W, Wu, x, nw, res = rnd((N, K), 3, 0.02), rnd((N, K), 8, 0.02), rnd((K,), 4), rnd((K,), 5, 0.02, 1.0), rnd((N,), 6)
+    plain, h = NM.linear(x.float()[None], W.float())[0], oq.rms_norm(NM, x.float(), nw.float(), 1e-6)
+    normed, up = NM.linear(h[None], W.float())[0], NM.linear(h[None], Wu.float())[0]
+    Wg_, Wu_, x_, nw_, res_ = (t.to(gpu) for t in (W, Wu, x, nw, res))
+    # (a few ten values at N = 1 and 7: every one within the bound instead of a share of them)
+    assert_close_ulps(ops.gemv(Wg_, x_), plain, 1, 0.98 if N > 100 else 0.0, "plain")
+    assert_close_ulps(ops.gemv(Wg_, x_, nw_, 1e-6), normed, 1, 0.98 if N > 100 else 0.0, "norm")
+    assert_close_ulps(ops.gemv(Wg_, x_, None, 1e-6, res_), NM.r(res.float() + plain), 1, 0.98 if N > 100 else 0.0, "residual")
+    assert_close_ulps(ops.gemv_gate_up(Wg_, Wu_, x_, nw_, 1e-6), NM.r(NM.r(oq.silu(normed)) * up), 2, 0.97 if N > 100 else 0.0, "gate_up")
+
+
 @pytest.mark.parametrize("I,K", [(3072, 1024), (12288, 4096), (1024, 512)])
 def test_gemv_gate_up(gpu, I, K):
     from aha_amd import ops
