@@ -35,7 +35,7 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
   bf16_t* qs = reinterpret_cast<bf16_t*>(smem);                 // [16][128]
   bf16_t* ksn = qs + 16 * 128;                                  // [128]
   bf16_t* vsn = ksn + 128;                                      // [128]
-  const int g = a.nh / a.kvh, P = DEFER ? g : 16;               // P: q slots
+  const int g = DEFER ? a.group : a.nh / a.kvh, P = DEFER ? g : 16;               // P: q slots
   float* mo = reinterpret_cast<float*>(vsn + 128);              // per wave O [NW][q P][d 128]
   float* mm = mo + NW * 128 * P;                                // [NW][16]
   float* mlz = mm + NW * 16;                                    // [NW][16]
@@ -44,7 +44,7 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, G = lane >> 4, c = lane & 15;
   const int nunits = nsplit * NW, unit = DEFER ? wave * nsplit + split : split * NW + wave;   // (DEFER: neighbouring pages to different blocks)
-  const int L = a.kv_len_v, slot_new = a.kv_start_v;
+  const int L = a.kv_len_v, slot_new = DEFER ? L - 1 : a.kv_start_v;
   const int L_old = L - 1;  // tokens already in the pages; the new one is handled from LDS
   const int npages = (L_old + KV_PAGE_TOKENS - 1) / KV_PAGE_TOKENS;
 
@@ -66,8 +66,13 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
   const bf16_t px0 = p_src[lane], px1 = p_src[lane + 64];
   const bf16_t pw0 = p_nw[lane], pw1 = p_nw[lane + 64];
   const float cs = a.rope[lane], sn = a.rope[64 + lane];   // bf16-representable values (rope_step_kernel)
-  bf16_t vnew = 0;
-  if (tid < 128) vnew = qkv[(int64_t)(a.nh + a.kvh + kvhd) * 128 + tid];
+  // more heads than waves (g >= 4): the second item of some waves, requested here too (DEFER), in front of the pages
+  const int h2 = wave + NW;
+  const bf16_t* p_src2 = qkv + (int64_t)(h2 >= g ? a.nh + kvhd : kvhd * g + h2) * 128;
+  const bf16_t* p_nw2 = (const bf16_t*)(h2 >= g ? a.k_norm_w : a.q_norm_w);
+  bf16_t px2 = 0, px3 = 0, pw2 = 0, pw3 = 0;
+  if (DEFER) px2 = p_src2[lane], px3 = p_src2[lane + 64], pw2 = p_nw2[lane], pw3 = p_nw2[lane + 64];
+  const bf16_t vnew = qkv[(int64_t)(a.nh + a.kvh + kvhd) * 128 + (tid & 127)];
 
   u32x4_t kf[4][4], vf[8][2];
   // Addresses: wave-uniform 64-bit base (scalar registers) + ONE 32-bit per-lane offset (lane * 16), the rest immediates:
@@ -75,7 +80,21 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
   // contiguous per wave instruction.
   typedef const __attribute__((address_space(1))) char* gchar_t;
   const uint32_t l_off = (uint32_t)lane * 16;
-  auto load_k = [&](uint64_t base) {
+  // DEFER: through a descriptor whose range is empty for a unit without pages.  Under a branch around the requests the compiler's wait for the prologue's
+  // inputs, good for both sides of the join, would be a wait for the pages (returns are in order), and norm and rope stood behind them.
+  auto page_rsrc = [&](uint64_t base, bool have) {
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(base), 0, have ? a.kvh * KV_PAGE_TOKENS * 512 : 0, 0x00020000);
+  };
+  auto load_k = [&](uint64_t base, bool have = true) {
+    if constexpr (DEFER) {
+      const auto rs = page_rsrc(base, have);
+      const int at = kvhd * KV_PAGE_TOKENS * 256;
+#pragma unroll
+      for (int sub = 0; sub < 4; ++sub)
+#pragma unroll
+        for (int k4 = 0; k4 < 4; ++k4) kf[sub][k4] = __builtin_amdgcn_raw_buffer_load_b128(rs, l_off + (sub * 4 + k4) % 4 * 1024, at + (sub * 4 + k4) / 4 * 4096, 2 /* nt */);
+      return;
+    }
     gchar_t kb = reinterpret_cast<gchar_t>(base + (uint64_t)kvhd * KV_PAGE_TOKENS * 256);
 #pragma unroll
     for (int sub = 0; sub < 4; ++sub)
@@ -83,7 +102,16 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
       for (int k4 = 0; k4 < 4; ++k4)
         kf[sub][k4] = __builtin_nontemporal_load(reinterpret_cast<gptr16_t>(kb + (sub * 4 + k4) * 1024 + l_off));
   };
-  auto load_v = [&](uint64_t base) {
+  auto load_v = [&](uint64_t base, bool have = true) {
+    if constexpr (DEFER) {
+      const auto rs = page_rsrc(base, have);
+      const int at = (a.kvh + kvhd) * KV_PAGE_TOKENS * 256;
+#pragma unroll
+      for (int ds = 0; ds < 8; ++ds)
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) vf[ds][kk] = __builtin_amdgcn_raw_buffer_load_b128(rs, l_off + (ds * 2 + kk) % 4 * 1024, at + (ds * 2 + kk) / 4 * 4096, 2 /* nt */);
+      return;
+    }
     gchar_t vb = reinterpret_cast<gchar_t>(base + (uint64_t)a.kvh * KV_PAGE_TOKENS * 256 + (uint64_t)kvhd * 128 * (KV_PAGE_TOKENS * 2));
 #pragma unroll
     for (int ds = 0; ds < 8; ++ds)
@@ -94,10 +122,15 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
   // This unit's page pointers (pages unit, unit + nunits, ...): ONE vector load up front, lane i holding the i-th of them,
   // broadcast per iteration with v_readlane.  (A load of page_ptrs[page] inside the loop is a VECTOR load -- the kernel also
   // stores, so the compiler will not use the scalar cache -- and its wait drains the K/V requests queued behind it.)
+  // DEFER: a unit has at most three pages, so lane 63 holds the new token's; and where the pages follow each other at one distance (a cache inside one
+  // slab) their addresses are arithmetic: the first page is requested in the same breath as the prologue's inputs instead of a round trip behind them
+  // (this and the descriptors below: 2048 + 256 tokens of 0.6B 181.7 -> 171.8 ms, 64 tokens of 8B 208.3 -> 206.0; the same bits).
   uint64_t my_pages = 0;
   auto fetch_page_ptrs = [&](int first_it) {
-    const int pg = unit + (first_it + lane) * nunits;
-    my_pages = pg < npages ? (uint64_t)(a.kv.page_ptrs[pg] + a.kv.layer_off) : 0;
+    const bool is_new = DEFER && lane == 63;
+    const int pg = is_new ? slot_new / KV_PAGE_TOKENS : unit + (first_it + lane) * nunits;
+    if (DEFER && a.page_stride != 0) my_pages = (uint64_t)(uintptr_t)a.kv.page_ptrs + (uint64_t)pg * a.page_stride;
+    else if (is_new || pg < npages) my_pages = (uint64_t)(a.kv.page_ptrs[pg] + a.kv.layer_off);
   };
   auto page_base = [&](int i) {
     const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)my_pages, i & 63), hi = __builtin_amdgcn_readlane((uint32_t)(my_pages >> 32), i & 63);
@@ -105,12 +138,12 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
   };
   fetch_page_ptrs(0);
   int page = unit, it = 0;
-  if (page < npages) {
+  if (DEFER || page < npages) {
     const uint64_t b0 = page_base(0);
     __builtin_amdgcn_sched_barrier(0);  // K strictly ahead of V (as in the loop): the loop's counted waits assume that order
-    load_k(b0);
+    load_k(b0, page < npages);
     __builtin_amdgcn_sched_barrier(0);
-    load_v(b0);
+    load_v(b0, page < npages);
     __builtin_amdgcn_sched_barrier(0);
   }
 
@@ -128,7 +161,8 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
       dst[lane + 64] = y1;
     };
     if (p_have) norm_rope(px0, px1, pw0, pw1, p_is_k ? ksn : qs + wave * 128);
-    for (int hs = wave + NW; hs <= g; hs += NW) {  // more heads than waves (g >= 4): a second round for some waves
+    if (DEFER && h2 <= g) norm_rope(px2, px3, pw2, pw3, h2 == g ? ksn : qs + h2 * 128);
+    for (int hs = wave + (DEFER ? 2 : 1) * NW; hs <= g; hs += NW) {  // more heads than waves (g >= 4): a second round for some waves
       const bool is_k = hs == g;
       const bf16_t* src = is_k ? qkv + (int64_t)(a.nh + kvhd) * 128 : qkv + (int64_t)(kvhd * g + hs) * 128;
       const bf16_t* nw = (const bf16_t*)(is_k ? a.k_norm_w : a.q_norm_w);
@@ -142,7 +176,7 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
     // global address space spelled out: a flat store here would make every later wait in the kernel a vmcnt(0)
     typedef __attribute__((address_space(1))) bf16_t* gbf_t;
     const int pg = slot_new / KV_PAGE_TOKENS, t = slot_new % KV_PAGE_TOKENS;
-    const uint64_t base = (uint64_t)(a.kv.page_ptrs[pg] + a.kv.layer_off);
+    const uint64_t base = DEFER ? page_base(63) : (uint64_t)(a.kv.page_ptrs[pg] + a.kv.layer_off);
     gbf_t kd = reinterpret_cast<gbf_t>(base) + (int64_t)kvhd * KV_PAGE_TOKENS * 128;
     gbf_t vd = reinterpret_cast<gbf_t>(base) + (int64_t)a.kvh * KV_PAGE_TOKENS * 128 + (int64_t)kvhd * 128 * KV_PAGE_TOKENS;
     for (int i = tid; i < 128; i += NT) {

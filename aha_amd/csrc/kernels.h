@@ -137,7 +137,10 @@ struct AttnDecodeFusedArgs {
   unsigned long long* trace;  // optional timeline (AHA_ATTN_TRACE)
   int nh, kvh, nsplit;
   float eps, scale;
-  int traced = 1;           // deferred merge only: `trace` is there (known without a load)
+  // deferred merge only (the launcher's but for page_stride):
+  int group = 0;            // nh / kvh
+  int traced = 1;           // `trace` is there (known without a load)
+  uint32_t page_stride = 0; // > 0: page p of this layer is at kv.page_ptrs (then an address, no table) + p * page_stride, without layer_off
 };
 void launch_attn_decode_fused(const AttnDecodeFusedArgs& a, hipStream_t st);
 // The same with the partials left for launch_gemv_merge (nsplit > 1; a single split writes `o`): nsplit from attn_decode_defer_splits, 0 = not here

@@ -155,7 +155,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_fused_kernel(AttnDecodeFus
   attn_decode_fused_body<ATTN_DECODE_NW, false>(a, smem, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.y);
 }
 __global__ __launch_bounds__(256, 2) void attn_decode_defer_kernel(const void* qkv, const void* q_norm_w, const void* k_norm_w, const float* rope, const uint64_t* page_ptrs, int kv_len,
-                                                                       int heads, int nsplit, AttnDecodeFusedArgs a) {
+                                                                       int heads, int nsplit, unsigned page_stride, AttnDecodeFusedArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_defer[];
   // (what the first requests need: in scalar registers at the start, gemv_body.h)
   a.qkv = qkv;
@@ -164,8 +164,10 @@ __global__ __launch_bounds__(256, 2) void attn_decode_defer_kernel(const void* q
   a.rope = rope;
   a.kv.page_ptrs = page_ptrs;
   a.kv_len_v = kv_len;
-  a.nh = heads & 0x7fff;
+  a.page_stride = page_stride;
+  a.group = heads & 0x7fff;
   a.kvh = heads >> 16;
+  a.nh = a.group * a.kvh;
   a.traced = heads >> 15 & 1;
   attn_decode_fused_body<ATTN_DECODE_NW, true>(a, smem_defer, (int)blockIdx.x, (int)blockIdx.y, nsplit);
 }
@@ -191,7 +193,7 @@ int attn_decode_defer_splits(int npages, int nq) {
 void launch_attn_decode_defer(const AttnDecodeFusedArgs& a, hipStream_t st) {
   const int lds = 16 * 128 * 2 + 2 * 128 * 2 + ATTN_DECODE_NW * 128 * (a.nh / a.kvh) * 4 + (2 * ATTN_DECODE_NW + 1) * 16 * 4;
   hipLaunchKernelGGL(attn_decode_defer_kernel, dim3(a.kvh, a.nsplit), dim3(256), lds, st, a.qkv, a.q_norm_w, a.k_norm_w, a.rope, a.kv.page_ptrs, a.kv_len_v,
-                     a.kvh << 16 | (a.trace != nullptr) << 15 | a.nh, a.nsplit, a);
+                     a.kvh << 16 | (a.trace != nullptr) << 15 | a.nh / a.kvh, a.nsplit, a.page_stride, a);
 }
 
 static int g_attn_smx_override = -1;

@@ -1447,6 +1447,11 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_read
   int defer = e_div || !m->decode_fused ? 0 : attn_decode_defer_splits(npages, nq);
   if (defer > 1 && m->tp_size > 1) defer = 0;
   if (defer) nsplit = defer;
+  // pages at one distance from each other: the attention computes their addresses
+  uint64_t page_stride = defer ? m->page_bytes : 0;
+  for (int p = 1; p < npages && page_stride; ++p)
+    if (m->h_page_ptrs[p] != m->h_page_ptrs[0] + p * page_stride) page_stride = 0;
+  if (page_stride > 0xffffffffu) page_stride = 0;
   for (int li = 0; li < c.num_hidden_layers; ++li) {
     const LayerWeights& L = m->layers[li];
     {  // h = RMSNorm(x); qkv = h Wqkv^T                      (qwen3/model.rs:79, modules.rs:538-552)
@@ -1466,6 +1471,10 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_read
       a.scale = m->attn_scale; a.o = m->d_attn; a.head_ctr = m->d_bar + DECODE_HEAD_CTR_WORD;
       if (nsplit > 1 && !defer) m->head_ctr_base += (unsigned)nsplit;  // (neither a single split nor a deferred merge touches the counter)
       a.ctr_target = m->head_ctr_base;
+      if (page_stride) {
+        a.kv.page_ptrs = (const uint64_t*)(uintptr_t)(m->h_page_ptrs[0] + a.kv.layer_off);
+        a.page_stride = (uint32_t)page_stride;
+      }
       static const char* e_at = getenv("AHA_ATTN_TRACE");
       if (e_at && atoi(e_at)) {
         if (!m->d_attn_trace) {
