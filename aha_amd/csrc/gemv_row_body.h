@@ -6,8 +6,17 @@
 
 namespace aha {
 
+// Blocks of a launch: two per CU at most, and whole rounds of tiles.  Three per CU (gemv_kernel's) find the second and third waiting for the first's
+// requests anyway and make the vector travel once more each: 2048 + 256 tokens of 0.6B 167.8 ms with 768 blocks, 166.1 with 384 and 512, 169.0 with 1024.
+inline int gemv_row_grid(int N, int R) {
+  const int ntiles = (N + 4 * R - 1) / (4 * R), rounds = (ntiles + 511) / 512;
+  return (ntiles + rounds - 1) / rounds;
+}
+
 // The input vector as a prologue leaves it: a lane's share of it is the columns of its own weights, h[u][i] = column 512 u + 8 lane + i.  A prologue is
-// a type with request(), its loads, issued ahead of the first weight tile (returns are in order within a wave), and make(h).
+// a type with request(), its loads, issued ahead of the first weight tile (returns are in order within a wave), and make(h).  With MAPPED it says too where
+// the weights are, ptr(row, u) -> this lane's columns of load u (GEMV_SILU_MUL: of the gate row; the up row 16 further), and what a row's sums are
+// multiplied by, scale(row) (GEMV_SILU_MUL only).
 //
 // h = x, or h = bf16(RMSNorm(x) * norm_w): every wave norms the whole row in its registers, no LDS and no barrier; the partial sums in the order of the
 // block form (chunks 0, 4, .. | 1, 5, .. | 2, 6, .. | 3, 7, ..), so the bits are the same.
@@ -50,6 +59,57 @@ struct RowNormPro {
   }
 };
 
+// h = (x - mean) / sqrt(var + eps) * w + b over `width` columns, x in 32 bits, w and b zero behind them; by every wave for itself as well
+template <int U>
+struct RowLayerNormPro {
+  const float* x;
+  const bf16_t *w, *b;
+  float eps;
+  int width;
+  float4 s[U][2];
+  u32x4_t wr[U], br[U];
+  __device__ __forceinline__ void request() {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      s[u][0] = *reinterpret_cast<const float4*>(x + u * 512 + lane * 8);
+      s[u][1] = *reinterpret_cast<const float4*>(x + u * 512 + lane * 8 + 4);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) wr[u] = ld16(w + u * 512 + lane * 8);
+#pragma unroll
+    for (int u = 0; u < U; ++u) br[u] = ld16(b + u * 512 + lane * 8);
+  }
+  __device__ __forceinline__ void make(float (&h)[U][8]) {
+    const int lane = threadIdx.x & 63;
+    float sum = 0.f;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) sum += (s[u][i].x + s[u][i].y) + (s[u][i].z + s[u][i].w);   // (pad columns are zero)
+    const float mean = wave_sum(sum) / (float)width;
+    sum = 0.f;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) { h[u][4 * i] = s[u][i].x; h[u][4 * i + 1] = s[u][i].y; h[u][4 * i + 2] = s[u][i].z; h[u][4 * i + 3] = s[u][i].w; }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        h[u][i] = u * 512 + lane * 8 + i < width ? h[u][i] - mean : 0.f;
+        sum += h[u][i] * h[u][i];
+      }
+    }
+    const float rinv = 1.0f / sqrtf(wave_sum(sum) / (float)width + eps);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        h[u][2 * j] = fmaf(h[u][2 * j] * rinv, lo_bf(wr[u][j]), lo_bf(br[u][j]));
+        h[u][2 * j + 1] = fmaf(h[u][2 * j + 1] * rinv, hi_bf(wr[u][j]), hi_bf(br[u][j]));
+      }
+  }
+};
+
 // aux: see GEMV_HOT_PARAMS.  Of `rest` only the outputs (and res_scale) are read, behind the first weights.
 template <int R, int U, int EPI, class Pro>
 __device__ __forceinline__ void gemv_row_body(const GemvArgs& rest, const void* W, const void* aux, unsigned long long* trace, const int N, const int bid, const int nblk, Pro& pro) {
@@ -85,6 +145,12 @@ __device__ __forceinline__ void gemv_row_body(const GemvArgs& rest, const void* 
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
+        if constexpr (gemv_mapped<Pro>::value) {
+          const bf16_t* p = pro.ptr(row, u);
+          buf[0][r][u] = ld_nt16(p);
+          if (NW == 2) buf[NW - 1][r][u] = ld_nt16(p + 16 * KK);
+          continue;
+        }
         buf[0][r][u] = ld_nt16(p0 + u * 512 + lane * 8);
         if (NW == 2) buf[NW - 1][r][u] = ld_nt16(p1 + u * 512 + lane * 8);
       }
@@ -121,6 +187,14 @@ __device__ __forceinline__ void gemv_row_body(const GemvArgs& rest, const void* 
     for (int m = 0; m < NW; ++m)
 #pragma unroll
       for (int r = 0; r < R; ++r) acc[m][r] = wave_sum(acc[m][r]);
+    if constexpr (gemv_mapped<Pro>::value && EPI == GEMV_SILU_MUL) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const float s = pro.scale(min((tile * GEMV_WAVES + wave) * R + r, N - 1));
+#pragma unroll
+        for (int m = 0; m < NW; ++m) acc[m][r] *= s;
+      }
+    }
     if (lane == 0) {
 #pragma unroll
       for (int r = 0; r < R; ++r) {

@@ -94,12 +94,13 @@ static bool launch_gemv_row(const GemvArgs& a, const GemvPlan& p, hipStream_t st
   auto go = [&](auto r, auto u) {
     constexpr int R = decltype(r)::value, U = decltype(u)::value;
     constexpr bool CAN_NORM = EPI == GEMV_STORE || EPI == GEMV_SILU_MUL || EPI == GEMV_PARTIAL_F32;
-    const dim3 grid(p.grid), block(GEMV_THREADS);
+    const int nblk = gemv_row_grid(a.N, R);
+    const dim3 grid(nblk), block(GEMV_THREADS);
     if (a.norm_w == nullptr) {
-      hipLaunchKernelGGL((gemv_row_kernel<R, U, EPI, false>), grid, block, 0, st, GEMV_HOT_ARGS(a, EPI, p.grid), a);
+      hipLaunchKernelGGL((gemv_row_kernel<R, U, EPI, false>), grid, block, 0, st, GEMV_HOT_ARGS(a, EPI, nblk), a);
       return true;
     }
-    if constexpr (CAN_NORM) hipLaunchKernelGGL((gemv_row_kernel<R, U, EPI, true>), grid, block, 0, st, GEMV_HOT_ARGS(a, EPI, p.grid), a);
+    if constexpr (CAN_NORM) hipLaunchKernelGGL((gemv_row_kernel<R, U, EPI, true>), grid, block, 0, st, GEMV_HOT_ARGS(a, EPI, nblk), a);
     return CAN_NORM;
   };
   using std::integral_constant;

@@ -6,6 +6,7 @@
 //   attention merge:               h = the split-KV attention partials of a decode step joined (attn_decode_body.h, DEFER)
 //   PolyNorm:                      h = a N(z) + b N(z^2) + c N(z^3) + e: the three row sums in the prologue
 #include "gemv_prologues.h"
+#include "gemv_row_body.h"
 
 namespace aha {
 
@@ -159,6 +160,65 @@ struct MergePro {
   __device__ __forceinline__ void finish(int, int) {}
 };
 
+// The same for K = 512 * U: a thread's group j of 4 columns is merged as above, the result read back from LDS as the columns of the lane's weights.
+template <int U, int MS>
+struct RowMergePro {
+  static constexpr int K = U * 512, XP = K / (4 * GEMV_THREADS);
+  const float* part_o;
+  const float* part_ml;
+  int nsplit;
+  float* xs;   // LDS, K floats
+  float4 v[XP][MS];
+  float2 ml[XP][MS];
+  __device__ __forceinline__ void request() {
+#pragma unroll
+    for (int s = 0; s < MS; ++s) {
+      const int64_t at = min(s, nsplit - 1) * (K / 128);   // (surplus slots repeat the last split: its lines are on their way)
+#pragma unroll
+      for (int j = 0; j < XP; ++j) ml[j][s] = *reinterpret_cast<const float2*>(part_ml + at * 2 + (j * GEMV_THREADS + threadIdx.x) / 32 * 2);
+    }
+#pragma unroll
+    for (int s = 0; s < MS; ++s) {
+      const int64_t at = min(s, nsplit - 1) * K;
+#pragma unroll
+      for (int j = 0; j < XP; ++j) v[j][s] = *reinterpret_cast<const float4*>(part_o + at + (j * GEMV_THREADS + threadIdx.x) * 4);
+    }
+  }
+  __device__ __forceinline__ void make(float (&h)[U][8]) {
+#pragma unroll
+    for (int j = 0; j < XP; ++j) {
+      float M = ml[j][0].x;
+#pragma unroll
+      for (int s = 1; s < MS; ++s) M = fmaxf(M, ml[j][s].x);
+      float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+      float z = 0.f;
+#pragma unroll
+      for (int s = 0; s < MS; ++s) {
+        const float w = s < nsplit && ml[j][s].x != -INFINITY ? __expf(ml[j][s].x - M) : 0.f;
+        z = fmaf(w, ml[j][s].y, z);
+        o.x = fmaf(w, v[j][s].x, o.x); o.y = fmaf(w, v[j][s].y, o.y); o.z = fmaf(w, v[j][s].z, o.z); o.w = fmaf(w, v[j][s].w, o.w);
+      }
+      const float inv = 1.0f / z;
+      *xs4(xs, (j * GEMV_THREADS + threadIdx.x) * 4) = make_float4(rbf(o.x * inv), rbf(o.y * inv), rbf(o.z * inv), rbf(o.w * inv));
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float4 lo = *xs4(xs, u * 512 + lane * 8), hi = *xs4(xs, u * 512 + lane * 8 + 4);
+      h[u][0] = lo.x; h[u][1] = lo.y; h[u][2] = lo.z; h[u][3] = lo.w;
+      h[u][4] = hi.x; h[u][5] = hi.y; h[u][6] = hi.z; h[u][7] = hi.w;
+    }
+  }
+};
+
+template <int U, int MS>
+__global__ __launch_bounds__(GEMV_THREADS) void gemv_row_merge_kernel(const float* part_o, const float* part_ml, const void* W, const void* residual, unsigned long long* trace, int N, int nsplit, int nblk,
+                                                                      GemvArgs rest) {
+  __shared__ __attribute__((aligned(16))) float xs[U * 512];
+  RowMergePro<U, MS> pro{part_o, part_ml, nsplit, xs};
+  gemv_row_body<1, U, GEMV_RESIDUAL>(rest, W, residual, trace, N, (int)blockIdx.x, nblk, pro);
+}
 template <int R, int U, bool FAST, int XP, int MS>
 __global__ __launch_bounds__(GEMV_THREADS) void gemv_merge_kernel(const float* part_o, const float* part_ml, const void* W, const void* residual, unsigned long long* trace, int N, int K, int nsplit, int nblk,
                                                                     GemvArgs rest) {
@@ -213,6 +273,15 @@ void launch_gemv_postnorm(const GemvArgs& a, const GemvPostNorm& p, GemvEpi epi,
 
 void launch_gemv_merge(const GemvArgs& a, const GemvMerge& p, hipStream_t st) {
   const GemvPlan pl = plan_gemv(a.N, a.K, GEMV_RESIDUAL);
+  if (a.K == 2048 && pl.R == 1) {   // (gemv_row_body.h)
+    auto row = [&](auto ms) {
+      hipLaunchKernelGGL((gemv_row_merge_kernel<4, decltype(ms)::value>), dim3(gemv_row_grid(a.N, 1)), dim3(GEMV_THREADS), 0, st, p.part_o, p.part_ml, a.W, a.residual, a.trace, a.N, p.nsplit, gemv_row_grid(a.N, 1), a);
+    };
+    if (p.nsplit > 4) row(std::integral_constant<int, 8>{});
+    else if (p.nsplit > 2) row(std::integral_constant<int, 4>{});
+    else row(std::integral_constant<int, 2>{});
+    return;
+  }
   auto go = [&](auto r, auto u) {
     constexpr int R = decltype(r)::value, U = decltype(u)::value;
     const dim3 grid(pl.grid), block(GEMV_THREADS);
