@@ -437,6 +437,90 @@ __global__ __launch_bounds__(NT) void qkv_post_kernel(QkvPostArgs a, SeqBatch b)
   }
 }
 
+// The same for 32-bit rows on token-major pages whose dims come in fours: the row, the norm weights and the angles are requested 16 bytes at a time before
+// anything waits (the loop above is a round trip per 256 columns and one more per pair of heads: 13.9 us at 16 + 2 x 8 heads x 128, 4.8).
+// Q4 groups of four columns per thread hold the row (4096 of 4 * NT * Q4 at most); a thread's piece of a head is dims d .. d + 3 with their partners half a
+// rotation further, or four dims behind the rotated ones.
+constexpr int QF_NT = 512, QF_Q4 = 4;
+__global__ __launch_bounds__(QF_NT) void qkv_post_f32_kernel(const float* qkv, const float* bias, const float* rope, const bf16_t* q_norm, const bf16_t* k_norm, int ld, int heads_kvh, QkvPostArgs a,
+                                                             SeqBatch b) {
+  extern __shared__ __attribute__((aligned(16))) float sm[];   // q | k of the row
+  __shared__ float red[2][QF_NT / 64];
+  const int r = blockIdx.x, tid = threadIdx.x;
+  const int heads = heads_kvh >> 16, kvh = heads_kvh & 0xffff;
+  const int nq = heads * a.dim, nk = kvh * a.dim, nv = kvh * a.vdim, n = nq + nk + nv;
+  float4 v[QF_Q4], bi[QF_Q4], first[QF_Q4];
+#pragma unroll
+  for (int j = 0; j < QF_Q4; ++j) {
+    const int i = min((tid + j * QF_NT) * 4, n - 4);
+    const int at = i < nq ? i : i < nq + nk ? i - nq + a.k_off : i - nq - nk + a.v_off;
+    v[j] = *reinterpret_cast<const float4*>(qkv + (int64_t)r * ld + at);
+    bi[j] = bias ? *reinterpret_cast<const float4*>(bias + at) : make_float4(0.f, 0.f, 0.f, 0.f);
+    first[j] = a.v_use && i >= nq + nk ? *reinterpret_cast<const float4*>(a.v_first + (int64_t)r * nv + i - nq - nk) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  // this thread's pieces of the heads: at most QF_Q4 of them (two quarters of the row's columns per piece where all dims rotate)
+  const int half = a.rope_dims >> 1, hp = half >> 2, per = (a.dim >> 2) - hp, np = (heads + kvh) * per;
+  uint2 wx[QF_Q4], wy[QF_Q4];
+  float4 cs[QF_Q4][2];
+#pragma unroll
+  for (int j = 0; j < QF_Q4; ++j) {
+    const int it = min(tid + j * QF_NT, np - 1), hd = it / per, p = it - hd * per, d = p < hp ? p * 4 : a.rope_dims + (p - hp) * 4;
+    const bf16_t* w = hd < heads ? q_norm + hd * a.dim : k_norm + (hd - heads) * a.dim;
+    wx[j] = *reinterpret_cast<const uint2*>(w + d);
+    wy[j] = *reinterpret_cast<const uint2*>(w + (p < hp ? d + half : d));
+    const float4* t = reinterpret_cast<const float4*>(rope + ((int64_t)r * half + (p < hp ? d : 0)) * 2);
+    cs[j][0] = hp > 0 ? t[0] : make_float4(1.f, 0.f, 1.f, 0.f);
+    cs[j][1] = hp > 0 ? t[1] : make_float4(1.f, 0.f, 1.f, 0.f);
+  }
+  const SeqEntry e = seq_entry_at(b, entry_of_row(b, r));
+  const int pos = e.pos0 + r - e.row0, page = pos / KV_PAGE_TOKENS, tk = pos % KV_PAGE_TOKENS, dq = a.kv.dq, dv = a.kv.dv;
+  float* kp = reinterpret_cast<float*>(a.kv.tab[(int64_t)e.slot * a.kv.ld + page] + a.kv.layer_off);
+  float* vp = kp + (int64_t)kvh * KV_PAGE_TOKENS * dq;
+  float sq = 0.f, sk = 0.f;
+#pragma unroll
+  for (int j = 0; j < QF_Q4; ++j) {
+    const int i = (tid + j * QF_NT) * 4;
+    if (i >= n) continue;
+    const float4 x = make_float4(v[j].x + bi[j].x, v[j].y + bi[j].y, v[j].z + bi[j].z, v[j].w + bi[j].w);
+    if (i < nq + nk) {
+      *reinterpret_cast<float4*>(sm + i) = x;
+      (i < nq ? sq : sk) += (x.x * x.x + x.y * x.y) + (x.z * x.z + x.w * x.w);
+      continue;
+    }
+    const int iv = i - nq - nk, h = iv / a.vdim, d = iv - h * a.vdim;
+    if (a.v_store) *reinterpret_cast<float4*>(a.v_first + (int64_t)r * nv + iv) = x;
+    const float4 f = a.v_store ? x : first[j];   // (stored and used at once: the value itself)
+    float4 y = x;
+    if (a.v_use) {
+      const float k0 = 1.f - a.lambda, k1 = a.lambda;
+      y = make_float4(k0 * x.x + k1 * f.x, k0 * x.y + k1 * f.y, k0 * x.z + k1 * f.z, k0 * x.w + k1 * f.w);
+    }
+    *reinterpret_cast<float4*>(vp + ((int64_t)h * KV_PAGE_TOKENS + tk) * dv + d) = y;
+  }
+  sq = block_sum_n<QF_NT>(sq, red[0]);
+  sk = block_sum_n<QF_NT>(sk, red[1]);   // (its barrier also publishes sm)
+  const float rq = 1.0f / sqrtf(sq / (float)nq + a.eps), rk = 1.0f / sqrtf(sk / (float)nk + a.eps);
+#pragma unroll
+  for (int j = 0; j < QF_Q4; ++j) {
+    const int it = tid + j * QF_NT;
+    if (it >= np) continue;
+    const int hd = it / per, p = it - hd * per, d = p < hp ? p * 4 : a.rope_dims + (p - hp) * 4;
+    const float rinv = hd < heads ? rq : rk;
+    float* dst = hd < heads ? (float*)a.q_out + ((int64_t)r * heads + hd) * dq : kp + ((int64_t)(hd - heads) * KV_PAGE_TOKENS + tk) * dq;
+    const float4 s = *reinterpret_cast<const float4*>(sm + hd * a.dim + d);
+    const float x[4] = {s.x * rinv * lo_bf(wx[j].x), s.y * rinv * hi_bf(wx[j].x), s.z * rinv * lo_bf(wx[j].y), s.w * rinv * hi_bf(wx[j].y)};
+    if (p >= hp) {
+      *reinterpret_cast<float4*>(dst + d) = make_float4(x[0], x[1], x[2], x[3]);
+      continue;
+    }
+    const float4 t = *reinterpret_cast<const float4*>(sm + hd * a.dim + d + half);
+    const float y[4] = {t.x * rinv * lo_bf(wy[j].x), t.y * rinv * hi_bf(wy[j].x), t.z * rinv * lo_bf(wy[j].y), t.w * rinv * hi_bf(wy[j].y)};
+    const float co[4] = {cs[j][0].x, cs[j][0].z, cs[j][1].x, cs[j][1].z}, si[4] = {cs[j][0].y, cs[j][0].w, cs[j][1].y, cs[j][1].w};
+    *reinterpret_cast<float4*>(dst + d) = make_float4(x[0] * co[0] - y[0] * si[0], x[1] * co[1] - y[1] * si[1], x[2] * co[2] - y[2] * si[2], x[3] * co[3] - y[3] * si[3]);
+    *reinterpret_cast<float4*>(dst + d + half) = make_float4(y[0] * co[0] + x[0] * si[0], y[1] * co[1] + x[1] * si[1], y[2] * co[2] + x[2] * si[2], y[3] * co[3] + x[3] * si[3]);
+  }
+}
+
 // The same for bf16 rows whose head dims, value dims and rotated half come in eights (16-byte pieces, fragment-major pages): blocks [0, rows)
 // norm and rotate the q and k heads of a row, an eight-dim piece per thread and step; the first v_blocks mix the values and write the V pages
 // (few blocks with a long chain each: first, so that they are no tail), a thread gathering eight token slots x eight dims (the slots of a piece are contiguous in the page).
@@ -738,6 +822,15 @@ void launch_qkv_post(const QkvPostArgs& a, const SeqBatch& b, bool f32, hipStrea
     const int64_t vt = (int64_t)b.n * pages * a.kvh * a.kv.dv;
     const int nth = 256, vb = (int)((vt + nth - 1) / nth);
     hipLaunchKernelGGL(qkv_post_frag_kernel, dim3((unsigned)(vb + b.rows)), dim3(nth), 0, st, a, b, pages, vb);
+    return;
+  }
+  const int n = (a.heads + a.kvh) * a.dim + a.kvh * a.vdim;
+  const bool fours = ((a.dim | a.vdim | a.k_off | a.v_off | a.kv.dq | a.kv.dv) & 3) == 0 && (a.ld & 3) == 0 && a.rope_dims % 8 == 0 && a.heads < 32768 && a.ld < (1 << 30) &&
+                     (((uintptr_t)a.qkv | (uintptr_t)a.bias | (uintptr_t)a.rope | (uintptr_t)a.q_norm | (uintptr_t)a.k_norm | (uintptr_t)a.v_first | (uintptr_t)a.q_out) & 15) == 0;
+  const int pieces = (a.heads + a.kvh) * ((a.dim >> 2) - (a.rope_dims >> 3));
+  if (f32 && fours && n <= 4 * QF_NT * QF_Q4 && pieces <= QF_NT * QF_Q4) {
+    hipLaunchKernelGGL(qkv_post_f32_kernel, grid, dim3(QF_NT), (size_t)(a.heads + a.kvh) * a.dim * 4, st, (const float*)a.qkv, a.bias, a.rope, (const bf16_t*)a.q_norm, (const bf16_t*)a.k_norm,
+                       (int)a.ld, a.heads << 16 | a.kvh, a, b);
     return;
   }
   if (f32) hipLaunchKernelGGL((qkv_post_kernel<float, false>), grid, block, lds, st, a, b);
