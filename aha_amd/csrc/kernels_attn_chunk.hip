@@ -2,7 +2,8 @@
 // floor(i / chunk) * chunk .. i of its own sequence; a sink adds a key of score 0 without a value, i.e. one to the softmax's denominator.
 //   prompt rows:   attn_prefill_kernel<.., CHUNK = 1> (attn_prefill_body.h) on fragment-major bf16 pages
 //   one token each: attn_chunk_decode_kernel: q / k norm + rotation + value mixing + KV append + split-KV attention + merge, one launch
-//   any head dims / the 32-bit mode: attn_chunk_rows_kernel on token-major pages
+//   the 32-bit mode, heads of 64 or 128 dims: attn_chunk_f32_kernel on token-major pages
+//   any head dims: attn_chunk_rows_kernel on token-major pages
 // q head h reads kv head h / (heads / kv heads).  Scores, maxima, exponentials and sums are f32; P feeds the MFMA as bf16.
 #include <algorithm>
 
@@ -462,6 +463,148 @@ __global__ __launch_bounds__(ROWS_NW * 64) void attn_chunk_rows_kernel(ChunkAttn
   }
 }
 
+// ---- 32 bits, heads of D = 64 or 128 dims, token-major pages: 16 (row, head) pairs per block -------------------------------------------------
+// Block (16 / GQ rows of a sequence, kv head or head, sequence): the GQ query heads of a kv head share its keys and values (GQ = 1 where the group does
+// not divide 16).  The eight waves take 16 keys each in turn and join (max, sum, O) in LDS.  Both products on v_mfma_f32_16x16x4_f32: S^T = K Q^T with
+// lane (c, G) holding dims 16 t + 4 G + i of key c and of pair c, so both operands come in 16-byte pieces; S^T leaves lane (c, G) with keys 4 G + i of
+// pair c, which is the operand layout of O^T = V^T P^T, its k index i running over those keys; V rows come in 16-byte pieces too, lane c taking value dims
+// 64 b + 4 c + x, so row 4 G + i of accumulator (b, x) is value dim 64 b + 16 G + 4 i + x.
+// What bounds it is a chain of round trips (entry, page, keys) and, for long prompts, the f32 matrix rate.  2 x 150 positions, 16 / 8 heads x 128, before (attn_chunk_rows_kernel: every
+// row read its keys and values again) and with it: prompt 96 -> 22 us, one token each 20.7 -> 11.8.
+constexpr int F32A_NW = 8;
+typedef float fv4 __attribute__((ext_vector_type(4)));
+template <int D>
+constexpr int f32a_lds() { return F32A_NW * 16 * (D + 2) * 4; }
+template <int D>
+__global__ __launch_bounds__(F32A_NW * 64) void attn_chunk_f32_kernel(const float* qp, float* op, const uint64_t* tab, int heads_kvh, int gq, SeqBatch b, ChunkAttnArgs a) {
+  constexpr int NT16 = D / 16, NB = D / 64;
+  extern __shared__ __attribute__((aligned(16))) float os[];   // O [wave][16][D], max [wave][16], sum [wave][16]
+  float *mls = os + F32A_NW * 16 * D, *lls = mls + F32A_NW * 16;
+  typedef const __attribute__((address_space(1))) fv4* g4_t;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, G = lane >> 4;
+  const int heads = heads_kvh >> 16, kvh = heads_kvh & 0xffff;
+  const int nrow = 16 / gq, head0 = blockIdx.y * gq, kvhd = gq > 1 ? blockIdx.y : head0 / (heads / kvh);
+  const SeqEntry e = seq_entry_at(b, blockIdx.z);
+  const int i0 = blockIdx.x * nrow;   // first row inside the entry
+  if (i0 >= e.len) return;
+  const int ic = min(i0 + c / gq, e.len - 1), pos = e.pos0 + ic, lo = a.chunk > 0 ? pos / a.chunk * a.chunk : 0;   // this lane's pair (c): surplus pairs repeat the last row
+  const int p_first = e.pos0 + i0, p_last = e.pos0 + min(i0 + nrow, e.len) - 1, lo_first = a.chunk > 0 ? p_first / a.chunk * a.chunk : 0;
+  const float* q = qp + ((int64_t)(e.row0 + ic) * heads + head0 + c % gq) * D + G * 4;
+  fv4 qf[NT16];
+#pragma unroll
+  for (int t = 0; t < NT16; ++t) qf[t] = *reinterpret_cast<const fv4*>(q + t * 16);
+  float m = a.sink && wave == 0 ? 0.f : -INFINITY, l = a.sink && wave == 0 ? 1.f : 0.f;
+  f32x4_t o[NB][4];
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int x = 0; x < 4; ++x) o[i][x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int u = lo_first / 16 + wave; u <= p_last / 16; u += F32A_NW) {   // keys 16 u .. 16 u + 15
+    const int k16 = u * 16 % KV_PAGE_TOKENS;
+    const uint64_t base = tab[(int64_t)e.slot * a.kv.ld + u * 16 / KV_PAGE_TOKENS] + a.kv.layer_off;
+    const uint64_t kb = base + ((uint64_t)kvhd * KV_PAGE_TOKENS + k16 + c) * (D * 4) + G * 16;
+    const uint64_t vrow = base + ((uint64_t)(kvh + kvhd) * KV_PAGE_TOKENS + k16) * (D * 4), vb = vrow + G * 4 * (D * 4) + c * 16;
+    fv4 kf[NT16], vf[4][NB];
+#pragma unroll
+    for (int t = 0; t < NT16; ++t) kf[t] = *reinterpret_cast<g4_t>(kb + t * 64);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) vf[i][nb] = *reinterpret_cast<g4_t>(vb + (i * D + nb * 64) * 4);
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4_t s2[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};   // two chains: a product's result is not waited for by the next
+#pragma unroll
+    for (int t = 0; t < NT16; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s2[i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][i], qf[t][i], s2[i & 1], 0, 0, 0);
+    f32x4_t st;
+    const int t0 = u * 16 + G * 4;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      st[i] = t0 + i >= lo && t0 + i <= pos ? (s2[0][i] + s2[1][i]) * a.scale : -INFINITY;
+      mx = fmaxf(mx, st[i]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    const float m_new = fmaxf(m, fmaxf(mx, __shfl_xor(mx, 32, 64)));
+    const float al = m == -INFINITY ? 0.f : expf(m - m_new);
+    float ps = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      st[i] = st[i] == -INFINITY ? 0.f : expf(st[i] - m_new);
+      ps += st[i];
+    }
+    l = l * al + group_sum(ps);
+    m = m_new;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) o[nb][x] *= al;
+    // A value is multiplied by the zero weight of a pair that does not see its key.  Where that could leave a NaN (a value that is not finite: behind the
+    // sequence's end in a page used before, or a later row's own), the keys go one by one, each to the pairs that see it.
+    float bad = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) bad = fmaf(vf[i][nb][x], 0.f, bad);
+    if (__any(bad != 0.f)) {
+#pragma unroll 1
+      for (int k = 0; k < 16; ++k) {
+        const float w01 = k & 1 ? st[1] : st[0], w23 = k & 1 ? st[3] : st[2];
+        const float w = __shfl(k & 2 ? w23 : w01, (k >> 2) * 16 + c, 64);
+        if (u * 16 + k < lo || u * 16 + k > pos) continue;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const fv4 v = *reinterpret_cast<g4_t>(vrow + (k * D + nb * 64 + G * 16 + i * 4) * 4);
+#pragma unroll
+            for (int x = 0; x < 4; ++x) o[nb][x][i] = fmaf(w, v[x], o[nb][x][i]);
+          }
+      }
+      continue;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) o[nb][x] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][nb][x], st[i], o[nb][x], 0, 0, 0);
+  }
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<fv4*>(os + (wave * 16 + c) * D + nb * 64 + G * 16 + i * 4) = fv4{o[nb][0][i], o[nb][1][i], o[nb][2][i], o[nb][3][i]};
+  if (G == 0) {
+    mls[wave * 16 + c] = m;
+    lls[wave * 16 + c] = l;
+  }
+  __syncthreads();
+  for (int it = threadIdx.x; it < 16 * (D / 4); it += F32A_NW * 64) {
+    const int j = it / (D / 4), d = it % (D / 4) * 4, ir = i0 + j / gq;
+    if (ir >= e.len) continue;
+    float M = mls[j], z = 0.f;
+#pragma unroll
+    for (int w = 1; w < F32A_NW; ++w) M = fmaxf(M, mls[w * 16 + j]);
+    fv4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < F32A_NW; ++w) {
+      const float f = mls[w * 16 + j] == -INFINITY ? 0.f : expf(mls[w * 16 + j] - M);
+      z = fmaf(lls[w * 16 + j], f, z);
+      const fv4 ow = *reinterpret_cast<const fv4*>(os + (w * 16 + j) * D + d);
+#pragma unroll
+      for (int x = 0; x < 4; ++x) v[x] = fmaf(ow[x], f, v[x]);
+    }
+    const float inv = 1.0f / z;
+    float* dst = op + (int64_t)(e.row0 + ir) * a.ldo + (int64_t)(head0 + j % gq) * a.dvo + d;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) dst[x] = v[x] * inv;
+  }
+}
+
 int pad_dim(int d) { return d <= 32 ? 32 : d <= 64 ? 64 : d <= 128 ? 128 : d <= 256 ? 256 : 0; }
 
 template <class F>
@@ -544,6 +687,16 @@ void launch_chunk_attn_decode(const ChunkDecodeArgs& a, const SeqBatch& b, hipSt
 
 void launch_chunk_attn_rows(const ChunkAttnArgs& a, const SeqBatch& b, bool f32, hipStream_t st) {
   if (b.rows <= 0) return;
+  // (16-byte requests of q and of the pages' rows: whole heads of D dims lie so)
+  if (f32 && a.dim == a.vdim && a.kv.dq == a.dim && a.kv.dv == a.dim && (a.dim == 64 || a.dim == 128) && ((uintptr_t)a.q & 15) == 0 && a.heads < 32768) {
+    const int g = a.heads / a.kv.kvh, gq = g <= 16 && 16 % g == 0 ? g : 1, nrow = 16 / gq;
+    const dim3 grid((unsigned)((b.max_len + nrow - 1) / nrow), (unsigned)(a.heads / gq), (unsigned)b.n), block(F32A_NW * 64);
+    auto k = a.dim == 128 ? attn_chunk_f32_kernel<128> : attn_chunk_f32_kernel<64>;
+    const int lds = a.dim == 128 ? f32a_lds<128>() : f32a_lds<64>();
+    if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    hipLaunchKernelGGL(k, grid, block, lds, st, (const float*)a.q, (float*)a.o, a.kv.tab, a.heads << 16 | a.kv.kvh, gq, b, a);
+    return;
+  }
   auto go = [&](auto t, auto nv) {
     using T = decltype(t);
     constexpr int NV = decltype(nv)::value;

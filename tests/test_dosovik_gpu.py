@@ -120,6 +120,37 @@ def test_prompt_and_decoding_follow_the_equations(ctx, name, dtype):
     assert err(half, whole) <= TOL_SAME[dtype], name
 
 
+F32_HEADS = [   # heads, kv heads, dims, chunk, rotated dims: groups of 1, 2, 3 (no divisor of 16), 16 and 32 heads; chunks around 16 keys and a page
+    (16, 8, 128, 150, 128), (4, 4, 64, 20, 64), (6, 2, 128, 1, 40), (16, 1, 64, 192, 0), (32, 1, 64, 33, 8), (4, 2, 128, 64, 64),
+]
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,chunk,rope_dims", F32_HEADS)
+def test_32_bit_heads_of_whole_pieces(ctx, heads, kv_heads, dim, chunk, rope_dims):
+    """attn_chunk_f32_kernel and qkv_post_f32_kernel: a prompt whose last tile is partly full, then token by token."""
+    cfg = config([layer(heads=heads, kv_heads=kv_heads, dim=dim, vdim=dim, chunk=chunk, rope_dims=rope_dims)] * 2)
+    w = dosovik_weights(cfg, seed=7)
+    ids = tokens(211, cfg.vocab_size, 3)
+    want = reference(cfg, w, ids)
+    with Model(ctx, cfg, w) as m:
+        assert err(all_logits(m, ids), want) <= TOL["float32"]
+        assert err(all_logits(m, ids, [1, 130, 63] + [1] * 17), want) <= TOL["float32"]
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+def test_32_bit_rows_do_not_see_a_later_row_that_is_not_finite(ctx, dim):
+    cfg = config([layer(heads=8, kv_heads=4, dim=dim, vdim=dim, chunk=100, rope_dims=dim)] * 2)
+    w = dosovik_weights(cfg, seed=8)
+    last = cfg.vocab_size - 1
+    w["embed"][last] = float("inf")
+    ids = [t % last for t in tokens(75, cfg.vocab_size, 4)]
+    want = reference(cfg, w, ids)
+    with Model(ctx, cfg, w) as m:
+        got = all_logits(m, ids + [last])
+        assert err(got[:-1], want) <= TOL["float32"] and not np.isfinite(got[-1]).all()
+        assert err(all_logits(m, ids), want) <= TOL["float32"]   # (in pages that hold that row)
+
+
 def neutral(cfg, seed):
     """Weights under which every mechanism but the projections is switched off: no convolution, unit norms, no biases, no mixing, act = N(z)."""
     w = dosovik_weights(cfg, seed=seed)
