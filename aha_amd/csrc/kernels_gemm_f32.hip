@@ -30,7 +30,15 @@ struct GemmF32Args {
 // A decoding step's products had one 64 x 64 tile per 64 columns (64 blocks for 4096 x 1024, every k step a load's latency): 80 us on average at 2
 // rows of the 0.6B widths, 6.4 us here; its 32768-column head 21 us (67 MB: 3.1 TB/s).
 template <int R8, int M8>
-__global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_f32_few_kernel(GemmF32Args a) {
+__global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_f32_few_kernel(const float* A, const bf16_t* W, int M, int N, int K, int64_t lda, int64_t ldw, GemmF32Args a) {
+  // (what the first requests need: in scalar registers at the start, gemv_body.h)
+  a.A = A;
+  a.W = W;
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  a.lda = lda;
+  a.ldw = ldw;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int MT = (M8 + 1) / 2, PER = skinny_requests(R8, M8, true);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), G = lane >> 4, c = lane & 15, n0 = (int)blockIdx.x * (R8 * 8);
@@ -38,12 +46,12 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_f32_few_kernel(GemmF32
 #pragma unroll
   for (int r = 0; r < R8; ++r) {
     const int local = r * 8 + (lane >> 3);
-    src[r] = (const char*)(a.W + blockIdx.y * a.sw + (int64_t)min(n0 + local, a.N - 1) * a.ldw) + skinny_piece(local, lane);
+    src[r] = (const char*)(a.W + (blockIdx.y > 0 ? blockIdx.y * a.sw : 0) + (int64_t)min(n0 + local, a.N - 1) * a.ldw) + skinny_piece(local, lane);
   }
 #pragma unroll
   for (int r = 0; r < 2 * M8; ++r) {
     const int local = r % M8 * 8 + (lane >> 3);
-    src[R8 + r] = (const char*)(a.A + blockIdx.y * a.sa + (int64_t)min(local, a.M - 1) * a.lda) + r / M8 * 128 + skinny_piece(local, lane);
+    src[R8 + r] = (const char*)(a.A + (blockIdx.y > 0 ? blockIdx.y * a.sa : 0) + (int64_t)min(local, a.M - 1) * a.lda) + r / M8 * 128 + skinny_piece(local, lane);
   }
   skinny_sums<R8, M8, true>(src, a.K / 64, smem, wave, lane);
   for (int i = wave; i < (R8 / 2) * MT; i += SKINNY_WAVES) {
@@ -182,7 +190,8 @@ void launch_gemm_f32(const float* A, int64_t lda, const void* W, int64_t ldw, fl
   auto go = [&](auto r8, auto m8) {
     constexpr int R8 = decltype(r8)::value, M8 = decltype(m8)::value, lds = skinny_lds(R8, M8, true);
     if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_f32_few_kernel<R8, M8>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    hipLaunchKernelGGL((gemm_f32_few_kernel<R8, M8>), dim3((unsigned)((N + R8 * 8 - 1) / (R8 * 8)), (unsigned)batch), dim3(SKINNY_WAVES * 64), lds, st, a);
+    hipLaunchKernelGGL((gemm_f32_few_kernel<R8, M8>), dim3((unsigned)((N + R8 * 8 - 1) / (R8 * 8)), (unsigned)batch), dim3(SKINNY_WAVES * 64), lds, st, a.A,
+                       a.W, a.M, a.N, a.K, a.lda, a.ldw, a);
   };
   using std::integral_constant;
   // 48 weight rows per block where they still make two blocks per CU (the head); f32 rows take twice the LDS, so more than 32 of them leave room for 16

@@ -27,7 +27,15 @@ namespace aha {
 namespace {
 
 template <int R8, int M8, bool PAIRS>
-__global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(GemmArgs a) {
+__global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const void* A, const void* W, int M, int N, int K, int64_t lda, int64_t ldw, GemmArgs a) {
+  // (what the first requests need: in scalar registers at the start, gemv_body.h)
+  a.A = A;
+  a.W = W;
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  a.lda = lda;
+  a.ldw = ldw;
   constexpr int NF = (R8 + 1) / 2, MT = (M8 + 1) / 2, PER = R8 + M8;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), G = lane >> 4, c = lane & 15;
   const char* src[PER];
@@ -78,7 +86,8 @@ void launch_one(const GemmArgs& a, hipStream_t st) {
   constexpr int lds = skinny_lds(R8, M8);
   if (lds > 64 * 1024)
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_skinny_kernel<R8, M8, PAIRS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  hipLaunchKernelGGL((gemm_skinny_kernel<R8, M8, PAIRS>), dim3((unsigned)((a.N + R8 * 8 - 1) / (R8 * 8)), (unsigned)((a.M + 63) / 64)), dim3(SKINNY_WAVES * 64), lds, st, a);
+  hipLaunchKernelGGL((gemm_skinny_kernel<R8, M8, PAIRS>), dim3((unsigned)((a.N + R8 * 8 - 1) / (R8 * 8)), (unsigned)((a.M + 63) / 64)), dim3(SKINNY_WAVES * 64), lds, st, a.A, a.W, a.M, a.N, a.K, a.lda,
+                     a.ldw, a);
 }
 
 template <int R8, bool PAIRS>

@@ -182,13 +182,22 @@ __global__ __launch_bounds__(NTH) void postnorm_conv_kernel(PostNormArgs a, SeqB
 // its chain of round trips -- entry, history, and in the general kernel one more per tap, per weight row and behind the norm (6.0 us at 8 rows of 4096
 // columns, 3 taps); here everything that the entry does not decide is requested in front of it, the history right behind: 4.1 us.
 template <typename T, int NTH, int TAPS, bool EMBED>
-__global__ __launch_bounds__(NTH) void postnorm_conv_step_kernel(PostNormArgs a, SeqBatch b) {
+__global__ __launch_bounds__(NTH) void postnorm_conv_step_kernel(const float* x_in, const void* yp, const void* norm_w, const void* conv_w, const SeqEntry* entries, int ld_, int64_t ldy, PostNormArgs a,
+                                                                  SeqBatch b) {
   constexpr int NH = TAPS - 1;
+  // (what the first requests need: in scalar registers at the start, gemv_body.h)
+  a.x_in = x_in;
+  a.y = yp;
+  a.norm_w = norm_w;
+  a.conv.w = conv_w;
+  a.ld = ld_;
+  a.ldy = ldy;
+  b.entries = entries;
   __shared__ float red[NTH / 64];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ld = (int)a.ld, r = (int)blockIdx.x;
   const bool in = wave * 256 < ld;
   const int c = min(tid * 4, ld - 4);
-  const int ei = entry_of_row(b, r);
+  const SeqEntry e = seq_entry_at(b, r);   // (one row per sequence)
   float4 v, y = make_float4(0.f, 0.f, 0.f, 0.f), nw = y, w[TAPS], hist[NH];
   if (EMBED) {
     v = wbf4((const bf16_t*)a.embed + (int64_t)a.ids[r] * ld, c);
@@ -199,7 +208,6 @@ __global__ __launch_bounds__(NTH) void postnorm_conv_step_kernel(PostNormArgs a,
   }
 #pragma unroll
   for (int j = 0; j < TAPS; ++j) w[j] = wbf4(a.conv.w, (int64_t)j * ld + c);
-  const SeqEntry e = seq_entry_at(b, ei);
   float* base = a.conv.hist + (int64_t)e.slot * a.conv.slot_stride + c;
   const float* hi = base + (int64_t)e.hist_in * TAPS * ld;
 #pragma unroll
@@ -690,7 +698,9 @@ __global__ __launch_bounds__(1024) void qkv_post_frag_kernel(QkvPostArgs a, SeqB
 
 // NVZ * 4 * NTH columns of the row in registers (NVZ = 0: any width, the row is read twice)
 template <typename T, int NTH, int NVZ>
-__global__ __launch_bounds__(NTH) void polynorm_rows_kernel(PolyNormArgs a) {
+__global__ __launch_bounds__(NTH) void polynorm_rows_kernel(const void* zp, int64_t ldz, PolyNormArgs a) {
+  a.z = zp;   // (what the first requests need: in scalar registers at the start, gemv_body.h)
+  a.ld = ldz;
   __shared__ float red[3][NTH / 64];
   constexpr bool REGS = NVZ > 0;
   const T* z = (const T*)a.z + (int64_t)blockIdx.x * a.ld;
@@ -741,7 +751,7 @@ void postnorm_conv_t(const PostNormArgs& a, const SeqBatch& b, hipStream_t st) {
   if (b.max_len == 1 && a.h_out && a.conv.taps >= 2 && a.conv.taps <= 4 && a.ld <= 4096) {
     auto step = [&](auto nth, auto taps) {
       constexpr int NTH = decltype(nth)::value, TAPS = decltype(taps)::value;
-      hipLaunchKernelGGL((postnorm_conv_step_kernel<T, NTH, TAPS, EMBED>), dim3((unsigned)b.rows), dim3(NTH), 0, st, a, b);
+      hipLaunchKernelGGL((postnorm_conv_step_kernel<T, NTH, TAPS, EMBED>), dim3((unsigned)b.rows), dim3(NTH), 0, st, a.x_in, a.y, a.norm_w, a.conv.w, b.entries, (int)a.ld, a.ldy, a, b);
     };
     auto by_taps = [&](auto nth) {
       if (a.conv.taps == 2) step(nth, integral_constant<int, 2>{});
@@ -840,7 +850,7 @@ void launch_qkv_post(const QkvPostArgs& a, const SeqBatch& b, bool f32, hipStrea
 
 void launch_polynorm_rows(const PolyNormArgs& a, bool f32, hipStream_t st) {
   if (a.rows <= 0) return;
-  auto go = [&](auto k, int nth) { hipLaunchKernelGGL(k, dim3((unsigned)a.rows), dim3(nth), 0, st, a); };
+  auto go = [&](auto k, int nth) { hipLaunchKernelGGL(k, dim3((unsigned)a.rows), dim3(nth), 0, st, a.z, (int64_t)a.ld, a); };
   if (f32) go(polynorm_rows_kernel<float, 256, 0>, 256);
   else if (a.ld <= 4096) go(polynorm_rows_kernel<bf16_t, 256, 4>, 256);
   else if (a.ld <= 8192) go(polynorm_rows_kernel<bf16_t, 512, 4>, 512);
