@@ -151,6 +151,25 @@ def test_32_bit_rows_do_not_see_a_later_row_that_is_not_finite(ctx, dim):
         assert err(all_logits(m, ids), want) <= TOL["float32"]   # (in pages that hold that row)
 
 
+@pytest.mark.parametrize("heads,kv_heads,chunk", [(16, 8, 8192), (14, 2, 192), (8, 8, 20), (32, 8, 64), (1, 1, 100), (16, 2, 192)])
+def test_decoding_with_whole_heads_of_128(ctx, heads, kv_heads, chunk):
+    """attn_chunk_decode_kernel's LEAN form (eight query heads per kv head: the other one), two sequences token by token and one alone, several pages per
+    unit and units without any, chunk edges on the way."""
+    cfg = config([layer(heads=heads, kv_heads=kv_heads, dim=128, vdim=128, chunk=chunk, rope_dims=128, scale=0.09)] * 3, dtype="bfloat16")
+    w = dosovik_weights(cfg, seed=9)
+    a, b = tokens(420, cfg.vocab_size, 5), tokens(90, cfg.vocab_size, 6)
+    want_a, want_b = reference(cfg, w, a), reference(cfg, w, b)
+    with Model(ctx, cfg, w) as m:
+        assert err(all_logits(m, a, [380] + [1] * 40), want_a) <= TOL["bfloat16"]
+        s, t = m.seq_open(), m.seq_open()
+        m.forward_batch([(s, a[:395], [394]), (t, b[:57], [56])])
+        got = [m.forward_batch([(s, [a[395 + i]], [0]), (t, [b[57 + i]], [0])])[0] for i in range(25)]
+        m.seq_close(s)
+        m.seq_close(t)
+    assert err(np.stack([g[0] for g in got]), want_a[395:420]) <= TOL["bfloat16"]
+    assert err(np.stack([g[1] for g in got]), want_b[57:82]) <= TOL["bfloat16"]
+
+
 def neutral(cfg, seed):
     """Weights under which every mechanism but the projections is switched off: no convolution, unit norms, no biases, no mixing, act = N(z)."""
     w = dosovik_weights(cfg, seed=seed)
