@@ -58,12 +58,14 @@ __device__ __forceinline__ GemvArgs gemv_args(GemvArgs a, const void* x, const v
 // xs: LDS, (ceil(K/512)*512 + 16) floats.  bid/nblk: this block's index in, and the size of, the persistent grid.
 // after_issue() runs once the block's first weight tile has been requested and before anything that depends on the
 // activation vector -- the stand-alone kernel passes a no-op, the persistent kernel waits on its grid barrier there.
-template <int R, int U, int EPI, bool COH, bool FAST, class AfterIssue, class Pro = GemvNormPrologue>
+// XP > 0 (FAST): K = 2048 * XP, known when the kernel is compiled: no divisions, no predicates in front of the first weight.
+template <int R, int U, int EPI, bool COH, bool FAST, int XP = 0, class AfterIssue, class Pro = GemvNormPrologue>
 __device__ __forceinline__ void gemv_body(const GemvArgs& a, float* xs, const int bid, const int nblk, AfterIssue&& after_issue, Pro pro = Pro()) {
   constexpr bool OWN_PRO = !std::is_same<Pro, GemvNormPrologue>::value, MAPPED = gemv_mapped<Pro>::value;
   using res_t = typename std::conditional<EPI == GEMV_AXPY_F32, float, bf16_t>::type;   // the tile's residual values (FAST form)
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int K = a.K, N = a.N;
+  static_assert(XP == 0 || (FAST && !COH && XP * 4 % U == 0), "whole load groups");
+  const int K = XP > 0 ? XP * 2048 : a.K, N = a.N;
   const int nchunks = (K + 511) >> 9;  // K % 8 == 0; the tail of the last chunk is zero-filled
   float* red = xs + (nchunks << 9);
 
@@ -73,8 +75,6 @@ __device__ __forceinline__ void gemv_body(const GemvArgs& a, float* xs, const in
   const int n_out = N;  // for SILU_MUL a "row" runs over the I outputs; the wave streams gate row j and up row j together
   const int ntiles = (n_out + ROWS_PER_TILE - 1) / ROWS_PER_TILE;
   const int gpt = (nchunks + U - 1) / U;                                  // chunk groups per tile
-  const int my_tiles = (ntiles - bid + nblk - 1) / nblk;
-  const int ngroups = my_tiles * gpt;
   const bf16_t* Wb = (const bf16_t*)a.W;
   const bf16_t* W2b = (const bf16_t*)a.W2;
 
@@ -144,14 +144,19 @@ __device__ __forceinline__ void gemv_body(const GemvArgs& a, float* xs, const in
   // Memory returns are IN ORDER within a wave: a load issued behind the first weight tile only returns after that
   // tile has arrived (several microseconds under a chip-wide burst).  The activation vector and the norm weights the
   // prologue needs are therefore requested FIRST (stand-alone kernels, K <= 8 * 2048), the weight tile right behind them.
-  constexpr int XPRE = 8;
-  const bool pre = !COH && !OWN_PRO && (nchunks << 6) <= XPRE * GEMV_THREADS;
+  constexpr int XPRE = XP > 0 ? XP : 8;
+  const bool pre = XP > 0 ? !OWN_PRO : !COH && !OWN_PRO && (nchunks << 6) <= XPRE * GEMV_THREADS;
   u32x4_t xpre[XPRE], npre[XPRE];
   if constexpr (OWN_PRO) pro.request(tid);
   if (pre) {
 #pragma unroll
     for (int j = 0; j < XPRE; ++j) {
       const int v = tid + j * GEMV_THREADS;
+      if constexpr (XP > 0) {
+        xpre[j] = ld16((const bf16_t*)a.x + v * 8);
+        npre[j] = ld16((const bf16_t*)(a.norm_w != nullptr ? a.norm_w : a.x) + v * 8);   // (without a norm: on its way already)
+        continue;
+      }
       xpre[j] = u32x4_t{0u, 0u, 0u, 0u};
       npre[j] = u32x4_t{0u, 0u, 0u, 0u};
       if (v * 8 < K) {
@@ -162,7 +167,8 @@ __device__ __forceinline__ void gemv_body(const GemvArgs& a, float* xs, const in
   }
   u32x4_t bufA[U][NW][R], bufB[U][NW][R];
   res_t resA[R], resB[R];   // FAST + GEMV_RESIDUAL / GEMV_AXPY_F32: the residual values of the buffer's tile, requested with it
-  if (ngroups > 0) issue(0, bufA, resA);
+  issue(0, bufA, resA);   // (bid < ntiles: no launch has more blocks than tiles)
+  const int ngroups = (ntiles - bid + nblk - 1) / nblk * gpt;
   stamp(1);
   after_issue();  // grid barrier of the persistent decode kernel: the first weight tile is already in flight
 

@@ -18,10 +18,10 @@ namespace aha {
 
 namespace {
 
-template <int R, int U, int EPI, bool FAST>
+template <int R, int U, int EPI, bool FAST, int XP = 0>
 __global__ __launch_bounds__(GEMV_THREADS) void gemv_kernel(GEMV_HOT_PARAMS, GemvArgs rest) {
   extern __shared__ __attribute__((aligned(16))) float xs[];  // K f32 + 8 floats reduction scratch
-  gemv_body<R, U, EPI, false, FAST>(gemv_args<EPI>(rest, GEMV_HOT), xs, (int)blockIdx.x, nblk, [] {});
+  gemv_body<R, U, EPI, false, FAST, XP>(gemv_args<EPI>(rest, GEMV_HOT), xs, (int)blockIdx.x, nblk, [] {});
 }
 
 template <int R, int U, int EPI, bool NORM>
@@ -128,8 +128,11 @@ static void launch_gemv_epi(const GemvArgs& a, const GemvPlan& p, hipStream_t st
   // FAST form (gemv_body.h): every chunk group full and in range, weights non-temporal
   static const bool fast_ok = [] { const char* e = getenv("AHA_GEMV_FAST"); return e ? atoi(e) != 0 : true; }();
   const bool fast = fast_ok && a.K % (512 * p.U) == 0 && !a.cached && a.N >= 1;
+  // K = 4096 and 12288 (8B) have instantiations that know it (gemv_body.h, XP)
 #define GV(RR, UU)                                                                            \
   do {                                                                                        \
+    if (UU >= 4 && fast && a.K == 4096) { hipLaunchKernelGGL((gemv_kernel<RR, UU, EPI, true, UU >= 4 ? 2 : 0>), grid, block, lds, st, GEMV_HOT_ARGS(a, EPI, p.grid), a); break; } \
+    if (UU == 8 && fast && a.K == 12288) { hipLaunchKernelGGL((gemv_kernel<RR, UU, EPI, true, UU == 8 ? 6 : 0>), grid, block, lds, st, GEMV_HOT_ARGS(a, EPI, p.grid), a); break; } \
     if (fast) hipLaunchKernelGGL((gemv_kernel<RR, UU, EPI, true>), grid, block, lds, st, GEMV_HOT_ARGS(a, EPI, p.grid), a);  \
     else hipLaunchKernelGGL((gemv_kernel<RR, UU, EPI, false>), grid, block, lds, st, GEMV_HOT_ARGS(a, EPI, p.grid), a);      \
   } while (0)

@@ -219,14 +219,15 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_row_merge_kernel(const floa
   RowMergePro<U, MS> pro{part_o, part_ml, nsplit, xs};
   gemv_row_body<1, U, GEMV_RESIDUAL>(rest, W, residual, trace, N, (int)blockIdx.x, nblk, pro);
 }
-template <int R, int U, bool FAST, int XP, int MS>
+template <int R, int U, bool FAST, int XP, int MS, int KX = 0>
 __global__ __launch_bounds__(GEMV_THREADS) void gemv_merge_kernel(const float* part_o, const float* part_ml, const void* W, const void* residual, unsigned long long* trace, int N, int K, int nsplit, int nblk,
                                                                     GemvArgs rest) {
   extern __shared__ __attribute__((aligned(16))) float xs[];
   MergePro<XP, MS> pro;
+  if (KX > 0) K = KX * 2048;
   pro.p = GemvMerge{part_o, part_ml, nsplit, K >> 7};
   pro.K = K;
-  gemv_body<R, U, GEMV_RESIDUAL, false, FAST>(gemv_args<GEMV_RESIDUAL>(rest, nullptr, W, nullptr, residual, trace, N, K, 0.f), xs, (int)blockIdx.x, nblk, [] {}, pro);
+  gemv_body<R, U, GEMV_RESIDUAL, false, FAST, KX>(gemv_args<GEMV_RESIDUAL>(rest, nullptr, W, nullptr, residual, trace, N, K, 0.f), xs, (int)blockIdx.x, nblk, [] {}, pro);
 }
 template <int R, int U, int EPI, bool FAST, int XP>
 __global__ __launch_bounds__(GEMV_THREADS) void gemv_postnorm_kernel(GemvArgs a, GemvPostNorm p) {
@@ -291,6 +292,11 @@ void launch_gemv_merge(const GemvArgs& a, const GemvMerge& p, hipStream_t st) {
     };
     using std::integral_constant;
     auto by_k = [&](auto fast) {
+      if constexpr (U == 8 && decltype(fast)::value)
+        if (a.K == 4096) {
+          hipLaunchKernelGGL((gemv_merge_kernel<R, U, true, 4, 4, 2>), grid, block, fused_lds(a), st, p.part_o, p.part_ml, a.W, a.residual, a.trace, a.N, a.K, p.nsplit, pl.grid, a);
+          return;
+        }
       if (a.K > 2048) run(fast, integral_constant<int, 4>{}, integral_constant<int, 4>{});
       else if (p.nsplit > 4) run(fast, integral_constant<int, 2>{}, integral_constant<int, 8>{});
       else run(fast, integral_constant<int, 2>{}, integral_constant<int, 4>{});
