@@ -26,7 +26,7 @@ namespace aha {
 
 namespace {
 
-template <int R8, int M8, bool PAIRS>
+template <int R8, int M8, bool PAIRS, bool ONE_BLOCK>
 __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const void* A, const void* W, int M, int N, int K, int64_t lda, int64_t ldw, GemmArgs a) {
   // (what the first requests need: in scalar registers at the start, gemv_body.h)
   a.A = A;
@@ -51,7 +51,7 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const vo
       src[r] = (const char*)a.W + (int64_t)min((int)blockIdx.x * (R8 * 8) + local, a.N - 1) * a.ldw * 2 + piece;
     }
   }
-  skinny_sums<R8, M8>(src, a.K / 64, gemm_smem, wave, lane);
+  skinny_sums<R8, M8, false, ONE_BLOCK>(src, a.K / 64, gemm_smem, wave, lane);
   for (int i = wave; i < NF * MT; i += SKINNY_WAVES) {
     const int r = i / MT, m = (int)blockIdx.y * 64 + (i - r * MT) * 16 + c;
     if (m >= a.M) continue;
@@ -81,12 +81,14 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const vo
   }
 }
 
-template <int R8, int M8, bool PAIRS>
+template <int R8, int M8, bool PAIRS, bool ONE_BLOCK = false>
 void launch_one(const GemmArgs& a, hipStream_t st) {
-  constexpr int lds = skinny_lds(R8, M8);
+  if constexpr (!ONE_BLOCK && skinny_stages(R8 + M8) != skinny_stages(R8 + M8, true))
+    if (gemm_skinny_rounds(a, R8) == 1) return launch_one<R8, M8, PAIRS, true>(a, st);
+  constexpr int lds = skinny_lds(R8, M8, false, ONE_BLOCK);
   if (lds > 64 * 1024)
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_skinny_kernel<R8, M8, PAIRS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  hipLaunchKernelGGL((gemm_skinny_kernel<R8, M8, PAIRS>), dim3((unsigned)((a.N + R8 * 8 - 1) / (R8 * 8)), (unsigned)((a.M + 63) / 64)), dim3(SKINNY_WAVES * 64), lds, st, a.A, a.W, a.M, a.N, a.K, a.lda,
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_skinny_kernel<R8, M8, PAIRS, ONE_BLOCK>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  hipLaunchKernelGGL((gemm_skinny_kernel<R8, M8, PAIRS, ONE_BLOCK>), dim3((unsigned)((a.N + R8 * 8 - 1) / (R8 * 8)), (unsigned)((a.M + 63) / 64)), dim3(SKINNY_WAVES * 64), lds, st, a.A, a.W, a.M, a.N, a.K, a.lda,
                      a.ldw, a);
 }
 

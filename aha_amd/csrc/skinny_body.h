@@ -1,6 +1,8 @@
 // Shared device code of the few-row products (kernels_gemm_skinny.hip: dense; kernels_moe.hip: experts with few slots).  A block of four waves owns
 // R8 * 8 weight rows, M8 * 8 activation rows and the whole K range; why and what it measured: kernels_gemm_skinny.hip.
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 
 namespace aha {
@@ -8,12 +10,15 @@ namespace aha {
 namespace {
 
 constexpr int SKINNY_WAVES = 4;
-// three stages hide a request's latency; wide ones have enough in flight with two (and three of them leave one block per CU)
-constexpr int skinny_stages(int requests) { return requests <= 6 ? 3 : 2; }
+// A CU's share of HBM's rate times a request's latency is ~50 KB.  Narrow stages come in as many as keep two blocks per CU (18 to 20 KB per wave); wide
+// ones have enough in flight with two where blocks share a CU (three of them leave one block), and take three in a launch of one block per CU.
+// Eight rows inside a batched step, three stages (two from seven requests on) before: 6144 x 4096 11.9 -> 10.9 us, 12288 x 4096 19.8 -> 18.0, 4096 x 4096
+// and 4096 x 12288 13.5 -> 12.7 on average.  Nothing is requested past the end (three surplus stages of a wave's four chunks at K = 1024 before).
+constexpr int skinny_stages(int requests, bool one_block = false) { return requests <= 3 ? 6 : requests == 4 ? 5 : requests == 5 ? 4 : requests <= 6 || (one_block && requests <= 8) ? 3 : 2; }
 constexpr int skinny_requests(int r8, int m8, bool f32) { return r8 + (f32 ? 2 : 1) * m8; }
-constexpr int skinny_lds(int r8, int m8, bool f32 = false) {
+constexpr int skinny_lds(int r8, int m8, bool f32 = false, bool one_block = false) {
   const int per = skinny_requests(r8, m8, f32);
-  const int ring = SKINNY_WAVES * skinny_stages(per) * per * 1024 + ((r8 | m8) & 1) * 1024;   // odd: half a fragment is read behind the last stage
+  const int ring = SKINNY_WAVES * skinny_stages(per, one_block) * per * 1024 + ((r8 | m8) & 1) * 1024;   // odd: half a fragment is read behind the last stage
   const int sums = SKINNY_WAVES * ((r8 + 1) / 2) * ((m8 + 1) / 2) * 1024;
   return ring > sums ? ring : sums;
 }
@@ -28,11 +33,11 @@ __device__ __forceinline__ int skinny_piece(int local_row, int lane) { return ((
 // v_mfma_f32_16x16x4_f32 (weights widened exactly): in step (h, j) lane group G feeds k = (h * 4 + G) * 8 + j of both operands.
 // On return the waves' sums of the 16 x 16 fragments (weight fragment r, activation fragment m) lie in LDS and every wave may read them
 // (skinny_total).
-template <int R8, int M8, bool F32 = false>
+template <int R8, int M8, bool F32 = false, bool ONE_BLOCK = false>
 __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R8, M8, F32)], int nc, char* smem, int wave, int lane) {
   typedef __attribute__((address_space(3))) void* lds_t;
   typedef const __attribute__((address_space(1))) void* glb_t;
-  constexpr int NF = (R8 + 1) / 2, MT = (M8 + 1) / 2, PER = skinny_requests(R8, M8, F32), S = skinny_stages(PER);
+  constexpr int NF = (R8 + 1) / 2, MT = (M8 + 1) / 2, PER = skinny_requests(R8, M8, F32), S = skinny_stages(PER, ONE_BLOCK);
   constexpr int LEFT = (S - 1) * PER;   // requests of the later stages
   static_assert(LEFT < 64, "vmcnt has six bits");
   const int G = lane >> 4, c = lane & 15;
@@ -44,19 +49,14 @@ __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R
     for (int r = 0; r < NF; ++r)
 #pragma unroll
       for (int m = 0; m < MT; ++m) acc[h][r][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  auto load = [&](int u, int ch) {   // (past the end: the last chunk again, never used)
-    const int k = min(ch, nc - 1) * 128, ka = F32 ? 2 * k : k;
+  auto load = [&](int u, int ch) {
+    const int k = ch * 128, ka = F32 ? 2 * k : k;
 #pragma unroll
     for (int r = 0; r < R8; ++r) __builtin_amdgcn_global_load_lds((glb_t)(src[r] + k), (lds_t)(ring + (u * PER + r) * 1024), 16, 0, 2);   // weights: non-temporal
 #pragma unroll
     for (int r = R8; r < PER; ++r) __builtin_amdgcn_global_load_lds((glb_t)(src[r] + ka), (lds_t)(ring + (u * PER + r) * 1024), 16, 0, 0);
   };
-#pragma unroll
-  for (int u = 0; u < S; ++u) load(u, wave + u * SKINNY_WAVES);
-  int u = 0;
-  for (int ch = wave; ch < nc; ch += SKINNY_WAVES) {
-    __builtin_amdgcn_s_waitcnt(0x0F70 | (LEFT & 15) | ((LEFT >> 4) << 14));
-    __builtin_amdgcn_sched_barrier(0);
+  auto consume = [&](int u) {
     const char *sw = ring + u * PER * 1024, *sa = sw + R8 * 1024;
     u32x4_t wf[2][NF];
 #pragma unroll
@@ -96,7 +96,34 @@ __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);   // the stage's fragments are in registers: it may be filled again
     __builtin_amdgcn_sched_barrier(0);
+  };
+  int u = 0, ch = wave;
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+    if (wave + s * SKINNY_WAVES < nc) load(s, wave + s * SKINNY_WAVES);
+  for (; ch + S * SKINNY_WAVES < nc; ch += SKINNY_WAVES) {   // S stages are on their way: the oldest is in when the later ones' requests are left
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (LEFT & 15) | ((LEFT >> 4) << 14));
+    __builtin_amdgcn_sched_barrier(0);
+    consume(u);
     load(u, ch + S * SKINNY_WAVES);
+    u = u + 1 == S ? 0 : u + 1;
+  }
+  for (; ch < nc; ch += SKINNY_WAVES) {   // the last ones: as many behind this one as there are chunks left
+    const int later = (nc - 1 - ch) / SKINNY_WAVES;
+    auto wait = [&](auto n) {
+      constexpr int L = decltype(n)::value * PER;
+      if constexpr (decltype(n)::value < S)
+        if (later == decltype(n)::value) __builtin_amdgcn_s_waitcnt(0x0F70 | (L & 15) | ((L >> 4) << 14));
+    };
+    wait(std::integral_constant<int, 0>{});
+    wait(std::integral_constant<int, 1>{});
+    wait(std::integral_constant<int, 2>{});
+    wait(std::integral_constant<int, 3>{});
+    wait(std::integral_constant<int, 4>{});
+    wait(std::integral_constant<int, 5>{});
+    static_assert(S <= 6, "a wait for every number of later stages");
+    __builtin_amdgcn_sched_barrier(0);
+    consume(u);
     u = u + 1 == S ? 0 : u + 1;
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);   // no DMA may land in what becomes the sums' space
