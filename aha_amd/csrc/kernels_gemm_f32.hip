@@ -60,67 +60,78 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_f32_few_kernel(const f
   }
 }
 
-// 32 rows x 64 columns, four waves of 16 x 32, 64-wide k stages.  A stage is 16 requests of 1 KB (8 of A: rows of 64 k are two lines; 8 of W), four per
-// wave; three stages keep two in flight under the one that multiplies, one barrier per stage.  The tile is this small so that a prompt of a few
-// hundred rows still makes two to three blocks per CU: the f32 MFMA (32 cycles for 16 x 16 x 4) is the bound, idle SIMDs are the loss.
+// WM * 16 rows x 64 columns, 64-wide k stages; WM = 2: four waves of 16 x 32, WM = 1: of 16 x 16.  A stage is requests of 1 KB (rows of 64 k of A are
+// two lines: 4 WM of them; 8 of W), a quarter per wave; three stages keep two in flight under the one that multiplies, one barrier per stage.  The tile is
+// this small so that a prompt of a few hundred rows still makes two to three blocks per CU: the f32 MFMA (32 cycles for 16 x 16 x 4) is the bound, idle
+// SIMDs are the loss.
 // 300 rows of the 0.6B widths: 87 us on average (64 x 64 tiles, one stage, through registers) -> 36 us.
-constexpr int F_S = 3, F_STAGE = 16 * 1024;
+// A wave of the wider tile multiplies for 0.43 us per stage, so a launch of fewer blocks than CUs takes 0.43 us * K / 64 however few they are: below
+// 1.5 blocks per CU the tile is 16 rows.  The sums' order is the same.  300 rows, 1024 columns: K = 2048 33 -> 26 us, K = 3072 49 -> 39.
+constexpr int F_S = 3;
+constexpr int f_stage(int wm) { return (4 * wm + 8) * 1024; }
+template <int WM>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(GemmF32Args a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];   // F_S x [A first halves | A second halves | W]
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), G = lane >> 4, c = lane & 15, wm = wave >> 1, wn = wave & 1;
-  const int n0 = (int)blockIdx.y * 64, m0 = (int)blockIdx.x * 32;   // (consecutive blocks share the weights' tile)
+  constexpr int STAGE = f_stage(WM), HALF = WM * 2048, NA = WM, NR = WM, LEFT = (F_S - 2) * (NA + 2);   // A requests per wave, 16-column groups per wave
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), G = lane >> 4, c = lane & 15, wm = WM == 2 ? wave >> 1 : 0, wn = WM == 2 ? wave & 1 : wave;
+  const int n0 = (int)blockIdx.y * 64, m0 = (int)blockIdx.x * (WM * 16);   // (consecutive blocks share the weights' tile)
   const float* A = a.A + blockIdx.z * a.sa;
   const bf16_t* W = a.W + blockIdx.z * a.sw;
-  const char* src[4];   // requests wave * 2, wave * 2 + 1 of A and of W
+  const char *asrc[NA], *wsrc[2];   // requests wave * NA + j of A, wave * 2 + j of W
+#pragma unroll
+  for (int j = 0; j < NA; ++j) {
+    const int q = wave * NA + j, ar = q % (2 * WM) * 8 + (lane >> 3);
+    asrc[j] = (const char*)(A + (int64_t)min(m0 + ar, a.M - 1) * a.lda) + q / (2 * WM) * 128 + skinny_piece(ar, lane);
+  }
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    const int q = wave * 2 + j, ar = (q & 3) * 8 + (lane >> 3), wr = q * 8 + (lane >> 3);
-    src[j] = (const char*)(A + (int64_t)min(m0 + ar, a.M - 1) * a.lda) + (q >> 2) * 128 + skinny_piece(ar, lane);
-    src[2 + j] = (const char*)(W + (int64_t)min(n0 + wr, a.N - 1) * a.ldw) + skinny_piece(wr, lane);
+    const int wr = (wave * 2 + j) * 8 + (lane >> 3);
+    wsrc[j] = (const char*)(W + (int64_t)min(n0 + wr, a.N - 1) * a.ldw) + skinny_piece(wr, lane);
   }
   const int nk = a.K / 64;
   auto load = [&](int kt) {   // (past the end: the last stage again, never used)
     const int k = min(kt, nk - 1) * 128;
-    char* st = smem + kt % F_S * F_STAGE;
+    char* st = smem + kt % F_S * STAGE;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      __builtin_amdgcn_global_load_lds((glb_ptr_t)(src[j] + 2 * k), (lds_ptr_t)(st + (wave * 2 + j) * 1024), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((glb_ptr_t)(src[2 + j] + k), (lds_ptr_t)(st + (8 + wave * 2 + j) * 1024), 16, 0, 0);
-    }
+    for (int j = 0; j < NA; ++j) __builtin_amdgcn_global_load_lds((glb_ptr_t)(asrc[j] + 2 * k), (lds_ptr_t)(st + (wave * NA + j) * 1024), 16, 0, 0);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) __builtin_amdgcn_global_load_lds((glb_ptr_t)(wsrc[j] + k), (lds_ptr_t)(st + (4 * WM + wave * 2 + j) * 1024), 16, 0, 0);
   };
-  f32x4_t acc[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+  f32x4_t acc[NR];
+#pragma unroll
+  for (int r = 0; r < NR; ++r) acc[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < F_S - 1; ++s) load(s);
   for (int kt = 0; kt < nk; ++kt) {
-    __builtin_amdgcn_s_waitcnt(0x0F70 | ((F_S - 2) * 4));   // this wave's part of stage kt is in; behind the barrier everyone's, and stage kt - 1 is read
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (LEFT & 15) | ((LEFT >> 4) << 14));   // this wave's part of stage kt is in; behind the barrier everyone's, and stage kt - 1 is read
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     load(kt + F_S - 1);
-    const char* st = smem + kt % F_S * F_STAGE;
-    u32x4_t wf[2][2];
+    const char* st = smem + kt % F_S * STAGE;
+    u32x4_t wf[2][NR];
     f32x4_t af[2][2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
 #pragma unroll
-      for (int r = 0; r < 2; ++r) wf[h][r] = *reinterpret_cast<const u32x4_t*>(st + 8192 + skinny_swz(wn * 32 + r * 16 + c, h * 4 + G));
+      for (int r = 0; r < NR; ++r) wf[h][r] = *reinterpret_cast<const u32x4_t*>(st + 2 * HALF + skinny_swz(wn * (NR * 16) + r * 16 + c, h * 4 + G));
 #pragma unroll
-      for (int q = 0; q < 2; ++q) af[h][q] = *reinterpret_cast<const f32x4_t*>(st + h * 4096 + skinny_swz(wm * 16 + c, 2 * G + q));
+      for (int q = 0; q < 2; ++q) af[h][q] = *reinterpret_cast<const f32x4_t*>(st + h * HALF + skinny_swz(wm * 16 + c, 2 * G + q));
     }
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int j = 0; j < 8; ++j)
 #pragma unroll
-        for (int r = 0; r < 2; ++r)
+        for (int r = 0; r < NR; ++r)
           acc[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(j & 1 ? hi_bf(wf[h][r][j >> 1]) : lo_bf(wf[h][r][j >> 1]), af[h][j >> 2][j & 3], acc[r], 0, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);   // (the surplus requests: LDS may belong to the next block)
   const int m = m0 + wm * 16 + c;
 #pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    const int n = n0 + wn * 32 + r * 16 + G * 4;
+  for (int r = 0; r < NR; ++r) {
+    const int n = n0 + wn * (NR * 16) + r * 16 + G * 4;
     if (m < a.M && n < a.N) *reinterpret_cast<f32x4_t*>(a.C + blockIdx.z * a.sc + (int64_t)m * a.ldc + n) = acc[r];
   }
 }
@@ -184,7 +195,9 @@ void launch_gemm_f32(const float* A, int64_t lda, const void* W, int64_t ldw, fl
     return;
   }
   if (M > 64) {
-    hipLaunchKernelGGL(gemm_f32_kernel, dim3((unsigned)((M + 31) / 32), (unsigned)((N + 63) / 64), (unsigned)batch), dim3(256), F_S * F_STAGE, st, a);
+    const unsigned tn = (unsigned)((N + 63) / 64);
+    if ((int64_t)((M + 31) / 32) * tn * batch < 384) hipLaunchKernelGGL(gemm_f32_kernel<1>, dim3((unsigned)((M + 15) / 16), tn, (unsigned)batch), dim3(256), F_S * f_stage(1), st, a);
+    else hipLaunchKernelGGL(gemm_f32_kernel<2>, dim3((unsigned)((M + 31) / 32), tn, (unsigned)batch), dim3(256), F_S * f_stage(2), st, a);
     return;
   }
   auto go = [&](auto r8, auto m8) {
