@@ -484,7 +484,16 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(SsmStepArgs a, SeqBatch b
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       S[vt][i] = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (e.pos0 > 0 && n0 + i * 64 < np) S[vt][i] = *reinterpret_cast<const float4*>(sin + (vt * np + n0 + i * 64) * 16 + v4);
+      if (e.pos0 > 0 && n0 + i * 64 < np) {
+        const float* at = sin + (vt * np + n0 + i * 64) * 16 + v4;
+        // many sequences: states of hundreds of MB that nothing reads before the next step (8B widths, 32 sequences: 59.7 -> 50.8 us)
+        if constexpr (VT == 4) {
+          const f32x4_t x = __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(at));
+          S[vt][i] = make_float4(x[0], x[1], x[2], x[3]);
+        } else {
+          S[vt][i] = *reinterpret_cast<const float4*>(at);
+        }
+      }
     }
   const TI* row = (const TI*)a.in.p + (int64_t)e.row0 * a.in.ld;
   const float dtz = Act<TI>::ld(row + a.in.dt_off + h) + a.p.dt_bias[h];
@@ -493,7 +502,7 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(SsmStepArgs a, SeqBatch b
   float* hout = a.h.hist + (int64_t)e.slot * a.h.slot_stride + (int64_t)e.hist_out * (taps - 1) * cp;
   // The block's channels: x, B and C, NIT per thread.  Inputs, weights and history of up to HT + 1 taps are requested together and the new history is
   // stored behind them: a store between two loads orders them, and tap by tap, channel by channel the chain was most of the launch (0.6B widths,
-  // one sequence: 7.5 -> 5.3 us; 8B widths, 32 sequences, bound by the 268 MB of their states: 60.7 -> 59.7 us).
+  // one sequence: 7.5 -> 5.3 us; 8B widths, 32 sequences, bound by the 268 MB of their states: 60.7 -> 59.7 us, 50.8 past the caches).
   constexpr int NIT = (2 * NI * 64 + VT * 16 + 255) / 256, HT = 4;
   const int total = 2 * np + VT * 16;
   auto channel = [&](int i) { return i >= 2 * np ? h * a.d.vdp + vs * 16 + i - 2 * np : inner + (i < np ? grp * np + i : a.d.groups * np + grp * np + i - np); };
@@ -565,7 +574,9 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(SsmStepArgs a, SeqBatch b
         const float db = dt * bc[n], cn = bc[NI * 64 + n];
         float4& s = S[vt][i];
         s = make_float4(fmaf(db, x.x, da * s.x), fmaf(db, x.y, da * s.y), fmaf(db, x.z, da * s.z), fmaf(db, x.w, da * s.w));
-        *reinterpret_cast<float4*>(sout + (vt * np + n) * 16 + v4) = s;
+        float* at = sout + (vt * np + n) * 16 + v4;
+        if constexpr (VT == 4) __builtin_nontemporal_store(f32x4_t{s.x, s.y, s.z, s.w}, reinterpret_cast<f32x4_t*>(at));
+        else *reinterpret_cast<float4*>(at) = s;
         y = make_float4(fmaf(cn, s.x, y.x), fmaf(cn, s.y, y.y), fmaf(cn, s.z, y.z), fmaf(cn, s.w, y.w));
       }
     }
