@@ -85,9 +85,9 @@ GemvPlan plan_gemv(int N, int K, GemvEpi epi) {
 
 int gemv_num_tiles(int N, int K) { return plan_gemv(N, K, GEMV_LOGITS).grid; }
 
-// gemv_row_kernel where a wave's load group is a whole row of up to 3072 columns (0.6B: 2048 + 256 tokens
-// 209 -> 182 ms, 19 + 12 sampled ones 10.4 -> 9.1; at 4096 columns and 8B outputs the vector's registers cost a block per CU and the launch streams for longer than it ramps: 208.7 -> 210.3 ms per
-// 64-token answer with it).  false = not such a shape, nothing launched.
+// gemv_row_kernel where a wave's load group is a whole row of up to 3072 columns (0.6B: 2048 + 256 tokens 209 -> 182 ms, 19 + 12 sampled ones
+// 10.4 -> 9.1).  At 4096 columns the vector's registers cost a block per CU and an 8B launch streams for longer than it ramps: 208.7 -> 210.3 ms per
+// 64-token answer with it.  false = not such a shape, nothing launched.
 template <int EPI>
 static bool launch_gemv_row(const GemvArgs& a, const GemvPlan& p, hipStream_t st) {
   if (a.K % 512 != 0 || a.cached || a.h_out != nullptr || p.R > 2 || a.N < 1) return false;

@@ -183,6 +183,25 @@ def test_prompt_and_decoding_follow_the_equations(ctx, name, dtype):
     assert err(half, whole) <= TOL_SAME[dtype], name
 
 
+SHORT_ROWS = {   # name: (layers, width): the sizes of gemv_row_body.h -- K of 1024 (norms, 1021 of them real), 2048 (parts of 256), 3072 (experts' down) -- and neighbours
+    "whole load groups": ([ssm(heads=32, vdim=64, state=128, groups=8, norm_groups=8, mlp=MoeConfig(ff=768, experts=32, top=2, shared_ff=1536)),
+                           att(heads=16, dim=128, rot_dim=64, vdim=128, kv_rank=256, mlp=GatedConfig(3072))], 1024),
+    "pad columns, four choices of 64": ([ssm(heads=32, vdim=64, state=64, groups=2, norm_groups=8, mlp=MoeConfig(ff=509, experts=64, top=4, shared_ff=1020)),
+                                         ssm(heads=32, vdim=64, state=40, groups=4, norm_groups=4, mlp=GatedConfig(1500))], 1021),
+    "one choice of 70": ([ssm(heads=16, vdim=64, state=64, groups=2, norm_groups=4, mlp=MoeConfig(ff=1024, experts=70, top=1, shared_ff=2048))], 1024),
+}
+
+
+@pytest.mark.parametrize("name", list(SHORT_ROWS))
+def test_one_token_steps_on_short_rows(ctx, name):
+    layers, width = SHORT_ROWS[name]
+    cfg = config(layers, width=width, dtype="bfloat16")
+    w = vamatar_weights(cfg, seed=len(name))
+    ids, want = clear_ids(cfg, w, 40, 1, 0.03)
+    with Model(ctx, cfg, w) as m:
+        assert err(all_logits(m, ids, [12] + [1] * 28), want) <= TOL["bfloat16"]
+
+
 # ---- every mechanism, by leaving it out or getting it wrong in the restatement ------------------------------------------------------------
 def mistakes():
     """name -> (function of the restatement, its mistaken version)"""
