@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "common.h"
+#include "expert_choice.h"
 #include "layered.h"
 #include "model.h"
 #include "audio.h"
@@ -361,6 +362,24 @@ int aha_hip_debug_streamk_plan(int32_t M, int32_t N, int32_t K, int32_t tile_n, 
     return AHA_ERR_INVALID;
   }
   return n;
+}
+int aha_hip_debug_expert_choice(const float* z, int32_t experts, int32_t top, int32_t* sel, float* weight) {
+  if (!z || !sel || !weight || experts <= 0 || experts > 64 || top <= 0 || top > experts || top >= 64) {
+    set_error("debug_expert_choice: bad argument");
+    return AHA_ERR_INVALID;
+  }
+  float v[64];
+  for (int lane = 0; lane < 64; ++lane) v[lane] = choice_logit(lane < experts ? z[lane] : -INFINITY);
+  for (int k = 0; k < top; ++k) {
+    float m = v[0];
+    for (int lane = 1; lane < 64; ++lane) m = fmaxf(m, v[lane]);
+    uint64_t at = 0;
+    for (int lane = 0; lane < 64; ++lane) at |= (uint64_t)(v[lane] == m) << lane;
+    sel[k] = choice_lane(m, at, experts);
+    weight[k] = choice_weight(m);
+    if (sel[k] >= 0 && sel[k] < 64) v[sel[k]] = -INFINITY;
+  }
+  return AHA_OK;
 }
 int aha_hip_set_gemm_reserved_cus(int32_t n) {
   set_gemm_reserved_cus(n);

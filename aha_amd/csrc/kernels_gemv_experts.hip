@@ -1,5 +1,6 @@
 // Decode matvecs of the routed experts (layered_prenorm.hip), as kernels_gemv_fused.hip: the chosen experts found in the prologue, their gate and up
 // rows and the shared expert's streamed as one matrix behind LayerNorm; then down of all of them as one product over the concatenated activations.
+#include "expert_choice.h"
 #include "gemv_prologues.h"
 #include "gemv_row_body.h"
 
@@ -136,13 +137,14 @@ struct RowExpertsUpPro : RowLayerNormPro<2> {
     RowLayerNormPro<2>::request();
     sel = 0;
     sw = 1.f;
-    for (int k = 0; k < top; ++k) {   // the largest, ties to the lower index (as wave_topk; nothing but -inf or NaN left: the last)
+    v = choice_logit(v);
+    for (int k = 0; k < top; ++k) {   // (wave_topk's choices)
       const float m = wave_max(v);
-      const int bi = m == -INFINITY ? experts - 1 : __builtin_ctzll(__ballot(v == m));
+      const int bi = choice_lane(m, __ballot(v == m), experts);
       if (lane == bi) v = -INFINITY;
       if (lane == k) {
         sel = bi;
-        sw = 1.0f / (1.0f + expf(-m));
+        sw = choice_weight(m);
       }
     }
     if (blockIdx.x == 0 && (int)threadIdx.x < top) sel_out[threadIdx.x] = sel;

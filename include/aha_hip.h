@@ -451,6 +451,9 @@ int aha_hip_debug_few_rows_gemm(int32_t M, int32_t N, int32_t K, int32_t act, in
  * that every (tile, K tile) is covered exactly once for the BASELINE shapes. */
 int aha_hip_debug_streamk_plan(int32_t M, int32_t N, int32_t K, int32_t tile_n, int32_t workers, size_t workspace_bytes, int32_t* out,
                                int32_t cap, int32_t* off_out, int32_t* info7);
+/* Host only (no GPU): the experts that the decode matvec of up to 64 of them chooses for a row of router logits (csrc/expert_choice.h), the wave restated
+ * lane by lane: sel, weight (top), largest first.  Lets the CPU tier pin the choice for logits that are not finite. */
+int aha_hip_debug_expert_choice(const float* z, int32_t experts, int32_t top, int32_t* sel, float* weight);
 /* CUs the persistent GEMM kernel leaves free (rounded so that its workgroup count stays a multiple of 8; 0 = use every CU; < 0 = take
  * AHA_GEMM_RESERVE_CUS from the environment).  Process-wide.  For tensor-parallel prefill: RCCL's kernels on the communication stream
  * need CUs next to a GEMM whose workgroups each fill one (csrc/model.hip gemm_row_parallel).  Must be the same on every rank only

@@ -124,6 +124,39 @@ def test_routing_picks_the_largest_scores_and_weights_the_input():
     assert torch.allclose(got, want)
 
 
+def largest_logits(z, top):
+    """The choice of any number of experts (wave_topk): a logit that is not a number, or -inf, is never larger than another; the lowest index among equals,
+    the last expert when nothing is left."""
+    left, out = z.copy(), []
+    for _ in range(top):
+        m = np.fmax.reduce(left, initial=np.float32(-np.inf))
+        i = int(np.flatnonzero(left == m)[0]) if m > -np.inf else len(z) - 1
+        left[i] = -np.inf
+        out.append((i, 1 / (1 + np.exp(-m, dtype=np.float32))))
+    return out
+
+
+@pytest.mark.parametrize("experts,top", [(1, 1), (2, 2), (63, 1), (63, 6), (63, 63), (64, 1), (64, 6), (64, 63)])
+def test_one_logit_per_lane_chooses_the_same_experts(hip_lib, experts, top):
+    """csrc/expert_choice.h: finite logits, ties, infinities, NaN in some, in all but one and in every place, with and without spare lanes"""
+    rng = np.random.default_rng(experts * 100 + top)
+    rows = [rng.standard_normal(experts), rng.integers(0, 3, experts).astype(float), np.full(experts, np.nan), np.full(experts, -np.inf), np.full(experts, np.inf)]
+    some = rng.standard_normal(experts)
+    some[rng.random(experts) < 0.5] = np.nan
+    one = np.full(experts, np.nan)
+    one[experts // 2] = -3
+    mixed = rng.standard_normal(experts)
+    mixed[::3], mixed[1::5], mixed[-1] = -np.inf, np.nan, np.inf
+    for z in rows + [some, one, mixed]:
+        z = z.astype(np.float32)
+        sel, weight = np.full(top, -77, np.int32), np.full(top, -77, np.float32)
+        assert hip_lib.aha_hip_debug_expert_choice(z.ctypes.data, experts, top, sel.ctypes.data, weight.ctypes.data) == 0
+        with np.errstate(over="ignore"):
+            want = largest_logits(z, top)
+        assert sel.tolist() == [i for i, _ in want], z
+        assert np.allclose(weight, [w for _, w in want], rtol=1e-6, atol=0), z
+
+
 def test_one_cache_serves_the_layers_that_name_it():
     cfg = cfg_small()
     w = {k: v.double() for k, v in vamatar_weights(cfg, seed=1).items()}

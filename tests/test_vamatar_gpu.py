@@ -202,6 +202,24 @@ def test_one_token_steps_on_short_rows(ctx, name):
         assert err(all_logits(m, ids, [12] + [1] * 28), want) <= TOL["bfloat16"]
 
 
+def test_a_token_that_is_not_finite_among_64_experts(ctx):
+    """All 64 router logits of its row are NaN: its own logits are not finite, the steps of another sequence around it keep their bits."""
+    cfg = config([ssm(heads=32, vdim=64, state=64, groups=2, norm_groups=8, mlp=MoeConfig(ff=512, experts=64, top=4, shared_ff=1024))], width=1024, dtype="bfloat16")
+    w = vamatar_weights(cfg, seed=3)
+    w["embed"][7] = float("nan")
+    ids = [i + (i == 7) for i in tokens(9, cfg.vocab_size, 2)]
+    with Model(ctx, cfg, w) as m:
+        want = all_logits(m, ids, [5, 1, 1, 1, 1])
+        s, bad = m.seq_open(), m.seq_open()
+        got = [m.forward_batch([(s, ids[:5], list(range(5)))])[0]]
+        m.forward_batch([(bad, ids[:5], [4])])
+        for i in range(5, 9):
+            lost, _ = m.forward_batch([(bad, [7], [0])])
+            assert not np.isfinite(lost).any()
+            got.append(m.forward_batch([(s, [ids[i]], [0])])[0])
+    assert np.isfinite(want).all() and (np.concatenate(got) == want).all()
+
+
 # ---- every mechanism, by leaving it out or getting it wrong in the restatement ------------------------------------------------------------
 def mistakes():
     """name -> (function of the restatement, its mistaken version)"""
