@@ -7,8 +7,8 @@
 // operands that waves load to registers themselves as MFMA fragments touch 16 rows x 64 bytes per request and ran at half the rate (6144 x 4096,
 // 8 rows: 17.5 us against 10.4 us).  A's rows go the same way: each block reads all of A, so blocks have as many weight rows as one round over
 // the chip allows (gemm_skinny_plan).
-// Rows past M, N repeat the last one; what they give is not stored.  Lanes of a fragment that no row backs read whatever LDS holds behind the
-// stage: an MFMA's output rows and columns do not mix.
+// Rows past M, N repeat the last one, lanes of a fragment that no row backs another row; what they give is not stored: an MFMA's output rows and columns
+// do not mix.
 //
 // Measured on MI355X, back to back from HBM, 8 rows (in brackets: the split-K ring kernel + its reduce pass it replaces, inside a batched step):
 //   6144 x 4096 10.4 us (4.8 TB/s), 4096 x 4096 8.1, 12288 x 4096 18.0 (5.6), 4096 x 12288 17.9 (5.6), 24576 x 4096 33.1 (6.1)
@@ -26,7 +26,7 @@ namespace aha {
 
 namespace {
 
-template <int R8, int M8, bool PAIRS, bool ONE_BLOCK>
+template <int R8, int M8, bool PAIRS, bool DEEP>
 __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const void* A, const void* W, int M, int N, int K, int64_t lda, int64_t ldw, GemmArgs a) {
   // (what the first requests need: in scalar registers at the start, gemv_body.h)
   a.A = A;
@@ -51,7 +51,7 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const vo
       src[r] = (const char*)a.W + (int64_t)min((int)blockIdx.x * (R8 * 8) + local, a.N - 1) * a.ldw * 2 + piece;
     }
   }
-  skinny_sums<R8, M8, false, ONE_BLOCK>(src, a.K / 64, gemm_smem, wave, lane);
+  skinny_sums<R8, M8, false, DEEP>(src, a.K / 64, gemm_smem, wave, lane);
   for (int i = wave; i < NF * MT; i += SKINNY_WAVES) {
     const int r = i / MT, m = (int)blockIdx.y * 64 + (i - r * MT) * 16 + c;
     if (m >= a.M) continue;
@@ -81,14 +81,14 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const vo
   }
 }
 
-template <int R8, int M8, bool PAIRS, bool ONE_BLOCK = false>
+template <int R8, int M8, bool PAIRS, bool DEEP = false>
 void launch_one(const GemmArgs& a, hipStream_t st) {
-  if constexpr (!ONE_BLOCK && skinny_stages(R8 + M8) != skinny_stages(R8 + M8, true))
+  if constexpr (!DEEP && skinny_stages(R8 + M8) != skinny_stages(R8 + M8, true))
     if (gemm_skinny_rounds(a, R8) == 1) return launch_one<R8, M8, PAIRS, true>(a, st);
-  constexpr int lds = skinny_lds(R8, M8, false, ONE_BLOCK);
+  constexpr int lds = skinny_lds(R8, M8, false, DEEP);
   if (lds > 64 * 1024)
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_skinny_kernel<R8, M8, PAIRS, ONE_BLOCK>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  hipLaunchKernelGGL((gemm_skinny_kernel<R8, M8, PAIRS, ONE_BLOCK>), dim3((unsigned)((a.N + R8 * 8 - 1) / (R8 * 8)), (unsigned)((a.M + 63) / 64)), dim3(SKINNY_WAVES * 64), lds, st, a.A, a.W, a.M, a.N, a.K, a.lda,
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_skinny_kernel<R8, M8, PAIRS, DEEP>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  hipLaunchKernelGGL((gemm_skinny_kernel<R8, M8, PAIRS, DEEP>), dim3((unsigned)((a.N + R8 * 8 - 1) / (R8 * 8)), (unsigned)((a.M + 63) / 64)), dim3(SKINNY_WAVES * 64), lds, st, a.A, a.W, a.M, a.N, a.K, a.lda,
                      a.ldw, a);
 }
 

@@ -10,18 +10,29 @@ namespace aha {
 namespace {
 
 constexpr int SKINNY_WAVES = 4;
-// A CU's share of HBM's rate times a request's latency is ~50 KB.  Narrow stages come in as many as keep two blocks per CU (18 to 20 KB per wave); wide
-// ones have enough in flight with two where blocks share a CU (three of them leave one block), and take three in a launch of one block per CU.
-// Eight rows inside a batched step, three stages (two from seven requests on) before: 6144 x 4096 11.9 -> 10.9 us, 12288 x 4096 19.8 -> 18.0, 4096 x 4096
-// and 4096 x 12288 13.5 -> 12.7 on average.  Nothing is requested past the end (three surplus stages of a wave's four chunks at K = 1024 before).
-constexpr int skinny_stages(int requests, bool one_block = false) { return requests <= 3 ? 6 : requests == 4 ? 5 : requests == 5 ? 4 : requests <= 6 || (one_block && requests <= 8) ? 3 : 2; }
+// Stages of a wave's ring.  Where blocks share a CU: three up to six requests each, two of wider ones.  Two to four blocks then hide each other's latency;
+// more stages take the LDS that a neighbour needs (blocks of 16 weight rows: 151936 x 1024, 8 rows, 47.6 us with three stages, 60.0 with six; 32 bits,
+// 12288 x 4096, 2 rows, 20.4 with three, 29.6 with five and one block per CU).  DEEP, a block that has its CU to itself: as many as cover a request's
+// latency at a CU's share of HBM's rate, ~50 KB (8 rows: 4096 x 4096 8.0 us against 8.1 with three, 2048 x 4096 6.1 against 6.3).  Nothing is requested
+// past the end.
+constexpr int skinny_stages(int requests, bool deep = false) {
+  if (deep) return requests <= 3 ? 6 : requests == 4 ? 5 : requests == 5 ? 4 : requests <= 8 ? 3 : 2;
+  return requests <= 6 ? 3 : 2;
+}
 constexpr int skinny_requests(int r8, int m8, bool f32) { return r8 + (f32 ? 2 : 1) * m8; }
-constexpr int skinny_lds(int r8, int m8, bool f32 = false, bool one_block = false) {
+constexpr int skinny_lds(int r8, int m8, bool f32 = false, bool deep = false) {
   const int per = skinny_requests(r8, m8, f32);
-  const int ring = SKINNY_WAVES * skinny_stages(per, one_block) * per * 1024 + ((r8 | m8) & 1) * 1024;   // odd: half a fragment is read behind the last stage
+  const int ring = SKINNY_WAVES * skinny_stages(per, deep) * per * 1024;
   const int sums = SKINNY_WAVES * ((r8 + 1) / 2) * ((m8 + 1) / 2) * 1024;
   return ring > sums ? ring : sums;
 }
+
+constexpr bool skinny_fits() {
+  for (int q = 2; q <= 14; ++q)
+    if ((q <= 10 ? 2 : 1) * SKINNY_WAVES * skinny_stages(q) * q > 160 || SKINNY_WAVES * skinny_stages(q, true) * q > 160) return false;
+  return true;
+}
+static_assert(skinny_fits(), "up to ten requests two blocks fit into the 160 KB of a CU");
 
 // 16-byte piece `slot` of row `row` inside a stage's [rows][64] bf16 image
 __device__ __forceinline__ int skinny_swz(int row, int slot) { return row * 128 + ((slot ^ ((row >> 1) & 7)) << 4); }
@@ -33,11 +44,11 @@ __device__ __forceinline__ int skinny_piece(int local_row, int lane) { return ((
 // v_mfma_f32_16x16x4_f32 (weights widened exactly): in step (h, j) lane group G feeds k = (h * 4 + G) * 8 + j of both operands.
 // On return the waves' sums of the 16 x 16 fragments (weight fragment r, activation fragment m) lie in LDS and every wave may read them
 // (skinny_total).
-template <int R8, int M8, bool F32 = false, bool ONE_BLOCK = false>
+template <int R8, int M8, bool F32 = false, bool DEEP = false>
 __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R8, M8, F32)], int nc, char* smem, int wave, int lane) {
   typedef __attribute__((address_space(3))) void* lds_t;
   typedef const __attribute__((address_space(1))) void* glb_t;
-  constexpr int NF = (R8 + 1) / 2, MT = (M8 + 1) / 2, PER = skinny_requests(R8, M8, F32), S = skinny_stages(PER, ONE_BLOCK);
+  constexpr int NF = (R8 + 1) / 2, MT = (M8 + 1) / 2, PER = skinny_requests(R8, M8, F32), S = skinny_stages(PER, DEEP);
   constexpr int LEFT = (S - 1) * PER;   // requests of the later stages
   static_assert(LEFT < 64, "vmcnt has six bits");
   const int G = lane >> 4, c = lane & 15;
@@ -56,13 +67,15 @@ __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R
 #pragma unroll
     for (int r = R8; r < PER; ++r) __builtin_amdgcn_global_load_lds((glb_t)(src[r] + ka), (lds_t)(ring + (u * PER + r) * 1024), 16, 0, 0);
   };
+  // an odd count leaves half a fragment without rows: its lanes read the other half's again (behind the last stage there may be no LDS)
+  const int cw = R8 % 2 ? c & 7 : c, ca = M8 % 2 ? c & 7 : c;   // (of the last fragment)
   auto consume = [&](int u) {
     const char *sw = ring + u * PER * 1024, *sa = sw + R8 * 1024;
     u32x4_t wf[2][NF];
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int r = 0; r < NF; ++r) wf[h][r] = *reinterpret_cast<const u32x4_t*>(sw + skinny_swz(r * 16 + c, h * 4 + G));
+      for (int r = 0; r < NF; ++r) wf[h][r] = *reinterpret_cast<const u32x4_t*>(sw + skinny_swz(r * 16 + (r + 1 == NF ? cw : c), h * 4 + G));
     if constexpr (F32) {
       f32x4_t af[2][MT][2];
 #pragma unroll
@@ -70,7 +83,7 @@ __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
-          for (int q = 0; q < 2; ++q) af[h][m][q] = *reinterpret_cast<const f32x4_t*>(sa + h * (M8 * 1024) + skinny_swz(m * 16 + c, 2 * G + q));
+          for (int q = 0; q < 2; ++q) af[h][m][q] = *reinterpret_cast<const f32x4_t*>(sa + h * (M8 * 1024) + skinny_swz(m * 16 + (m + 1 == MT ? ca : c), 2 * G + q));
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -86,7 +99,7 @@ __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int m = 0; m < MT; ++m) af[h][m] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(sa + skinny_swz(m * 16 + c, h * 4 + G)));
+        for (int m = 0; m < MT; ++m) af[h][m] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(sa + skinny_swz(m * 16 + (m + 1 == MT ? ca : c), h * 4 + G)));
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
