@@ -123,7 +123,7 @@ double gemm_skinny_plan(const GemmArgs& a, int* r8_out) {
     double c = 3.0 + (r8 + 0.4 * m8) * chunk / 30e3;
     if (rounds > 1) {
       if (a.M > 64) continue;
-      const int resident = std::min(4, 160 * 1024 / skinny_lds(r8, m8)), rows8 = (a.M + 7) / 8;
+      const int resident = std::min(4, skinny_blocks(r8, m8)), rows8 = (a.M + 7) / 8;
       const double cu = rounds * r8 * chunk / 60e3, chip = a.N / 8 * chunk / 8.2e6 * (r8 == 4 && a.ldw * 64 % (256 << 10) == 0 ? 1.34 : 1.0);
       c = 3.5 + sqrt(cu * cu + chip * chip) + rounds * rows8 * chunk / 96e3 + ((rounds + resident - 1) / resident - 1) * 0.25 * rows8 + 0.075 * rounds * m8;
     }

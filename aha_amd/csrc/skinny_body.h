@@ -27,12 +27,10 @@ constexpr int skinny_lds(int r8, int m8, bool f32 = false, bool deep = false) {
   return ring > sums ? ring : sums;
 }
 
-constexpr bool skinny_fits() {
-  for (int q = 2; q <= 14; ++q)
-    if ((q <= 10 ? 2 : 1) * SKINNY_WAVES * skinny_stages(q) * q > 160 || SKINNY_WAVES * skinny_stages(q, true) * q > 160) return false;
-  return true;
-}
-static_assert(skinny_fits(), "up to ten requests two blocks fit into the 160 KB of a CU");
+constexpr int skinny_blocks(int r8, int m8, bool f32 = false) { return 160 * 1024 / skinny_lds(r8, m8, f32); }   // per CU
+static_assert(skinny_blocks(2, 1) == 4 && skinny_blocks(2, 2) == 3 && skinny_blocks(3, 1) == 3 && skinny_blocks(2, 1, true) == 3, "narrow stages: room for three and more blocks");
+static_assert(skinny_blocks(2, 4) == 2 && skinny_blocks(2, 8) == 2 && skinny_blocks(3, 4) == 2 && skinny_blocks(4, 2) == 2 && skinny_blocks(6, 4) == 2 && skinny_blocks(6, 2, true) == 2,
+              "up to ten requests: two");
 
 // 16-byte piece `slot` of row `row` inside a stage's [rows][64] bf16 image
 __device__ __forceinline__ int skinny_swz(int row, int slot) { return row * 128 + ((slot ^ ((row >> 1) & 7)) << 4); }
