@@ -3,7 +3,7 @@
 // What bounds it is the weight matrix, read once from HBM; the 128-row tiles of kernels_gemm.hip stage 16 times the rows a batch of eight has and
 // need K slices and a reduce pass to fill the chip.  Here a block owns R8 * 8 weight rows and the whole K range, its four waves take the 64-wide
 // k chunks in turn, and every wave has a ring of S chunks of its own in LDS that it fills by DMA and drains by itself: no barrier before the sums
-// of the four waves are joined, 2 KB to 9 KB of weights per stage in flight per wave.  A DMA request covers eight rows x 128 bytes (whole lines);
+// of the four waves are joined, two to six stages of 3 KB to 14 KB in flight per wave (skinny_stages).  A DMA request covers eight rows x 128 bytes (whole lines);
 // operands that waves load to registers themselves as MFMA fragments touch 16 rows x 64 bytes per request and ran at half the rate (6144 x 4096,
 // 8 rows: 17.5 us against 10.4 us).  A's rows go the same way: each block reads all of A, so blocks have as many weight rows as one round over
 // the chip allows (gemm_skinny_plan).
@@ -11,10 +11,10 @@
 // do not mix.
 //
 // Measured on MI355X, back to back from HBM, 8 rows (in brackets: the split-K ring kernel + its reduce pass it replaces, inside a batched step):
-//   6144 x 4096 10.4 us (4.8 TB/s), 4096 x 4096 8.1, 12288 x 4096 18.0 (5.6), 4096 x 12288 17.9 (5.6), 24576 x 4096 33.1 (6.1)
-//   [18.1 + 4.6 us on average over the first four]; 32 rows: 12.1, 10.1, 19.7, 25.9, 37.2; 64 rows: 15.5, 13.4, 23.3, 35.5, 45.9
-//   64-row tiles, 96 / 128 rows (tiled kernels with their reduce pass): 4096 x 1024 6.7 / 6.9 us (10.7 / 10.7), 6144 x 1024 8.5 / 8.6 (12.1 / 12.9),
-//   1024 x 2048 7.0 / 7.7 (11.3 / 12.1), 1024 x 3072 9.0 / 10.2 (12.3 / 13.2); a 0.6B prompt of 96 / 128 / 180 / 250 tokens 1.66 / 1.67 / 1.95 / 2.03 ms
+//   6144 x 4096 10.4 us (4.8 TB/s), 4096 x 4096 8.0, 12288 x 4096 18.5 (5.4), 4096 x 12288 17.7 (5.7), 24576 x 4096 32.8 (6.1)
+//   [18.1 + 4.6 us on average over the first four]; 32 rows: 11.9, 9.7, 19.3, 25.5, 34.9; 64 rows: 15.7, 13.1, 23.2, 35.1, 45.0
+//   64-row tiles, 96 / 128 rows (tiled kernels with their reduce pass): 4096 x 1024 6.2 / 6.4 us (10.7 / 10.7), 6144 x 1024 8.1 / 8.3 (12.1 / 12.9),
+//   1024 x 2048 6.6 / 7.1 (11.3 / 12.1), 1024 x 3072 8.7 / 9.7 (12.3 / 13.2); a 0.6B prompt of 96 / 128 / 180 / 250 tokens 1.66 / 1.67 / 1.95 / 2.03 ms
 //   (1.97 / 2.06 / 2.07 / 2.14), of 300 2.14 (2.09): 256 rows at most.  The 8B shapes stay on the tiles:
 //   their weight rows need more than one round or a longer K than a block streams in the tiles' time (6144 x 4096, 96 rows: 21.3 against 21.0).
 #include <algorithm>
@@ -110,9 +110,12 @@ int gemm_skinny_rounds(const GemmArgs& a, int r8) { return ((a.N + r8 * 8 - 1) /
 // More rounds, up to 64 rows (4096 x 1024, 180 rows, 384 blocks: 12.0 us against 10.9 of the tiles): a CU requests at most 60 bytes of weights per ns and
 // the chip delivers at most 8.2 TB/s (32 rows per block that lie whole 256 KB apart: 1.34 times as long, their requests meet in the same channels),
 // rounded where the two meet; A's rows at 96 bytes per ns and CU, the last row's repetitions for nothing; a block's first requests and the joined sums
-// show where no neighbour on the CU covers them.  Fitted to 23 shapes (512 x 4096 to 151936 x 4096) at 1 to 64 rows with every R8, 6 % off on average.
-// The price of one round times their number said 41 us with 32 rows per block for 32768 x 4096 and 8 rows (60.6; 44.5 with 48) and 76 us for
-// 151936 x 1024 and 64 rows (102; the tiles 73).
+// show where no neighbour on the CU covers them.  Fitted to 23 shapes (512 x 4096 to 151936 x 4096) at 1 to 64 rows with every R8 before the rings asked
+// for nothing past the end; since then 12 % dear on average in several rounds (mostly short K), and a width chosen with it is 1.5 % behind the best on average:
+// at most 4 % but for 32 weight rows per block that lie 256 KB apart in ONE round, where it knows nothing of their channels (8192 x 4096, 8 rows: 18.2 us, 13.0
+// with 48), 16384 x 4096 at 16 rows (27.0, 23.8 with 24) and 12288 x 4096 at 8 (18.5, 17.4 with 24).
+// The price of one round times their number said 41 us with 32 rows per block for 32768 x 4096 and 8 rows (57.7; 42.6 with 48) and 76 us for
+// 151936 x 1024 and 64 rows (96.6; the tiles 73).
 double gemm_skinny_plan(const GemmArgs& a, int* r8_out) {
   const int m8 = a.M <= 8 ? 1 : a.M <= 16 ? 2 : a.M <= 32 ? 4 : 8;
   const double chunk = a.K * 16.0;   // bytes of eight rows
