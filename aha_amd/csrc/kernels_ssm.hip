@@ -468,7 +468,8 @@ __global__ __launch_bounds__(256) void ssm_segments_kernel(SsmScanArgs a, SeqBat
 // ---- one token per sequence ------------------------------------------------------------------------------------------------------------------
 // Block (head and VT * 16 of its columns, sequence): thread (n, four columns of 16), n = tid / 4, + 64, ...  The state is requested first; the
 // convolution of the block's channels (its x columns, the group's B and C) runs under that.
-template <typename TI, int NI, int VT>
+// NT: the state past the caches (launch_ssm_step).
+template <typename TI, int NI, int VT, bool NT>
 __global__ __launch_bounds__(256) void ssm_step_kernel(SsmStepArgs a, SeqBatch b) {
   __shared__ __attribute__((aligned(16))) float bc[2 * NI * 64], xs[VT * 16], red[4][VT * 16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nvs = a.d.vdp >> 4, h = blockIdx.x / (nvs / VT), vs = (blockIdx.x - h * (nvs / VT)) * VT, np = a.d.np, taps = a.d.taps;
@@ -486,8 +487,7 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(SsmStepArgs a, SeqBatch b
       S[vt][i] = make_float4(0.f, 0.f, 0.f, 0.f);
       if (e.pos0 > 0 && n0 + i * 64 < np) {
         const float* at = sin + (vt * np + n0 + i * 64) * 16 + v4;
-        // many sequences: states of hundreds of MB that nothing reads before the next step (8B widths, 32 sequences: 59.7 -> 50.8 us)
-        if constexpr (VT == 4) {
+        if constexpr (NT) {
           const f32x4_t x = __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(at));
           S[vt][i] = make_float4(x[0], x[1], x[2], x[3]);
         } else {
@@ -575,7 +575,7 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(SsmStepArgs a, SeqBatch b
         float4& s = S[vt][i];
         s = make_float4(fmaf(db, x.x, da * s.x), fmaf(db, x.y, da * s.y), fmaf(db, x.z, da * s.z), fmaf(db, x.w, da * s.w));
         float* at = sout + (vt * np + n) * 16 + v4;
-        if constexpr (VT == 4) __builtin_nontemporal_store(f32x4_t{s.x, s.y, s.z, s.w}, reinterpret_cast<f32x4_t*>(at));
+        if constexpr (NT) __builtin_nontemporal_store(f32x4_t{s.x, s.y, s.z, s.w}, reinterpret_cast<f32x4_t*>(at));
         else *reinterpret_cast<float4*>(at) = s;
         y = make_float4(fmaf(cn, s.x, y.x), fmaf(cn, s.y, y.y), fmaf(cn, s.z, y.z), fmaf(cn, s.w, y.w));
       }
@@ -796,16 +796,22 @@ void launch_ssm_step(const SsmStepArgs& a, const SeqBatch& b, hipStream_t st) {
   if (b.n <= 0) return;
   const int nvs = a.d.vdp >> 4;
   const bool wide = nvs % 4 == 0 && (int64_t)a.d.heads * nvs / 4 * b.n >= 512;   // B and C of the group once per 64 columns
+  // From 16 MB of states per launch on, past the caches: nothing reads them before the next step, and they push out what is read (128 dims of state, 16 MB:
+  // 10.4 -> 9.0 us at 4 sequences of the 8B widths, 11.4 -> 10.0 at 16 of the 0.6B ones, in stacks of 2 to 28 layers; 268 MB: 59.7 -> 50.8).  Smaller ones
+  // are still there in the next step (2 MB 6.6 against 7.2 us past the caches, 8 MB 7.4 against 8.1).
+  const bool past = (int64_t)b.n * a.d.heads * a.d.vdp * a.d.np * 4 >= 16 << 20;
   const dim3 grid((unsigned)(a.d.heads * nvs / (wide ? 4 : 1)), (unsigned)b.n), block(256);
   auto go = [&](auto ni) {
     constexpr int NI = decltype(ni)::value;
-    auto run = [&](auto vt) {
+    auto run = [&](auto vt, auto nt) {
       constexpr int VT = decltype(vt)::value;
-      if (a.in_f32) hipLaunchKernelGGL((ssm_step_kernel<float, NI, VT>), grid, block, 0, st, a, b);
-      else hipLaunchKernelGGL((ssm_step_kernel<bf16_t, NI, VT>), grid, block, 0, st, a, b);
+      constexpr bool NT = decltype(nt)::value;
+      if (a.in_f32) hipLaunchKernelGGL((ssm_step_kernel<float, NI, VT, NT>), grid, block, 0, st, a, b);
+      else hipLaunchKernelGGL((ssm_step_kernel<bf16_t, NI, VT, NT>), grid, block, 0, st, a, b);
     };
-    if (wide) run(std::integral_constant<int, 4>{});
-    else run(std::integral_constant<int, 1>{});
+    if (!wide) run(std::integral_constant<int, 1>{}, std::false_type{});
+    else if (past) run(std::integral_constant<int, 4>{}, std::true_type{});
+    else run(std::integral_constant<int, 4>{}, std::false_type{});
   };
   if (a.d.np <= 64) go(std::integral_constant<int, 1>{});
   else if (a.d.np <= 128) go(std::integral_constant<int, 2>{});

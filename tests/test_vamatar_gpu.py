@@ -465,6 +465,20 @@ def test_more_sequences_than_the_first_slots_keep_their_states(ctx, dtype, wide)
         assert row_err(got[:, i], want[6:14]).max() <= TOL[dtype], i
 
 
+@pytest.mark.parametrize("state,n", [(64, 4), (60, 7), (64, 8), (90, 6)])
+def test_step_of_states_on_both_sides_of_the_caches(ctx, state, n):
+    """128 heads x 64 values in blocks of 64 columns: 8 to 17 MB of states per layer (16 MB: past the caches)"""
+    cfg = config([ssm(heads=128, vdim=64, state=state, groups=8, norm_groups=8)] * 2, dtype="bfloat16")
+    w = vamatar_weights(cfg, seed=state)
+    ids = [tokens(9, cfg.vocab_size, 50 + i) for i in range(n)]
+    with Model(ctx, cfg, w) as m:
+        seqs = [m.seq_open() for _ in ids]
+        m.forward_batch([(s, x[:5], []) for s, x in zip(seqs, ids)])
+        got = np.stack([m.forward_batch([(s, x[i:i + 1], [0]) for s, x in zip(seqs, ids)])[0] for i in range(5, 9)], 1)
+    for i, x in enumerate(ids):
+        assert err(got[i], reference(cfg, w, x)[5:]) <= TOL["bfloat16"], i
+
+
 def test_a_slot_used_again_starts_from_nothing(ctx):
     cfg = config([ssm(), att(window=30), ssm()], dtype="bfloat16")
     w = vamatar_weights(cfg, seed=10)
