@@ -363,6 +363,13 @@ int aha_hip_debug_streamk_plan(int32_t M, int32_t N, int32_t K, int32_t tile_n, 
   }
   return n;
 }
+int aha_hip_debug_gemv_row_groups(int32_t N, int32_t K, int32_t epi) {
+  if (N <= 0 || K <= 0 || epi < GEMV_STORE || epi > GEMV_AXPY_F32) {
+    set_error("debug_gemv_row_groups: bad argument");
+    return AHA_ERR_INVALID;
+  }
+  return gemv_row_groups(N, K, (GemvEpi)epi);
+}
 int aha_hip_debug_expert_choice(const float* z, int32_t experts, int32_t top, int32_t* sel, float* weight) {
   if (!z || !sel || !weight || experts <= 0 || experts > 64 || top <= 0 || top > experts || top >= 64) {
     set_error("debug_expert_choice: bad argument");

@@ -51,6 +51,8 @@ struct GemvMerge {
 void launch_gemv_merge(const GemvArgs& a, const GemvMerge& p, hipStream_t st);
 struct GemvPlan { int R, U, grid; };   // rows per wave, 512-column chunks per load group, persistent blocks
 GemvPlan plan_gemv(int N, int K, GemvEpi epi);
+bool gemv_row_on();   // the short forms (gemv_row_body.h) are not switched off by a knob of the block form
+int gemv_row_groups(int N, int K, GemvEpi epi);   // load groups per row of the short form that launch_gemv takes, 0: the block form (host only)
 int gemv_num_tiles(int N, int K);  // number of (max,idx) partials GEMV_LOGITS writes
 
 void launch_argmax_partials(const float* blk_max, const uint32_t* blk_idx, int n, uint32_t* out, hipStream_t st);

@@ -85,12 +85,41 @@ GemvPlan plan_gemv(int N, int K, GemvEpi epi) {
 
 int gemv_num_tiles(int N, int K) { return plan_gemv(N, K, GEMV_LOGITS).grid; }
 
-// gemv_row_kernel where a wave's load group is a whole row of up to 3072 columns (0.6B: 2048 + 256 tokens 209 -> 182 ms, 19 + 12 sampled ones
-// 10.4 -> 9.1).  At 4096 columns the vector's registers cost a block per CU and an 8B launch streams for longer than it ramps: 208.7 -> 210.3 ms per
-// 64-token answer with it.  false = not such a shape, nothing launched.
+// The knobs of the block form are heard: it runs where one is set.
+bool gemv_row_on() {
+  static const bool on = [] {
+    for (const char* k : {"AHA_GEMV_GRID", "AHA_GEMV_GRID_R1", "AHA_GEMV_R", "AHA_GEMV_U"})
+      if (getenv(k)) return false;
+    const char* cached = getenv("AHA_GEMV_CACHED");
+    if (cached && atoi(cached) != 0) return false;
+    for (const char* k : {"AHA_GEMV_FAST", "AHA_GEMV_EVEN_GRID"}) {
+      const char* e = getenv(k);
+      if (e && atoi(e) == 0) return false;
+    }
+    return true;
+  }();
+  return on;
+}
+// gemv_row_kernel where a wave's load group is a whole row of 1024, 1536, 2048 or 3072 columns -- the widths of the 0.6B stacks, with two rows per wave
+// the first and third (0.6B: 2048 + 256 tokens 209 -> 182 ms, 19 + 12 sampled ones 10.4 -> 9.1); other widths have no instantiation and take the block
+// form.  At 4096 columns the vector's registers cost a block per CU and an 8B launch streams for longer than it ramps: 208.7 -> 210.3 ms per 64-token
+// answer with it.  The two matrices of GEMV_SILU_MUL have none at 3072 and, with two rows, at 2048: two buffers of that many loads leave two blocks per
+// CU.  -> load groups per row, 0: the block form
+int gemv_row_groups(int N, int K, GemvEpi epi, const GemvPlan& p) {
+  if (!gemv_row_on() || K % 512 != 0 || N < 1) return 0;
+  const int u = K / 512;
+  const bool two = epi == GEMV_SILU_MUL;
+  if (epi == GEMV_LOGITS) return 0;
+  if (p.R == 2) return u == 2 || (u == 4 && !two) ? u : 0;
+  if (p.R == 1) return (u >= 2 && u <= 4) || (u == 6 && !two) ? u : 0;
+  return 0;
+}
+int gemv_row_groups(int N, int K, GemvEpi epi) { return gemv_row_groups(N, K, epi, plan_gemv(N, K, epi)); }
+
+// false = not such a shape, nothing launched
 template <int EPI>
 static bool launch_gemv_row(const GemvArgs& a, const GemvPlan& p, hipStream_t st) {
-  if (a.K % 512 != 0 || a.cached || a.h_out != nullptr || p.R > 2 || a.N < 1) return false;
+  if (a.cached || a.h_out != nullptr) return false;
   auto go = [&](auto r, auto u) {
     constexpr int R = decltype(r)::value, U = decltype(u)::value;
     constexpr bool CAN_NORM = EPI == GEMV_STORE || EPI == GEMV_SILU_MUL || EPI == GEMV_PARTIAL_F32;
@@ -104,7 +133,7 @@ static bool launch_gemv_row(const GemvArgs& a, const GemvPlan& p, hipStream_t st
     return CAN_NORM;
   };
   using std::integral_constant;
-  const int u = a.K / 512;
+  const int u = gemv_row_groups(a.N, a.K, (GemvEpi)EPI, p);
   if (p.R == 2) {
     if (u == 2) return go(integral_constant<int, 2>{}, integral_constant<int, 2>{});
     if constexpr (EPI != GEMV_SILU_MUL)
@@ -114,7 +143,7 @@ static bool launch_gemv_row(const GemvArgs& a, const GemvPlan& p, hipStream_t st
   if (u == 2) return go(integral_constant<int, 1>{}, integral_constant<int, 2>{});
   if (u == 3) return go(integral_constant<int, 1>{}, integral_constant<int, 3>{});
   if (u == 4) return go(integral_constant<int, 1>{}, integral_constant<int, 4>{});
-  if constexpr (EPI != GEMV_SILU_MUL)   // (two matrices: two buffers of that many loads leave two blocks per CU)
+  if constexpr (EPI != GEMV_SILU_MUL)
     if (u == 6) return go(integral_constant<int, 1>{}, integral_constant<int, 6>{});
   return false;
 }

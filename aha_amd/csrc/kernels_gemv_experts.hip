@@ -240,7 +240,7 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_experts_down_kernel(GemvArg
 
 void launch_gemv_experts_up(const GemvArgs& a, const GemvLayerNorm& p, const GemvExperts& e, hipStream_t st) {
   const GemvPlan pl = plan_gemv(a.N, a.K, GEMV_SILU_MUL);
-  if (a.K == 1024 && e.experts <= 64 && pl.R == 1) {
+  if (a.K == 1024 && e.experts <= 64 && pl.R == 1 && gemv_row_on()) {
     const int nblk = gemv_row_grid(a.N, 1);
     hipLaunchKernelGGL(gemv_row_experts_up_kernel, dim3(nblk), dim3(GEMV_THREADS), 0, st, e.z, p.x, e.w_experts, e.w_shared, e.experts | e.top << 16, e.effp, a.N, nblk, a, p, e);
     return;
@@ -255,7 +255,7 @@ void launch_gemv_experts_up(const GemvArgs& a, const GemvLayerNorm& p, const Gem
 
 void launch_gemv_experts_down(const GemvArgs& a, const GemvExpertsDown& d, hipStream_t st) {
   const GemvPlan pl = plan_gemv(a.N, a.K, GEMV_AXPY_F32);
-  if (a.K == 3072 && pl.R == 1 && d.n_rows == a.N) {
+  if (a.K == 3072 && pl.R == 1 && d.n_rows == a.N && gemv_row_on()) {
     const int nblk = gemv_row_grid(a.N, 1);
     hipLaunchKernelGGL(gemv_row_experts_down_kernel, dim3(nblk), dim3(GEMV_THREADS), 0, st, a.x, d.sel, d.w_experts, d.w_shared, a.res_f32, d.top, d.effp, a.N, nblk, a);
     return;

@@ -131,7 +131,7 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_row_partsnorm_kernel(const 
 
 void launch_gemv_layernorm(const GemvArgs& a, const GemvLayerNorm& p, GemvEpi epi, hipStream_t st) {
   const GemvPlan pl = plan_gemv(a.N, a.K, epi);
-  if (a.K == 1024 && pl.R <= 2 && a.W2 == nullptr) {   // (gemv_row_body.h)
+  if (a.K == 1024 && pl.R <= 2 && a.W2 == nullptr && gemv_row_on()) {   // (gemv_row_body.h)
     auto row = [&](auto r) {
       constexpr int R = decltype(r)::value;
       const int nblk = gemv_row_grid(a.N, R);
@@ -158,7 +158,7 @@ void launch_gemv_layernorm(const GemvArgs& a, const GemvLayerNorm& p, GemvEpi ep
 
 void launch_gemv_partsnorm(const GemvArgs& a, const GemvPartsNorm& p, hipStream_t st) {
   const GemvPlan pl = plan_gemv(a.N, a.K, GEMV_AXPY_F32);
-  if (a.K == 2048 && p.n == a.K && pl.R == 1 && p.n == p.parts * 256) {
+  if (a.K == 2048 && p.n == a.K && pl.R == 1 && p.n == p.parts * 256 && gemv_row_on()) {
     hipLaunchKernelGGL(gemv_row_partsnorm_kernel<4>, dim3(gemv_row_grid(a.N, 1)), dim3(GEMV_THREADS), 0, st, p.g, p.ssq, p.w, a.W, a.res_f32, p.eps, p.part, a.N, gemv_row_grid(a.N, 1), a);
     return;
   }

@@ -451,6 +451,9 @@ int aha_hip_debug_few_rows_gemm(int32_t M, int32_t N, int32_t K, int32_t act, in
  * that every (tile, K tile) is covered exactly once for the BASELINE shapes. */
 int aha_hip_debug_streamk_plan(int32_t M, int32_t N, int32_t K, int32_t tile_n, int32_t workers, size_t workspace_bytes, int32_t* out,
                                int32_t cap, int32_t* off_out, int32_t* info7);
+/* Host only (no GPU): the 512-column loads per row of the short decode matvec (csrc/gemv_row_body.h) where the launcher takes it for a (N, K) bf16
+ * matrix, 0 where the block form runs; epi = 0 store, 1 + residual, 2 silu(gate) * up, 4 f32 store, 5 f32 residual (csrc/kernels.h GemvEpi). */
+int aha_hip_debug_gemv_row_groups(int32_t N, int32_t K, int32_t epi);
 /* Host only (no GPU): the experts that the decode matvec of up to 64 of them chooses for a row of router logits (csrc/expert_choice.h), the wave restated
  * lane by lane: sel, weight (top), largest first.  Lets the CPU tier pin the choice for logits that are not finite. */
 int aha_hip_debug_expert_choice(const float* z, int32_t experts, int32_t top, int32_t* sel, float* weight);

@@ -1,5 +1,6 @@
 """GPU microbenchmark of the weight-streaming matvec at the Qwen3-VL-8B decode shapes (rotating over enough distinct
-matrices to defeat the 256 MB Infinity Cache).  Knobs: AHA_GEMV_GRID / AHA_GEMV_R / AHA_GEMV_U env vars."""
+matrices to defeat the 256 MB Infinity Cache).  Knobs: AHA_GEMV_GRID / AHA_GEMV_R / AHA_GEMV_U env vars
+(with one of them set, rows of 1024 to 3072 columns run on the block form too)."""
 import os, sys, time
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 import torch

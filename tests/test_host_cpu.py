@@ -4,6 +4,8 @@ reference's."""
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -46,6 +48,21 @@ def test_no_gpu_is_a_loud_error_not_a_fallback(hip_lib):
     from aha_amd.model import HipContext
     with pytest.raises(AhaHipError):
         HipContext(0)
+
+
+GEMV_KNOBS = {"AHA_GEMV_FAST": "0", "AHA_GEMV_EVEN_GRID": "0", "AHA_GEMV_GRID": "512", "AHA_GEMV_GRID_R1": "512", "AHA_GEMV_R": "1", "AHA_GEMV_U": "2", "AHA_GEMV_CACHED": "1"}
+
+
+@pytest.mark.parametrize("knob", [None, *GEMV_KNOBS])
+def test_knobs_of_the_decode_matvec_reach_its_short_rows(hip_lib, knob):
+    """The short form takes rows of 1024 to 3072 columns, and leaves them to the block form that a set knob is for."""
+    shapes = [(4096, 1024, 0), (1024, 2048, 1), (3072, 1024, 2), (1024, 3072, 1), (2048, 1536, 4), (6144, 4096, 0), (1024, 2560, 0), (1024, 3072, 2), (151936, 1024, 3)]
+    code = f"from aha_amd import _lib; l = _lib.lib(); print([l.aha_hip_debug_gemv_row_groups(*s) for s in {shapes}])"
+    env = {k: v for k, v in os.environ.items() if k not in GEMV_KNOBS}
+    if knob:
+        env[knob] = GEMV_KNOBS[knob]
+    out = subprocess.run([sys.executable, "-c", code], env=env, cwd=ROOT, capture_output=True, text=True, check=True).stdout
+    assert eval(out.strip().splitlines()[-1]) == ([0] * len(shapes) if knob else [2, 4, 2, 6, 3, 0, 0, 0, 0])
 
 
 def test_product_code_never_imports_the_oracle():
