@@ -74,18 +74,20 @@ def decode_bytes_per_token(cfg, L):
 MFMA_PEAK_BF16_TFLOPS = 2500.0   # dense bf16 (MI355X_MICROARCH.md; AMD's headline 5 PF includes 2:1 sparsity)
 
 
-def prefill_flops(cfg, S, kv_offset=0, vit_segments=()):
+def prefill_flops(cfg, S, kv_offset=0, vit_segments=(), last_rows=None):
     """Algorithmic FLOPs of one prefill of S prompt tokens (2 per multiply-add), the decoder stack + the vision tower:
-      * text GEMMs: 2 S K N for qkv, o_proj, gate+up, down_proj of every layer; lm_head for ONE row (qwen3/model.rs:187: last position only);
+      * text GEMMs: 2 S K N for qkv, o_proj, gate+up, down_proj of every layer, with `last_rows` in the place of S behind the last layer's
+        attention (one GPU: only the row that is read, csrc/model.hip); lm_head for ONE row (qwen3/model.rs:187: last position only);
       * text attention, CAUSAL-counted: row i sees kv_offset + i + 1 keys, QK^T + P.V = 4 d per (query, key, head);
       * ViT (one entry of `vit_segments` per image / video frame group = its patch count n): the four GEMMs of each block over all
         patches, FULL attention inside a segment (4 n^2 D per block), the patch-embed GEMM and the mergers' two GEMMs each.
     Element-wise work (norms, rope, softmax, activations) is not counted."""
     t = cfg.text if hasattr(cfg, "text") else cfg
     H, I, L = t.hidden_size, t.intermediate_size, t.num_hidden_layers
-    gemm = 2.0 * S * H * (t.q_dim + 2 * t.kv_dim) + 2.0 * S * t.q_dim * H + 2.0 * S * H * 2 * I + 2.0 * S * I * H
+    qkv, behind = 2.0 * H * (t.q_dim + 2 * t.kv_dim), 2.0 * t.q_dim * H + 2.0 * H * 2 * I + 2.0 * I * H   # of a row
+    gemm = L * S * qkv + ((L - 1) * S + (S if last_rows is None else last_rows)) * behind
     attn = 4.0 * t.q_dim * (S * kv_offset + S * (S + 1) / 2.0)
-    out = {"text_gemm": L * gemm + 2.0 * t.vocab_size * H, "text_attention_causal": L * attn, "vit_gemm": 0.0, "vit_attention": 0.0}
+    out = {"text_gemm": gemm + 2.0 * t.vocab_size * H, "text_attention_causal": L * attn, "vit_gemm": 0.0, "vit_attention": 0.0}
     v = getattr(cfg, "vision", None)
     if v is not None and vit_segments:
         n = float(sum(vit_segments))
@@ -781,13 +783,13 @@ def main():
             segs += [int(g[1]) * int(g[2]) for g in np.asarray(data.image_grid_thw).reshape(-1, 3) for _ in range(int(g[0]))]
         if data is not None and getattr(data, "video_grid_thw", None) is not None:
             segs += [int(g[1]) * int(g[2]) for g in np.asarray(data.video_grid_thw).reshape(-1, 3) for _ in range(int(g[0]))]
-        pf = prefill_flops(cfg, len(ids), 0, segs if is_vl else ())
+        pf = prefill_flops(cfg, len(ids), 0, segs if is_vl else (), last_rows=1)
         ach = pf["total"] / t_prefill / 1e12
         roof_prefill = {"bound": "mfma", "achieved": round(ach, 1), "peak": MFMA_PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                         "frac": round(ach / MFMA_PEAK_BF16_TFLOPS, 4), "flops": {k: round(v / 1e12, 3) for k, v in pf.items()},
                         "flops_unit": "TFLOP per prefill", "seconds": round(t_prefill, 5),
                         "counting": "2 FLOP per multiply-add; text attention causal (row i: i + 1 keys), ViT attention full within an image; "
-                                    "lm_head for the last position only; element-wise work not counted; whole prefill wall clock (ViT + "
+                                    "behind the last layer's attention and in lm_head the last position only; element-wise work not counted; whole prefill wall clock (ViT + "
                                     "36 layers + lm_head + host-side position / page bookkeeping) in the denominator"}
         step_bytes = decode_bytes_per_token(cfg, kv_mid)
         line = {

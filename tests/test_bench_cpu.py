@@ -58,6 +58,10 @@ def test_prefill_flops_formula():
     assert abs(pf["text_attention_causal"] - 36 * 4.0 * t.q_dim * S * (S + 1) / 2) < 1e6
     assert abs(pf["vit_attention"] - 27 * 4.0 * v.hidden_size * n * n) < 1e6
     assert 21.0e12 < pf["text_gemm"] < 21.8e12 and 3.5e12 < pf["vit_gemm"] < 3.9e12 and 27.5e12 < pf["total"] < 28.3e12
+    # one row behind the last layer's attention, what one GPU computes: o_proj, gate, up and down of the other 1541 are not counted
+    one = bench.prefill_flops(cfg, S, 0, [n], last_rows=1)
+    assert abs(pf["total"] - one["total"] - 2.0 * (S - 1) * t.hidden_size * (t.q_dim + 3 * t.intermediate_size)) < 1e6
+    assert 27.0e12 < one["total"] < 27.6e12 and one["text_attention_causal"] == pf["text_attention_causal"]
     # text only: no ViT terms; a cache offset adds S * offset (query, key) pairs
     tx = bench.prefill_flops(cfg.text, 128)
     assert tx["vit_gemm"] == 0.0 and tx["vit_attention"] == 0.0
