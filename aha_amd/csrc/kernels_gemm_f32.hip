@@ -65,8 +65,9 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_f32_few_kernel(const f
 // this small so that a prompt of a few hundred rows still makes two to three blocks per CU: the f32 MFMA (32 cycles for 16 x 16 x 4) is the bound, idle
 // SIMDs are the loss.
 // 300 rows of the 0.6B widths: 87 us on average (64 x 64 tiles, one stage, through registers) -> 36 us.
-// A wave of the wider tile multiplies for 0.43 us per stage, so a launch of fewer blocks than CUs takes 0.43 us * K / 64 however few they are: below
-// 1.5 blocks per CU the tile is 16 rows.  The sums' order is the same.  300 rows, 1024 columns: K = 2048 33 -> 26 us, K = 3072 49 -> 39.
+// A wave of the wider tile multiplies for 0.43 us per stage, so a launch takes that times K / 64 however few blocks it has, and few blocks are spread over
+// the CUs better in halves: 16 rows below 736 blocks of 32.  Blocks of 32 rows: us with 32 / 16 rows, K = 2048: 160: 30.6 / 24.9, 320: 44.9 / 33.8,
+// 400: 45.1 / 33.8, 480: 45.2 / 42.6, 640: 60.2 / 55.3, 672: 60.8 / 55.9, 760 (nearly three for every CU): 60.6 / 62.7.  The sums' order is the same.
 constexpr int F_S = 3;
 constexpr int f_stage(int wm) { return (4 * wm + 8) * 1024; }
 template <int WM>
@@ -196,7 +197,7 @@ void launch_gemm_f32(const float* A, int64_t lda, const void* W, int64_t ldw, fl
   }
   if (M > 64) {
     const unsigned tn = (unsigned)((N + 63) / 64);
-    if ((int64_t)((M + 31) / 32) * tn * batch < 384) hipLaunchKernelGGL(gemm_f32_kernel<1>, dim3((unsigned)((M + 15) / 16), tn, (unsigned)batch), dim3(256), F_S * f_stage(1), st, a);
+    if ((int64_t)((M + 31) / 32) * tn * batch < 736) hipLaunchKernelGGL(gemm_f32_kernel<1>, dim3((unsigned)((M + 15) / 16), tn, (unsigned)batch), dim3(256), F_S * f_stage(1), st, a);
     else hipLaunchKernelGGL(gemm_f32_kernel<2>, dim3((unsigned)((M + 31) / 32), tn, (unsigned)batch), dim3(256), F_S * f_stage(2), st, a);
     return;
   }

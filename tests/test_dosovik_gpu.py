@@ -99,6 +99,7 @@ VARIANTS = {
     "large eps, alpha 1, embedding scale 1": ([layer(scale=0.4)] * 2, dict(eps=0.3, alpha=1.0, scale=1.0)),
     "rows of whole load groups": ([layer(heads=8, kv_heads=2, dim=64, vdim=64, ff=2048), layer(heads=16, kv_heads=4, dim=64, vdim=128, ff=1024, v_mix=False)], dict(width=1024)),
     "wide feed-forward of whole load groups": ([layer(heads=8, kv_heads=2, dim=64, vdim=64, ff=5120)], dict(width=1024)),
+    "feed-forward of whole rounds of 32 x 64 tiles": ([layer(heads=8, kv_heads=2, dim=64, vdim=64, ff=9600)], dict(width=1024)),
     "wide rows": ([layer(heads=4, kv_heads=2, ff=2600)], dict(width=2100)),
 }
 
