@@ -122,7 +122,8 @@ struct ExpertsDownPro {
 // i / effp, at most top (exact for i < 2^20: the nearest multiple is half a column away)
 __device__ __forceinline__ int choice_of(int i, float inv_effp, int top) { return min((int)(((float)i + 0.5f) * inv_effp), top); }
 
-// The row forms (gemv_row_body.h): up to 64 experts, one logit per lane; K = 1024 (up), 3072 (down).
+// The row forms (gemv_row_body.h) of the 0.6B stack's widths: up to 64 experts, one logit per lane; K = 1024 (up), 3072 (down, whatever the choices' and the
+// shared expert's parts of it).  Other widths have no instantiation and take the block form.
 struct RowExpertsUpPro : RowLayerNormPro<2> {
   static constexpr bool MAPPED = true;
   const float* z;

@@ -274,7 +274,7 @@ void launch_gemv_postnorm(const GemvArgs& a, const GemvPostNorm& p, GemvEpi epi,
 
 void launch_gemv_merge(const GemvArgs& a, const GemvMerge& p, hipStream_t st) {
   const GemvPlan pl = plan_gemv(a.N, a.K, GEMV_RESIDUAL);
-  if (a.K == 2048 && pl.R == 1 && gemv_row_on()) {   // (gemv_row_body.h)
+  if (a.K == 2048 && pl.R == 1 && gemv_row_on()) {   // (gemv_row_body.h; the one width that is instantiated)
     auto row = [&](auto ms) {
       hipLaunchKernelGGL((gemv_row_merge_kernel<4, decltype(ms)::value>), dim3(gemv_row_grid(a.N, 1)), dim3(GEMV_THREADS), 0, st, p.part_o, p.part_ml, a.W, a.residual, a.trace, a.N, p.nsplit, gemv_row_grid(a.N, 1), a);
     };

@@ -66,7 +66,7 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_partsnorm_kernel(GemvArgs a
   gemv_body<R, U, GEMV_AXPY_F32, false, FAST>(a, xs, (int)blockIdx.x, (int)gridDim.x, [] {}, pro);
 }
 
-// parts norm for K = n = 512 U in parts of 256 columns: their 16 sums of squares each are added up by the 16 lanes of a DPP row
+// parts norm for K = n = 512 U (instantiated: 2048) in parts of 256 columns: their 16 sums of squares each are added up by the 16 lanes of a DPP row
 template <int U>
 struct RowPartsNormPro {
   const float *g, *ssq;
@@ -131,7 +131,7 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_row_partsnorm_kernel(const 
 
 void launch_gemv_layernorm(const GemvArgs& a, const GemvLayerNorm& p, GemvEpi epi, hipStream_t st) {
   const GemvPlan pl = plan_gemv(a.N, a.K, epi);
-  if (a.K == 1024 && pl.R <= 2 && a.W2 == nullptr && gemv_row_on()) {   // (gemv_row_body.h)
+  if (a.K == 1024 && pl.R <= 2 && a.W2 == nullptr && gemv_row_on()) {   // (gemv_row_body.h; the one width that is instantiated)
     auto row = [&](auto r) {
       constexpr int R = decltype(r)::value;
       const int nblk = gemv_row_grid(a.N, R);
