@@ -1,8 +1,11 @@
-// Matrix products of the layer-list decoders' 32-bit mode: C[M,N] f32 = A[M,K] f32 . W[N,K]^T, W bf16 (widened exactly), on v_mfma_f32_16x16x4_f32,
-// optionally a batch of them (operands sa / sw / sc elements behind the first's).
-//   gemm_f32_few_kernel   up to 64 rows: bound by the weights' stream (skinny_body.h)
-//   gemm_f32_kernel       32 x 64 tiles behind an LDS-DMA ring: bound by the f32 MFMA
-//   gemm_f32_any_kernel   K or pitches that 16-byte pieces of 64-wide chunks do not divide
+// Matrix products of the layer-list decoders' 32-bit mode: C[M,N] f32 = A[M,K] f32 . W[N,K]^T, W bf16, optionally a batch of them (operands sa / sw / sc
+// elements behind the first's).
+//   gemm_f32_few_kernel   few rows: bound by the weights' stream (skinny_body.h)
+//   gemm_f32_kernel       tiles of 16, 32 or 64 rows x 64 columns behind an LDS-DMA ring
+//   gemm_f32_any_kernel   K or pitches that 16-byte pieces of 64-wide chunks do not divide, on v_mfma_f32_16x16x4_f32
+// The first two multiply on the bf16 units without loss: W is bf16, and an f32 is the sum of three bf16 (split_bf16).  On v_mfma_f32_16x16x4_f32, the bound
+// of both before, the same products took 5.3 times the matrix cycles, in more and shorter sums: error against 64 bits 5.7e-7 (K = 1024) and 1.0e-6 (3072) in
+// tiles, 2.1e-7 and 3.3e-7 in few rows; now 1.0 to 1.9e-7 and 1.6 to 3.4e-7, 1.0e-7 and 1.6e-7.
 #include <math.h>
 
 #include <algorithm>
@@ -27,8 +30,8 @@ struct GemmF32Args {
   int M, N, K;
 };
 
-// A decoding step's products had one 64 x 64 tile per 64 columns (64 blocks for 4096 x 1024, every k step a load's latency): 80 us on average at 2
-// rows of the 0.6B widths, 6.4 us here; its 32768-column head 21 us (67 MB: 3.1 TB/s).
+// 2 / 32 rows back to back (in brackets: f32 MFMA): 4096 x 1024 4.5 / 5.7 us (4.7 / 6.5), 1024 x 2048 5.1 / 7.6 (6.2 / 9.2), 1024 x 3072 6.2 / 10.2 (8.1 / 12.4),
+// 32768 x 1024 12.7 us (19.0): 5.3 TB/s of weights.
 template <int R8, int M8>
 __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_f32_few_kernel(const float* A, const bf16_t* W, int M, int N, int K, int64_t lda, int64_t ldw, GemmF32Args a) {
   // (what the first requests need: in scalar registers at the start, gemv_body.h)
@@ -60,47 +63,55 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_f32_few_kernel(const f
   }
 }
 
-// WM * 16 rows x 64 columns, 64-wide k stages; WM = 2: four waves of 16 x 32, WM = 1: of 16 x 16.  A stage is requests of 1 KB (rows of 64 k of A are
-// two lines: 4 WM of them; 8 of W), a quarter per wave; three stages keep two in flight under the one that multiplies, one barrier per stage.  The tile is
-// this small so that a prompt of a few hundred rows still makes two to three blocks per CU: the f32 MFMA (32 cycles for 16 x 16 x 4) is the bound, idle
-// SIMDs are the loss.
-// 300 rows of the 0.6B widths: 87 us on average (64 x 64 tiles, one stage, through registers) -> 36 us.
-// A wave of the wider tile multiplies for 0.43 us per stage, so a launch takes that times K / 64 however few blocks it has, and few blocks are spread over
-// the CUs better in halves: 16 rows below 736 blocks of 32.  Blocks of 32 rows: us with 32 / 16 rows, K = 2048: 160: 30.6 / 24.9, 320: 44.9 / 33.8,
-// 400: 45.1 / 33.8, 480: 45.2 / 42.6, 640: 60.2 / 55.3, 672: 60.8 / 55.9, 760 (nearly three for every CU): 60.6 / 62.7.  The sums' order is the same.
-constexpr int F_S = 3;
-constexpr int f_stage(int wm) { return (4 * wm + 8) * 1024; }
-template <int WM>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(GemmF32Args a) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];   // F_S x [A first halves | A second halves | W]
-  constexpr int STAGE = f_stage(WM), HALF = WM * 2048, NA = WM, NR = WM, LEFT = (F_S - 2) * (NA + 2);   // A requests per wave, 16-column groups per wave
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), G = lane >> 4, c = lane & 15, wm = WM == 2 ? wave >> 1 : 0, wn = WM == 2 ? wave & 1 : wave;
-  const int n0 = (int)blockIdx.y * 64, m0 = (int)blockIdx.x * (WM * 16);   // (consecutive blocks share the weights' tile)
+// WR * 16 rows x 64 columns, WR * WK waves of 16 x 64: WR side by side over the rows, WK over the 64-wide k chunks of a stage (their sums are joined at the
+// end).  A stage is requests of 1 KB: per chunk 4 WR of A (rows of 64 k of A are two lines) and 8 of W.  The fragments of a stage are read whole before the next
+// requests go out.
+// A wave's chunk is 88 instructions of splitting and 24 MFMAs, ~0.42 us, its stage's bytes ~0.35 us: with one wave per SIMD a launch takes their sum times the
+// chunks of its longest wave, however few blocks it has.  So the k chunks are dealt to WK waves where blocks are few; four chunks of 16 rows as long as one block
+// per CU does it, then 32 rows, of four chunks for one block per CU and of two for two, then 64 rows of one (launch_gemm_f32).  us (in brackets: the tiles of 16
+// or 32 rows on the f32 MFMA), 252 rows: 4096 x 1024 11.8 (26.2), 1024 x 2048 10.0 (19.3), 3072 x 1024 9.7 (20.2), 1024 x 3072 13.4 (28.1), 6176 x 1024 17.5 (48.4);
+// 66 rows: 7.5 (14.6), 9.1 (18.5), 6.6 (11.0), 11.8 (26.7), 10.5 (15.6); 1000 rows: 35 (93), 20 (48), 27.5 (71), 26.1 (75.6), 61 (144).
+// The other shapes at 252 rows, 16 rows x 4 chunks / 32 x 4 / 32 x 2 / 64 x 1: 4096 x 1024 22 / 15.3 / 11.8 / 12.0, 1024 x 2048 10.0 / 10.8 / 12.7 / 19.2.
+// Fragments a stage ahead in registers: no difference; 32 rows per wave: slower (a wave's chunk takes twice as long).
+constexpr int f_stage(int rows, int wk) { return (rows / 4 + 8) * wk * 1024; }
+template <int WR, int WK, int F_S>
+__global__ __launch_bounds__(WR * WK * 64) void gemm_f32_kernel(GemmF32Args a, int tiles_m) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];   // F_S x [A: chunks x halves x rows | W: chunks x 64 rows]
+  constexpr int ROWS = WR * 16, STAGE = f_stage(ROWS, WK), HALF = ROWS * 128, NA = ROWS / 4 * WK, QA = 4, NW = 8 / WR, LEFT = (F_S - 2) * (QA + NW);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), G = lane >> 4, c = lane & 15, wr = wave % WR, wk = wave / WR;
+  // the row tiles of a column tile stay on one XCD: its weights leave HBM once
+  const int xcd = (int)blockIdx.x & 7, local = (int)blockIdx.x >> 3, n0 = (local / tiles_m * 8 + xcd) * 64, m0 = local % tiles_m * ROWS;
+  if (n0 >= a.N) return;
   const float* A = a.A + blockIdx.z * a.sa;
   const bf16_t* W = a.W + blockIdx.z * a.sw;
-  const char *asrc[NA], *wsrc[2];   // requests wave * NA + j of A, wave * 2 + j of W
+  const int nc = a.K / 64, nk = (nc + WK - 1) / WK;
+  const char *asrc[QA], *wsrc[NW];   // requests wave * QA + j of A, wave * NW + j of W
 #pragma unroll
-  for (int j = 0; j < NA; ++j) {
-    const int q = wave * NA + j, ar = q % (2 * WM) * 8 + (lane >> 3);
-    asrc[j] = (const char*)(A + (int64_t)min(m0 + ar, a.M - 1) * a.lda) + q / (2 * WM) * 128 + skinny_piece(ar, lane);
+  for (int j = 0; j < QA; ++j) {
+    const int q = wave * QA + j, ar = q % (ROWS / 8) * 8 + (lane >> 3);
+    asrc[j] = (const char*)(A + (int64_t)min(m0 + ar, a.M - 1) * a.lda) + q % (ROWS / 4) / (ROWS / 8) * 128 + skinny_piece(ar, lane);
   }
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int wr = (wave * 2 + j) * 8 + (lane >> 3);
-    wsrc[j] = (const char*)(W + (int64_t)min(n0 + wr, a.N - 1) * a.ldw) + skinny_piece(wr, lane);
+  for (int j = 0; j < NW; ++j) {
+    const int wrow = (wave * NW + j) % 8 * 8 + (lane >> 3);
+    wsrc[j] = (const char*)(W + (int64_t)min(n0 + wrow, a.N - 1) * a.ldw) + skinny_piece(wrow, lane);
   }
-  const int nk = a.K / 64;
-  auto load = [&](int kt) {   // (past the end: the last stage again, never used)
-    const int k = min(kt, nk - 1) * 128;
+  auto load = [&](int kt) {   // (past the end: the last chunk again, never used)
     char* st = smem + kt % F_S * STAGE;
 #pragma unroll
-    for (int j = 0; j < NA; ++j) __builtin_amdgcn_global_load_lds((glb_ptr_t)(asrc[j] + 2 * k), (lds_ptr_t)(st + (wave * NA + j) * 1024), 16, 0, 0);
+    for (int j = 0; j < QA; ++j) {
+      const int q = wave * QA + j;
+      __builtin_amdgcn_global_load_lds((glb_ptr_t)(asrc[j] + min(kt * WK + q / (ROWS / 4), nc - 1) * 256), (lds_ptr_t)(st + q * 1024), 16, 0, 0);
+    }
 #pragma unroll
-    for (int j = 0; j < 2; ++j) __builtin_amdgcn_global_load_lds((glb_ptr_t)(wsrc[j] + k), (lds_ptr_t)(st + (4 * WM + wave * 2 + j) * 1024), 16, 0, 0);
+    for (int j = 0; j < NW; ++j) {
+      const int q = wave * NW + j;
+      __builtin_amdgcn_global_load_lds((glb_ptr_t)(wsrc[j] + min(kt * WK + q / 8, nc - 1) * 128), (lds_ptr_t)(st + (NA + q) * 1024), 16, 0, 0);
+    }
   };
-  f32x4_t acc[NR];
+  f32x4_t big[4], rest[4];
 #pragma unroll
-  for (int r = 0; r < NR; ++r) acc[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int r = 0; r < 4; ++r) big[r] = rest[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < F_S - 1; ++s) load(s);
   for (int kt = 0; kt < nk; ++kt) {
@@ -108,32 +119,55 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(GemmF32Args a) {
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    load(kt + F_S - 1);
-    const char* st = smem + kt % F_S * STAGE;
-    u32x4_t wf[2][NR];
-    f32x4_t af[2][2];
+    const char *sa = smem + kt % F_S * STAGE + wk * (ROWS / 4 * 1024), *sw = smem + kt % F_S * STAGE + (NA + wk * 8) * 1024;
+    f32x4_t x[2][2];
+    bf16x8_t wf[2][4];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
 #pragma unroll
-      for (int r = 0; r < NR; ++r) wf[h][r] = *reinterpret_cast<const u32x4_t*>(st + 2 * HALF + skinny_swz(wn * (NR * 16) + r * 16 + c, h * 4 + G));
+      for (int q = 0; q < 2; ++q) x[h][q] = *reinterpret_cast<const f32x4_t*>(sa + h * HALF + skinny_swz(wr * 16 + c, 2 * G + q));
 #pragma unroll
-      for (int q = 0; q < 2; ++q) af[h][q] = *reinterpret_cast<const f32x4_t*>(st + h * HALF + skinny_swz(wm * 16 + c, 2 * G + q));
+      for (int r = 0; r < 4; ++r) wf[h][r] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(sw + skinny_swz(r * 16 + c, h * 4 + G)));
     }
+    __builtin_amdgcn_sched_barrier(0);
+    load(kt + F_S - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    if (WK == 1 || kt * WK + wk < nc) {   // (K / 64 no multiple of WK: the last stage lacks a chunk)
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+      for (int h = 0; h < 2; ++h) {
+        const SplitBf16x8 p = split_bf16(x[h][0], x[h][1]);
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
+        for (int r = 0; r < 4; ++r) big[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[h][r], p.hi, big[r], 0, 0, 0);
 #pragma unroll
-        for (int r = 0; r < NR; ++r)
-          acc[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(j & 1 ? hi_bf(wf[h][r][j >> 1]) : lo_bf(wf[h][r][j >> 1]), af[h][j >> 2][j & 3], acc[r], 0, 0, 0);
+        for (int r = 0; r < 4; ++r) rest[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[h][r], p.lo, rest[r], 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) rest[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[h][r], p.mid, rest[r], 0, 0, 0);
+      }
+    }
     __builtin_amdgcn_sched_barrier(0);
   }
-  __builtin_amdgcn_s_waitcnt(0x0F70);   // (the surplus requests: LDS may belong to the next block)
-  const int m = m0 + wm * 16 + c;
+  __builtin_amdgcn_s_waitcnt(0x0F70);   // (the surplus requests: LDS may belong to the next block, or to the sums)
+  f32x4_t sum[4];
 #pragma unroll
-  for (int r = 0; r < NR; ++r) {
-    const int n = n0 + wn * (NR * 16) + r * 16 + G * 4;
-    if (m < a.M && n < a.N) *reinterpret_cast<f32x4_t*>(a.C + blockIdx.z * a.sc + (int64_t)m * a.ldc + n) = acc[r];
+  for (int r = 0; r < 4; ++r) sum[r] = split_sum(big[r], rest[r]);
+  if constexpr (WK > 1) {   // wave wk = 0 of a row group adds the others' sums in their order
+    __syncthreads();
+    auto red = reinterpret_cast<f32x4_t(*)[4][64]>(smem);
+    if (wk > 0)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[wave - WR][r][lane] = sum[r];
+    __syncthreads();
+    if (wk > 0) return;
+#pragma unroll
+    for (int w = 1; w < WK; ++w)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sum[r] += red[(w - 1) * WR + wr][r][lane];
+  }
+  const int m = m0 + wr * 16 + c;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int n = n0 + r * 16 + G * 4;
+    if (m < a.M && n < a.N) *reinterpret_cast<f32x4_t*>(a.C + blockIdx.z * a.sc + (int64_t)m * a.ldc + n) = sum[r];
   }
 }
 
@@ -195,10 +229,23 @@ void launch_gemm_f32(const float* A, int64_t lda, const void* W, int64_t ldw, fl
                        ldw, C, ldc, M, N, K, sa, sw, sc);
     return;
   }
-  if (M > 64) {
-    const unsigned tn = (unsigned)((N + 63) / 64);
-    if ((int64_t)((M + 31) / 32) * tn * batch < 736) hipLaunchKernelGGL(gemm_f32_kernel<1>, dim3((unsigned)((M + 15) / 16), tn, (unsigned)batch), dim3(256), F_S * f_stage(1), st, a);
-    else hipLaunchKernelGGL(gemm_f32_kernel<2>, dim3((unsigned)((M + 31) / 32), tn, (unsigned)batch), dim3(256), F_S * f_stage(2), st, a);
+  using std::integral_constant;
+  // the few-row form: 48 weight rows per block where they still make two blocks per CU (the head), up to 16 rows
+  // (32768 x 1024 at 32 rows: 23 us, in tiles 15.4); else 16.  From 33 rows on the tiles are ahead (64 rows, 4096 x 1024: 9.7 / 7.2, 1024 x 3072: 17.7 / 12.4)
+  const bool wide = (int64_t)((N + 47) / 48) * batch >= 512;
+  if (M > 32 || (M > 16 && wide)) {
+    auto tiles = [&](auto wr, auto wk, auto stages) {
+      constexpr int WR = decltype(wr)::value, WK = decltype(wk)::value, S = decltype(stages)::value, lds = S * f_stage(WR * 16, WK);
+      auto k = gemm_f32_kernel<WR, WK, S>;
+      if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+      const int tm = (M + WR * 16 - 1) / (WR * 16), tn = ((N + 63) / 64 + 7) / 8 * 8;
+      hipLaunchKernelGGL(k, dim3((unsigned)(tm * tn), 1, (unsigned)batch), dim3(WR * WK * 64), lds, st, a, tm);
+    };
+    const int64_t cols = (int64_t)((N + 63) / 64) * batch, b16 = (M + 15) / 16 * cols, b32 = (M + 31) / 32 * cols;   // (kernel's comment)
+    if (b16 <= 256) tiles(integral_constant<int, 1>{}, integral_constant<int, 4>{}, integral_constant<int, 3>{});
+    else if (b32 <= 256) tiles(integral_constant<int, 2>{}, integral_constant<int, 4>{}, integral_constant<int, 2>{});
+    else if (b32 <= 512) tiles(integral_constant<int, 2>{}, integral_constant<int, 2>{}, integral_constant<int, 2>{});
+    else tiles(integral_constant<int, 4>{}, integral_constant<int, 1>{}, integral_constant<int, 3>{});
     return;
   }
   auto go = [&](auto r8, auto m8) {
@@ -207,13 +254,9 @@ void launch_gemm_f32(const float* A, int64_t lda, const void* W, int64_t ldw, fl
     hipLaunchKernelGGL((gemm_f32_few_kernel<R8, M8>), dim3((unsigned)((N + R8 * 8 - 1) / (R8 * 8)), (unsigned)batch), dim3(SKINNY_WAVES * 64), lds, st, a.A,
                        a.W, a.M, a.N, a.K, a.lda, a.ldw, a);
   };
-  using std::integral_constant;
-  // 48 weight rows per block where they still make two blocks per CU (the head); f32 rows take twice the LDS, so more than 32 of them leave room for 16
-  const bool wide = (int64_t)((N + 47) / 48) * batch >= 512;
   if (M <= 8) wide ? go(integral_constant<int, 6>{}, integral_constant<int, 1>{}) : go(integral_constant<int, 2>{}, integral_constant<int, 1>{});
   else if (M <= 16) wide ? go(integral_constant<int, 6>{}, integral_constant<int, 2>{}) : go(integral_constant<int, 2>{}, integral_constant<int, 2>{});
-  else if (M <= 32) wide ? go(integral_constant<int, 6>{}, integral_constant<int, 4>{}) : go(integral_constant<int, 2>{}, integral_constant<int, 4>{});
-  else go(integral_constant<int, 2>{}, integral_constant<int, 8>{});
+  else go(integral_constant<int, 2>{}, integral_constant<int, 4>{});
 }
 
 }  // namespace aha

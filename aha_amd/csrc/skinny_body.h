@@ -37,9 +37,36 @@ __device__ __forceinline__ int skinny_swz(int row, int slot) { return row * 128 
 // the byte offset inside its 128-byte line that lane `lane` of a request fetches (a request: eight rows, eight lanes each)
 __device__ __forceinline__ int skinny_piece(int local_row, int lane) { return ((lane & 7) ^ ((local_row >> 1) & 7)) * 16; }
 
+// A float as the sum of three bf16 (its 24 significant bits cut 8 / 8 / 8: exact unless the parts fall below bf16's range, 2^-133), eight floats at a time in the
+// order of an MFMA operand.  With weights that are bf16 themselves all three products are exact and nothing is left out, so a product on the bf16 units has
+// an f32 unit's error (the sums are f32) at three sixteenths of its matrix cycles.
+struct SplitBf16x8 { bf16x8_t hi, mid, lo; };
+__device__ __forceinline__ SplitBf16x8 split_bf16(const f32x4_t& x0, const f32x4_t& x1) {
+  u32x4_t p[3];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float a = i < 2 ? x0[2 * i] : x1[2 * i - 4], b = i < 2 ? x0[2 * i + 1] : x1[2 * i - 3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const unsigned ua = __builtin_bit_cast(unsigned, a), ub = __builtin_bit_cast(unsigned, b);
+      p[k][i] = __builtin_amdgcn_perm(ub, ua, 0x07060302u);   // the upper halves
+      a -= __builtin_bit_cast(float, ua & 0xffff0000u);
+      b -= __builtin_bit_cast(float, ub & 0xffff0000u);
+    }
+  }
+  return {__builtin_bit_cast(bf16x8_t, p[0]), __builtin_bit_cast(bf16x8_t, p[1]), __builtin_bit_cast(bf16x8_t, p[2])};
+}
+// the upper parts' sums and the others'.  An infinity's rest is NaN (inf - inf), so where the upper parts' sum is not finite it is the result, as it would
+// be without the split
+__device__ __forceinline__ f32x4_t split_sum(const f32x4_t& big, const f32x4_t& rest) {
+  f32x4_t s;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) s[i] = fabsf(big[i]) < INFINITY ? big[i] + rest[i] : big[i];
+  return s;
+}
+
 // src[r]: where this lane's piece of request r starts at k = 0 -- R8 weight groups (bf16), then M8 activation groups (bf16); F32: activations are f32,
-// a row's 64 k are two requests, the first halves of all groups before the second halves.  The 32-bit form multiplies on
-// v_mfma_f32_16x16x4_f32 (weights widened exactly): in step (h, j) lane group G feeds k = (h * 4 + G) * 8 + j of both operands.
+// a row's 64 k are two requests, the first halves of all groups before the second halves, and the activations' parts (split_bf16) multiply in turn.
 // On return the waves' sums of the 16 x 16 fragments (weight fragment r, activation fragment m) lie in LDS and every wave may read them
 // (skinny_total).
 template <int R8, int M8, bool F32 = false, bool DEEP = false>
@@ -51,7 +78,7 @@ __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R
   static_assert(LEFT < 64, "vmcnt has six bits");
   const int G = lane >> 4, c = lane & 15;
   char* ring = smem + wave * (S * PER * 1024);
-  f32x4_t acc[2][NF][MT];   // the two halves of a chunk in chains of their own: half the dependent steps, half the roundings in a row
+  f32x4_t acc[2][NF][MT];   // the two halves of a chunk (F32: the upper parts and the others) in chains of their own: half the dependent steps, half the roundings in a row
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -85,13 +112,15 @@ __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
+        for (int m = 0; m < MT; ++m) {
+          const SplitBf16x8 x = split_bf16(af[h][m][0], af[h][m][1]);
 #pragma unroll
-          for (int r = 0; r < NF; ++r) {
-            const float w = j & 1 ? hi_bf(wf[h][r][j >> 1]) : lo_bf(wf[h][r][j >> 1]);
+          for (int r = 0; r < NF; ++r) acc[0][r][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[h][r]), x.hi, acc[0][r][m], 0, 0, 0);
 #pragma unroll
-            for (int m = 0; m < MT; ++m) acc[h][r][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, af[h][m][j >> 2][j & 3], acc[h][r][m], 0, 0, 0);
-          }
+          for (int r = 0; r < NF; ++r) acc[1][r][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[h][r]), x.lo, acc[1][r][m], 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < NF; ++r) acc[1][r][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[h][r]), x.mid, acc[1][r][m], 0, 0, 0);
+        }
     } else {
       bf16x8_t af[2][MT];
 #pragma unroll
@@ -143,7 +172,7 @@ __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R
 #pragma unroll
   for (int r = 0; r < NF; ++r)
 #pragma unroll
-    for (int m = 0; m < MT; ++m) red[wave][r * MT + m][lane] = acc[0][r][m] + acc[1][r][m];
+    for (int m = 0; m < MT; ++m) red[wave][r * MT + m][lane] = F32 ? split_sum(acc[0][r][m], acc[1][r][m]) : acc[0][r][m] + acc[1][r][m];
   __syncthreads();
 }
 

@@ -139,6 +139,19 @@ def test_32_bit_heads_of_whole_pieces(ctx, heads, kv_heads, dim, chunk, rope_dim
         assert err(all_logits(m, ids, [1, 130, 63] + [1] * 17), want) <= TOL["float32"]
 
 
+@pytest.mark.parametrize("rows,ff,vocab", [(8, 2624, 24600), (16, 2624, 322), (20, 2624, 24600), (32, 2624, 322), (33, 2624, 322), (65, 2624, 322), (97, 2624, 322),
+                                           (150, 2624, 322), (300, 2624, 322), (500, 2624, 322), (257, 4160, 322)])
+def test_32_bit_products_of_every_tile(ctx, rows, ff, vocab):
+    """gemm_f32_kernel and gemm_f32_few_kernel: every tile and row count that launch_gemm_f32 chooses between, K of five chunks (no multiple of the chunks of a
+    stage), columns that are no multiple of the eight column tiles that the XCDs take in turn; against 64 bits."""
+    cfg = config([layer(heads=4, kv_heads=2, dim=64, vdim=64, chunk=600, rope_dims=64, ff=ff)], width=320, vocab=vocab)
+    w = dosovik_weights(cfg, seed=11)
+    ids = tokens(rows, vocab, 12)
+    want = reference(cfg, w, ids)
+    with Model(ctx, cfg, w) as m:
+        assert err(all_logits(m, ids), want) <= TOL["float32"]
+
+
 @pytest.mark.parametrize("dim", [64, 128])
 def test_32_bit_rows_do_not_see_a_later_row_that_is_not_finite(ctx, dim):
     cfg = config([layer(heads=8, kv_heads=4, dim=dim, vdim=dim, chunk=100, rope_dims=dim)] * 2)
