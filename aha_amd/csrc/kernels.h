@@ -223,6 +223,7 @@ struct GemmArgs {
                                  // persistent kernel, kernels_gemm_sk.hip; every launch leaves them zero again)
   int tile_group = 8;            // band width of the grouped tile order inside an XCD's run (kernels_gemm.hip tile_of_block); 0 = plain
   int few_rows = 1;              // the few-row kernel (kernels_gemm_skinny.hip): 0 never, 1 where it is expected to be faster, 2 wherever it can
+  int few_rows_spread = 1;       // ... whose blocks start at different k (skinny_first); 0: all at k = 0, so that column blocks of a projection sum as the whole does
   int partial_rows = 1;          // ACT_PARTIAL_F32 on the four-wave kernel: f32 sums stored in row order through LDS (0: fragment order; A/B)
   // Row groups (launch_gemm_grouped; tensor-parallel prefill: the staging layout of the chunked all-gather, csrc/model.hip
   // norm_gather_gemm): `groups` row segments of M rows each share W.  Segment g reads A rows [g * a_gstride, + M) and writes C rows

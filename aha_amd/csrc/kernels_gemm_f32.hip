@@ -56,7 +56,7 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_f32_few_kernel(const f
     const int local = r % M8 * 8 + (lane >> 3);
     src[R8 + r] = (const char*)(a.A + (blockIdx.y > 0 ? blockIdx.y * a.sa : 0) + (int64_t)min(local, a.M - 1) * a.lda) + r / M8 * 128 + skinny_piece(local, lane);
   }
-  skinny_sums<R8, M8, true>(src, a.K / 64, smem, wave, lane);
+  skinny_sums<R8, M8, true>(src, a.K / 64, skinny_first(n0, a.K / 64), smem, wave, lane);
   for (int i = wave; i < (R8 / 2) * MT; i += SKINNY_WAVES) {
     const int f = i / MT, m = (i - f * MT) * 16 + c, n = n0 + f * 16 + G * 4;
     if (m < a.M && n < a.N) *reinterpret_cast<f32x4_t*>(a.C + blockIdx.y * a.sc + (int64_t)m * a.ldc + n) = skinny_total<R8, M8>(smem, i, lane);

@@ -10,9 +10,11 @@
 // Rows past M, N repeat the last one, lanes of a fragment that no row backs another row; what they give is not stored: an MFMA's output rows and columns
 // do not mix.
 //
+// Up to 64 rows blocks start at different k (skinny_first; row tiles of more rows: no difference, and they keep the common start).
+//
 // Measured on MI355X, back to back from HBM, 8 rows (in brackets: the split-K ring kernel + its reduce pass it replaces, inside a batched step):
-//   6144 x 4096 10.4 us (4.8 TB/s), 4096 x 4096 8.0, 12288 x 4096 18.5 (5.4), 4096 x 12288 17.7 (5.7), 24576 x 4096 32.8 (6.1)
-//   [18.1 + 4.6 us on average over the first four]; 32 rows: 11.9, 9.7, 19.3, 25.5, 34.9; 64 rows: 15.7, 13.1, 23.2, 35.1, 45.0
+//   6144 x 4096 9.9 us (5.1 TB/s), 4096 x 4096 7.2, 12288 x 4096 17.0 (5.9), 4096 x 12288 16.9 (6.0), 24576 x 4096 31.4 (6.4)
+//   [18.1 + 4.6 us on average over the first four]; 32 rows: 11.8, 9.6, 18.1, 25.1, 33.0; 64 rows: 15.7, 13.1, 22.4, 35.3, 43.8
 //   64-row tiles, 96 / 128 rows (tiled kernels with their reduce pass): 4096 x 1024 6.2 / 6.4 us (10.7 / 10.7), 6144 x 1024 8.1 / 8.3 (12.1 / 12.9),
 //   1024 x 2048 6.6 / 7.1 (11.3 / 12.1), 1024 x 3072 8.7 / 9.7 (12.3 / 13.2); a 0.6B prompt of 96 / 128 / 180 / 250 tokens 1.66 / 1.67 / 1.95 / 2.03 ms
 //   (1.97 / 2.06 / 2.07 / 2.14), of 300 2.14 (2.09): 256 rows at most.  The 8B shapes stay on the tiles:
@@ -51,7 +53,7 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const vo
       src[r] = (const char*)a.W + (int64_t)min((int)blockIdx.x * (R8 * 8) + local, a.N - 1) * a.ldw * 2 + piece;
     }
   }
-  skinny_sums<R8, M8, false, DEEP>(src, a.K / 64, gemm_smem, wave, lane);
+  skinny_sums<R8, M8, false, DEEP>(src, a.K / 64, a.few_rows_spread && a.M <= 64 ? skinny_first((int)blockIdx.x * (R8 * 8), a.K / 64) : 0, gemm_smem, wave, lane);
   for (int i = wave; i < NF * MT; i += SKINNY_WAVES) {
     const int r = i / MT, m = (int)blockIdx.y * 64 + (i - r * MT) * 16 + c;
     if (m >= a.M) continue;
@@ -110,10 +112,10 @@ int gemm_skinny_rounds(const GemmArgs& a, int r8) { return ((a.N + r8 * 8 - 1) /
 // More rounds, up to 64 rows (4096 x 1024, 180 rows, 384 blocks: 12.0 us against 10.9 of the tiles): a CU requests at most 60 bytes of weights per ns and
 // the chip delivers at most 8.2 TB/s (32 rows per block that lie whole 256 KB apart: 1.34 times as long, their requests meet in the same channels),
 // rounded where the two meet; A's rows at 96 bytes per ns and CU, the last row's repetitions for nothing; a block's first requests and the joined sums
-// show where no neighbour on the CU covers them.  Fitted to 23 shapes (512 x 4096 to 151936 x 4096) at 1 to 64 rows with every R8 before the rings asked
-// for nothing past the end; since then 12 % dear on average in several rounds (mostly short K), and a width chosen with it is 1.5 % behind the best on average:
-// at most 4 % but for 32 weight rows per block that lie 256 KB apart in ONE round, where it knows nothing of their channels (8192 x 4096, 8 rows: 18.2 us, 13.0
-// with 48), 16384 x 4096 at 16 rows (27.0, 23.8 with 24) and 12288 x 4096 at 8 (18.5, 17.4 with 24).
+// show where no neighbour on the CU covers them.  Fitted to 23 shapes (512 x 4096 to 151936 x 4096) at 1 to 64 rows with every R8, before the blocks started
+// at different k; it is 7 % dear on average since, and 32 rows 256 KB apart are only 10 % slower than others.  The width chosen with it is at most 5 % behind the
+// best of the four at 20 shapes (1024 x 2048 to 151936 x 1024) with 3 to 64 rows, but for 16384 x 4096 at 16 and more (26.2 us, 21.7 with 32 weight rows), 6208 x
+// 4096 at 8 (10.9, 9.9 with 32) and 32768 x 1024 at 3 (12.8, 11.6 with 16); with 1.1 for 1.34 48 rows of 16384 x 4096 leave the tiles.
 // The price of one round times their number said 41 us with 32 rows per block for 32768 x 4096 and 8 rows (57.7; 42.6 with 48) and 76 us for
 // 151936 x 1024 and 64 rows (96.6; the tiles 73).
 double gemm_skinny_plan(const GemmArgs& a, int* r8_out) {

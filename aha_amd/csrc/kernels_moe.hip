@@ -233,7 +233,7 @@ __device__ __forceinline__ void moe_few_body(const MoeGemmArgs& a, const MoeRout
       src[q] = W + (int64_t)min(n_blk * (R8 * 8) + local, a.n - 1) * a.k * 2 + piece;
     }
   }
-  skinny_sums<R8, M8>(src, a.k / 64, smem, wave, lane);
+  skinny_sums<R8, M8>(src, a.k / 64, skinny_first(n_blk * (R8 * 8), a.k / 64), smem, wave, lane);
   for (int i = wave; i < (R8 / 2) * MT; i += SKINNY_WAVES) {
     const int f = i / MT, row = (i - f * MT) * 16 + c;
     if (row >= ns) continue;

@@ -1066,6 +1066,7 @@ static int gemm_row_parallel(aha_model* m, GemmArgs g, int rows_per_rank = 0) {
     return AHA_OK;
   }
   void* xres = g.C;
+  g.few_rows_spread = 0;   // (cut into column blocks or whole, the same sums)
   const int nch = rows_per_rank > 0 ? tp_overlap_chunks(m, g) : 1;
   if (nch > 1) {
     const int N = g.N, Nc = N / nch;

@@ -37,6 +37,15 @@ __device__ __forceinline__ int skinny_swz(int row, int slot) { return row * 128 
 // the byte offset inside its 128-byte line that lane `lane` of a request fetches (a request: eight rows, eight lanes each)
 __device__ __forceinline__ int skinny_piece(int local_row, int lane) { return ((lane & 7) ^ ((local_row >> 1) & 7)) * 16; }
 
+// Where a block starts in K.  All blocks stream at one pace, so from a common start their requests at any moment lie in one narrow band of columns of all
+// weight rows -- one value of the address bits below the row pitch, a few of the memory's channels.  The blocks of 96 weight rows (whole blocks of 16, 24, 32
+// and 48: an element's sum has the same order for every R8 and M8) start four chunks behind their neighbours: 8 rows, 12288 x 4096 17.5 -> 16.4 us (6.1 TB/s),
+// 4096 x 4096 8.0 -> 7.0, 4096 x 12288 17.7 -> 16.6, 6144 x 4096 10.6 -> 9.8; 32 rows, 4096 x 8192 17.8 -> 15.9, 24576 x 4096 35.0 -> 32.7; 48 weight rows, 5 % in
+// the mean of 14 shapes.  One or nine chunks behind: 2 and 0 %.  K < 2048: no difference.
+__device__ __forceinline__ int skinny_first(int weight_row, int nc) {
+  return nc < 32 ? 0 : weight_row / 96 * 4 & ((1 << (31 - __builtin_clz(nc))) - 1);   // (below the largest power of two in nc)
+}
+
 // A float as the sum of three bf16 (its 24 significant bits cut 8 / 8 / 8: exact unless the parts fall below bf16's range, 2^-133), eight floats at a time in the
 // order of an MFMA operand.  With weights that are bf16 themselves all three products are exact and nothing is left out, so a product on the bf16 units has
 // an f32 unit's error (the sums are f32) at three sixteenths of its matrix cycles.
@@ -67,10 +76,11 @@ __device__ __forceinline__ f32x4_t split_sum(const f32x4_t& big, const f32x4_t& 
 
 // src[r]: where this lane's piece of request r starts at k = 0 -- R8 weight groups (bf16), then M8 activation groups (bf16); F32: activations are f32,
 // a row's 64 k are two requests, the first halves of all groups before the second halves, and the activations' parts (split_bf16) multiply in turn.
+// nc: 64-wide k chunks, first: the chunk that wave 0 starts at (skinny_first), wrapping round behind the last.
 // On return the waves' sums of the 16 x 16 fragments (weight fragment r, activation fragment m) lie in LDS and every wave may read them
 // (skinny_total).
 template <int R8, int M8, bool F32 = false, bool DEEP = false>
-__device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R8, M8, F32)], int nc, char* smem, int wave, int lane) {
+__device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R8, M8, F32)], int nc, int first, char* smem, int wave, int lane) {
   typedef __attribute__((address_space(3))) void* lds_t;
   typedef const __attribute__((address_space(1))) void* glb_t;
   constexpr int NF = (R8 + 1) / 2, MT = (M8 + 1) / 2, PER = skinny_requests(R8, M8, F32), S = skinny_stages(PER, DEEP);
@@ -86,7 +96,8 @@ __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R
 #pragma unroll
       for (int m = 0; m < MT; ++m) acc[h][r][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   auto load = [&](int u, int ch) {
-    const int k = ch * 128, ka = F32 ? 2 * k : k;
+    ch += first;
+    const int k = (ch < nc ? ch : ch - nc) * 128, ka = F32 ? 2 * k : k;
 #pragma unroll
     for (int r = 0; r < R8; ++r) __builtin_amdgcn_global_load_lds((glb_t)(src[r] + k), (lds_t)(ring + (u * PER + r) * 1024), 16, 0, 2);   // weights: non-temporal
 #pragma unroll
