@@ -8,6 +8,8 @@ namespace aha {
 constexpr int ATTN_DECODE_NW = 4;  // waves (= KV units) per workgroup
 constexpr int ATTN_DECODE_FUSED_LDS = 16 * 128 * 2 + 128 * 2 + 128 * 2 + ATTN_DECODE_NW * 128 * 16 * 4 + (2 * ATTN_DECODE_NW + 1) * 16 * 4;  // bytes
 
+constexpr int ATTN_DEFER_LDS(int group) { return 16 * 128 * 2 + 2 * 128 * 2 + ATTN_DECODE_NW * 128 * group * 4 + (2 * ATTN_DECODE_NW + 1) * 16 * 4; }
+
 // ---- decode, fused: q/k RMSNorm + (M-)RoPE + KV append + split-KV attention + in-block merge --------------------
 // One launch replaces qknorm_rope_kernel + attn_decode_kernel + the combine: every block redoes the (tiny) norm/rope of
 // its kv head's g query heads and of the new key in LDS (QKNormAttention::forward, modules.rs:538-557), block (kvhd, 0)
@@ -28,9 +30,12 @@ constexpr int ATTN_DECODE_FUSED_LDS = 16 * 128 * 2 + 128 * 2 + 128 * 2 + ATTN_DE
 // DEFER: the blocks leave their partials to the o_proj matvec, whose prologue merges up to eight of them (kernels_gemv_fused.hip MergePro): the kernel
 // boundary orders the plain stores, and the publish -> acknowledge -> arrive -> re-read chain of the last-block merge (1.9 + 0.7 + 2.3 of 9.7 us at
 // 1536 positions) is gone.
-template <int NW, bool DEFER>
+//
+// OUT (DEFER, one split): the output goes to o_lds as f32 (group x 128, rounded to bf16) instead of a.o; `append`: this block appends; after_issue() runs
+// once the first pages have been requested.
+template <int NW, bool DEFER, bool OUT = false, class AfterIssue>
 __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs& a, char* smem, const int kvhd, const int split,
-                                                       const int nsplit) {
+                                                       const int nsplit, float* o_lds, const bool append, AfterIssue&& after_issue) {
   constexpr int NT = NW * 64;
   bf16_t* qs = reinterpret_cast<bf16_t*>(smem);                 // [16][128]
   bf16_t* ksn = qs + 16 * 128;                                  // [128]
@@ -146,6 +151,7 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
     load_v(b0, page < npages);
     __builtin_amdgcn_sched_barrier(0);
   }
+  after_issue();
 
   // ---- prologue: norm + rope of the g q heads and the k head; v raw ------------------------------------------------
   {
@@ -172,7 +178,7 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
   }
   __syncthreads();
   stamp(1);
-  if (split == 0) {  // append (k roped, v raw) for the following steps
+  if (append) {  // append (k roped, v raw) for the following steps
     // global address space spelled out: a flat store here would make every later wait in the kernel a vmcnt(0)
     typedef __attribute__((address_space(1))) bf16_t* gbf_t;
     const int pg = slot_new / KV_PAGE_TOKENS, t = slot_new % KV_PAGE_TOKENS;
@@ -298,6 +304,10 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
     const int head = kvhd * g + q;
     if (single) {  // the whole cache went through this block: normalise and write the attention output tensor (bf16)
       const float inv = 1.0f / ls;
+      if constexpr (OUT) {
+        *reinterpret_cast<float4*>(o_lds + q * 128 + d0) = make_float4(rbf(acc[0] * inv), rbf(acc[1] * inv), rbf(acc[2] * inv), rbf(acc[3] * inv));
+        continue;
+      }
       uint2 w2;
       w2.x = pack_bf(acc[0] * inv, acc[1] * inv);
       w2.y = pack_bf(acc[2] * inv, acc[3] * inv);
@@ -408,6 +418,11 @@ __device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs
   }
   stamp(5);
   return true;
+}
+
+template <int NW, bool DEFER>
+__device__ __forceinline__ bool attn_decode_fused_body(const AttnDecodeFusedArgs& a, char* smem, const int kvhd, const int split, const int nsplit) {
+  return attn_decode_fused_body<NW, DEFER>(a, smem, kvhd, split, nsplit, nullptr, split == 0, [] {});
 }
 
 }  // namespace aha

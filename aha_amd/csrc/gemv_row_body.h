@@ -59,6 +59,58 @@ struct RowNormPro {
   }
 };
 
+// h = bf16(RMSNorm(xn) * norm_w), xn = x + bf16(the sum of P slices of o_proj's f32 sums) (oproj_slices.h); xn is what the layer continues with: block 0
+// writes it to x_out, another vector than x, which other blocks still read.  U = 2.  The block reads the slices once, a wave a quarter of the columns, and
+// shares xn through LDS: every wave for itself would be 4 P KB more per wave.
+template <int P>
+struct RowSlicesPro {
+  static constexpr int K = 1024;
+  const bf16_t *x, *w;
+  const float* parts;   // (P, K)
+  bf16_t* x_out;
+  float eps;
+  int bid;
+  float* xs;   // LDS, K + 4 floats
+  uint2 xr;
+  float4 pr[P];
+  u32x4_t nr[2];
+  __device__ __forceinline__ void request() {
+    const int lane = threadIdx.x & 63, k = threadIdx.x * 4;
+    xr = *reinterpret_cast<const uint2*>(x + k);
+#pragma unroll
+    for (int p = 0; p < P; ++p) pr[p] = *reinterpret_cast<const float4*>(parts + p * K + k);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) nr[u] = ld16(w + u * 512 + lane * 8);
+  }
+  __device__ __forceinline__ void make(float (&h)[2][8]) {
+    const int lane = threadIdx.x & 63, k = threadIdx.x * 4;
+    float4 s = pr[0];
+#pragma unroll
+    for (int p = 1; p < P; ++p) { s.x += pr[p].x; s.y += pr[p].y; s.z += pr[p].z; s.w += pr[p].w; }
+    uint2 o;
+    o.x = pack_bf(lo_bf(xr.x) + rbf(s.x), hi_bf(xr.x) + rbf(s.y));
+    o.y = pack_bf(lo_bf(xr.y) + rbf(s.z), hi_bf(xr.y) + rbf(s.w));
+    const float4 v = make_float4(lo_bf(o.x), hi_bf(o.x), lo_bf(o.y), hi_bf(o.y));
+    *reinterpret_cast<float4*>(xs + xs_index(k)) = v;
+    const float ss = wave_sum((v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w));
+    if (lane == 0) xs[K + (threadIdx.x >> 6)] = ss;
+    if (bid == 0) *reinterpret_cast<uint2*>(x_out + k) = o;
+    __syncthreads();
+    const float4 q = *reinterpret_cast<const float4*>(xs + K);
+    const float rinv = 1.0f / sqrtf(((q.x + q.y) + (q.z + q.w)) / (float)K + eps);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const float4 lo = *reinterpret_cast<const float4*>(xs + xs_index(u * 512 + lane * 8)), hi = *reinterpret_cast<const float4*>(xs + xs_index(u * 512 + lane * 8 + 4));
+      const float f[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        h[u][2 * j] = rbf(f[2 * j] * rinv * lo_bf(nr[u][j]));
+        h[u][2 * j + 1] = rbf(f[2 * j + 1] * rinv * hi_bf(nr[u][j]));
+      }
+    }
+  }
+};
+
 // h = (x - mean) / sqrt(var + eps) * w + b over `width` columns, x in 32 bits, w and b zero behind them; by every wave for itself as well
 template <int U>
 struct RowLayerNormPro {

@@ -49,6 +49,11 @@ struct GemvMerge {
   int nsplit, heads;
 };
 void launch_gemv_merge(const GemvArgs& a, const GemvMerge& p, hipStream_t st);
+// o_proj in slices (oproj_slices.h): f32 sums y, four (launch_oproj_slices) or eight (launch_attn_oproj) times n, which gate + up adds up in front of its norm, writing the sum that the layer
+// continues with to x_out
+bool oproj_slices_ok(int width, int heads, int kv_heads, int head_dim, int ff);
+void launch_oproj_slices(const GemvMerge& p, const void* W, float* y, int n, hipStream_t st);   // p.nsplit <= 16
+void launch_gemv_slices(const GemvArgs& a, const float* parts, int slices, void* x_out, hipStream_t st);   // GEMV_SILU_MUL
 struct GemvPlan { int R, U, grid; };   // rows per wave, 512-column chunks per load group, persistent blocks
 GemvPlan plan_gemv(int N, int K, GemvEpi epi);
 bool gemv_row_on();   // the short forms (gemv_row_body.h) are not switched off by a knob of the block form
@@ -148,6 +153,9 @@ void launch_attn_decode_fused(const AttnDecodeFusedArgs& a, hipStream_t st);
 // The same with the partials left for launch_gemv_merge (nsplit > 1; a single split writes `o`): nsplit from attn_decode_defer_splits, 0 = not here
 int attn_decode_defer_splits(int npages, int nq);
 void launch_attn_decode_defer(const AttnDecodeFusedArgs& a, hipStream_t st);
+// Where o_proj runs in slices: -1: attention and o_proj in one launch (launch_attn_oproj: y (kv heads, n) f32), 1 .. 16: splits for launch_oproj_slices, 0: not so
+int attn_decode_slice_splits(int npages);
+void launch_attn_oproj(const AttnDecodeFusedArgs& a, const void* W, float* y, int n, hipStream_t st);
 
 struct AttnPrefillArgs {
   const void* q;           // (S, nh*d) bf16

@@ -22,6 +22,7 @@
 #include <stdlib.h>
 
 #include "attn_decode_body.h"
+#include "oproj_slices.h"
 #include "attn_prefill_body.h"
 
 namespace aha {
@@ -172,7 +173,41 @@ __global__ __launch_bounds__(256, 2) void attn_decode_defer_kernel(const void* q
   attn_decode_fused_body<ATTN_DECODE_NW, true>(a, smem_defer, (int)blockIdx.x, (int)blockIdx.y, nsplit);
 }
 
+// Short contexts: attention of one kv head (two query heads: 256 columns of W_o) and its share of 32 rows of o_proj, left as f32 for the next norm to add up.
+// The 32 blocks of a kv head, all on one XCD, each do its attention: up to six pages that costs less than the launch of its own that o_proj
+// takes elsewhere (attn_decode_slice_splits).  W_o's rows are requested behind the pages and arrive under the attention.  (Two kv heads and 16 rows per block of eight waves, half as
+// many slices for the norm: 7.3 us + 4.3 of gate + up, here 5.4 + 5.2; attention, o_proj and gate + up in launches of their own 4.8 + 2.9 + 4.4; 19 positions.)
+__global__ __launch_bounds__(256, 2) void attn_oproj_kernel(const void* qkv, const void* q_norm_w, const void* k_norm_w, const float* rope, const uint64_t* page_ptrs, const void* W,
+                                                            int kvh_len, unsigned page_stride, AttnDecodeFusedArgs a, float* y, int n) {
+  extern __shared__ __attribute__((aligned(16))) char smem_defer[];
+  // (what the first requests need: in scalar registers at the start, gemv_body.h)
+  a.qkv = qkv;
+  a.q_norm_w = q_norm_w;
+  a.k_norm_w = k_norm_w;
+  a.rope = rope;
+  a.kv.page_ptrs = page_ptrs;
+  const int kvh = kvh_len >> 20;
+  a.kv_len_v = kvh_len & 0xfffff;
+  a.page_stride = page_stride;
+  a.group = 2;
+  a.kvh = kvh;
+  a.nh = 2 * kvh;
+  a.traced = 0;
+  float* o = reinterpret_cast<float*>(smem_defer);
+  const int kvhd = (int)blockIdx.x, slab = (int)blockIdx.y;
+  OprojRows<4, 256> rows;
+  const int row0 = rows.row0(slab, ATTN_DECODE_NW);
+  attn_decode_fused_body<ATTN_DECODE_NW, true, true>(a, smem_defer + 256 * 4, kvhd, 0, 1, o, slab == 0, [&] { rows.request((const bf16_t*)W, 256 * kvh, kvhd, row0); });
+  __syncthreads();
+  rows.multiply(o, y + kvhd * n, row0);
+}
+
 }  // namespace
+
+void launch_attn_oproj(const AttnDecodeFusedArgs& a, const void* W, float* y, int n, hipStream_t st) {
+  hipLaunchKernelGGL(attn_oproj_kernel, dim3(a.kvh, n / 32), dim3(256), 256 * 4 + ATTN_DEFER_LDS(2), st, a.qkv, a.q_norm_w, a.k_norm_w, a.rope, a.kv.page_ptrs, W, a.kvh << 20 | a.kv_len_v,
+                     a.page_stride, a, y, n);
+}
 
 void launch_attn_decode_fused(const AttnDecodeFusedArgs& a, hipStream_t st) {
   hipLaunchKernelGGL(attn_decode_fused_kernel, dim3(a.kvh, a.nsplit), dim3(256), 0, st, a);
@@ -190,8 +225,13 @@ int attn_decode_defer_splits(int npages, int nq) {
   if (npages > 6 * most) return 0;
   return nq > 2048 && npages <= 4 ? 1 : std::min((npages + 1) / 2, most);
 }
+// 0.6B, us per token, merged by gemv_row_merge_kernel (beyond 48 pages inside the launch) / in slices: 20 positions 561 / 518, 200: 569 / 550, 300: 575 / 564, 400 (seven
+// pages: every block of attn_oproj_kernel streams them all) 576 / 575, 470: 577 / 591; with splits of their own 470: 577 / 594, 900: 593 / 594, 1200: 602 / 596,
+// 2000: 619 / 602, 4000: 713 / 625, 12000: 896 / 783.  In between the slices' extra bytes in front of gate + up cost what the merge saves.  (A unit has at most three
+// pages, attn_decode_body.h: 192.)
+int attn_decode_slice_splits(int npages) { return npages <= 6 ? -1 : npages <= 16 || npages > 192 ? 0 : std::min((npages + 1) / 2, 16); }
 void launch_attn_decode_defer(const AttnDecodeFusedArgs& a, hipStream_t st) {
-  const int lds = 16 * 128 * 2 + 2 * 128 * 2 + ATTN_DECODE_NW * 128 * (a.nh / a.kvh) * 4 + (2 * ATTN_DECODE_NW + 1) * 16 * 4;
+  const int lds = ATTN_DEFER_LDS(a.nh / a.kvh);
   hipLaunchKernelGGL(attn_decode_defer_kernel, dim3(a.kvh, a.nsplit), dim3(256), lds, st, a.qkv, a.q_norm_w, a.k_norm_w, a.rope, a.kv.page_ptrs, a.kv_len_v,
                      a.kvh << 16 | (a.trace != nullptr) << 15 | a.nh / a.kvh, a.nsplit, a.page_stride, a);
 }

@@ -7,6 +7,7 @@
 //   PolyNorm:                      h = a N(z) + b N(z^2) + c N(z^3) + e: the three row sums in the prologue
 #include "gemv_prologues.h"
 #include "gemv_row_body.h"
+#include "oproj_slices.h"
 
 namespace aha {
 
@@ -219,6 +220,47 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_row_merge_kernel(const floa
   RowMergePro<U, MS> pro{part_o, part_ml, nsplit, xs};
   gemv_row_body<1, U, GEMV_RESIDUAL>(rest, W, residual, trace, N, (int)blockIdx.x, nblk, pro);
 }
+// o_proj behind split attention, in slices (oproj_slices.h): block (two kv heads, 16 rows) merges the partials of its four heads alone, two KB a split and
+// block, where a block of gemv_row_merge_kernel merges all of them (eight splits: 64 KB, twice per CU).  A wave per head: lane l < 16 has split l for the weights,
+// every lane two columns of all splits.  2048 + 256 positions of 0.6B: attention + o_proj + gate + up 6.5 + 4.0 + 4.4 us with eight splits, 5.5 + 3.4 + 4.8 with sixteen
+// in slices (166.4 -> 159.5 ms in all); more splits cost the merge of all heads what they save the attention.
+__global__ __launch_bounds__(256) void oproj_slice_kernel(const float* part_o, const float* part_ml, const void* W, float* y, int heads, int n, int nsplit) {
+  __shared__ __attribute__((aligned(16))) float hs[512];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), slice = (int)blockIdx.x, head = slice * 4 + wave;
+  const float2 ml = *reinterpret_cast<const float2*>(part_ml + (min(lane & 15, nsplit - 1) * heads + head) * 2);
+  float2 v[16];
+#pragma unroll
+  for (int s = 0; s < 16; ++s) v[s] = *reinterpret_cast<const float2*>(part_o + (min(s, nsplit - 1) * heads + head) * 128 + lane * 2);   // (surplus ones repeat the last split)
+  OprojRows<4, 512> rows;
+  const int row0 = rows.row0((int)blockIdx.y, 4);
+  __builtin_amdgcn_sched_barrier(0);
+  rows.request((const bf16_t*)W, heads * 128, slice, row0);
+  __builtin_amdgcn_sched_barrier(0);
+  float M = ml.x;
+#pragma unroll
+  for (int d = 8; d >= 1; d >>= 1) M = fmaxf(M, __shfl_xor(M, d, 64));
+  const float e = (lane & 15) < nsplit && ml.x != -INFINITY ? __expf(ml.x - M) : 0.f;
+  float z = e * ml.y;
+#pragma unroll
+  for (int d = 8; d >= 1; d >>= 1) z += __shfl_xor(z, d, 64);
+  float2 o = make_float2(0.f, 0.f);
+#pragma unroll
+  for (int s = 0; s < 16; ++s) {
+    const float w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(e), s));
+    o.x = fmaf(w, v[s].x, o.x);
+    o.y = fmaf(w, v[s].y, o.y);
+  }
+  const float inv = 1.0f / z;
+  *reinterpret_cast<float2*>(hs + wave * 128 + lane * 2) = make_float2(rbf(o.x * inv), rbf(o.y * inv));   // (the attention output tensor is bf16)
+  __syncthreads();
+  rows.multiply(hs, y + slice * n, row0);
+}
+template <int P>
+__global__ __launch_bounds__(GEMV_THREADS) void gemv_row_slices_kernel(const void* x, const float* parts, const void* W, const void* norm_w, void* x_out, int N, float eps, int nblk, GemvArgs rest) {
+  __shared__ __attribute__((aligned(16))) float xs[1024 + 4];
+  RowSlicesPro<P> pro{(const bf16_t*)x, (const bf16_t*)norm_w, parts, (bf16_t*)x_out, eps, (int)blockIdx.x, xs};
+  gemv_row_body<1, 2, GEMV_SILU_MUL>(rest, W, nullptr, nullptr, N, (int)blockIdx.x, nblk, pro);
+}
 template <int R, int U, bool FAST, int XP, int MS, int KX = 0>
 __global__ __launch_bounds__(GEMV_THREADS) void gemv_merge_kernel(const float* part_o, const float* part_ml, const void* W, const void* residual, unsigned long long* trace, int N, int K, int nsplit, int nblk,
                                                                     GemvArgs rest) {
@@ -310,6 +352,19 @@ void launch_gemv_merge(const GemvArgs& a, const GemvMerge& p, hipStream_t st) {
   else if (pl.U >= 8) go(integral_constant<int, 1>{}, integral_constant<int, 8>{});
   else if (pl.U >= 4) go(integral_constant<int, 1>{}, integral_constant<int, 4>{});
   else go(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+}
+
+bool oproj_slices_ok(int width, int heads, int kv_heads, int head_dim, int ff) {
+  return width == 1024 && heads == 16 && kv_heads == 8 && head_dim == 128 && gemv_row_groups(ff, width, GEMV_SILU_MUL) == 2 && plan_gemv(ff, width, GEMV_SILU_MUL).R == 1;
+}
+void launch_oproj_slices(const GemvMerge& p, const void* W, float* y, int n, hipStream_t st) {
+  hipLaunchKernelGGL(oproj_slice_kernel, dim3((unsigned)(p.heads / 4), (unsigned)(n / 16)), dim3(256), 0, st, p.part_o, p.part_ml, W, y, p.heads, n, p.nsplit);
+}
+void launch_gemv_slices(const GemvArgs& a, const float* parts, int n, void* x_out, hipStream_t st) {
+  const int nblk = gemv_row_grid(a.N, 1);
+  auto go = [&](auto k) { hipLaunchKernelGGL(k, dim3(nblk), dim3(GEMV_THREADS), 0, st, a.x, parts, a.W, a.norm_w, x_out, a.N, a.eps, nblk, a); };
+  if (n == 4) go(gemv_row_slices_kernel<4>);
+  else go(gemv_row_slices_kernel<8>);
 }
 
 void launch_gemv_polynorm(const GemvArgs& a, const PolyNormArgs& p, GemvEpi epi, hipStream_t st) {

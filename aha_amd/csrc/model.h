@@ -116,6 +116,8 @@ struct aha_model {
   float* d_logits = nullptr;
   float* d_blk_max = nullptr;
   uint32_t* d_blk_idx = nullptr;
+  void* d_x2 = nullptr;          // the residual stream between a layer's halves, d_part_y: o_proj's slices (oproj_slices_ok)
+  float* d_part_y = nullptr;
   float* d_part_o = nullptr;
   float* d_part_ml = nullptr;
   int max_nsplit = 64;

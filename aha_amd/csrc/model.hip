@@ -775,6 +775,11 @@ int model_create(aha_ctx* ctx, const aha_model_desc* desc, const aha_tensor_view
   m->d_part_o = (float*)p;
   if ((rc = dev_alloc(m, (size_t)m->max_nsplit * 4 * c.num_attention_heads * 2 * 4, &p))) return fail(rc);
   m->d_part_ml = (float*)p;
+  if (c.tp_size <= 1 && oproj_slices_ok(H, c.num_attention_heads, c.num_key_value_heads, d, I)) {
+    if ((rc = dev_alloc(m, (size_t)H * 2, &m->d_x2))) return fail(rc);
+    if ((rc = dev_alloc(m, (size_t)c.num_key_value_heads * H * 4, &p))) return fail(rc);
+    m->d_part_y = (float*)p;
+  }
   if ((rc = dev_alloc(m, 128 * 4, &p, true))) return fail(rc);
   m->d_rope = (float*)p;
 
@@ -1447,6 +1452,8 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_read
   // short and middle contexts: the merge of the splits in the o_proj matvec (one GPU)
   int defer = e_div || !m->decode_fused ? 0 : attn_decode_defer_splits(npages, nq);
   if (defer > 1 && m->tp_size > 1) defer = 0;
+  const int slices = e_div || !m->decode_fused || !m->d_part_y ? 0 : attn_decode_slice_splits(npages);
+  if (slices) defer = std::abs(slices);
   if (defer) nsplit = defer;
   // pages at one distance from each other: the attention computes their addresses
   uint64_t page_stride = defer ? m->page_bytes : 0;
@@ -1491,11 +1498,14 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_read
       const double gemv_bytes = (double)g.N * g.K * 2 + g.K * 2.0 + g.N * 4.0;
       {
         ProfScope ps(m, "attn_decode", attn_bytes, 4.0 * kv_len_after * nq);
-        if (defer) launch_attn_decode_defer(a, st);
+        if (slices < 0) launch_attn_oproj(a, L.wo, m->d_part_y, H, st);
+        else if (defer) launch_attn_decode_defer(a, st);
         else launch_attn_decode_fused(a, st);
       }
       ProfScope ps(m, "gemv", gemv_bytes, 2.0 * g.N * g.K);
-      if (defer > 1) launch_gemv_merge(g, GemvMerge{m->d_part_o, m->d_part_ml, nsplit, nh}, st);
+      if (slices > 0) launch_oproj_slices(GemvMerge{m->d_part_o, m->d_part_ml, nsplit, nh}, L.wo, m->d_part_y, H, st);
+      else if (slices < 0) {   // (o_proj is done)
+      } else if (defer > 1) launch_gemv_merge(g, GemvMerge{m->d_part_o, m->d_part_ml, nsplit, nh}, st);
       else gemv_row_parallel(m, g);
     } else {  // three-launch variant (A/B knob AHA_DECODE_FUSED=0)
       {  // q/k norm + rope + append                            (modules.rs:544-566)
@@ -1526,11 +1536,12 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_read
       g.W = L.wgu; g.W2 = nullptr; g.x = m->d_x; g.norm_w = L.post_norm; g.eps = c.rms_norm_eps; g.y = m->d_act; g.N = I; g.K = H;
       g.trace = gemv_trace_slot(m, li * 4 + 2);
       ProfScope ps(m, "gemv", (double)2 * I * H * 2 + H * 4.0 + I * 2.0, 4.0 * I * H);
-      launch_gemv(g, GEMV_SILU_MUL, st);
+      if (slices) launch_gemv_slices(g, m->d_part_y, slices < 0 ? kvh : nq / 512, m->d_x2, st);
+      else launch_gemv(g, GEMV_SILU_MUL, st);
     }
     {  // x = x + act Wd^T                                     (modules.rs:85, qwen3/model.rs:86)
       GemvArgs g{};
-      g.W = L.wdown; g.x = m->d_act; g.residual = m->d_x; g.y = m->d_x; g.N = H; g.K = I;
+      g.W = L.wdown; g.x = m->d_act; g.residual = slices ? m->d_x2 : m->d_x; g.y = m->d_x; g.N = H; g.K = I;
       g.trace = gemv_trace_slot(m, li * 4 + 3);
       ProfScope ps(m, "gemv", (double)g.N * g.K * 2 + g.K * 2.0 + g.N * 4.0, 2.0 * g.N * g.K);
       gemv_row_parallel(m, g);

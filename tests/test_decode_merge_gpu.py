@@ -42,6 +42,34 @@ def test_partials_merged_by_the_projection(gpu, monkeypatch, heads, kv_heads, le
     merged.close(); plain.close()
 
 
+@pytest.mark.parametrize("scrambled", [False, True])
+@pytest.mark.parametrize("lens", [[1, 2, 62, 63, 64, 65], [127, 128, 191, 256, 319, 320], [381, 382, 383, 500], [1021, 1022, 1023, 1500], [2047, 12286]])
+def test_projection_in_slices(gpu, monkeypatch, lens, scrambled):
+    """attn_oproj_kernel (up to six pages), oproj_slice_kernel (9 to 16 splits, 17 to 192 pages) and gemv_row_slices_kernel at the widths they are built for,
+    across the lengths where one takes over from another, pages at one distance from each other and not; the bound as above."""
+    from aha_amd.model import HipInferenceModel
+    cfg = tiny_qwen3(layers=3, hidden=1024, heads=16, kv_heads=8, inter=1536, vocab=1024)
+    w = qwen3_text_weights(cfg, seed=14)
+    monkeypatch.setenv("AHA_DECODE_FUSED", "1")
+    sliced = HipInferenceModel(cfg, w)
+    monkeypatch.setenv("AHA_DECODE_FUSED", "0")
+    plain = HipInferenceModel(cfg, w)
+    sliced.debug_scramble_pages(scrambled)
+    for S in lens:
+        ids = ids_for(cfg, S, 9 + S)
+        sliced.clear_cache(); plain.clear_cache()
+        _, tok = plain.forward_initial(ids, 0)
+        sliced.forward_initial(ids, 0)
+        for step in range(4):
+            a, am = plain.forward_step(tok, S + step)
+            b, _ = sliced.forward_step(tok, S + step)
+            std = float(a.std())
+            assert np.isfinite(b).all()
+            assert float(np.abs(a - b).max()) <= LOGIT_TOL_STD * std and float(np.sqrt(((a - b) ** 2).mean())) <= LOGIT_RMS_STD * std, (S, step)
+            tok = am
+    sliced.close(); plain.close()
+
+
 @pytest.mark.parametrize("hidden, vocab", [(256, 64), (256, 5000), (1024, 70001)])
 def test_between_two_steps(gpu, hidden, vocab):
     """The launch between two steps of the greedy loop (arg-max, state, embedding row, rope table) against the same tokens fed one by one: the kernels
