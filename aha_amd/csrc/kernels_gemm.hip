@@ -1248,7 +1248,10 @@ static bool takes_few_rows(const GemmArgs& a, const GemmPlan& plan, int* r8) {
   const bool slices = plan.splitk > 1;
   const double plan_us = gemm_skinny_plan(a, r8);
   if (a.few_rows == 2) return plan_us < 1e30;
-  const double few = plan_us + (a.norm_w && slices ? 3.0 : 0.0);   // (a norm that the reduce pass would have taken along: its own launch)
+  // A norm that the reduce pass would have taken along costs its own launch: up to 32 rows 1 us of the chain between two products, not the 3 us that it
+  // takes alone (with 1 against 3, whole prompts in us: 0.6B at 19 / 24 / 32 tokens 1394 -> 1300, 1306 -> 1289, 1312 -> 1305; 8B 4278 -> 3898,
+  // 4282 -> 3976, 4302 -> 4147; 0 and -2 as 1).  Above, 8B gains nothing (40 tokens 4578 -> 4617, 48 and 64 the same) and it stays.
+  const double few = plan_us + (a.norm_w && slices ? (a.M <= 32 ? 1.0 : 3.0) : 0.0);
   if (few < 1e30 && gemm_skinny_rounds(a, *r8) > 1)
     return few * 1.02 < std::max(plan.cost, bytes / 4.84e6 + (slices ? 8.0 : 2.0) + (a.act == ACT_SILU_MUL_PAIRS ? 4.0 : 0.0));
   return few < std::max(plan.cost, bytes / 4.2e6 + (slices ? 5.0 : 2.0));
