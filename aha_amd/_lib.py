@@ -98,6 +98,7 @@ SIGNATURES = {
     "aha_hip_model_destroy": (None, [_P]),
     "aha_hip_forward_initial": (C.c_int, [_P, C.POINTER(C.c_uint32), C.c_size_t, C.c_size_t, C.POINTER(MmInput),
                                           C.POINTER(C.c_float), C.POINTER(C.c_uint32)]),
+    "aha_hip_forward_step_enqueue": (C.c_int, [_P, C.c_uint32, C.c_size_t]),
     "aha_hip_forward_step": (C.c_int, [_P, C.c_uint32, C.c_size_t, C.POINTER(C.c_float), C.POINTER(C.c_uint32)]),
     "aha_hip_clear_cache": (C.c_int, [_P]),
     "aha_hip_stop_token_ids": (C.c_int, [_P, C.POINTER(C.c_uint32), C.c_size_t]),

@@ -116,6 +116,15 @@ int aha_hip_forward_initial(aha_model* m, const uint32_t* input_ids, size_t n_id
   return model_forward_initial(m, input_ids, n_ids, seqlen_offset, mm, logits_out, argmax_out);
   API_GUARD_END
 }
+int aha_hip_forward_step_enqueue(aha_model* m, uint32_t token, size_t seqlen_offset) {
+  API_GUARD_BEGIN
+  if (!m) {
+    set_error("null model");
+    return AHA_ERR_INVALID;
+  }
+  return model_forward_step_enqueue(m, token, seqlen_offset);
+  API_GUARD_END
+}
 int aha_hip_forward_step(aha_model* m, uint32_t token, size_t seqlen_offset, float* logits_out, uint32_t* argmax_out) {
   API_GUARD_BEGIN
   if (!m) {
@@ -243,6 +252,7 @@ int aha_hip_debug_graph_step(aha_model* m, int32_t replays, double* us_launches,
 int aha_hip_kv_export(aha_model* m, void* out_dev, size_t out_bytes, size_t* bytes_needed, size_t* n_tokens, int64_t* rope_delta) {
   if (!m) return AHA_ERR_INVALID;
   API_GUARD_BEGIN
+  if (int rc = model_wait_step(m)) return rc;
   return model_kv_export(m, out_dev, out_bytes, bytes_needed, n_tokens, rope_delta);
   API_GUARD_END
 }
@@ -250,6 +260,7 @@ int aha_hip_kv_import(aha_model* m, const void* in_dev, size_t in_bytes, int32_t
                       size_t n_tokens, int64_t rope_delta) {
   if (!m) return AHA_ERR_INVALID;
   API_GUARD_BEGIN
+  if (int rc = model_wait_step(m)) return rc;
   return model_kv_import(m, in_dev, in_bytes, src_heads, src_head0, dst_head0, n_heads, n_tokens, rope_delta);
   API_GUARD_END
 }
@@ -398,6 +409,7 @@ int aha_hip_debug_last_hidden(aha_model* m, float* out, size_t n) {
     set_error("debug_last_hidden: bad size");
     return AHA_ERR_INVALID;
   }
+  if (int rc = model_wait_step(m)) return rc;
   std::vector<uint16_t> tmp(n);
   AHA_HIP_CHECK(hipMemcpy(tmp.data(), m->d_hlast, n * 2, hipMemcpyDeviceToHost));
   for (size_t i = 0; i < n; ++i) {
@@ -757,6 +769,7 @@ int aha_hip_embed(aha_model* m, const uint32_t* input_ids, size_t n_ids, float* 
     set_error("null model");
     return AHA_ERR_INVALID;
   }
+  if (int rc = model_wait_step(m)) return rc;
   return model_embed(m, input_ids, n_ids, out);
   API_GUARD_END
 }
@@ -766,6 +779,7 @@ int aha_hip_embed_multi(aha_model* m, const uint32_t* input_ids, const uint64_t*
     set_error("null model");
     return AHA_ERR_INVALID;
   }
+  if (int rc = model_wait_step(m)) return rc;
   return model_embed_multi(m, input_ids, n_ids, n_docs, out);
   API_GUARD_END
 }

@@ -159,6 +159,7 @@ struct aha_model {
   unsigned long long* d_attn_trace = nullptr;  // AHA_ATTN_TRACE timeline
   bool decode_fused = true;  // attention block of a decode step in one launch (kernels_attn.hip attn_decode_fused_kernel)
   float* h_logits = nullptr;  // pinned
+  bool step_in_flight = false;   // model_forward_step_enqueue: the stream has not been waited for since (model_wait_step)
   bool have_logits = false;   // d_logits holds the logits of a completed forward call
   bool logits_assembled = false;  // vocab-parallel TP: d_logits already all-reduced into the full vector
   // D11 candidate extraction (kernels_sample.hip), allocated on first use
@@ -210,6 +211,8 @@ int model_embed_multi(aha_model* m, const uint32_t* ids, const uint64_t* lens, s
 int model_forward_initial(aha_model* m, const uint32_t* ids, size_t n, size_t offset, const aha_mm_input* mm,
                           float* logits_out, uint32_t* argmax_out);
 int model_forward_step(aha_model* m, uint32_t token, size_t offset, float* logits_out, uint32_t* argmax_out);
+int model_forward_step_enqueue(aha_model* m, uint32_t token, size_t offset);
+int model_wait_step(aha_model* m);   // before anything that the host or another stream does to what a step reads or writes
 int model_decode_greedy(aha_model* m, uint32_t first_token, size_t offset, size_t max_new, uint32_t* out);
 int model_clear_cache(aha_model* m);
 int model_last_logits(aha_model* m, float* logits_out);

@@ -330,6 +330,10 @@ class HipInferenceModel:
         check(lib().aha_hip_forward_step(self.handle, int(token), seqlen_offset, lp, C.byref(am)))
         return (self._logits.copy() if want_logits else None), int(am.value)
 
+    def forward_step_enqueue(self, token: int, seqlen_offset: int) -> None:
+        """forward_step without its outputs: the logits stay on the device for sample_candidates / last_logits, and nothing is waited for."""
+        check(lib().aha_hip_forward_step_enqueue(self.handle, int(token), seqlen_offset))
+
     def clear_cache(self):
         check(lib().aha_hip_clear_cache(self.handle))
 

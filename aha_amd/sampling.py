@@ -202,7 +202,7 @@ def draw_from_candidates(lp: "LogitsProcessor", w: np.ndarray, idx: np.ndarray) 
     return int(idx[lp.draw(w)])
 
 
-def sample_and_push(ctx: GenerationContext, model, argmax_token: int, generated: List[int]) -> int:
+def sample_and_push(ctx: GenerationContext, model, argmax_token: Optional[int], generated: List[int]) -> int:
     """common/generate.rs:70-86 on the logits of the model's last forward call."""
     lp = ctx.logit_processor
     pen, pctx = penalty_context(ctx.repeat_penalty, ctx.repeat_last_n, generated)
@@ -235,6 +235,14 @@ def sample_and_push(ctx: GenerationContext, model, argmax_token: int, generated:
     return token
 
 
+def _step(model, token: int, seqlen_offset: int, lp) -> Optional[int]:
+    """One decoding step in front of sample_and_push: its arg-max, or None where the sampler reads candidates off the device anyway."""
+    if lp.sampling.kind != "ArgMax" and hasattr(model, "forward_step_enqueue"):
+        model.forward_step_enqueue(token, seqlen_offset)
+        return None
+    return model.forward_step(token, seqlen_offset, want_logits=False)[1]
+
+
 def generate_generic_sampled(model, input_ids: Sequence[int], ctx: GenerationContext, data=None) -> List[int]:
     """generate_generic_text's token loop (common/generate.rs:87-112) with the sampler of `ctx`."""
     eos = set(model.stop_token_ids())
@@ -244,7 +252,7 @@ def generate_generic_sampled(model, input_ids: Sequence[int], ctx: GenerationCon
     ctx.seqlen_offset += ctx.seq_len  # prepare_for_next_token
     ctx.seq_len = 1
     for _ in range(1, ctx.sample_len):
-        _, am = model.forward_step(tok, ctx.seqlen_offset, want_logits=False)
+        am = _step(model, tok, ctx.seqlen_offset, ctx.logit_processor)
         tok = sample_and_push(ctx, model, am, generated)
         if tok in eos:
             break
@@ -278,7 +286,7 @@ def generate_asr(model, audio_datas, temperature: float, top_p: Optional[float] 
             if seqlen_offset == 0:
                 _, am = model.forward_initial(input_ids, 0, data, want_logits=False)
             else:
-                _, am = model.forward_step(tok, seqlen_offset, want_logits=False)
+                am = _step(model, tok, seqlen_offset, lp)
             mark = len(generated)
             tok = sample_and_push(ctx, model, am, generated)
             assert len(generated) == mark + 1
@@ -320,7 +328,7 @@ def generate_stream_generic_text(model, decode, input_ids: Sequence[int], ctx: G
                 tok = pending.pop(0)
                 generated.append(tok)
             else:
-                _, am = model.forward_step(generated[-1], ctx.seqlen_offset, want_logits=False)
+                am = _step(model, generated[-1], ctx.seqlen_offset, lp)
                 tok = sample_and_push(ctx, model, am, generated)
             piece = decode(error_tokens + [tok])
             # prepare_for_next_token (generate.rs:54-66)

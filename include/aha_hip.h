@@ -239,6 +239,9 @@ int aha_hip_forward_initial(aha_model* m, const uint32_t* input_ids, size_t n_id
                             const aha_mm_input* mm, float* logits_out, uint32_t* argmax_out);
 /* forward_step(&mut self, input_ids (1,1), seqlen_offset) -> logits (1,1,V). */
 int aha_hip_forward_step(aha_model* m, uint32_t token, size_t seqlen_offset, float* logits_out, uint32_t* argmax_out);
+/* forward_step whose logits stay on the device and whose arg-max is not computed: returns once the step is enqueued.  What reads them -- aha_hip_sample_candidates,
+ * aha_hip_last_logits -- waits, and so does the next forward call. */
+int aha_hip_forward_step_enqueue(aha_model* m, uint32_t token, size_t seqlen_offset);
 /* clear_cache(&mut self) */
 int aha_hip_clear_cache(aha_model* m);
 /* stop_token_ids(&self) -> Vec<u32>: writes up to cap ids, returns the count (>=0) or a negative status. */

@@ -204,6 +204,7 @@ pub mod sys {
             argmax_out: *mut u32,
         ) -> i32;
         pub fn aha_hip_forward_step(m: *mut AhaModel, token: u32, seqlen_offset: usize, logits_out: *mut f32, argmax_out: *mut u32) -> i32;
+        pub fn aha_hip_forward_step_enqueue(m: *mut AhaModel, token: u32, seqlen_offset: usize) -> i32;
         pub fn aha_hip_clear_cache(m: *mut AhaModel) -> i32;
         pub fn aha_hip_stop_token_ids(m: *const AhaModel, out: *mut u32, cap: usize) -> i32;
         pub fn aha_hip_decode_greedy(m: *mut AhaModel, first_token: u32, seqlen_offset: usize, max_new: usize, tokens_out: *mut u32) -> i32;

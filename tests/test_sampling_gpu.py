@@ -204,3 +204,37 @@ def test_a_wave_of_minus_infinity(gpu, vocab, ks):
                 m.sample_candidates([], 1.0, 1.0, ks[-1] + 1)
     finally:
         m.close()
+
+
+def test_enqueued_steps(gpu):
+    """forward_step_enqueue leaves what forward_step computes: logits, cache and candidates are the same, over a page's end, with steps enqueued behind one
+    another, and whatever call comes next waits for the step (another step, a prompt, clear_cache, last_hidden).  Tokens and offsets are checked alike."""
+    cfg, m = make(3000)
+    try:
+        ids = [int(x) for x in np.random.default_rng(4).integers(0, 3000, size=120)]
+        toks = [int(x) for x in np.random.default_rng(5).integers(0, 3000, size=12)]
+        m.forward_initial(ids, 0, want_logits=False)
+        want, hidden = [], []
+        for i, t in enumerate(toks):
+            want.append(m.forward_step(t, 120 + i)[0])
+            hidden.append(m.debug_last_hidden())
+        for every in (1, 3, 12):   # logits read after every so many steps
+            m.clear_cache()
+            m.forward_initial(ids, 0, want_logits=False)
+            for i, t in enumerate(toks):
+                m.forward_step_enqueue(t, 120 + i)
+                if (i + 1) % every == 0:
+                    np.testing.assert_array_equal(m.debug_last_hidden(), hidden[i])
+                    check_candidates(m, want[i], [3, 5], 1.2, 0.8, 20)
+                    np.testing.assert_array_equal(m.last_logits(), want[i])
+        m.forward_step_enqueue(7, 132)
+        m.clear_cache()
+        assert m.cache_len() == 0
+        m.forward_initial(ids, 0, want_logits=False)
+        m.forward_step_enqueue(toks[0], 120)
+        np.testing.assert_array_equal(m.forward_step(toks[1], 121)[0], want[1])
+        with pytest.raises(_lib.AhaHipError):
+            m.forward_step_enqueue(3000, 122)
+        np.testing.assert_array_equal(m.forward_step(toks[2], 122)[0], want[2])
+    finally:
+        m.close()
