@@ -466,18 +466,47 @@ __global__ __launch_bounds__(256) void ssm_segments_kernel(SsmScanArgs a, SeqBat
 }
 
 // ---- one token per sequence ------------------------------------------------------------------------------------------------------------------
-// Block (head and VT * 16 of its columns, sequence): thread (n, four columns of 16), n = tid / 4, + 64, ...  The state is requested first; the
+// Block (VT * 16 columns, head of the group, group and sequence): thread (n, four columns of 16), n = tid / 4, + 64, ...  The state is requested first; the
 // convolution of the block's channels (its x columns, the group's B and C) runs under that.
-// NT: the state past the caches (launch_ssm_step).
-template <typename TI, int NI, int VT, bool NT>
-__global__ __launch_bounds__(256) void ssm_step_kernel(SsmStepArgs a, SeqBatch b) {
-  __shared__ __attribute__((aligned(16))) float bc[2 * NI * 64], xs[VT * 16], red[4][VT * 16];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nvs = a.d.vdp >> 4, h = blockIdx.x / (nvs / VT), vs = (blockIdx.x - h * (nvs / VT)) * VT, np = a.d.np, taps = a.d.taps;
-  const SeqEntry e = seq_entry_at(b, blockIdx.y);
-  const int cp = a.d.cp(), inner = a.d.inner(), hpg = a.d.heads / a.d.groups, grp = h / hpg;
+// NT: the state past the caches (launch_ssm_step).  ONE: one sequence and 2 to 5 taps, its places in the leading arguments (SsmStepLead), which are in registers
+// before the first instruction.
+// Below 16 MB of states the launch is one chain of waits, not bytes: nothing that the end needs is requested behind a barrier (the gate), wave 2 computes the
+// step size that all used to, no divisions, the sums over n without the LDS crossbar.  0.6B widths, one sequence: 5.0 -> 3.6 us.
+__device__ __forceinline__ float sum_stride4(float v) {   // over the sixteen lanes of one lane & 3
+  v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x124 /* row_ror:4 */, 0xf, 0xf, false));
+  v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x128 /* row_ror:8 */, 0xf, 0xf, false));
+  unsigned u = __float_as_uint(v);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  u = __float_as_uint(v);
+  const auto q = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __uint_as_float(q[0]) + __uint_as_float(q[1]);
+}
+struct SsmStepLead {   // sizes in two words
+  int np_taps_hpg, vdp_groups;
+  __host__ __device__ int np() const { return np_taps_hpg & 1023; }
+  __host__ __device__ int taps() const { return np_taps_hpg >> 10 & 63; }   // (63: that many or more)
+  __host__ __device__ int hpg() const { return (int)((unsigned)np_taps_hpg >> 16); }
+  __host__ __device__ int vdp() const { return vdp_groups & 65535; }
+  __host__ __device__ int groups() const { return (int)((unsigned)vdp_groups >> 16); }
+};
+template <typename TI, int NI, int VT, bool NT, bool ONE>
+__global__ __launch_bounds__(256) void ssm_step_kernel(const float* sin, const TI* in_c, const float* hin, const float* conv_w, const float* conv_b, int inner, int np_taps_hpg,
+                                                       int vdp_groups, int pos0, SsmStepArgs a, SeqBatch b) {
+  __shared__ __attribute__((aligned(16))) float bc[2 * NI * 64], xs[VT * 16], red[4][VT * 16], step[2];
+  const SsmStepLead lead{np_taps_hpg, vdp_groups};
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), vdp = lead.vdp(), nvs = vdp >> 4, vs = blockIdx.x * VT, np = lead.np(), taps = lead.taps(), groups = lead.groups();
+  const int seq = ONE ? 0 : (int)blockIdx.z / groups, grp = ONE ? (int)blockIdx.z : (int)blockIdx.z - seq * groups, h = grp * lead.hpg() + blockIdx.y, cp = inner + 2 * groups * np;
+  SeqEntry e = b.one;
+  if constexpr (!ONE) {
+    e = seq_entry_at(b, seq);
+    sin += (int64_t)e.state_in * a.s.pool_stride;
+    in_c += (int64_t)e.row0 * a.in.ld;
+    hin += (int64_t)e.slot * a.h.slot_stride + (int64_t)e.hist_in * (a.d.taps - 1) * cp;
+    pos0 = e.pos0;
+  }
   const int64_t so = ((int64_t)h * nvs + vs) * np * 16;
-  const float* sin = a.s.state + (int64_t)e.state_in * a.s.pool_stride + so;
-  float* sout = a.s.state + (int64_t)e.state_out * a.s.pool_stride + so;
+  sin += so;
   const int n0 = tid >> 2, v4 = (tid & 3) * 4;
   float4 S[VT][NI];
 #pragma unroll
@@ -485,7 +514,7 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(SsmStepArgs a, SeqBatch b
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       S[vt][i] = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (e.pos0 > 0 && n0 + i * 64 < np) {
+      if (pos0 > 0 && n0 + i * 64 < np) {
         const float* at = sin + (vt * np + n0 + i * 64) * 16 + v4;
         if constexpr (NT) {
           const f32x4_t x = __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(at));
@@ -495,37 +524,48 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(SsmStepArgs a, SeqBatch b
         }
       }
     }
-  const TI* row = (const TI*)a.in.p + (int64_t)e.row0 * a.in.ld;
-  const float dtz = Act<TI>::ld(row + a.in.dt_off + h) + a.p.dt_bias[h];
-  const float A = a.p.a[h], D = a.p.d[h];
-  const float* hin = a.h.hist + (int64_t)e.slot * a.h.slot_stride + (int64_t)e.hist_in * (taps - 1) * cp;
-  float* hout = a.h.hist + (int64_t)e.slot * a.h.slot_stride + (int64_t)e.hist_out * (taps - 1) * cp;
+  // what wave 2 (the step size) and wave 3 (the gate of the columns it ends with) need, requested behind the convolution's inputs: it is found through the
+  // arguments in memory
+  const int fin = tid - 192, col = h * vdp + vs * 16 + min(fin, VT * 16 - 1);
+  float ex, per_head, dt_bias;
+  float* hout;
+  auto others = [&] {
+    ex = Act<TI>::ld(in_c - a.in.c_off + (fin >= 0 ? col : a.in.dt_off + h));
+    per_head = (wave == 3 ? a.p.d : a.p.a)[h];
+    dt_bias = a.p.dt_bias[h];
+    hout = a.h.hist + (int64_t)e.slot * a.h.slot_stride + (int64_t)e.hist_out * (a.d.taps - 1) * cp;
+  };
   // The block's channels: x, B and C, NIT per thread.  Inputs, weights and history of up to HT + 1 taps are requested together and the new history is
-  // stored behind them: a store between two loads orders them, and tap by tap, channel by channel the chain was most of the launch (0.6B widths,
+  // stored at the end (a wait for the state, in flight since before them, would wait for these stores too): a store between two loads orders them, and tap by tap, channel by channel the chain was most of the launch (0.6B widths,
   // one sequence: 7.5 -> 5.3 us; 8B widths, 32 sequences, bound by the 268 MB of their states: 60.7 -> 59.7 us, 50.8 past the caches).
   constexpr int NIT = (2 * NI * 64 + VT * 16 + 255) / 256, HT = 4;
   const int total = 2 * np + VT * 16;
-  auto channel = [&](int i) { return i >= 2 * np ? h * a.d.vdp + vs * 16 + i - 2 * np : inner + (i < np ? grp * np + i : a.d.groups * np + grp * np + i - np); };
+  auto channel = [&](int i) { return i >= 2 * np ? h * vdp + vs * 16 + i - 2 * np : inner + (i < np ? grp * np + i : groups * np + grp * np + i - np); };
   auto put = [&](int i, float acc) {
     acc = silu_f32(acc);
     if (i >= 2 * np) xs[i - 2 * np] = acc;
     else bc[i < np ? i : NI * 64 + i - np] = acc;
   };
-  if (taps >= 2 && taps <= HT + 1) {
-    float cur[NIT], wl[NIT], bias[NIT], x[NIT][HT], w[NIT][HT];
+  const bool few_taps = ONE || (taps >= 2 && taps <= HT + 1);
+  float cur[NIT], x[NIT][HT];
+  if (few_taps) {
+    float wl[NIT], bias[NIT], w[NIT][HT];
 #pragma unroll
     for (int k = 0; k < NIT; ++k) {
+      if (wave * 64 + k * 256 >= total) continue;
       const int ch = channel(min(tid + k * 256, total - 1));
-      cur[k] = Act<TI>::ld(row + a.in.c_off + ch);
-      wl[k] = a.p.conv_w[(int64_t)(taps - 1) * cp + ch];
-      bias[k] = a.p.conv_b[ch];
+      cur[k] = Act<TI>::ld(in_c + ch);
+      wl[k] = conv_w[(int64_t)(taps - 1) * cp + ch];
+      bias[k] = conv_b[ch];
 #pragma unroll
       for (int q = 0; q < HT; ++q) {   // (taps that are not there: the oldest one again)
         const int qq = min(q, taps - 2);
         x[k][q] = hin[(int64_t)qq * cp + ch];
-        w[k][q] = a.p.conv_w[(int64_t)(taps - 2 - qq) * cp + ch];
+        w[k][q] = conv_w[(int64_t)(taps - 2 - qq) * cp + ch];
       }
     }
+    asm volatile("" ::: "memory");
+    others();
 #pragma unroll
     for (int k = 0; k < NIT; ++k) {
       const int i = tid + k * 256;
@@ -534,35 +574,40 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(SsmStepArgs a, SeqBatch b
 #pragma unroll
       for (int q = 0; q < HT; ++q) {
         if (q >= taps - 1) continue;
-        if (e.pos0 - 1 - q < 0) x[k][q] = 0.f;
+        if (pos0 - 1 - q < 0) x[k][q] = 0.f;
         acc = fmaf(w[k][q], x[k][q], acc);
       }
       put(i, acc);
-      if (i >= 2 * np || (h == grp * hpg && vs == 0)) {
-        const int ch = channel(i);
-#pragma unroll
-        for (int q = 0; q < HT; ++q)
-          if (q < taps - 1) hout[(int64_t)q * cp + ch] = q == 0 ? cur[k] : x[k][q > 0 ? q - 1 : 0];
-      }
     }
   } else {
+    const int taps = a.d.taps;
+    others();
     for (int i = tid; i < total; i += 256) {
       const int ch = channel(i);
-      const float cur = Act<TI>::ld(row + a.in.c_off + ch);
-      float acc = fmaf(a.p.conv_w[(int64_t)(taps - 1) * cp + ch], cur, a.p.conv_b[ch]);
-      const bool owner = i >= 2 * np || (h == grp * hpg && vs == 0);
+      const float cur = Act<TI>::ld(in_c + ch);
+      float acc = fmaf(conv_w[(int64_t)(taps - 1) * cp + ch], cur, conv_b[ch]);
+      const bool owner = i >= 2 * np || (blockIdx.y == 0 && vs == 0);
       float prev = cur;
       for (int q = 0; q < taps - 1; ++q) {   // the input q + 1 tokens back
-        const float x = e.pos0 - 1 - q >= 0 ? hin[(int64_t)q * cp + ch] : 0.f;
-        acc = fmaf(a.p.conv_w[(int64_t)(taps - 2 - q) * cp + ch], x, acc);
+        const float x = pos0 - 1 - q >= 0 ? hin[(int64_t)q * cp + ch] : 0.f;
+        acc = fmaf(conv_w[(int64_t)(taps - 2 - q) * cp + ch], x, acc);
         if (owner) hout[(int64_t)q * cp + ch] = prev;
         prev = x;
       }
       put(i, acc);
     }
   }
-  const float dt = softplus_f32(dtz), da = expf(A * dt);
+  if (wave == 2) {
+    const float t = softplus_f32(ex + dt_bias);
+    step[0] = t;
+    step[1] = expf(per_head * t);
+  } else if (wave == 3) {
+    ex = silu_f32(ex);
+  }
+  asm volatile("" : "+v"(ex));   // (here, not behind the barriers)
   __syncthreads();
+  const float dt = step[0], da = step[1];
+  float* sout = a.s.state + (int64_t)e.state_out * a.s.pool_stride + so;
 #pragma unroll
   for (int vt = 0; vt < VT; ++vt) {
     const float4 x = *reinterpret_cast<const float4*>(xs + vt * 16 + v4);
@@ -580,22 +625,30 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(SsmStepArgs a, SeqBatch b
         y = make_float4(fmaf(cn, s.x, y.x), fmaf(cn, s.y, y.y), fmaf(cn, s.z, y.z), fmaf(cn, s.w, y.w));
       }
     }
-#pragma unroll
-    for (int o = 4; o < 64; o <<= 1) {
-      y.x += __shfl_xor(y.x, o, 64); y.y += __shfl_xor(y.y, o, 64); y.z += __shfl_xor(y.z, o, 64); y.w += __shfl_xor(y.w, o, 64);
-    }
+    y = make_float4(sum_stride4(y.x), sum_stride4(y.y), sum_stride4(y.z), sum_stride4(y.w));
     if (lane < 4) *reinterpret_cast<float4*>(&red[wave][vt * 16 + v4]) = y;
   }
   __syncthreads();
-  if (tid < VT * 16) {
-    const int col = h * a.d.vdp + vs * 16 + tid;
-    const float yy = fmaf(D, xs[tid], (red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid]));
-    const float g = yy * silu_f32(Act<TI>::ld(row + col));
-    a.g[(int64_t)blockIdx.y * inner + col] = g;
+  if (fin >= 0 && fin < VT * 16) {
+    const float yy = fmaf(per_head, xs[fin], (red[0][fin] + red[1][fin]) + (red[2][fin] + red[3][fin]));
+    const float g = yy * ex;
+    a.g[(int64_t)seq * inner + col] = g;
     float s = g * g;
 #pragma unroll
     for (int o = 1; o < 16; o <<= 1) s += __shfl_xor(s, o, 16);
-    if ((tid & 15) == 0) a.ssq[(int64_t)blockIdx.y * (inner >> 4) + h * nvs + vs + (tid >> 4)] = s;
+    if ((fin & 15) == 0) a.ssq[(int64_t)seq * (inner >> 4) + h * nvs + vs + (fin >> 4)] = s;
+  }
+  if (few_taps) {
+#pragma unroll
+    for (int k = 0; k < NIT; ++k) {
+      const int i = tid + k * 256;
+      if (i < total && (i >= 2 * np || (blockIdx.y == 0 && vs == 0))) {
+        const int ch = channel(i);
+#pragma unroll
+        for (int q = 0; q < HT; ++q)
+          if (q < taps - 1) hout[(int64_t)q * cp + ch] = q == 0 ? cur[k] : x[k][q > 0 ? q - 1 : 0];
+      }
+    }
   }
 }
 
@@ -800,14 +853,31 @@ void launch_ssm_step(const SsmStepArgs& a, const SeqBatch& b, hipStream_t st) {
   // 10.4 -> 9.0 us at 4 sequences of the 8B widths, 11.4 -> 10.0 at 16 of the 0.6B ones, in stacks of 2 to 28 layers; 268 MB: 59.7 -> 50.8).  Smaller ones
   // are still there in the next step (2 MB 6.6 against 7.2 us past the caches, 8 MB 7.4 against 8.1).
   const bool past = (int64_t)b.n * a.d.heads * a.d.vdp * a.d.np * 4 >= 16 << 20;
-  const dim3 grid((unsigned)(a.d.heads * nvs / (wide ? 4 : 1)), (unsigned)b.n), block(256);
+  const int hpg = a.d.heads / a.d.groups;
+  const dim3 grid((unsigned)(nvs / (wide ? 4 : 1)), (unsigned)hpg, (unsigned)(a.d.groups * b.n)), block(256);
+  const SsmStepLead lead{a.d.np | std::min(a.d.taps, 63) << 10 | hpg << 16, a.d.vdp | a.d.groups << 16};
   auto go = [&](auto ni) {
     constexpr int NI = decltype(ni)::value;
-    auto run = [&](auto vt, auto nt) {
+    auto launch = [&](auto ti, auto vt, auto nt, auto one) {
+      using TI = decltype(ti);
       constexpr int VT = decltype(vt)::value;
-      constexpr bool NT = decltype(nt)::value;
-      if (a.in_f32) hipLaunchKernelGGL((ssm_step_kernel<float, NI, VT, NT>), grid, block, 0, st, a, b);
-      else hipLaunchKernelGGL((ssm_step_kernel<bf16_t, NI, VT, NT>), grid, block, 0, st, a, b);
+      constexpr bool NT = decltype(nt)::value, ONE = decltype(one)::value;
+      const float *sin = a.s.state, *hin = a.h.hist;
+      const TI* in_c = (const TI*)a.in.p + a.in.c_off;
+      if (ONE) {
+        sin += (int64_t)b.one.state_in * a.s.pool_stride;
+        hin += (int64_t)b.one.slot * a.h.slot_stride + (int64_t)b.one.hist_in * (a.d.taps - 1) * a.d.cp();
+        in_c += (int64_t)b.one.row0 * a.in.ld;
+      }
+      hipLaunchKernelGGL((ssm_step_kernel<TI, NI, VT, NT, ONE>), grid, block, 0, st, sin, in_c, hin, a.p.conv_w, a.p.conv_b, a.d.inner(), lead.np_taps_hpg, lead.vdp_groups, b.one.pos0, a, b);
+    };
+    auto run = [&](auto vt, auto nt) {
+      auto typed = [&](auto ti) {
+        if (b.has_one && a.d.taps >= 2 && a.d.taps <= 5) launch(ti, vt, nt, std::true_type{});
+        else launch(ti, vt, nt, std::false_type{});
+      };
+      if (a.in_f32) typed(float{});
+      else typed(bf16_t{});
     };
     if (!wide) run(std::integral_constant<int, 1>{}, std::false_type{});
     else if (past) run(std::integral_constant<int, 4>{}, std::true_type{});
