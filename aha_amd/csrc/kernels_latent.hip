@@ -32,28 +32,51 @@ __device__ __forceinline__ T* cache_row(const LatentCache& c, const LatentDims& 
   return reinterpret_cast<T*>(c.tab[(int64_t)slot * c.ld + pos / KV_PAGE_TOKENS] + c.off) + (int64_t)(pos % KV_PAGE_TOKENS) * d.ldc();
 }
 
-// the token's cache row: latent normed, key part rotated (256 threads; red: 4 floats, not reused before the next barrier)
+// the token's cache row: latent normed, key part rotated (256 threads; red: 4 floats, not reused before the next barrier).  All that a row of up to 1024 and
+// 256 columns takes is requested before its sum.
 template <typename TI, typename T>
 __device__ __forceinline__ void append_row(const LatentPostArgs& a, const SeqEntry& e, int r, int pos, const float2* cs, float* red) {
+  constexpr int NV = 4;
   const int tid = threadIdx.x, half = a.d.rot >> 1;
   const TI* kv = (const TI*)a.in + (int64_t)r * a.ld + a.kv_off;
+  const bf16_t* nw = (const bf16_t*)a.norm_w;
+  float v[NV], w[NV], u0 = 0.f, u1 = 0.f;
+  float2 t0 = make_float2(0.f, 0.f);
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    v[j] = w[j] = 0.f;
+    if (j * 256 < a.d.rank) {
+      const int i = min(tid + j * 256, a.d.rank - 1);
+      v[j] = Act<TI>::ld(kv + i);
+      w[j] = bf2f(nw[i]);
+    }
+  }
+  auto key_part = [&](int i, float& x0, float& x1, float2& t) {
+    const int k = i < half ? i : i - half;
+    x0 = Act<TI>::ld(kv + a.d.rp + k);
+    x1 = Act<TI>::ld(kv + a.d.rp + k + half);
+    t = cs[k];
+  };
+  if (tid < a.d.rot) key_part(tid, u0, u1, t0);
   T* out = cache_row<T>(a.c, a.d, e.slot, pos);
   float s = 0.f;
-  for (int i = tid; i < a.d.rank; i += 256) {
-    const float v = Act<TI>::ld(kv + i);
-    s = fmaf(v, v, s);
+#pragma unroll
+  for (int j = 0; j < NV; ++j)
+    if (tid + j * 256 < a.d.rank) s = fmaf(v[j], v[j], s);
+  for (int i = tid + NV * 256; i < a.d.rank; i += 256) {
+    const float x = Act<TI>::ld(kv + i);
+    s = fmaf(x, x, s);
   }
   const float rinv = 1.0f / sqrtf(block_sum_n<256>(s, red) / (float)a.d.rank + a.eps);
-  for (int i = tid; i < a.d.rp; i += 256) Act<T>::st(out + i, i < a.d.rank ? Act<TI>::ld(kv + i) * rinv * bf2f(((const bf16_t*)a.norm_w)[i]) : 0.f);
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int i = tid + j * 256;
+    if (i < a.d.rp) Act<T>::st(out + i, i < a.d.rank ? v[j] * rinv * w[j] : 0.f);
+  }
+  for (int i = tid + NV * 256; i < a.d.rp; i += 256) Act<T>::st(out + i, i < a.d.rank ? Act<TI>::ld(kv + i) * rinv * bf2f(nw[i]) : 0.f);
   for (int i = tid; i < a.d.tp; i += 256) {
-    float o = 0.f;
-    if (i < a.d.rot) {
-      const int k = i < half ? i : i - half;
-      const float u = Act<TI>::ld(kv + a.d.rp + k), v = Act<TI>::ld(kv + a.d.rp + k + half);
-      const float2 t = cs[k];
-      o = i < half ? u * t.x - v * t.y : v * t.x + u * t.y;
-    }
-    Act<T>::st(out + a.d.rp + i, o);
+    if (i >= 256 && i < a.d.rot) key_part(i, u0, u1, t0);
+    Act<T>::st(out + a.d.rp + i, i >= a.d.rot ? 0.f : i < half ? u0 * t0.x - u1 * t0.y : u1 * t0.x + u0 * t0.y);
   }
 }
 
@@ -76,45 +99,51 @@ __global__ __launch_bounds__(256) void latent_post_kernel(LatentPostArgs a, SeqB
   if (a.kv_off >= 0) append_row<TI, T>(a, e, r, pos, cs, red);
 }
 
-// One token per sequence: blocks (64 latent dims, head, 16 sequences) as heads_gemm_kernel, the first of a head's blocks rotates its queries; the
-// blocks behind the last head append the cache rows.
+// One token per sequence: blocks (64 latent dims, head, 16 sequences) as heads_gemm_kernel, a head's blocks rotate its queries between them; the blocks
+// behind the last head append the cache rows, one each.  A chain of waits at these sizes: the rotation's inputs are requested in front of the product, and
+// what the first requests take is in the leading arguments (0.6B widths, one sequence: 4.1 -> 3.9 us; 8B,
+// 32 sequences: 7.0 -> 5.0).
 template <typename TI>
-__global__ __launch_bounds__(256) void latent_query_kernel(LatentQueryArgs a, SeqBatch b) {
-  __shared__ float red[2][4];
-  const LatentDims& d = a.p.d;
-  const int tid = threadIdx.x, h = blockIdx.y, m0 = blockIdx.z * 16, half = d.rot >> 1, rows = b.n;
-  const float2* rope = reinterpret_cast<const float2*>(a.p.rope);
-  if (h == d.heads) {
-    int flip = 0;
-    for (int r = m0 + blockIdx.x; r < min(m0 + 16, rows); r += gridDim.x, flip ^= 1) {
-      const SeqEntry e = seq_entry_at(b, r);
-      append_row<TI, bf16_t>(a.p, e, r, e.pos0, rope + (int64_t)r * half, red[flip]);
-    }
+__global__ __launch_bounds__(256) void latent_query_kernel(const TI* in, const bf16_t* w_ukt, const float2* rope, int ld, int heads, int rp, int dp, int tp, int rot, int rows, LatentQueryArgs a, SeqBatch b) {
+  __shared__ float red[4];
+  const int tid = threadIdx.x, h = blockIdx.y, m0 = blockIdx.z * 16, half = rot >> 1, nx = rp >> 6;
+  if (h >= heads) {
+    const int r = m0 + (h - heads) * nx + blockIdx.x;
+    if (r >= min(m0 + 16, rows)) return;
+    const SeqEntry e = seq_entry_at(b, r);
+    append_row<TI, bf16_t>(a.p, e, r, e.pos0, rope + (int64_t)r * half, red);
     return;
   }
-  const TI* in = (const TI*)a.p.in + h * d.qd();
+  in += (int64_t)h * (dp + tp);
   const int lane = tid & 63, wave = tid >> 6, G = lane >> 4, c = lane & 15, n0 = blockIdx.x * 64 + wave * 16;
-  const bf16_t* w = (const bf16_t*)a.w_ukt + ((int64_t)h * d.rp + n0 + c) * d.dp + G * 8;
-  const TI* x = in + (int64_t)min(m0 + c, rows - 1) * a.p.ld + G * 8;
+  const bf16_t* w = w_ukt + ((int64_t)h * rp + n0 + c) * dp + G * 8;
+  const TI* x = in + (int64_t)min(m0 + c, rows - 1) * ld + G * 8;
+  float u = 0.f, v = 0.f;
+  float2 t = make_float2(0.f, 0.f);
+  auto request = [&](int i) {
+    const int rr = (unsigned)i / (unsigned)tp, j = i - rr * tp, r = m0 + rr;
+    if (j < rot) {
+      const int k = j < half ? j : j - half;
+      const TI* q = in + (int64_t)r * ld + dp;
+      u = Act<TI>::ld(q + k);
+      v = Act<TI>::ld(q + k + half);
+      t = rope[(int64_t)r * half + k];
+    }
+  };
+  const int turns = min(16, rows - m0) * tp;
+  int i = blockIdx.x * 256 + tid;
+  if (i < turns) request(i);
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
-  for (int k = 0; k < d.dp; k += 32) {
+  for (int k = 0; k < dp; k += 32) {
     const float4 lo = Act<TI>::ld4(x + k), hi = Act<TI>::ld4(x + k + 4);
     acc = mfma16(as_frag(ld16(w + k)), as_frag(u32x4_t{pack_bf(lo.x, lo.y), pack_bf(lo.z, lo.w), pack_bf(hi.x, hi.y), pack_bf(hi.z, hi.w)}), acc);
   }
-  if (m0 + c < rows) *reinterpret_cast<uint2*>((bf16_t*)a.qa + ((int64_t)(m0 + c) * d.heads + h) * d.rp + n0 + G * 4) = make_uint2(pack_bf(acc[0], acc[1]), pack_bf(acc[2], acc[3]));
-  if (blockIdx.x != 0) return;
-  for (int i = tid; i < min(16, rows - m0) * d.tp; i += 256) {
-    const int rr = i / d.tp, j = i - rr * d.tp, r = m0 + rr;
-    float o = 0.f;
-    if (j < d.rot) {
-      const int k = j < half ? j : j - half;
-      const TI* q = in + (int64_t)r * a.p.ld + d.dp;
-      const float u = Act<TI>::ld(q + k), v = Act<TI>::ld(q + k + half);
-      const float2 t = rope[(int64_t)r * half + k];
-      o = j < half ? u * t.x - v * t.y : v * t.x + u * t.y;
-    }
-    ((bf16_t*)a.qr)[((int64_t)r * d.heads + h) * d.tp + j] = f2bf(o);
+  if (m0 + c < rows) *reinterpret_cast<uint2*>((bf16_t*)a.qa + ((int64_t)(m0 + c) * heads + h) * rp + n0 + G * 4) = make_uint2(pack_bf(acc[0], acc[1]), pack_bf(acc[2], acc[3]));
+  for (; i < turns; i += nx * 256) {
+    if (i >= nx * 256) request(i);
+    const int rr = (unsigned)i / (unsigned)tp, j = i - rr * tp;
+    ((bf16_t*)a.qr)[((int64_t)(m0 + rr) * heads + h) * tp + j] = f2bf(j >= rot ? 0.f : j < half ? u * t.x - v * t.y : v * t.x + u * t.y);
   }
 }
 
@@ -437,39 +466,155 @@ __global__ __launch_bounds__(LD_NT) void latent_decode_kernel(LatentDecodeArgs a
   if (wave == 0 && G == 0) *reinterpret_cast<float2*>(a.part_ml + at * 2) = make_float2(m, l);
 }
 
+// The same for rp of 128, 256 or 512 and tp of 32 or 64, where a tile's keys and its sums fit one wave: every wave takes tiles of its own, requested at once
+// -- no barrier, no exchange of scores and no wait of one tile for another until the four waves' sums meet in LDS.  (Four waves on one tile at a time,
+// 4096 positions at rp 256: 8.9 us, 7.1 now; 32 sequences of 100 at rp 512: 10.6, 10.5.)
+// ONE: one sequence, its places in the leading arguments, which are in registers before the first instruction; else from the batch's table.
+__host__ __device__ inline bool latent_waves_ok(const LatentDims& d) { return (d.rp == 128 || d.rp == 256 || d.rp == 512) && (d.tp == 32 || d.tp == 64); }
+__host__ __device__ constexpr int latent_waves_lds(int ldc) { return ldc / 32 * 1024 * 2 * 4 + 4 * 16 * 8; }   // (the sums: rp / 4 KB, fewer)
+template <int RS, int TS, bool ONE>   // 32-dim blocks of the latent and of the key part
+__global__ __launch_bounds__(LD_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void latent_waves_kernel(const bf16_t* qa, const bf16_t* qr, const uint64_t* tab, uint64_t off, int heads, int pos, int lo,
+                                                                                                        int nsplit, float scale, LatentDecodeArgs a, SeqBatch b) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  constexpr int KS = RS + TS, rp = RS * 32, tp = TS * 32, ldc = rp + tp;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), G = lane >> 4, c = lane & 15;
+  const int split = blockIdx.x, hg = blockIdx.y, seq = ONE ? 0 : blockIdx.z, head = min(hg * 16 + c, heads - 1);
+  if constexpr (!ONE) {
+    const SeqEntry e = seq_entry_at(b, seq);
+    tab += (int64_t)e.slot * a.c.ld;
+    pos = e.pos0;
+    lo = a.d.first(pos);
+    qa += (int64_t)seq * heads * rp;
+    qr += (int64_t)seq * heads * tp;
+  }
+  const int tl0 = lo >> 5, nt = (pos >> 5) - tl0 + 1, per = (nt + nsplit - 1) / nsplit;
+  const int ta = tl0 + min(split * per, nt), tb = tl0 + min((split + 1) * per, nt);
+  char* const ks = smem + wave * (KS * 2048);   // [2 halves of 16 positions][KS] fragments
+  const int own = ta + wave;
+  uint64_t base = own < tb ? tab[own >> 1] + off : 0;
+  qa += (int64_t)head * rp + G * 8;
+  qr += (int64_t)head * tp + G * 8;
+  f32x4_t o[RS * 2];
+#pragma unroll
+  for (int i = 0; i < RS * 2; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  const int tr_row = G * 4 + (c >> 2), tr_col = (c & 3) * 4;
+  for (int tile = own; tile < tb; tile += 4) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (the stage's reads are done)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int p = min((tile >> 1) * 64 + (tile & 1) * 32 + u * 16 + c, pos) & 63;   // (positions behind the newest: its row)
+      const uint64_t src = base + (uint32_t)(p * ldc + G * 8) * 2u;
+#pragma unroll
+      for (int k4 = 0; k4 < KS; ++k4) __builtin_amdgcn_global_load_lds((glb_ptr_t)(src + k4 * 64), (lds_ptr_t)(ks + (u * KS + k4) * 1024), 16, 0, 0);
+    }
+    bf16x8_t q[KS];   // (for every tile again: 512 dims of them and of the sums are more registers than a wave has)
+#pragma unroll
+    for (int k4 = 0; k4 < KS; ++k4) q[k4] = as_frag(ld16(k4 < RS ? qa + k4 * 32 : qr + (k4 - RS) * 32));
+    if (tile + 4 < tb) base = tab[(tile + 4) >> 1] + off;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    f32x4_t x[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int k4 = 0; k4 < KS; ++k4)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) x[u] = mfma16(as_frag(*reinterpret_cast<const u32x4_t*>(ks + ((u * KS + k4) * 64 + lane) * 16)), q[k4], x[u]);
+    float sc[8];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int p = tile * 32 + u * 16 + G * 4 + r;
+        sc[u * 4 + r] = p >= lo && p <= pos ? x[u][r] * (scale * LOG2E) : -INFINITY;
+      }
+    float tm = sc[0];
+#pragma unroll
+    for (int j = 1; j < 8; ++j) tm = fmaxf(tm, sc[j]);
+    tm = group_max(tm);                          // (a tile of the range holds at least one visible position)
+    const float mn = fmaxf(m, tm), al = __builtin_amdgcn_exp2f(m - mn);
+    float p[8], sum = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      p[j] = __builtin_amdgcn_exp2f(sc[j] - mn);
+      sum += p[j];
+    }
+    l = l * al + sum;
+    m = mn;
+    const bf16x8_t pf = as_frag(u32x4_t{pack_bf(p[0], p[1]), pack_bf(p[2], p[3]), pack_bf(p[4], p[5]), pack_bf(p[6], p[7])});
+#pragma unroll
+    for (int i = 0; i < RS * 2; ++i) {
+      const int n = i * 16 + tr_col;
+      const char* at = ks + (((n >> 5) * 64 + ((n >> 3) & 3) * 16 + tr_row) * 16) + (n & 7) * 2;
+      union { tr4_t t[2]; u32x4_t u; } v;
+      v.t[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_t)at);
+      v.t[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_t)(at + KS * 1024));
+      o[i] = mfma16(as_frag(v.u), pf, o[i] * al);
+    }
+  }
+  l = group_sum(l);
+  // the waves' sums over the stages: [wave][16-dim tile][lane]
+  float2* const ml = reinterpret_cast<float2*>(smem + KS * 8192);
+  if (G == 0) ml[wave * 16 + c] = make_float2(m, l);
+  __syncthreads();   // everyone is past its stage
+  float M = -INFINITY, L = 0.f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) M = fmaxf(M, ml[w * 16 + c].x);
+  const float from = M == -INFINITY ? 0.f : M;   // (waves without a tile: exp2(-inf) of nothing)
+#pragma unroll
+  for (int w = 0; w < 4; ++w) L = fmaf(ml[w * 16 + c].y, __builtin_amdgcn_exp2f(ml[w * 16 + c].x - from), L);
+  const float f = __builtin_amdgcn_exp2f(m - from);
+#pragma unroll
+  for (int i = 0; i < RS * 2; ++i) *reinterpret_cast<f32x4_t*>(smem + ((wave * RS * 2 + i) * 64 + lane) * 16) = o[i] * f;
+  __syncthreads();
+  if (hg * 16 + c >= heads) return;
+  const int64_t at = ((int64_t)seq * nsplit + split) * heads + head;
+#pragma unroll
+  for (int j = 0; j < RS / 2; ++j) {
+    const int i = j * 4 + wave;
+    f32x4_t v = *reinterpret_cast<const f32x4_t*>(smem + (i * 64 + lane) * 16);
+#pragma unroll
+    for (int w = 1; w < 4; ++w) v += *reinterpret_cast<const f32x4_t*>(smem + ((w * RS * 2 + i) * 64 + lane) * 16);
+    *reinterpret_cast<f32x4_t*>(a.part_o + at * rp + i * 16 + G * 4) = v;
+  }
+  if (wave == 0 && G == 0) *reinterpret_cast<float2*>(a.part_ml + at * 2) = make_float2(M, L);
+}
+
 // Block (head, 32 rows of its W_uv, sequence): the splits' latent sums joined into LDS, then eight rows per wave.  wuv null: the joined sums
 template <int RQ>   // rp / 256, rounded up
-__global__ __launch_bounds__(256) void latent_merge_kernel(LatentMergeArgs a) {
+__global__ __launch_bounds__(256) void latent_merge_kernel(const float* part_o, const float* part_ml, const bf16_t* wuv, int nsplit, int heads, int rp, int vp, LatentMergeArgs a) {
   __shared__ float lat[RQ * 256], wt[LATENT_MAX_SPLIT];
-  const int h = blockIdx.x, n = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, rp = a.d.rp, heads = a.d.heads;
-  const int64_t at = (int64_t)n * a.nsplit * heads + h;
+  const int h = blockIdx.x, n = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int64_t at = (int64_t)n * nsplit * heads + h;
   const int row0 = blockIdx.y * 32 + wave * 8;
   constexpr int RC = (RQ + 1) / 2;   // 16-byte pieces of a W_uv row per lane
-  u32x4_t w[8][RC];
-  if (a.wuv) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-#pragma unroll
-      for (int q = 0; q < RC; ++q) w[j][q] = ld16((const bf16_t*)a.wuv + ((int64_t)h * a.d.vp + row0 + j) * rp + min((q * 64 + lane) * 8, rp - 8));
-  }
-  // The splits' sums, 32 of them requested at once and ahead of the weights that join them (one after the other behind the weights' barrier, the 64 of
-  // a 4096-position window made the launch 8.8 us; 6.6 now).  Past the end the last one again, never used.
-  constexpr int NB = RQ <= 2 ? 32 : 16;
-  const char* part = reinterpret_cast<const char*>(a.part_o + at * rp);
+  float2 ml = make_float2(-INFINITY, 0.f);
+  if (tid < nsplit) ml = *reinterpret_cast<const float2*>(part_ml + (at + (int64_t)tid * heads) * 2);   // (nsplit <= 64: wave 0)
+  // The splits' sums, up to 64 of them requested at once and ahead of the weights that join them (one after the other behind the weights' barrier, the 64 of
+  // a 4096-position window made the launch 8.8 us, 32 at a time 5.7; 4.4 now, in 43 splits).  Eight at a time are skipped behind the end; the last one again within.
+  constexpr int NB = RQ == 1 ? 64 : RQ == 2 ? 32 : 16;
+  const char* part = reinterpret_cast<const char*>(part_o + at * rp);
   uint32_t col[RQ];   // (byte offsets: LATENT_MAX_SPLIT x heads x rp floats, latent_decode_ok)
   float v[RQ][NB];
   auto request = [&](int s0) {
 #pragma unroll
-    for (int j = 0; j < NB; ++j)
+    for (int j8 = 0; j8 < NB; j8 += 8) {
+      if (s0 + j8 >= nsplit) break;
 #pragma unroll
-      for (int q = 0; q < RQ; ++q) v[q][j] = *reinterpret_cast<const float*>(part + (col[q] + (uint32_t)(min(s0 + j, a.nsplit - 1) * heads * rp) * 4u));
+      for (int j = j8; j < j8 + 8; ++j)
+#pragma unroll
+        for (int q = 0; q < RQ; ++q) v[q][j] = *reinterpret_cast<const float*>(part + (col[q] + (uint32_t)(min(s0 + j, nsplit - 1) * heads * rp) * 4u));
+    }
   };
 #pragma unroll
   for (int q = 0; q < RQ; ++q) col[q] = (uint32_t)min(q * 256 + tid, rp - 1) * 4u;
   request(0);
+  u32x4_t w[8][RC];
+  if (wuv) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int q = 0; q < RC; ++q) w[j][q] = ld16(wuv + ((int64_t)h * vp + row0 + j) * rp + min((q * 64 + lane) * 8, rp - 8));
+  }
   if (tid < 64) {
-    float2 ml = make_float2(-INFINITY, 0.f);
-    if (lane < a.nsplit) ml = *reinterpret_cast<const float2*>(a.part_ml + (at + (int64_t)lane * heads) * 2);
     const float M = wave_max(ml.x), e = ml.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml.x - M), s = wave_sum(e * ml.y);
     wt[lane] = e / s;
   }
@@ -477,16 +622,20 @@ __global__ __launch_bounds__(256) void latent_merge_kernel(LatentMergeArgs a) {
   float sum[RQ];
 #pragma unroll
   for (int q = 0; q < RQ; ++q) sum[q] = 0.f;
-  for (int s0 = 0; s0 < a.nsplit; s0 += NB) {
+  for (int s0 = 0; s0 < nsplit; s0 += NB) {
     if (s0 > 0) request(s0);
 #pragma unroll
-    for (int q = 0; q < RQ; ++q)
+    for (int j8 = 0; j8 < NB; j8 += 8) {
+      if (s0 + j8 >= nsplit) break;
 #pragma unroll
-      for (int j = 0; j < NB; ++j) sum[q] = s0 + j < a.nsplit ? fmaf(wt[s0 + j], v[q][j], sum[q]) : sum[q];
+      for (int j = j8; j < j8 + 8; ++j)
+#pragma unroll
+        for (int q = 0; q < RQ; ++q) sum[q] = s0 + j < nsplit ? fmaf(wt[s0 + j], v[q][j], sum[q]) : sum[q];
+    }
   }
 #pragma unroll
   for (int q = 0; q < RQ; ++q) lat[q * 256 + tid] = q * 256 + tid < rp ? sum[q] : 0.f;
-  if (!a.wuv) {
+  if (!wuv) {
     for (int d = tid; d < rp; d += 256) ((bf16_t*)a.o)[((int64_t)n * heads + h) * rp + d] = f2bf(lat[d]);   // (own elements)
     return;
   }
@@ -513,7 +662,7 @@ __global__ __launch_bounds__(256) void latent_merge_kernel(LatentMergeArgs a) {
     u32x4_t v;
 #pragma unroll
     for (int j = 0; j < 4; ++j) v[j] = pack_bf(acc[2 * j], acc[2 * j + 1]);
-    *reinterpret_cast<u32x4_t*>((bf16_t*)a.o + (int64_t)n * a.ldo + h * a.d.vp + row0) = v;
+    *reinterpret_cast<u32x4_t*>((bf16_t*)a.o + (int64_t)n * a.ldo + h * vp + row0) = v;
   }
 }
 
@@ -562,9 +711,15 @@ void launch_latent_post(const LatentPostArgs& a, const SeqBatch& b, bool f32, hi
 
 void launch_latent_query(const LatentQueryArgs& a, const SeqBatch& b, hipStream_t st) {
   if (b.n <= 0) return;
-  const dim3 grid((unsigned)(a.p.d.rp / 64), (unsigned)(a.p.d.heads + (a.p.kv_off >= 0 ? 1 : 0)), (unsigned)((b.n + 15) / 16)), block(256);
-  if (a.p.in_f32) hipLaunchKernelGGL(latent_query_kernel<float>, grid, block, 0, st, a, b);
-  else hipLaunchKernelGGL(latent_query_kernel<bf16_t>, grid, block, 0, st, a, b);
+  const LatentDims& d = a.p.d;
+  const int nx = d.rp / 64, append = a.p.kv_off >= 0 ? (std::min(b.n, 16) + nx - 1) / nx : 0;
+  const dim3 grid((unsigned)nx, (unsigned)(d.heads + append), (unsigned)((b.n + 15) / 16)), block(256);
+  auto go = [&](auto ti) {
+    using TI = decltype(ti);
+    hipLaunchKernelGGL(latent_query_kernel<TI>, grid, block, 0, st, (const TI*)a.p.in, (const bf16_t*)a.w_ukt, (const float2*)a.p.rope, (int)a.p.ld, d.heads, d.rp, d.dp, d.tp, d.rot, b.n, a, b);
+  };
+  if (a.p.in_f32) go(float{});
+  else go(bf16_t{});
 }
 
 void launch_heads_gemm(const HeadsGemmArgs& a, bool f32, hipStream_t st) {
@@ -614,17 +769,40 @@ void launch_latent_prefill(const LatentPrefillArgs& a, const SeqBatch& b, hipStr
   });
 }
 
-int latent_decode_blocks_per_cu(const LatentDims& d) { return std::max(1, std::min(2, 160 * 1024 / latent_decode_lds(d))); }
+int latent_decode_blocks_per_cu(const LatentDims& d) { return std::max(1, std::min(2, 160 * 1024 / (latent_waves_ok(d) ? latent_waves_lds((int)d.ldc()) : latent_decode_lds(d)))); }
 bool latent_decode_ok(const LatentDims& d) { return d.rp <= 1024 && (int64_t)d.heads * d.rp < 1 << 24 && latent_decode_lds(d) <= 160 * 1024 && d.scale > 0.f; }
 
 void launch_latent_decode(const LatentDecodeArgs& a, const SeqBatch& b, hipStream_t st) {
   if (b.n <= 0) return;
-  const int lds = latent_decode_lds(a.d);
-  auto go = [&](auto nds) {
-    auto k = latent_decode_kernel<decltype(nds)::value>;
+  const bool waves = latent_waves_ok(a.d);
+  const int lds = waves ? latent_waves_lds((int)a.d.ldc()) : latent_decode_lds(a.d);
+  const dim3 grid((unsigned)a.nsplit, (unsigned)((a.d.heads + 15) / 16), (unsigned)b.n);
+  auto allow = [&](auto k) {
     if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    hipLaunchKernelGGL(k, dim3((unsigned)a.nsplit, (unsigned)((a.d.heads + 15) / 16), (unsigned)b.n), dim3(LD_NT), lds, st, a, b);
+    return k;
   };
+  if (waves) {
+    auto go = [&](auto rs, auto ts, auto one) {
+      constexpr bool ONE = decltype(one)::value;
+      auto k = allow(latent_waves_kernel<decltype(rs)::value, decltype(ts)::value, ONE>);
+      const int pos = b.one.pos0;
+      hipLaunchKernelGGL(k, grid, dim3(LD_NT), lds, st, (const bf16_t*)a.qa, (const bf16_t*)a.qr, a.c.tab + (ONE ? (int64_t)b.one.slot * a.c.ld : 0), a.c.off, a.d.heads, pos, a.d.first(pos),
+                         a.nsplit, a.d.scale, a, b);
+    };
+    auto by_rank = [&](auto ts, auto one) {
+      if (a.d.rp == 128) go(std::integral_constant<int, 4>{}, ts, one);
+      else if (a.d.rp == 256) go(std::integral_constant<int, 8>{}, ts, one);
+      else go(std::integral_constant<int, 16>{}, ts, one);
+    };
+    auto by_key = [&](auto one) {
+      if (a.d.tp == 32) by_rank(std::integral_constant<int, 1>{}, one);
+      else by_rank(std::integral_constant<int, 2>{}, one);
+    };
+    if (b.has_one) by_key(std::true_type{});
+    else by_key(std::false_type{});
+    return;
+  }
+  auto go = [&](auto nds) { hipLaunchKernelGGL(allow(latent_decode_kernel<decltype(nds)::value>), grid, dim3(LD_NT), lds, st, a, b); };
   if (a.d.rp <= 128) go(std::integral_constant<int, 2>{});
   else if (a.d.rp <= 256) go(std::integral_constant<int, 4>{});
   else if (a.d.rp <= 512) go(std::integral_constant<int, 8>{});
@@ -634,9 +812,12 @@ void launch_latent_decode(const LatentDecodeArgs& a, const SeqBatch& b, hipStrea
 void launch_latent_merge(const LatentMergeArgs& a, hipStream_t st) {
   if (a.n <= 0) return;
   const dim3 grid((unsigned)a.d.heads, (unsigned)(a.wuv ? a.d.vp / 32 : 1), (unsigned)a.n), block(256);
-  if (a.d.rp <= 256) hipLaunchKernelGGL(latent_merge_kernel<1>, grid, block, 0, st, a);
-  else if (a.d.rp <= 512) hipLaunchKernelGGL(latent_merge_kernel<2>, grid, block, 0, st, a);
-  else hipLaunchKernelGGL(latent_merge_kernel<4>, grid, block, 0, st, a);
+  auto go = [&](auto rq) {
+    hipLaunchKernelGGL(latent_merge_kernel<decltype(rq)::value>, grid, block, 0, st, a.part_o, a.part_ml, (const bf16_t*)a.wuv, a.nsplit, a.d.heads, a.d.rp, a.d.vp, a);
+  };
+  if (a.d.rp <= 256) go(std::integral_constant<int, 1>{});
+  else if (a.d.rp <= 512) go(std::integral_constant<int, 2>{});
+  else go(std::integral_constant<int, 4>{});
 }
 
 }  // namespace aha

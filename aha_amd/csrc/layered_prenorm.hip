@@ -249,12 +249,14 @@ SsmHist ssm_hist(const LayeredModel& l, const PWeights& W) { return SsmHist{l.d_
 SsmState ssm_state(const LayeredModel& l, const PWeights& W) { return SsmState{l.d_pool + W.state_off, l.pool_stride}; }
 LatentCache latent_cache(const LayeredModel& l, const PWeights& W) { return LatentCache{l.d_tab, (int64_t)l.tab_ld, W.kv_off}; }
 
-// KV splits of a decode launch: at least two 32-position tiles per block, and the blocks in one round over the CUs
+// KV splits of a decode launch: at least two 32-position tiles per block, the blocks in one round over the CUs, and none without a tile (129 tiles are 43
+// blocks of three, not 64).  Four tiles per block, one a wave, read their keys through too few CUs: 7.2 -> 8.0 us at 4096 positions, 5.1 -> 4.4 for the join.
 int latent_splits(const LatentDims& d, const SeqEntry* e, int n) {
   int nt = 1;
   for (int i = 0; i < n; ++i) nt = std::max(nt, (e[i].pos0 >> 5) - (d.first(e[i].pos0) >> 5) + 1);
   const int round = 256 * latent_decode_blocks_per_cu(d);
-  return std::max(1, std::min({LATENT_MAX_SPLIT, (nt + 1) / 2, round / std::max(1, n * ((d.heads + 15) / 16))}));
+  const int most = std::max(1, std::min({LATENT_MAX_SPLIT, (nt + 1) / 2, round / std::max(1, n * ((d.heads + 15) / 16))})), per = (nt + most - 1) / most;
+  return (nt + per - 1) / per;
 }
 
 // mixer over the rows of a step: h -> y

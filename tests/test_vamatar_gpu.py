@@ -582,6 +582,28 @@ def test_a_far_key_among_thousands(ctx, dtype):
         assert np.abs(o - outs[0]).max() < 0.3 * spread     # wherever the key is, it is found
 
 
+@pytest.mark.parametrize("rank,rot,window", [(256, 64, 0), (256, 20, 100), (512, 64, 0), (500, 32, 96), (128, 64, 33), (288, 64, 0)])
+def test_decoding_where_tiles_end(ctx, rank, rot, window):
+    """A wave per tile of 32 positions (ranks padded to 128, 256 and 512, key parts to 32 and 64; 288: four waves per tile): contexts that end in front of,
+    at and behind a tile, a round of four waves and a page, the sequences one by one and in one step, with a head group that is not full."""
+    cfg = config([att(heads=17, dim=32, rot_dim=rot, vdim=32, kv_rank=rank, window=window, scale=0.3, mlp=None)], dtype="bfloat16", cap=0.0)
+    w = vamatar_weights(cfg, seed=14)
+    ids = tokens(420, cfg.vocab_size, seed=15)
+    want = reference(cfg, w, ids)
+    at = [1, 31, 32, 33, 63, 64, 127, 128, 129, 256, 419]
+    with Model(ctx, cfg, w) as m:
+        seqs = [m.seq_open() for _ in at]
+        for s, p in zip(seqs, at):
+            m.forward_batch([(s, ids[:p], [])])
+            t = m.seq_open()
+            m.forward_batch([(t, ids[:p], [])])
+            one, _ = m.forward_batch([(t, ids[p:p + 1], [0])])
+            assert err(one, want[p:p + 1]) <= TOL["bfloat16"], p
+            m.seq_close(t)
+        got, _ = m.forward_batch([(s, ids[p:p + 1], [0]) for s, p in zip(seqs, at)])
+    assert err(got, want[at]) <= TOL["bfloat16"]
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 128, 200])
 def test_a_token_far_back_in_the_state(ctx, dtype, n):
