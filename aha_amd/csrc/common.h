@@ -62,6 +62,15 @@ __device__ __forceinline__ float wave_sum(float v) {
   v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x121 /* row_ror:1 */, 0xf, 0xf, false));
   return v;
 }
+// the sum over the four lanes of one lane & 15
+__device__ __forceinline__ float rows_sum(float v) {
+  unsigned u = __float_as_uint(v);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  u = __float_as_uint(v);
+  const auto q = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __uint_as_float(q[0]) + __uint_as_float(q[1]);
+}
 // the sum over each half of the wave, lanes 0-31 and 32-63 (the last steps of wave_sum)
 __device__ __forceinline__ float half_wave_sum(float v) {
   const unsigned u = __float_as_uint(v);

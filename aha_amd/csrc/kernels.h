@@ -245,6 +245,16 @@ bool gemm_takes_few_rows(const GemmArgs& a);   // (launch_gemm's choice; host on
 double gemm_skinny_plan(const GemmArgs& a, int* r8_out);
 int gemm_skinny_rounds(const GemmArgs& a, int r8);   // blocks of r8 * 8 weight rows over the CUs
 void launch_gemm_skinny(const GemmArgs& a, hipStream_t st);
+// z = up(A), y = down(PolyNorm(z)) for up to 16 rows in two launches; false: not these sizes, nothing is launched (launch_gemm, launch_polynorm_rows, launch_gemm)
+struct SkinnyPoly {
+  float* stats;                // gemm_skinny_poly_floats()
+  int parts;
+  float coef[4], eps, inv_ff;
+};
+bool gemm_skinny_poly_ok(const GemmArgs& up, const GemmArgs& down);
+size_t gemm_skinny_poly_floats();
+void launch_gemm_skinny_poly(const GemmArgs& up, const GemmArgs& down, SkinnyPoly p, hipStream_t st);
+bool gemm_takes_poly(const GemmArgs& up, const GemmArgs& down);   // gemm_skinny_poly_ok, and launch_gemm would take the few-row kernel for both
 // One launch over all row segments on the four-wave 256 x 256 / 256 x 192 kernels (plain and gate+up epilogues, whole K tiles, M >= 256);
 // any other shape: one launch_gemm per segment.  On the same kernel every output element is the same K-ordered sum as in an ungrouped GEMM over its
 // row; a short segment's own plan may be another (K slices, the few-row kernel).
@@ -485,7 +495,7 @@ struct PolyNormArgs {
   int rows;
 };
 void launch_polynorm_rows(const PolyNormArgs& a, bool f32, hipStream_t st);
-// C (M, N) f32 = A (M, K) f32 . W (N, K)^T bf16, true f32 products and sums (f32 MFMA); K a multiple of 32
+// C (M, N) f32 = A (M, K) f32 . W (N, K)^T bf16 on the bf16 matrix units, activations in three exact parts (skinny_body.h split_bf16); K a multiple of 32
 // batch > 1: that many products, the operands of one sa / sw / sc elements behind those of the one before
 void launch_gemm_f32(const float* A, int64_t lda, const void* W, int64_t ldw, float* C, int64_t ldc, int M, int N, int K, hipStream_t st, int batch = 1,
                      int64_t sa = 0, int64_t sw = 0, int64_t sc = 0);

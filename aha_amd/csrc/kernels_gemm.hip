@@ -1323,6 +1323,8 @@ bool gemm_takes_few_rows(const GemmArgs& a_in) {
   return gemm_skinny_ok(a) && takes_few_rows(a, plan_gemm(a), &r8);
 }
 
+bool gemm_takes_poly(const GemmArgs& up, const GemmArgs& down) { return gemm_skinny_poly_ok(up, down) && gemm_takes_few_rows(up) && gemm_takes_few_rows(down); }
+
 void launch_gemm(const GemmArgs& a_in, hipStream_t st) {
   if (a_in.M <= 0 || a_in.N <= 0) return;
   GemmArgs a = a_in;

@@ -28,8 +28,8 @@ namespace aha {
 
 namespace {
 
-template <int R8, int M8, bool PAIRS, bool DEEP>
-__global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const void* A, const void* W, int M, int N, int K, int64_t lda, int64_t ldw, GemmArgs a) {
+template <int R8, int M8, bool PAIRS, bool DEEP, typename PRO, typename EPI>
+__device__ __forceinline__ void skinny_product(const void* A, const void* W, int M, int N, int K, int64_t lda, int64_t ldw, GemmArgs& a, PRO pro, EPI epilogue) {
   // (what the first requests need: in scalar registers at the start, gemv_body.h)
   a.A = A;
   a.W = W;
@@ -38,8 +38,8 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const vo
   a.K = K;
   a.lda = lda;
   a.ldw = ldw;
-  constexpr int NF = (R8 + 1) / 2, MT = (M8 + 1) / 2, PER = R8 + M8;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), G = lane >> 4, c = lane & 15;
+  constexpr int PER = R8 + M8;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const char* src[PER];
 #pragma unroll
   for (int r = 0; r < PER; ++r) {
@@ -53,34 +53,143 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const vo
       src[r] = (const char*)a.W + (int64_t)min((int)blockIdx.x * (R8 * 8) + local, a.N - 1) * a.ldw * 2 + piece;
     }
   }
-  skinny_sums<R8, M8, false, DEEP>(src, a.K / 64, a.few_rows_spread && a.M <= 64 ? skinny_first((int)blockIdx.x * (R8 * 8), a.K / 64) : 0, gemm_smem, wave, lane);
-  for (int i = wave; i < NF * MT; i += SKINNY_WAVES) {
-    const int r = i / MT, m = (int)blockIdx.y * 64 + (i - r * MT) * 16 + c;
-    if (m >= a.M) continue;
-    if constexpr (PAIRS) {   // rows 0-7 of a fragment: gate, 8-15: up
-      if (G >= 2) continue;
-      const f32x4_t g = skinny_total<R8, M8>(gemm_smem, i, lane), p = skinny_total<R8, M8>(gemm_smem, i, lane + 32);
-      const float gt[4] = {g[0], g[1], g[2], g[3]}, up[4] = {p[0], p[1], p[2], p[3]};
-      const int oc = ((int)blockIdx.x * (R8 / 2) + r) * 8 + G * 4;
-      epi_pairs(a, m, 2 * oc, oc, gt, up);   // (oc < N / 2 decides)
-    } else {
-      const int local = r * 16 + G * 4, n = (int)blockIdx.x * (R8 * 8) + local;
-      if (local >= R8 * 8) continue;   // (odd R8: half a fragment)
-      const f32x4_t s = skinny_total<R8, M8>(gemm_smem, i, lane);
-      auto epi = [&](auto act) {
-        constexpr int ACT = decltype(act)::value;
-        if (a.bias && a.residual) epi_group<ACT, true, true>(a, m, n, s[0], s[1], s[2], s[3]);
-        else if (a.bias) epi_group<ACT, true, false>(a, m, n, s[0], s[1], s[2], s[3]);
-        else if (a.residual) epi_group<ACT, false, true>(a, m, n, s[0], s[1], s[2], s[3]);
-        else epi_group<ACT, false, false>(a, m, n, s[0], s[1], s[2], s[3]);
-      };
-      if (a.act == ACT_NONE) epi(std::integral_constant<int, ACT_NONE>{});
-      else if (a.act == ACT_PARTIAL_F32) epi_group<ACT_PARTIAL_F32, false, false>(a, m, n, s[0], s[1], s[2], s[3]);
-      else if (a.act == ACT_GELU_TANH) epi(std::integral_constant<int, ACT_GELU_TANH>{});
-      else if (a.act == ACT_GELU_ERF) epi(std::integral_constant<int, ACT_GELU_ERF>{});
-      else epi(std::integral_constant<int, ACT_SILU>{});
+  skinny_sums<R8, M8, false, DEEP>(src, a.K / 64, a.few_rows_spread && a.M <= 64 ? skinny_first((int)blockIdx.x * (R8 * 8), a.K / 64) : 0, gemm_smem, wave, lane, pro);
+  epilogue(wave, lane);
+}
+
+
+template <int R8, int M8, bool PAIRS, bool DEEP>
+__global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const void* A, const void* W, int M, int N, int K, int64_t lda, int64_t ldw, GemmArgs a) {
+  skinny_product<R8, M8, PAIRS, DEEP>(A, W, M, N, K, lda, ldw, a, SkinnyPlain{}, [&](int wave, int lane) {
+    constexpr int NF = (R8 + 1) / 2, MT = (M8 + 1) / 2;
+    const int G = lane >> 4, c = lane & 15;
+    for (int i = wave; i < NF * MT; i += SKINNY_WAVES) {
+      const int r = i / MT, m = (int)blockIdx.y * 64 + (i - r * MT) * 16 + c;
+      if (m >= a.M) continue;
+      if constexpr (PAIRS) {   // rows 0-7 of a fragment: gate, 8-15: up
+        if (G >= 2) continue;
+        const f32x4_t g = skinny_total<R8, M8>(gemm_smem, i, lane), p = skinny_total<R8, M8>(gemm_smem, i, lane + 32);
+        const float gt[4] = {g[0], g[1], g[2], g[3]}, up[4] = {p[0], p[1], p[2], p[3]};
+        const int oc = ((int)blockIdx.x * (R8 / 2) + r) * 8 + G * 4;
+        epi_pairs(a, m, 2 * oc, oc, gt, up);   // (oc < N / 2 decides)
+      } else {
+        const int local = r * 16 + G * 4, n = (int)blockIdx.x * (R8 * 8) + local;
+        if (local >= R8 * 8) continue;   // (odd R8: half a fragment)
+        const f32x4_t s = skinny_total<R8, M8>(gemm_smem, i, lane);
+        auto epi = [&](auto act) {
+          constexpr int ACT = decltype(act)::value;
+          if (a.bias && a.residual) epi_group<ACT, true, true>(a, m, n, s[0], s[1], s[2], s[3]);
+          else if (a.bias) epi_group<ACT, true, false>(a, m, n, s[0], s[1], s[2], s[3]);
+          else if (a.residual) epi_group<ACT, false, true>(a, m, n, s[0], s[1], s[2], s[3]);
+          else epi_group<ACT, false, false>(a, m, n, s[0], s[1], s[2], s[3]);
+        };
+        if (a.act == ACT_NONE) epi(std::integral_constant<int, ACT_NONE>{});
+        else if (a.act == ACT_PARTIAL_F32) epi_group<ACT_PARTIAL_F32, false, false>(a, m, n, s[0], s[1], s[2], s[3]);
+        else if (a.act == ACT_GELU_TANH) epi(std::integral_constant<int, ACT_GELU_TANH>{});
+        else if (a.act == ACT_GELU_ERF) epi(std::integral_constant<int, ACT_GELU_ERF>{});
+        else epi(std::integral_constant<int, ACT_SILU>{});
+      }
     }
+  });
+}
+
+// ---- PolyNorm between two few-row products ------------------------------------------------------------------------------------------------
+// A launch of its own between an up and a down projection of up to 16 rows is a link of the chain like any other, for 8 x 12288 numbers (4.9 us).  Here the
+// first product leaves, beside its bf16 result z, the sums of z^2, z^4 and z^6 over each block's columns, [block][M8 * 8 rows]; the second joins them while its
+// first stages are on their way and maps the fragments that it reads from LDS: three fma and a rounding per number, under the wait for the weights.
+// 8 rows, 12288 x 4096 and back: 17.0 + 4.9 + 16.8 us in three launches, 17.1 + 19.1 in two; 12 layers of 8B sizes, 8 requests and 32 steps 39.0 -> 38.0 ms.
+constexpr int POLY_PARTS = 256;   // blocks of the first product, at most
+template <int M8>
+struct SkinnyPolyIn {
+  static constexpr bool ON = true;
+  static constexpr int R = M8 * 8, PER = 64 / R, NL = POLY_PARTS / (PER * SKINNY_WAVES);
+  static_assert(M8 == 1 || M8 == 2, "one activation fragment");
+  const SkinnyPoly& p;
+  f32x4_t (*red)[16];   // [SKINNY_WAVES]
+  f32x4_t v[NL];
+  float r1 = 0.f, r2 = 0.f, r3 = 0.f, e = 0.f;
+  __device__ __forceinline__ SkinnyPolyIn(const SkinnyPoly& p_, f32x4_t (*red_)[16]) : p(p_), red(red_) {}
+  __device__ __forceinline__ int part(int j) const { return (j * SKINNY_WAVES + (int)(threadIdx.x >> 6)) * PER + (int)(threadIdx.x & 63) / R; }
+  __device__ __forceinline__ void request() {
+    const f32x4_t* at = reinterpret_cast<const f32x4_t*>(p.stats) + (threadIdx.x & (R - 1));
+#pragma unroll
+    for (int j = 0; j < NL; ++j) v[j] = at[min(part(j), p.parts - 1) * R];
   }
+  __device__ __forceinline__ void join() {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    f32x4_t mine = {0.f, 0.f, 0.f, 0.f};   // (all four, though the last is nothing: a loaded register that nobody reads is taken for something else, behind a wait for its load)
+#pragma unroll
+    for (int j = 0; j < NL; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) mine[i] += part(j) < p.parts ? v[j][i] : 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (R == 8) mine[i] += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(mine[i]), 0x128 /* row_ror:8 */, 0xf, 0xf, false));
+      mine[i] = rows_sum(mine[i]);
+    }
+    // The waves' sums meet in LDS by hand: what the compiler knows to touch LDS it lets wait for every stage on its way (and __syncthreads with it).
+    typedef __attribute__((address_space(3))) f32x4_t* lds_t;
+    const uint32_t at = (uint32_t)(uintptr_t)(lds_t)&red[0][lane & 15];
+    f32x4_t w0, w1, w2, w3;
+    asm volatile("ds_write_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::"v"(at + wave * 256), "v"(mine) : "memory");   // (the four lanes of one lane & 15: the same)
+    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:256\n\tds_read_b128 %2, %4 offset:512\n\tds_read_b128 %3, %4 offset:768\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(w0), "=&v"(w1), "=&v"(w2), "=&v"(w3)
+                 : "v"(at)
+                 : "memory");
+    const f32x4_t t = (w0 + w1) + (w2 + w3);
+    r1 = p.coef[0] / sqrtf(t[0] * p.inv_ff + p.eps);
+    r2 = p.coef[1] / sqrtf(t[1] * p.inv_ff + p.eps);
+    r3 = p.coef[2] / sqrtf(t[2] * p.inv_ff + p.eps);
+    e = p.coef[3];
+  }
+  __device__ __forceinline__ u32x4_t map(u32x4_t x) const {   // (pad columns become e: their weights are zero)
+    u32x4_t o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float lo = lo_bf(x[i]), hi = hi_bf(x[i]);
+      o[i] = pack_bf(fmaf(lo, fmaf(lo, fmaf(lo, r3, r2), r1), e), fmaf(hi, fmaf(hi, fmaf(hi, r3, r2), r1), e));
+    }
+    return o;
+  }
+};
+// IN: the second product, else the first.  bf16 results, no bias, residual or activation.
+template <int R8, int M8, bool DEEP, bool IN>
+__global__ __launch_bounds__(SKINNY_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1, 4))) void gemm_skinny_poly_kernel(const void* A, const void* W, int M, int N, int K, int64_t lda, int64_t ldw, SkinnyPoly p, GemmArgs a) {
+  constexpr int NF = (R8 + 1) / 2, R = M8 * 8;
+  __shared__ f32x4_t red[SKINNY_WAVES][16];
+  auto epilogue = [&](int wave, int lane) {
+    const int G = lane >> 4, c = lane & 15, local = wave * 16 + G * 4, n = (int)blockIdx.x * (R8 * 8) + local;
+    float t[3] = {0.f, 0.f, 0.f};
+    if (wave < NF) {
+      const f32x4_t s = skinny_total<R8, M8>(gemm_smem, wave, lane);
+      if (local < R8 * 8) {   // (odd R8: half a fragment)
+        if (c < a.M) epi_group<ACT_NONE, false, false>(a, c, n, s[0], s[1], s[2], s[3]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float z = n + j < a.N ? bf2f(f2bf(s[j])) : 0.f, z2 = z * z, z4 = z2 * z2;
+          t[0] += z2;
+          t[1] += z4;
+          t[2] = fmaf(z4, z2, t[2]);
+        }
+      }
+    }
+    if constexpr (!IN) {   // (rows past M: the last one's again)
+      if (wave < NF) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) t[i] = rows_sum(t[i]);
+        if (G == 0) red[wave][c] = f32x4_t{t[0], t[1], t[2], 0.f};
+      }
+      __syncthreads();
+      if (threadIdx.x < R) {
+        f32x4_t v = red[0][threadIdx.x];
+#pragma unroll
+        for (int r = 1; r < NF; ++r) v += red[r][threadIdx.x];
+        reinterpret_cast<f32x4_t*>(p.stats)[blockIdx.x * R + threadIdx.x] = v;
+      }
+    }
+  };
+  if constexpr (IN) skinny_product<R8, M8, false, DEEP>(A, W, M, N, K, lda, ldw, a, SkinnyPolyIn<M8>(p, red), epilogue);
+  else skinny_product<R8, M8, false, DEEP>(A, W, M, N, K, lda, ldw, a, SkinnyPlain{}, epilogue);
 }
 
 template <int R8, int M8, bool PAIRS, bool DEEP = false>
@@ -165,6 +274,50 @@ void launch_gemm_skinny(const GemmArgs& a, hipStream_t st) {
     else if (r8 == 4) launch_rows<4, false>(a, st);
     else launch_rows<6, false>(a, st);
   }
+}
+
+namespace {
+
+template <int R8, int M8, bool IN, bool DEEP = false>
+void launch_poly_one(const GemmArgs& a, const SkinnyPoly& p, hipStream_t st) {
+  if constexpr (!DEEP && skinny_stages(R8 + M8) != skinny_stages(R8 + M8, true))
+    if (gemm_skinny_rounds(a, R8) == 1) return launch_poly_one<R8, M8, IN, true>(a, p, st);
+  constexpr int lds = skinny_lds(R8, M8, false, DEEP);
+  auto k = gemm_skinny_poly_kernel<R8, M8, DEEP, IN>;
+  if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  hipLaunchKernelGGL(k, dim3((unsigned)((a.N + R8 * 8 - 1) / (R8 * 8))), dim3(SKINNY_WAVES * 64), lds, st, a.A, a.W, a.M, a.N, a.K, a.lda, a.ldw, p, a);
+}
+
+template <bool IN>
+void launch_poly(const GemmArgs& a, const SkinnyPoly& p, int r8, hipStream_t st) {
+  auto go = [&](auto r) {
+    if (a.M <= 8) launch_poly_one<decltype(r)::value, 1, IN>(a, p, st);
+    else launch_poly_one<decltype(r)::value, 2, IN>(a, p, st);
+  };
+  if (r8 == 2) go(std::integral_constant<int, 2>{});
+  else if (r8 == 3) go(std::integral_constant<int, 3>{});
+  else if (r8 == 4) go(std::integral_constant<int, 4>{});
+  else go(std::integral_constant<int, 6>{});
+}
+
+}  // namespace
+
+// K of 24 chunks and more: the deepest ring's first requests (skinny_sums)
+bool gemm_skinny_poly_ok(const GemmArgs& up, const GemmArgs& down) {
+  if (up.M > 16 || down.M != up.M || down.K != up.N || down.K < 24 * 64) return false;
+  int r8 = 2;
+  gemm_skinny_plan(up, &r8);
+  return (up.N + r8 * 8 - 1) / (r8 * 8) <= POLY_PARTS;
+}
+size_t gemm_skinny_poly_floats() { return (size_t)POLY_PARTS * 16 * 4; }
+
+void launch_gemm_skinny_poly(const GemmArgs& up, const GemmArgs& down, SkinnyPoly p, hipStream_t st) {
+  int r8 = 2;
+  gemm_skinny_plan(up, &r8);
+  p.parts = (up.N + r8 * 8 - 1) / (r8 * 8);
+  launch_poly<false>(up, p, r8, st);
+  gemm_skinny_plan(down, &r8);
+  launch_poly<true>(down, p, r8, st);
 }
 
 }  // namespace aha

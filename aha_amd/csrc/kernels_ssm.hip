@@ -475,12 +475,7 @@ __global__ __launch_bounds__(256) void ssm_segments_kernel(SsmScanArgs a, SeqBat
 __device__ __forceinline__ float sum_stride4(float v) {   // over the sixteen lanes of one lane & 3
   v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x124 /* row_ror:4 */, 0xf, 0xf, false));
   v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x128 /* row_ror:8 */, 0xf, 0xf, false));
-  unsigned u = __float_as_uint(v);
-  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  u = __float_as_uint(v);
-  const auto q = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return __uint_as_float(q[0]) + __uint_as_float(q[1]);
+  return rows_sum(v);
 }
 struct SsmStepLead {   // sizes in two words
   int np_taps_hpg, vdp_groups;

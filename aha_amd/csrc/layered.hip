@@ -341,6 +341,16 @@ Tail run_rows(aha_model* m, const SeqBatch& b, const SeqEntry* h_ents, const uin
     norm = W.norm1;
     if (d.mlp == AHA_MLP_NONE) continue;
     enter(li, 1);
+    const GemmArgs up = gemm_args(l.h, l.ld, W.wup, l.z, W.ffp, rows, W.ffp, (int)l.ld), down = gemm_args(l.z, W.ffp, W.wdown, l.y, l.ld, rows, (int)l.ld, W.ffp);
+    if (!l.f32 && gemm_takes_poly(up, down)) {
+      SkinnyPoly p{};
+      p.stats = l.zstats; p.eps = c.rms_norm_eps; p.inv_ff = 1.0f / (float)d.ff;
+      memcpy(p.coef, W.act, sizeof(p.coef));
+      ProfScope ps(m, "gemm", (double)rows * (2.0 * l.ld + 2.0 * W.ffp) * 2 + (double)l.ld * W.ffp * 4, 4.0 * rows * W.ffp * l.ld);
+      launch_gemm_skinny_poly(up, down, p, st);
+      norm = W.norm2;
+      continue;
+    }
     gemm(m, l.h, l.ld, W.wup, l.z, W.ffp, rows, W.ffp, (int)l.ld);
     {
       PolyNormArgs a{};
@@ -623,6 +633,7 @@ int layered_create(aha_model* m, const aha_tensor_view* w, size_t nw) {
     TRY(dev_alloc(m, (size_t)l.ld * 4, (void**)&l.x1, true));
     TRY(dev_alloc(m, (size_t)l.max_nqkv * 4, (void**)&l.qkv1, true));
     TRY(dev_alloc(m, (size_t)std::max(l.max_ffp, 64) * 4, (void**)&l.z1, true));
+    if (!l.f32) TRY(dev_alloc(m, gemm_skinny_poly_floats() * 4, (void**)&l.zstats, true));
   }
   TRY(ensure_rows(m, 1));
   TRY(ensure_entries(m, 1));

@@ -107,6 +107,7 @@ struct LayeredModel {
   unsigned* ctr = nullptr;
   // single-token buffers
   float *s1 = nullptr, *x1 = nullptr, *qkv1 = nullptr, *z1 = nullptr;
+  float* zstats = nullptr;   // PolyNorm between two few-row products (SkinnyPoly)
   void* act1 = nullptr;
   // logits of the last batch
   size_t last_want = 0;
@@ -189,6 +190,12 @@ inline int grow(aha_model* m, std::vector<void*>& owner, size_t bytes, void** ou
   return AHA_OK;
 }
 
+inline GemmArgs gemm_args(const void* A, int64_t lda, const void* W, void* C, int64_t ldc, int M, int N, int K, int act = ACT_NONE) {
+  GemmArgs g{};
+  g.A = A; g.W = W; g.C = C;
+  g.M = M; g.N = N; g.K = K; g.lda = lda; g.ldw = K; g.ldc = ldc; g.act = act;
+  return g;
+}
 inline void gemm(aha_model* m, const void* A, int64_t lda, const void* W, void* C, int64_t ldc, int M, int N, int K, int act = ACT_NONE) {
   const LayeredModel& l = *m->layered;
   ProfScope ps(m, "gemm", ((double)M * K + (double)M * N) * (l.f32 ? 4 : 2) + (double)N * K * 2, 2.0 * M * N * K);
@@ -196,10 +203,7 @@ inline void gemm(aha_model* m, const void* A, int64_t lda, const void* W, void* 
     launch_gemm_f32((const float*)A, lda, W, K, (float*)C, ldc, M, N, K, m->stream);
     return;
   }
-  GemmArgs g{};
-  g.A = A; g.W = W; g.C = C;
-  g.M = M; g.N = N; g.K = K; g.lda = lda; g.ldw = K; g.ldc = ldc; g.act = act;
-  launch_gemm(g, m->stream);
+  launch_gemm(gemm_args(A, lda, W, C, ldc, M, N, K, act), m->stream);
 }
 
 inline void keep_rows(aha_model* m, const float* x, int rows, int layer) {

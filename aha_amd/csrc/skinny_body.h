@@ -74,18 +74,30 @@ __device__ __forceinline__ f32x4_t split_sum(const f32x4_t& big, const f32x4_t& 
   return s;
 }
 
+// What a product does to its bf16 activations on the way from LDS: nothing
+struct SkinnyPlain {
+  static constexpr bool ON = false;
+  __device__ __forceinline__ void request() {}
+  __device__ __forceinline__ void join() {}
+  __device__ __forceinline__ u32x4_t map(u32x4_t x) const { return x; }
+};
+
 // src[r]: where this lane's piece of request r starts at k = 0 -- R8 weight groups (bf16), then M8 activation groups (bf16); F32: activations are f32,
 // a row's 64 k are two requests, the first halves of all groups before the second halves, and the activations' parts (split_bf16) multiply in turn.
 // nc: 64-wide k chunks, first: the chunk that wave 0 starts at (skinny_first), wrapping round behind the last.
 // On return the waves' sums of the 16 x 16 fragments (weight fragment r, activation fragment m) lie in LDS and every wave may read them
 // (skinny_total).
-template <int R8, int M8, bool F32 = false, bool DEEP = false>
-__device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R8, M8, F32)], int nc, int first, char* smem, int wave, int lane) {
+// pro: request() in front of the ring's first requests, join() behind them (with pro all of them are made: nc >= S * SKINNY_WAVES), map() on every fragment.
+template <int R8, int M8, bool F32 = false, bool DEEP = false, typename PRO = SkinnyPlain>
+__device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R8, M8, F32)], int nc, int first, char* smem, int wave, int lane, PRO pro = {}) {
   typedef __attribute__((address_space(3))) void* lds_t;
   typedef const __attribute__((address_space(1))) void* glb_t;
   constexpr int NF = (R8 + 1) / 2, MT = (M8 + 1) / 2, PER = skinny_requests(R8, M8, F32), S = skinny_stages(PER, DEEP);
   constexpr int LEFT = (S - 1) * PER;   // requests of the later stages
   static_assert(LEFT < 64, "vmcnt has six bits");
+  // Eight rows that are mapped: a fragment's columns 0-7 are their first 32 k of a chunk and columns 8-15 the second 32, so that nothing is mapped twice; what a
+  // product gives for the columns of the other half is nobody's, and the second half's sums move by eight lanes at the end.
+  constexpr bool HALVES = PRO::ON && M8 == 1;
   const int G = lane >> 4, c = lane & 15;
   char* ring = smem + wave * (S * PER * 1024);
   f32x4_t acc[2][NF][MT];   // the two halves of a chunk (F32: the upper parts and the others) in chains of their own: half the dependent steps, half the roundings in a row
@@ -134,10 +146,11 @@ __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R
         }
     } else {
       bf16x8_t af[2][MT];
+      if constexpr (HALVES) af[0][0] = af[1][0] = __builtin_bit_cast(bf16x8_t, pro.map(*reinterpret_cast<const u32x4_t*>(sa + skinny_swz(c & 7, (c >> 3) * 4 + G))));
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+      for (int h = 0; h < (HALVES ? 0 : 2); ++h)
 #pragma unroll
-        for (int m = 0; m < MT; ++m) af[h][m] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(sa + skinny_swz(m * 16 + (m + 1 == MT ? ca : c), h * 4 + G)));
+        for (int m = 0; m < MT; ++m) af[h][m] = __builtin_bit_cast(bf16x8_t, pro.map(*reinterpret_cast<const u32x4_t*>(sa + skinny_swz(m * 16 + (m + 1 == MT ? ca : c), h * 4 + G))));
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -149,9 +162,12 @@ __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R
     __builtin_amdgcn_sched_barrier(0);
   };
   int u = 0, ch = wave;
+  pro.request();
 #pragma unroll
   for (int s = 0; s < S; ++s)
-    if (wave + s * SKINNY_WAVES < nc) load(s, wave + s * SKINNY_WAVES);
+    if (PRO::ON || wave + s * SKINNY_WAVES < nc) load(s, wave + s * SKINNY_WAVES);
+  if constexpr (PRO::ON) __builtin_amdgcn_sched_barrier(0);
+  pro.join();
   for (; ch + S * SKINNY_WAVES < nc; ch += SKINNY_WAVES) {   // S stages are on their way: the oldest is in when the later ones' requests are left
     __builtin_amdgcn_s_waitcnt(0x0F70 | (LEFT & 15) | ((LEFT >> 4) << 14));
     __builtin_amdgcn_sched_barrier(0);
@@ -180,6 +196,11 @@ __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R
   __builtin_amdgcn_s_waitcnt(0x0F70);   // no DMA may land in what becomes the sums' space
   __syncthreads();
   auto red = reinterpret_cast<f32x4_t(*)[NF * MT][64]>(smem);
+  if constexpr (HALVES)
+#pragma unroll
+    for (int r = 0; r < NF; ++r)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[1][r][0][i] = __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(acc[1][r][0][i]), 0x128 /* row_ror:8 */, 0xf, 0xf, false));
 #pragma unroll
   for (int r = 0; r < NF; ++r)
 #pragma unroll

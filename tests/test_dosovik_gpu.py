@@ -152,6 +152,21 @@ def test_32_bit_products_of_every_tile(ctx, rows, ff, vocab):
         assert err(all_logits(m, ids), want) <= TOL["float32"]
 
 
+@pytest.mark.parametrize("width,ff", [(1024, 1536), (1030, 1599), (832, 4100), (2048, 12288)])
+@pytest.mark.parametrize("rows", [2, 7, 8, 9, 16, 17])
+def test_polynorm_between_few_row_products(ctx, width, ff, rows):
+    """2 to 16 rows at once, 17 by the launch of its own; part blocks, pad columns and rows that a fragment does not fill.  Each row against the restatement."""
+    cfg = config([layer(heads=4, kv_heads=2, dim=64, vdim=64, ff=ff)] * 2, width=width, dtype="bfloat16")
+    w = dosovik_weights(cfg, seed=31)
+    ids = [tokens(3, cfg.vocab_size, seed=40 + i) for i in range(rows)]
+    with Model(ctx, cfg, w) as m:
+        seqs = [m.seq_open() for _ in range(rows)]
+        m.forward_batch([(s, x[:2], []) for s, x in zip(seqs, ids)])
+        got, _ = m.forward_batch([(s, x[2:], [0]) for s, x in zip(seqs, ids)])
+    want = np.stack([reference(cfg, w, x)[-1] for x in ids])
+    assert err(got, want) <= TOL["bfloat16"]
+
+
 @pytest.mark.parametrize("dim", [64, 128])
 def test_32_bit_rows_do_not_see_a_later_row_that_is_not_finite(ctx, dim):
     cfg = config([layer(heads=8, kv_heads=4, dim=dim, vdim=dim, chunk=100, rope_dims=dim)] * 2)
