@@ -71,6 +71,19 @@ __device__ __forceinline__ float rows_sum(float v) {
   const auto q = __builtin_amdgcn_permlane32_swap(u, u, false, false);
   return __uint_as_float(q[0]) + __uint_as_float(q[1]);
 }
+// the sum and the maximum over the sixteen lanes of one lane >> 4
+__device__ __forceinline__ float row_sum(float v) {
+  v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x128, 0xf, 0xf, false));
+  v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x124, 0xf, 0xf, false));
+  v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x122, 0xf, 0xf, false));
+  return v + __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x121, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float row_max(float v) {
+  v = fmaxf(v, __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x128, 0xf, 0xf, false)));
+  v = fmaxf(v, __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x124, 0xf, 0xf, false)));
+  v = fmaxf(v, __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x122, 0xf, 0xf, false)));
+  return fmaxf(v, __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x121, 0xf, 0xf, false)));
+}
 // the sum over each half of the wave, lanes 0-31 and 32-63 (the last steps of wave_sum)
 __device__ __forceinline__ float half_wave_sum(float v) {
   const unsigned u = __float_as_uint(v);

@@ -470,6 +470,9 @@ struct ChunkAttnArgs {
 bool chunk_attn_dims_ok(int dim, int vdim, int* dq, int* dv);   // MFMA kernels: padded dims, false = no instantiation
 void launch_chunk_attn_prefill(const ChunkAttnArgs& a, const SeqBatch& b, hipStream_t st);   // bf16, frag pages
 void launch_chunk_attn_rows(const ChunkAttnArgs& a, const SeqBatch& b, bool f32, hipStream_t st);   // any dims, token-major pages
+// one token per sequence, 32 bits: QkvPost + attention in one launch (token-major pages); t's q unused
+bool chunk_attn_f32_decode_ok(const QkvPostArgs& a, const ChunkAttnArgs& t, const SeqBatch& b);
+void launch_chunk_attn_f32_decode(const QkvPostArgs& a, const ChunkAttnArgs& t, const SeqBatch& b, hipStream_t st);
 // One token per sequence: QkvPost + attention in one launch (frag pages, heads / kvh <= 16)
 struct ChunkDecodeArgs {
   QkvPostArgs p;

@@ -2,7 +2,7 @@
 // floor(i / chunk) * chunk .. i of its own sequence; a sink adds a key of score 0 without a value, i.e. one to the softmax's denominator.
 //   prompt rows:   attn_prefill_kernel<.., CHUNK = 1> (attn_prefill_body.h) on fragment-major bf16 pages
 //   one token each: attn_chunk_decode_kernel: q / k norm + rotation + value mixing + KV append + split-KV attention + merge, one launch
-//   the 32-bit mode, heads of 64 or 128 dims: attn_chunk_f32_kernel on token-major pages
+//   the 32-bit mode, heads of 64 or 128 dims: attn_chunk_f32_kernel on token-major pages, one token each: attn_chunk_f32_decode_kernel
 //   any head dims: attn_chunk_rows_kernel on token-major pages
 // q head h reads kv head h / (heads / kv heads).  Scores, maxima, exponentials and sums are f32; P feeds the MFMA as bf16.
 #include <algorithm>
@@ -745,6 +745,254 @@ __global__ __launch_bounds__(F32A_NW * 64) void attn_chunk_f32_kernel(const floa
   }
 }
 
+// ---- 32 bits, one token per sequence, heads of D = 64 or 128 dims: q / k norm + rotation + value mixing + KV append + attention, one launch ----------
+// Block (kv head, sequence), eight or sixteen waves; wave w takes 16 keys in turn, requested as soon as their page is known and before the
+// block redoes the per-token work (sums of squares over the whole q / k projections, its GQ query heads, its key and value).  Lane (c, G) holds dims
+// 16 t + 4 G + i of key c and value dims 64 b + 4 c + x of keys 4 G + i, as in attn_chunk_f32_kernel, but the products are plain f32 fma: of the matrix
+// cores' sixteen columns a token has GQ, and their f32 rate (256 flops a cycle and CU) leaves nothing over for the rest.  The new token joins from LDS.
+// A chain of round trips all the same: 2 x 150 positions, 16 / 8 heads x 128,
+// 11.9 us for the 13.6 + 5.0 of attn_chunk_f32_kernel and qkv_post_f32_kernel.
+constexpr int f32d_waves(int d, int gq) { return d * gq > 256 ? 8 : 16; }   // (four heads of 128: their sums and a unit are more than 128 registers)
+constexpr int F32D_COLUMNS = 8192;   // of q and k
+template <int D, int GQ>   // GQ: query heads per kv head, at most
+constexpr int f32d_lds() {
+  constexpr int NW = f32d_waves(D, GQ);
+  return (2 * (GQ + 2) * D + NW * GQ * (D + 2 + 16) + GQ + 2 * NW) * 4;
+}
+template <int D, int GQ>
+__global__ __launch_bounds__(f32d_waves(D, GQ) * 64) void attn_chunk_f32_decode_kernel(const float* qkv, const float* bias, const SeqEntry* entries, const uint64_t* tab, int ld, int heads_kvh, int slot, int pos, QkvPostArgs a,
+                                                                           ChunkAttnArgs t) {
+  constexpr int NW = f32d_waves(D, GQ), NTH = NW * 64, NT16 = D / 16, NB = D / 64, NC = F32D_COLUMNS / (4 * NTH);
+  extern __shared__ __attribute__((aligned(16))) float sm[];
+  float *raw = sm, *qs = raw + (GQ + 2) * D, *ks = qs + GQ * D, *vs = ks + D;   // raw: the heads' q, k; then with norm and rotation
+  float *os = vs + D, *ml = os + NW * GQ * D, *ll = ml + NW * GQ, *ps = ll + NW * GQ, *fresh = ps + NW * GQ * 16, *red = fresh + GQ;
+  typedef const __attribute__((address_space(1))) fv4* g4_t;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, G = lane >> 4;
+  const int heads = heads_kvh >> 16, kvh = heads_kvh & 0xffff, g = heads / kvh, kv = blockIdx.x, r = blockIdx.y, head0 = kv * g;
+  const int k_off = a.k_off, v_off = a.v_off, rope_dims = a.rope_dims, v_use = a.v_use, v_store = a.v_store, chunk = t.chunk;
+  const bf16_t *q_norm = (const bf16_t*)a.q_norm, *k_norm = (const bf16_t*)a.k_norm;
+  const float* rope = a.rope;
+  float* v_first = a.v_first;
+  const int64_t tab_ld = a.kv.ld;
+  const uint64_t layer_off = a.kv.layer_off;
+  const float lambda = a.lambda, eps = a.eps;
+  const int nq = heads * D, nk = kvh * D, half = rope_dims >> 1;
+  if (entries) {   // (one sequence: its place comes with the launch)
+    typedef const __attribute__((address_space(1))) int32_t* gint_t;
+    const gint_t p = (gint_t)(uintptr_t)(entries + r);
+    pos = p[2];
+    slot = p[3];
+  }
+  const int lo = chunk > 0 ? pos / chunk * chunk : 0;
+  tab += (int64_t)slot * tab_ld;
+  // the row
+  float4 x[NC], bi[NC];
+  const float* row = qkv + (int64_t)r * ld;
+#pragma unroll
+  for (int j = 0; j < NC; ++j) {
+    x[j] = bi[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (j * NTH * 4 >= nq + nk) continue;
+    const int i = min((tid + j * NTH) * 4, nq + nk - 4), at = i < nq ? i : i - nq + k_off;
+    x[j] = *reinterpret_cast<const float4*>(row + at);
+    if (bias) bi[j] = *reinterpret_cast<const float4*>(bias + at);
+  }
+  // this thread's four value columns; its piece of a head: dims d .. d + 3 with their partners half a rotation further, or four behind the rotated ones
+  const bool val = tid >= NTH - D / 4;
+  const int vd = (tid - (NTH - D / 4)) * 4, hp = half >> 2, per = (D >> 2) - hp, np = (g + 1) * per;
+  float4 xv = make_float4(0.f, 0.f, 0.f, 0.f), bv = xv, first = xv;
+  if (val) {
+    xv = *reinterpret_cast<const float4*>(row + v_off + kv * D + vd);
+    if (bias) bv = *reinterpret_cast<const float4*>(bias + v_off + kv * D + vd);
+    if (v_use && !v_store) first = *reinterpret_cast<const float4*>(v_first + ((int64_t)r * kvh + kv) * D + vd);
+  }
+  const int hd = min(tid, np - 1) / per, pc = min(tid, np - 1) - hd * per, pd = pc < hp ? pc * 4 : rope_dims + (pc - hp) * 4;
+  uint2 wx = make_uint2(0u, 0u), wy = wx;
+  float4 cs0 = make_float4(1.f, 0.f, 1.f, 0.f), cs1 = cs0;
+  if (tid < np) {
+    const bf16_t* w = hd < g ? q_norm + (head0 + hd) * D : k_norm + kv * D;
+    wx = *reinterpret_cast<const uint2*>(w + pd);
+    wy = *reinterpret_cast<const uint2*>(w + (pc < hp ? pd + half : pd));
+    if (hp > 0) {
+      const float4* at = reinterpret_cast<const float4*>(rope + ((int64_t)r * half + (pc < hp ? pd : 0)) * 2);
+      cs0 = at[0];
+      cs1 = at[1];
+    }
+  }
+  fv4 kf[NT16], vf[4][NB];
+  uint64_t at_k = 0;   // this lane's piece of the unit's first key
+  auto request_keys = [&](int u) {   // 16 u .. 16 u + 15
+    at_k = tab[u * 16 / KV_PAGE_TOKENS] + layer_off + ((uint64_t)kv * KV_PAGE_TOKENS + u * 16 % KV_PAGE_TOKENS) * (D * 4);
+    const uint64_t kb = at_k + c * (D * 4) + G * 16;
+#pragma unroll
+    for (int i = 0; i < NT16; ++i) kf[i] = *reinterpret_cast<g4_t>(kb + i * 64);
+  };
+  auto request_values = [&] {   // of the same keys
+    const uint64_t vb = at_k + (uint64_t)kvh * KV_PAGE_TOKENS * (D * 4) + G * 4 * (D * 4) + c * 16;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) vf[i][nb] = *reinterpret_cast<g4_t>(vb + (i * D + nb * 64) * 4);
+  };
+  const int u0 = lo / 16 + wave, last = pos / 16;
+  const uint64_t new_page = tab[pos / KV_PAGE_TOKENS] + layer_off;
+  request_keys(min(u0, last));   // (waves without keys too: behind a branch nothing requested before is waited for by itself)
+  // sums of squares; the heads' own columns to LDS
+  float sq = 0.f, sk = 0.f;
+#pragma unroll
+  for (int j = 0; j < NC; ++j) {
+    const int i = (tid + j * NTH) * 4;
+    if (i >= nq + nk) continue;
+    const float4 y = make_float4(x[j].x + bi[j].x, x[j].y + bi[j].y, x[j].z + bi[j].z, x[j].w + bi[j].w);
+    (i < nq ? sq : sk) += (y.x * y.x + y.y * y.y) + (y.z * y.z + y.w * y.w);
+    const int own = i < nq ? i - head0 * D : i - nq - kv * D;
+    if (own >= 0 && own < (i < nq ? g * D : D)) *reinterpret_cast<float4*>(raw + (i < nq ? 0 : GQ * D) + own) = y;
+  }
+  sq = wave_sum(sq);
+  sk = wave_sum(sk);
+  if (lane == 0) {
+    red[wave] = sq;
+    red[NW + wave] = sk;
+  }
+  __syncthreads();
+  request_values();
+  float tq = 0.f, tk = 0.f;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    tq += red[w];
+    tk += red[NW + w];
+  }
+  const float rq = 1.0f / sqrtf(tq / (float)nq + eps), rk = 1.0f / sqrtf(tk / (float)nk + eps);
+  const int tok = pos % KV_PAGE_TOKENS;
+  typedef __attribute__((address_space(1))) fv4* s4_t;
+  const uint64_t kpage = new_page + ((uint64_t)kv * KV_PAGE_TOKENS + tok) * (D * 4), vpage = kpage + (uint64_t)kvh * KV_PAGE_TOKENS * (D * 4);
+  if (tid < np) {
+    const float rinv = hd < g ? rq : rk;
+    float* dst = hd < g ? qs + hd * D : ks;
+    const float* src = raw + (hd < g ? hd : GQ) * D;
+    const float4 s4 = *reinterpret_cast<const float4*>(src + pd);
+    const float4 y0 = make_float4(s4.x * rinv * lo_bf(wx.x), s4.y * rinv * hi_bf(wx.x), s4.z * rinv * lo_bf(wx.y), s4.w * rinv * hi_bf(wx.y));
+    float4 out0 = y0, out1 = y0;
+    if (pc < hp) {
+      const float4 t4 = *reinterpret_cast<const float4*>(src + pd + half);
+      const float4 y1 = make_float4(t4.x * rinv * lo_bf(wy.x), t4.y * rinv * hi_bf(wy.x), t4.z * rinv * lo_bf(wy.y), t4.w * rinv * hi_bf(wy.y));
+      out0 = make_float4(y0.x * cs0.x - y1.x * cs0.y, y0.y * cs0.z - y1.y * cs0.w, y0.z * cs1.x - y1.z * cs1.y, y0.w * cs1.z - y1.w * cs1.w);
+      out1 = make_float4(y1.x * cs0.x + y0.x * cs0.y, y1.y * cs0.z + y0.y * cs0.w, y1.z * cs1.x + y0.z * cs1.y, y1.w * cs1.z + y0.w * cs1.w);
+    }
+    const int pd1 = pc < hp ? pd + half : pd;
+    *reinterpret_cast<float4*>(dst + pd) = out0;
+    *reinterpret_cast<float4*>(dst + pd1) = out1;
+    if (hd == g) {
+      *reinterpret_cast<s4_t>(kpage + pd * 4) = fv4{out0.x, out0.y, out0.z, out0.w};
+      *reinterpret_cast<s4_t>(kpage + pd1 * 4) = fv4{out1.x, out1.y, out1.z, out1.w};
+    }
+  }
+  if (val) {
+    const float4 y = make_float4(xv.x + bv.x, xv.y + bv.y, xv.z + bv.z, xv.w + bv.w);
+    if (v_store) *reinterpret_cast<float4*>(v_first + ((int64_t)r * kvh + kv) * D + vd) = y;
+    const float4 f = v_store ? y : first;   // (stored and used at once: the value itself)
+    const float k0 = 1.f - lambda, k1 = lambda;
+    const float4 o = v_use ? make_float4(k0 * y.x + k1 * f.x, k0 * y.y + k1 * f.y, k0 * y.z + k1 * f.z, k0 * y.w + k1 * f.w) : y;
+    *reinterpret_cast<float4*>(vs + vd) = o;
+    *reinterpret_cast<s4_t>(vpage + vd * 4) = fv4{o.x, o.y, o.z, o.w};
+  }
+  __syncthreads();
+  if (wave < g) {   // the new token's score for head `wave`
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < NB; ++i) s = fmaf(qs[wave * D + i * 64 + lane], ks[i * 64 + lane], s);
+    s = wave_sum(s) * t.scale;
+    if (lane == 0) fresh[wave] = s;
+  }
+  float m[GQ], l[GQ];
+  f32x4_t o[GQ][NB];
+#pragma unroll
+  for (int h = 0; h < GQ; ++h) {
+    m[h] = -INFINITY;
+    l[h] = 0.f;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) o[h][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  for (int u = u0; u <= last; u += NW) {
+    const bool key = u * 16 + c >= lo && u * 16 + c < pos;
+#pragma unroll
+    for (int h = 0; h < GQ; ++h) {
+      if (h >= g) continue;
+      float s2[2] = {0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < NT16; ++i) {
+        const fv4 q = *reinterpret_cast<const fv4*>(qs + h * D + i * 16 + G * 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s2[j & 1] = fmaf(kf[i][j], q[j], s2[j & 1]);
+      }
+      const float s = key ? rows_sum(s2[0] + s2[1]) * t.scale : -INFINITY;
+      const float mn = fmaxf(m[h], row_max(s)), from = mn == -INFINITY ? 0.f : mn;   // (nothing of this unit or before is visible)
+      const float al = expf(m[h] - from), p = expf(s - from);
+      l[h] = l[h] * al + p;
+      m[h] = mn;
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) o[h][nb] *= al;
+      ps[(wave * GQ + h) * 16 + c] = p;   // (the four lanes of one key: the same)
+    }
+    // a value whose key is not visible may be anything: it must not meet its zero weight
+    const int k0 = u * 16 + G * 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) vf[i][nb][j] = k0 + i >= lo && k0 + i < pos ? vf[i][nb][j] : 0.f;
+#pragma unroll
+    for (int h = 0; h < GQ; ++h) {
+      if (h >= g) continue;
+      const fv4 p = *reinterpret_cast<const fv4*>(ps + (wave * GQ + h) * 16 + G * 4);
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[h][nb][j] = fmaf(p[i], vf[i][nb][j], o[h][nb][j]);
+    }
+    if (u + NW <= last) {
+      request_keys(u + NW);
+      request_values();
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < GQ; ++h) {
+    if (h >= g) continue;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      f32x4_t v;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = rows_sum(o[h][nb][j]);
+      if (G == 0) *reinterpret_cast<f32x4_t*>(os + (wave * GQ + h) * D + nb * 64 + c * 4) = v;
+    }
+    const float z = row_sum(l[h]);
+    if (lane == 0) {
+      ml[wave * GQ + h] = m[h];
+      ll[wave * GQ + h] = z;
+    }
+  }
+  __syncthreads();
+  if (wave == 0 && G < g) {   // sixteen lanes a head: the waves' factors, then the new token's and 1 / sum
+    const float mine = fresh[G], mw = c < NW ? ml[c * GQ + G] : -INFINITY, M = fmaxf(t.sink ? fmaxf(mine, 0.f) : mine, row_max(mw));
+    const float f = expf(mw - M), f0 = expf(mine - M), z = row_sum(c < NW ? ll[c * GQ + G] * f : 0.f) + f0 + (t.sink ? expf(-M) : 0.f);
+    ps[G * 20 + c] = f;
+    if (c == 0) {
+      ps[G * 20 + 16] = f0;
+      ps[G * 20 + 17] = 1.0f / z;
+    }
+  }
+  __syncthreads();
+  for (int it = tid; it < g * D; it += NTH) {
+    const int h = it / D, d = it - h * D;
+    float v = ps[h * 20 + 16] * vs[d];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) v = fmaf(os[(w * GQ + h) * D + d], ps[h * 20 + w], v);
+    ((float*)t.o)[(int64_t)r * t.ldo + (int64_t)(head0 + h) * t.dvo + d] = v * ps[h * 20 + 17];
+  }
+}
+
 int pad_dim(int d) { return d <= 32 ? 32 : d <= 64 ? 64 : d <= 128 ? 128 : d <= 256 ? 256 : 0; }
 
 template <class F>
@@ -835,6 +1083,32 @@ void launch_chunk_attn_decode(const ChunkDecodeArgs& a, const SeqBatch& b, hipSt
     if (a.qkv_f32) go(attn_chunk_decode_kernel<DQK, DV, float>);
     else go(attn_chunk_decode_kernel<DQK, DV, bf16_t>);
   });
+}
+
+// Row i of the step is sequence i's only one; whole heads of 64 or 128 dims whose columns come in fours, up to four query heads per kv head and 8192 columns
+// of q and k
+bool chunk_attn_f32_decode_ok(const QkvPostArgs& a, const ChunkAttnArgs& t, const SeqBatch& b) {
+  return b.max_len == 1 && b.rows == b.n && a.dim == a.vdim && (a.dim == 64 || a.dim == 128) && a.kv.dq == a.dim && a.kv.dv == a.dim && !a.kv.frag && a.heads % a.kvh == 0 && a.heads / a.kvh <= 4 &&
+         a.heads < 32768 && (a.heads + a.kvh) * a.dim <= F32D_COLUMNS && ((a.k_off | a.v_off) & 3) == 0 && (a.ld & 3) == 0 && a.ld < (1 << 30) && a.rope_dims % 8 == 0 &&
+         (((uintptr_t)a.qkv | (uintptr_t)a.bias | (uintptr_t)a.rope | (uintptr_t)a.q_norm | (uintptr_t)a.k_norm | (uintptr_t)a.v_first) & 15) == 0 && t.heads == a.heads && t.dim == a.dim;
+}
+
+void launch_chunk_attn_f32_decode(const QkvPostArgs& a, const ChunkAttnArgs& t, const SeqBatch& b, hipStream_t st) {
+  if (b.n <= 0) return;
+  auto go = [&](auto d, auto gq) {
+    constexpr int D = decltype(d)::value, GQ = decltype(gq)::value, lds = f32d_lds<D, GQ>();
+    auto k = attn_chunk_f32_decode_kernel<D, GQ>;
+    if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    hipLaunchKernelGGL(k, dim3((unsigned)a.kvh, (unsigned)b.n), dim3(f32d_waves(D, GQ) * 64), lds, st, (const float*)a.qkv, a.bias, b.has_one ? nullptr : b.entries, a.kv.tab, (int)a.ld, a.heads << 16 | a.kvh, b.one.slot, b.one.pos0, a, t);
+  };
+  auto by_group = [&](auto d) {
+    const int g = a.heads / a.kvh;
+    if (g == 1) go(d, std::integral_constant<int, 1>{});
+    else if (g == 2) go(d, std::integral_constant<int, 2>{});
+    else go(d, std::integral_constant<int, 4>{});
+  };
+  if (a.dim == 128) by_group(std::integral_constant<int, 128>{});
+  else by_group(std::integral_constant<int, 64>{});
 }
 
 void launch_chunk_attn_rows(const ChunkAttnArgs& a, const SeqBatch& b, bool f32, hipStream_t st) {

@@ -322,19 +322,21 @@ Tail run_rows(aha_model* m, const SeqBatch& b, const SeqEntry* h_ents, const uin
       ProfScope ps(m, "attn_decode", (double)rows * W.nqkv * 2, 0);
       launch_chunk_attn_decode(a, b, st);
     } else {
-      {
+      ChunkAttnArgs a{};
+      a.q = l.q; a.o = l.o; a.kv = qp.kv; a.heads = d.heads; a.dvo = W.dvo; a.ldo = W.o_ld; a.vdim = d.vdim; a.dim = d.dim; a.chunk = d.chunk; a.sink = 1; a.scale = d.scale;
+      const bool one_launch = l.f32 && chunk_attn_f32_decode_ok(qp, a, b);
+      if (!one_launch) {
         ProfScope ps(m, "elem", (double)rows * (W.nqkv + W.nk + W.nv + d.heads * W.dq) * es, 0);
         launch_qkv_post(qp, b, l.f32, st);
       }
-      ChunkAttnArgs a{};
-      a.q = l.q; a.o = l.o; a.kv = qp.kv; a.heads = d.heads; a.dvo = W.dvo; a.ldo = W.o_ld; a.vdim = d.vdim; a.dim = d.dim; a.chunk = d.chunk; a.sink = 1; a.scale = d.scale;
       double flops = 0;
       for (int i = 0; i < b.n; ++i) {
         const double keys = d.chunk > 0 ? std::min<double>(d.chunk, h_ents[i].pos0 + h_ents[i].len) : h_ents[i].pos0 + h_ents[i].len;
         flops += 2.0 * h_ents[i].len * keys * 0.5 * d.heads * (d.dim + d.vdim);
       }
       ProfScope ps(m, "attn_prefill", (double)rows * d.heads * (W.dq + W.dvo) * es, flops);
-      if (W.frag) launch_chunk_attn_prefill(a, b, st);
+      if (one_launch) launch_chunk_attn_f32_decode(qp, a, b, st);
+      else if (W.frag) launch_chunk_attn_prefill(a, b, st);
       else launch_chunk_attn_rows(a, b, l.f32, st);
     }
     gemm(m, l.o, W.o_ld, W.wo, l.y, l.ld, rows, (int)l.ld, W.ldo);

@@ -139,6 +139,28 @@ def test_32_bit_heads_of_whole_pieces(ctx, heads, kv_heads, dim, chunk, rope_dim
         assert err(all_logits(m, ids, [1, 130, 63] + [1] * 17), want) <= TOL["float32"]
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,chunk,rope_dims,v_mix", [(8, 8, 128, 700, 128, True), (16, 8, 128, 600, 64, True), (12, 4, 64, 50, 0, False), (8, 2, 128, 300, 128, True),
+                                                                      (16, 4, 64, 16, 32, True), (10, 2, 128, 300, 128, True), (32, 32, 128, 300, 128, False), (48, 24, 128, 300, 128, False)])
+def test_32_bit_decoding_in_one_launch(ctx, heads, kv_heads, dim, chunk, rope_dims, v_mix):
+    """One token each of sequences that end around 16 keys, a page and a round of 128 or 256 keys, the first token among them; groups of 1 to 4 heads, five
+    heads, 8192 columns of q and k and more of them in the launches they had."""
+    cfg = config([layer(heads=heads, kv_heads=kv_heads, dim=dim, vdim=dim, chunk=chunk, rope_dims=rope_dims, v_mix=v_mix)] * 2)
+    w = dosovik_weights(cfg, seed=17)
+    ids = tokens(560, cfg.vocab_size, 18)
+    want = reference(cfg, w, ids)
+    at = [0, 1, 15, 16, 17, 63, 64, 127, 128, 255, 256, 257, 513, 559]
+    with Model(ctx, cfg, w) as m:
+        seqs = [m.seq_open() for _ in at]
+        for s, p in zip(seqs, at):
+            if p:
+                m.forward_batch([(s, ids[:p], [])])
+        got, _ = m.forward_batch([(s, ids[p:p + 1], [0]) for s, p in zip(seqs, at)])
+        assert err(got, want[at]) <= TOL["float32"]
+        for k in range(3):   # on from the keys and values that the launch appended, alone
+            one, _ = m.forward_batch([(seqs[4], ids[18 + k:19 + k], [0])])
+            assert err(one, want[18 + k:19 + k]) <= TOL["float32"]
+
+
 @pytest.mark.parametrize("rows,ff,vocab", [(8, 2624, 24600), (16, 2624, 322), (20, 2624, 24600), (32, 2624, 322), (33, 2624, 322), (65, 2624, 322), (97, 2624, 322),
                                            (150, 2624, 322), (300, 2624, 322), (500, 2624, 322), (257, 4160, 322)])
 def test_32_bit_products_of_every_tile(ctx, rows, ff, vocab):
