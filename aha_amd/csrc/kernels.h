@@ -317,8 +317,6 @@ struct VitRopeArgs {
   const void* qkv;          // (N, 3*nh*hd) bf16: [q heads | k heads | v heads]
   const int32_t* rowcol;    // (N, 2) patch (row, col)
   const float* inv_freq;    // (hd/4)
-  const int32_t* page_of;   // (N) page index of token n
-  const int32_t* slot_of;   // (N) slot (0..63) of token n inside its page
   void* q_out;              // (N, nh, VIT_DQK) bf16, zero padded
   KvLayer kv;               // pages: K block [nh][64][VIT_DQK], V block [nh][VIT_DV][64]
   int N, nh, hd;

@@ -110,82 +110,23 @@ void launch_pos_embed_add(void* x, const void* table, const int32_t* idx, const 
 }
 
 // ---- V3/V4 staging: 2-D rotary on q,k (apply_rotary_pos_emb_vision, rope.rs:75-94; rot_pos_emb qwen3vl/model.rs:641-690)
-// and repack into the attention kernel's operand layouts.  One wave per (token, head).  head_dim hd = 72:
-// rotate_half pairs element e with e + hd/2; angle(e) = (e < hd/4 ? row : col) * inv_freq[e % (hd/4)] for e < hd/2,
-// and the same again for e >= hd/2 (emb = cat(rotary, rotary), model.rs:704).
-// 8 bytes per lane: a (token, q | k) unit is 9 lanes that walk over the heads, lane g holding elements 4g..4g+3 AND their rotate_half partners
-// 36 + 4g.. (two 8-byte loads, no cross-lane traffic: 36 elements are 4.5 sixteen-byte pieces, so the pair is not a lane shift);
-// every store is 8 bytes (half a piece of the fragment-major K page, or of the padded q row).  The first 6 lanes of a unit also
-// zero the pad elements 72..95.  cos / sin come from the per-image table (launch_vit_rope_table).
-// V rows take the second block role: 80 lanes per (page, head) -- (token-slot half kk, lane group G, 8-dim chunk) -- load 8 tokens x
+// and repack into the attention kernel's operand layouts.  head_dim hd = 72: rotate_half pairs element e with e + hd/2;
+// angle(e) = (e < hd/4 ? row : col) * inv_freq[e % (hd/4)] for e < hd/2, and the same again for e >= hd/2 (emb = cat(rotary, rotary), model.rs:704).
+// cos / sin come from the per-image table (launch_vit_rope_table).
+// Block: a head's 64 tokens of a page.  Rows come and go in whole 16-byte pieces, a wave's stores to the fragment-major K page 1 KB in a row, and the pairs
+// (36 elements apart: four and a half pieces) meet in LDS; pads 72..95 are zeros.  Blocks of a page's heads follow one another on one XCD, whose cache holds the
+// lines that neighbouring heads (144 bytes) share.  Bound by those bytes, 28 MB in and 38 out at 4096 tokens: with lanes that walked over the heads and
+// stored halves of pieces 17.9 us, 16.0 here (16384 tokens: 74.5 and 61.8; 640: 9.0 and 7.5).
+// V: 80 lanes -- (token-slot half kk, lane group G, 8-dim chunk) -- load 8 tokens x
 // 8 dims, transpose 8 x 8 in registers and store eight 16-byte pieces of the fragment-major V block; pad dim 72 is 1.0 on real tokens
 // (the row-sum column, see below), pad dims 73..79 and the slots of a tail page past its last token are zeros (they must be finite).
-// (The first version moved 2 bytes per lane and instruction and ran at 1.5 TB/s: 29 us per call at N = 4096, 2.7 ms at 8 x 2048^2.)
-__global__ __launch_bounds__(256) void vit_rope_pack_kernel(VitRopeArgs a, int n_qk_blocks) {
-  const int lane = threadIdx.x & 63;
-  const int hd = a.hd, half = hd / 2;   // 72, 36
-  const int D = a.nh * hd;
-  if ((int)blockIdx.x < n_qk_blocks) {
-    // a 9-lane unit = (token, q | k); it walks over the heads, 4 at a time in flight
-    const int64_t wid = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int64_t unit = wid * 7 + lane / 9;
-    const int g = lane % 9;
-    if (lane >= 63 || unit >= (int64_t)a.N * 2) return;
-    const int which = (int)(unit & 1), n = (int)(unit >> 1);
-    const int e0 = 4 * g;
-    const float4 cs01 = *reinterpret_cast<const float4*>(a.cs_tab + ((int64_t)n * half + e0) * 2);
-    const float4 cs23 = *reinterpret_cast<const float4*>(a.cs_tab + ((int64_t)n * half + e0 + 2) * 2);
-    const float c[4] = {cs01.x, cs01.z, cs23.x, cs23.z}, s[4] = {cs01.y, cs01.w, cs23.y, cs23.w};
-    const bf16_t* src = (const bf16_t*)a.qkv + (int64_t)n * 3 * D + (int64_t)which * D + e0;
-    bf16_t* dq = (bf16_t*)a.q_out + (int64_t)n * a.nh * VIT_DQK;
-    const int slot = a.slot_of[n];
-    bf16_t* dk = reinterpret_cast<bf16_t*>(a.kv.page_ptrs[a.page_of[n]] + a.kv.layer_off);
-    const int k0 = kpage_elem(slot, e0, VIT_DQK / 32), k1 = kpage_elem(slot, e0 + half, VIT_DQK / 32), kz = kpage_elem(slot, hd + 4 * (g % 6), VIT_DQK / 32);
-    const uint2 zero = {0u, 0u};
-    for (int h0 = 0; h0 < a.nh; h0 += 4) {
-      uint2 x0w[4], x1w[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (h0 + i < a.nh) {
-          x0w[i] = *reinterpret_cast<const uint2*>(src + (int64_t)(h0 + i) * hd);
-          x1w[i] = *reinterpret_cast<const uint2*>(src + (int64_t)(h0 + i) * hd + half);
-        }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int h = h0 + i;
-        if (h >= a.nh) break;
-        const float x0[4] = {lo_bf(x0w[i].x), hi_bf(x0w[i].x), lo_bf(x0w[i].y), hi_bf(x0w[i].y)};
-        const float x1[4] = {lo_bf(x1w[i].x), hi_bf(x1w[i].x), lo_bf(x1w[i].y), hi_bf(x1w[i].y)};
-        float y0[4], y1[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          y0[j] = rbf(x0[j] * c[j]) + rbf(-x1[j] * s[j]);
-          y1[j] = rbf(x1[j] * c[j]) + rbf(x0[j] * s[j]);
-        }
-        const uint2 o0 = {pack_bf(y0[0], y0[1]), pack_bf(y0[2], y0[3])}, o1 = {pack_bf(y1[0], y1[1]), pack_bf(y1[2], y1[3])};
-        if (which == 0) {
-          bf16_t* qd = dq + (int64_t)h * VIT_DQK;
-          *reinterpret_cast<uint2*>(qd + e0) = o0;
-          *reinterpret_cast<uint2*>(qd + e0 + half) = o1;
-          if (g < (VIT_DQK - 72) / 4) *reinterpret_cast<uint2*>(qd + hd + 4 * g) = zero;
-        } else {
-          bf16_t* kd = dk + (int64_t)h * KV_PAGE_TOKENS * VIT_DQK;
-          *reinterpret_cast<uint2*>(kd + k0) = o0;
-          *reinterpret_cast<uint2*>(kd + k1) = o1;
-          if (g < (VIT_DQK - 72) / 4) *reinterpret_cast<uint2*>(kd + kz) = zero;
-        }
-      }
-    }
-    return;
-  }
-  // ---- V: 80 lanes per (page, head) ----
-  const int64_t u = (int64_t)(blockIdx.x - n_qk_blocks) * 256 + threadIdx.x;
-  const int64_t unit = u / 80;
-  const int lu = (int)(u % 80);
-  if (unit >= (int64_t)a.n_pages * a.nh) return;
-  const int page = (int)(unit / a.nh), h = (int)(unit % a.nh);
-  const int kk = lu / 40, G = (lu % 40) / 10, dchunk = lu % 10;
-  const int first = a.page_first[page], cnt = a.page_cnt[page];
+__global__ __launch_bounds__(256) void vit_rope_pack_kernel(VitRopeArgs a) {
+  constexpr int hd = 72, half = hd / 2, PIECES = hd / 8, TOK = KV_PAGE_TOKENS, CSP = 2 * half + 4;   // (cos / sin rows: an odd number of 16-byte pieces)
+  __shared__ __attribute__((aligned(16))) bf16_t rows[2][TOK * hd];
+  __shared__ __attribute__((aligned(16))) float cs[TOK * CSP];
+  const int tid = threadIdx.x, xcd = blockIdx.x & 7, rest = blockIdx.x >> 3, page = rest / a.nh * 8 + xcd, h = rest % a.nh, D = a.nh * hd;
+  if (page >= a.n_pages) return;
+  const int first = a.page_first[page], cnt = a.page_cnt[page], lu = min(tid, 79), kk = lu / 40, G = (lu % 40) / 10, dchunk = lu % 10;
   uint32_t in[8][4];
 #pragma unroll
   for (int e = 0; e < 8; ++e) {   // slot order inside a piece: e = sub1 * 4 + j  <->  token slot kk*32 + sub1*16 + G*4 + j
@@ -193,12 +134,62 @@ __global__ __launch_bounds__(256) void vit_rope_pack_kernel(VitRopeArgs a, int n
     u32x4_t v = {0u, 0u, 0u, 0u};
     if (tslot < cnt && dchunk < 9)
       v = ld16((const bf16_t*)a.qkv + (int64_t)(first + tslot) * 3 * D + 2 * (int64_t)D + (int64_t)h * hd + dchunk * 8);
-    // pad dim 72 = 1.0 on every real token (round 5): V^T . P^T then delivers the softmax row sum in output row 72 -- rescaled with the
+    // pad dim 72 = 1.0 on every real token: V^T . P^T then delivers the softmax row sum in output row 72 -- rescaled with the
     // accumulators, from the SAME rounded probabilities as the numerator -- and the f32-chain attention kernel drops its own sum
     // (kernels_attn.hip LSUM).  Rows 72..79 of the output are never stored.
     if (tslot < cnt && dchunk == 9) v[0] = 0x3F80u;
     in[e][0] = v[0]; in[e][1] = v[1]; in[e][2] = v[2]; in[e][3] = v[3];
   }
+  const bf16_t* src = (const bf16_t*)a.qkv + (int64_t)first * 3 * D + (int64_t)h * hd;
+  u32x4_t x[2][3], t[5];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const int p = min(tid + i * 256, cnt * PIECES - 1), token = p / PIECES;
+#pragma unroll
+    for (int w = 0; w < 2; ++w) x[w][i] = ld16(src + (int64_t)token * 3 * D + w * D + (p - token * PIECES) * 8);
+  }
+  constexpr int CP = half / 2;   // 16-byte pieces of a token's table row
+#pragma unroll
+  for (int i = 0; i < 5; ++i) t[i] = ld16((const bf16_t*)(a.cs_tab + (int64_t)first * 2 * half) + min(tid + i * 256, cnt * CP - 1) * 8);
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int w = 0; w < 2; ++w)
+      if (tid + i * 256 < TOK * PIECES) *reinterpret_cast<u32x4_t*>(rows[w] + (tid + i * 256) * 8) = x[w][i];
+#pragma unroll
+  for (int i = 0; i < 5; ++i) {
+    const int p = tid + i * 256, token = p / CP;
+    if (p < TOK * CP) *reinterpret_cast<u32x4_t*>(cs + token * CSP + (p - token * CP) * 4) = t[i];
+  }
+  __syncthreads();
+  auto rotated = [&](const bf16_t* row, const float* tab, int piece) {
+    u32x4_t o = {0u, 0u, 0u, 0u};
+    if (piece >= PIECES) return o;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int e = piece * 8 + j * 4, other = e < half ? e + half : e - half, i = e < half ? e : other;
+      const uint2 xw = *reinterpret_cast<const uint2*>(row + e), yw = *reinterpret_cast<const uint2*>(row + other);
+      const float4 c0 = *reinterpret_cast<const float4*>(tab + i * 2), c1 = *reinterpret_cast<const float4*>(tab + i * 2 + 4);
+      const float xs[4] = {lo_bf(xw.x), hi_bf(xw.x), lo_bf(xw.y), hi_bf(xw.y)}, ys[4] = {lo_bf(yw.x), hi_bf(yw.x), lo_bf(yw.y), hi_bf(yw.y)};
+      const float co[4] = {c0.x, c0.z, c1.x, c1.z}, si[4] = {c0.y, c0.w, c1.y, c1.w};
+      float y[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) y[k] = rbf(xs[k] * co[k]) + rbf(ys[k] * (e < half ? -si[k] : si[k]));
+      o[j * 2] = pack_bf(y[0], y[1]);
+      o[j * 2 + 1] = pack_bf(y[2], y[3]);
+    }
+    return o;
+  };
+  constexpr int OUT = VIT_DQK / 8;   // pieces of a padded row
+  bf16_t* q = (bf16_t*)a.q_out + ((int64_t)first * a.nh + h) * VIT_DQK;
+  bf16_t* kd = reinterpret_cast<bf16_t*>(a.kv.page_ptrs[page] + a.kv.layer_off) + (int64_t)h * TOK * VIT_DQK;
+#pragma unroll
+  for (int i = 0; i < TOK * OUT / 256; ++i) {
+    const int p = tid + i * 256, token = p / OUT, slot = p / (64 * OUT / 4) * 16 + (p & 15), piece = p / 64 % (OUT / 4) * 4 + (p >> 4 & 3);   // (kpage_elem's order)
+    if (token < cnt) *reinterpret_cast<u32x4_t*>(q + (int64_t)token * a.nh * VIT_DQK + (p - token * OUT) * 8) = rotated(rows[0] + token * hd, cs + token * CSP, p - token * OUT);
+    if (slot < cnt) *reinterpret_cast<u32x4_t*>(kd + p * 8) = rotated(rows[1] + slot * hd, cs + slot * CSP, piece);
+  }
+  if (tid >= 80) return;
   bf16_t* vd = reinterpret_cast<bf16_t*>(a.kv.page_ptrs[page] + a.kv.layer_off) + (int64_t)a.nh * KV_PAGE_TOKENS * VIT_DQK +
                (int64_t)h * VIT_DV * KV_PAGE_TOKENS;
 #pragma unroll
@@ -230,10 +221,7 @@ void launch_vit_rope_table(const int32_t* rowcol, const float* inv_freq, int N, 
 }
 void launch_vit_rope_pack(const VitRopeArgs& a, hipStream_t st) {
   if (a.N <= 0) return;
-  const int64_t units = (int64_t)a.N * 2, waves = (units + 6) / 7;
-  const int n_qk_blocks = (int)((waves + 3) / 4);
-  const int n_v_blocks = (int)(((int64_t)a.n_pages * a.nh * 80 + 255) / 256);
-  hipLaunchKernelGGL(vit_rope_pack_kernel, dim3((unsigned)(n_qk_blocks + n_v_blocks)), dim3(256), 0, st, a, n_qk_blocks);
+  hipLaunchKernelGGL(vit_rope_pack_kernel, dim3((unsigned)((a.n_pages + 7) / 8 * 8 * a.nh)), dim3(256), 0, st, a);
 }
 
 // ---- M3: dst[rows[i], :] = src[i, :]  (masked_scatter_dim0, tensor_utils.rs:294-321)

@@ -41,9 +41,9 @@ struct VisionModel {
   void* gemm_ws = nullptr;   // split-K slabs of the tower's GEMMs (vision_ensure_scratch)
   size_t gemm_ws_bytes = 0;
   void *pix = nullptr, *x = nullptr, *h = nullptr, *qkv = nullptr, *q = nullptr, *attn = nullptr, *mlp = nullptr, *mh = nullptr;
-  int32_t *d_idx = nullptr, *d_rowcol = nullptr, *d_page_of = nullptr, *d_slot_of = nullptr, *d_vis_rows = nullptr;
+  int32_t *d_idx = nullptr, *d_rowcol = nullptr, *d_vis_rows = nullptr;
   float* d_cs_tab = nullptr;   // rotary (cos, sin) per patch and lane, shared by all blocks (launch_vit_rope_table)
-  int32_t *d_page_first = nullptr, *d_page_cnt = nullptr;   // per page: first token / token count (vit_rope_pack_kernel's V role)
+  int32_t *d_page_first = nullptr, *d_page_cnt = nullptr;   // per page: first token / token count (vit_rope_pack_kernel)
   float* d_wt = nullptr;
   void* page_store = nullptr;
   uint64_t* d_page_ptrs = nullptr;
@@ -192,8 +192,6 @@ static int vision_ensure_scratch(aha_model* m, size_t N, size_t npages) {
   if ((rc = al(cap * 4 * 4, (void**)&v->d_wt))) return rc;
   if ((rc = al(cap * 2 * 4, (void**)&v->d_rowcol))) return rc;
   if ((rc = al(cap * (size_t)v->hd * 4, (void**)&v->d_cs_tab))) return rc;   // (cap, hd/2, 2) f32
-  if ((rc = al(cap * 4, (void**)&v->d_page_of))) return rc;
-  if ((rc = al(cap * 4, (void**)&v->d_slot_of))) return rc;
   if ((rc = al(n4 * 4, (void**)&v->d_vis_rows))) return rc;
   if ((rc = al(pcap * v->page_bytes, &v->page_store, true))) return rc;  // zero: pad slots of tail pages must stay finite
   if ((rc = al(pcap * 8, (void**)&v->d_page_ptrs))) return rc;
@@ -336,7 +334,7 @@ int vision_forward_and_scatter(aha_model* m, const uint32_t* ids, size_t n, cons
       return AHA_ERR_SHAPE;
     }
   }
-  std::vector<int32_t> idx(4 * N), rowcol(2 * N), page_of(N), slot_of(N);
+  std::vector<int32_t> idx(4 * N), rowcol(2 * N);
   std::vector<float> wt(4 * N);
   struct Seg { int64_t start, len, page0; };
   std::vector<Seg> segs;
@@ -379,8 +377,6 @@ int vision_forward_and_scatter(aha_model* m, const uint32_t* ids, size_t n, cons
               wt[3 * N + nn] = dh * dw;
               rowcol[2 * nn] = y;
               rowcol[2 * nn + 1] = xq;
-              page_of[nn] = (int32_t)(pages + local / KV_PAGE_TOKENS);
-              slot_of[nn] = (int32_t)(local % KV_PAGE_TOKENS);
             }
       pages += ((int64_t)h * w + KV_PAGE_TOKENS - 1) / KV_PAGE_TOKENS;
     }
@@ -411,8 +407,6 @@ int vision_forward_and_scatter(aha_model* m, const uint32_t* ids, size_t n, cons
   AHA_HIP_CHECK(hipMemcpyAsync(v->d_idx, idx.data(), idx.size() * 4, hipMemcpyHostToDevice, st));
   AHA_HIP_CHECK(hipMemcpyAsync(v->d_wt, wt.data(), wt.size() * 4, hipMemcpyHostToDevice, st));
   AHA_HIP_CHECK(hipMemcpyAsync(v->d_rowcol, rowcol.data(), rowcol.size() * 4, hipMemcpyHostToDevice, st));
-  AHA_HIP_CHECK(hipMemcpyAsync(v->d_page_of, page_of.data(), page_of.size() * 4, hipMemcpyHostToDevice, st));
-  AHA_HIP_CHECK(hipMemcpyAsync(v->d_slot_of, slot_of.data(), slot_of.size() * 4, hipMemcpyHostToDevice, st));
   std::vector<int32_t> page_first((size_t)pages), page_cnt((size_t)pages);
   for (const Seg& sg : segs)
     for (int64_t p = 0; p * KV_PAGE_TOKENS < sg.len; ++p) {
@@ -452,7 +446,7 @@ int vision_forward_and_scatter(aha_model* m, const uint32_t* ids, size_t n, cons
     vgemm(m, v->h, b.qkv_w, v->qkv, (int)N, 3 * v->D, v->D, b.qkv_b, nullptr, ACT_NONE);
     {
       VitRopeArgs r{};
-      r.qkv = v->qkv; r.rowcol = v->d_rowcol; r.inv_freq = v->d_inv_freq; r.page_of = v->d_page_of; r.slot_of = v->d_slot_of;
+      r.qkv = v->qkv; r.rowcol = v->d_rowcol; r.inv_freq = v->d_inv_freq;
       r.q_out = v->q; r.kv = kv; r.N = (int)N; r.nh = v->nh; r.hd = v->hd; r.cs_tab = v->d_cs_tab;
       r.page_first = v->d_page_first; r.page_cnt = v->d_page_cnt; r.n_pages = (int)pages;
       ProfScope ps(m, "elem", (double)N * v->D * 3 * 4, 0);

@@ -279,3 +279,18 @@ def test_vit_tower_on_every_score_chain_variant(vl, gpu, smx):
     for k in range(len(cfg.vision.deepstack_visual_indexes)):
         d_max, d_rms = rel_err(emb[k + 1].float().cpu().numpy(), o.last_deepstack[k].numpy())
         assert d_max < 0.08 and d_rms < 0.02, f"smx {smx}: deepstack {k} off: max {d_max:.4f} rms {d_rms:.4f}"
+
+
+@pytest.mark.parametrize("sizes", [[(32, 32)], [(128, 128), (64, 256)], [(352, 352), (32, 64), (224, 160)]])
+def test_vit_tower_where_pages_end(vl, gpu, sizes):
+    """vit_rope_pack_kernel takes a head of a page per block, the pages dealt to eight XCDs: segments of 4 patches, of whole pages, of 484 / 8 / 140, up to
+    twelve pages; the bound of every other tower test."""
+    from aha_amd.model import MultiModalData
+    cfg, m, o = vl
+    imgs, pv, grid, ids = make_request(cfg, sizes, 6, 37)
+    o.clear_cache()
+    o.forward_initial(ids, 0, (pv, grid))
+    emb = m.vision_encode(MultiModalData(pv.to(torch.bfloat16), grid))
+    for k, ref in enumerate([o.last_image_embeds] + list(o.last_deepstack)):
+        e_max, e_rms = rel_err(emb[k].float().cpu().numpy(), ref.numpy())
+        assert e_max < 0.08 and e_rms < 0.02, f"embeds {k} off: max {e_max:.4f} rms {e_rms:.4f} (in std units)"
