@@ -1089,8 +1089,12 @@ GemmPlan plan_gemm(const GemmArgs& a) {
   const bool ring128 = t128 <= (double)gemm_streamk_cus() && nk >= 4;
   // (a norm riding on the call is folded into a split plan's reduce pass; behind an unsplit ring launch it is a ~6-us launch of its own --
   // cfg 2 o_proj, 2048 x 1024 x 2048: 23.1 us unsplit against 27.6 us as 256^2 x 4 slices, but 4.99 against 4.57 ms per prefill)
-  const double cost128 = std::max(ceil(t128 / 256.0) * nk * 0.68, t128 < 512.0 ? nk * (ring128 ? lat_ring : lat128) + 4.5 : 0.0) +
-                         (ring128 && a.norm_w ? 6.0 : 0.0);
+  // Up to 2048 columns (behind them no vision tower's or 8B stack's sums): a ring launch at its own k step whatever the depth -- 0.68 us is a CU's that holds four
+  // blocks -- and 5 us for the norm: 2432 x 1024 x 3072 and its norm 36.5 us as three slices of 192 columns, 32.4 here (1024 x 2048 / 3072 at 256 to 4096 rows: 18
+  // to 22.7 us by the rule's 20.5, 24.9 to 30.8 by 28.5).
+  const bool narrow = a.N <= 2048 && !a.bias && ring128;
+  const double cost128 = narrow ? nk * lat_ring + 4.5 + (a.norm_w ? 5.0 : 0.0)
+                                           : std::max(ceil(t128 / 256.0) * nk * 0.68, t128 < 512.0 ? nk * (ring128 ? lat_ring : lat128) + 4.5 : 0.0) + (ring128 && a.norm_w ? 6.0 : 0.0);
   const bool can_split = a.act != ACT_SILU_MUL_PAIRS && a.act != ACT_PARTIAL_F32 && a.workspace != nullptr && (a.N & 3) == 0;
   GemmPlan best{128, 1};
   double best_cost = cost128;
@@ -1112,8 +1116,15 @@ GemmPlan plan_gemm(const GemmArgs& a) {
   // small and launch-sized: ~2 TB/s over its (slices + 1) slabs, not the 4 TB/s of the 256^2 plans' larger ones (scripts/tune_gemm.py at
   // 406 x 1024: 4 -> 8 slices + 1.9 us with four k steps less)
   static const bool ring_sk_on = [] { const char* e = getenv("AHA_GEMM_RING_SPLITK"); return e ? atoi(e) != 0 : true; }();
+  // bytes per us: a reduce pass of < 1 M outputs does not fill the chip, whichever tiles it sums.  With the 256-row plans' passes at 4 TB/s all the same, 512 to 976
+  // rows of 1024 columns and their like took them: 768 x 1024 x 2048 24.9 -> 15.7 us, 640 x 1024 x 3072 23.0 -> 16.4, 384 x 2048 x 2048 24.6 -> 17.5,
+  // 512 x 1536 x 4096 25.5 -> 19.4; the best 256-row plan of 43 such shapes is 5 to 10 us behind the best here.  Calls with a bias (vision towers) keep the plans
+  // they had, at 640 x 1152 x 4352 26.8 us for 20.1: the stack behind them is bf16, and another order of a tower's sums moves the 8B model's logits by 3.1 % of
+  // their spread -- no further from 64 bits (2.7 % either way), but further from what the same weights gave.
+  const double red_rate = (double)a.M * a.N < 1.0e6 ? 2.0e6 : 4.0e6, red_rate256 = a.bias ? 4.0e6 : red_rate;
+  // (f32 slabs of narrow results, written: 2432 x 1024 x 3072 in three slices 32.8 us, 30.2 without; a norm in the reduce pass 1.5 us)
+  auto slabs_us = [&](int sk) { return narrow ? sk * (double)a.M * a.N * 4.0 / 5.0e6 + (a.norm_w ? 1.5 : 0.0) : 3.0; };
   if (ring_sk_on && can_split && nk >= 24 && !e_tile && !(e_sk && atoi(e_sk) == 1)) {   // (K >= 1536: below, the slices save ~2 us by the model -- inside its error)
-    const double red_rate = (double)a.M * a.N < 1.0e6 ? 2.0e6 : 4.0e6;   // (bytes per us: a reduce pass of < 1 M outputs does not fill the chip)
     for (int sk : {2, 3, 4, 6, 8}) {
       if (e_sk && atoi(e_sk) != sk) continue;
       if ((size_t)sk * a.M * a.N * 4 > a.workspace_bytes || nk / sk < 4 || t128 * sk > (double)gemm_streamk_cus()) continue;
@@ -1134,7 +1145,7 @@ GemmPlan plan_gemm(const GemmArgs& a) {
     if (sk > 1 && (!can_split || (size_t)sk * a.M * a.N * 4 > a.workspace_bytes || nk / sk < 8)) continue;
     const bool q4 = a.K % BK == 0 && (sk > 1 || nk >= 32 || !a.residual || (!a.bias && a.act != ACT_GELU_TANH && a.act != ACT_GELU_ERF));   // gemm256q (launch256_one)
     double c = ceil(t256 * sk / 256.0) * ceil(nk / sk) * (q4 ? 1.5 : 1.75);
-    if (sk > 1) c += (double)(sk + 1) * a.M * a.N * 4.0 / 4.0e6 + 3.0;
+    if (sk > 1) c += (double)(sk + 1) * a.M * a.N * 4.0 / red_rate256 + slabs_us(sk);
     if (e_sk && atoi(e_sk) != sk) continue;
     if (c < best_cost || (e_tile && atoi(e_tile) == 256 && best.tile != 256)) {
       best = GemmPlan{256, sk};
@@ -1184,7 +1195,7 @@ GemmPlan plan_gemm(const GemmArgs& a) {
     const double t192 = (double)((a.M + 255) / 256) * ((a.N + 191) / 192);
     for (int sk : {2, 3, 4}) {
       if ((size_t)sk * a.M * a.N * 4 > a.workspace_bytes || nk / sk < 16 || t192 * sk > 256.0 || t192 * sk < 128.0) continue;   // (short K loops: ViT proj, K = 1152, 28.5 us against 26.3 us on the 128^2 kernel)
-      const double c = ceil(nk / sk) * 1.5 * 0.72 + (double)(sk + 1) * a.M * a.N * 4.0 / 4.0e6 + 3.0;
+      const double c = ceil(nk / sk) * 1.5 * 0.72 + (double)(sk + 1) * a.M * a.N * 4.0 / red_rate256 + slabs_us(sk);
       if (c < best_cost) {
         best = GemmPlan{192, sk};
         best_cost = c;

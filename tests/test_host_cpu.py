@@ -302,6 +302,17 @@ def test_gemm_plans_of_the_baseline_shapes(hip_lib):
         assert hip_lib.aha_hip_debug_plan_gemm(0, 1, 1, 0, 0, 0, 0, (ctypes.c_int32 * 3)()) == 0
 
 
+@pytest.mark.parametrize("M,N,K,bias,norm,want", [
+    (512, 1024, 3072, 0, 1, (128, 4)), (640, 1024, 3072, 0, 1, (128, 4)), (768, 1024, 2048, 0, 1, (128, 3)), (976, 1024, 3072, 0, 1, (128, 4)), (384, 2048, 2048, 0, 0, (128, 3)),   # under 1 M outputs
+    (2048, 1024, 3072, 0, 1, (128, 2)), (2304, 1024, 3072, 0, 1, (128, 1)), (2432, 1024, 3072, 0, 1, (128, 1)), (4096, 1024, 3072, 0, 1, (128, 1)), (2432, 1024, 2048, 0, 0, (128, 1)),   # one block per CU
+    (768, 1024, 2048, 1, 1, (256, 4)), (2432, 1024, 3072, 1, 1, (192, 3)), (5067, 1024, 2048, 0, 0, (192, 2)),   # with a bias, or more blocks than CUs: as without either
+])
+def test_gemm_plans_of_narrow_results(hip_lib, M, N, K, bias, norm, want):
+    out = (ctypes.c_int32 * 3)()
+    assert hip_lib.aha_hip_debug_plan_gemm(M, N, K, 0, bias, 1 | 2 * norm, 1 << 30, out) == 0
+    assert tuple(out[:2]) == want and out[2] == 0
+
+
 def test_few_row_gemm_where_it_is_the_faster_one(hip_lib):
     """csrc/kernels_gemm_skinny.hip gemm_skinny_plan against the tiled plans: weight rows per block of the few-row kernel, 0 where the tiles run.  Times on
     MI355X from HBM in us, few-row kernel with 16 / 24 / 32 / 48 weight rows | tiles."""
