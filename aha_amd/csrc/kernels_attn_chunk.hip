@@ -746,13 +746,13 @@ __global__ __launch_bounds__(F32A_NW * 64) void attn_chunk_f32_kernel(const floa
 }
 
 // ---- 32 bits, one token per sequence, heads of D = 64 or 128 dims: q / k norm + rotation + value mixing + KV append + attention, one launch ----------
-// Block (kv head, sequence), eight or sixteen waves; wave w takes 16 keys in turn, requested as soon as their page is known and before the
+// Block (kv head, sequence), eight to sixteen waves; wave w takes 16 keys in turn, requested as soon as their page is known and before the
 // block redoes the per-token work (sums of squares over the whole q / k projections, its GQ query heads, its key and value).  Lane (c, G) holds dims
 // 16 t + 4 G + i of key c and value dims 64 b + 4 c + x of keys 4 G + i, as in attn_chunk_f32_kernel, but the products are plain f32 fma: of the matrix
 // cores' sixteen columns a token has GQ, and their f32 rate (256 flops a cycle and CU) leaves nothing over for the rest.  The new token joins from LDS.
 // A chain of round trips all the same: 2 x 150 positions, 16 / 8 heads x 128,
-// 11.9 us for the 13.6 + 5.0 of attn_chunk_f32_kernel and qkv_post_f32_kernel.
-constexpr int f32d_waves(int d, int gq) { return d * gq > 256 ? 8 : 16; }   // (four heads of 128: their sums and a unit are more than 128 registers)
+// 11.1 us for the 13.6 + 5.0 of attn_chunk_f32_kernel and qkv_post_f32_kernel.
+constexpr int f32d_waves(int d, int gq) { return d * gq > 256 ? 8 : d * gq > 128 ? 12 : 16; }   // (the heads' sums and a unit of keys in registers)
 constexpr int F32D_COLUMNS = 8192;   // of q and k
 template <int D, int GQ>   // GQ: query heads per kv head, at most
 constexpr int f32d_lds() {
@@ -762,7 +762,7 @@ constexpr int f32d_lds() {
 template <int D, int GQ>
 __global__ __launch_bounds__(f32d_waves(D, GQ) * 64) void attn_chunk_f32_decode_kernel(const float* qkv, const float* bias, const SeqEntry* entries, const uint64_t* tab, int ld, int heads_kvh, int slot, int pos, QkvPostArgs a,
                                                                            ChunkAttnArgs t) {
-  constexpr int NW = f32d_waves(D, GQ), NTH = NW * 64, NT16 = D / 16, NB = D / 64, NC = F32D_COLUMNS / (4 * NTH);
+  constexpr int NW = f32d_waves(D, GQ), NTH = NW * 64, NT16 = D / 16, NB = D / 64, NC = (F32D_COLUMNS + 4 * NTH - 1) / (4 * NTH);
   extern __shared__ __attribute__((aligned(16))) float sm[];
   float *raw = sm, *qs = raw + (GQ + 2) * D, *ks = qs + GQ * D, *vs = ks + D;   // raw: the heads' q, k; then with norm and rotation
   float *os = vs + D, *ml = os + NW * GQ * D, *ll = ml + NW * GQ, *ps = ll + NW * GQ, *fresh = ps + NW * GQ * 16, *red = fresh + GQ;

@@ -477,6 +477,7 @@ __device__ __forceinline__ float sum_stride4(float v) {   // over the sixteen la
   v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x128 /* row_ror:8 */, 0xf, 0xf, false));
   return rows_sum(v);
 }
+enum { STEP_ANY, STEP_FEW, STEP_ONE };
 struct SsmStepLead {   // sizes in two words
   int np_taps_hpg, vdp_groups;
   __host__ __device__ int np() const { return np_taps_hpg & 1023; }
@@ -485,9 +486,10 @@ struct SsmStepLead {   // sizes in two words
   __host__ __device__ int vdp() const { return vdp_groups & 65535; }
   __host__ __device__ int groups() const { return (int)((unsigned)vdp_groups >> 16); }
 };
-template <typename TI, int NI, int VT, bool NT, bool ONE>
+template <typename TI, int NI, int VT, bool NT, int FORM>
 __global__ __launch_bounds__(256) void ssm_step_kernel(const float* sin, const TI* in_c, const float* hin, const float* conv_w, const float* conv_b, int inner, int np_taps_hpg,
                                                        int vdp_groups, int pos0, SsmStepArgs a, SeqBatch b) {
+  constexpr bool ONE = FORM == STEP_ONE;
   __shared__ __attribute__((aligned(16))) float bc[2 * NI * 64], xs[VT * 16], red[4][VT * 16], step[2];
   const SsmStepLead lead{np_taps_hpg, vdp_groups};
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), vdp = lead.vdp(), nvs = vdp >> 4, vs = blockIdx.x * VT, np = lead.np(), taps = lead.taps(), groups = lead.groups();
@@ -541,9 +543,9 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(const float* sin, const T
     if (i >= 2 * np) xs[i - 2 * np] = acc;
     else bc[i < np ? i : NI * 64 + i - np] = acc;
   };
-  const bool few_taps = ONE || (taps >= 2 && taps <= HT + 1);
+  constexpr bool few_taps = FORM != STEP_ANY;
   float cur[NIT], x[NIT][HT];
-  if (few_taps) {
+  if constexpr (few_taps) {
     float wl[NIT], bias[NIT], w[NIT][HT];
 #pragma unroll
     for (int k = 0; k < NIT; ++k) {
@@ -633,7 +635,7 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(const float* sin, const T
     for (int o = 1; o < 16; o <<= 1) s += __shfl_xor(s, o, 16);
     if ((fin & 15) == 0) a.ssq[(int64_t)seq * (inner >> 4) + h * nvs + vs + (fin >> 4)] = s;
   }
-  if (few_taps) {
+  if constexpr (few_taps) {
 #pragma unroll
     for (int k = 0; k < NIT; ++k) {
       const int i = tid + k * 256;
@@ -853,23 +855,25 @@ void launch_ssm_step(const SsmStepArgs& a, const SeqBatch& b, hipStream_t st) {
   const SsmStepLead lead{a.d.np | std::min(a.d.taps, 63) << 10 | hpg << 16, a.d.vdp | a.d.groups << 16};
   auto go = [&](auto ni) {
     constexpr int NI = decltype(ni)::value;
-    auto launch = [&](auto ti, auto vt, auto nt, auto one) {
+    auto launch = [&](auto ti, auto vt, auto nt, auto form) {
       using TI = decltype(ti);
       constexpr int VT = decltype(vt)::value;
-      constexpr bool NT = decltype(nt)::value, ONE = decltype(one)::value;
+      constexpr bool NT = decltype(nt)::value;
+      constexpr int FORM = decltype(form)::value;
       const float *sin = a.s.state, *hin = a.h.hist;
       const TI* in_c = (const TI*)a.in.p + a.in.c_off;
-      if (ONE) {
+      if (FORM == STEP_ONE) {
         sin += (int64_t)b.one.state_in * a.s.pool_stride;
         hin += (int64_t)b.one.slot * a.h.slot_stride + (int64_t)b.one.hist_in * (a.d.taps - 1) * a.d.cp();
         in_c += (int64_t)b.one.row0 * a.in.ld;
       }
-      hipLaunchKernelGGL((ssm_step_kernel<TI, NI, VT, NT, ONE>), grid, block, 0, st, sin, in_c, hin, a.p.conv_w, a.p.conv_b, a.d.inner(), lead.np_taps_hpg, lead.vdp_groups, b.one.pos0, a, b);
+      hipLaunchKernelGGL((ssm_step_kernel<TI, NI, VT, NT, FORM>), grid, block, 0, st, sin, in_c, hin, a.p.conv_w, a.p.conv_b, a.d.inner(), lead.np_taps_hpg, lead.vdp_groups, b.one.pos0, a, b);
     };
     auto run = [&](auto vt, auto nt) {
       auto typed = [&](auto ti) {
-        if (b.has_one && a.d.taps >= 2 && a.d.taps <= 5) launch(ti, vt, nt, std::true_type{});
-        else launch(ti, vt, nt, std::false_type{});
+        if (a.d.taps < 2 || a.d.taps > 5) launch(ti, vt, nt, std::integral_constant<int, STEP_ANY>{});
+        else if (b.has_one) launch(ti, vt, nt, std::integral_constant<int, STEP_ONE>{});
+        else launch(ti, vt, nt, std::integral_constant<int, STEP_FEW>{});
       };
       if (a.in_f32) typed(float{});
       else typed(bf16_t{});
