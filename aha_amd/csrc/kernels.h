@@ -245,7 +245,7 @@ bool gemm_takes_few_rows(const GemmArgs& a);   // (launch_gemm's choice; host on
 double gemm_skinny_plan(const GemmArgs& a, int* r8_out);
 int gemm_skinny_rounds(const GemmArgs& a, int r8);   // blocks of r8 * 8 weight rows over the CUs
 void launch_gemm_skinny(const GemmArgs& a, hipStream_t st);
-// z = up(A), y = down(PolyNorm(z)) for up to 16 rows in two launches; false: not these sizes, nothing is launched (launch_gemm, launch_polynorm_rows, launch_gemm)
+// z = up(A), y = down(PolyNorm(z)) for up to 16 rows in two launches (elsewhere launch_gemm, launch_polynorm_rows, launch_gemm)
 struct SkinnyPoly {
   float* stats;                // gemm_skinny_poly_floats()
   int parts;
