@@ -844,6 +844,17 @@ void launch_ssm_chunks(const SsmScanArgs& a, const SeqBatch& b, float* scratch, 
 
 void launch_ssm_step(const SsmStepArgs& a, const SeqBatch& b, hipStream_t st) {
   if (b.n <= 0) return;
+  if (const int most = 65535 / a.d.groups; b.n > most) {   // (the grid's z)
+    SsmStepArgs rest = a;
+    rest.g += (int64_t)most * a.d.inner();
+    rest.ssq += (int64_t)most * (a.d.inner() >> 4);
+    SeqBatch first = b, later = b;
+    first.n = most;
+    later.n -= most;
+    later.entries += most;
+    launch_ssm_step(a, first, st);
+    return launch_ssm_step(rest, later, st);
+  }
   const int nvs = a.d.vdp >> 4;
   const bool wide = nvs % 4 == 0 && (int64_t)a.d.heads * nvs / 4 * b.n >= 512;   // B and C of the group once per 64 columns
   // From 16 MB of states per launch on, past the caches: nothing reads them before the next step, and they push out what is read (128 dims of state, 16 MB:
