@@ -159,7 +159,7 @@ struct aha_model {
   unsigned long long* d_attn_trace = nullptr;  // AHA_ATTN_TRACE timeline
   bool decode_fused = true;  // attention block of a decode step in one launch (kernels_attn.hip attn_decode_fused_kernel)
   float* h_logits = nullptr;  // pinned
-  bool step_in_flight = false;   // model_forward_step_enqueue: the stream has not been waited for since (model_wait_step)
+  bool step_in_flight = false;   // a step was queued (model_forward_step_enqueue, or one that failed behind its first launch) and not waited for since (model_wait_step)
   bool have_logits = false;   // d_logits holds the logits of a completed forward call
   bool logits_assembled = false;  // vocab-parallel TP: d_logits already all-reduced into the full vector
   // D11 candidate extraction (kernels_sample.hip), allocated on first use

@@ -958,6 +958,7 @@ int model_fetch_outputs(aha_model* m, float* logits_out, uint32_t* argmax_out) {
   if (logits_out) AHA_HIP_CHECK(hipMemcpyAsync(m->h_logits, m->d_logits, (size_t)c.vocab_size * 4, hipMemcpyDeviceToHost, m->stream));
   AHA_HIP_CHECK(hipMemcpyAsync(&m->h_state->next_token, &m->d_state->next_token, 4, hipMemcpyDeviceToHost, m->stream));
   AHA_HIP_CHECK(hipStreamSynchronize(m->stream));
+  m->step_in_flight = false;
   if (m->d_gemv_trace) gemv_trace_dump(m);
   if (m->d_attn_trace) {
     const int L = m->desc.num_hidden_layers;
@@ -1578,6 +1579,9 @@ static int enqueue_forward_step(aha_model* m, uint32_t token, size_t offset, boo
   }
   const int64_t pos[3] = {p, p, p};
   if ((rc = push_state(m, token, pos, m->cache_len, m->cache_len + 1))) return rc;
+  // from here on work is queued that overwrites the logits, and an error below returns without waiting for it
+  m->step_in_flight = true;
+  m->have_logits = false;
   enqueue_decode_step(m, m->cache_len + 1, false, arg_max);
   m->cache_len += 1;
   AHA_HIP_CHECK(hipGetLastError());
@@ -1606,7 +1610,6 @@ int model_forward_step_enqueue(aha_model* m, uint32_t token, size_t offset) {
   if ((rc = enqueue_forward_step(m, token, offset, false))) return rc;
   m->have_logits = true;
   m->logits_assembled = false;
-  m->step_in_flight = true;
   return AHA_OK;
 }
 

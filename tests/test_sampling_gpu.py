@@ -238,3 +238,40 @@ def test_enqueued_steps(gpu):
         np.testing.assert_array_equal(m.forward_step(toks[2], 122)[0], want[2])
     finally:
         m.close()
+
+
+@pytest.mark.parametrize("enqueue", [False, True])
+def test_a_step_that_fails_behind_its_launches(gpu, enqueue):
+    """An all-reduce that fails in the middle of a step: the step's logits are nobody's (those of the call before are overwritten by then), what was queued is
+    waited for by the next call, and the model goes on from an empty cache."""
+    from aha_amd.model import HipInferenceModel
+    cfg = tiny_qwen3(layers=3, hidden=256, heads=4, kv_heads=2, inter=512, vocab=512)
+    fail = []
+
+    def summed(ptr, count):   # (one rank alone: its partial sums as they are)
+        if fail and not fail.pop():
+            raise RuntimeError("no partner")
+
+    m = HipInferenceModel(cfg, qwen3_text_weights(cfg, seed=0), tp_rank=0, tp_size=2, allreduce=summed)
+    try:
+        def go():
+            m.clear_cache()
+            m.forward_initial([5, 6, 7], 0, want_logits=False)
+            return m.forward_step(8, 3)[0]
+        want = go()
+        np.testing.assert_array_equal(m.last_logits(), want)
+        fail += [False, True, True]   # the third of the step's sums
+        with pytest.raises(_lib.AhaHipError):
+            if enqueue:
+                m.forward_step_enqueue(9, 4)
+            else:
+                m.forward_step(9, 4)
+        assert not fail
+        with pytest.raises(_lib.AhaHipError):
+            m.last_logits()
+        with pytest.raises(_lib.AhaHipError):
+            m.sample_candidates([], 1.0, 1.0, 4)
+        np.testing.assert_array_equal(go(), want)
+        np.testing.assert_array_equal(m.last_logits(), want)
+    finally:
+        m.close()
