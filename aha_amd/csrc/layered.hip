@@ -334,7 +334,7 @@ Tail run_rows(aha_model* m, const SeqBatch& b, const SeqEntry* h_ents, const uin
         const double keys = d.chunk > 0 ? std::min<double>(d.chunk, h_ents[i].pos0 + h_ents[i].len) : h_ents[i].pos0 + h_ents[i].len;
         flops += 2.0 * h_ents[i].len * keys * 0.5 * d.heads * (d.dim + d.vdim);
       }
-      ProfScope ps(m, "attn_prefill", (double)rows * d.heads * (W.dq + W.dvo) * es, flops);
+      ProfScope ps(m, "attn_prefill", (double)rows * (one_launch ? W.nqkv + W.nk + W.nv + d.heads * W.dvo : d.heads * (W.dq + W.dvo)) * es, flops);
       if (one_launch) launch_chunk_attn_f32_decode(qp, a, b, st);
       else if (W.frag) launch_chunk_attn_prefill(a, b, st);
       else launch_chunk_attn_rows(a, b, l.f32, st);

@@ -1466,6 +1466,7 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_read
   int defer = e_div || !m->decode_fused ? 0 : attn_decode_defer_splits(npages, nq);
   if (defer > 1 && m->tp_size > 1) defer = 0;
   const int slices = e_div || !m->decode_fused || !m->d_part_y ? 0 : attn_decode_slice_splits(npages);
+  const int n_sums = slices < 0 ? kvh : slices > 0 ? nq / 512 : 0;   // o_proj's f32 sums of H, added up by gate + up
   if (slices) defer = std::abs(slices);
   if (defer) nsplit = defer;
   // pages at one distance from each other: the attention computes their addresses
@@ -1508,18 +1509,21 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_read
       g.W = L.wo; g.x = m->d_attn; g.residual = m->d_x; g.y = m->d_x; g.N = H; g.K = nq;
       g.trace = gemv_trace_slot(m, li * 4 + 1);
       const double attn_bytes = (double)kv_len_after * 2 * nkv * 2 + (nq + 2 * nkv) * 2.0 + nsplit * nq * 4.0;
-      const double gemv_bytes = (double)g.N * g.K * 2 + g.K * 2.0 + g.N * 4.0;
-      {
-        ProfScope ps(m, "attn_decode", attn_bytes, 4.0 * kv_len_after * nq);
-        if (slices < 0) launch_attn_oproj(a, L.wo, m->d_part_y, H, st);
-        else if (defer) launch_attn_decode_defer(a, st);
-        else launch_attn_decode_fused(a, st);
+      const double o_bytes = (double)g.N * g.K * 2 + (slices ? n_sums * H * 4.0 : g.N * 4.0), o_flops = 2.0 * g.N * g.K;
+      if (slices < 0) {   // (one launch: o_proj's weights are read by it)
+        ProfScope ps(m, "attn_decode", attn_bytes + o_bytes, 4.0 * kv_len_after * nq + o_flops);
+        launch_attn_oproj(a, L.wo, m->d_part_y, H, st);
+      } else {
+        {
+          ProfScope ps(m, "attn_decode", attn_bytes, 4.0 * kv_len_after * nq);
+          if (defer) launch_attn_decode_defer(a, st);
+          else launch_attn_decode_fused(a, st);
+        }
+        ProfScope ps(m, "gemv", o_bytes + g.K * 2.0, o_flops);
+        if (slices) launch_oproj_slices(GemvMerge{m->d_part_o, m->d_part_ml, nsplit, nh}, L.wo, m->d_part_y, H, st);
+        else if (defer > 1) launch_gemv_merge(g, GemvMerge{m->d_part_o, m->d_part_ml, nsplit, nh}, st);
+        else gemv_row_parallel(m, g);
       }
-      ProfScope ps(m, "gemv", gemv_bytes, 2.0 * g.N * g.K);
-      if (slices > 0) launch_oproj_slices(GemvMerge{m->d_part_o, m->d_part_ml, nsplit, nh}, L.wo, m->d_part_y, H, st);
-      else if (slices < 0) {   // (o_proj is done)
-      } else if (defer > 1) launch_gemv_merge(g, GemvMerge{m->d_part_o, m->d_part_ml, nsplit, nh}, st);
-      else gemv_row_parallel(m, g);
     } else {  // three-launch variant (A/B knob AHA_DECODE_FUSED=0)
       {  // q/k norm + rope + append                            (modules.rs:544-566)
         RopeArgs r{};
@@ -1548,8 +1552,8 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_read
       GemvArgs g{};
       g.W = L.wgu; g.W2 = nullptr; g.x = m->d_x; g.norm_w = L.post_norm; g.eps = c.rms_norm_eps; g.y = m->d_act; g.N = I; g.K = H;
       g.trace = gemv_trace_slot(m, li * 4 + 2);
-      ProfScope ps(m, "gemv", (double)2 * I * H * 2 + H * 4.0 + I * 2.0, 4.0 * I * H);
-      if (slices) launch_gemv_slices(g, m->d_part_y, slices < 0 ? kvh : nq / 512, m->d_x2, st);
+      ProfScope ps(m, "gemv", (double)2 * I * H * 2 + H * 4.0 + I * 2.0 + n_sums * H * 4.0, 4.0 * I * H);
+      if (slices) launch_gemv_slices(g, m->d_part_y, n_sums, m->d_x2, st);
       else launch_gemv(g, GEMV_SILU_MUL, st);
     }
     {  // x = x + act Wd^T                                     (modules.rs:85, qwen3/model.rs:86)

@@ -70,6 +70,28 @@ def test_projection_in_slices(gpu, monkeypatch, lens, scrambled):
     sliced.close(); plain.close()
 
 
+@pytest.mark.parametrize("positions, launches", [(20, 3), (500, 4), (1200, 4)])
+def test_profile_of_the_projection_in_slices(gpu, positions, launches):
+    """Bytes and launches are booked where they run: o_proj's weights with the attention where one launch does both (20 positions), with the matvecs elsewhere."""
+    from aha_amd.model import HipInferenceModel
+    H, nq, nkv, I, V, layers = 1024, 2048, 1024, 1536, 1024, 3
+    cfg = tiny_qwen3(layers=layers, hidden=H, heads=16, kv_heads=8, inter=I, vocab=V)
+    m = HipInferenceModel(cfg, qwen3_text_weights(cfg, seed=14))
+    m.forward_initial(ids_for(cfg, positions, 3), 0)
+    m.set_profiling(True)
+    m.forward_step(5, positions)
+    m.set_profiling(False)
+    gemv, attn = m.get_profile("gemv"), m.get_profile("attn_decode")
+    m.close()
+    o = nq * H
+    weights = layers * ((nq + 2 * nkv) * H + 3 * I * H + (0 if launches == 3 else o)) + V * H
+    cache = layers * (positions + 1) * 2 * nkv
+    assert gemv["launches"] == layers * launches + 1 and attn["launches"] == layers
+    assert 2 * weights <= gemv["bytes"] <= 1.02 * 2 * weights and 2 * weights <= gemv["flops"] <= 1.02 * 2 * weights
+    both = 2 * (cache + (layers * o if launches == 3 else 0))
+    assert both <= attn["bytes"] <= 1.02 * both + layers * (17 * nq * 4 + 8 * H * 4)   # (the splits' partials, the slices' sums)
+
+
 @pytest.mark.parametrize("hidden, vocab", [(256, 64), (256, 5000), (1024, 70001)])
 def test_between_two_steps(gpu, hidden, vocab):
     """The launch between two steps of the greedy loop (arg-max, state, embedding row, rope table) against the same tokens fed one by one: the kernels
