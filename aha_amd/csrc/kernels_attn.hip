@@ -186,15 +186,15 @@ __global__ __launch_bounds__(256, 2) void attn_oproj_kernel(const void* qkv, con
   a.k_norm_w = k_norm_w;
   a.rope = rope;
   a.kv.page_ptrs = page_ptrs;
-  const int kvh = kvh_len >> 20;
+  const int kvh = kvh_len >> 21;
   a.kv_len_v = kvh_len & 0xfffff;
   a.page_stride = page_stride;
   a.group = 2;
   a.kvh = kvh;
   a.nh = 2 * kvh;
-  a.traced = 0;
   float* o = reinterpret_cast<float*>(smem_defer);
   const int kvhd = (int)blockIdx.x, slab = (int)blockIdx.y;
+  a.traced = (kvh_len >> 20 & 1) && slab == 0;
   OprojRows<4, 256> rows;
   const int row0 = rows.row0(slab, ATTN_DECODE_NW);
   attn_decode_fused_body<ATTN_DECODE_NW, true, true>(a, smem_defer + 256 * 4, kvhd, 0, 1, o, slab == 0, [&] { rows.request((const bf16_t*)W, 256 * kvh, kvhd, row0); });
@@ -205,8 +205,8 @@ __global__ __launch_bounds__(256, 2) void attn_oproj_kernel(const void* qkv, con
 }  // namespace
 
 void launch_attn_oproj(const AttnDecodeFusedArgs& a, const void* W, float* y, int n, hipStream_t st) {
-  hipLaunchKernelGGL(attn_oproj_kernel, dim3(a.kvh, n / 32), dim3(256), 256 * 4 + ATTN_DEFER_LDS(2), st, a.qkv, a.q_norm_w, a.k_norm_w, a.rope, a.kv.page_ptrs, W, a.kvh << 20 | a.kv_len_v,
-                     a.page_stride, a, y, n);
+  hipLaunchKernelGGL(attn_oproj_kernel, dim3(a.kvh, n / 32), dim3(256), 256 * 4 + ATTN_DEFER_LDS(2), st, a.qkv, a.q_norm_w, a.k_norm_w, a.rope, a.kv.page_ptrs, W,
+                     a.kvh << 21 | (a.trace != nullptr) << 20 | a.kv_len_v, a.page_stride, a, y, n);
 }
 
 void launch_attn_decode_fused(const AttnDecodeFusedArgs& a, hipStream_t st) {

@@ -256,10 +256,10 @@ __global__ __launch_bounds__(256) void oproj_slice_kernel(const float* part_o, c
   rows.multiply(hs, y + slice * n, row0);
 }
 template <int P>
-__global__ __launch_bounds__(GEMV_THREADS) void gemv_row_slices_kernel(const void* x, const float* parts, const void* W, const void* norm_w, void* x_out, int N, float eps, int nblk, GemvArgs rest) {
+__global__ __launch_bounds__(GEMV_THREADS) void gemv_row_slices_kernel(const void* x, const float* parts, const void* W, const void* norm_w, void* x_out, unsigned long long* trace, int N, float eps, int nblk, GemvArgs rest) {
   __shared__ __attribute__((aligned(16))) float xs[1024 + 4];
   RowSlicesPro<P> pro{(const bf16_t*)x, (const bf16_t*)norm_w, parts, (bf16_t*)x_out, eps, (int)blockIdx.x, xs};
-  gemv_row_body<1, 2, GEMV_SILU_MUL>(rest, W, nullptr, nullptr, N, (int)blockIdx.x, nblk, pro);
+  gemv_row_body<1, 2, GEMV_SILU_MUL>(rest, W, nullptr, trace, N, (int)blockIdx.x, nblk, pro);
 }
 template <int R, int U, bool FAST, int XP, int MS, int KX = 0>
 __global__ __launch_bounds__(GEMV_THREADS) void gemv_merge_kernel(const float* part_o, const float* part_ml, const void* W, const void* residual, unsigned long long* trace, int N, int K, int nsplit, int nblk,
@@ -362,7 +362,7 @@ void launch_oproj_slices(const GemvMerge& p, const void* W, float* y, int n, hip
 }
 void launch_gemv_slices(const GemvArgs& a, const float* parts, int n, void* x_out, hipStream_t st) {
   const int nblk = gemv_row_grid(a.N, 1);
-  auto go = [&](auto k) { hipLaunchKernelGGL(k, dim3(nblk), dim3(GEMV_THREADS), 0, st, a.x, parts, a.W, a.norm_w, x_out, a.N, a.eps, nblk, a); };
+  auto go = [&](auto k) { hipLaunchKernelGGL(k, dim3(nblk), dim3(GEMV_THREADS), 0, st, a.x, parts, a.W, a.norm_w, x_out, a.trace, a.N, a.eps, nblk, a); };
   if (n == 4) go(gemv_row_slices_kernel<4>);
   else go(gemv_row_slices_kernel<8>);
 }

@@ -1399,6 +1399,7 @@ __global__ __launch_bounds__(1024) void next_step_kernel(const float* __restrict
 }
 
 // AHA_GEMV_TRACE=1: in-kernel timeline of the decode matvecs (launch-per-op path), dumped by fetch_outputs
+// (o_proj in slices: the attention's launch, or one of its own without stamps)
 static unsigned long long* gemv_trace_slot(aha_model* m, int launch_idx) {
   static const char* e = getenv("AHA_GEMV_TRACE");
   if (!e || !atoi(e)) return nullptr;
@@ -1422,6 +1423,7 @@ static void gemv_trace_dump(aha_model* m) {
     for (int li = 1; li < L; ++li) {
       const unsigned long long* p = t.data() + (size_t)(li * 4 + k) * 18;
       const unsigned long long* prev = p - 18;
+      if (prev[4] == 0) prev -= 18;   // (o_proj in slices is not traced)
       if (p[0] == 0 || prev[4] == 0) continue;
       for (int b = 0; b < 3; ++b)
         for (int j = 0; j < 4; ++j) d[b][j] += (double)(p[b * 6 + j + 1] - p[b * 6 + j]) * 0.01;
@@ -1451,6 +1453,9 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_read
   const int H = c.hidden_size, I = c.intermediate_size, d = c.head_dim, nh = c.num_attention_heads, kvh = c.num_key_value_heads;
   const int nq = nh * d, nkv = kvh * d;
   hipStream_t st = m->stream;
+  // the timelines: a launch that this step does not have, or does not trace, leaves zeros
+  if (m->d_gemv_trace) launch_row_to_f32(nullptr, (float*)m->d_gemv_trace, (4 * c.num_hidden_layers + 1) * 18 * 2, st);
+  if (m->d_attn_trace) launch_row_to_f32(nullptr, (float*)m->d_attn_trace, c.num_hidden_layers * 12 * 2, st);
   if (!row_ready) {
     ProfScope ps(m, "elem", H * 4.0, 0);
     hipLaunchKernelGGL(embed_state_kernel, dim3(1), dim3(256), 0, st, (const bf16_t*)m->embed, m->d_state, (bf16_t*)m->d_x, H,

@@ -151,3 +151,35 @@ print("LOGITS", h.hexdigest())
         assert r.returncode == 0, r.stderr[-2000:]
         seen.append([ln for ln in r.stdout.splitlines() if ln.startswith("LOGITS")][0])
     assert seen[0] == seen[1]
+
+
+def test_timelines_of_the_projection_in_slices(gpu):
+    """AHA_GEMV_TRACE and AHA_ATTN_TRACE (read once per process: a child): the attention and gate + up leave their stamps in every form; o_proj has a line where
+    it is a traced launch (500 positions) and none, not that of the step before, where it is not (20 and 1200)."""
+    import os
+    import subprocess
+    import sys
+    code = """
+import sys
+from aha_amd.configs import tiny_qwen3
+from aha_amd.model import HipInferenceModel
+from aha_amd.weights import qwen3_text_weights
+from tests.test_model_gpu import ids_for
+cfg = tiny_qwen3(layers=3, hidden=1024, heads=16, kv_heads=8, inter=1536, vocab=1024)
+m = HipInferenceModel(cfg, qwen3_text_weights(cfg, seed=4))
+for S in (500, 20, 500, 1200):
+    m.clear_cache()
+    _, tok = m.forward_initial(ids_for(cfg, S, S), 0)
+    print("positions", S, file=sys.stderr, flush=True)
+    m.forward_step(tok, S)
+    print("end", file=sys.stderr, flush=True)
+m.close()
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", code], cwd=root, env=dict(os.environ, PYTHONPATH=root, AHA_GEMV_TRACE="1", AHA_ATTN_TRACE="1"), capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
+    for part in r.stderr.split("positions ")[1:]:
+        S = int(part.split()[0])
+        part = part.split("\nend")[0].splitlines()
+        assert [ln.split()[2] for ln in part if ln.startswith("[gemv trace]")] == ["qkv"] + ["o_proj"] * (S == 500) + ["gate_up", "down"], S
+        assert [ln.split()[3] for ln in part if ln.startswith("[attn trace]")] == ["0:"] + ["1:"] * (S > 20), S
