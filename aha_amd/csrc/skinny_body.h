@@ -107,13 +107,16 @@ __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R
     for (int r = 0; r < NF; ++r)
 #pragma unroll
       for (int m = 0; m < MT; ++m) acc[h][r][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  auto load = [&](int u, int ch) {
-    ch += first;
-    const int k = (ch < nc ? ch : ch - nc) * 128, ka = F32 ? 2 * k : k;
+  const int end = nc * 128;
+  int k = (first + wave < nc ? first + wave : first + wave - nc) * 128;   // the next chunk to request, in bytes of a weight row
+  auto load = [&](int u) {
+    const int ka = F32 ? 2 * k : k;
 #pragma unroll
     for (int r = 0; r < R8; ++r) __builtin_amdgcn_global_load_lds((glb_t)(src[r] + k), (lds_t)(ring + (u * PER + r) * 1024), 16, 0, 2);   // weights: non-temporal
 #pragma unroll
     for (int r = R8; r < PER; ++r) __builtin_amdgcn_global_load_lds((glb_t)(src[r] + ka), (lds_t)(ring + (u * PER + r) * 1024), 16, 0, 0);
+    k += SKINNY_WAVES * 128;
+    k -= k < end ? 0 : end;
   };
   // an odd count leaves half a fragment without rows: its lanes read the other half's again (behind the last stage there may be no LDS)
   const int cw = R8 % 2 ? c & 7 : c, ca = M8 % 2 ? c & 7 : c;   // (of the last fragment)
@@ -165,14 +168,14 @@ __device__ __forceinline__ void skinny_sums(const char* (&src)[skinny_requests(R
   pro.request();
 #pragma unroll
   for (int s = 0; s < S; ++s)
-    if (PRO::ON || wave + s * SKINNY_WAVES < nc) load(s, wave + s * SKINNY_WAVES);
+    if (PRO::ON || wave + s * SKINNY_WAVES < nc) load(s);
   if constexpr (PRO::ON) __builtin_amdgcn_sched_barrier(0);
   pro.join();
   for (; ch + S * SKINNY_WAVES < nc; ch += SKINNY_WAVES) {   // S stages are on their way: the oldest is in when the later ones' requests are left
     __builtin_amdgcn_s_waitcnt(0x0F70 | (LEFT & 15) | ((LEFT >> 4) << 14));
     __builtin_amdgcn_sched_barrier(0);
     consume(u);
-    load(u, ch + S * SKINNY_WAVES);
+    load(u);
     u = u + 1 == S ? 0 : u + 1;
   }
   for (; ch < nc; ch += SKINNY_WAVES) {   // the last ones: as many behind this one as there are chunks left

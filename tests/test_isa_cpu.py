@@ -146,6 +146,33 @@ def test_hot_kernels_have_no_flat_loads(kernels, tmp_path):
     assert not bad, f"flat loads / scratch in hot kernels: { {k: v[:3] for k, v in bad.items()} }"
 
 
+def test_few_row_products_request_before_scalar_loads(kernels, tmp_path):
+    """What a few-row product's first requests need comes with the launch, in scalar registers: an argument that is read from memory in front of them costs
+    its round trip, 0.25 to 0.35 us of launches of 3 to 15 us (csrc/kernels_gemm_skinny.hip skinny_product).  Behind the entry's copy of the arguments for
+    firmware that does not preload them, nothing waits for a scalar load before the first request of the ring."""
+    shutil.copy(os.path.join(ROOT, "aha_amd", "csrc", "libaha_hip.so"), tmp_path / "lib.so")
+    subprocess.run([f"{LLVM}/llvm-objdump", "--offloading", "lib.so"], cwd=tmp_path, capture_output=True, check=True)
+    few = ("gemm_skinny_kernel",)
+    seen, bad = {}, []
+    for o in sorted(glob.glob(str(tmp_path / "lib.so.*gfx950"))):
+        names = [n for n in subprocess.run([f"{LLVM}/llvm-readelf", "--symbols", "--wide", o], capture_output=True, text=True, check=True).stdout.split()
+                 if n.startswith("_Z") and not n.endswith(".kd") and family(n) in few]
+        if not names:
+            continue
+        dis = subprocess.run([f"{LLVM}/llvm-objdump", "-d", "--no-show-raw-insn", "--disassemble-symbols=" + ",".join(names), o], capture_output=True, text=True, check=True).stdout
+        for part in re.split(r"^[0-9a-f]+ <(?=_Z)", dis, flags=re.M)[1:]:
+            name, body = part.split(">:", 1)
+            ops = [ln.strip() for ln in body.splitlines() if ln.strip()]
+            entry = next(i for i, op in enumerate(ops) if op.startswith("s_branch"))   # (over the copy for old firmware)
+            first = next(i for i, op in enumerate(ops) if op.startswith("global_load_lds"))
+            assert entry < 12 < first, name
+            seen[family(name)] = seen.get(family(name), 0) + 1
+            if any(op.startswith("s_waitcnt") and "lgkmcnt" in op for op in ops[entry + 1:first]):
+                bad.append(name)
+    assert seen.get("gemm_skinny_kernel", 0) >= 28, seen
+    assert not bad, bad
+
+
 def test_no_packed_f32_arithmetic(tmp_path):
     """Some operand forms of `v_pk_{add,mul,fma}_f32` were measured on MI355X to read the wrong element when the wave shares a SIMD with a
     wave of a kernel on another stream (profiles/r03_simd_coresidency.md), and clang forms them from ordinary float code.  The library is
