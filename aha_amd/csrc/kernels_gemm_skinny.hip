@@ -98,23 +98,26 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const vo
 // A launch of its own between an up and a down projection of up to 16 rows is a link of the chain like any other, for 8 x 12288 numbers (4.9 us).  Here the
 // first product leaves, beside its bf16 result z, the sums of z^2, z^4 and z^6 over each block's columns, [block][M8 * 8 rows]; the second joins them while its
 // first stages are on their way and maps the fragments that it reads from LDS: three fma and a rounding per number, under the wait for the weights.
-// 8 rows, 12288 x 4096 and back: 17.0 + 4.9 + 16.8 us in three launches, 17.1 + 19.1 in two; 12 layers of 8B sizes, 8 requests and 32 steps 39.0 -> 38.0 ms.
+// 8 rows, 12288 x 4096 and back: 39.3 us in three launches, 38.0 in two (gemm_takes_poly: where it pays); 12 layers of 8B sizes, 8 requests and 32 steps 39.0 -> 38.0 ms.
+// The sums' place and number come with the launch, as all that stands in front of the first requests.
 constexpr int POLY_PARTS = 256;   // blocks of the first product, at most
 template <int M8>
-struct SkinnyPolyIn {
+struct SkinnyPolyIn {   // stats, parts: from the leading arguments (skinny_product)
   static constexpr bool ON = true;
   static constexpr int R = M8 * 8, PER = 64 / R, NL = POLY_PARTS / (PER * SKINNY_WAVES);
   static_assert(M8 == 1 || M8 == 2, "one activation fragment");
   const SkinnyPoly& p;
+  const float* stats;
+  int parts;
   f32x4_t (*red)[16];   // [SKINNY_WAVES]
   f32x4_t v[NL];
   float r1 = 0.f, r2 = 0.f, r3 = 0.f, e = 0.f;
-  __device__ __forceinline__ SkinnyPolyIn(const SkinnyPoly& p_, f32x4_t (*red_)[16]) : p(p_), red(red_) {}
+  __device__ __forceinline__ SkinnyPolyIn(const SkinnyPoly& p_, const float* stats_, int parts_, f32x4_t (*red_)[16]) : p(p_), stats(stats_), parts(parts_), red(red_) {}
   __device__ __forceinline__ int part(int j) const { return (j * SKINNY_WAVES + (int)(threadIdx.x >> 6)) * PER + (int)(threadIdx.x & 63) / R; }
   __device__ __forceinline__ void request() {
-    const f32x4_t* at = reinterpret_cast<const f32x4_t*>(p.stats) + (threadIdx.x & (R - 1));
+    const f32x4_t* at = reinterpret_cast<const f32x4_t*>(stats) + (threadIdx.x & (R - 1));
 #pragma unroll
-    for (int j = 0; j < NL; ++j) v[j] = at[min(part(j), p.parts - 1) * R];
+    for (int j = 0; j < NL; ++j) v[j] = at[min(part(j), parts - 1) * R];
   }
   __device__ __forceinline__ void join() {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -122,7 +125,7 @@ struct SkinnyPolyIn {
 #pragma unroll
     for (int j = 0; j < NL; ++j)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) mine[i] += part(j) < p.parts ? v[j][i] : 0.f;
+      for (int i = 0; i < 4; ++i) mine[i] += part(j) < parts ? v[j][i] : 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if (R == 8) mine[i] += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(mine[i]), 0x128 /* row_ror:8 */, 0xf, 0xf, false));
@@ -155,7 +158,8 @@ struct SkinnyPolyIn {
 };
 // IN: the second product, else the first.  bf16 results, no bias, residual or activation.
 template <int R8, int M8, bool DEEP, bool IN>
-__global__ __launch_bounds__(SKINNY_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1, 4))) void gemm_skinny_poly_kernel(const void* A, const void* W, int M, int N, int K, int spread, int64_t lda, int64_t ldw, SkinnyPoly p, GemmArgs a) {
+__global__ __launch_bounds__(SKINNY_WAVES * 64) __attribute__((amdgpu_waves_per_eu(1, 4))) void gemm_skinny_poly_kernel(const void* A, const void* W, int M, int N, int K, int parts_spread, int64_t lda, int64_t ldw, float* stats, SkinnyPoly p, GemmArgs a) {
+  const int spread = parts_spread & 1;
   constexpr int NF = (R8 + 1) / 2, R = M8 * 8;
   __shared__ f32x4_t red[SKINNY_WAVES][16];
   auto epilogue = [&](int wave, int lane) {
@@ -185,11 +189,11 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) __attribute__((amdgpu_waves_per_
         f32x4_t v = red[0][threadIdx.x];
 #pragma unroll
         for (int r = 1; r < NF; ++r) v += red[r][threadIdx.x];
-        reinterpret_cast<f32x4_t*>(p.stats)[blockIdx.x * R + threadIdx.x] = v;
+        reinterpret_cast<f32x4_t*>(stats)[blockIdx.x * R + threadIdx.x] = v;
       }
     }
   };
-  if constexpr (IN) skinny_product<R8, M8, false, DEEP>(A, W, M, N, K, spread, lda, ldw, a, SkinnyPolyIn<M8>(p, red), epilogue);
+  if constexpr (IN) skinny_product<R8, M8, false, DEEP>(A, W, M, N, K, spread, lda, ldw, a, SkinnyPolyIn<M8>(p, stats, parts_spread >> 1, red), epilogue);
   else skinny_product<R8, M8, false, DEEP>(A, W, M, N, K, spread, lda, ldw, a, SkinnyPlain{}, epilogue);
 }
 
@@ -288,7 +292,7 @@ void launch_poly_one(const GemmArgs& a, const SkinnyPoly& p, hipStream_t st) {
   constexpr int lds = skinny_lds(R8, M8, false, DEEP);
   auto k = gemm_skinny_poly_kernel<R8, M8, DEEP, IN>;
   if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  hipLaunchKernelGGL(k, dim3((unsigned)((a.N + R8 * 8 - 1) / (R8 * 8))), dim3(SKINNY_WAVES * 64), lds, st, a.A, a.W, a.M, a.N, a.K, skinny_spread(a), a.lda, a.ldw, p, a);
+  hipLaunchKernelGGL(k, dim3((unsigned)((a.N + R8 * 8 - 1) / (R8 * 8))), dim3(SKINNY_WAVES * 64), lds, st, a.A, a.W, a.M, a.N, a.K, p.parts << 1 | skinny_spread(a), a.lda, a.ldw, p.stats, p, a);
 }
 
 template <bool IN>

@@ -152,7 +152,7 @@ def test_few_row_products_request_before_scalar_loads(kernels, tmp_path):
     firmware that does not preload them, nothing waits for a scalar load before the first request of the ring."""
     shutil.copy(os.path.join(ROOT, "aha_amd", "csrc", "libaha_hip.so"), tmp_path / "lib.so")
     subprocess.run([f"{LLVM}/llvm-objdump", "--offloading", "lib.so"], cwd=tmp_path, capture_output=True, check=True)
-    few = ("gemm_skinny_kernel",)
+    few = ("gemm_skinny_kernel", "gemm_skinny_poly_kernel")
     seen, bad = {}, []
     for o in sorted(glob.glob(str(tmp_path / "lib.so.*gfx950"))):
         names = [n for n in subprocess.run([f"{LLVM}/llvm-readelf", "--symbols", "--wide", o], capture_output=True, text=True, check=True).stdout.split()
@@ -169,7 +169,7 @@ def test_few_row_products_request_before_scalar_loads(kernels, tmp_path):
             seen[family(name)] = seen.get(family(name), 0) + 1
             if any(op.startswith("s_waitcnt") and "lgkmcnt" in op for op in ops[entry + 1:first]):
                 bad.append(name)
-    assert seen.get("gemm_skinny_kernel", 0) >= 28, seen
+    assert seen.get("gemm_skinny_kernel", 0) >= 28 and seen.get("gemm_skinny_poly_kernel", 0) >= 24, seen
     assert not bad, bad
 
 
