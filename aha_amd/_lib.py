@@ -163,6 +163,7 @@ SIGNATURES = {
     "aha_hip_debug_expert_choice": (C.c_int, [_P, C.c_int32, C.c_int32, _P, _P]),
     "aha_hip_set_gemm_reserved_cus": (C.c_int, [C.c_int32]),
     "aha_hip_debug_few_rows_gemm": (C.c_int, [C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_size_t]),
+    "aha_hip_debug_poly_plan": (C.c_int, [C.c_int32, C.c_int32, C.c_int32, C.c_size_t]),
     "aha_hip_debug_plan_gemm": (C.c_int, [C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_size_t, _P]),
     "aha_hip_get_rope_index": (C.c_int, [_P, _P, C.c_size_t, _P, C.c_int32, _P, _P]),
     "aha_hip_get_rope_index_mm": (C.c_int, [_P, _P, C.c_size_t, _P, C.c_int32, _P, C.c_int32, _P, _P]),

@@ -361,6 +361,13 @@ int aha_hip_debug_few_rows_gemm(int32_t M, int32_t N, int32_t K, int32_t act, in
   int o[3];
   return debug_plan_gemm(M, N, K, act, has_bias != 0, (has_residual & 1) != 0, workspace_bytes, o, (has_residual & 2) != 0);
 }
+int aha_hip_debug_poly_plan(int32_t rows, int32_t width, int32_t ff, size_t workspace_bytes) {
+  if (rows <= 0 || width <= 0 || ff <= 0) {
+    set_error("debug_poly_plan: bad argument");
+    return AHA_ERR_INVALID;
+  }
+  return debug_poly_plan(rows, width, ff, workspace_bytes);
+}
 int aha_hip_debug_streamk_plan(int32_t M, int32_t N, int32_t K, int32_t tile_n, int32_t workers, size_t workspace_bytes, int32_t* out,
                                int32_t cap, int32_t* off_out, int32_t* info7) {
   if (!out || cap < 0 || M <= 0 || N <= 0 || K <= 0) {

@@ -254,7 +254,8 @@ struct SkinnyPoly {
 bool gemm_skinny_poly_ok(const GemmArgs& up, const GemmArgs& down);
 size_t gemm_skinny_poly_floats();
 void launch_gemm_skinny_poly(const GemmArgs& up, const GemmArgs& down, SkinnyPoly p, hipStream_t st);
-bool gemm_takes_poly(const GemmArgs& up, const GemmArgs& down);   // gemm_skinny_poly_ok, and launch_gemm would take the few-row kernel for both
+bool gemm_takes_poly(const GemmArgs& up, const GemmArgs& down);   // gemm_skinny_poly_ok, launch_gemm would take the few-row kernel for both, and it is the faster way
+int debug_poly_plan(int rows, int width, int ff, size_t ws_bytes);
 // One launch over all row segments on the four-wave 256 x 256 / 256 x 192 kernels (plain and gate+up epilogues, whole K tiles, M >= 256);
 // any other shape: one launch_gemm per segment.  On the same kernel every output element is the same K-ordered sum as in an ungrouped GEMM over its
 // row; a short segment's own plan may be another (K slices, the few-row kernel).

@@ -1334,7 +1334,30 @@ bool gemm_takes_few_rows(const GemmArgs& a_in) {
   return gemm_skinny_ok(a) && takes_few_rows(a, plan_gemm(a), &r8);
 }
 
-bool gemm_takes_poly(const GemmArgs& up, const GemmArgs& down) { return gemm_skinny_poly_ok(up, down) && gemm_takes_few_rows(up) && gemm_takes_few_rows(down); }
+// PolyNorm inside the two products around it: up to 8 rows wherever both run here (at most 0.2 us behind three launches, 1024 x 4096 and 2 rows, 1.5 ahead).  More rows
+// cost the second product the mapping of whole fragments, which hides under its weights from 64 MB on.  us in three / two launches, 12 rows, up and down of
+// 1024 x 3072: 13.4 / 14.5, 2048 x 6144: 20.2 / 21.0, 4096 x 4096: 19.4 / 20.5, 3072 x 8192: 26.1 / 27.4, 4096 x 6144: 25.0 / 25.4, 3840 x 8192 (63 MB): 29.4 / 29.5,
+// 4096 x 8192: 30.5 / 30.1, 6400 x 6656: 38.8 / 38.1, 4096 x 12288: 40.8 / 40.2; 9 and 16 rows fall on the same sides but for 3840 x 8192 at 16 (30.3 / 30.1).
+bool gemm_takes_poly(const GemmArgs& up, const GemmArgs& down) {
+  return gemm_skinny_poly_ok(up, down) && (down.M <= 8 || (int64_t)down.N * down.K * 2 >= 64 << 20) && gemm_takes_few_rows(up) && gemm_takes_few_rows(down);
+}
+int debug_poly_plan(int rows, int width, int ff, size_t ws_bytes) {
+  static int dummy;
+  GemmArgs up{}, down{};
+  for (GemmArgs* a : {&up, &down}) {
+    a->M = rows;
+    a->N = a == &up ? ff : width;
+    a->K = a->lda = a->ldw = a == &up ? width : ff;
+    a->ldc = a->N;
+    a->workspace = ws_bytes ? &dummy : nullptr;
+    a->workspace_bytes = ws_bytes;
+  }
+  if (!gemm_takes_poly(up, down)) return 0;
+  int r_up = 0, r_down = 0;
+  gemm_skinny_plan(up, &r_up);
+  gemm_skinny_plan(down, &r_down);
+  return r_up * 8 | r_down * 8 << 8;
+}
 
 void launch_gemm(const GemmArgs& a_in, hipStream_t st) {
   if (a_in.M <= 0 || a_in.N <= 0) return;

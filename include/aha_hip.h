@@ -446,6 +446,9 @@ int aha_hip_debug_plan_gemm(int32_t M, int32_t N, int32_t K, int32_t act, int32_
 /* Host only (no GPU): the few-row kernel's weight rows per block (16, 24, 32 or 48) where the launcher takes that kernel instead of the plan above
  * (csrc/kernels_gemm_skinny.hip), 0 where the plan above runs. */
 int aha_hip_debug_few_rows_gemm(int32_t M, int32_t N, int32_t K, int32_t act, int32_t has_bias, int32_t has_residual, size_t workspace_bytes);
+/* Host only (no GPU): weight rows per block of the up product | those of the down product << 8 where PolyNorm runs inside the two products of a layer list's
+ * feed-forward (csrc/kernels_gemm.hip gemm_takes_poly; padded sizes), 0 where it is a launch of its own. */
+int aha_hip_debug_poly_plan(int32_t rows, int32_t width, int32_t ff, size_t workspace_bytes);
 /* Host only (no GPU): the segment lists the persistent GEMM kernel (csrc/kernels_gemm_sk.hip) would walk for a shape on `workers`
  * workgroups (a multiple of 8) with `tile_n` (256 | 192) column tiles: out = 8 ints per segment {m0, n0, first K tile, end K tile,
  * pieces the tile is cut into, this piece's index in K order, first chunk of the tile, counter of the tile}, grouped by worker;

@@ -340,6 +340,18 @@ def test_few_row_gemm_where_it_is_the_faster_one(hip_lib):
         assert rows(0, 1, 1) >= 0
 
 
+def test_polynorm_inside_its_products_where_it_is_the_faster_way(hip_lib):
+    """csrc/kernels_gemm.hip gemm_takes_poly: up to 8 rows wherever both products are few-row products of one round, 9 to 16 rows from 64 MB of weights on (both
+    sides measured at the sizes here); never more rows, fewer than 24 chunks of k in the second product or more than 256 blocks in the first."""
+    def plan(rows, width, ff):
+        return hip_lib.aha_hip_debug_poly_plan(rows, width, ff, 32 << 20)
+    assert [plan(M, 1024, 3072) for M in (2, 8, 9, 16)] == [16 | 16 << 8] * 2 + [0] * 2
+    assert [plan(M, 4096, 6144) > 0 for M in (8, 9, 16)] == [plan(M, 3840, 8192) > 0 for M in (8, 9, 16)] == [True, False, False]
+    assert [plan(M, 4096, 8192) for M in (8, 9, 16)] == [32 | 16 << 8] * 3 and [plan(M, 4096, 12288) for M in (8, 9, 16, 17)] == [48 | 16 << 8] * 3 + [0]
+    assert plan(8, 1024, 1472) == plan(8, 4608, 9216) == 0
+    assert hip_lib.aha_hip_debug_poly_plan(0, 1024, 3072, 0) < 0
+
+
 @pytest.mark.parametrize("S", [512, 1542, 2048, 8192, 40980, 131072])
 @pytest.mark.parametrize("world", [2, 3, 4, 8])
 def test_context_parallel_plan_partitions_the_prompt(hip_lib, S, world):
