@@ -342,24 +342,24 @@ int aha_hip_debug_gemm_plan(int32_t tile, int32_t splitk) {
   set_gemm_plan_override(tile, splitk);
   return AHA_OK;
 }
-int aha_hip_debug_plan_gemm(int32_t M, int32_t N, int32_t K, int32_t act, int32_t has_bias, int32_t has_residual, size_t workspace_bytes,
+int aha_hip_debug_plan_gemm(int32_t M, int32_t N, int32_t K, int32_t act, int32_t bias, int32_t has_residual, size_t workspace_bytes,
                             int32_t* out3) {
   if (!out3 || M <= 0 || N <= 0 || K <= 0) {
     set_error("debug_plan_gemm: bad argument");
     return AHA_ERR_INVALID;
   }
   int o[3];
-  debug_plan_gemm(M, N, K, act, has_bias != 0, (has_residual & 1) != 0, workspace_bytes, o, (has_residual & 2) != 0);
+  debug_plan_gemm(M, N, K, act, bias, (has_residual & 1) != 0, workspace_bytes, o, (has_residual & 2) != 0);
   out3[0] = o[0]; out3[1] = o[1]; out3[2] = o[2];
   return AHA_OK;
 }
-int aha_hip_debug_few_rows_gemm(int32_t M, int32_t N, int32_t K, int32_t act, int32_t has_bias, int32_t has_residual, size_t workspace_bytes) {
+int aha_hip_debug_few_rows_gemm(int32_t M, int32_t N, int32_t K, int32_t act, int32_t bias, int32_t has_residual, size_t workspace_bytes) {
   if (M <= 0 || N <= 0 || K <= 0) {
     set_error("debug_few_rows_gemm: bad argument");
     return AHA_ERR_INVALID;
   }
   int o[3];
-  return debug_plan_gemm(M, N, K, act, has_bias != 0, (has_residual & 1) != 0, workspace_bytes, o, (has_residual & 2) != 0);
+  return debug_plan_gemm(M, N, K, act, bias, (has_residual & 1) != 0, workspace_bytes, o, (has_residual & 2) != 0);
 }
 int aha_hip_debug_poly_plan(int32_t rows, int32_t width, int32_t ff, size_t workspace_bytes) {
   if (rows <= 0 || width <= 0 || ff <= 0) {

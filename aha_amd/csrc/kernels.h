@@ -232,6 +232,10 @@ struct GemmArgs {
   int tile_group = 8;            // band width of the grouped tile order inside an XCD's run (kernels_gemm.hip tile_of_block); 0 = plain
   int few_rows = 1;              // the few-row kernel (kernels_gemm_skinny.hip): 0 never, 1 where it is expected to be faster, 2 wherever it can
   int few_rows_spread = 1;       // ... whose blocks start at different k (skinny_first); 0: all at k = 0, so that column blocks of a projection sum as the whole does
+  int tower_order = 0;           // 1: the tiled plan, and with it the order of the sums, of an image tower whatever its price: where reduce passes of < 1 M outputs and narrow
+                                 // results are priced as they run (plan_gemm), towers of a few hundred patches would take other plans (640 x 1152 x 4352 20.1 us for
+                                 // 26.8).  The stack behind them is bf16: another order moves the 8B model's logits by 3.1 % of their spread -- no further from 64 bits
+                                 // (2.7 % either way), but further from what the same weights and image gave
   int partial_rows = 1;          // ACT_PARTIAL_F32 on the four-wave kernel: f32 sums stored in row order through LDS (0: fragment order; A/B)
   // Row groups (launch_gemm_grouped; tensor-parallel prefill: the staging layout of the chunked all-gather, csrc/model.hip
   // norm_gather_gemm): `groups` row segments of M rows each share W.  Segment g reads A rows [g * a_gstride, + M) and writes C rows
@@ -276,7 +280,7 @@ bool acquire_gemm_cu_reservation(int cus);   // the automatic, reference-counted
 void release_gemm_cu_reservation();
 int debug_streamk_plan(int M, int N, int K, int tile_n, int workers, int group, size_t ws_bytes, int* out, int cap, int* off_out, int* info);
 // host only: {tile, splitk, n_split} of the tiled kernels; returns the few-row kernel's weight rows per block where that one is taken, else 0
-int debug_plan_gemm(int M, int N, int K, int act, bool has_bias, bool has_res, size_t ws_bytes, int* out, bool has_norm = false);
+int debug_plan_gemm(int M, int N, int K, int act, int bias, bool has_res, size_t ws_bytes, int* out, bool has_norm = false);
 void set_gemm_plan_override(int tile, int splitk);  // tests: force the 128 / 256 tile kernel and a split-K factor; 0 = automatic
 void get_gemm_workspace(void** ws, size_t* bytes, void** sk_counters);
 struct GemmWorkspaceScope {   // nests: the vision tower's own workspace inside the prefill's

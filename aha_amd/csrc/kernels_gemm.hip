@@ -1089,10 +1089,10 @@ GemmPlan plan_gemm(const GemmArgs& a) {
   const bool ring128 = t128 <= (double)gemm_streamk_cus() && nk >= 4;
   // (a norm riding on the call is folded into a split plan's reduce pass; behind an unsplit ring launch it is a ~6-us launch of its own --
   // cfg 2 o_proj, 2048 x 1024 x 2048: 23.1 us unsplit against 27.6 us as 256^2 x 4 slices, but 4.99 against 4.57 ms per prefill)
-  // Up to 2048 columns (behind them no vision tower's or 8B stack's sums): a ring launch at its own k step whatever the depth -- 0.68 us is a CU's that holds four
+  // Up to 2048 columns (measured there; an 8B stack's have more): a ring launch at its own k step whatever the depth -- 0.68 us is a CU's that holds four
   // blocks -- and 5 us for the norm: 2432 x 1024 x 3072 and its norm 36.5 us as three slices of 192 columns, 32.4 here (1024 x 2048 / 3072 at 256 to 4096 rows: 18
   // to 22.7 us by the rule's 20.5, 24.9 to 30.8 by 28.5).
-  const bool narrow = a.N <= 2048 && !a.bias && ring128;
+  const bool narrow = a.N <= 2048 && !a.tower_order && ring128;
   const double cost128 = narrow ? nk * lat_ring + 4.5 + (a.norm_w ? 5.0 : 0.0)
                                            : std::max(ceil(t128 / 256.0) * nk * 0.68, t128 < 512.0 ? nk * (ring128 ? lat_ring : lat128) + 4.5 : 0.0) + (ring128 && a.norm_w ? 6.0 : 0.0);
   const bool can_split = a.act != ACT_SILU_MUL_PAIRS && a.act != ACT_PARTIAL_F32 && a.workspace != nullptr && (a.N & 3) == 0;
@@ -1118,10 +1118,8 @@ GemmPlan plan_gemm(const GemmArgs& a) {
   static const bool ring_sk_on = [] { const char* e = getenv("AHA_GEMM_RING_SPLITK"); return e ? atoi(e) != 0 : true; }();
   // bytes per us: a reduce pass of < 1 M outputs does not fill the chip, whichever tiles it sums.  With the 256-row plans' passes at 4 TB/s all the same, 512 to 976
   // rows of 1024 columns and their like took them: 768 x 1024 x 2048 24.9 -> 15.7 us, 640 x 1024 x 3072 23.0 -> 16.4, 384 x 2048 x 2048 24.6 -> 17.5,
-  // 512 x 1536 x 4096 25.5 -> 19.4; the best 256-row plan of 43 such shapes is 5 to 10 us behind the best here.  Calls with a bias (vision towers) keep the plans
-  // they had, at 640 x 1152 x 4352 26.8 us for 20.1: the stack behind them is bf16, and another order of a tower's sums moves the 8B model's logits by 3.1 % of
-  // their spread -- no further from 64 bits (2.7 % either way), but further from what the same weights gave.
-  const double red_rate = (double)a.M * a.N < 1.0e6 ? 2.0e6 : 4.0e6, red_rate256 = a.bias ? 4.0e6 : red_rate;
+  // 512 x 1536 x 4096 25.5 -> 19.4; the best 256-row plan of 43 such shapes is 5 to 10 us behind the best here.  (tower_order: a rule about bits, not a price.)
+  const double red_rate = (double)a.M * a.N < 1.0e6 ? 2.0e6 : 4.0e6, red_rate256 = a.tower_order ? 4.0e6 : red_rate;
   // (f32 slabs of narrow results, written: 2432 x 1024 x 3072 in three slices 32.8 us, 30.2 without; a norm in the reduce pass 1.5 us)
   auto slabs_us = [&](int sk) { return narrow ? sk * (double)a.M * a.N * 4.0 / 5.0e6 + (a.norm_w ? 1.5 : 0.0) : 3.0; };
   if (ring_sk_on && can_split && nk >= 24 && !e_tile && !(e_sk && atoi(e_sk) == 1)) {   // (K >= 1536: below, the slices save ~2 us by the model -- inside its error)
@@ -1271,11 +1269,12 @@ static bool takes_few_rows(const GemmArgs& a, const GemmPlan& plan, int* r8) {
 // The launch(es) launch_gemm would issue for a shape, without issuing them (host only): out[0..2] = {tile, splitk, 1 if the columns are
 // split into a multiple of 256 + a tail launch}.  `ws_bytes` > 0 stands for a caller workspace of that size.  These are the tiled kernels' plans:
 // returns the few-row kernel's weight rows per block where launch_gemm takes that one instead, else 0.
-int debug_plan_gemm(int M, int N, int K, int act, bool has_bias, bool has_res, size_t ws_bytes, int* out, bool has_norm) {
+int debug_plan_gemm(int M, int N, int K, int act, int bias, bool has_res, size_t ws_bytes, int* out, bool has_norm) {
   GemmArgs a{};
   a.M = M; a.N = N; a.K = K; a.lda = K; a.ldw = K; a.ldc = act == ACT_SILU_MUL_PAIRS ? N / 2 : N; a.act = act;
   static int dummy;
-  a.bias = has_bias ? &dummy : nullptr;
+  a.bias = bias ? &dummy : nullptr;
+  a.tower_order = bias == 1;
   a.residual = has_res ? &dummy : nullptr;
   a.norm_w = has_norm ? &dummy : nullptr;
   a.workspace = ws_bytes ? &dummy : nullptr;

@@ -231,6 +231,7 @@ static void vgemm(aha_model* m, const void* A, const void* W, void* C, int M, in
   g.A = A; g.W = W; g.C = C; g.M = M; g.N = N; g.K = K; g.lda = K; g.ldw = K; g.ldc = ldc ? ldc : N; g.bias = bias; g.residual = residual; g.act = act;
   if (ln_w) { g.norm_w = ln_w; g.norm_b = ln_b; g.norm_out = ln_out; g.norm_eps = 1e-6f; }
   ProfScope ps(m, "gemm", ((double)M * K + (double)N * K + (double)M * N * (residual ? 2 : 1)) * 2, 2.0 * M * N * K);
+  g.tower_order = 1;
   g.few_rows = 0;   // an image encoded by itself gives the rows it gives among others (image-parallel encoding), and real ones have more rows
   launch_gemm(g, m->stream);
 }

@@ -438,14 +438,15 @@ int aha_hip_debug_attn_form(int32_t form);
  * 192-column tiles wherever it has an instantiation and a workspace (128^2 kernel elsewhere). */
 int aha_hip_debug_gemm_plan(int32_t tile, int32_t splitk);
 /* Host only (no GPU): the plan the GEMM launcher would pick among its tiled kernels for a shape -- out3 = {tile (128 | 256), split-K factor, 1 if the
- * columns run as a multiple of 256 + a tail launch}; workspace_bytes = size of the caller's split-K scratch (0 = none); has_residual
+ * columns run as a multiple of 256 + a tail launch}; workspace_bytes = size of the caller's split-K scratch (0 = none); bias
+ * 1 = as an image tower calls it (a bias, the order of its sums kept: GemmArgs::tower_order), 2 = a bias alone; has_residual
  * bit 0 = a residual is added, bit 1 = an RMSNorm of the output rides on the call (o_proj / down_proj in the layer loop).  Lets the
  * CPU tier pin the plans of the BASELINE shapes (csrc/kernels_gemm.hip plan_gemm is a cost model fitted on MI355X). */
-int aha_hip_debug_plan_gemm(int32_t M, int32_t N, int32_t K, int32_t act, int32_t has_bias, int32_t has_residual, size_t workspace_bytes,
+int aha_hip_debug_plan_gemm(int32_t M, int32_t N, int32_t K, int32_t act, int32_t bias, int32_t has_residual, size_t workspace_bytes,
                             int32_t* out3);
 /* Host only (no GPU): the few-row kernel's weight rows per block (16, 24, 32 or 48) where the launcher takes that kernel instead of the plan above
  * (csrc/kernels_gemm_skinny.hip), 0 where the plan above runs. */
-int aha_hip_debug_few_rows_gemm(int32_t M, int32_t N, int32_t K, int32_t act, int32_t has_bias, int32_t has_residual, size_t workspace_bytes);
+int aha_hip_debug_few_rows_gemm(int32_t M, int32_t N, int32_t K, int32_t act, int32_t bias, int32_t has_residual, size_t workspace_bytes);
 /* Host only (no GPU): weight rows per block of the up product | those of the down product << 8 where PolyNorm runs inside the two products of a layer list's
  * feed-forward (csrc/kernels_gemm.hip gemm_takes_poly; padded sizes), 0 where it is a launch of its own. */
 int aha_hip_debug_poly_plan(int32_t rows, int32_t width, int32_t ff, size_t workspace_bytes);

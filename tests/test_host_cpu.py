@@ -305,7 +305,8 @@ def test_gemm_plans_of_the_baseline_shapes(hip_lib):
 @pytest.mark.parametrize("M,N,K,bias,norm,want", [
     (512, 1024, 3072, 0, 1, (128, 4)), (640, 1024, 3072, 0, 1, (128, 4)), (768, 1024, 2048, 0, 1, (128, 3)), (976, 1024, 3072, 0, 1, (128, 4)), (384, 2048, 2048, 0, 0, (128, 3)),   # under 1 M outputs
     (2048, 1024, 3072, 0, 1, (128, 2)), (2304, 1024, 3072, 0, 1, (128, 1)), (2432, 1024, 3072, 0, 1, (128, 1)), (4096, 1024, 3072, 0, 1, (128, 1)), (2432, 1024, 2048, 0, 0, (128, 1)),   # one block per CU
-    (768, 1024, 2048, 1, 1, (256, 4)), (2432, 1024, 3072, 1, 1, (192, 3)), (5067, 1024, 2048, 0, 0, (192, 2)),   # with a bias, or more blocks than CUs: as without either
+    (768, 1024, 2048, 1, 1, (256, 4)), (2432, 1024, 3072, 1, 1, (192, 3)), (5067, 1024, 2048, 0, 0, (192, 2)),   # as an image tower calls it (its plans are kept), or more blocks than CUs: as without either
+    (768, 1024, 2048, 2, 1, (128, 3)), (2432, 1024, 3072, 2, 1, (128, 1)), (640, 1152, 4352, 1, 0, (256, 8)), (640, 1152, 4352, 2, 0, (128, 4)),   # a bias alone costs nothing
 ])
 def test_gemm_plans_of_narrow_results(hip_lib, M, N, K, bias, norm, want):
     out = (ctypes.c_int32 * 3)()
