@@ -517,6 +517,16 @@ int aha_hip_debug_gemm_grouped(const void* A, const void* W, void* C, int32_t M,
   return AHA_OK;
 }
 
+int aha_hip_debug_gemm_f32(const float* A, const void* W, float* C, int32_t M, int32_t N, int32_t K, int32_t batch, void* stream) {
+  if (!A || !W || !C || M <= 0 || N <= 0 || K <= 0 || batch <= 0 || batch > 65535) {
+    set_error("debug_gemm_f32: bad argument");
+    return AHA_ERR_INVALID;
+  }
+  launch_gemm_f32(A, K, W, K, C, N, M, N, K, (hipStream_t)stream, batch, (int64_t)M * K, (int64_t)N * K, (int64_t)M * N);
+  AHA_HIP_CHECK(hipGetLastError());
+  return AHA_OK;
+}
+
 int aha_hip_qknorm_rope(const void* qkv, const void* q_norm_w, const void* k_norm_w, const int32_t* pos,
                         const int32_t* axis_map, void* q_out, void* k_out, void* v_out, int32_t S, int32_t nh,
                         int32_t kvh, int32_t d, float eps, float theta, void* stream) {

@@ -420,6 +420,8 @@ int aha_hip_debug_poison_lds(uint32_t seed, void* stream);
  * [c_row0 + g * c_gstride, + M) (row pitch ldc), clipped to rows < m_total.  act: plain (0) or gate+up pairs (4). */
 int aha_hip_debug_gemm_grouped(const void* A, const void* W, void* C, int32_t M, int32_t N, int32_t K, int32_t ldc, int32_t act,
                                int32_t groups, int32_t a_gstride, int32_t c_gstride, int32_t c_row0, int32_t m_total, void* stream);
+/* Test entry of the layer lists' 32-bit products (csrc/kernels_gemm_f32.hip): C (M, N) f32 = A (M, K) f32 . W (N, K)^T bf16, `batch` of them one behind another. */
+int aha_hip_debug_gemm_f32(const float* A, const void* W, float* C, int32_t M, int32_t N, int32_t K, int32_t batch, void* stream);
 /* Test hook: the prefill attention's score chain.  3 (the default since round 5; env AHA_ATTN_SMX) = the scores stay the f32 QK^T
  * accumulators through scale, mask, maximum and exponential, P is rounded to bf16 once for the P.V product; 1 / 0 = the reference's
  * eager path, which materialises `q.k^T` and `* scaling` in bf16 (modules.rs:782-783), with the scale multiply on the matrix pipe
