@@ -303,16 +303,19 @@ void launch_poly(const GemmArgs& a, const SkinnyPoly& p, int r8, hipStream_t st)
   };
   if (r8 == 2) go(std::integral_constant<int, 2>{});
   else if (r8 == 3) go(std::integral_constant<int, 3>{});
-  else if (r8 == 4) go(std::integral_constant<int, 4>{});
-  else go(std::integral_constant<int, 6>{});
+  else if (IN || r8 == 4) go(std::integral_constant<int, 4>{});
+  else if constexpr (!IN) go(std::integral_constant<int, 6>{});
 }
 
 }  // namespace
 
-// K of 24 chunks and more: the deepest ring's first requests (skinny_sums)
+// K of 24 chunks and more: the deepest ring's first requests (skinny_sums).  A second product of 48 weight rows per block has more than 8192 columns, the
+// widest that a layer list can be.
 bool gemm_skinny_poly_ok(const GemmArgs& up, const GemmArgs& down) {
   if (up.M > 16 || down.M != up.M || down.K != up.N || down.K < 24 * 64) return false;
   int r8 = 2;
+  gemm_skinny_plan(down, &r8);
+  if (r8 > 4) return false;
   gemm_skinny_plan(up, &r8);
   return (up.N + r8 * 8 - 1) / (r8 * 8) <= POLY_PARTS;
 }

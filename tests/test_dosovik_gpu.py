@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 import torch
 
+from aha_amd import _lib
 from aha_amd.configs_layered import DosovikConfig, LayerConfig
 from aha_amd.model import HipContext, HipInferenceModel, generate_generic
 from aha_amd.weights_layered import dosovik_weights
@@ -185,6 +186,27 @@ def test_polynorm_between_few_row_products(ctx, width, ff, rows):
         seqs = [m.seq_open() for _ in range(rows)]
         m.forward_batch([(s, x[:2], []) for s, x in zip(seqs, ids)])
         got, _ = m.forward_batch([(s, x[2:], [0]) for s, x in zip(seqs, ids)])
+    want = np.stack([reference(cfg, w, x)[-1] for x in ids])
+    assert err(got, want) <= TOL["bfloat16"]
+
+
+# PolyNorm inside the two products around it: (width, ff, rows, weight rows per block of the up product, of the down product).  Every block width of either product
+# with one group of eight rows and with two (from 64 MB on, csrc/kernels_gemm.hip gemm_takes_poly), pad columns among them.
+POLY = [(1030, 1599, 2, 16, 16), (1024, 6208, 7, 32, 16), (832, 4100, 8, 24, 16), (768, 8256, 8, 48, 16), (4130, 1536, 8, 16, 24), (6210, 1536, 5, 16, 32), (4096, 12288, 9, 48, 16), (4096, 8192, 16, 32, 16),
+        (8190, 4096, 16, 16, 32), (6100, 5504, 13, 24, 24)]
+
+
+@pytest.mark.parametrize("width,ff,rows,up,down", POLY)
+def test_polynorm_inside_every_form_of_the_products(ctx, width, ff, rows, up, down):
+    """The launch has to be the fused pair, of the block widths named; each row against the restatement."""
+    assert {_lib.lib().aha_hip_debug_poly_plan(rows, -(-width // 256) * 256, -(-ff // 64) * 64, ws) for ws in (0, 32 << 20, 96 << 20)} == {up | down << 8}
+    cfg = config([layer(heads=2, kv_heads=1, dim=64, vdim=64, ff=ff)], width=width, vocab=130, taps=3 if width < 2048 else 1, dtype="bfloat16")
+    w = dosovik_weights(cfg, seed=33)
+    ids = [tokens(2, cfg.vocab_size, seed=60 + i) for i in range(rows)]
+    with Model(ctx, cfg, w) as m:
+        seqs = [m.seq_open() for _ in range(rows)]
+        m.forward_batch([(s, x[:1], []) for s, x in zip(seqs, ids)])
+        got, _ = m.forward_batch([(s, x[1:], [0]) for s, x in zip(seqs, ids)])
     want = np.stack([reference(cfg, w, x)[-1] for x in ids])
     assert err(got, want) <= TOL["bfloat16"]
 
