@@ -93,7 +93,7 @@ struct SsmSegments {
   float* cum;                        // [entry][segment][head]: sum of a dt
   int n, chunks;                     // segments per entry, chunks per segment
 };
-bool ssm_chunk_ok(const SsmDims& d);                                                         // sizes launch_ssm_chunks takes
+bool ssm_chunk_ok(const SsmDims& d);                                                         // sizes launch_ssm_chunks and launch_ssm_step take
 size_t ssm_segment_floats(const SsmDims& d);                                                 // scratch with which no prompt runs in fewer segments than it could
 // bf16 rows, 64 tokens at a time on the matrix cores; long prompts in segments beside each other, whose states are in `scratch`
 void launch_ssm_chunks(const SsmScanArgs& a, const SeqBatch& b, float* scratch, size_t scratch_floats, hipStream_t st);

@@ -478,7 +478,10 @@ __device__ __forceinline__ float sum_stride4(float v) {   // over the sixteen la
   return rows_sum(v);
 }
 enum { STEP_ANY, STEP_FEW, STEP_ONE };
-struct SsmStepLead {   // sizes in two words
+constexpr int SSM_CHUNK_NP = 256;   // state dims (padded) of launch_ssm_chunks and launch_ssm_step, at most (ssm_chunk_ok)
+// sizes in two words; a model's heads times their padded columns fit the LDS (layered_prenorm.hip), so heads, groups and columns fit sixteen bits
+struct SsmStepLead {
+  static_assert(SSM_CHUNK_NP < 1024, "np has ten bits");
   int np_taps_hpg, vdp_groups;
   __host__ __device__ int np() const { return np_taps_hpg & 1023; }
   __host__ __device__ int taps() const { return np_taps_hpg >> 10 & 63; }   // (63: that many or more)
@@ -774,7 +777,7 @@ void launch_ssm_scan(const SsmScanArgs& a, const SeqBatch& b, bool f32, hipStrea
   else go(ssm_scan_kernel<bf16_t>);
 }
 
-bool ssm_chunk_ok(const SsmDims& d) { return d.np <= 256; }
+bool ssm_chunk_ok(const SsmDims& d) { return d.np <= SSM_CHUNK_NP; }
 
 // Columns (16 VT of them) per block and segments per entry of a launch: enough blocks for the chip where the prompt has the chunks, at least two chunks
 // per segment

@@ -604,6 +604,22 @@ def test_decoding_where_tiles_end(ctx, rank, rot, window):
     assert err(got, want[at]) <= TOL["bfloat16"]
 
 
+@pytest.mark.parametrize("groups,state,conv,rows", [(256, 8, 4, 257), (512, 4, 7, 254)])
+def test_steps_in_parts(ctx, groups, state, conv, rows):
+    """launch_ssm_step: groups x sequences beyond the grid's 65535 go in parts (255 sequences at 256 groups, 127 at 512); a second part of two sequences and a
+    full one, whose logits come from what the step before left of state and history; against the restatement."""
+    cfg = config([ssm(heads=groups, vdim=8, state=state, groups=groups, norm_groups=8, conv=conv, mlp=None)], width=64, vocab=64, dtype="bfloat16", cap=0.0)
+    w = vamatar_weights(cfg, seed=21)
+    ids = [tokens(4, cfg.vocab_size, seed=70 + i) for i in range(rows)]
+    want = [reference(cfg, w, x) for x in ids]
+    with Model(ctx, cfg, w) as m:
+        seqs = [m.seq_open() for _ in ids]
+        m.forward_batch([(s, x[:2], []) for s, x in zip(seqs, ids)])
+        for at in (2, 3):
+            got, _ = m.forward_batch([(s, x[at:at + 1], [0]) for s, x in zip(seqs, ids)])
+            assert err(got, np.stack([r[at] for r in want])) <= TOL["bfloat16"]
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 128, 200])
 def test_a_token_far_back_in_the_state(ctx, dtype, n):
