@@ -319,13 +319,11 @@ void launch_layernorm_rows(const void* x, const void* w, const void* b, void* y,
 void launch_pos_embed_add(void* x, const void* table, const int32_t* idx, const float* wt, int64_t N, int D,
                           hipStream_t st);
 struct VitRopeArgs {
-  const void* qkv;          // (N, 3*nh*hd) bf16: [q heads | k heads | v heads]
-  const int32_t* rowcol;    // (N, 2) patch (row, col)
-  const float* inv_freq;    // (hd/4)
+  const void* qkv;          // (N, 3*nh*72) bf16: [q heads | k heads | v heads] of 72 dims, the only head dim that a tower is created with
   void* q_out;              // (N, nh, VIT_DQK) bf16, zero padded
   KvLayer kv;               // pages: K block [nh][64][VIT_DQK], V block [nh][VIT_DV][64]
-  int N, nh, hd;
-  const float* cs_tab = nullptr;   // (N, hd/2, 2) f32: bf16-rounded (cos, sin) per patch and rotary lane (launch_vit_rope_table)
+  int nh;
+  const float* cs_tab = nullptr;   // (N, 36, 2) f32: bf16-rounded (cos, sin) per patch and rotary lane (launch_vit_rope_table)
   const int32_t* page_first = nullptr;  // (n_pages) first token of each page (a page holds consecutive tokens of one segment)
   const int32_t* page_cnt = nullptr;    // (n_pages) tokens in the page (64 except a segment's last page)
   int n_pages = 0;

@@ -220,7 +220,7 @@ void launch_vit_rope_table(const int32_t* rowcol, const float* inv_freq, int N, 
   hipLaunchKernelGGL(vit_rope_table_kernel, dim3((unsigned)(((int64_t)N * (hd / 2) + 255) / 256)), dim3(256), 0, st, rowcol, inv_freq, N, hd, tab);
 }
 void launch_vit_rope_pack(const VitRopeArgs& a, hipStream_t st) {
-  if (a.N <= 0) return;
+  if (a.n_pages <= 0) return;
   hipLaunchKernelGGL(vit_rope_pack_kernel, dim3((unsigned)((a.n_pages + 7) / 8 * 8 * a.nh)), dim3(256), 0, st, a);
 }
 

@@ -447,8 +447,7 @@ int vision_forward_and_scatter(aha_model* m, const uint32_t* ids, size_t n, cons
     vgemm(m, v->h, b.qkv_w, v->qkv, (int)N, 3 * v->D, v->D, b.qkv_b, nullptr, ACT_NONE);
     {
       VitRopeArgs r{};
-      r.qkv = v->qkv; r.rowcol = v->d_rowcol; r.inv_freq = v->d_inv_freq;
-      r.q_out = v->q; r.kv = kv; r.N = (int)N; r.nh = v->nh; r.hd = v->hd; r.cs_tab = v->d_cs_tab;
+      r.qkv = v->qkv; r.q_out = v->q; r.kv = kv; r.nh = v->nh; r.cs_tab = v->d_cs_tab;
       r.page_first = v->d_page_first; r.page_cnt = v->d_page_cnt; r.n_pages = (int)pages;
       ProfScope ps(m, "elem", (double)N * v->D * 3 * 4, 0);
       launch_vit_rope_pack(r, st);
