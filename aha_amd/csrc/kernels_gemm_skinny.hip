@@ -10,7 +10,11 @@
 // Rows past M, N repeat the last one, lanes of a fragment that no row backs another row; what they give is not stored: an MFMA's output rows and columns
 // do not mix.
 //
-// Up to 64 rows blocks start at different k (skinny_first; row tiles of more rows: no difference, and they keep the common start).
+// Up to 64 rows blocks start at different k (skinny_first; row tiles of more rows: no difference in time, and they keep the common start).  The start is a
+// rotation of the sum's order, by the weight row in the matrix that the call is given and from K = 2048 on.  So an element is the same sum in a call of 1 to 64 rows and
+// another in one of 65 to 256, as it already is where the tiles take over; and a tensor-parallel rank's columns (a matrix of its own, its rows counted from the shard's
+// first) are summed in another order than the whole matrix' -- the same rounding, not the same bits.  Row-parallel blocks, cut into columns or not by how
+// the collective overlaps, keep the common start (GemmArgs::few_rows_spread).
 //
 // Measured on MI355X, back to back from HBM, 8 rows (in brackets: the split-K ring kernel + its reduce pass it replaces, inside a batched step):
 //   6144 x 4096 9.9 us (5.1 TB/s), 4096 x 4096 7.2, 12288 x 4096 17.0 (5.9), 4096 x 12288 16.9 (6.0), 24576 x 4096 31.4 (6.4)

@@ -354,6 +354,9 @@ void launch_gemv_merge(const GemvArgs& a, const GemvMerge& p, hipStream_t st) {
   else go(integral_constant<int, 1>{}, integral_constant<int, 1>{});
 }
 
+// The sizes that both kernels and the norm behind them are written for, which are the only ones measured: a slice of 256 columns and a wave's 128-dim heads, 1024 columns of
+// x, a float4 per thread (RowSlicesPro).  Other stacks keep o_proj in a launch of its own.  What decides is not the sizes but that o_proj's 4 MB take less time than the
+// link of the chain that its launch is; at 2048 columns they are 8 to 16 MB, and the norm would read twice the slices in front of gate + up.
 bool oproj_slices_ok(int width, int heads, int kv_heads, int head_dim, int ff) {
   return width == 1024 && heads == 16 && kv_heads == 8 && head_dim == 128 && gemv_row_groups(ff, width, GEMV_SILU_MUL) == 2 && plan_gemv(ff, width, GEMV_SILU_MUL).R == 1;
 }
