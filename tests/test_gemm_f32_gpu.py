@@ -7,9 +7,9 @@ from aha_amd._lib import check, lib
 
 pytestmark = pytest.mark.gpu
 
-# The weights are bf16 and an f32 activation is the sum of its three bf16 parts, so nothing is lost but in the f32 sums: up to 3.4e-7 of the results' spread
-# at K = 3072, growing as its root.  Without the third part an activation is cut behind 16 bits, by 2^-17 of its value in the mean and always towards zero:
-# 5e-6 of the spread at any K (2^-9 without the second).  In between, three times the sums' error:
+# The weights are bf16 and an f32 activation is the sum of its three bf16 parts, so nothing is lost but in the f32 sums: 1 to 4e-7 of the results' spread.
+# Without the third part every row is off by 0.6 to 1.4e-5 of it at K = 64 to 3072 (computed with the part left out, in 64 bits), without the second by 2.5 to 4.2e-3.
+# In between:
 BOUND = 1e-6
 
 
