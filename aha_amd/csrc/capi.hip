@@ -296,6 +296,17 @@ int aha_hip_debug_memory_limit(aha_model* m, size_t bytes) {
   m->mem_left = bytes;
   return AHA_OK;
 }
+int aha_hip_debug_decode_stack(aha_model* m, int32_t polls, int64_t* steps, int64_t* given_up) {
+  if (!m) {
+    set_error("null model");
+    return AHA_ERR_INVALID;
+  }
+  if (int rc = model_wait_step(m)) return rc;
+  if (polls >= 0) m->stack_polls = polls;
+  if (steps) *steps = m->stack_epoch;
+  if (given_up) *given_up = m->stack_fails;
+  return AHA_OK;
+}
 int aha_hip_debug_scramble_pages(aha_model* m, int enable) {
   if (!m) return AHA_ERR_INVALID;
   m->scramble_pages = enable != 0;

@@ -157,6 +157,28 @@ void launch_attn_decode_defer(const AttnDecodeFusedArgs& a, hipStream_t st);
 int attn_decode_slice_splits(int npages);
 void launch_attn_oproj(const AttnDecodeFusedArgs& a, const void* W, float* y, int n, hipStream_t st);
 
+// All layers of one decode step in one launch (kernels_decode_stack.hip)
+constexpr int DECODE_STACK_BLOCKS = 256;          // a block per CU: all of them have to be on the GPU together
+constexpr int DECODE_STACK_EXCHANGE = 800 * 1024; // bytes, zeroed once
+constexpr int DECODE_STACK_POLLS = 100000;        // 50 ms or more
+struct DecodeStackLayer { const void *wqkv, *wo, *wgu, *wdown, *in_norm, *post_norm, *q_norm, *k_norm; };
+struct DecodeStackArgs {
+  const DecodeStackLayer* layers;   // (n_layers), device memory
+  const void* x_in;                 // (hidden) bf16: the step's embedding row
+  void* x_out;                      // (hidden) bf16: what the last layer leaves
+  const float* rope;                // (128) f32: cos, sin of the step
+  const uint64_t* page_ptrs;
+  uint64_t layer_stride;            // bytes between the layers of a page
+  unsigned* exchange;
+  unsigned *fail_dev, *fail_host;   // the epoch of a launch in which a block gave up waiting (fail_dev: later launches do not wait at all)
+  uint32_t epoch;                   // > 0, another one for each launch on this exchange buffer
+  int n_layers, kv_len;             // kv_len: with the new token
+  int polls;                        // in vain, per wave and launch, until it gives up
+  float eps, scale;
+};
+bool decode_stack_sizes_ok(int width, int heads, int kv_heads, int head_dim, int ff);
+void launch_decode_stack(const DecodeStackArgs& a, hipStream_t st);
+
 struct AttnPrefillArgs {
   const void* q;           // (S, nh*d) bf16
   KvLayer kv;

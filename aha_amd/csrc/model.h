@@ -120,6 +120,15 @@ struct aha_model {
   float* d_part_y = nullptr;
   float* d_part_o = nullptr;
   float* d_part_ml = nullptr;
+  // all layers of a decode step in one launch (kernels_decode_stack.hip); null: this stack or device does not take it
+  aha::DecodeStackLayer* d_stack_layers = nullptr;
+  unsigned* d_stack_exchange = nullptr;
+  unsigned* d_stack_fail = nullptr;
+  unsigned *h_stack_fail = nullptr, *h_stack_fail_dev = nullptr;   // (pinned, behind the token ring)
+  uint32_t stack_epoch = 0;      // of the last such launch
+  int stack_fails = 0;           // steps that had to be run again as separate launches
+  int stack_hold = 0;            // > 0: separate launches for now
+  int stack_polls = aha::DECODE_STACK_POLLS;
   int max_nsplit = 64;
   // tensor parallelism (desc.tp_rank / tp_size); desc.num_attention_heads etc. hold the LOCAL (per-rank) sizes
   int tp_rank = 0, tp_size = 1;

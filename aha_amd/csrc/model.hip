@@ -11,6 +11,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 
 #include "argmax.h"
@@ -324,9 +325,46 @@ int alloc_slab(aha_model* m) {
   return AHA_OK;
 }
 
+// ---- one launch per decode step: who may, and what happens when it gives up (kernels_decode_stack.hip) ----
+// The blocks of such a launch wait for each other, so two of them that share the GPU could each hold what the other needs: one model per device at a time has
+// the right to it, from its first step in flight until that step has been waited for; a step of another model meanwhile runs as separate launches.
+constexpr int STACK_MAX_FAILS = 3;    // steps given up after which a model stays with separate launches
+constexpr int STACK_MAX_PAGES = 512;   // 32768 positions: 980 us a token, 1210 as separate launches (a page more costs 1.3 us here, 0.9 there)
+static std::atomic<aha_model*> g_stack_owner[64];
+static bool stack_acquire(aha_model* m) {
+  auto& owner = g_stack_owner[m->ctx->device & 63];
+  aha_model* none = nullptr;
+  return owner.load() == m || owner.compare_exchange_strong(none, m);
+}
+static void stack_release(aha_model* m) {
+  aha_model* me = m;
+  g_stack_owner[m->ctx->device & 63].compare_exchange_strong(me, nullptr);
+}
+static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_ready = false, bool arg_max = true);
+// The epoch of the step that gave up waiting (another process has the GPU), 0: none.  Clears it; the stream is idle.
+static uint32_t stack_failed(aha_model* m) {
+  stack_release(m);
+  if (!m->h_stack_fail) return 0;
+  const uint32_t e = __atomic_load_n(m->h_stack_fail, __ATOMIC_ACQUIRE);
+  if (!e) return 0;
+  *m->h_stack_fail = 0;
+  if (hipMemcpy(m->d_stack_fail, m->h_stack_fail, 4, hipMemcpyHostToDevice) != hipSuccess) m->stack_fails = STACK_MAX_FAILS;
+  ++m->stack_fails;
+  return e;
+}
+// Behind a wait for a single step: true if the step has been enqueued again, as separate launches
+static bool stack_redo(aha_model* m) {
+  if (!stack_failed(m)) return false;
+  ++m->stack_hold;
+  enqueue_decode_step(m, m->cache_len);
+  --m->stack_hold;
+  return true;
+}
+
 int model_wait_step(aha_model* m) {
   if (!m->step_in_flight) return AHA_OK;
   AHA_HIP_CHECK(hipStreamSynchronize(m->stream));
+  if (stack_redo(m)) AHA_HIP_CHECK(hipStreamSynchronize(m->stream));
   m->step_in_flight = false;
   return AHA_OK;
 }
@@ -525,6 +563,7 @@ int model_sample_candidates(aha_model* m, const uint32_t* ctx, size_t n_ctx, flo
   uint32_t* h_out = m->h_samp + m->samp_ctx_cap;
   AHA_HIP_CHECK(hipMemcpyAsync(h_out, out_val, OUT_WORDS * 4, hipMemcpyDeviceToHost, m->stream));
   AHA_HIP_CHECK(hipStreamSynchronize(m->stream));
+  if (stack_redo(m)) return model_sample_candidates(m, ctx, n_ctx, repeat_penalty, temperature, k, vals_out, idx_out, max_out, sumexp_out);
   m->step_in_flight = false;
   memcpy(vals_out, h_out, (size_t)k * 4);
   memcpy(idx_out, h_out + 66, (size_t)k * 4);
@@ -541,6 +580,7 @@ int model_last_logits(aha_model* m, float* logits_out) {
   if (int rc = assemble_logits(m)) return rc;
   AHA_HIP_CHECK(hipMemcpyAsync(m->h_logits, m->d_logits, (size_t)m->desc.vocab_size * 4, hipMemcpyDeviceToHost, m->stream));
   AHA_HIP_CHECK(hipStreamSynchronize(m->stream));
+  if (stack_redo(m)) return model_last_logits(m, logits_out);
   m->step_in_flight = false;
   memcpy(logits_out, m->h_logits, (size_t)m->desc.vocab_size * 4);
   return AHA_OK;
@@ -579,6 +619,8 @@ static int create_step_state(aha_model* m) {
   memset(m->h_ring, 0, (RING_CAP + 16) * 4);
   m->h_done = m->h_ring + RING_CAP;
   m->h_done_dev = m->h_ring_dev + RING_CAP;
+  m->h_stack_fail = m->h_ring + RING_CAP + 8;
+  m->h_stack_fail_dev = m->h_ring_dev + RING_CAP + 8;
   m->token_log_cap = 1 << 16;
   if ((rc = dev_alloc(m, m->token_log_cap * 4, &p))) return (rc);
   m->d_token_log = (uint32_t*)p;
@@ -590,6 +632,15 @@ static int create_step_state(aha_model* m) {
   if ((rc = dev_alloc(m, (size_t)nt * 4, &p))) return (rc);
   m->d_blk_idx = (uint32_t*)p;
   return AHA_OK;
+}
+
+// (a block per CU: a device with fewer would wait for blocks that cannot start)
+static bool stack_wanted(const aha_model* m) {
+  const aha_model_desc& c = m->desc;
+  int cus = 0;
+  const char* e = getenv("AHA_DECODE_STACK");
+  if ((e && !atoi(e)) || c.tp_size > 1 || m->layered || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, m->ctx->device) != hipSuccess) return false;
+  return cus >= DECODE_STACK_BLOCKS && decode_stack_sizes_ok(c.hidden_size, c.num_attention_heads, c.num_key_value_heads, c.head_dim, c.intermediate_size);
 }
 
 int model_create(aha_ctx* ctx, const aha_model_desc* desc, const aha_tensor_view* w, size_t nw, aha_model** out) {
@@ -791,6 +842,20 @@ int model_create(aha_ctx* ctx, const aha_model_desc* desc, const aha_tensor_view
     if ((rc = dev_alloc(m, (size_t)c.num_key_value_heads * H * 4, &p))) return fail(rc);
     m->d_part_y = (float*)p;
   }
+  if (stack_wanted(m)) {
+    std::vector<DecodeStackLayer> sl;
+    for (const LayerWeights& L : m->layers) sl.push_back({L.wqkv, L.wo, L.wgu, L.wdown, L.in_norm, L.post_norm, L.q_norm, L.k_norm});
+    if ((rc = dev_alloc(m, sl.size() * sizeof(DecodeStackLayer), &p))) return fail(rc);
+    m->d_stack_layers = (DecodeStackLayer*)p;
+    if (hipMemcpy(p, sl.data(), sl.size() * sizeof(DecodeStackLayer), hipMemcpyHostToDevice) != hipSuccess) {
+      set_error("model_create: copying the layer table failed");
+      return fail(AHA_ERR_HIP);
+    }
+    if ((rc = dev_alloc(m, DECODE_STACK_EXCHANGE, &p, true))) return fail(rc);
+    m->d_stack_exchange = (unsigned*)p;
+    if ((rc = dev_alloc(m, 64, &p, true))) return fail(rc);
+    m->d_stack_fail = (unsigned*)p;
+  }
   if ((rc = dev_alloc(m, 128 * 4, &p, true))) return fail(rc);
   m->d_rope = (float*)p;
 
@@ -818,6 +883,7 @@ int model_create(aha_ctx* ctx, const aha_model_desc* desc, const aha_tensor_view
 void model_destroy(aha_model* m) {
   if (!m) return;
   hipStreamSynchronize(m->stream);
+  stack_release(m);
   for (auto& r : m->prof) { hipEventDestroy(r.e0); hipEventDestroy(r.e1); }
   vision_destroy(m);
   audio_destroy(m);
@@ -958,6 +1024,7 @@ int model_fetch_outputs(aha_model* m, float* logits_out, uint32_t* argmax_out) {
   if (logits_out) AHA_HIP_CHECK(hipMemcpyAsync(m->h_logits, m->d_logits, (size_t)c.vocab_size * 4, hipMemcpyDeviceToHost, m->stream));
   AHA_HIP_CHECK(hipMemcpyAsync(&m->h_state->next_token, &m->d_state->next_token, 4, hipMemcpyDeviceToHost, m->stream));
   AHA_HIP_CHECK(hipStreamSynchronize(m->stream));
+  if (stack_redo(m)) return model_fetch_outputs(m, logits_out, argmax_out);
   m->step_in_flight = false;
   if (m->d_gemv_trace) gemv_trace_dump(m);
   if (m->d_attn_trace) {
@@ -1442,8 +1509,15 @@ static void gemv_trace_dump(aha_model* m) {
   }
 }
 
+// One launch for the layers of a step?  Not where a profile, a timeline or a knob asks for the separate ones.
+static bool stack_takes(aha_model* m, int npages) {
+  if (!m->d_stack_exchange || m->stack_hold > 0 || m->stack_fails >= STACK_MAX_FAILS || !m->decode_fused || m->profiling || npages > STACK_MAX_PAGES) return false;
+  static const bool knobs = getenv("AHA_ATTN_PAGES_PER_BLOCK") || getenv("AHA_ATTN_TRACE") || getenv("AHA_GEMV_TRACE") || !gemv_row_on();
+  return !knobs && stack_acquire(m);
+}
+
 // row_ready: the step's embedding row and rope table are there already (next_step_kernel); arg_max: next_token is left in the state
-static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_ready = false, bool arg_max = true) {
+static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_ready, bool arg_max) {
   if (m->layered) {
     const int rc = layered_enqueue_step(m, kv_len_after);
     if (rc && !m->async_rc) m->async_rc = rc;
@@ -1462,6 +1536,16 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_read
                        m->d_inv_freq, m->d_axis_map, m->d_rope);
   }
   const int npages = (int)((kv_len_after + KV_PAGE_TOKENS - 1) / KV_PAGE_TOKENS);
+  if (stack_takes(m, npages)) {
+    DecodeStackArgs a{};
+    a.layers = m->d_stack_layers; a.x_in = m->d_x; a.x_out = m->d_x; a.rope = m->d_rope; a.page_ptrs = m->d_page_ptrs; a.layer_stride = m->layer_stride;
+    a.exchange = m->d_stack_exchange; a.fail_dev = m->d_stack_fail; a.fail_host = m->h_stack_fail_dev;
+    if (++m->stack_epoch == 0) ++m->stack_epoch;
+    a.epoch = m->stack_epoch; a.n_layers = c.num_hidden_layers; a.kv_len = (int)kv_len_after; a.polls = m->stack_polls; a.eps = c.rms_norm_eps; a.scale = m->attn_scale;
+    launch_decode_stack(a, st);
+    enqueue_lm_head(m, m->d_x, arg_max);
+    return;
+  }
   // KV splits of the fused decode attention: one block (4 waves = 4 KV units) per `div` pages
   static const char* e_div = getenv("AHA_ATTN_PAGES_PER_BLOCK");
   const int div = e_div ? std::max(1, atoi(e_div)) : 4;
@@ -1641,6 +1725,7 @@ int model_debug_graph_step(aha_model* m, int replays, double* us_launches, doubl
   AHA_HIP_CHECK(hipEventCreate(&e0));
   AHA_HIP_CHECK(hipEventCreate(&e1));
   const unsigned base = m->head_ctr_base;
+  ++m->stack_hold;   // (a replay of the one-launch form would find the tags of the step before)
   auto step_with_fixed_args = [&] {
     m->head_ctr_base = base;   // the same arguments every repetition (see above)
     enqueue_decode_step(m, m->cache_len + 1);
@@ -1673,6 +1758,7 @@ int model_debug_graph_step(aha_model* m, int replays, double* us_launches, doubl
   // leave a consistent model behind: arrival counters back to zero, cache cleared
   AHA_HIP_CHECK(hipMemsetAsync(m->d_bar, 0, DECODE_SYNC_BYTES, m->stream));
   m->head_ctr_base = 0;
+  --m->stack_hold;
   AHA_HIP_CHECK(hipStreamSynchronize(m->stream));
   return model_clear_cache(m);
 }
@@ -1708,12 +1794,17 @@ int model_decode_greedy(aha_model* m, uint32_t first_token, size_t offset, size_
   // token sequence alone: whole groups of `ahead` steps, the next group only after every token of the last one has been read.
   const bool lockstep = m->tp_size > 1;
   const bool joined = !m->layered && m->lm_rows == c.vocab_size;
+  std::vector<uint32_t> epochs;   // of the steps that ran as one launch (0: separate ones)
+  epochs.reserve(max_new);
+  size_t good = max_new;          // steps in front of one that gave up
   while (seen < max_new && !stop) {
     size_t want = 0;
     if (!lockstep) want = enq < max_new && enq - seen < ahead ? std::min(max_new - enq, ahead - (enq - seen)) : 0;
     else if (seen == enq) want = std::min(max_new - enq, ahead);
     for (size_t i = 0; i < want; ++i) {
+      const uint32_t before = m->stack_epoch;
       enqueue_decode_step(m, base_len + enq + 1, joined && enq > 0, !joined);
+      epochs.push_back(m->stack_epoch != before ? m->stack_epoch : 0);
       if (joined) {
         ProfScope ps(m, "argmax", 0, 0);
         hipLaunchKernelGGL(next_step_kernel, dim3(1), dim3(1024), 0, m->stream, m->d_blk_max, m->d_blk_idx, gemv_num_tiles(c.vocab_size, c.hidden_size), m->d_state,
@@ -1734,17 +1825,33 @@ int model_decode_greedy(aha_model* m, uint32_t first_token, size_t offset, size_
       }
       done = __atomic_load_n(m->h_done, __ATOMIC_ACQUIRE);
     }
+    if (const uint32_t failed = m->h_stack_fail ? __atomic_load_n(m->h_stack_fail, __ATOMIC_ACQUIRE) : 0) {
+      while (good > 0 && (good > epochs.size() || epochs[good - 1] != failed)) --good;
+      if (good > 0) --good;
+      if (done > good) done = good;
+    }
     for (; seen < done && !stop; ++seen) {
       const uint32_t t = __atomic_load_n(m->h_ring + (seen % RING_CAP), __ATOMIC_RELAXED);
       out[produced++] = t;
       for (int e = 0; e < c.n_stop_tokens; ++e)
         if (t == c.stop_tokens[e]) stop = true;
     }
+    if (seen == good) break;
   }
   // steps queued past a stop token still run (at most `ahead` - 1 of them): their KV slots lie beyond the cache length kept below
   // and are overwritten by the next append; wait for them so nothing of this call is in flight when it returns
   AHA_HIP_CHECK(hipStreamSynchronize(m->stream));
+  stack_failed(m);
   m->steps_executed = (int64_t)enq;
+  if (good < max_new && !stop) {   // the rest as separate launches
+    m->cache_len = base_len + produced;
+    ++m->stack_hold;
+    const int more = model_decode_greedy(m, produced ? out[produced - 1] : first_token, offset + produced, max_new - produced, out + produced);
+    --m->stack_hold;
+    if (more < 0) return more;
+    m->steps_executed += (int64_t)enq;
+    return (int)produced + more;
+  }
   if (m->layered) layered_end_greedy(m, produced);
   m->cache_len = base_len + produced;  // inputs consumed: first_token and the first produced-1 generated tokens
   m->have_logits = produced > 0 || m->have_logits;

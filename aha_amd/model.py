@@ -487,6 +487,11 @@ class HipInferenceModel:
     def debug_scramble_pages(self, on: bool = True):
         check(lib().aha_hip_debug_scramble_pages(self.handle, int(on)))
 
+    def debug_decode_stack(self, polls: int = -1):
+        steps, given_up = C.c_int64(), C.c_int64()
+        check(lib().aha_hip_debug_decode_stack(self.handle, polls, C.byref(steps), C.byref(given_up)))
+        return steps.value, given_up.value
+
     def debug_last_hidden(self) -> np.ndarray:
         out = np.empty(self.text_cfg.hidden_size, dtype=np.float32)
         check(lib().aha_hip_debug_last_hidden(self.handle, out.ctypes.data_as(C.POINTER(C.c_float)), out.size))

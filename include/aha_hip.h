@@ -408,6 +408,9 @@ int aha_hip_debug_scramble_pages(aha_model* m, int enable);
 /* Test hook: how many more bytes this model's cache slabs and prefill scratch may take before they fail with AHA_ERR_OOM (scratch that is freed
  * counts back); a new model has no limit. */
 int aha_hip_debug_memory_limit(aha_model* m, size_t bytes);
+/* Test hook for decode steps whose layers run as one launch: polls >= 0 sets how often a wave of it asks in vain before it gives up and the step is run again as
+ * separate launches (0: at once); steps run so and steps given up so far. */
+int aha_hip_debug_decode_stack(aha_model* m, int32_t polls, int64_t* steps, int64_t* given_up);
 /* Copies the last hidden state before lm_head (hidden_size floats) / the image embeddings of the last
  * forward_initial (rows x out_hidden floats) to the host, for parity tests of intermediate tensors. */
 int aha_hip_debug_last_hidden(aha_model* m, float* out, size_t n);

@@ -1,0 +1,137 @@
+"""-m gpu: a decode step whose layers run as one launch (kernels_decode_stack.hip) against the separate launches, and what happens when it gives up waiting."""
+import threading
+
+import numpy as np
+import pytest
+
+from aha_amd.configs import tiny_qwen3
+from aha_amd.weights import qwen3_text_weights
+from tests.test_model_gpu import LOGIT_RMS_STD, LOGIT_TOL_STD, ids_for
+
+pytestmark = pytest.mark.gpu
+
+
+def models(monkeypatch, n=1, layers=3, vocab=1024):
+    """A model of separate launches and n of one launch, the sizes it is written for."""
+    from aha_amd.model import HipInferenceModel
+    cfg = tiny_qwen3(layers=layers, hidden=1024, heads=16, kv_heads=8, inter=3072, vocab=vocab)
+    w = qwen3_text_weights(cfg, seed=14)
+    monkeypatch.setenv("AHA_DECODE_STACK", "0")
+    plain = HipInferenceModel(cfg, w)
+    monkeypatch.setenv("AHA_DECODE_STACK", "1")
+    return cfg, plain, [HipInferenceModel(cfg, w) for _ in range(n)]
+
+
+def close_to(a, b, what):
+    """The bound of two decode forms' own test (test_model_gpu.py): the same arithmetic per token, sums in another order."""
+    std = float(a.std())
+    assert np.isfinite(b).all(), what
+    assert float(np.abs(a - b).max()) <= LOGIT_TOL_STD * std and float(np.sqrt(((a - b) ** 2).mean())) <= LOGIT_RMS_STD * std, what
+
+
+@pytest.mark.parametrize("scrambled", [False, True])
+@pytest.mark.parametrize("lens", [[1, 2, 62, 63, 64, 65], [127, 128, 700], [1983, 1984, 2046, 2047, 2048, 2110], [4095, 4159, 6300], [32764]])
+def test_one_launch_against_separate_ones(gpu, monkeypatch, lens, scrambled):
+    """No page behind the new token, pages' edges, the last length with a page per block at most (2048), two and three pages a block, the last length that is taken
+    (32768 positions; the steps behind it are separate launches again)."""
+    cfg, plain, (m,) = models(monkeypatch)
+    m.debug_scramble_pages(scrambled)
+    for S in lens:
+        ids = ids_for(cfg, S, 9 + S)
+        m.clear_cache(); plain.clear_cache()
+        _, tok = plain.forward_initial(ids, 0)
+        m.forward_initial(ids, 0)
+        before = m.debug_decode_stack()[0]
+        for step in range(6 if S > 32000 else 4):
+            a, am = plain.forward_step(tok, S + step)
+            b, _ = m.forward_step(tok, S + step)
+            close_to(a, b, (S, step))
+            tok = am
+        assert m.debug_decode_stack() == (before + 4, 0), S
+    assert plain.debug_decode_stack()[0] == 0
+    m.close(); plain.close()
+
+
+def test_waits_that_end(gpu, monkeypatch):
+    """Waves that may not ask even once give up, the launch ends, and the step is run as separate launches: a single step, steps of the device's loop (from the first
+    one, and behind steps that went well), a step whose logits are fetched or sampled from later, one that nobody asks for.  After three of them the model stays with
+    separate launches."""
+    cfg, plain, ms = models(monkeypatch, 6)
+    S = 70
+    ids = ids_for(cfg, S, 5)
+    _, tok = plain.forward_initial(ids, 0)
+    ref, _ = plain.forward_step(tok, S)
+    want_vals, want_idx = plain.sample_candidates([], 1.0, 1.0, 5)[:2]
+    plain.clear_cache()
+    plain.forward_initial(ids, 0)
+    want = plain.decode_greedy(tok, S, 12)
+    last = plain.last_logits()
+    for m in ms:
+        m.forward_initial(ids, 0)
+
+    ms[0].debug_decode_stack(0)
+    got, _ = ms[0].forward_step(tok, S)
+    np.testing.assert_array_equal(got, ref)     # (the launches of the other model)
+    assert ms[0].debug_decode_stack() == (1, 1)
+
+    ms[1].debug_decode_stack(0)
+    assert ms[1].decode_greedy(tok, S, 12) == want
+    np.testing.assert_array_equal(ms[1].last_logits(), last)
+    assert ms[1].debug_decode_stack()[1] == 1
+
+    assert ms[2].decode_greedy(tok, S, 4) == want[:4]
+    ms[2].debug_decode_stack(0)
+    assert ms[2].decode_greedy(want[3], S + 4, 8) == want[4:]
+    close_to(last, ms[2].last_logits(), "behind steps that went well")
+    assert ms[2].debug_decode_stack()[1] == 1
+
+    ms[3].debug_decode_stack(0)
+    ms[3].forward_step_enqueue(tok, S)
+    np.testing.assert_array_equal(ms[3].last_logits(), ref)
+
+    ms[4].debug_decode_stack(0)
+    ms[4].forward_step_enqueue(tok, S)
+    vals, idx = ms[4].sample_candidates([], 1.0, 1.0, 5)[:2]
+    np.testing.assert_array_equal(idx, want_idx)
+    np.testing.assert_array_equal(vals, want_vals)
+
+    ms[5].debug_decode_stack(0)
+    ms[5].forward_step_enqueue(tok, S)
+    ms[5].clear_cache()
+    ms[5].forward_initial(ids, 0)
+    for step in range(3):
+        ms[5].forward_step(tok, S + step)
+    assert ms[5].debug_decode_stack() == (3, 3)
+    for m in [plain] + ms:
+        m.close()
+
+
+def test_two_models_at_once(gpu, monkeypatch):
+    """Two threads with a model each: one has the right to the one launch at a time, the other runs separate ones; nobody waits in vain.  Both are fed the same
+    tokens as a model alone (greedy tokens of random weights hang on the order of sums), under the bound of the two forms."""
+    cfg, plain, ms = models(monkeypatch, 2)
+    prompts, fed = [ids_for(cfg, 50, 1), ids_for(cfg, 90, 2)], ids_for(cfg, 40, 3)
+    want, got = [], [[], []]
+    for p in prompts:
+        plain.clear_cache()
+        plain.forward_initial(p, 0)
+        want.append([plain.forward_step(t, len(p) + i)[0] for i, t in enumerate(fed)])
+
+    def run(i):
+        ms[i].forward_initial(prompts[i], 0)
+        got[i] = [ms[i].forward_step(t, len(prompts[i]) + k)[0] for k, t in enumerate(fed)]
+        ms[i].clear_cache()
+        _, tok = ms[i].forward_initial(prompts[i], 0)
+        assert len(ms[i].decode_greedy(tok, len(prompts[i]), 60)) == 60
+    threads = [threading.Thread(target=run, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for i in range(2):
+        assert len(got[i]) == len(fed)
+        for k in range(len(fed)):
+            close_to(want[i][k], got[i][k], (i, k))
+    assert [m.debug_decode_stack()[1] for m in ms] == [0, 0] and max(m.debug_decode_stack()[0] for m in ms) > 0
+    for m in [plain] + ms:
+        m.close()
