@@ -24,10 +24,12 @@
 // enough waits no more in this launch; the launch then ends by itself with garbage and says so in `fail`, and the host runs the step as separate launches (model.hip).
 #include "attn_common.h"
 #include "kernels.h"
+#include "stack_exchange.h"
 
 namespace aha {
 
 namespace {
+using namespace stack;
 
 constexpr int H = 1024, NH = 16, KVH = 8, D = 128, FF = 3072, NQ = NH * D;
 constexpr int BLOCKS = DECODE_STACK_BLOCKS, XCDS = 8, GROUP = BLOCKS / XCDS;   // blocks of an XCD
@@ -40,18 +42,7 @@ constexpr int PER_XCD = (AT_P + GROUP * P_SPLIT + 127) / 128 * 128;
 constexpr int AT_O = XCDS * PER_XCD, AT_D = AT_O + BLOCKS * RB * 8;            // (x, row) f32 with its tag
 constexpr int EXCHANGE = AT_D + BLOCKS * RB * 8;
 static_assert(EXCHANGE <= DECODE_STACK_EXCHANGE, "exchange buffer");
-constexpr uint32_t NOWHERE = 0x7fffffffu;                                      // past every descriptor's range: the store is dropped
-
-constexpr int AUX_NT = 2, AUX_SC1 = 16;   // a load past the L1; a store through to memory
-
-typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_t;
 typedef const __attribute__((address_space(4))) DecodeStackLayer* layer_ptr_t;
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* p, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
-}
-// LDS of this wave written and read, everybody here; requests of weights stay in flight
-__device__ __forceinline__ void meet() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 struct Lds {
   bf16_t x[H], x2[H], a[OC], m[DC];   // x, x2: behind the norm
@@ -61,27 +52,7 @@ struct Lds {
 };
 
 // ---- the waves that compute ------------------------------------------------------------------------------------------------------------------
-// Eight products: what a stage takes in is bf16, as the weights are, so v_dot2_f32_bf16 adds two exact products at a time.  Against 64 bits its sums are as close as
-// those of an fma chain (1024 elements: 2.4e-7 and 2.5e-7 of the sum's own size), at a quarter of the instructions: a SIMD has one of these waves, and the 500
-// instructions of gate and up were 1.3 us.
-__device__ __forceinline__ float dot8(u32x4_t h, u32x4_t w, float s) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) s = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, (uint32_t)h[j]), __builtin_bit_cast(bf16x2_t, (uint32_t)w[j]), s, false);
-  return s;
-}
-// a in the lower half of the wave, b in the upper one: each the sum of its two halves
-__device__ __forceinline__ float halves(float a, float b) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-// a in the even rows of 16 lanes, b in the odd ones: each the sum of a pair of rows
-__device__ __forceinline__ float quarters(float a, float b) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-// row G of 16 lanes: the sum of y[G] over the wave
-__device__ __forceinline__ float four_sums(float y0, float y1, float y2, float y3) { return row_sum(quarters(halves(y0, y2), halves(y1, y3))); }
-__device__ __forceinline__ float silu_exact(float x) { return x / (1.0f + expf(-x)); }
+__device__ __forceinline__ float silu_of(float x) { return x / (1.0f + expf(-x)); }
 
 // PG: pages that are requested a layer ahead (1: no block has a second one)
 template <int PG>
@@ -196,7 +167,7 @@ __device__ __forceinline__ void compute_waves(const DecodeStackArgs& a, Lds& lds
       for (int u = 0; u < 2; ++u) h[u] = *reinterpret_cast<const u32x4_t*>(lds.x + u * 512 + lane * 8);
       float y[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) y[r] = dot8(h[1], wq[r * 2 + 1], dot8(h[0], wq[r * 2], 0.f));
+      for (int r = 0; r < 4; ++r) y[r] = dot8_bf(h[1], wq[r * 2 + 1], dot8_bf(h[0], wq[r * 2], 0.f));
       const float v = four_sums(y[0], y[1], y[2], y[3]);
       __builtin_amdgcn_raw_buffer_store_b32(((uint32_t)f2bf(v) << 16) | t16, ex, c == 0 ? mine + AT_Q + (r16 + w * 4 + G) * 4 : NOWHERE, 0, 0);
       IN_ORDER;
@@ -279,7 +250,7 @@ __device__ __forceinline__ void compute_waves(const DecodeStackArgs& a, Lds& lds
       const u32x4_t h = *reinterpret_cast<const u32x4_t*>(lds.a + (lane & 31) * 8);
       float y[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) y[i] = dot8(h, wo[i], 0.f);
+      for (int i = 0; i < 4; ++i) y[i] = dot8_bf(h, wo[i], 0.f);
       const float y01 = row_sum(quarters(y[0], y[1])), y23 = row_sum(quarters(y[2], y[3]));   // load 2 c + (G & 1), row G >> 1 of its two
       const u32x2_t p = {__float_as_uint(c == 0 ? y01 : y23), tag};
       __builtin_amdgcn_raw_buffer_store_b64(p, ex, c < 2 ? AT_O + (x * H + row8 + c * 4 + (G & 1) * 2 + (G >> 1)) * 8 : NOWHERE, 0, AUX_SC1);
@@ -300,9 +271,9 @@ __device__ __forceinline__ void compute_waves(const DecodeStackArgs& a, Lds& lds
       for (int u = 0; u < 2; ++u) h[u] = *reinterpret_cast<const u32x4_t*>(lds.x2 + u * 512 + lane * 8);
       float y[6];
 #pragma unroll
-      for (int r = 0; r < 6; ++r) y[r] = dot8(h[1], wg[r * 2 + 1], dot8(h[0], wg[r * 2], 0.f));
+      for (int r = 0; r < 6; ++r) y[r] = dot8_bf(h[1], wg[r * 2 + 1], dot8_bf(h[0], wg[r * 2], 0.f));
       const float gt = four_sums(y[0], y[2], y[4], y[4]), up = four_sums(y[1], y[3], y[5], y[5]);   // feature G
-      const bf16_t v = f2bf(rbf(silu_exact(rbf(gt))) * rbf(up));
+      const bf16_t v = f2bf(rbf(silu_of(rbf(gt))) * rbf(up));
       __builtin_amdgcn_raw_buffer_store_b32(((uint32_t)v << 16) | t16, ex, c == 0 && G < 3 ? mine + AT_M + (s * 12 + w * 3 + G) * 4 : NOWHERE, 0, 0);
       IN_ORDER;
     }
@@ -315,7 +286,7 @@ __device__ __forceinline__ void compute_waves(const DecodeStackArgs& a, Lds& lds
       for (int j = 0; j < 3; ++j) {
         const u32x4_t h = *reinterpret_cast<const u32x4_t*>(lds.m + j * 128 + c * 8);
 #pragma unroll
-        for (int q = 0; q < 2; ++q) y[q] = dot8(h, wd[q * 3 + j], y[q]);
+        for (int q = 0; q < 2; ++q) y[q] = dot8_bf(h, wd[q * 3 + j], y[q]);
       }
 #pragma unroll
       for (int q = 0; q < 2; ++q) y[q] = row_sum(y[q]);
@@ -332,48 +303,6 @@ __device__ __forceinline__ void compute_waves(const DecodeStackArgs& a, Lds& lds
 // How long a stage's results are not asked for, in naps of 64 clocks (27 ns): a poll sent earlier finds nothing, and the next one waits for it.  Without any: 360 / 367 /
 // 397 us a token at 19 / 400 / 2048 positions; 338 / 346 / 368 with (each tried from 0 to 58: flat by 4 either way).
 constexpr int NAP_Q = 24, NAP_P = 8, NAP_A = 28, NAP_O = 44, NAP_X = 20, NAP_M = 24, NAP_D = 50;
-__device__ __forceinline__ void nap(int n) {
-  for (int i = 0; i < n; ++i) __builtin_amdgcn_s_sleep(1);
-}
-struct Poller {
-  __amdgpu_buffer_rsrc_t ex;
-  int left;   // polls in vain that this wave still makes
-  template <class Load>   // load(): requests, and says whether everything is there
-  __device__ __forceinline__ void until(bool ok, Load&& load) {
-    for (;;) {
-      if (!ok) ok = load();
-      asm volatile("" ::: "memory");
-      if (__all(ok) || left <= 0) return;
-      --left;
-    }
-  }
-  // four values (of a lane that takes part)
-  __device__ __forceinline__ u32x4_t values(bool part, uint32_t at, uint32_t t16) {
-    u32x4_t v = {0u, 0u, 0u, 0u};
-    until(!part, [&] {
-      v = __builtin_amdgcn_raw_buffer_load_b128(ex, at, 0, AUX_SC1);
-      return (((v[0] ^ t16) | (v[1] ^ t16) | (v[2] ^ t16) | (v[3] ^ t16)) & 0xffffu) == 0;
-    });
-    return v;
-  }
-  // row r = lane & 31 of the block's: the sum of the XCDs' parts
-  __device__ __forceinline__ float sum_parts(uint32_t at, int row, uint32_t tag) {
-    const uint32_t lane = threadIdx.x & 63, off = at + ((lane >> 5) * 4 * H + row) * 8;
-    u32x2_t p[4] = {};
-    until(false, [&] {
-      uint32_t bad = 0;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) p[i] = __builtin_amdgcn_raw_buffer_load_b64(ex, off + i * (H * 8), 0, AUX_SC1);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) bad |= p[i][1] ^ tag;
-      return bad == 0;
-    });
-    const float y = (__uint_as_float(p[0][0]) + __uint_as_float(p[1][0])) + (__uint_as_float(p[2][0]) + __uint_as_float(p[3][0]));
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(y), __float_as_uint(y), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  }
-};
-__device__ __forceinline__ uint2 pack4(u32x4_t v) { return make_uint2((v[0] >> 16) | (v[1] & 0xffff0000u), (v[2] >> 16) | (v[3] & 0xffff0000u)); }
 __device__ __forceinline__ void put4(bf16_t* dst, u32x4_t v) { *reinterpret_cast<uint2*>(dst) = pack4(v); }
 
 __device__ __forceinline__ void gather_waves(const DecodeStackArgs& a, Lds& lds, const int b, const int w) {
@@ -394,7 +323,7 @@ __device__ __forceinline__ void gather_waves(const DecodeStackArgs& a, Lds& lds,
   if (w == 0) res = ((const bf16_t*)a.x_in)[row];
   // res + the sum of the parts (o_proj, down), shared with the XCD
   auto add_parts = [&](uint32_t at, uint32_t tag, uint32_t to, uint32_t t16) {
-    res = f2bf(bf2f(res) + rbf(poll.sum_parts(at, row, tag)));
+    res = f2bf(bf2f(res) + rbf(poll.sum_parts<H>(at, row, tag)));
     __builtin_amdgcn_raw_buffer_store_b32(((uint32_t)res << 16) | t16, poll.ex, lane < 32 ? mine + to + row * 4 : NOWHERE, 0, 0);
   };
 
@@ -408,8 +337,11 @@ __device__ __forceinline__ void gather_waves(const DecodeStackArgs& a, Lds& lds,
     const float rinv = 1.0f / sqrtf(((q.x + q.y) + (q.z + q.w)) / (float)H + a.eps);
     *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf(x0 * rinv * lo_bf(nw.x), x1 * rinv * hi_bf(nw.x)), pack_bf(x2 * rinv * lo_bf(nw.y), x3 * rinv * hi_bf(nw.y)));
   };
-  auto norm_w = [&](const void* p) { return *reinterpret_cast<const uint2*>((const bf16_t*)p + t * 4); };
-  auto head_w = [&](int l) { return (const bf16_t*)(w == 2 ? layers[l].k_norm : layers[l].q_norm); };
+  auto norm_w = [&](const void* p) {
+    const u32x2_t v = global_at<u32x2_t>(p)[t];
+    return make_uint2(v[0], v[1]);
+  };
+  auto head_w = [&](int l) { return global_at<bf16_t>(w == 2 ? layers[l].k_norm : layers[l].q_norm); };
 
   uint2 in_w = norm_w(layers[0].in_norm), post_w;
   bf16_t w0 = head_w(0)[lane], w1 = head_w(0)[lane + 64];
@@ -509,7 +441,7 @@ __device__ __forceinline__ void gather_waves(const DecodeStackArgs& a, Lds& lds,
   }
   if (w == 0) {
     const uint32_t tag = a.epoch * (uint32_t)a.n_layers + (uint32_t)a.n_layers - 1;
-    res = f2bf(bf2f(res) + rbf(poll.sum_parts(AT_D, row, tag)));
+    res = f2bf(bf2f(res) + rbf(poll.sum_parts<H>(AT_D, row, tag)));
     if (x == 0 && lane < 32) ((bf16_t*)a.x_out)[row] = res;
   }
   if (poll.left <= 0 && !failed && lane == 0) {

@@ -291,4 +291,34 @@ struct GemvExpertsDown {
 };
 void launch_gemv_experts_down(const GemvArgs& a, const GemvExpertsDown& d, hipStream_t st);
 
+// ---- runs of sublayers of one token of one sequence in one launch (kernels_prenorm_stack.hip) ----------------------------------------------------
+enum { PRENORM_SSM, PRENORM_DENSE, PRENORM_MOE };
+struct PrenormOp {                   // a sublayer; what its kind does not have is null
+  int kind;
+  const void *w1, *w2;               // input and output projection; gate / up and down (of the shared expert)
+  const void *nw, *nb;               // the norm in front
+  const float* par;                  // f32: convolution weights (taps, cp), bias (cp), per head dt_bias, a, d
+  const void* gnorm;
+  int64_t hist, state;               // floats in front of the layer's share of the histories and states
+  const void *router, *egu, *edown;
+};
+constexpr int PRENORM_STACK_OPS = 16;   // of a launch, at most
+struct PrenormStackArgs {
+  const PrenormOp* ops;              // device memory
+  const float* x_in;                 // (1024): the residual stream in front of the first sublayer and behind the last; may be the same
+  float* x_out;
+  const float *hist_in, *state_in;   // the sequence's histories and states, and where the step leaves them (elsewhere)
+  float *hist_out, *state_out;
+  unsigned* exchange;
+  unsigned *fail_dev, *fail_host;    // as DecodeStackArgs
+  uint32_t epoch;
+  int n_ops, pos0, polls;
+  float eps;
+};
+bool prenorm_stack_width_ok(int64_t ld, int width);
+bool prenorm_stack_ssm_ok(const SsmDims& d, int n_out);
+bool prenorm_stack_dense_ok(int ff);
+bool prenorm_stack_moe_ok(int experts, int top, int ff, int shared_ff);
+void launch_prenorm_stack(const PrenormStackArgs& a, hipStream_t st);
+
 }  // namespace aha

@@ -748,7 +748,7 @@ int layered_forward_batch(aha_model* m, const aha_batch_entry* en, size_t n_en, 
     b.one = he[0];
   }
   const uint32_t* ids = (const uint32_t*)(l.d_meta + o_ids);
-  const Tail t = run_step(m, b, he, ids);
+  Tail t = run_step(m, b, he, ids);
   for (size_t i = 0; i < n_en; ++i) advance_seq(m, l.seqs[en[i].seq], en[i].n_tokens);
   m->cache_len = l.seqs[0].len;
   m->have_logits = false;
@@ -756,6 +756,7 @@ int layered_forward_batch(aha_model* m, const aha_batch_entry* en, size_t n_en, 
   const int32_t* dw = (const int32_t*)(l.d_meta + o_want);
   uint32_t* dam = (uint32_t*)(l.d_meta + o_am);
   const size_t V = c.vocab_size;
+again:
   for (size_t w0 = 0; w0 < want; w0 += SLICE) {
     const size_t n = std::min(SLICE, want - w0);
     float* lg = want == 1 ? m->d_logits : l.logits;
@@ -774,6 +775,12 @@ int layered_forward_batch(aha_model* m, const aha_batch_entry* en, size_t n_en, 
   else if (argmax_out && want) AHA_HIP_CHECK(hipMemcpyAsync(l.h_meta + o_am, dam, want * 4, hipMemcpyDeviceToHost, m->stream));
   AHA_HIP_CHECK(hipGetLastError());
   AHA_HIP_CHECK(hipStreamSynchronize(m->stream));   // (the pinned step buffer is free again)
+  if (model_stack_failed(m)) {   // (a token of one sequence: as separate launches)
+    ++m->stack_hold;
+    t = run_step(m, b, he, ids);
+    --m->stack_hold;
+    goto again;
+  }
   if (argmax_out && want) memcpy(argmax_out, l.h_meta + o_am, want * 4);
   if (want <= SLICE) l.last_want = want;
   return AHA_OK;

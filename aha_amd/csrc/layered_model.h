@@ -129,6 +129,11 @@ struct LayeredModel {
   std::vector<int> windows;       // the layers' distinct windows
   const int32_t* ext_dev = nullptr;   // (windows, entries) first gathered row of every entry
   std::vector<int> ext_total, ext_max;
+  // one token of one sequence: which layers' halves run together (kernels_prenorm_stack.hip); first < 0: this half by itself
+  struct StackItem { int layer, half, first, n; };
+  std::vector<StackItem> schedule;
+  PrenormOp* d_ops = nullptr;     // null: every half by itself
+  int64_t stack_hist = 0;         // floats of a history of its state-space layers
   // debug
   bool keep = false;
   float* resid = nullptr;

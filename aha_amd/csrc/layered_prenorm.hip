@@ -577,12 +577,72 @@ bool prenorm_single_ok(const aha_model* m) {
   }
   return true;
 }
+static int prenorm_schedule(aha_model* m);
 int prenorm_alloc_single(aha_model* m) {
   LayeredModel& l = *m->layered;
   int rc = dev_alloc(m, (size_t)std::max(l.max_proj, 1) * 4, (void**)&l.qkv1, true);
   if (!rc) rc = dev_alloc(m, (size_t)std::max(l.max_ep, 64) * 4, (void**)&l.z1, true);
   if (!rc) rc = dev_alloc(m, (size_t)(l.max_slots * l.max_effp + l.max_ffp + 64) * 2, &l.act1, true);
+  if (!rc && l.single_ok) rc = prenorm_schedule(m);
   return rc;
+}
+
+// Halves of layers that follow each other and that the kernel takes run as one launch; a half alone is no faster there (its weights are cold).
+static int prenorm_schedule(aha_model* m) {
+  LayeredModel& l = *m->layered;
+  std::vector<PrenormOp> ops;
+  l.schedule.clear();
+  auto add = [&](int li, int half, const PrenormOp* op) {
+    if (op && !l.schedule.empty() && l.schedule.back().first >= 0 && l.schedule.back().n < PRENORM_STACK_OPS) ++l.schedule.back().n;
+    else l.schedule.push_back({li, half, op ? (int)ops.size() : -1, op ? 1 : 0});
+    if (op) ops.push_back(*op);
+  };
+  bool have = false;
+  if (prenorm_stack_width_ok(l.ld, m->desc.hidden_size))
+    if (int rc = model_stack_alloc(m, &have)) return rc;
+  for (int li = 0; li < m->desc.num_hidden_layers; ++li) {
+    const PWeights& W = l.P[li];
+    const aha_layer_desc& d = m->desc.layers[li];
+    PrenormOp op{};
+    op.nw = W.n1w; op.nb = W.n1b;
+    if (have && d.mixer == AHA_MIXER_MAMBA2 && prenorm_stack_ssm_ok(W.sd, W.ko)) {
+      l.stack_hist = (int64_t)(W.sd.taps - 1) * W.sd.cp();   // (one geometry)
+      op.kind = PRENORM_SSM; op.w1 = W.w_in; op.w2 = W.wo; op.gnorm = W.gnorm; op.hist = W.hist_off; op.state = W.state_off;
+      const size_t cp = W.sd.cp(), taps = W.sd.taps, heads = W.sd.heads;
+      void* p = nullptr;
+      if (int rc = dev_alloc(m, ((taps + 1) * cp + 3 * heads) * 4, &p)) return rc;
+      float* at = (float*)p;
+      op.par = at;
+      auto put = [&](const float* src, size_t n) {
+        const hipError_t e = hipMemcpy(at, src, n * 4, hipMemcpyDeviceToDevice);
+        at += n;
+        return e == hipSuccess;
+      };
+      if (!put(W.sp.conv_w, taps * cp) || !put(W.sp.conv_b, cp) || !put(W.sp.dt_bias, heads) || !put(W.sp.a, heads) || !put(W.sp.d, heads))
+        return err(AHA_ERR_HIP, "model_create: copying the mixers' parameters failed");
+      add(li, 0, &op);
+    } else {
+      add(li, 0, nullptr);
+    }
+    if (d.mlp == AHA_MLP_NONE) continue;
+    op = PrenormOp{};
+    op.nw = W.n2w; op.nb = W.n2b; op.w1 = W.wgu; op.w2 = W.wdown;
+    if (have && d.mlp == AHA_MLP_GATED && prenorm_stack_dense_ok(W.ffp)) {
+      op.kind = PRENORM_DENSE;
+      add(li, 1, &op);
+    } else if (have && d.mlp == AHA_MLP_MOE && prenorm_stack_moe_ok(d.experts, d.top, W.effp, W.ffp)) {
+      op.kind = PRENORM_MOE; op.router = W.w_router; op.egu = W.w_egu; op.edown = W.w_edown;
+      add(li, 1, &op);
+    } else {
+      add(li, 1, nullptr);
+    }
+  }
+  if (ops.empty()) return AHA_OK;
+  void* p = nullptr;
+  if (int rc = dev_alloc(m, ops.size() * sizeof(PrenormOp), &p)) return rc;
+  l.d_ops = (PrenormOp*)p;
+  AHA_HIP_CHECK(hipMemcpy(p, ops.data(), ops.size() * sizeof(PrenormOp), hipMemcpyHostToDevice));
+  return AHA_OK;
 }
 
 // one token of one sequence: matvecs whose prologue is the norm in front of the projection.  Per layer three launches (state space) or five
@@ -605,7 +665,7 @@ static Tail prenorm_single(aha_model* m, const SeqBatch& b, const uint32_t* ids)
     g.W = W; g.N = n; g.K = k; g.y_f32 = y; g.eps = eps; g.res_f32 = l.xa; g.res_scale = 1.f;
     return g;
   };
-  for (int li = 0; li < c.num_hidden_layers; ++li) {
+  auto mixer = [&](int li) {
     const PWeights& W = l.P[li];
     const aha_layer_desc& d = c.layers[li];
     if (d.mixer == AHA_MIXER_MAMBA2) {
@@ -635,6 +695,10 @@ static Tail prenorm_single(aha_model* m, const SeqBatch& b, const uint32_t* ids)
       ProfScope ps(m, "gemv", bytes(g.N, g.K), 2.0 * g.N * g.K);
       launch_gemv(g, GEMV_AXPY_F32, st);
     }
+  };
+  auto feed_forward = [&](int li) {
+    const PWeights& W = l.P[li];
+    const aha_layer_desc& d = c.layers[li];
     if (d.mlp == AHA_MLP_GATED) {
       GemvArgs g = args(W.wgu, W.ffp, (int)l.ld, nullptr);
       g.y = l.act;
@@ -665,7 +729,30 @@ static Tail prenorm_single(aha_model* m, const SeqBatch& b, const uint32_t* ids)
       ProfScope ps(m, "moe", bytes(g.N, g.K), 2.0 * g.N * g.K);
       launch_gemv_experts_down(g, GemvExpertsDown{W.w_edown, W.wdown, e.sel, d.top, W.effp, W.ffp, (int)l.ld}, st);
     }
-    keep_rows(m, l.xa, 1, li);
+  };
+  // (the recurrence of a run that gave up is run again: its states must not have been written over)
+  const bool stacked = l.d_ops && !l.keep && b.one.state_in != b.one.state_out && model_stack_takes(m);
+  if (!stacked) {
+    for (int li = 0; li < c.num_hidden_layers; ++li) {
+      mixer(li);
+      feed_forward(li);
+      keep_rows(m, l.xa, 1, li);
+    }
+    return Tail{l.xa, nullptr, nullptr, 1.f, {}};
+  }
+  for (const LayeredModel::StackItem& it : l.schedule) {
+    if (it.n < 2) {
+      if (it.half == 0) mixer(it.layer);
+      else feed_forward(it.layer);
+      continue;
+    }
+    PrenormStackArgs p{};
+    p.ops = l.d_ops + it.first; p.n_ops = it.n; p.x_in = p.x_out = l.xa; p.pos0 = b.one.pos0; p.eps = eps; p.exchange = m->d_stack_exchange;
+    p.fail_dev = m->d_stack_fail; p.fail_host = m->h_stack_fail_dev; p.epoch = model_stack_epoch(m); p.polls = m->stack_polls;
+    float* const hist = l.d_hist + l.hist_slot * b.one.slot;
+    p.hist_in = hist + b.one.hist_in * l.stack_hist; p.hist_out = hist + b.one.hist_out * l.stack_hist;
+    p.state_in = l.d_pool + b.one.state_in * l.pool_stride; p.state_out = l.d_pool + b.one.state_out * l.pool_stride;
+    launch_prenorm_stack(p, st);
   }
   return Tail{l.xa, nullptr, nullptr, 1.f, {}};
 }

@@ -221,6 +221,11 @@ int model_forward_initial(aha_model* m, const uint32_t* ids, size_t n, size_t of
                           float* logits_out, uint32_t* argmax_out);
 int model_forward_step(aha_model* m, uint32_t token, size_t offset, float* logits_out, uint32_t* argmax_out);
 int model_forward_step_enqueue(aha_model* m, uint32_t token, size_t offset);
+// steps whose layers run as one launch or a few (kernels_decode_stack.hip, kernels_prenorm_stack.hip)
+int model_stack_alloc(aha_model* m, bool* have);   // the exchange buffer, where the device takes such launches
+bool model_stack_takes(aha_model* m);              // may the step that is being enqueued use them?
+uint32_t model_stack_epoch(aha_model* m);          // of its next one
+uint32_t model_stack_failed(aha_model* m);         // the stream is idle: the epoch of a launch that gave up (0: none), which is forgotten; others may use them now
 int model_wait_step(aha_model* m);   // before anything that the host or another stream does to what a step reads or writes
 int model_decode_greedy(aha_model* m, uint32_t first_token, size_t offset, size_t max_new, uint32_t* out);
 int model_clear_cache(aha_model* m);

@@ -341,8 +341,18 @@ static void stack_release(aha_model* m) {
   g_stack_owner[m->ctx->device & 63].compare_exchange_strong(me, nullptr);
 }
 static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_ready = false, bool arg_max = true);
+// Not where a profile, a timeline or a knob asks for the separate launches.
+bool model_stack_takes(aha_model* m) {
+  if (!m->d_stack_exchange || m->stack_hold > 0 || m->stack_fails >= STACK_MAX_FAILS || !m->decode_fused || m->profiling) return false;
+  static const bool knobs = getenv("AHA_ATTN_PAGES_PER_BLOCK") || getenv("AHA_ATTN_TRACE") || getenv("AHA_GEMV_TRACE") || !gemv_row_on();
+  return !knobs && stack_acquire(m);
+}
+uint32_t model_stack_epoch(aha_model* m) {
+  if (++m->stack_epoch == 0) ++m->stack_epoch;
+  return m->stack_epoch;
+}
 // The epoch of the step that gave up waiting (another process has the GPU), 0: none.  Clears it; the stream is idle.
-static uint32_t stack_failed(aha_model* m) {
+uint32_t model_stack_failed(aha_model* m) {
   stack_release(m);
   if (!m->h_stack_fail) return 0;
   const uint32_t e = __atomic_load_n(m->h_stack_fail, __ATOMIC_ACQUIRE);
@@ -354,7 +364,7 @@ static uint32_t stack_failed(aha_model* m) {
 }
 // Behind a wait for a single step: true if the step has been enqueued again, as separate launches
 static bool stack_redo(aha_model* m) {
-  if (!stack_failed(m)) return false;
+  if (!model_stack_failed(m)) return false;
   ++m->stack_hold;
   enqueue_decode_step(m, m->cache_len);
   --m->stack_hold;
@@ -635,12 +645,17 @@ static int create_step_state(aha_model* m) {
 }
 
 // (a block per CU: a device with fewer would wait for blocks that cannot start)
-static bool stack_wanted(const aha_model* m) {
-  const aha_model_desc& c = m->desc;
+int model_stack_alloc(aha_model* m, bool* have) {
   int cus = 0;
   const char* e = getenv("AHA_DECODE_STACK");
-  if ((e && !atoi(e)) || c.tp_size > 1 || m->layered || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, m->ctx->device) != hipSuccess) return false;
-  return cus >= DECODE_STACK_BLOCKS && decode_stack_sizes_ok(c.hidden_size, c.num_attention_heads, c.num_key_value_heads, c.head_dim, c.intermediate_size);
+  *have = !(e && !atoi(e)) && m->desc.tp_size <= 1 && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, m->ctx->device) == hipSuccess && cus >= DECODE_STACK_BLOCKS;
+  if (!*have) return AHA_OK;
+  void* p;
+  if (int rc = dev_alloc(m, 64, &p, true)) return rc;
+  m->d_stack_fail = (unsigned*)p;
+  if (int rc = dev_alloc(m, DECODE_STACK_EXCHANGE, &p, true)) return rc;
+  m->d_stack_exchange = (unsigned*)p;
+  return AHA_OK;
 }
 
 int model_create(aha_ctx* ctx, const aha_model_desc* desc, const aha_tensor_view* w, size_t nw, aha_model** out) {
@@ -842,19 +857,18 @@ int model_create(aha_ctx* ctx, const aha_model_desc* desc, const aha_tensor_view
     if ((rc = dev_alloc(m, (size_t)c.num_key_value_heads * H * 4, &p))) return fail(rc);
     m->d_part_y = (float*)p;
   }
-  if (stack_wanted(m)) {
-    std::vector<DecodeStackLayer> sl;
-    for (const LayerWeights& L : m->layers) sl.push_back({L.wqkv, L.wo, L.wgu, L.wdown, L.in_norm, L.post_norm, L.q_norm, L.k_norm});
-    if ((rc = dev_alloc(m, sl.size() * sizeof(DecodeStackLayer), &p))) return fail(rc);
-    m->d_stack_layers = (DecodeStackLayer*)p;
-    if (hipMemcpy(p, sl.data(), sl.size() * sizeof(DecodeStackLayer), hipMemcpyHostToDevice) != hipSuccess) {
-      set_error("model_create: copying the layer table failed");
-      return fail(AHA_ERR_HIP);
+  if (bool have = decode_stack_sizes_ok(H, c.num_attention_heads, c.num_key_value_heads, d, I)) {
+    if ((rc = model_stack_alloc(m, &have))) return fail(rc);
+    if (have) {
+      std::vector<DecodeStackLayer> sl;
+      for (const LayerWeights& L : m->layers) sl.push_back({L.wqkv, L.wo, L.wgu, L.wdown, L.in_norm, L.post_norm, L.q_norm, L.k_norm});
+      if ((rc = dev_alloc(m, sl.size() * sizeof(DecodeStackLayer), &p))) return fail(rc);
+      m->d_stack_layers = (DecodeStackLayer*)p;
+      if (hipMemcpy(p, sl.data(), sl.size() * sizeof(DecodeStackLayer), hipMemcpyHostToDevice) != hipSuccess) {
+        set_error("model_create: copying the layer table failed");
+        return fail(AHA_ERR_HIP);
+      }
     }
-    if ((rc = dev_alloc(m, DECODE_STACK_EXCHANGE, &p, true))) return fail(rc);
-    m->d_stack_exchange = (unsigned*)p;
-    if ((rc = dev_alloc(m, 64, &p, true))) return fail(rc);
-    m->d_stack_fail = (unsigned*)p;
   }
   if ((rc = dev_alloc(m, 128 * 4, &p, true))) return fail(rc);
   m->d_rope = (float*)p;
@@ -1509,13 +1523,6 @@ static void gemv_trace_dump(aha_model* m) {
   }
 }
 
-// One launch for the layers of a step?  Not where a profile, a timeline or a knob asks for the separate ones.
-static bool stack_takes(aha_model* m, int npages) {
-  if (!m->d_stack_exchange || m->stack_hold > 0 || m->stack_fails >= STACK_MAX_FAILS || !m->decode_fused || m->profiling || npages > STACK_MAX_PAGES) return false;
-  static const bool knobs = getenv("AHA_ATTN_PAGES_PER_BLOCK") || getenv("AHA_ATTN_TRACE") || getenv("AHA_GEMV_TRACE") || !gemv_row_on();
-  return !knobs && stack_acquire(m);
-}
-
 // row_ready: the step's embedding row and rope table are there already (next_step_kernel); arg_max: next_token is left in the state
 static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_ready, bool arg_max) {
   if (m->layered) {
@@ -1536,12 +1543,11 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_read
                        m->d_inv_freq, m->d_axis_map, m->d_rope);
   }
   const int npages = (int)((kv_len_after + KV_PAGE_TOKENS - 1) / KV_PAGE_TOKENS);
-  if (stack_takes(m, npages)) {
+  if (npages <= STACK_MAX_PAGES && model_stack_takes(m)) {
     DecodeStackArgs a{};
     a.layers = m->d_stack_layers; a.x_in = m->d_x; a.x_out = m->d_x; a.rope = m->d_rope; a.page_ptrs = m->d_page_ptrs; a.layer_stride = m->layer_stride;
     a.exchange = m->d_stack_exchange; a.fail_dev = m->d_stack_fail; a.fail_host = m->h_stack_fail_dev;
-    if (++m->stack_epoch == 0) ++m->stack_epoch;
-    a.epoch = m->stack_epoch; a.n_layers = c.num_hidden_layers; a.kv_len = (int)kv_len_after; a.polls = m->stack_polls; a.eps = c.rms_norm_eps; a.scale = m->attn_scale;
+    a.epoch = model_stack_epoch(m); a.n_layers = c.num_hidden_layers; a.kv_len = (int)kv_len_after; a.polls = m->stack_polls; a.eps = c.rms_norm_eps; a.scale = m->attn_scale;
     launch_decode_stack(a, st);
     enqueue_lm_head(m, m->d_x, arg_max);
     return;
@@ -1794,7 +1800,7 @@ int model_decode_greedy(aha_model* m, uint32_t first_token, size_t offset, size_
   // token sequence alone: whole groups of `ahead` steps, the next group only after every token of the last one has been read.
   const bool lockstep = m->tp_size > 1;
   const bool joined = !m->layered && m->lm_rows == c.vocab_size;
-  std::vector<uint32_t> epochs;   // of the steps that ran as one launch (0: separate ones)
+  std::vector<uint32_t> epochs;   // of the last launch of several stages behind each step
   epochs.reserve(max_new);
   size_t good = max_new;          // steps in front of one that gave up
   while (seen < max_new && !stop) {
@@ -1802,9 +1808,8 @@ int model_decode_greedy(aha_model* m, uint32_t first_token, size_t offset, size_
     if (!lockstep) want = enq < max_new && enq - seen < ahead ? std::min(max_new - enq, ahead - (enq - seen)) : 0;
     else if (seen == enq) want = std::min(max_new - enq, ahead);
     for (size_t i = 0; i < want; ++i) {
-      const uint32_t before = m->stack_epoch;
       enqueue_decode_step(m, base_len + enq + 1, joined && enq > 0, !joined);
-      epochs.push_back(m->stack_epoch != before ? m->stack_epoch : 0);
+      epochs.push_back(m->stack_epoch);
       if (joined) {
         ProfScope ps(m, "argmax", 0, 0);
         hipLaunchKernelGGL(next_step_kernel, dim3(1), dim3(1024), 0, m->stream, m->d_blk_max, m->d_blk_idx, gemv_num_tiles(c.vocab_size, c.hidden_size), m->d_state,
@@ -1826,8 +1831,7 @@ int model_decode_greedy(aha_model* m, uint32_t first_token, size_t offset, size_
       done = __atomic_load_n(m->h_done, __ATOMIC_ACQUIRE);
     }
     if (const uint32_t failed = m->h_stack_fail ? __atomic_load_n(m->h_stack_fail, __ATOMIC_ACQUIRE) : 0) {
-      while (good > 0 && (good > epochs.size() || epochs[good - 1] != failed)) --good;
-      if (good > 0) --good;
+      for (good = 0; good < epochs.size() && (int32_t)(epochs[good] - failed) < 0; ++good) {}
       if (done > good) done = good;
     }
     for (; seen < done && !stop; ++seen) {
@@ -1841,10 +1845,11 @@ int model_decode_greedy(aha_model* m, uint32_t first_token, size_t offset, size_
   // steps queued past a stop token still run (at most `ahead` - 1 of them): their KV slots lie beyond the cache length kept below
   // and are overwritten by the next append; wait for them so nothing of this call is in flight when it returns
   AHA_HIP_CHECK(hipStreamSynchronize(m->stream));
-  stack_failed(m);
+  model_stack_failed(m);
   m->steps_executed = (int64_t)enq;
   if (good < max_new && !stop) {   // the rest as separate launches
     m->cache_len = base_len + produced;
+    if (m->layered) layered_end_greedy(m, produced);
     ++m->stack_hold;
     const int more = model_decode_greedy(m, produced ? out[produced - 1] : first_token, offset + produced, max_new - produced, out + produced);
     --m->stack_hold;

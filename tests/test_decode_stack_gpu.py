@@ -135,3 +135,87 @@ def test_two_models_at_once(gpu, monkeypatch):
     assert [m.debug_decode_stack()[1] for m in ms] == [0, 0] and max(m.debug_decode_stack()[0] for m in ms) > 0
     for m in [plain] + ms:
         m.close()
+
+
+def pre_norm_models(monkeypatch, n=1, layers=7):
+    """The layer list of the state-space / latent-attention / experts design at the sizes kernels_prenorm_stack.hip is written for: a model of separate launches and n
+    of runs of sublayers.  Seven layers: runs of four, seven and one of two; attention in the third and the last."""
+    from aha_amd import configs, configs_layered
+    from aha_amd.model import HipInferenceModel
+    from aha_amd.weights_layered import vamatar_weights
+    t = configs.qwen3_0_6b()
+    t.vocab_size = 2048
+    cfg = configs_layered.vamatar_like(t, layers=layers)
+    w = vamatar_weights(cfg, seed=3, device="cuda:0")
+    monkeypatch.setenv("AHA_DECODE_STACK", "0")
+    plain = HipInferenceModel(cfg, w)
+    monkeypatch.setenv("AHA_DECODE_STACK", "1")
+    return cfg, plain, [HipInferenceModel(cfg, w) for _ in range(n)]
+
+
+@pytest.mark.parametrize("S", [1, 2, 3, 4, 70])
+def test_runs_of_sublayers_against_separate_launches(gpu, monkeypatch, S):
+    """Step by step from prompts with fewer tokens than taps on, past the turn of the histories (8): sums in f32 in another order, and features rounded to bf16 behind
+    them, so a share of an ulp of theirs: a quarter of the bound of the stacks whose residual stream is bf16.  Then the same tokens by the device's loop."""
+    cfg, plain, (m,) = pre_norm_models(monkeypatch)
+    ids = ids_for(cfg, S + 20, 11)
+    plain.forward_initial(ids[:S], 0)
+    m.forward_initial(ids[:S], 0)
+    before = m.debug_decode_stack()[0]
+    for i in range(20):
+        a, _ = plain.forward_step(ids[S + i], S + i)
+        b, _ = m.forward_step(ids[S + i], S + i)
+        std = float(a.std())
+        assert np.isfinite(b).all() and float(np.abs(a - b).max()) <= LOGIT_TOL_STD * std and float(np.sqrt(((a - b) ** 2).mean())) <= LOGIT_RMS_STD / 4 * std, (S, i)
+    assert m.debug_decode_stack() == (before + 20 * 2, 0)      # (a lone sublayer behind the last attention is separate launches)
+    first = int(np.argmax(b))
+    got = m.decode_greedy(first, S + 20, 12)
+    last = m.last_logits()
+    m.clear_cache()
+    m.forward_initial(ids[:S], 0)
+    for i in range(20):
+        m.forward_step(ids[S + i], S + i)
+    ref, tok = [], first
+    for i in range(12):
+        logits, tok = m.forward_step(tok, S + 20 + i)
+        ref.append(int(tok))
+    assert got == ref
+    np.testing.assert_array_equal(last, logits)
+    m.close(); plain.close()
+
+
+def test_runs_that_give_up(gpu, monkeypatch):
+    """A step and the device's loop with waves that may not ask even once: run again as separate launches, from the states and histories in front of the step.  Further
+    sequences keep their states in place and never use the runs."""
+    cfg, plain, ms = pre_norm_models(monkeypatch, 2)
+    S = 30
+    ids = ids_for(cfg, S + 3, 12)
+    plain.forward_initial(ids[:S], 0)
+    refs = [plain.forward_step(ids[S + i], S + i)[0] for i in range(3)]
+    want = plain.decode_greedy(7, S + 3, 10)
+    last = plain.last_logits()
+    for m in ms:
+        m.forward_initial(ids[:S], 0)
+    ms[0].debug_decode_stack(0)
+    for i in range(3):
+        np.testing.assert_array_equal(ms[0].forward_step(ids[S + i], S + i)[0], refs[i])
+    assert ms[0].debug_decode_stack() == (6, 3)
+    assert ms[0].decode_greedy(7, S + 3, 10) == want
+    np.testing.assert_array_equal(ms[0].last_logits(), last)
+
+    for i in range(3):
+        ms[1].forward_step(ids[S + i], S + i)
+    ms[1].debug_decode_stack(0)
+    assert len(ms[1].decode_greedy(7, S + 3, 10)) == 10
+    assert ms[1].debug_decode_stack()[1] == 1
+    close_to(last, ms[1].last_logits(), "behind steps that went well")
+
+    steps = ms[1].debug_decode_stack(100000)[0]
+    q = ms[1].seq_open()
+    ms[1].forward_batch([(q, ids[:S], [S - 1])], want_logits=True)
+    got, _ = ms[1].forward_batch([(q, [ids[S]], [0])], want_logits=True)
+    close_to(refs[0], got[0], "a further sequence")
+    assert ms[1].debug_decode_stack() == (steps, 1)
+    ms[1].seq_close(q)
+    for m in [plain] + ms:
+        m.close()
