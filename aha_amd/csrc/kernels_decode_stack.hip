@@ -17,7 +17,7 @@
 // of 1024 values to everyone took 3.5 us.  Every place is written once a layer, by the same block, and its next value needs something that every reader of this
 // one sends later: one buffer per stage.
 //
-// What it gives, us a token of 28 layers with the head's 50: 19 positions 524 (separate launches) -> 337, 400: 580 -> 346, 2048: 607 -> 370, 7000: 682 -> 475, 32000:
+// What it gives, us a token of 28 layers with the head's 50: 19 positions 524 (separate launches) -> 326, 400: 580 -> 348, 2048: 607 -> 370, 7000: 682 -> 475, 32000:
 // 1210 -> 980.  A layer is 10 us: 31 MB of weights (5.4 at the rate HBM reaches, most of it under what follows), 2.7 of arithmetic, four hand-offs inside an XCD, two across.
 //
 // Waits are bounded: the blocks have to be on the GPU together (and where they are thought to be), which nothing promises.  A wave that has polled in vain for long
@@ -302,6 +302,8 @@ __device__ __forceinline__ void compute_waves(const DecodeStackArgs& a, Lds& lds
 // ---- the waves that wait ---------------------------------------------------------------------------------------------------------------------
 // How long a stage's results are not asked for, in naps of 64 clocks (27 ns): a poll sent earlier finds nothing, and the next one waits for it.  Without any: 360 / 367 /
 // 397 us a token at 19 / 400 / 2048 positions; 338 / 346 / 368 with (each tried from 0 to 58: flat by 4 either way).
+// Splits that every block joins for itself: one hand-off less for twice (one split: eight times) the values.  us a token: 1 page 337 -> 326, 7 pages 346 -> 350, so up to two.
+constexpr int DIRECT = 2;
 constexpr int NAP_Q = 24, NAP_P = 8, NAP_A = 28, NAP_O = 44, NAP_X = 20, NAP_M = 24, NAP_D = 50;
 __device__ __forceinline__ void put4(bf16_t* dst, u32x4_t v) { *reinterpret_cast<uint2*>(dst) = pack4(v); }
 
@@ -397,10 +399,40 @@ __device__ __forceinline__ void gather_waves(const DecodeStackArgs& a, Lds& lds,
     }
     meet();
     for (int i = 0; i < my_np; ++i) meet();
-    if (w == 0) nap(NAP_P);
 
-    // ---- the splits and the new token joined: 8 of the kv head's 256 sums per block ----
-    if (w == 0) {
+    // ---- the splits and the new token joined.  Few splits: all 256 sums by every block for itself, a value a thread; more: 8 per block, shared ----
+    if (nsplit <= DIRECT) {
+      constexpr int N = DIRECT;   // (splits past the last: the last again, without weight)
+      const int hh = w >> 1, dim = t & (D - 1);
+      const float s_new = wave_sum(fmaf(bf2f(lds.q[hh * D + lane]), bf2f(lds.k[lane]), bf2f(lds.q[hh * D + lane + 64]) * bf2f(lds.k[lane + 64]))) * a.scale;
+      nap(NAP_P);
+      u32x4_t ml[N];
+      u32x2_t p[N];
+      poll.until(nsplit == 0, [&] {
+        uint32_t bad = 0;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          const uint32_t at = mine + AT_P + min(i, nsplit - 1) * P_SPLIT + hh * P_HEAD;
+          ml[i] = __builtin_amdgcn_raw_buffer_load_b128(poll.ex, at, 0, AUX_SC1);
+          p[i] = __builtin_amdgcn_raw_buffer_load_b64(poll.ex, at + 16 + dim * 8, 0, AUX_SC1);
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) bad |= (ml[i][1] ^ tag) | (ml[i][3] ^ tag) | (p[i][1] ^ tag);
+        return bad == 0;
+      });
+      float M = s_new;
+#pragma unroll
+      for (int i = 0; i < N; ++i) M = fmaxf(M, i < nsplit ? __uint_as_float(ml[i][0]) : -INFINITY);
+      float z = __expf(s_new - M), o = z * bf2f(lds.v[dim]);
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const float wt = i < nsplit ? __expf(__uint_as_float(ml[i][0]) - M) : 0.f;
+        z = fmaf(wt, i < nsplit ? __uint_as_float(ml[i][2]) : 0.f, z);
+        o = fmaf(wt, i < nsplit ? __uint_as_float(p[i][0]) : 0.f, o);
+      }
+      lds.a[t] = f2bf(o * (1.0f / z));
+    } else if (w == 0) {
+      nap(NAP_P);
       const float dot = wave_sum(fmaf(bf2f(lds.q[hd * D + lane]), bf2f(lds.k[lane]), bf2f(lds.q[hd * D + lane + 64]) * bf2f(lds.k[lane + 64])));
       const float s_new = dot * a.scale;
       const int split = lane & 31;
@@ -421,8 +453,10 @@ __device__ __forceinline__ void gather_waves(const DecodeStackArgs& a, Lds& lds,
       const float o = fmaf(wn, bf2f(lds.v[d0 + (e & 3)]), (lane & 15) == 0 ? s01 : s23) * (1.0f / z);
       __builtin_amdgcn_raw_buffer_store_b32(((uint32_t)f2bf(o) << 16) | t16, poll.ex, e < 4 ? mine + AT_A + (hd * D + d0 + e) * 4 : NOWHERE, 0, 0);
     }
-    if (w == 1) nap(NAP_A);
-    if (w == 1) put4(lds.a + lane * 4, poll.values(true, mine + AT_A + lane * 16, t16));
+    if (w == 1 && nsplit > DIRECT) {
+      nap(NAP_A);
+      put4(lds.a + lane * 4, poll.values(true, mine + AT_A + lane * 16, t16));
+    }
     meet();
     w0 = head_w(next)[lane], w1 = head_w(next)[lane + 64];
     nap(NAP_O);
