@@ -15,7 +15,7 @@
 // has the value, so nothing is acknowledged, counted or fenced.  Inside an XCD stores stop at its L2 (0.46 us from store to use on an idle chip); what crosses is
 // stored through to memory (1.0 us), in 64 bytes that one wave writes -- with four waves' dwords side by side a line is written piece by piece, and the hand-off
 // of 1024 values to everyone took 3.5 us.  Every place is written once a layer, by the same block, and its next value needs something that every reader of this
-// one sends later: one buffer per stage.
+// one sends later: one buffer per stage.  And every launch writes every place that is told by the low half of a tag, which comes again after 65536 layers.
 //
 // What it gives, us a token of 28 layers with the head's 50: 19 positions 524 (separate launches) -> 326, 400: 580 -> 348, 2048: 607 -> 370, 7000: 682 -> 475, 32000:
 // 1210 -> 980.  A layer is 10 us: 31 MB of weights (5.4 at the rate HBM reaches, most of it under what follows), 2.7 of arithmetic, four hand-offs inside an XCD, two across.
@@ -431,6 +431,8 @@ __device__ __forceinline__ void gather_waves(const DecodeStackArgs& a, Lds& lds,
         o = fmaf(wt, i < nsplit ? __uint_as_float(p[i][0]) : 0.f, o);
       }
       lds.a[t] = f2bf(o * (1.0f / z));
+      // the places of the shared sums, which this launch has no use for: a value that thousands of launches leave there has the 16 bits of a tag to come
+      if (l + 1 == a.n_layers && w == 0) __builtin_amdgcn_raw_buffer_store_b32(t16, poll.ex, lane < 8 ? mine + AT_A + (s * 8 + lane) * 4 : NOWHERE, 0, 0);
     } else if (w == 0) {
       nap(NAP_P);
       const float dot = wave_sum(fmaf(bf2f(lds.q[hd * D + lane]), bf2f(lds.k[lane]), bf2f(lds.q[hd * D + lane + 64]) * bf2f(lds.k[lane + 64])));

@@ -52,6 +52,31 @@ def test_one_launch_against_separate_ones(gpu, monkeypatch, lens, scrambled):
     m.close(); plain.close()
 
 
+def test_tags_that_come_again(gpu, monkeypatch):
+    """A step with more splits than every block joins for itself, behind as many with fewer as bring its first layer the low half of the tag that the last such step's
+    last layer had: 21846 steps of three layers are 65538."""
+    cfg, plain, (m,) = models(monkeypatch, vocab=256)
+    short, long = ids_for(cfg, 3, 1), ids_for(cfg, 200, 2)
+    _, tok = plain.forward_initial(long, 0)
+    want, _ = plain.forward_step(tok, 200)
+    m.forward_initial(ids_for(cfg, 200, 3), 0)
+    m.forward_step(5, 200)
+    start = m.debug_decode_stack()[0]
+    left = 21845
+    while left:
+        m.clear_cache()
+        _, t = m.forward_initial(short, 0)
+        m.decode_greedy(t, len(short), min(left, 110))
+        left = start + 21845 - m.debug_decode_stack()[0]
+        assert left >= 0
+    m.clear_cache()
+    m.forward_initial(long, 0)
+    got, _ = m.forward_step(tok, 200)
+    assert m.debug_decode_stack() == (start + 21846, 0)
+    close_to(want, got, "a tag that came again")
+    m.close(); plain.close()
+
+
 def test_waits_that_end(gpu, monkeypatch):
     """Waves that may not ask even once give up, the launch ends, and the step is run as separate launches: a single step, steps of the device's loop (from the first
     one, and behind steps that went well), a step whose logits are fetched or sampled from later, one that nobody asks for.  After three of them the model stays with
