@@ -179,6 +179,24 @@ struct DecodeStackArgs {
 bool decode_stack_sizes_ok(int width, int heads, int kv_heads, int head_dim, int ff);
 void launch_decode_stack(const DecodeStackArgs& a, hipStream_t st);
 
+// Norm, q k v, attention, o_proj and residual of one layer of a decode step in one launch (kernels_decode_attn.hip); blocks, exchange, epochs and polls as above
+struct DecodeAttnArgs {
+  void* x;                          // (hidden) bf16, in place
+  const void *in_norm, *wqkv, *wo, *q_norm, *k_norm;
+  const float* rope;
+  const uint64_t* page_ptrs;
+  uint64_t layer_off;
+  unsigned* exchange;
+  unsigned *fail_dev, *fail_host;
+  uint32_t epoch;
+  int kv_len, nsplit;               // nsplit: of attn_decode_defer_splits, whose sums these are
+  int polls;
+  float eps, scale;
+};
+bool decode_attn_sizes_ok(int width, int heads, int kv_heads, int head_dim);
+bool decode_attn_splits_ok(int nsplit, int npages);
+void launch_decode_attn(const DecodeAttnArgs& a, hipStream_t st);
+
 struct AttnPrefillArgs {
   const void* q;           // (S, nh*d) bf16
   KvLayer kv;

@@ -857,9 +857,11 @@ int model_create(aha_ctx* ctx, const aha_model_desc* desc, const aha_tensor_view
     if ((rc = dev_alloc(m, (size_t)c.num_key_value_heads * H * 4, &p))) return fail(rc);
     m->d_part_y = (float*)p;
   }
-  if (bool have = decode_stack_sizes_ok(H, c.num_attention_heads, c.num_key_value_heads, d, I)) {
+  const bool one_launch = decode_stack_sizes_ok(H, c.num_attention_heads, c.num_key_value_heads, d, I);
+  if (one_launch || decode_attn_sizes_ok(H, c.num_attention_heads, c.num_key_value_heads, d)) {
+    bool have = false;
     if ((rc = model_stack_alloc(m, &have))) return fail(rc);
-    if (have) {
+    if (have && one_launch) {
       std::vector<DecodeStackLayer> sl;
       for (const LayerWeights& L : m->layers) sl.push_back({L.wqkv, L.wo, L.wgu, L.wdown, L.in_norm, L.post_norm, L.q_norm, L.k_norm});
       if ((rc = dev_alloc(m, sl.size() * sizeof(DecodeStackLayer), &p))) return fail(rc);
@@ -1543,7 +1545,7 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_read
                        m->d_inv_freq, m->d_axis_map, m->d_rope);
   }
   const int npages = (int)((kv_len_after + KV_PAGE_TOKENS - 1) / KV_PAGE_TOKENS);
-  if (npages <= STACK_MAX_PAGES && model_stack_takes(m)) {
+  if (m->d_stack_layers && npages <= STACK_MAX_PAGES && model_stack_takes(m)) {
     DecodeStackArgs a{};
     a.layers = m->d_stack_layers; a.x_in = m->d_x; a.x_out = m->d_x; a.rope = m->d_rope; a.page_ptrs = m->d_page_ptrs; a.layer_stride = m->layer_stride;
     a.exchange = m->d_stack_exchange; a.fail_dev = m->d_stack_fail; a.fail_host = m->h_stack_fail_dev;
@@ -1569,16 +1571,26 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_read
   for (int p = 1; p < npages && page_stride; ++p)
     if (m->h_page_ptrs[p] != m->h_page_ptrs[0] + p * page_stride) page_stride = 0;
   if (page_stride > 0xffffffffu) page_stride = 0;
+  // 8B sizes, up to 24 pages: a layer's attention half in one launch, the same bits
+  const bool joined = m->d_stack_exchange && !slices && defer && decode_attn_sizes_ok(H, nh, kvh, d) && decode_attn_splits_ok(defer, npages) && model_stack_takes(m);
   for (int li = 0; li < c.num_hidden_layers; ++li) {
     const LayerWeights& L = m->layers[li];
-    {  // h = RMSNorm(x); qkv = h Wqkv^T                      (qwen3/model.rs:79, modules.rs:538-552)
+    if (joined) {
+      DecodeAttnArgs a{};
+      const KvLayer kv = model_kv_layer(m, li);
+      a.x = m->d_x; a.in_norm = L.in_norm; a.wqkv = L.wqkv; a.wo = L.wo; a.q_norm = L.q_norm; a.k_norm = L.k_norm; a.rope = m->d_rope;
+      a.page_ptrs = kv.page_ptrs; a.layer_off = kv.layer_off; a.exchange = m->d_stack_exchange; a.fail_dev = m->d_stack_fail; a.fail_host = m->h_stack_fail_dev;
+      a.epoch = model_stack_epoch(m); a.kv_len = (int)kv_len_after; a.nsplit = defer; a.polls = m->stack_polls; a.eps = c.rms_norm_eps; a.scale = m->attn_scale;
+      launch_decode_attn(a, st);
+    } else {  // h = RMSNorm(x); qkv = h Wqkv^T                      (qwen3/model.rs:79, modules.rs:538-552)
       GemvArgs g{};
       g.W = L.wqkv; g.x = m->d_x; g.norm_w = L.in_norm; g.eps = c.rms_norm_eps; g.y = m->d_qkv; g.N = nq + 2 * nkv; g.K = H;
       g.trace = gemv_trace_slot(m, li * 4 + 0);
       ProfScope ps(m, "gemv", (double)g.N * g.K * 2 + g.K * 4.0 + g.N * 2.0, 2.0 * g.N * g.K);
       launch_gemv(g, GEMV_STORE, st);
     }
-    if (m->decode_fused) {
+    if (joined) {   // (done)
+    } else if (m->decode_fused) {
       // q/k norm + rope + KV append + attention over the paged cache (modules.rs:544-574, 757-813), then
       // x = x + attn Wo^T with the KV-split partials merged in the matvec prologue (modules.rs:577, qwen3/model.rs:81)
       AttnDecodeFusedArgs a{};

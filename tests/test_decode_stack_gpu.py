@@ -244,3 +244,55 @@ def test_runs_that_give_up(gpu, monkeypatch):
     ms[1].seq_close(q)
     for m in [plain] + ms:
         m.close()
+
+
+def wide_models(monkeypatch, layers=2):
+    from aha_amd.model import HipInferenceModel
+    cfg = tiny_qwen3(layers=layers, hidden=4096, heads=32, kv_heads=8, inter=1024, vocab=512)
+    w = qwen3_text_weights(cfg, seed=15)
+    monkeypatch.setenv("AHA_DECODE_STACK", "0")
+    plain = HipInferenceModel(cfg, w)
+    monkeypatch.setenv("AHA_DECODE_STACK", "1")
+    return cfg, plain, HipInferenceModel(cfg, w)
+
+
+@pytest.mark.parametrize("scrambled", [False, True])
+def test_attention_half_in_one_launch(gpu, monkeypatch, scrambled):
+    """4096 columns: a layer's q k v, attention and o_proj in one launch (kernels_decode_attn.hip) give the bits of three.  No page behind the new token, pages' edges, one,
+    three and four splits, units with two pages, the last length that is taken (24 pages) and the first that is not."""
+    cfg, plain, m = wide_models(monkeypatch)
+    m.debug_scramble_pages(scrambled)
+    for S in [1, 63, 64, 65, 255, 256, 257, 319, 320, 384, 448, 700, 1023, 1024, 1025, 1471, 1534]:
+        ids = ids_for(cfg, S, 9 + S)
+        m.clear_cache(); plain.clear_cache()
+        _, tok = plain.forward_initial(ids, 0)
+        m.forward_initial(ids, 0)
+        before = m.debug_decode_stack()[0]
+        for step in range(3):
+            a, am = plain.forward_step(tok, S + step)
+            b, _ = m.forward_step(tok, S + step)
+            np.testing.assert_array_equal(a, b, err_msg=str((S, step)))
+            tok = am
+        assert m.debug_decode_stack() == (before + 2 * (2 if S == 1534 else 3), 0), S
+    assert plain.debug_decode_stack()[0] == 0
+    m.close(); plain.close()
+
+
+def test_attention_half_that_gives_up(gpu, monkeypatch):
+    """The same with waves that may not ask even once, in a single step and in the device's loop: run again as separate launches."""
+    cfg, plain, m = wide_models(monkeypatch)
+    ids = ids_for(cfg, 300, 4)
+    _, tok = plain.forward_initial(ids, 0)
+    m.forward_initial(ids, 0)
+    ref, first = plain.forward_step(tok, 300)
+    m.debug_decode_stack(0)
+    np.testing.assert_array_equal(m.forward_step(tok, 300)[0], ref)
+    assert m.debug_decode_stack() == (2, 1)
+    m.debug_decode_stack(100000)
+    want = plain.decode_greedy(first, 301, 12)
+    assert m.decode_greedy(first, 301, 4) == want[:4]
+    m.debug_decode_stack(0)
+    assert m.decode_greedy(want[3], 305, 8) == want[4:]
+    np.testing.assert_array_equal(m.last_logits(), plain.last_logits())
+    assert m.debug_decode_stack()[1] == 2
+    m.close(); plain.close()
