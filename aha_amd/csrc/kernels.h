@@ -103,6 +103,10 @@ struct RopeArgs {
   int kv_start_host = -1;   // the same value as *kv_start when the caller knows it on the host (prefill): selects the row-vectorised kernel
   const void* rope_tab = nullptr;  // optional (S, 128) bf16: cos[64] | sin[64] of every token's angles (launch_rope_table), else computed in place
   int skip_q = 0;           // row-vectorised prefill kernel only: the q heads are normed and rotated by the attention kernel's Q load (AttnPrefillArgs::q_norm_w); K and V only here
+  // documents that each begin on a cache page (row-vectorised kernel only): the slot of every row, the first row and the number of rows of every page, slots in all
+  const int32_t* row_slot = nullptr;
+  const int2* page_rows = nullptr;
+  int slots = 0;
 };
 void launch_qknorm_rope(const RopeArgs& a, hipStream_t st);
 // cos / sin of pos[axis(i)] * inv_freq[i], rounded to bf16 as apply_rotary_pos_emb casts them (rope.rs:96-132): computed ONCE per

@@ -228,7 +228,7 @@ __global__ __launch_bounds__(256) void qknorm_rope_rows_kernel(RopeArgs a, int n
     }
     const bf16_t* row = (const bf16_t*)a.qkv + (int64_t)tokc * a.ld + sub * 8;
     const int slot0 = first + chunk * ROPE_ROWS_CHUNK, slot1 = min(nqk, slot0 + ROPE_ROWS_CHUNK);
-    const int ctok = a.kv_start_host + tokc;
+    const int ctok = a.kv_start_host + (a.row_slot ? a.row_slot[tokc] : tokc);
     const int page = ctok / KV_PAGE_TOKENS, t = ctok % KV_PAGE_TOKENS;
     char* kbase = reinterpret_cast<char*>(a.kv.page_ptrs[page] + a.kv.layer_off);
     const bool hi_half = sub >= 8;
@@ -284,21 +284,28 @@ __global__ __launch_bounds__(256) void qknorm_rope_rows_kernel(RopeArgs a, int n
   // ---- role B: V rows, 128 lanes per (page of this call, kv head) ----
   const int64_t u = ((int64_t)(bid - n_qk_blocks) * 256 + threadIdx.x);
   const int unit = (int)(u >> 7), lu = (int)(u & 127);
-  const int p0 = a.kv_start_host / KV_PAGE_TOKENS, p1 = (a.kv_start_host + a.S - 1) / KV_PAGE_TOKENS;
+  const int p0 = a.kv_start_host / KV_PAGE_TOKENS, p1 = (a.kv_start_host + (a.page_rows ? a.slots : a.S) - 1) / KV_PAGE_TOKENS;
   const int page = p0 + unit / a.kvh, h = unit % a.kvh;
   if (page > p1) return;
   const int kk = lu >> 6, G = (lu >> 4) & 3, dchunk = lu & 15;
   uint32_t in[8][4];
   bool ok[8];
   bool all = true;
+  const int2 doc = a.page_rows ? a.page_rows[page - p0] : make_int2(0, 0);
 #pragma unroll
   for (int e = 0; e < 8; ++e) {   // slot order inside the piece: e = sub1 * 4 + j  <->  token kk*32 + sub1*16 + G*4 + j
     const int tokp = kk * 32 + (e >> 2) * 16 + G * 4 + (e & 3);
-    const int srow = page * KV_PAGE_TOKENS + tokp - a.kv_start_host;
-    ok[e] = srow >= 0 && srow < a.S;
+    const int srow = a.page_rows ? doc.x + tokp : page * KV_PAGE_TOKENS + tokp - a.kv_start_host;
+    ok[e] = a.page_rows ? tokp < doc.y : srow >= 0 && srow < a.S;
     all &= ok[e];
     const u32x4_t v = ld16((const bf16_t*)a.qkv + (int64_t)min(max(srow, 0), a.S - 1) * a.ld + (int64_t)(a.nh + a.kvh + h) * 128 + dchunk * 8);
     in[e][0] = v[0]; in[e][1] = v[1]; in[e][2] = v[2]; in[e][3] = v[3];
+  }
+  if (a.page_rows) {   // (the page is this document's alone: zeros behind it)
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (!ok[e]) in[e][0] = in[e][1] = in[e][2] = in[e][3] = 0;
+    all = true;
   }
   bf16_t* vb = reinterpret_cast<bf16_t*>(reinterpret_cast<char*>(a.kv.page_ptrs[page] + a.kv.layer_off)) +
                (int64_t)a.kvh * KV_PAGE_TOKENS * 128 + (int64_t)h * 128 * KV_PAGE_TOKENS;
@@ -339,7 +346,7 @@ void launch_rope_table(const int32_t* pos, int64_t pos_ld, const float* inv_freq
 
 void launch_qknorm_rope(const RopeArgs& a, hipStream_t st) {
   static const bool rows_on = [] { const char* e = getenv("AHA_ROPE_ROWS"); return e ? atoi(e) != 0 : true; }();
-  if (rows_on && a.kv_start_host >= 0 && a.kv.page_ptrs != nullptr && a.d == 128 && a.S >= 16) {
+  if ((rows_on && a.kv_start_host >= 0 && a.kv.page_ptrs != nullptr && a.d == 128 && a.S >= 16) || a.row_slot) {
     static const int chunk_env = [] { const char* e = getenv("AHA_ROPE_CHUNK"); return e ? atoi(e) : 8; }();
     // K heads only (skip_q): two heads per wave -- eight would leave S / 4 waves walking all kv heads one after the other (cfg 3: 386 waves on
     // 1024 SIMDs, ~3.7 us of dependent vector work each)
@@ -348,7 +355,7 @@ void launch_qknorm_rope(const RopeArgs& a, hipStream_t st) {
     const int nqk = (a.skip_q ? 0 : a.nh) + a.kvh, nchunk = (nqk + chunk - 1) / chunk;
     const int64_t qk_waves = (int64_t)((a.S + 3) / 4) * nchunk;
     const int n_qk_blocks = (int)((qk_waves + 3) / 4);
-    const int npages = (a.kv_start_host + a.S - 1) / KV_PAGE_TOKENS - a.kv_start_host / KV_PAGE_TOKENS + 1;
+    const int npages = (a.kv_start_host + (a.page_rows ? a.slots : a.S) - 1) / KV_PAGE_TOKENS - a.kv_start_host / KV_PAGE_TOKENS + 1;
     const int n_v_blocks = (npages * a.kvh * 128 + 255) / 256;
     const dim3 grid((unsigned)(n_qk_blocks + n_v_blocks));
     if (chunk == 2) hipLaunchKernelGGL(qknorm_rope_rows_kernel<2>, grid, dim3(256), 0, st, a, n_qk_blocks);

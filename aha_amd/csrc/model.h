@@ -180,7 +180,7 @@ struct aha_model {
   size_t samp_ctx_cap = 0;
   // prefill scratch (grown on demand)
   size_t pf_cap = 0;
-  void* d_docs = nullptr;        // joint prefill of documents (model_embed_multi): their SeqEntry records, then their last rows' numbers
+  void* d_docs = nullptr;        // joint prefill of documents (model_embed_multi): DocTables
   uint32_t* p_ids = nullptr;
   int32_t* p_pos = nullptr;
   void *p_x = nullptr, *p_h = nullptr, *p_qkv = nullptr, *p_q = nullptr, *p_attn = nullptr, *p_act = nullptr;

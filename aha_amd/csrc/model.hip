@@ -1920,12 +1920,17 @@ int model_embed(aha_model* m, const uint32_t* ids, size_t n, float* out) {
 
 // Several documents: as many consecutive ones as fit into EMBED_ROWS rows go through the decoder stack as ONE prefill.  A document of a few hundred
 // rows leaves most of the chip idle in every GEMM of a small model (0.6B, 300 rows: N = 1024 gives 24 tiles of 128^2) and each costs its launches:
-// eight documents of 75 to 600 tokens were 16.1 ms one by one, 4.1 ms together.  Each begins on a cache page of its own (its rows are padded to
-// whole pages by repeating its last token, behind everything its last position sees), so row = cache slot as in any prefill and only the attention
-// knows about documents.  4096 rows fill the chip with the narrowest GEMM (N = 1024: 256 tiles); a document alone, of one token (a decode step) or
+// eight documents of 75 to 600 tokens were 16.1 ms one by one, 4.1 ms together.  Each begins on a cache page of its own; its rows follow the last
+// document's at once, so only the attention and what writes keys and values know about documents.  4096 rows fill the chip with the narrowest GEMM (N = 1024: 256 tiles); a document alone, of one token (a decode step) or
 // longer than that runs as before, and so does everything where the joint prefill finds no memory: its scratch, larger than a single document's, is
 // given back first.
-constexpr size_t EMBED_ROWS = 4096;
+constexpr size_t EMBED_ROWS = 4096;   // (slots: rows with every document's last page filled up)
+struct DocTables {
+  SeqEntry docs[EMBED_ROWS / KV_PAGE_TOKENS];
+  uint32_t last[EMBED_ROWS / KV_PAGE_TOKENS];    // rows
+  int2 page_rows[EMBED_ROWS / KV_PAGE_TOKENS];   // RopeArgs
+  int32_t row_slot[EMBED_ROWS];
+};
 int model_embed_multi(aha_model* m, const uint32_t* ids, const uint64_t* lens, size_t n_docs, float* out) {
   if (!out || !lens || n_docs == 0) {
     set_error("embed: out or lens is null, or there are no documents");
@@ -1938,16 +1943,16 @@ int model_embed_multi(aha_model* m, const uint32_t* ids, const uint64_t* lens, s
   for (size_t d = 0, pos = 0; d < n_docs;) {
     std::vector<SeqEntry> docs;
     std::vector<uint32_t> rows;
-    size_t at = pos;
-    for (size_t e = d; joint && e < n_docs && lens[e] > 1 && lens[e] <= EMBED_ROWS && rows.size() + padded(lens[e]) <= EMBED_ROWS; ++e) {
+    size_t at = pos, slots = 0;
+    for (size_t e = d; joint && e < n_docs && lens[e] > 1 && lens[e] <= EMBED_ROWS && slots + padded(lens[e]) <= EMBED_ROWS; ++e) {
       bool ok = true;
       for (size_t i = 0; i < lens[e]; ++i) ok &= ids[at + i] < (uint32_t)m->desc.vocab_size;
       if (!ok) break;   // (reported when its turn comes)
       const size_t row0 = rows.size();
       rows.insert(rows.end(), ids + at, ids + at + lens[e]);
-      rows.resize(row0 + padded(lens[e]), rows.back());
-      docs.push_back(SeqEntry{(int32_t)row0, (int32_t)lens[e], 0, (int32_t)(row0 / KV_PAGE_TOKENS), 0, 0, 0, 0});
+      docs.push_back(SeqEntry{(int32_t)row0, (int32_t)lens[e], 0, (int32_t)(slots / KV_PAGE_TOKENS), 0, 0, 0, 0});
       at += lens[e];
+      slots += padded(lens[e]);
     }
     if (docs.size() > 1) {
       int rc = model_clear_cache(m);
@@ -2013,7 +2018,8 @@ static int forward_initial_impl(aha_model* m, const uint32_t* ids, size_t n, siz
   int rc;
   if ((rc = ensure_prefill_scratch(m, n))) return rc;
   GemmWorkspaceScope ws_scope(m->p_gemm_ws, m->gemm_ws_bytes, m->d_sk_ctrs);  // split-K slabs / persistent-kernel chunks of this thread's GEMM launches
-  if ((rc = model_ensure_pages(m, m->cache_len + n))) return rc;
+  const size_t slots = docs ? (size_t)docs->back().slot * KV_PAGE_TOKENS + docs->back().len : n;   // (a document begins on a page)
+  if ((rc = model_ensure_pages(m, m->cache_len + slots))) return rc;
 
   // Context-parallel prefill (cp_make_plan above): this rank owns two row chunks of the prompt.  Its activation buffers are COMPACT --
   // buffer row l0 + i holds prompt row r0 + i of a segment -- so every norm and GEMM below runs ONCE over all of the rank's rows; only
@@ -2052,21 +2058,27 @@ static int forward_initial_impl(aha_model* m, const uint32_t* ids, size_t n, siz
     for (int a = 0; a < 3; ++a)
       for (int i = 0; i < S; ++i) pos[(size_t)a * S + i] = (int32_t)(offset + i);
   }
-  std::vector<uint32_t> doc_rows;   // joint prefill of documents: each counts from 0; its last row is what it leaves
+  // joint prefill of documents: each counts from 0; its last row is what it leaves
   int doc_most = 0;
   if (docs) {
-    if (!m->d_docs && (rc = dev_alloc(m, EMBED_ROWS / KV_PAGE_TOKENS * (sizeof(SeqEntry) + 4), &m->d_docs, false))) return rc;
-    std::vector<SeqEntry> whole = *docs;   // (the padding rows too: nothing reads rows that nobody wrote)
-    for (SeqEntry& e : whole) {
-      for (int i = e.row0; i < S; ++i) pos[(size_t)i] = pos[(size_t)S + i] = pos[2 * (size_t)S + i] = i - e.row0;
-      doc_rows.push_back((uint32_t)(e.row0 + e.len - 1));
-      e.len = (e.len + KV_PAGE_TOKENS - 1) / KV_PAGE_TOKENS * KV_PAGE_TOKENS;
+    if (!m->d_docs && (rc = dev_alloc(m, sizeof(DocTables), &m->d_docs, false))) return rc;
+    std::vector<DocTables> one(1);
+    DocTables& t = one[0];
+    for (size_t k = 0; k < docs->size(); ++k) {
+      const SeqEntry& e = (*docs)[k];
+      t.docs[k] = e;
+      t.last[k] = (uint32_t)(e.row0 + e.len - 1);
       doc_most = std::max(doc_most, (int)e.len);
+      for (int i = 0; i < e.len; ++i) {
+        pos[(size_t)e.row0 + i] = pos[(size_t)S + e.row0 + i] = pos[2 * (size_t)S + e.row0 + i] = i;
+        t.row_slot[e.row0 + i] = e.slot * KV_PAGE_TOKENS + i;
+      }
+      for (int i = 0; i < e.len; i += KV_PAGE_TOKENS) t.page_rows[e.slot + i / KV_PAGE_TOKENS] = make_int2(e.row0 + i, std::min(KV_PAGE_TOKENS, e.len - i));
     }
-    AHA_HIP_CHECK(hipMemcpyAsync(m->d_docs, whole.data(), whole.size() * sizeof(SeqEntry), hipMemcpyHostToDevice, st));
-    AHA_HIP_CHECK(hipMemcpyAsync((char*)m->d_docs + EMBED_ROWS / KV_PAGE_TOKENS * sizeof(SeqEntry), doc_rows.data(), doc_rows.size() * 4, hipMemcpyHostToDevice, st));
+    AHA_HIP_CHECK(hipMemcpyAsync(m->d_docs, &t, sizeof(t), hipMemcpyHostToDevice, st));
     AHA_HIP_CHECK(hipStreamSynchronize(st));   // (pageable host memory)
   }
+  const DocTables* const tables = (const DocTables*)m->d_docs;   // (on the device)
   const int64_t p0[3] = {pos[0], pos[S], pos[2 * (size_t)S]};
   std::vector<uint32_t> ids_loc;
   std::vector<int32_t> pos_loc;
@@ -2085,7 +2097,7 @@ static int forward_initial_impl(aha_model* m, const uint32_t* ids, size_t n, siz
   }
   AHA_HIP_CHECK(hipMemcpyAsync(m->p_ids, ids_up, (size_t)Mloc * 4, hipMemcpyHostToDevice, st));
   AHA_HIP_CHECK(hipMemcpyAsync(m->p_pos, pos_up, 3 * (size_t)Mloc * 4, hipMemcpyHostToDevice, st));
-  if ((rc = push_state(m, ids[n - 1], p0, m->cache_len, m->cache_len + n))) return rc;
+  if ((rc = push_state(m, ids[n - 1], p0, m->cache_len, m->cache_len + slots))) return rc;
   pstamp("ids / positions enqueued");
   AHA_HIP_CHECK(hipStreamSynchronize(st));  // pos / ids are pageable host memory
   pstamp("... and landed");
@@ -2153,6 +2165,7 @@ static int forward_initial_impl(aha_model* m, const uint32_t* ids, size_t n, siz
       r.kv_start_host = kv_off + sg.r0;   // == d_state->kv_start (push_state above) for the whole prompt
       r.rope_tab = rows(m->p_rope, sg.l0, 128);
       r.skip_q = q_fused ? 1 : 0;
+      if (docs) { r.row_slot = tables->row_slot; r.page_rows = tables->page_rows; r.slots = (int)slots; }
       ProfScope ps(m, "elem", (double)sg.len * ((q_fused ? 0 : nq) + 2 * nkv) * 4, 0);
       launch_qknorm_rope(r, st);
     }
@@ -2178,7 +2191,7 @@ static int forward_initial_impl(aha_model* m, const uint32_t* ids, size_t n, siz
         Lk = a.kv_total2; flops += 4.0 * s2.len * (a.kv_offset2 + 0.5 * s2.len) * nq; rows_io += s2.len;
       }
       if (docs) {
-        a.seqs = m->d_docs;
+        a.seqs = tables->docs;
         a.seq_tab_ld = 1;   // (slot = the document's first page)
         flops = 0;
         for (const SeqEntry& e : *docs) flops += 2.0 * e.len * e.len * nq;
@@ -2189,11 +2202,10 @@ static int forward_initial_impl(aha_model* m, const uint32_t* ids, size_t n, siz
       if (one_launch) break;
     }
     if (li + 1 == c.num_hidden_layers && m->tp_size <= 1 && !(has_image && vision_has_deepstack(m, li)) && nq * 4 >= H) {
-      if (docs) {   // (at most one document per 64 rows, so their rows fit where the attention's were)
+      if (docs) {   // (a document has two rows or more, so theirs fit where the attention's were)
         n_rows = (int)docs->size();
-        const uint32_t* at = (const uint32_t*)((char*)m->d_docs + EMBED_ROWS / KV_PAGE_TOKENS * sizeof(SeqEntry));
-        launch_embed_gather(m->p_attn, at, m->p_q, n_rows, nq, st);
-        launch_embed_gather(m->p_x, at, m->p_attn, n_rows, H, st);
+        launch_embed_gather(m->p_attn, tables->last, m->p_q, n_rows, nq, st);
+        launch_embed_gather(m->p_x, tables->last, m->p_attn, n_rows, H, st);
         att_rows = m->p_q;
         x_rows = m->p_attn;
       } else {      // (a context-parallel rank: its own last row; rank 0's is the prompt's)
@@ -2257,12 +2269,12 @@ static int forward_initial_impl(aha_model* m, const uint32_t* ids, size_t n, siz
   if (docs) {   // every document's last row after the final norm -> p_qkv
     if (x_rows == m->p_x) {
       launch_rmsnorm_rows(m->p_x, m->final_norm, m->p_h, Mloc, H, H, H, c.rms_norm_eps, st);
-      launch_embed_gather(m->p_h, (const uint32_t*)((char*)m->d_docs + EMBED_ROWS / KV_PAGE_TOKENS * sizeof(SeqEntry)), m->p_qkv, (int)docs->size(), H, st);
+      launch_embed_gather(m->p_h, tables->last, m->p_qkv, (int)docs->size(), H, st);
     } else {
       launch_rmsnorm_rows(x_rows, m->final_norm, m->p_qkv, n_rows, H, H, H, c.rms_norm_eps, st);
     }
     AHA_HIP_CHECK(hipMemcpyAsync(m->d_hlast, (const char*)m->p_qkv + (docs->size() - 1) * H * 2, (size_t)H * 2, hipMemcpyDeviceToDevice, st));
-    m->cache_len += n;
+    m->cache_len += slots;
     AHA_HIP_CHECK(hipGetLastError());
     return AHA_OK;
   }

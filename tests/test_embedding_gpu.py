@@ -114,6 +114,21 @@ def test_documents_together(gpu, heads, kv_heads):
         m.close()
 
 
+def test_documents_on_pages_of_others(gpu):
+    """Keys and values that are not numbers, left by an earlier call on the pages that a document now fills in part: its vector is what it was on fresh ones."""
+    from aha_amd.model import HipInferenceModel
+    cfg = tiny_qwen3(layers=2, hidden=256, heads=4, kv_heads=2, inter=512, vocab=2048)
+    w = qwen3_text_weights(cfg, seed=1)
+    w["model.embed_tokens.weight"][7] = float("nan")
+    m = HipInferenceModel(cfg, w)
+    docs = [[t if t != 7 else 8 for t in d] for d in seqs_for(cfg, [3, 70, 33, 128, 5], 6)]
+    first = m.embed_multi(docs)
+    assert np.isfinite(first).all()
+    assert np.isnan(m.embed_multi([[7] * 320, [7] * 320])).all()
+    np.testing.assert_array_equal(m.embed_multi(docs), first)
+    m.close()
+
+
 @pytest.mark.parametrize("how", ["environment", "hook"])
 def test_documents_one_by_one_in_a_form_that_was_asked_for(gpu, how):
     """AHA_ATTN_FORM (read once per process: a child) and aha_hip_debug_attn_form name the attention kernel of every prefill: no joint one, the vectors of
