@@ -458,10 +458,16 @@ __global__ __launch_bounds__(256) void argmax_f32_stage1(const float* __restrict
   x += blockIdx.y * ld;
   float bv = -INFINITY;
   uint32_t bi = 0xffffffffu;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-    const float v = x[i];
-    // NaN never wins (v > bv is false), matching a partial_cmp-style scan that keeps the first non-NaN max
-    argmax_combine(bv, bi, v, (uint32_t)i);
+  // NaN never wins (v > bv is false), matching a partial_cmp-style scan that keeps the first non-NaN max.  Eight values at a time are asked for
+  // together: 8 rows of 32768, 7.0 us with a load at a time, 5.0 so.
+  const int64_t step = (int64_t)gridDim.x * 256;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += 8 * step) {
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = x[min(i + k * step, n - 1)];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (i + k * step < n) argmax_combine(bv, bi, v[k], (uint32_t)(i + k * step));
   }
   wave_argmax(bv, bi);
   if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = bv; si[threadIdx.x >> 6] = bi; }
