@@ -163,7 +163,7 @@ void launch_attn_oproj(const AttnDecodeFusedArgs& a, const void* W, float* y, in
 
 // All layers of one decode step in one launch (kernels_decode_stack.hip)
 constexpr int DECODE_STACK_BLOCKS = 256;          // a block per CU: all of them have to be on the GPU together
-constexpr int DECODE_STACK_EXCHANGE = 800 * 1024; // bytes, zeroed once
+constexpr int DECODE_STACK_EXCHANGE = 2200 * 1024; // bytes, zeroed once
 constexpr int DECODE_STACK_POLLS = 100000;        // 50 ms or more
 struct DecodeStackLayer { const void *wqkv, *wo, *wgu, *wdown, *in_norm, *post_norm, *q_norm, *k_norm; };
 struct DecodeStackArgs {
@@ -193,12 +193,13 @@ struct DecodeAttnArgs {
   unsigned* exchange;
   unsigned *fail_dev, *fail_host;
   uint32_t epoch;
-  int kv_len, nsplit;               // nsplit: of attn_decode_defer_splits, whose sums these are
+  int kv_len, nsplit;               // nsplit: of attn_decode_defer_splits, whose sums these are, or (direct) of the launch that joins its splits itself: a page a wave
+  int direct;
   int polls;
   float eps, scale;
 };
 bool decode_attn_sizes_ok(int width, int heads, int kv_heads, int head_dim);
-bool decode_attn_splits_ok(int nsplit, int npages);
+bool decode_attn_splits_ok(int nsplit, int npages, bool direct);
 void launch_decode_attn(const DecodeAttnArgs& a, hipStream_t st);
 
 struct AttnPrefillArgs {

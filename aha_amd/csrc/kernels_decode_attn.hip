@@ -1,15 +1,17 @@
-// The attention half of a layer of one decode step in ONE launch: norm, q k v, attention, o_proj, residual (4096 columns, 32 query and 8 kv heads of 128 dims, up to 24
+// The attention half of a layer of one decode step in ONE launch: norm, q k v, attention, o_proj, residual (4096 columns, 32 query and 8 kv heads of 128 dims, up to 64
 // pages of positions).
 //
 // As three launches these took 24.1 us a layer for 84 MB of weights (13.3 at the rate HBM reaches): q k v 9.4, attention 5.5 with HBM idle, o_proj 9.3 of which 4 are
 // its own start and the merge of the attention's splits in every block.  Here a block per CU has its part of both projections (196 KB and 131 KB, in the registers of four
 // waves), and o_proj's weights come while four other waves exchange and attend.  XCD x = b % 8 has kv head x with its four query heads, block s = b / 8 there
 //   24 of the head's 768 rows of q, k, v, shared inside the XCD;
-//   the pages of attention unit s (16 units at most; a wave the scores of 16 tokens, then 32 dims of the sums), shared inside the XCD;
-//   from block 16 on: 32 of the head's 512 joined sums, which go to everybody;
+//   the pages of attention unit s (16 units at most; a wave the scores of 16 tokens, then 32 dims of the sums), shared inside the XCD; beyond 24 pages (DIRECT) pages s and
+//     s + 32, each a unit of its own, as the attention launch has it there;
+//   from block 16 on: 32 of the head's 512 joined sums, which go to everybody (DIRECT: 16 by every block);
 //   16 whole rows of o_proj.
 // Of 19 us q k v take 8.5, the hand-off of q k v 1.2, norm and rotation 0.4, a page 1.0, the units' hand-off and the join 2.1, the joined sums' 2.5 (all 256 blocks ask for
-// all of them), o_proj behind them 1.3.  us a layer of 8B with gate, up and down (49.6): 20 positions 71.1 -> 69.6, 300: 73.5 -> 69.8, 900: 74.3 -> 69.9, 1400: 75.1 -> 70.3.
+// all of them), o_proj behind them 1.3.  us a layer of 8B with gate, up and down (49.6): 20 positions 71.4 -> 70.1, 900: 74.6 -> 70.4, 1550: 76.4 -> 70.5,
+// 2200: 76.5 -> 71.2, 3900: 76.9 -> 72.5.
 // Exchange and bounded waits: kernels_decode_stack.hip.
 //
 // The same bits as the three launches (kernels_gemv.hip, attn_decode_body.h, kernels_gemv_fused.hip MergePro): lanes take the same columns in the same order, units
@@ -27,14 +29,14 @@ using namespace stack;
 
 constexpr int H = 4096, NH = 32, KVH = 8, D = 128, GR = NH / KVH, XCDS = 8, GROUP = DECODE_STACK_BLOCKS / XCDS;
 constexpr int QKV = (GR + 2) * D, QR = QKV / GROUP / 4, OR = H / DECODE_STACK_BLOCKS / 4;   // a kv head's rows; rows of q k v and of o_proj per wave
-constexpr int MAX_SPLITS = 4, NW = 4, MAX_UNITS = MAX_SPLITS * NW, PG = 2;                  // units of a split; pages of a unit
+constexpr int MAX_SPLITS = 4, NW = 4, MAX_UNITS = MAX_SPLITS * NW, PG = 2, DIRECT_SPLITS = GROUP * PG / NW;                  // units of a split; pages of a unit
 constexpr int VALUES = GR * D / (GROUP - MAX_UNITS);                                        // joined sums of a block without pages
 static_assert(QR == 6 && OR == 4 && VALUES == 32, "rows of a wave");
 
-// places of the exchange, bytes: per XCD q k v and the units' sums, for all the joined sums
+// places of the exchange, bytes: all the joined sums; per XCD q k v, then the units' sums
 constexpr int P_HEAD = 16 + D * 8, P_UNIT = GR * P_HEAD;   // max and sum, then the 128 sums, each with its tag
-constexpr int AT_Q = 0, AT_P = AT_Q + QKV * 4, PER_XCD = (AT_P + MAX_UNITS * P_UNIT + 127) / 128 * 128;
-constexpr int AT_A = XCDS * PER_XCD, EXCHANGE = AT_A + H * 4;
+constexpr int AT_A = 0, AT_Q = AT_A + H * 4, AT_P = AT_Q + XCDS * QKV * 4, EXCHANGE = AT_P + XCDS * DIRECT_SPLITS * NW * P_UNIT;
+static_assert(AT_P % 128 == 0 && P_UNIT % 64 == 0, "a tag's place never holds a value, whichever number of units is in use");
 static_assert(EXCHANGE <= DECODE_STACK_EXCHANGE, "exchange buffer");
 
 struct Lds {
@@ -42,10 +44,11 @@ struct Lds {
   bf16_t q[GR * D], k[D], v[D];
   float sc[PG][GR * 64];
   float red[4];
-  float4 part[2][64];
+  float4 part[4][64];
 };
-// naps of 64 clocks (27 ns): before the first weights are asked for (x comes first), before the units' sums, before all the joined sums
-constexpr int NAP_W = 8, NAP_P = 20, NAP_A = 40;
+// naps of 64 clocks (27 ns): before the first weights are asked for (x comes first: 8 naps 70.9 us a layer, 12: 70.1,
+// 16: 70.3, 22: 70.4), before the units' sums, before all the joined sums
+constexpr int NAP_W = 12, NAP_P = 20, NAP_A = 40;
 #define IN_ORDER __builtin_amdgcn_sched_barrier(0)
 
 // h of eight columns and eight weights, in the order of gemv_body.h
@@ -61,7 +64,8 @@ __device__ __forceinline__ float add_group(const Lds& lds, int u, int lane, u32x
 // ---- the waves that hold weights -------------------------------------------------------------------------------------------------------------
 // What a CU loads comes back in the order it was asked for, whoever asked, so a poll waits for every weight in front of it.  o_proj's are therefore asked for two
 // rows x 512 columns a wave at a time, 16 KB a block in flight: at 24 the hand-offs, at 8 the weights are what the block waits for.  us a layer at 300 and 1400 positions: all
-// asked for as registers become free, by the four waves that wait as well 71.3 / 72.3; four rows at a time 69.9 / 70.3; two 69.8 / 70.3.
+// asked for as registers become free, by the four waves that wait as well 71.3 / 72.3; four rows at a time 69.9 / 70.3; two 69.8 / 70.3 (each with a later start, as NAP_W has it now).
+template <bool DIRECT>
 __device__ __forceinline__ void weight_waves(const DecodeAttnArgs& a, Lds& lds, const int b, const int w, const bool has_page, const bool has_second) {
   const int lane = threadIdx.x & 63, G = lane >> 4, c = lane & 15, x = b % XCDS, s = b / XCDS;
   const uint32_t t16 = a.epoch & 0xffffu, l16 = (uint32_t)lane * 16;
@@ -115,13 +119,14 @@ __device__ __forceinline__ void weight_waves(const DecodeAttnArgs& a, Lds& lds, 
     }
     const float ya = four_sums(y[0], y[1], y[2], y[3]), yb = four_sums(y[4], y[5], y[4], y[5]);   // (the order of wave_sum)
     const int j = r24 + (c == 0 ? G : 4 + G);
-    __builtin_amdgcn_raw_buffer_store_b32(((uint32_t)f2bf(c == 0 ? ya : yb) << 16) | t16, ex, c == 0 || (c == 1 && G < 2) ? x * PER_XCD + AT_Q + j * 4 : NOWHERE, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b32(((uint32_t)f2bf(c == 0 ? ya : yb) << 16) | t16, ex, c == 0 || (c == 1 && G < 2) ? AT_Q + x * QKV * 4 + j * 4 : NOWHERE, 0, 0);
   }
   next_o(1);
   meet();
   next_o(2);
   if (has_page) meet();
   if (has_second) meet();
+  if constexpr (DIRECT) meet();
   next_o(3);
   next_o(4);
   next_o(5);
@@ -161,13 +166,14 @@ __device__ __forceinline__ void weight_waves(const DecodeAttnArgs& a, Lds& lds, 
 }
 
 // ---- the waves that wait, and attend ---------------------------------------------------------------------------------------------------------
+template <bool DIRECT>
 __device__ __forceinline__ void gather_waves(const DecodeAttnArgs& a, Lds& lds, const int b, const int w, const int npages, const bool has_page, const bool has_second) {
   const int lane = threadIdx.x & 63, tid = w * 64 + lane, G = lane >> 4, c = lane & 15, x = b % XCDS, s = b / XCDS;
-  const uint32_t tag = a.epoch, t16 = tag & 0xffffu, mine = x * PER_XCD, l16 = (uint32_t)lane * 16;
-  const int L_old = a.kv_len - 1, nunits = a.nsplit * NW, new_pg = L_old / KV_PAGE_TOKENS;
+  const uint32_t tag = a.epoch, t16 = tag & 0xffffu, q_at = AT_Q + x * QKV * 4, p_at = AT_P + x * (DIRECT ? DIRECT_SPLITS * NW : MAX_UNITS) * P_UNIT, l16 = (uint32_t)lane * 16;
+  const int L_old = a.kv_len - 1, step = DIRECT ? GROUP : a.nsplit * NW, new_pg = L_old / KV_PAGE_TOKENS;   // step: from a block's first page to its second
 
   // ---- requests ----
-  const uint64_t my_page = a.page_ptrs[lane < PG ? min(s + lane * nunits, new_pg) : new_pg];   // lanes 0, 1: the unit's pages, 2: the new token's
+  const uint64_t my_page = a.page_ptrs[lane < PG ? min(s + lane * step, new_pg) : new_pg];   // lanes 0, 1: the unit's pages, 2: the new token's
   u32x4_t xv[2], nv[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
@@ -227,7 +233,7 @@ __device__ __forceinline__ void gather_waves(const DecodeAttnArgs& a, Lds& lds, 
   // ---- a query head per wave, k by wave 0, v by wave 1 ----
   bf16_t y0, y1;
   {
-    const uint32_t at0 = mine + AT_Q + (w * D + lane) * 4, at1 = mine + AT_Q + ((GR + (w & 1)) * D + lane) * 4;
+    const uint32_t at0 = q_at + (w * D + lane) * 4, at1 = q_at + ((GR + (w & 1)) * D + lane) * 4;
     uint32_t v[4];
     poll.until(false, [&] {
       v[0] = __builtin_amdgcn_raw_buffer_load_b32(poll.ex, at0, 0, AUX_SC1);
@@ -289,21 +295,31 @@ __device__ __forceinline__ void gather_waves(const DecodeAttnArgs& a, Lds& lds, 
         for (int kk = 0; kk < 2; ++kk) o[i] = mfma16(as_frag(vf[i * 2 + kk]), pf[kk], o[i]);
       }
     };
-    do_page(s, lds.sc[0], kf[0], vf[0]);
-    if (has_second) do_page(s + nunits, lds.sc[1], kf[1], vf[1]);
-    z = group_sum(z);
-    const uint32_t at = mine + AT_P + s * P_UNIT + c * P_HEAD;
-    if (w == 0) {
-      const u32x4_t v = {__float_as_uint(m), tag, __float_as_uint(z), tag};
-      __builtin_amdgcn_raw_buffer_store_b128(v, poll.ex, lane < GR ? at : NOWHERE, 0, 0);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const u32x4_t v = {__float_as_uint(o[i][2 * j]), tag, __float_as_uint(o[i][2 * j + 1]), tag};
-        __builtin_amdgcn_raw_buffer_store_b128(v, poll.ex, c < GR ? at + 16 + (w * 32 + i * 16 + G * 4 + j * 2) * 8 : NOWHERE, 0, 0);
+    auto publish = [&](int unit) {
+      z = group_sum(z);
+      const uint32_t at = p_at + unit * P_UNIT + c * P_HEAD;
+      if (w == 0) {
+        const u32x4_t v = {__float_as_uint(m), tag, __float_as_uint(z), tag};
+        __builtin_amdgcn_raw_buffer_store_b128(v, poll.ex, lane < GR ? at : NOWHERE, 0, 0);
       }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const u32x4_t v = {__float_as_uint(o[i][2 * j]), tag, __float_as_uint(o[i][2 * j + 1]), tag};
+          __builtin_amdgcn_raw_buffer_store_b128(v, poll.ex, c < GR ? at + 16 + (w * 32 + i * 16 + G * 4 + j * 2) * 8 : NOWHERE, 0, 0);
+        }
+    };
+    do_page(s, lds.sc[0], kf[0], vf[0]);
+    if (has_second) {
+      if (DIRECT) {   // (a unit of its own)
+        publish(s);
+        m = -INFINITY, z = 0.f;
+        o[0] = o[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      }
+      do_page(s + step, lds.sc[1], kf[1], vf[1]);
+    }
+    publish(DIRECT && has_second ? s + step : s);
     IN_ORDER;
   }
 
@@ -315,10 +331,12 @@ __device__ __forceinline__ void gather_waves(const DecodeAttnArgs& a, Lds& lds, 
     at[w == 0 ? kpage_elem(t, lane + 64, 4) : vpage_elem(t, lane + 64)] = y1;
   }
 
-  // ---- 32 sums joined, by the XCD's blocks without pages: lane (split, value) what was a block's four waves, then the splits ----
-  if (s >= MAX_UNITS && w < 2) {
-    const int at32 = (s - MAX_UNITS) * VALUES + w * 16, q = at32 / D, dim = at32 % D + c;
-    const bool part = G < a.nsplit, own = G == a.nsplit - 1;
+  // ---- sums joined: lane (split, value) what was a block's four waves, then the splits ----
+  // up to four splits: 32 values by each of the XCD's blocks without pages, two waves of (4 splits, 16 values); more: 16 by every block, four such waves for 16 splits
+  const int first = DIRECT ? s * 16 : (s - MAX_UNITS) * VALUES + w * 16, q = first / D, dim = first % D + c;
+  if (DIRECT || (s >= MAX_UNITS && w < 2)) {
+    const int split = DIRECT ? w * 4 + G : G;
+    const bool part = split < a.nsplit, own = split == a.nsplit - 1;
     // the new token's scores (lane: head c, 32 dims)
     float d4[4] = {0.f, 0.f, 0.f, 0.f};
     const u32x4_t* qr = reinterpret_cast<const u32x4_t*>(lds.q + min(c, GR - 1) * D + G * 32);
@@ -334,23 +352,24 @@ __device__ __forceinline__ void gather_waves(const DecodeAttnArgs& a, Lds& lds, 
     nap(NAP_P);
     u32x4_t ml[NW];
     u32x2_t p[NW];
+    auto unit_of = [&](int i) { return DIRECT ? split * NW + i : i * a.nsplit + split; };   // of the block's wave i
     poll.until(!part, [&] {
       uint32_t bad = 0;
 #pragma unroll
       for (int i = 0; i < NW; ++i) {
-        const int unit = i * a.nsplit + G;
-        const uint32_t at = unit < npages ? mine + AT_P + unit * P_UNIT + q * P_HEAD : NOWHERE;   // (past the range: zeros)
+        const int unit = unit_of(i);
+        const uint32_t at = unit < npages ? p_at + unit * P_UNIT + q * P_HEAD : NOWHERE;   // (past the range: zeros)
         ml[i] = __builtin_amdgcn_raw_buffer_load_b128(poll.ex, at, 0, AUX_SC1);
         p[i] = __builtin_amdgcn_raw_buffer_load_b64(poll.ex, unit < npages ? at + 16 + dim * 8 : NOWHERE, 0, AUX_SC1);
       }
 #pragma unroll
       for (int i = 0; i < NW; ++i)
-        if (i * a.nsplit + G < npages) bad |= (ml[i][1] ^ tag) | (ml[i][3] ^ tag) | (p[i][1] ^ tag);
+        if (unit_of(i) < npages) bad |= (ml[i][1] ^ tag) | (ml[i][3] ^ tag) | (p[i][1] ^ tag);
       return bad == 0;
     });
     float mw[NW];
 #pragma unroll
-    for (int i = 0; i < NW; ++i) mw[i] = part && i * a.nsplit + G < npages ? __uint_as_float(ml[i][0]) : -INFINITY;
+    for (int i = 0; i < NW; ++i) mw[i] = part && unit_of(i) < npages ? __uint_as_float(ml[i][0]) : -INFINITY;
     float M = own ? s_new : -INFINITY, acc = 0.f, z = 0.f;
 #pragma unroll
     for (int i = 0; i < NW; ++i) M = fmaxf(M, mw[i]);
@@ -364,8 +383,29 @@ __device__ __forceinline__ void gather_waves(const DecodeAttnArgs& a, Lds& lds, 
       acc = fmaf(wt, mw[i] == -INFINITY ? 0.f : __uint_as_float(p[i][0]), acc);
       z = fmaf(wt, mw[i] == -INFINITY ? 0.f : __uint_as_float(ml[i][2]), z);
     }
-    lds.part[w][lane] = make_float4(M, z, acc, 0.f);   // (read by this wave alone; a split that is not there: nothing, by weight 0)
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    lds.part[w][lane] = make_float4(M, z, acc, 0.f);   // (a split that is not there: nothing, by weight 0)
+  }
+  auto share = [&](float v) {
+    __builtin_amdgcn_raw_buffer_store_b32(((uint32_t)f2bf(v) << 16) | t16, poll.ex, lane < 16 ? AT_A + (x * GR * D + first + c) * 4 : NOWHERE, 0, AUX_SC1);
+  };
+  if (DIRECT) {
+    meet();
+    if (w == 0) {
+      const float4* const part = &lds.part[0][0];
+      const float4 mine4 = part[c * 16];   // lane c: split c's maximum and sum
+      const float MM = row_max(mine4.x), wt = mine4.x == -INFINITY ? 0.f : __expf(mine4.x - MM);
+      float wz = wt * mine4.y;
+      asm volatile("" : "+v"(wz));   // (rounded, not fused into the sum)
+      const float inv = 1.0f / row_sum(wz);
+      float t[DIRECT_SPLITS], h = 0.f;
+#pragma unroll
+      for (int i = 0; i < DIRECT_SPLITS; ++i) t[i] = part[i * 16 + c].z;
+#pragma unroll
+      for (int i = 0; i < DIRECT_SPLITS; ++i) h = fmaf(__uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(wt), i)), t[i], h);
+      share(h * inv);
+    }
+  } else if (s >= MAX_UNITS && w < 2) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (of this wave, read by it alone)
     float4 t[MAX_SPLITS];
 #pragma unroll
     for (int i = 0; i < MAX_SPLITS; ++i) t[i] = lds.part[w][i * 16 + c];
@@ -377,7 +417,7 @@ __device__ __forceinline__ void gather_waves(const DecodeAttnArgs& a, Lds& lds, 
       zz = fmaf(wt, t[i].y, zz);
       h = fmaf(wt, t[i].z, h);
     }
-    __builtin_amdgcn_raw_buffer_store_b32(((uint32_t)f2bf(h * (1.0f / zz)) << 16) | t16, poll.ex, lane < 16 ? AT_A + (x * GR * D + at32 + c) * 4 : NOWHERE, 0, AUX_SC1);
+    share(h * (1.0f / zz));
   }
   nap(NAP_A);
 
@@ -403,19 +443,22 @@ __device__ __forceinline__ void gather_waves(const DecodeAttnArgs& a, Lds& lds, 
   }
 }
 
+template <bool DIRECT>
 __global__ __launch_bounds__(512, 2) void decode_attn_kernel(const DecodeAttnArgs a) {
   __shared__ __attribute__((aligned(16))) Lds lds;
   const int b = blockIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), s = b / XCDS;
-  const int npages = (a.kv_len - 1 + KV_PAGE_TOKENS - 1) / KV_PAGE_TOKENS, nunits = a.nsplit * NW;
-  const bool has_page = s < nunits && s < npages, has_second = s < nunits && s + nunits < npages;
-  if (wave < 4) weight_waves(a, lds, b, wave, has_page, has_second);
-  else gather_waves(a, lds, b, wave - 4, npages, has_page, has_second);
+  const int npages = (a.kv_len - 1 + KV_PAGE_TOKENS - 1) / KV_PAGE_TOKENS, units = DIRECT ? GROUP : a.nsplit * NW;   // (direct: as many blocks as there are)
+  const bool has_page = s < units && s < npages, has_second = s < units && s + units < npages;
+  if (wave < 4) weight_waves<DIRECT>(a, lds, b, wave, has_page, has_second);
+  else gather_waves<DIRECT>(a, lds, b, wave - 4, npages, has_page, has_second);
 }
 
 }  // namespace
 
 bool decode_attn_sizes_ok(int width, int heads, int kv_heads, int head_dim) { return width == H && heads == NH && kv_heads == KVH && head_dim == D; }
-bool decode_attn_splits_ok(int nsplit, int npages) { return nsplit >= 1 && nsplit <= MAX_SPLITS && npages <= PG * NW * nsplit; }
-void launch_decode_attn(const DecodeAttnArgs& a, hipStream_t st) { hipLaunchKernelGGL(decode_attn_kernel, dim3(DECODE_STACK_BLOCKS), dim3(512), 0, st, a); }
+bool decode_attn_splits_ok(int nsplit, int npages, bool direct) {
+  return direct ? nsplit <= DIRECT_SPLITS && npages <= NW * nsplit : nsplit >= 1 && nsplit <= MAX_SPLITS && npages <= PG * NW * nsplit;
+}
+void launch_decode_attn(const DecodeAttnArgs& a, hipStream_t st) { hipLaunchKernelGGL(a.direct ? decode_attn_kernel<true> : decode_attn_kernel<false>, dim3(DECODE_STACK_BLOCKS), dim3(512), 0, st, a); }
 
 }  // namespace aha

@@ -1571,8 +1571,8 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_read
   for (int p = 1; p < npages && page_stride; ++p)
     if (m->h_page_ptrs[p] != m->h_page_ptrs[0] + p * page_stride) page_stride = 0;
   if (page_stride > 0xffffffffu) page_stride = 0;
-  // 8B sizes, up to 24 pages: a layer's attention half in one launch, the same bits
-  const bool joined = m->d_stack_exchange && !slices && defer && decode_attn_sizes_ok(H, nh, kvh, d) && decode_attn_splits_ok(defer, npages) && model_stack_takes(m);
+  // 8B sizes, up to 64 pages: a layer's attention half in one launch, the same bits
+  const bool joined = m->d_stack_exchange && !slices && !e_div && decode_attn_sizes_ok(H, nh, kvh, d) && decode_attn_splits_ok(nsplit, npages, !defer) && model_stack_takes(m);
   for (int li = 0; li < c.num_hidden_layers; ++li) {
     const LayerWeights& L = m->layers[li];
     if (joined) {
@@ -1580,7 +1580,7 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_read
       const KvLayer kv = model_kv_layer(m, li);
       a.x = m->d_x; a.in_norm = L.in_norm; a.wqkv = L.wqkv; a.wo = L.wo; a.q_norm = L.q_norm; a.k_norm = L.k_norm; a.rope = m->d_rope;
       a.page_ptrs = kv.page_ptrs; a.layer_off = kv.layer_off; a.exchange = m->d_stack_exchange; a.fail_dev = m->d_stack_fail; a.fail_host = m->h_stack_fail_dev;
-      a.epoch = model_stack_epoch(m); a.kv_len = (int)kv_len_after; a.nsplit = defer; a.polls = m->stack_polls; a.eps = c.rms_norm_eps; a.scale = m->attn_scale;
+      a.epoch = model_stack_epoch(m); a.kv_len = (int)kv_len_after; a.nsplit = nsplit; a.direct = !defer; a.polls = m->stack_polls; a.eps = c.rms_norm_eps; a.scale = m->attn_scale;
       launch_decode_attn(a, st);
     } else {  // h = RMSNorm(x); qkv = h Wqkv^T                      (qwen3/model.rs:79, modules.rs:538-552)
       GemvArgs g{};

@@ -259,10 +259,11 @@ def wide_models(monkeypatch, layers=2):
 @pytest.mark.parametrize("scrambled", [False, True])
 def test_attention_half_in_one_launch(gpu, monkeypatch, scrambled):
     """4096 columns: a layer's q k v, attention and o_proj in one launch (kernels_decode_attn.hip) give the bits of three.  No page behind the new token, pages' edges, one,
-    three and four splits, units with two pages, the last length that is taken (24 pages) and the first that is not."""
+    three and four splits, units with two pages (up to 24 pages); splits of a page a wave, seven to sixteen of them, a page and two pages a block (33 and on); the last length that is
+    taken (64 pages) and the first that is not."""
     cfg, plain, m = wide_models(monkeypatch)
     m.debug_scramble_pages(scrambled)
-    for S in [1, 63, 64, 65, 255, 256, 257, 319, 320, 384, 448, 700, 1023, 1024, 1025, 1471, 1534]:
+    for S in [1, 63, 64, 65, 255, 256, 257, 319, 320, 384, 448, 700, 1023, 1024, 1025, 1471, 1534, 1599, 1791, 2046, 2048, 2111, 3000, 4094]:
         ids = ids_for(cfg, S, 9 + S)
         m.clear_cache(); plain.clear_cache()
         _, tok = plain.forward_initial(ids, 0)
@@ -273,7 +274,7 @@ def test_attention_half_in_one_launch(gpu, monkeypatch, scrambled):
             b, _ = m.forward_step(tok, S + step)
             np.testing.assert_array_equal(a, b, err_msg=str((S, step)))
             tok = am
-        assert m.debug_decode_stack() == (before + 2 * (2 if S == 1534 else 3), 0), S
+        assert m.debug_decode_stack() == (before + 2 * (2 if S == 4094 else 3), 0), S
     assert plain.debug_decode_stack()[0] == 0
     m.close(); plain.close()
 
