@@ -1433,11 +1433,12 @@ __global__ void embed_state_kernel(const bf16_t* __restrict__ table, const StepS
     rope[64 + i] = rbf(sinf(ang));
   }
 }
-__device__ __forceinline__ void advance_state(StepState* st, uint32_t t, uint32_t* token_log, uint32_t* host_ring, uint32_t* host_done) {
+// t: 0xffffffff where no logit is a number.  The host is told so; the next step, which may be queued already, embeds a token that there is.
+__device__ __forceinline__ void advance_state(StepState* st, uint32_t t, int vocab, uint32_t* token_log, uint32_t* host_ring, uint32_t* host_done) {
   const int32_t step = st->step;
   token_log[step & 0xffff] = t;
   st->step = step + 1;
-  st->token = t;
+  st->token = min(t, (uint32_t)vocab - 1u);
   st->pos[0] += 1;
   st->pos[1] += 1;
   st->pos[2] += 1;
@@ -1447,8 +1448,8 @@ __device__ __forceinline__ void advance_state(StepState* st, uint32_t t, uint32_
   __hip_atomic_store(host_ring + ((uint32_t)step % RING_CAP), t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   __hip_atomic_store(host_done, (uint32_t)step + 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-__global__ void advance_state_kernel(StepState* st, uint32_t* token_log, uint32_t* host_ring, uint32_t* host_done) {
-  advance_state(st, st->next_token, token_log, host_ring, host_done);
+__global__ void advance_state_kernel(StepState* st, int vocab, uint32_t* token_log, uint32_t* host_ring, uint32_t* host_done) {
+  advance_state(st, st->next_token, vocab, token_log, host_ring, host_done);
 }
 // Between two steps of the greedy loop in one launch: the arg-max of the lm_head's partials (argmax_partials_kernel), advance_state_kernel, and the next
 // step's embed_state_kernel.  One block: three dependent round trips to memory (partials, embedding row, the publication) -- 5.1 us where the three launches
@@ -1477,7 +1478,7 @@ __global__ __launch_bounds__(1024) void next_step_kernel(const float* __restrict
   for (int i = tid; i < H / 8; i += 1024) reinterpret_cast<u32x4_t*>(out)[i] = src[i];
   if (tid == 1023) {
     st->next_token = bi;
-    advance_state(st, bi, token_log, host_ring, host_done);
+    advance_state(st, bi, vocab, token_log, host_ring, host_done);
   }
 }
 
@@ -1828,7 +1829,7 @@ int model_decode_greedy(aha_model* m, uint32_t first_token, size_t offset, size_
                            (const bf16_t*)m->embed, c.vocab_size, c.hidden_size, (bf16_t*)m->d_x, m->d_inv_freq, m->d_axis_map, m->d_rope, m->d_token_log, m->h_ring_dev,
                            m->h_done_dev);
       } else {
-        hipLaunchKernelGGL(advance_state_kernel, dim3(1), dim3(1), 0, m->stream, m->d_state, m->d_token_log, m->h_ring_dev, m->h_done_dev);
+        hipLaunchKernelGGL(advance_state_kernel, dim3(1), dim3(1), 0, m->stream, m->d_state, c.vocab_size, m->d_token_log, m->h_ring_dev, m->h_done_dev);
       }
       ++enq;
     }

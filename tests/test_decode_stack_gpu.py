@@ -297,3 +297,27 @@ def test_attention_half_that_gives_up(gpu, monkeypatch):
     np.testing.assert_array_equal(m.last_logits(), plain.last_logits())
     assert m.debug_decode_stack()[1] == 2
     m.close(); plain.close()
+
+
+@pytest.mark.parametrize("design, dtype", [("dense", "bfloat16"), ("post-norm", "bfloat16"), ("post-norm", "float32"), ("state-space", "bfloat16"), ("state-space", "float32")])
+def test_device_loop_without_an_arg_max(gpu, design, dtype):
+    """No logit is a number: the loop's steps, queued ahead of the host, embed a token that there is, and every token is reported as none (0xffffffff)."""
+    from aha_amd.model import HipInferenceModel
+    if design == "dense":
+        cfg = tiny_qwen3(layers=2, hidden=256, heads=4, kv_heads=2, inter=512, vocab=512)
+        w, norm = qwen3_text_weights(cfg, seed=1), "model.norm.weight"
+    elif design == "post-norm":
+        from tests import test_dosovik_gpu as t
+        cfg = t.config([t.layer(), t.layer()], dtype=dtype)
+        w, norm = t.dosovik_weights(cfg, seed=1), "final.norm"
+    else:
+        from tests import test_vamatar_gpu as t
+        cfg = t.config([t.ssm(), t.att()], dtype=dtype)
+        w, norm = t.vamatar_weights(cfg, seed=1), "final.norm"
+    assert norm in w
+    w[norm][:] = float("nan")
+    m = HipInferenceModel(cfg, w)
+    m.forward_initial([3, 1, 2], 0)
+    assert m.decode_greedy(5, 3, 9) == [0xffffffff] * 9
+    assert not np.isfinite(m.last_logits()).any()
+    m.close()
