@@ -748,6 +748,7 @@ int layered_forward_batch(aha_model* m, const aha_batch_entry* en, size_t n_en, 
     b.one = he[0];
   }
   const uint32_t* ids = (const uint32_t*)(l.d_meta + o_ids);
+  const uint32_t before = m->stack_epoch;
   Tail t = run_step(m, b, he, ids);
   for (size_t i = 0; i < n_en; ++i) advance_seq(m, l.seqs[en[i].seq], en[i].n_tokens);
   m->cache_len = l.seqs[0].len;
@@ -775,7 +776,7 @@ again:
   else if (argmax_out && want) AHA_HIP_CHECK(hipMemcpyAsync(l.h_meta + o_am, dam, want * 4, hipMemcpyDeviceToHost, m->stream));
   AHA_HIP_CHECK(hipGetLastError());
   AHA_HIP_CHECK(hipStreamSynchronize(m->stream));   // (the pinned step buffer is free again)
-  if (model_stack_failed(m)) {   // (a token of one sequence: as separate launches)
+  if (model_stack_failed(m) && m->stack_epoch != before) {   // (a token of one sequence, where such launches ran: as separate ones)
     ++m->stack_hold;
     t = run_step(m, b, he, ids);
     --m->stack_hold;

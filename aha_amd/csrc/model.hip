@@ -364,7 +364,7 @@ uint32_t model_stack_failed(aha_model* m) {
 }
 // Behind a wait for a single step: true if the step has been enqueued again, as separate launches
 static bool stack_redo(aha_model* m) {
-  if (!model_stack_failed(m)) return false;
+  if (!model_stack_failed(m) || !m->step_in_flight) return false;
   ++m->stack_hold;
   enqueue_decode_step(m, m->cache_len);
   --m->stack_hold;
@@ -1816,6 +1816,17 @@ int model_decode_greedy(aha_model* m, uint32_t first_token, size_t offset, size_
   std::vector<uint32_t> epochs;   // of the last launch of several stages behind each step
   epochs.reserve(max_new);
   size_t good = max_new;          // steps in front of one that gave up
+  auto enqueue_error = [&]() -> int {
+    AHA_HIP_CHECK(hipGetLastError());
+    const int e = m->async_rc;
+    m->async_rc = 0;
+    return e;
+  };
+  auto drained = [&](int e) {   // the call ends with an error: nothing of it is in flight or, given up, waits to be run again
+    (void)hipStreamSynchronize(m->stream);
+    model_stack_failed(m);
+    return e;
+  };
   while (seen < max_new && !stop) {
     size_t want = 0;
     if (!lockstep) want = enq < max_new && enq - seen < ahead ? std::min(max_new - enq, ahead - (enq - seen)) : 0;
@@ -1833,13 +1844,12 @@ int model_decode_greedy(aha_model* m, uint32_t first_token, size_t offset, size_
       }
       ++enq;
     }
-    AHA_HIP_CHECK(hipGetLastError());
-    if (m->async_rc) { const int e = m->async_rc; m->async_rc = 0; hipStreamSynchronize(m->stream); return e; }
+    if (const int e = enqueue_error()) return drained(e);
     size_t done = __atomic_load_n(m->h_done, __ATOMIC_ACQUIRE);
     for (unsigned spins = 0; done == seen; ++spins) {   // the next token: ~one step of GPU time away at most
       if ((spins & 1023u) == 1023u && hipStreamQuery(m->stream) == hipSuccess && __atomic_load_n(m->h_done, __ATOMIC_ACQUIRE) == seen) {
         set_error("decode loop: the stream drained without publishing a token");
-        return AHA_ERR_STATE;
+        return drained(AHA_ERR_STATE);
       }
       done = __atomic_load_n(m->h_done, __ATOMIC_ACQUIRE);
     }

@@ -321,3 +321,43 @@ def test_device_loop_without_an_arg_max(gpu, design, dtype):
     assert m.decode_greedy(5, 3, 9) == [0xffffffff] * 9
     assert not np.isfinite(m.last_logits()).any()
     m.close()
+
+
+def test_a_loop_that_ended_with_an_error_leaves_nothing(gpu, monkeypatch):
+    """The device loop returns an error (one that an earlier call of the host's thread left) with steps queued that give up: the prompt behind it is a prompt, not a
+    step to run again."""
+    import ctypes
+    cfg, plain, (m,) = models(monkeypatch)
+    ids, other = ids_for(cfg, 70, 5), ids_for(cfg, 90, 6)
+    _, tok = m.forward_initial(ids, 0)
+    m.debug_decode_stack(0)
+    assert ctypes.CDLL("libamdhip64.so").hipSetDevice(1000) != 0
+    with pytest.raises(RuntimeError):
+        m.decode_greedy(tok, 70, 12)
+    m.debug_decode_stack(100000)
+    m.clear_cache()
+    want, tok = plain.forward_initial(other, 0)
+    got, _ = m.forward_initial(other, 0)
+    np.testing.assert_array_equal(got, want)
+    close_to(plain.forward_step(tok, 90)[0], m.forward_step(tok, 90)[0], "the step behind")
+    m.close(); plain.close()
+
+
+def test_a_batch_that_ended_with_an_error_leaves_nothing(gpu, monkeypatch):
+    """The same for a step of the state-space design: the next portion of a further sequence, whose states are updated in place, runs once."""
+    import ctypes
+    cfg, plain, (m,) = pre_norm_models(monkeypatch)
+    ids = ids_for(cfg, 40, 7)
+    seqs = {}
+    for x in (plain, m):
+        seqs[x] = x.seq_open()
+        x.forward_batch([(seqs[x], ids[:20], [])])
+    m.forward_initial(ids[:5], 0)
+    m.debug_decode_stack(0)
+    assert ctypes.CDLL("libamdhip64.so").hipSetDevice(1000) != 0
+    with pytest.raises(RuntimeError):
+        m.forward_step(ids[5], 5)
+    m.debug_decode_stack(100000)
+    want, got = (x.forward_batch([(seqs[x], ids[20:30], [9])])[0] for x in (plain, m))
+    np.testing.assert_array_equal(got, want)
+    m.close(); plain.close()
