@@ -241,7 +241,7 @@ __device__ __forceinline__ void gather_waves(const DecodeAttnArgs& a, Lds& lds, 
       v[2] = __builtin_amdgcn_raw_buffer_load_b32(poll.ex, at1, 0, AUX_SC1);
       v[3] = __builtin_amdgcn_raw_buffer_load_b32(poll.ex, at1 + 256, 0, AUX_SC1);
       return (((v[0] ^ t16) | (v[1] ^ t16) | (v[2] ^ t16) | (v[3] ^ t16)) & 0xffffu) == 0;
-    });
+    }, [&] { v[0] = v[1] = v[2] = v[3] = 0; });
     auto norm_rope = [&](uint32_t d0, uint32_t d1, bf16_t w0, bf16_t w1, bf16_t& y0, bf16_t& y1) {
       float x0 = bf2f((bf16_t)(d0 >> 16)), x1 = bf2f((bf16_t)(d1 >> 16));
       const float ss = wave_sum(fmaf(x0, x0, x1 * x1));
@@ -366,6 +366,9 @@ __device__ __forceinline__ void gather_waves(const DecodeAttnArgs& a, Lds& lds, 
       for (int i = 0; i < NW; ++i)
         if (unit_of(i) < npages) bad |= (ml[i][1] ^ tag) | (ml[i][3] ^ tag) | (p[i][1] ^ tag);
       return bad == 0;
+    }, [&] {
+#pragma unroll
+      for (int i = 0; i < NW; ++i) ml[i] = NO_SPLIT, p[i] = u32x2_t{0u, 0u};
     });
     float mw[NW];
 #pragma unroll
@@ -431,7 +434,7 @@ __device__ __forceinline__ void gather_waves(const DecodeAttnArgs& a, Lds& lds, 
 #pragma unroll
       for (int j = 0; j < 4; ++j) bad |= (v[j][0] ^ t16) | (v[j][1] ^ t16) | (v[j][2] ^ t16) | (v[j][3] ^ t16);
       return (bad & 0xffffu) == 0;
-    });
+    }, [&] { v[0] = v[1] = v[2] = v[3] = u32x4_t{0u, 0u, 0u, 0u}; });
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       *reinterpret_cast<float4*>(lds.xs + xs_index(tid * 4 + j * 1024)) = make_float4(hi_bf(v[j][0]), hi_bf(v[j][1]), hi_bf(v[j][2]), hi_bf(v[j][3]));

@@ -369,7 +369,7 @@ __device__ __forceinline__ void gather_waves(const DecodeStackArgs& a, Lds& lds,
         v0 = __builtin_amdgcn_raw_buffer_load_b32(poll.ex, at, 0, AUX_SC1);
         v1 = __builtin_amdgcn_raw_buffer_load_b32(poll.ex, at + 256, 0, AUX_SC1);
         return (((v0 ^ t16) | (v1 ^ t16)) & 0xffffu) == 0;
-      });
+      }, [&] { v0 = v1 = 0; });
       bf16_t y0 = (bf16_t)(v0 >> 16), y1 = (bf16_t)(v1 >> 16);
       if (w < 3) {
         float x0 = bf2f(y0), x1 = bf2f(y1);
@@ -419,6 +419,9 @@ __device__ __forceinline__ void gather_waves(const DecodeStackArgs& a, Lds& lds,
 #pragma unroll
         for (int i = 0; i < N; ++i) bad |= (ml[i][1] ^ tag) | (ml[i][3] ^ tag) | (p[i][1] ^ tag);
         return bad == 0;
+      }, [&] {
+#pragma unroll
+        for (int i = 0; i < N; ++i) ml[i] = NO_SPLIT, p[i] = u32x2_t{0u, 0u};
       });
       float M = s_new;
 #pragma unroll
@@ -439,13 +442,13 @@ __device__ __forceinline__ void gather_waves(const DecodeStackArgs& a, Lds& lds,
       const float s_new = dot * a.scale;
       const int split = lane & 31;
       const uint32_t at = mine + AT_P + split * P_SPLIT + hd * P_HEAD;
-      u32x4_t ml = {__float_as_uint(-INFINITY), 0u, 0u, 0u}, p0 = {0u, 0u, 0u, 0u}, p1 = {0u, 0u, 0u, 0u};
+      u32x4_t ml = NO_SPLIT, p0 = {0u, 0u, 0u, 0u}, p1 = {0u, 0u, 0u, 0u};
       poll.until(split >= nsplit, [&] {
         ml = __builtin_amdgcn_raw_buffer_load_b128(poll.ex, at, 0, AUX_SC1);
         p0 = __builtin_amdgcn_raw_buffer_load_b128(poll.ex, at + 16 + d0 * 8, 0, AUX_SC1);
         p1 = __builtin_amdgcn_raw_buffer_load_b128(poll.ex, at + 32 + d0 * 8, 0, AUX_SC1);
         return ml[1] == tag && ml[3] == tag && p0[1] == tag && p0[3] == tag && p1[1] == tag && p1[3] == tag;
-      });
+      }, [&] { ml = NO_SPLIT, p0 = p1 = u32x4_t{0u, 0u, 0u, 0u}; });
       const float m = __uint_as_float(ml[0]), M = fmaxf(wave_max(m), s_new);
       const float wt = __expf(m - M), wn = __expf(s_new - M);
       const float z = half_wave_sum(wt * __uint_as_float(ml[2])) + wn;

@@ -301,7 +301,7 @@ __device__ __forceinline__ void gather_waves(const PrenormStackArgs& a, Lds& lds
     poll.until(!part, [&] {
       v = __builtin_amdgcn_raw_buffer_load_b64(poll.ex, at, 0, AUX_SC1);
       return v[1] == tag;
-    });
+    }, [&] { v = u32x2_t{0u, 0u}; });
     return __uint_as_float(v[0]);
   };
   auto four = [&](const void* p) {
@@ -346,7 +346,7 @@ __device__ __forceinline__ void gather_waves(const PrenormStackArgs& a, Lds& lds
         v0 = __builtin_amdgcn_raw_buffer_load_b128(poll.ex, mine + AT_X + t * 32, 0, AUX_SC1);
         v1 = __builtin_amdgcn_raw_buffer_load_b128(poll.ex, mine + AT_X + t * 32 + 16, 0, AUX_SC1);
         return v0[1] == tag && v0[3] == tag && v1[1] == tag && v1[3] == tag;
-      });
+      }, [&] { v0 = v1 = u32x4_t{0u, 0u, 0u, 0u}; });
       xv = make_float4(__uint_as_float(v0[0]), __uint_as_float(v0[2]), __uint_as_float(v1[0]), __uint_as_float(v1[2]));
     }
     {   // LayerNorm: the waves' means and squares about them, joined

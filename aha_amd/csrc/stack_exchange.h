@@ -11,6 +11,7 @@ constexpr uint32_t NOWHERE = 0x7fffffffu;   // past every descriptor's range: th
 constexpr int AUX_NT = 2, AUX_SC1 = 16;   // a load past the L1; a store through to memory
 
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_t;
+constexpr u32x4_t NO_SPLIT = {0xff800000u, 0u, 0u, 0u};   // what a split of the attention leaves that has no keys: its maximum (-inf) and its sum, each with its tag
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
 }
@@ -43,16 +44,19 @@ __device__ __forceinline__ void nap(int n) {
 // an address from memory, in the address space that it is in (a generic one would make flat loads)
 template <typename T>
 __device__ __forceinline__ const __attribute__((address_space(1))) T* global_at(const void* p) { return (const __attribute__((address_space(1))) T*)(uintptr_t)p; }
-// A wave that waits for values
+// A wave that waits for values.  One that has given up goes on with none() instead of what it last found: parts of other steps need not fit together (splits that
+// nobody ever wrote have the sum 0), and what such a step and the ones queued behind it append to the cache must be numbers, since the step that is run again
+// reads it with weight zero.
 struct Poller {
   __amdgpu_buffer_rsrc_t ex;
   int left;   // polls in vain that this wave still makes
-  template <class Load>   // load(): requests, and says whether everything is there
-  __device__ __forceinline__ void until(bool ok, Load&& load) {
+  template <class Load, class None>   // load(): requests, and says whether everything is there
+  __device__ __forceinline__ void until(bool ok, Load&& load, None&& none) {
     for (;;) {
       if (!ok) ok = load();
       asm volatile("" ::: "memory");
-      if (__all(ok) || left <= 0) return;
+      if (__all(ok)) return;
+      if (left <= 0) return none();
       --left;
     }
   }
@@ -62,7 +66,7 @@ struct Poller {
     until(!part, [&] {
       v = __builtin_amdgcn_raw_buffer_load_b128(ex, at, 0, AUX_SC1);
       return (((v[0] ^ t16) | (v[1] ^ t16) | (v[2] ^ t16) | (v[3] ^ t16)) & 0xffffu) == 0;
-    });
+    }, [&] { v = u32x4_t{0u, 0u, 0u, 0u}; });
     return v;
   }
   // `row` (a lane's, the same in both halves of the wave): the sum of what the eight XCDs left at `at`, (XCD, PITCH) f32 with their tags
@@ -77,7 +81,7 @@ struct Poller {
 #pragma unroll
       for (int i = 0; i < 4; ++i) bad |= p[i][1] ^ tag;
       return bad == 0;
-    });
+    }, [&] { p[0] = p[1] = p[2] = p[3] = u32x2_t{0u, 0u}; });
     const float y = (__uint_as_float(p[0][0]) + __uint_as_float(p[1][0])) + (__uint_as_float(p[2][0]) + __uint_as_float(p[3][0]));
     return halves(y, y);
   }

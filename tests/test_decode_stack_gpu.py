@@ -361,3 +361,36 @@ def test_a_batch_that_ended_with_an_error_leaves_nothing(gpu, monkeypatch):
     want, got = (x.forward_batch([(seqs[x], ids[20:30], [9])])[0] for x in (plain, m))
     np.testing.assert_array_equal(got, want)
     m.close(); plain.close()
+
+
+@pytest.mark.parametrize("hidden, heads, inter", [(1024, 16, 3072), (4096, 32, 1024)])
+@pytest.mark.parametrize("polls", [0, 1, 3, 10, 40])
+def test_what_gave_up_leaves_numbers(gpu, monkeypatch, polls, hidden, heads, inter):
+    """Scores of hundreds, among them a new token's far below zero: a step that gives up joins splits that are not there, and what it and the steps queued behind
+    it append lies on the pages that the step run again reads (with weight zero, which NaN survives).  Both one-launch forms of the dense stack."""
+    from aha_amd.model import HipInferenceModel
+    cfg = tiny_qwen3(layers=3, hidden=hidden, heads=heads, kv_heads=8, inter=inter, vocab=1024)
+    w = qwen3_text_weights(cfg, seed=14)
+    for k in w:
+        if k.endswith(("q_norm.weight", "k_norm.weight")):
+            w[k] = w[k] * 20
+    monkeypatch.setenv("AHA_DECODE_STACK", "0")
+    plain = HipInferenceModel(cfg, w)
+    monkeypatch.setenv("AHA_DECODE_STACK", "1")
+    launches = 3 if hidden == 4096 else 1
+    for S in (70, 130, 200):
+        m = HipInferenceModel(cfg, w)
+        ids = ids_for(cfg, S, S)
+        for _ in range(2):      # (the second time the exchange has values of the first)
+            plain.clear_cache(); m.clear_cache()
+            _, tok = plain.forward_initial(ids, 0)
+            m.forward_initial(ids, 0)
+            n, gone = m.debug_decode_stack(polls)
+            want, got = plain.decode_greedy(tok, S, 8), m.decode_greedy(tok, S, 8)
+            assert np.isfinite(m.last_logits()).all(), S
+            after = m.debug_decode_stack()
+            if hidden == 4096 or after == (n + 4 * launches, gone + 1):   # (the same bits in any case; or none of its four queued steps counted)
+                assert got == want, S
+                np.testing.assert_array_equal(m.last_logits(), plain.last_logits())
+        m.close()
+    plain.close()
