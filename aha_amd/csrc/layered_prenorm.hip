@@ -731,7 +731,8 @@ static Tail prenorm_single(aha_model* m, const SeqBatch& b, const uint32_t* ids)
     }
   };
   // (the recurrence of a run that gave up is run again: its states must not have been written over)
-  const bool stacked = l.d_ops && !l.keep && b.one.state_in != b.one.state_out && model_stack_takes(m);
+  StackTurn turn;
+  const bool stacked = l.d_ops && !l.keep && b.one.state_in != b.one.state_out && turn.take(m, false);
   if (!stacked) {
     for (int li = 0; li < c.num_hidden_layers; ++li) {
       mixer(li);

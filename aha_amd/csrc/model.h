@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -223,9 +224,12 @@ int model_forward_step(aha_model* m, uint32_t token, size_t offset, float* logit
 int model_forward_step_enqueue(aha_model* m, uint32_t token, size_t offset);
 // steps whose layers run as one launch or a few (kernels_decode_stack.hip, kernels_prenorm_stack.hip)
 int model_stack_alloc(aha_model* m, bool* have);   // the exchange buffer, where the device takes such launches
-bool model_stack_takes(aha_model* m);              // may the step that is being enqueued use them?
+struct StackTurn {                                 // the device's turn at such launches, from before a step's first one until its last is enqueued
+  bool take(aha_model* m, bool same_bits);         // may the step that is being enqueued use them?  same_bits: the separate launches give the same
+  std::unique_lock<std::mutex> lk;
+};
 uint32_t model_stack_epoch(aha_model* m);          // of its next one
-uint32_t model_stack_failed(aha_model* m);         // the stream is idle: the epoch of a launch that gave up (0: none), which is forgotten; others may use them now
+uint32_t model_stack_failed(aha_model* m);         // the stream is idle: the epoch of a launch that gave up (0: none), which is forgotten
 int model_wait_step(aha_model* m);   // before anything that the host or another stream does to what a step reads or writes
 int model_decode_greedy(aha_model* m, uint32_t first_token, size_t offset, size_t max_new, uint32_t* out);
 int model_clear_cache(aha_model* m);

@@ -11,7 +11,6 @@
 #include <string.h>
 
 #include <algorithm>
-#include <atomic>
 #include <chrono>
 
 #include "argmax.h"
@@ -326,26 +325,48 @@ int alloc_slab(aha_model* m) {
 }
 
 // ---- one launch per decode step: who may, and what happens when it gives up (kernels_decode_stack.hip) ----
-// The blocks of such a launch wait for each other, so two of them that share the GPU could each hold what the other needs: one model per device at a time has
-// the right to it, from its first step in flight until that step has been waited for; a step of another model meanwhile runs as separate launches.
+// The blocks of such a launch wait for each other, so two of them that share the GPU could each hold what the other needs: models on one device take turns.  A
+// step's launches are enqueued under the device's lock, behind what the model of the turn before has in flight.  Which form a step takes must hang on its own
+// model alone where the forms sum in different orders (0.6B): a request's tokens are not to depend on who else is decoding.  Two 0.6B models in their loops
+// take 710 us a token each (345 alone); with separate launches for whoever came second they took 690 and 362, and tokens that differed from run to run.
+// Where both forms give the same bits (8B) the second one does not wait: 5.0 and 4.15 ms a token that way, 5.5 each by turns.
 constexpr int STACK_MAX_FAILS = 3;    // steps given up after which a model stays with separate launches
 constexpr int STACK_MAX_PAGES = 512;   // 32768 positions: 980 us a token, 1210 as separate launches (a page more costs 1.3 us here, 0.9 there)
-static std::atomic<aha_model*> g_stack_owner[64];
-static bool stack_acquire(aha_model* m) {
-  auto& owner = g_stack_owner[m->ctx->device & 63];
-  aha_model* none = nullptr;
-  return owner.load() == m || owner.compare_exchange_strong(none, m);
-}
-static void stack_release(aha_model* m) {
-  aha_model* me = m;
-  g_stack_owner[m->ctx->device & 63].compare_exchange_strong(me, nullptr);
+struct StackTurns {
+  std::mutex mu;
+  aha_model* last = nullptr;    // had the last turn and has not been waited for since
+  hipEvent_t behind = nullptr;
+};
+static StackTurns g_stack_turns[64];
+static StackTurns& stack_turns(const aha_model* m) { return g_stack_turns[m->ctx->device & 63]; }
+static void stack_release(aha_model* m) {   // its stream is idle
+  StackTurns& t = stack_turns(m);
+  std::lock_guard<std::mutex> lk(t.mu);
+  if (t.last == m) t.last = nullptr;
 }
 static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_ready = false, bool arg_max = true);
 // Not where a profile, a timeline or a knob asks for the separate launches.
-bool model_stack_takes(aha_model* m) {
+bool StackTurn::take(aha_model* m, bool same_bits) {
   if (!m->d_stack_exchange || m->stack_hold > 0 || m->stack_fails >= STACK_MAX_FAILS || !m->decode_fused || m->profiling) return false;
   static const bool knobs = getenv("AHA_ATTN_PAGES_PER_BLOCK") || getenv("AHA_ATTN_TRACE") || getenv("AHA_GEMV_TRACE") || !gemv_row_on();
-  return !knobs && stack_acquire(m);
+  if (knobs) return false;
+  StackTurns& t = stack_turns(m);
+  lk = std::unique_lock<std::mutex>(t.mu);
+  if (t.last && t.last != m) {
+    if (same_bits) {
+      lk.unlock();
+      return false;
+    }
+    // (its stream lives: a model gives its turn back before it goes)
+    if ((!t.behind && hipEventCreateWithFlags(&t.behind, hipEventDisableTiming) != hipSuccess) || hipEventRecord(t.behind, t.last->stream) != hipSuccess ||
+        hipStreamWaitEvent(m->stream, t.behind, 0) != hipSuccess) {
+      (void)hipGetLastError();
+      lk.unlock();
+      return false;
+    }
+  }
+  t.last = m;
+  return true;
 }
 uint32_t model_stack_epoch(aha_model* m) {
   if (++m->stack_epoch == 0) ++m->stack_epoch;
@@ -1546,7 +1567,8 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_read
                        m->d_inv_freq, m->d_axis_map, m->d_rope);
   }
   const int npages = (int)((kv_len_after + KV_PAGE_TOKENS - 1) / KV_PAGE_TOKENS);
-  if (m->d_stack_layers && npages <= STACK_MAX_PAGES && model_stack_takes(m)) {
+  StackTurn turn;
+  if (m->d_stack_layers && npages <= STACK_MAX_PAGES && turn.take(m, false)) {
     DecodeStackArgs a{};
     a.layers = m->d_stack_layers; a.x_in = m->d_x; a.x_out = m->d_x; a.rope = m->d_rope; a.page_ptrs = m->d_page_ptrs; a.layer_stride = m->layer_stride;
     a.exchange = m->d_stack_exchange; a.fail_dev = m->d_stack_fail; a.fail_host = m->h_stack_fail_dev;
@@ -1573,7 +1595,7 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_read
     if (m->h_page_ptrs[p] != m->h_page_ptrs[0] + p * page_stride) page_stride = 0;
   if (page_stride > 0xffffffffu) page_stride = 0;
   // 8B sizes, up to 64 pages: a layer's attention half in one launch, the same bits
-  const bool joined = m->d_stack_exchange && !slices && !e_div && decode_attn_sizes_ok(H, nh, kvh, d) && decode_attn_splits_ok(nsplit, npages, !defer) && model_stack_takes(m);
+  const bool joined = m->d_stack_exchange && !slices && !e_div && decode_attn_sizes_ok(H, nh, kvh, d) && decode_attn_splits_ok(nsplit, npages, !defer) && turn.take(m, true);
   for (int li = 0; li < c.num_hidden_layers; ++li) {
     const LayerWeights& L = m->layers[li];
     if (joined) {

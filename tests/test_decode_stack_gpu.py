@@ -394,3 +394,40 @@ def test_what_gave_up_leaves_numbers(gpu, monkeypatch, polls, hidden, heads, int
                 np.testing.assert_array_equal(m.last_logits(), plain.last_logits())
         m.close()
     plain.close()
+
+
+def test_two_models_give_the_bits_of_one(gpu, monkeypatch):
+    """Beside another model, its prompts and its steps, one that nobody has waited for among them, a model's steps take the form that they take alone: its logits and
+    tokens are those of a model alone."""
+    cfg, plain, (alone, *ms) = models(monkeypatch, 3)
+    plain.close()
+    prompts, fed = [ids_for(cfg, 50, 1), ids_for(cfg, 90, 2)], ids_for(cfg, 40, 3)
+
+    def run(m, i):
+        out = []
+        for _ in range(3):
+            m.clear_cache()
+            _, tok = m.forward_initial(prompts[i], 0)
+            out += [m.forward_step(t, len(prompts[i]) + k)[0] for k, t in enumerate(fed)]
+            out.append(np.array(m.decode_greedy(tok, len(prompts[i]) + len(fed), 60)))
+        m.forward_step_enqueue(5, len(prompts[i]) + len(fed) + 60)
+        return out
+    want, got = [run(alone, i) for i in range(2)], [None, None]
+    steps = alone.debug_decode_stack()[0] // 2     # (and waits for it)
+    ms[0].forward_initial(prompts[0], 0)
+    ms[0].forward_step_enqueue(7, 50)
+
+    def thread(i):
+        got[i] = run(ms[i], i)
+    threads = [threading.Thread(target=thread, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for i in range(2):
+        assert len(got[i]) == len(want[i])
+        for k, (a, b) in enumerate(zip(want[i], got[i])):
+            np.testing.assert_array_equal(a, b, err_msg=str((i, k)))
+    assert [m.debug_decode_stack() for m in ms] == [(steps + 1, 0), (steps, 0)]
+    for m in [alone] + ms:
+        m.close()
