@@ -128,6 +128,7 @@ struct aha_model {
   unsigned *h_stack_fail = nullptr, *h_stack_fail_dev = nullptr;   // (pinned, behind the token ring)
   uint32_t stack_epoch = 0;      // of the last such launch
   int stack_fails = 0;           // steps that had to be run again as separate launches
+  int64_t stack_pause = 0;       // steps that run as separate launches because others gave up
   int stack_hold = 0;            // > 0: separate launches for now
   int stack_polls = aha::DECODE_STACK_POLLS;
   int max_nsplit = 64;

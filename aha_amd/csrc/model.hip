@@ -330,7 +330,8 @@ int alloc_slab(aha_model* m) {
 // model alone where the forms sum in different orders (0.6B): a request's tokens are not to depend on who else is decoding.  Two 0.6B models in their loops
 // take 710 us a token each (345 alone); with separate launches for whoever came second they took 690 and 362, and tokens that differed from run to run.
 // Where both forms give the same bits (8B) the second one does not wait: 5.0 and 4.15 ms a token that way, 5.5 each by turns.
-constexpr int STACK_MAX_FAILS = 3;    // steps given up after which a model stays with separate launches
+constexpr int STACK_MAX_FAILS = 3;    // steps given up (50 ms and more each) after which a model stays with separate launches,
+constexpr int64_t STACK_PAUSE = 16384;   // for so many steps (8 s at 0.6B, more elsewhere), and then after every other one: at most 1 % is waited in vain
 constexpr int STACK_MAX_PAGES = 512;   // 32768 positions: 980 us a token, 1210 as separate launches (a page more costs 1.3 us here, 0.9 there)
 struct StackTurns {
   std::mutex mu;
@@ -347,9 +348,13 @@ static void stack_release(aha_model* m) {   // its stream is idle
 static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_ready = false, bool arg_max = true);
 // Not where a profile, a timeline or a knob asks for the separate launches.
 bool StackTurn::take(aha_model* m, bool same_bits) {
-  if (!m->d_stack_exchange || m->stack_hold > 0 || m->stack_fails >= STACK_MAX_FAILS || !m->decode_fused || m->profiling) return false;
+  if (!m->d_stack_exchange || m->stack_hold > 0 || !m->decode_fused || m->profiling) return false;
   static const bool knobs = getenv("AHA_ATTN_PAGES_PER_BLOCK") || getenv("AHA_ATTN_TRACE") || getenv("AHA_GEMV_TRACE") || !gemv_row_on();
   if (knobs) return false;
+  if (m->stack_pause > 0) {
+    --m->stack_pause;
+    return false;
+  }
   StackTurns& t = stack_turns(m);
   lk = std::unique_lock<std::mutex>(t.mu);
   if (t.last && t.last != m) {
@@ -379,8 +384,8 @@ uint32_t model_stack_failed(aha_model* m) {
   const uint32_t e = __atomic_load_n(m->h_stack_fail, __ATOMIC_ACQUIRE);
   if (!e) return 0;
   *m->h_stack_fail = 0;
-  if (hipMemcpy(m->d_stack_fail, m->h_stack_fail, 4, hipMemcpyHostToDevice) != hipSuccess) m->stack_fails = STACK_MAX_FAILS;
-  ++m->stack_fails;
+  if (++m->stack_fails >= STACK_MAX_FAILS) m->stack_pause = STACK_PAUSE;
+  if (hipMemcpy(m->d_stack_fail, m->h_stack_fail, 4, hipMemcpyHostToDevice) != hipSuccess) m->stack_pause = INT64_MAX;
   return e;
 }
 // Behind a wait for a single step: true if the step has been enqueued again, as separate launches

@@ -431,3 +431,32 @@ def test_two_models_give_the_bits_of_one(gpu, monkeypatch):
     assert [m.debug_decode_stack() for m in ms] == [(steps + 1, 0), (steps, 0)]
     for m in [alone] + ms:
         m.close()
+
+
+def test_a_model_that_gave_up_tries_again(gpu, monkeypatch):
+    """Three steps that gave up: 16384 steps as separate launches, then one launch again; a fourth that gives up: as many again."""
+    cfg, plain, (m,) = models(monkeypatch, vocab=256)
+    plain.close()
+    ids = ids_for(cfg, 30, 1)
+
+    def steps(n):
+        while n:
+            m.clear_cache()
+            _, tok = m.forward_initial(ids, 0)
+            n -= len(m.decode_greedy(tok, len(ids), min(n, 500)))
+    m.forward_initial(ids, 0)
+    m.debug_decode_stack(0)
+    for i in range(3):
+        m.forward_step(5, len(ids) + i)
+    assert m.debug_decode_stack(100000) == (3, 3)
+    steps(16384)
+    assert m.debug_decode_stack() == (3, 3)
+    steps(5)
+    assert m.debug_decode_stack(0) == (8, 3)
+    m.clear_cache()
+    m.forward_initial(ids, 0)
+    m.forward_step(5, len(ids))
+    assert m.debug_decode_stack(100000) == (9, 4)
+    steps(700)
+    assert m.debug_decode_stack() == (9, 4)
+    m.close()
