@@ -130,7 +130,7 @@ struct LayeredModel {
   const int32_t* ext_dev = nullptr;   // (windows, entries) first gathered row of every entry
   std::vector<int> ext_total, ext_max;
   // one token of one sequence: which layers' halves run together (kernels_prenorm_stack.hip); first < 0: this half by itself
-  struct StackItem { int layer, half, first, n; };
+  struct StackItem { int layer, half, first, n; double weights, states; };   // (elements of its matrices that a step reads, f32s of its states)
   std::vector<StackItem> schedule;
   PrenormOp* d_ops = nullptr;     // null: every half by itself
   int64_t stack_hist = 0;         // floats of a history of its state-space layers

@@ -592,9 +592,11 @@ static int prenorm_schedule(aha_model* m) {
   LayeredModel& l = *m->layered;
   std::vector<PrenormOp> ops;
   l.schedule.clear();
-  auto add = [&](int li, int half, const PrenormOp* op) {
+  auto add = [&](int li, int half, const PrenormOp* op, double weights = 0, double states = 0) {
     if (op && !l.schedule.empty() && l.schedule.back().first >= 0 && l.schedule.back().n < PRENORM_STACK_OPS) ++l.schedule.back().n;
-    else l.schedule.push_back({li, half, op ? (int)ops.size() : -1, op ? 1 : 0});
+    else l.schedule.push_back({li, half, op ? (int)ops.size() : -1, op ? 1 : 0, 0, 0});
+    l.schedule.back().weights += weights;
+    l.schedule.back().states += states;
     if (op) ops.push_back(*op);
   };
   bool have = false;
@@ -620,7 +622,7 @@ static int prenorm_schedule(aha_model* m) {
       };
       if (!put(W.sp.conv_w, taps * cp) || !put(W.sp.conv_b, cp) || !put(W.sp.dt_bias, heads) || !put(W.sp.a, heads) || !put(W.sp.d, heads))
         return err(AHA_ERR_HIP, "model_create: copying the mixers' parameters failed");
-      add(li, 0, &op);
+      add(li, 0, &op, (double)l.ld * (W.n_in + W.ko), W.sd.state_floats());
     } else {
       add(li, 0, nullptr);
     }
@@ -629,10 +631,10 @@ static int prenorm_schedule(aha_model* m) {
     op.nw = W.n2w; op.nb = W.n2b; op.w1 = W.wgu; op.w2 = W.wdown;
     if (have && d.mlp == AHA_MLP_GATED && prenorm_stack_dense_ok(W.ffp)) {
       op.kind = PRENORM_DENSE;
-      add(li, 1, &op);
+      add(li, 1, &op, 3.0 * l.ld * W.ffp);
     } else if (have && d.mlp == AHA_MLP_MOE && prenorm_stack_moe_ok(d.experts, d.top, W.effp, W.ffp)) {
       op.kind = PRENORM_MOE; op.router = W.w_router; op.egu = W.w_egu; op.edown = W.w_edown;
-      add(li, 1, &op);
+      add(li, 1, &op, (double)l.ld * (d.experts + 3.0 * d.top * W.effp + 3.0 * W.ffp));
     } else {
       add(li, 1, nullptr);
     }
@@ -753,6 +755,7 @@ static Tail prenorm_single(aha_model* m, const SeqBatch& b, const uint32_t* ids)
     float* const hist = l.d_hist + l.hist_slot * b.one.slot;
     p.hist_in = hist + b.one.hist_in * l.stack_hist; p.hist_out = hist + b.one.hist_out * l.stack_hist;
     p.state_in = l.d_pool + b.one.state_in * l.pool_stride; p.state_out = l.d_pool + b.one.state_out * l.pool_stride;
+    ProfScope ps(m, "decode_run", it.weights * 2 + it.states * 8, 2.0 * it.weights);
     launch_prenorm_stack(p, st);
   }
   return Tail{l.xa, nullptr, nullptr, 1.f, {}};

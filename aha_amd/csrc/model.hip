@@ -346,9 +346,9 @@ static void stack_release(aha_model* m) {   // its stream is idle
   if (t.last == m) t.last = nullptr;
 }
 static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_ready = false, bool arg_max = true);
-// Not where a profile, a timeline or a knob asks for the separate launches.
+// Not where a timeline or a knob asks for the separate launches.
 bool StackTurn::take(aha_model* m, bool same_bits) {
-  if (!m->d_stack_exchange || m->stack_hold > 0 || !m->decode_fused || m->profiling) return false;
+  if (!m->d_stack_exchange || m->stack_hold > 0 || !m->decode_fused) return false;
   static const bool knobs = getenv("AHA_ATTN_PAGES_PER_BLOCK") || getenv("AHA_ATTN_TRACE") || getenv("AHA_GEMV_TRACE") || !gemv_row_on();
   if (knobs) return false;
   if (m->stack_pause > 0) {
@@ -1578,7 +1578,11 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_read
     a.layers = m->d_stack_layers; a.x_in = m->d_x; a.x_out = m->d_x; a.rope = m->d_rope; a.page_ptrs = m->d_page_ptrs; a.layer_stride = m->layer_stride;
     a.exchange = m->d_stack_exchange; a.fail_dev = m->d_stack_fail; a.fail_host = m->h_stack_fail_dev;
     a.epoch = model_stack_epoch(m); a.n_layers = c.num_hidden_layers; a.kv_len = (int)kv_len_after; a.polls = m->stack_polls; a.eps = c.rms_norm_eps; a.scale = m->attn_scale;
-    launch_decode_stack(a, st);
+    const double weights = (double)c.num_hidden_layers * H * (2.0 * nq + 2.0 * nkv + 3.0 * I);
+    {
+      ProfScope ps(m, "decode_stack", weights * 2 + (double)c.num_hidden_layers * kv_len_after * 2 * nkv * 2, 2.0 * weights + 4.0 * c.num_hidden_layers * kv_len_after * nq);
+      launch_decode_stack(a, st);
+    }
     enqueue_lm_head(m, m->d_x, arg_max);
     return;
   }
@@ -1609,6 +1613,8 @@ static void enqueue_decode_step(aha_model* m, size_t kv_len_after, bool row_read
       a.x = m->d_x; a.in_norm = L.in_norm; a.wqkv = L.wqkv; a.wo = L.wo; a.q_norm = L.q_norm; a.k_norm = L.k_norm; a.rope = m->d_rope;
       a.page_ptrs = kv.page_ptrs; a.layer_off = kv.layer_off; a.exchange = m->d_stack_exchange; a.fail_dev = m->d_stack_fail; a.fail_host = m->h_stack_fail_dev;
       a.epoch = model_stack_epoch(m); a.kv_len = (int)kv_len_after; a.nsplit = nsplit; a.direct = !defer; a.polls = m->stack_polls; a.eps = c.rms_norm_eps; a.scale = m->attn_scale;
+      const double weights = (double)H * (2.0 * nq + 2.0 * nkv);
+      ProfScope ps(m, "decode_attn", weights * 2 + (double)kv_len_after * 2 * nkv * 2 + H * 4.0, 2.0 * weights + 4.0 * kv_len_after * nq);
       launch_decode_attn(a, st);
     } else {  // h = RMSNorm(x); qkv = h Wqkv^T                      (qwen3/model.rs:79, modules.rs:538-552)
       GemvArgs g{};

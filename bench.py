@@ -10,8 +10,8 @@ inputs are synthetic and resident in HBM when the timed region starts.  Prefill 
 and reported as prefill_tok_s.  Decode stays single-GPU: with N > 1 every rank serves its
 own request (independent replicas, no data-path collective) => "scaling": "weak".
 
-Extra objects on the JSON line: roofline (dominant kernel = the batch-1 weight-streaming matvec, HIP-event timed over
-K further steps) and cpu_baseline (the oracle restatement timed on the host cores on a bounded sample).
+Extra objects on the JSON line: roofline (the dominant class of kernels, at 8B the batch-1 weight-streaming matvec, HIP-event timed over
+K further steps with the launches that the timed ones have), several_stages_in_one_launch (the other ones that stream weights) and cpu_baseline (the oracle restatement timed on the host cores on a bounded sample).
 """
 from __future__ import annotations
 
@@ -442,6 +442,19 @@ def source_digest(files) -> str:
 
 GEMV_SOURCES = ("gemv_body.h", "kernels_gemv.hip", "common.h")
 
+
+def dominant_class(prof: dict) -> str:
+    """The class of launches that a decode step spends most of its time in."""
+    return max(("gemv", "decode_attn", "decode_stack"), key=lambda c: prof[c]["ms"])
+
+
+def class_label(cls: str, prof: dict) -> str:
+    if cls == "gemv":
+        rest = "lm_head" if prof["decode_stack"]["launches"] else "gate / up, down + lm_head" if prof["decode_attn"]["launches"] else "all projections + lm_head"
+        return f"gemv_kernel (batch-1 weight streaming, {rest})"
+    return {"decode_attn": "decode_attn_kernel (a layer's norm, q k v, attention, o_proj and residual)", "decode_stack": "decode_stack_kernel (all layers of a step)"}[cls]
+
+
 def attach_committed_profiles(roof: dict, workload: str, profiles_dir: str = None) -> dict:
     """Numbers that cannot be collected inside the bench process (rocprofv3 kernel-only durations, PMC traffic) come from the committed
     summaries under profiles/ -- attached ONLY when they were taken with the same matvec sources (the digest scripts/stats_to_md.py /
@@ -515,7 +528,7 @@ def layered_bench(args) -> int:
 
         def classes(m):
             r = {}
-            for c in ("gemm", "moe", "ssm", "attn_prefill", "elem", "gemv", "attn_decode"):
+            for c in ("gemm", "moe", "ssm", "attn_prefill", "elem", "gemv", "attn_decode", "decode_run"):
                 p = m.get_profile(c)
                 if p["launches"]:
                     r[c] = {"us_per_launch": round(1e3 * p["ms"] / p["launches"], 2), "launches": p["launches"], "GB_s": round(p["bytes"] / p["ms"] / 1e6, 1),
@@ -756,25 +769,28 @@ def main():
     job_value, dt = parallel.aggregate_throughput(float(args.steps), dt, device=dev)  # sum of tokens / max over ranks
     kv_mid = off - args.steps // 2
 
-    # ---- roofline of the dominant kernel (weight-streaming matvec), HIP events on the model's stream ----
+    # ---- roofline of the dominant kernel class, HIP events on the model's stream around the launches that the timed steps have ----
     model.set_profiling(True)
     tok, off = run_steps(args.steps, tok, off)
-    prof = {k: model.get_profile(k) for k in ("gemv", "attn_decode", "elem", "argmax")}
+    prof = {k: model.get_profile(k) for k in ("gemv", "attn_decode", "elem", "argmax", "decode_attn", "decode_stack")}
     model.set_profiling(False)
-    # dominant kernel class of a decode step: the weight-streaming matvec (all projections + lm_head)
-    gv = prof["gemv"]
+    dominant = dominant_class(prof)
+    gv = prof[dominant]
     achieved = gv["bytes"] / (gv["ms"] * 1e-3) / 1e9 if gv["ms"] > 0 else 0.0
     roof = {"bound": "hbm",
-            "kernel": "gemv_kernel (batch-1 weight streaming, all projections + lm_head)",
+            "kernel": class_label(dominant, prof),
             "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
             "launches": gv["launches"], "avg_us": round(1e3 * gv["ms"] / max(gv["launches"], 1), 2),
             "algorithmic_bytes_per_launch": round(gv["bytes"] / max(gv["launches"], 1)),
             "timing": "HIP event pairs on the model's stream around every launch of the class, collected in THIS run (a pair also sees "
                       "the ~2.5 us of dispatch latency in front of a kernel: the rocprofv3 kernel-only figure, when attached, is the higher one)"}
-    attach_committed_profiles(roof, args.workload)
-    ad = prof["attn_decode"]
-    attn_gbs = ad["bytes"] / (ad["ms"] * 1e-3) / 1e9 if ad["ms"] > 0 else 0.0
+    if dominant == "gemv":
+        attach_committed_profiles(roof, args.workload)
+    one_launch = {c: {"kernel": class_label(c, prof), "launches": prof[c]["launches"], "avg_us": round(1e3 * prof[c]["ms"] / prof[c]["launches"], 2),
+                      "GBs": round(prof[c]["bytes"] / prof[c]["ms"] / 1e6, 1)} for c in ("decode_attn", "decode_stack") if prof[c]["launches"]}
+    ad = prof["attn_decode"]      # (None: the attention is part of one of the launches above)
+    attn_gbs = round(ad["bytes"] / (ad["ms"] * 1e-3) / 1e9, 1) if ad["ms"] > 0 else None
 
     if rank == 0:
         # the other half of BASELINE's metric: the prefill against the dense bf16 MFMA peak (attention counted causally; stated)
@@ -805,7 +821,7 @@ def main():
             "roofline_prefill": roof_prefill,
             "prefill_ms_samples": [round(1e3 * t, 2) for t in t_prefills],
             "decode_step_hbm_frac": round(step_bytes / (dt / args.steps) / 1e9 / HBM_PEAK_GBS, 4),
-            "attn_decode_GBs": round(attn_gbs, 1),
+            "attn_decode_GBs": attn_gbs, "several_stages_in_one_launch": one_launch,
             "load_s": round(t_load, 1),
             "roofline": roof,
         }

@@ -400,7 +400,8 @@ int64_t aha_hip_debug_steps_executed(const aha_model* m);
 int aha_hip_debug_graph_step(aha_model* m, int32_t replays, double* us_launches, double* us_graph);
 /* Per-kernel-class HIP-event timing of subsequent forward calls (adds one event pair per launch).  0 = off. */
 int aha_hip_set_profiling(aha_model* m, int enable);
-/* name: e.g. "gemv", "gemm", "attn_decode", "attn_prefill".  Returns accumulated ms and launch count since enable. */
+/* name: e.g. "gemv", "gemm", "attn_decode", "attn_prefill"; steps with several stages in one launch: "decode_stack" (all layers), "decode_attn" (a layer's q k v,
+ * attention and o_proj), "decode_run" (sublayers of the state-space design).  A step takes the same launches as without a profile.  Returns accumulated ms and launch count since enable. */
 int aha_hip_get_profile(aha_model* m, const char* kernel_class, double* total_ms, int64_t* launches, double* bytes,
                         double* flops);
 /* Debug knob for the paged-KV property tests: 1 => hand out physical pages in a scrambled order. */

@@ -460,3 +460,48 @@ def test_a_model_that_gave_up_tries_again(gpu, monkeypatch):
     steps(700)
     assert m.debug_decode_stack() == (9, 4)
     m.close()
+
+
+def test_profile_of_the_launches_that_run(gpu, monkeypatch):
+    """A profiled step is the step without a profile: the same bits, the one-launch forms booked as classes of their own with the bytes of what they read."""
+    def profiled(m, step, classes):
+        m.set_profiling(True)
+        step()
+        m.set_profiling(False)
+        return [m.get_profile(c) for c in classes]
+
+    def near(p, elements, launches):
+        assert p["launches"] == launches and 2 * elements <= p["bytes"] <= 1.02 * 2 * elements, p
+
+    S, cache = 300, 301 * 2 * 1024                       # (of a layer)
+    for make, layers, H, nq, inter, vocab in ((models, 3, 1024, 2048, 3072, 1024), (wide_models, 2, 4096, 4096, 1024, 512)):
+        cfg, plain, m = make(monkeypatch)
+        m = m[0] if isinstance(m, list) else m
+        plain.close()
+        ids = ids_for(cfg, S, 2)
+        m.forward_initial(ids, 0)
+        want, _ = m.forward_step(5, S)
+        m.clear_cache()
+        m.forward_initial(ids, 0)
+        got = []
+        stack, attn, gemv, separate = profiled(m, lambda: got.append(m.forward_step(5, S)[0]), ("decode_stack", "decode_attn", "gemv", "attn_decode"))
+        np.testing.assert_array_equal(got[0], want)
+        half, ff = H * (2 * nq + 2 * 1024), 3 * H * inter
+        assert separate["launches"] == 0
+        if make is models:
+            near(stack, layers * (half + ff + cache), 1)
+            near(gemv, vocab * H, 1)
+            assert attn["launches"] == 0
+        else:
+            near(attn, layers * (half + cache), layers)
+            near(gemv, layers * ff + vocab * H, 2 * layers + 1)
+            assert stack["launches"] == 0
+        m.close()
+
+    cfg, plain, (m,) = pre_norm_models(monkeypatch)
+    plain.close()
+    ids = ids_for(cfg, 30, 2)
+    m.forward_initial(ids, 0)
+    (runs,) = profiled(m, lambda: m.forward_step(5, 30), ("decode_run",))
+    assert runs["launches"] == 2 and runs["bytes"] > 0
+    m.close()
