@@ -505,3 +505,54 @@ def test_profile_of_the_launches_that_run(gpu, monkeypatch):
     (runs,) = profiled(m, lambda: m.forward_step(5, 30), ("decode_run",))
     assert runs["launches"] == 2 and runs["bytes"] > 0
     m.close()
+
+
+@pytest.mark.parametrize("S, pages", [(700, (0, 1, 5, 10)), (2100, (0, 1, 31, 32)), (4159, (0, 32, 63, 64)), (6330, (2, 34, 66, 98)), (6300, (1, 33, 65, 97)),
+                                      (32700, (30, 62, 94, 126)), (32700, (30, 286, 478, 510))])
+def test_every_page_counts_once(gpu, monkeypatch, S, pages):
+    """Four keys, one on each of four pages, take the whole weight of the new token's attention in every layer, a quarter each, and their values differ: without one
+    of these pages, or with one twice, the logits are others.  A block's first, second and later pages, the first and the last page.  How: half of the columns of the
+    residual stream never change; keys read those alone, queries the same in reverse order, values the rest; the dims that rotate visibly have no weight."""
+    import dataclasses
+    import torch
+    from aha_amd.model import HipInferenceModel
+    cfg = dataclasses.replace(tiny_qwen3(layers=3, hidden=1024, heads=16, kv_heads=8, inter=3072, vocab=1024), rope_theta=1e12)
+    w = qwen3_text_weights(cfg, seed=21)
+    emb, mid = w["model.embed_tokens.weight"], 512
+    emb[1:5, :mid] = emb[1, :mid].clone()                  # tokens 1 to 4: the same key, four values
+    emb[0, :mid] = emb[1, :mid].flip(0)                    # token 0: the query of that key
+    for i in range(cfg.num_hidden_layers):
+        p = f"model.layers.{i}."
+        k = w[p + "self_attn.k_proj.weight"]
+        k[:, mid:] = 0
+        heads = k.view(8, 1, 128, 1024).expand(8, 2, 128, 1024).reshape(2048, 1024)
+        w[p + "self_attn.q_proj.weight"] = torch.cat([heads[:, :mid].flip(1), heads[:, mid:]], 1).contiguous()
+        w[p + "self_attn.v_proj.weight"][:, :mid] = 0
+        w[p + "self_attn.o_proj.weight"][:mid] = 0
+        w[p + "mlp.down_proj.weight"][:mid] = 0
+        for n in ("q_norm", "k_norm"):                     # pairs 32 to 63 of the rotation: an angle of 0.03 at most; scores of 51 for the four, 6.4 of spread for others
+            g = torch.zeros(128)
+            g[32:64] = g[96:128] = 3.0
+            w[p + f"self_attn.{n}.weight"] = g.bfloat16()
+        w[p + "input_layernorm.weight"][:] = 1
+    monkeypatch.setenv("AHA_DECODE_STACK", "0")
+    plain = HipInferenceModel(cfg, w)
+    monkeypatch.setenv("AHA_DECODE_STACK", "1")
+    m = HipInferenceModel(cfg, w)
+    ids = [5 + t % 1019 for t in ids_for(cfg, S, S + pages[1])]
+    places = [p * 64 + (0, 63, 17, 40)[j] for j, p in enumerate(pages)]
+    assert places[-1] < S
+    for j, at in enumerate(places):
+        ids[at] = 1 + j
+
+    def step(x, ids):
+        x.clear_cache()
+        x.forward_initial(ids, 0, want_logits=False)
+        return x.forward_step(0, S)[0]
+    want = step(plain, ids)
+    close_to(want, step(m, ids), (S, pages))
+    assert m.debug_decode_stack() == (1, 0)
+    for j, at in enumerate(places):                        # (what the test can see: without one of the four the logits are far outside the bound)
+        other = step(plain, ids[:at] + [77 + j] + ids[at + 1:])
+        assert float(np.sqrt(((want - other) ** 2).mean())) > 10 * LOGIT_RMS_STD * float(want.std()), (S, at)
+    m.close(); plain.close()
