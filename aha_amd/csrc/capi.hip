@@ -538,6 +538,16 @@ int aha_hip_debug_gemm_f32(const float* A, const void* W, float* C, int32_t M, i
   return AHA_OK;
 }
 
+int aha_hip_debug_dot_bf16(const void* W, const void* x, float* y, int32_t N, int32_t K, int32_t chain, void* stream) {
+  if (!W || !x || !y || N <= 0 || K <= 0 || K % 512) {
+    set_error("debug_dot_bf16: bad argument");
+    return AHA_ERR_INVALID;
+  }
+  launch_stack_dot(W, x, y, N, K, chain != 0, (hipStream_t)stream);
+  AHA_HIP_CHECK(hipGetLastError());
+  return AHA_OK;
+}
+
 int aha_hip_qknorm_rope(const void* qkv, const void* q_norm_w, const void* k_norm_w, const int32_t* pos,
                         const int32_t* axis_map, void* q_out, void* k_out, void* v_out, int32_t S, int32_t nh,
                         int32_t kvh, int32_t d, float eps, float theta, void* stream) {

@@ -182,6 +182,7 @@ struct DecodeStackArgs {
 };
 bool decode_stack_sizes_ok(int width, int heads, int kv_heads, int head_dim, int ff);
 void launch_decode_stack(const DecodeStackArgs& a, hipStream_t st);
+void launch_stack_dot(const void* w, const void* x, float* y, int n, int k, bool chain, hipStream_t st);   // its dot products by themselves, for a test
 
 // Norm, q k v, attention, o_proj and residual of one layer of a decode step in one launch (kernels_decode_attn.hip); blocks, exchange, epochs and polls as above
 struct DecodeAttnArgs {

@@ -497,8 +497,23 @@ __global__ __launch_bounds__(512, 2) void decode_stack_kernel(const DecodeStackA
   else gather_waves(a, lds, b, wave - 4);
 }
 
+__global__ __launch_bounds__(64) void stack_dot_kernel(const bf16_t* __restrict__ w, const bf16_t* __restrict__ x, float* __restrict__ y, int k, bool chain) {
+  float s = 0.f;
+  for (int i = threadIdx.x * 8; i < k; i += 512) {
+    const u32x4_t h = ld16(x + i), wt = ld16(w + (int64_t)blockIdx.x * k + i);
+    if (!chain) s = dot8_bf(h, wt, s);
+    else
+      for (int j = 0; j < 4; ++j) s = fmaf(hi_bf(h[j]), hi_bf(wt[j]), fmaf(lo_bf(h[j]), lo_bf(wt[j]), s));
+  }
+  s = wave_sum(s);
+  if (threadIdx.x == 0) y[blockIdx.x] = s;
+}
+
 }  // namespace
 
+void launch_stack_dot(const void* w, const void* x, float* y, int n, int k, bool chain, hipStream_t st) {
+  hipLaunchKernelGGL(stack_dot_kernel, dim3((unsigned)n), dim3(64), 0, st, (const bf16_t*)w, (const bf16_t*)x, y, k, chain);
+}
 bool decode_stack_sizes_ok(int width, int heads, int kv_heads, int head_dim, int ff) {
   return width == H && heads == NH && kv_heads == KVH && head_dim == D && ff == FF;
 }

@@ -410,7 +410,8 @@ int aha_hip_debug_scramble_pages(aha_model* m, int enable);
  * counts back); a new model has no limit. */
 int aha_hip_debug_memory_limit(aha_model* m, size_t bytes);
 /* Test hook for decode steps whose layers run as one launch: polls >= 0 sets how often a wave of it asks in vain before it gives up and the step is run again as
- * separate launches (0: at once); steps run so and steps given up so far. */
+ * separate launches (0: at once); steps: launches with several stages so far (one a step at 0.6B, one a layer at 8B, one a run of sublayers), given_up: steps that had to be run
+ * again. */
 int aha_hip_debug_decode_stack(aha_model* m, int32_t polls, int64_t* steps, int64_t* given_up);
 /* Copies the last hidden state before lm_head (hidden_size floats) / the image embeddings of the last
  * forward_initial (rows x out_hidden floats) to the host, for parity tests of intermediate tensors. */
@@ -426,6 +427,9 @@ int aha_hip_debug_gemm_grouped(const void* A, const void* W, void* C, int32_t M,
                                int32_t groups, int32_t a_gstride, int32_t c_gstride, int32_t c_row0, int32_t m_total, void* stream);
 /* Test entry of the layer lists' 32-bit products (csrc/kernels_gemm_f32.hip): C (M, N) f32 = A (M, K) f32 . W (N, K)^T bf16, `batch` of them one behind another. */
 int aha_hip_debug_gemm_f32(const float* A, const void* W, float* C, int32_t M, int32_t N, int32_t K, int32_t batch, void* stream);
+/* Test entry of the dot products inside the one-launch decode step (csrc/stack_exchange.h dot8_bf): y (N) f32 = W (N, K) . x (K), bf16, K a multiple of 512, a wave a
+ * row as there; chain != 0: the same sums as a chain of f32 fma. */
+int aha_hip_debug_dot_bf16(const void* W, const void* x, float* y, int32_t N, int32_t K, int32_t chain, void* stream);
 /* Test hook: the prefill attention's score chain.  3 (the default since round 5; env AHA_ATTN_SMX) = the scores stay the f32 QK^T
  * accumulators through scale, mask, maximum and exponential, P is rounded to bf16 once for the P.V product; 1 / 0 = the reference's
  * eager path, which materialises `q.k^T` and `* scaling` in bf16 (modules.rs:782-783), with the scale multiply on the matrix pipe
