@@ -49,7 +49,6 @@ struct Lds {
 // naps of 64 clocks (27 ns): before the first weights are asked for (x comes first: 8 naps 70.9 us a layer, 12: 70.1,
 // 16: 70.3, 22: 70.4), before the units' sums, before all the joined sums
 constexpr int NAP_W = 12, NAP_P = 20, NAP_A = 40;
-#define IN_ORDER __builtin_amdgcn_sched_barrier(0)
 
 // h of eight columns and eight weights, in the order of gemv_body.h
 __device__ __forceinline__ float add_group(const Lds& lds, int u, int lane, u32x4_t wt, float y) {
@@ -440,10 +439,7 @@ __device__ __forceinline__ void gather_waves(const DecodeAttnArgs& a, Lds& lds, 
       *reinterpret_cast<float4*>(lds.xs + xs_index(tid * 4 + j * 1024)) = make_float4(hi_bf(v[j][0]), hi_bf(v[j][1]), hi_bf(v[j][2]), hi_bf(v[j][3]));
     meet();
   }
-  if (poll.left <= 0 && !failed && lane == 0) {
-    __hip_atomic_store(a.fail_dev, a.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(a.fail_host, a.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  }
+  poll.report(failed, a.fail_dev, a.fail_host, a.epoch);
 }
 
 template <bool DIRECT>

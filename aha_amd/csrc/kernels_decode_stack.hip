@@ -52,7 +52,6 @@ struct Lds {
 };
 
 // ---- the waves that compute ------------------------------------------------------------------------------------------------------------------
-__device__ __forceinline__ float silu_of(float x) { return x / (1.0f + expf(-x)); }
 
 // PG: pages that are requested a layer ahead (1: no block has a second one)
 template <int PG>
@@ -133,7 +132,6 @@ __device__ __forceinline__ void compute_waves(const DecodeStackArgs& a, Lds& lds
   // requests are spread over the layer: small ones where a stage begins to compute (HBM's latency passes under it), 32 KB behind what q, k, v of the next layer and
   // gate and up left, where the others' parts need a microsecond to cross anyway.  us a token at 400 / 2048 positions: everything requested behind its stage
   // 424 / 469; all in front of the stages 362 / 413; in two bursts in front of what crosses 394 / 448, behind it 362 / 413; so 346 / 368.
-#define IN_ORDER __builtin_amdgcn_sched_barrier(0)
   auto get_pages = [&](int l, bool have) {
 #pragma unroll
     for (int i = 0; i < PG; ++i) {
@@ -483,10 +481,7 @@ __device__ __forceinline__ void gather_waves(const DecodeStackArgs& a, Lds& lds,
     res = f2bf(bf2f(res) + rbf(poll.sum_parts<H>(AT_D, row, tag)));
     if (x == 0 && lane < 32) ((bf16_t*)a.x_out)[row] = res;
   }
-  if (poll.left <= 0 && !failed && lane == 0) {
-    __hip_atomic_store(a.fail_dev, a.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(a.fail_host, a.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  }
+  poll.report(failed, a.fail_dev, a.fail_host, a.epoch);
 }
 
 template <int PG>

@@ -59,7 +59,6 @@ struct Lds {
   int sel[TOP];
   float wt[TOP];
 };
-__device__ __forceinline__ float silu_of(float x) { return x / (1.0f + expf(-x)); }
 __device__ __forceinline__ float softplus(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
 
 __device__ __forceinline__ float dot8(const float (&h)[8], u32x4_t w, float s) {
@@ -75,7 +74,6 @@ __device__ __forceinline__ void ld8(const float* p, float (&h)[8]) {
   h[0] = a.x; h[1] = a.y; h[2] = a.z; h[3] = a.w; h[4] = b.x; h[5] = b.y; h[6] = b.z; h[7] = b.w;
 }
 __device__ __forceinline__ int pair_row(int f) { return (f >> 4) * 32 + (f & 15); }   // gate row of a feature (16-row blocks alternating gate / up)
-#define IN_ORDER __builtin_amdgcn_sched_barrier(0)
 
 // ---- the waves that compute ------------------------------------------------------------------------------------------------------------------
 __device__ __forceinline__ void compute_waves(const PrenormStackArgs& a, Lds& lds, const int b, const int w) {
@@ -421,10 +419,7 @@ __device__ __forceinline__ void gather_waves(const PrenormStackArgs& a, Lds& lds
     res += poll.sum_parts<H>(AT_PART + ((a.n_ops - 1) & 1) * PART, row, a.epoch * PRENORM_STACK_OPS + a.n_ops - 1);
     if (x == 0 && lane < 32) a.x_out[row] = res;
   }
-  if (poll.left <= 0 && !failed && lane == 0) {
-    __hip_atomic_store(a.fail_dev, a.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(a.fail_host, a.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  }
+  poll.report(failed, a.fail_dev, a.fail_host, a.epoch);
 }
 
 __global__ __launch_bounds__(512, 2) void prenorm_stack_kernel(const PrenormStackArgs a) {

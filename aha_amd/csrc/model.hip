@@ -332,7 +332,9 @@ int alloc_slab(aha_model* m) {
 // Where both forms give the same bits (8B) the second one does not wait: 5.0 and 4.15 ms a token that way, 5.5 each by turns.
 constexpr int STACK_MAX_FAILS = 3;    // steps given up (50 ms and more each) after which a model stays with separate launches,
 constexpr int64_t STACK_PAUSE = 16384;   // for so many steps (8 s at 0.6B, more elsewhere), and then after every other one: at most 1 % is waited in vain
-constexpr int STACK_MAX_PAGES = 512;   // 32768 positions: 980 us a token, 1210 as separate launches (a page more costs 1.3 us here, 0.9 there)
+// 32768 positions, as far as the two forms are held against each other by tests: 985 us a token here, 1225 as separate launches.  Speed would carry it to some 105 000, where
+// the forms meet: a page more costs 1.30 us here and 1.05 there (us a token at 7 k positions 475 and 685, 16 k 657 and 966, 56 k 1476 and 1616, 100 k 2377 and 2405, 125 k 2897 and 2825).
+constexpr int STACK_MAX_PAGES = 512;
 struct StackTurns {
   std::mutex mu;
   aha_model* last = nullptr;    // had the last turn and has not been waited for since

@@ -15,6 +15,8 @@ constexpr u32x4_t NO_SPLIT = {0xff800000u, 0u, 0u, 0u};   // what a split of the
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
 }
+#define IN_ORDER __builtin_amdgcn_sched_barrier(0)   // of requests and results, as written
+__device__ __forceinline__ float silu_of(float x) { return x / (1.0f + expf(-x)); }
 // LDS of this wave written and read, everybody here; requests of weights stay in flight
 __device__ __forceinline__ void meet() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
@@ -60,6 +62,12 @@ struct Poller {
       if (left <= 0) return none();
       --left;
     }
+  }
+  // behind the last wait: the launch is marked where this wave gave up (and no earlier one had been)
+  __device__ __forceinline__ void report(bool failed, unsigned* fail_dev, unsigned* fail_host, uint32_t epoch) const {
+    if (left > 0 || failed || (threadIdx.x & 63)) return;
+    __hip_atomic_store(fail_dev, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(fail_host, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
   // four values (of a lane that takes part)
   __device__ __forceinline__ u32x4_t values(bool part, uint32_t at, uint32_t t16) {
