@@ -359,12 +359,11 @@ bool StackTurn::take(aha_model* m, bool same_bits) {
   }
   StackTurns& t = stack_turns(m);
   lk = std::unique_lock<std::mutex>(t.mu);
-  if (t.last && t.last != m) {
+  if (t.last && t.last != m && hipStreamQuery(t.last->stream) != hipSuccess) {   // (it lives: a model gives its turn back before it goes)
     if (same_bits) {
       lk.unlock();
       return false;
     }
-    // (its stream lives: a model gives its turn back before it goes)
     if ((!t.behind && hipEventCreateWithFlags(&t.behind, hipEventDisableTiming) != hipSuccess) || hipEventRecord(t.behind, t.last->stream) != hipSuccess ||
         hipStreamWaitEvent(m->stream, t.behind, 0) != hipSuccess) {
       (void)hipGetLastError();
@@ -2248,7 +2247,7 @@ static int forward_initial_impl(aha_model* m, const uint32_t* ids, size_t n, siz
       if (one_launch) break;
     }
     if (li + 1 == c.num_hidden_layers && m->tp_size <= 1 && !(has_image && vision_has_deepstack(m, li)) && nq * 4 >= H) {
-      if (docs) {   // (a document has two rows or more, so theirs fit where the attention's were)
+      if (docs) {   // (64 documents at most, and 256 rows or more in every buffer: their rows of H <= 4 nq fit where the attention's were)
         n_rows = (int)docs->size();
         launch_embed_gather(m->p_attn, tables->last, m->p_q, n_rows, nq, st);
         launch_embed_gather(m->p_x, tables->last, m->p_attn, n_rows, H, st);

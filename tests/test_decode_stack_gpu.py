@@ -586,3 +586,19 @@ def test_dot_products_of_pairs(gpu, K, what):
         off.append(float((((y.double() - exact) / size) ** 2).mean().sqrt()))
     # (rms over 8192 sums: drawn anew they differ by 1 %)
     assert off[0] <= (2 ** 0.5 if what == "wide" else 1.02) * off[1] and off[0] < 2 ** -24, off
+
+
+def test_a_step_that_nobody_asked_for_holds_nobody_up(gpu, monkeypatch):
+    """A model's queued step has run and is not asked for: the next step of another one, also where it would make way (4096 columns), takes the one launch."""
+    import torch
+    _, plain, (first,) = models(monkeypatch)
+    cfg, plain2, wide = wide_models(monkeypatch)
+    plain.close(); plain2.close()
+    ids = ids_for(cfg, 40, 1)
+    wide.forward_initial(ids, 0)
+    first.forward_initial(ids, 0)
+    first.forward_step_enqueue(3, 40)
+    torch.cuda.synchronize()
+    wide.forward_step(3, 40)
+    assert wide.debug_decode_stack() == (2, 0)
+    wide.close(); first.close()
