@@ -21,7 +21,8 @@
 // 1210 -> 980.  A layer is 10 us: 31 MB of weights (5.4 at the rate HBM reaches, most of it under what follows), 2.7 of arithmetic, four hand-offs inside an XCD, two across.
 //
 // Waits are bounded: the blocks have to be on the GPU together (and where they are thought to be), which nothing promises.  A wave that has polled in vain for long
-// enough waits no more in this launch; the launch then ends by itself with garbage and says so in `fail`, and the host runs the step as separate launches (model.hip).
+// enough waits no more in this launch and goes on with zeros; the launch then ends by itself, with numbers that mean nothing, and says so in `fail`, and the host runs the
+// step as separate launches (model.hip).
 #include "attn_common.h"
 #include "kernels.h"
 #include "stack_exchange.h"

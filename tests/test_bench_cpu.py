@@ -172,3 +172,16 @@ def test_sharded_legs_order_and_survival_of_an_exception():
     line = {}
     bench.run_sharded_legs(["tp", "cp"], run_leg, 3, 8, 8, line, 30)
     assert line == {}
+
+
+def test_the_dominant_class_is_named_for_what_it_has():
+    """The roofline's class is the one with the most time, under a name that leaves out what another launch of the step does."""
+    import bench
+    none = {"ms": 0.0, "launches": 0}
+    separate = {"gemv": {"ms": 40.0, "launches": 145}, "decode_attn": none, "decode_stack": none}
+    joined = {"gemv": {"ms": 40.0, "launches": 73}, "decode_attn": {"ms": 15.0, "launches": 36}, "decode_stack": none}
+    stack = {"gemv": {"ms": 1.0, "launches": 20}, "decode_attn": none, "decode_stack": {"ms": 6.0, "launches": 20}}
+    assert [bench.dominant_class(p) for p in (separate, joined, stack)] == ["gemv", "gemv", "decode_stack"]
+    assert "all projections" in bench.class_label("gemv", separate)
+    assert "gate / up" in bench.class_label("gemv", joined) and "all projections" not in bench.class_label("gemv", joined)
+    assert "all layers" in bench.class_label("decode_stack", stack)
